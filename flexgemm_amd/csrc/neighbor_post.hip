@@ -13,6 +13,7 @@
 
 #include <rocprim/rocprim.hpp>
 
+#include "cache_parts.h"
 #include "fgx_common.h"
 #include "radix_sort.h"
 
@@ -20,8 +21,7 @@ namespace fgx {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kPairRows = 256;       // voxels per block in the pair-list passes (larger blocks were not faster)
-constexpr int kPairThreads = 256;    // ... walked in chunks of this many
+constexpr int kPairThreads = 256;    // a block of the pair-list passes is walked in chunks of this many voxels (larger blocks were not faster)
 
 __global__ void __launch_bounds__(kBlock) iota_u32_kernel(uint32_t* out, size_t n) {
     size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
@@ -65,7 +65,7 @@ __global__ void __launch_bounds__(kBlock) chunk_code_key_kernel(const uint32_t* 
 }
 
 struct LocalityLayout {
-    size_t keys_a, keys_b, vals_a, vals_b, temp, temp_bytes, total;
+    size_t keys_a, keys_b, vals_a, vals_b, temp, temp_bytes, radix, total;
 };
 
 LocalityLayout locality_layout(size_t n) {
@@ -81,6 +81,8 @@ LocalityLayout locality_layout(size_t n) {
     L.vals_b = off; off = align_up(off + nn * 4, 256);
     L.temp = off;   off = align_up(off + temp_bytes, 256);
     L.temp_bytes = temp_bytes;
+    L.radix = off;
+    if (n <= kRsMaxItems) off += radix_layout(n).total;
     L.total = off;
     return L;
 }
@@ -92,15 +94,60 @@ int bits_for(size_t x) {   // smallest b with 2^b > x
 }
 
 
-// The mask sort: between these sizes the radix sort of radix_sort.h is ahead of the library's (measured, 27-bit keys:
-// 0.095 against 0.154 ms at 669 288 items; 0.077 against 0.068 ms at 166 232, where the library sorts blocks and merges
-// them; 0.189 against 0.182 ms at 2 667 120, where it runs onesweep passes with tiles sorted in LDS first).
-constexpr size_t kOwnSortMin = 393216, kOwnSortMax = 2097152;
+// Mask sort of up to this many rows: every row counts the rows that come before it (rank_sort_kernel) -- one launch of n^2
+// compares against nine of the radix sort (8 192 rows 0.017 ms against 0.037, 16 384 rows 0.030 against 0.039; the crossing lies
+// near 20 000).
+constexpr size_t kRankSortMax = 16384;
+constexpr int kRankSlices = 16;      // wavefronts of a workgroup, each counting over a sixteenth of the keys for the same 64 rows
+
+// order[rank of row i] = i, rows by (key, row).  A wavefront takes its keys 64 at a time, one per lane, and compares its 64
+// rows with each of them in turn (read from the lane that holds it).  Chunks are aligned to the workgroup's own 64 rows, so
+// whether equal keys come before or after is the same for a whole chunk, but for the one that is the rows themselves.
+template <typename Before>
+__device__ __forceinline__ uint32_t count_before(uint32_t held, uint32_t len, Before before) {
+    uint32_t count = 0u;
+    if (len == 64u) {
+#pragma unroll
+        for (int k = 0; k < 64; ++k) count += before((uint32_t)__builtin_amdgcn_readlane((int)held, k), (uint32_t)k) ? 1u : 0u;
+    } else {
+        for (uint32_t k = 0; k < len; ++k) count += before((uint32_t)__builtin_amdgcn_readlane((int)held, (int)k), k) ? 1u : 0u;
+    }
+    return count;
+}
+
+__global__ void __launch_bounds__(64 * kRankSlices) rank_sort_kernel(const uint32_t* __restrict__ keys, uint32_t n, uint32_t flip,
+                                                                     int64_t* __restrict__ order) {
+    __shared__ uint32_t part[kRankSlices][64];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t i0 = blockIdx.x * 64u, i = i0 + lane;
+    const uint32_t mine = i < n ? keys[i] ^ flip : 0u;
+    uint32_t before = 0u;
+    uint32_t j = wave * 64u;                                        // the wavefronts take the chunks in turn
+    uint32_t next = j + lane < n ? keys[j + lane] ^ flip : 0u;
+    while (j < n) {
+        const uint32_t held = next, len = n - j < 64u ? n - j : 64u, at = j;
+        j += kRankSlices * 64u;
+        next = j + lane < n ? keys[j + lane] ^ flip : 0u;           // the next chunk is on its way
+        if (at < i0) before += count_before(held, len, [&](uint32_t other, uint32_t) { return other <= mine; });
+        else if (at > i0) before += count_before(held, len, [&](uint32_t other, uint32_t) { return other < mine; });
+        else before += count_before(held, len, [&](uint32_t other, uint32_t k) { return other < mine || (other == mine && k < lane); });
+    }
+    part[wave][lane] = before;
+    __syncthreads();
+    if (wave == 0u && i < n) {
+        uint32_t rank = 0u;
+#pragma unroll
+        for (int w = 0; w < kRankSlices; ++w) rank += part[w][lane];
+        order[rank] = (int64_t)i;
+    }
+}
 
 struct SortLayout {
     size_t keys_out, vals_in, vals_out, temp, temp_bytes, total;
 };
 
+// the library sort, for more rows than the radix sort of radix_sort.h takes
 SortLayout sort_layout(size_t n) {
     SortLayout L{};
     size_t nn = n ? n : 1;
@@ -145,12 +192,56 @@ __global__ void __launch_bounds__(kPairThreads) pair_count_kernel(const int32_t*
     }
 }
 
-// seg[v] = offsets[v * nblk] for v < V, seg[V] = total (last offset + last count)
-__global__ void pair_seg_kernel(const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ counts, int V,
-                                unsigned nblk, uint32_t* __restrict__ seg) {
-    int v = threadIdx.x;
-    if (v < V) seg[v] = nblk ? offsets[(size_t)v * nblk] : 0u;
-    if (v == V) seg[V] = nblk ? offsets[(size_t)V * nblk - 1] + counts[(size_t)V * nblk - 1] : 0u;
+// offsets[v * nblk + blk] = pairs of offset v in the blocks before blk, totals[v] = all of them: one workgroup per offset, four
+// blocks per thread and turn.  A block's count is the sum of GROUP consecutive entries of counts[v][m].
+template <int GROUP>
+__global__ void __launch_bounds__(256) pair_scan_kernel(const uint32_t* __restrict__ counts, size_t m, unsigned nblk,
+                                                        uint32_t* __restrict__ offsets, uint32_t* __restrict__ totals) {
+    __shared__ uint32_t part[4];
+    const uint32_t* row = counts + (size_t)blockIdx.x * m;
+    uint32_t* out = offsets + (size_t)blockIdx.x * nblk;
+    uint32_t carry = 0u;
+    for (unsigned t0 = 0; t0 < nblk; t0 += 1024) {               // (uniform)
+        const unsigned t = t0 + threadIdx.x * 4;
+        uint32_t v[4], sum = 0u, all;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            v[k] = 0u;
+#pragma unroll
+            for (int q = 0; q < GROUP; ++q) {
+                const size_t i = (size_t)(t + k) * GROUP + q;
+                v[k] += i < m ? row[i] : 0u;
+            }
+            sum += v[k];
+        }
+        uint32_t run = carry + block_exclusive_sum<4>(sum, part, &all);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (t + k < nblk) out[t + k] = run;
+            run += v[k];
+        }
+        carry += all;
+    }
+    if (threadIdx.x == 0) totals[blockIdx.x] = carry;
+}
+
+// first pair of offset `v` = pairs of the offsets before it, for lane v of a wavefront (lane V: all pairs)
+__device__ __forceinline__ uint32_t pair_segment(const uint32_t* __restrict__ totals, int V, int lane) {
+    const uint32_t mine = lane < V ? totals[lane] : 0u;
+    uint32_t incl = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)incl, d, 64);
+        if (lane >= d) incl += o;
+    }
+    return incl - mine;
+}
+
+// seg[0 .. V] of an empty (totals == nullptr) or a counted cache
+__global__ void pair_seg_kernel(const uint32_t* __restrict__ totals, int V, uint32_t* __restrict__ seg) {
+    const int v = threadIdx.x;
+    const uint32_t first = totals != nullptr ? pair_segment(totals, V, v) : 0u;
+    if (v <= V) seg[v] = first;
 }
 
 // A block takes kPairRows voxels in chunks of kPairThreads: the chunk's map rows are staged in LDS with coalesced loads,
@@ -161,6 +252,7 @@ __global__ void pair_seg_kernel(const uint32_t* __restrict__ offsets, const uint
 __global__ void __launch_bounds__(kPairThreads) pair_fill_kernel(const uint32_t* __restrict__ map,
                                                                  const int32_t* __restrict__ gray, size_t n, int V,
                                                                  unsigned nblk, const uint32_t* __restrict__ offsets,
+                                                                 const uint32_t* __restrict__ totals, uint32_t* __restrict__ seg,
                                                                  uint32_t* __restrict__ sig_i, uint32_t* __restrict__ sig_o) {
     extern __shared__ uint32_t lds[];
     constexpr int kWaves = kPairThreads / 64;
@@ -168,7 +260,11 @@ __global__ void __launch_bounds__(kPairThreads) pair_fill_kernel(const uint32_t*
     uint32_t* wave_cnt2 = lds + (size_t)kPairThreads * V;    // [2][kWaves][32], by chunk parity
     uint32_t* first = wave_cnt2 + 2 * kWaves * 32;           // [32] where the next pairs of each offset go
     // fetched once, up front: a load inside the offset loop below would put a memory round trip into each of its turns
-    if (threadIdx.x < V) first[threadIdx.x] = offsets[(size_t)threadIdx.x * nblk + blockIdx.x];
+    if (threadIdx.x < 64) {
+        const uint32_t start = pair_segment(totals, V, (int)threadIdx.x);
+        if (threadIdx.x < V) first[threadIdx.x] = start + offsets[(size_t)threadIdx.x * nblk + blockIdx.x];
+        if (seg != nullptr && blockIdx.x == 0 && threadIdx.x <= V) seg[threadIdx.x] = start;
+    }
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     for (int c = 0; c < kPairRows / kPairThreads; ++c) {
@@ -446,7 +542,7 @@ size_t scan_temp_bytes(size_t count) {
 
 struct PairLayout {
     unsigned nblk;
-    size_t counts, offsets, temp, temp_bytes, total;
+    size_t counts, offsets, totals, total;
 };
 
 PairLayout pair_layout(size_t n, int V) {
@@ -456,10 +552,18 @@ PairLayout pair_layout(size_t n, int V) {
     size_t off = 0;
     L.counts = off;  off = align_up(off + (cnt ? cnt : 1) * 4, 256);
     L.offsets = off; off = align_up(off + (cnt ? cnt : 1) * 4, 256);
-    L.temp_bytes = scan_temp_bytes(cnt);
-    L.temp = off;    off = align_up(off + L.temp_bytes, 256);
+    L.totals = off;  off += 256;
     L.total = off;
     return L;
+}
+
+int pair_fill_launch(const uint32_t* map, const int32_t* gray, size_t n, int V, const uint32_t* offsets, const uint32_t* totals, uint32_t* seg,
+                     uint32_t* sig_i, uint32_t* sig_o, hipStream_t s) {
+    const size_t lds = ((size_t)kPairThreads * V + 2 * (kPairThreads / 64) * 32 + 32) * sizeof(uint32_t);
+    const unsigned nblk = cdiv(n, kPairRows);
+    pair_fill_kernel<<<nblk, kPairThreads, lds, s>>>(map, gray, n, V, nblk, offsets, totals, seg, sig_i, sig_o);
+    FGX_CHECK_LAUNCH("fgx_pair_fill");
+    return FGX_OK;
 }
 
 struct TileLayout {
@@ -477,31 +581,59 @@ TileLayout tile_layout(size_t n, int block) {
     return L;
 }
 
-// rows ranked along the Z-order curve (batch index above 3 * bits interleaved coordinate bits) into ranked[]: a radix sort
-// over the key bits a coordinate of the grid can differ in, on 32-bit keys when they fit
+// Rows ranked along the Z-order curve (batch index above 3 * bits interleaved coordinate bits): a radix sort over the key
+// bits a coordinate of the grid can differ in, on 32-bit keys when they fit.  The ranking goes to wide[] (64-bit) or, when
+// that is null, to *ranked (a buffer of the workspace).
 int zorder_rank(const int32_t* coords, size_t n, int bits_per_axis, int batch_bits, const LocalityLayout& L, char* ws,
-                uint32_t* ranked, uint32_t* other, hipStream_t s, const char* what) {
+                const uint32_t** ranked, int64_t* wide, hipStream_t s, const char* what) {
     const unsigned grid = cdiv(n, kBlock);
     const unsigned end_bit = (unsigned)(3 * bits_per_axis + batch_bits);
+    uint32_t* vals_a = (uint32_t*)(ws + L.vals_a);
+    uint32_t* vals_b = (uint32_t*)(ws + L.vals_b);
     size_t temp_bytes = L.temp_bytes;
     if (end_bit <= 32) {
         uint32_t* keys_a = (uint32_t*)(ws + L.keys_a);
         uint32_t* keys_b = (uint32_t*)(ws + L.keys_b);
-        morton_key_packed_kernel<uint32_t><<<grid, kBlock, 0, s>>>(coords, n, bits_per_axis, keys_a, other);
+        morton_key_packed_kernel<uint32_t><<<grid, kBlock, 0, s>>>(coords, n, bits_per_axis, keys_a, vals_a);
         FGX_CHECK_LAUNCH(what);
-        FGX_CHECK_HIP(rocprim::radix_sort_pairs(ws + L.temp, temp_bytes, keys_a, keys_b, other, ranked, n, 0u, end_bit, s));
+        if (n <= kRsMaxItems)
+            return radix_sort_pairs_u32(keys_a, nullptr, n, end_bit, false, ws + L.radix, radix_layout(n), nullptr, ranked, wide, s, what);
+        FGX_CHECK_HIP(rocprim::radix_sort_pairs(ws + L.temp, temp_bytes, keys_a, keys_b, vals_a, vals_b, n, 0u, end_bit, s));
     } else {
         uint64_t* keys_a = (uint64_t*)(ws + L.keys_a);
         uint64_t* keys_b = (uint64_t*)(ws + L.keys_b);
-        morton_key_packed_kernel<uint64_t><<<grid, kBlock, 0, s>>>(coords, n, bits_per_axis, keys_a, other);
+        morton_key_packed_kernel<uint64_t><<<grid, kBlock, 0, s>>>(coords, n, bits_per_axis, keys_a, vals_a);
         FGX_CHECK_LAUNCH(what);
-        FGX_CHECK_HIP(rocprim::radix_sort_pairs(ws + L.temp, temp_bytes, keys_a, keys_b, other, ranked, n, 0u, end_bit, s));
+        FGX_CHECK_HIP(rocprim::radix_sort_pairs(ws + L.temp, temp_bytes, keys_a, keys_b, vals_a, vals_b, n, 0u, end_bit, s));
+    }
+    *ranked = vals_b;
+    if (wide != nullptr) {
+        widen_u32_i64_kernel<<<grid, kBlock, 0, s>>>(vals_b, wide, n);
+        FGX_CHECK_LAUNCH(what);
     }
     return FGX_OK;
 }
 
-
 }  // namespace
+
+int pair_counts(const int32_t* gray, size_t n, int V, uint32_t* counts, hipStream_t s) {
+    const unsigned nblk = cdiv(n, kPairRows);
+    phase_mark("pair count", s);
+    pair_count_kernel<<<nblk, kPairThreads, 0, s>>>(gray, n, V, nblk, counts);
+    FGX_CHECK_LAUNCH("fgx_pair_count(count)");
+    return FGX_OK;
+}
+
+int pair_lists_from_counts(const uint32_t* map, const int32_t* gray, size_t n, int V, const uint32_t* counts, size_t m, bool sub,
+                           uint32_t* offsets, uint32_t* totals, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, hipStream_t s) {
+    const unsigned nblk = cdiv(n, kPairRows);
+    phase_mark("pair fill", s);
+    if (sub) pair_scan_kernel<kPairRows / kPairSubRows><<<V, 256, 0, s>>>(counts, m, nblk, offsets, totals);
+    else pair_scan_kernel<1><<<V, 256, 0, s>>>(counts, m, nblk, offsets, totals);
+    FGX_CHECK_LAUNCH("fgx_pair_count(scan)");
+    return pair_fill_launch(map, gray, n, V, offsets, totals, seg, sig_i, sig_o, s);
+}
+
 }  // namespace fgx
 
 using namespace fgx;
@@ -509,11 +641,8 @@ using namespace fgx;
 extern "C" {
 
 size_t fgx_sort_workspace_bytes(size_t n) {
-    // (in the radix sort's range a call with a full 32-bit code still takes the library sort: room for either)
-    const size_t lib_sort = sort_layout(n).total;
-    if (n < kOwnSortMin || n > kOwnSortMax) return lib_sort;
-    const size_t own = radix_layout(n).total;
-    return own > lib_sort ? own : lib_sort;
+    if (n <= kRankSortMax) return 256;
+    return n <= kRsMaxItems ? radix_layout(n).total : sort_layout(n).total;
 }
 
 int fgx_sort_by_code(const int32_t* binary, size_t n, int V, int64_t* sorted_idx, void* workspace,
@@ -521,7 +650,6 @@ int fgx_sort_by_code(const int32_t* binary, size_t n, int V, int64_t* sorted_idx
     FGX_CHECK_ARG(V >= 1 && V <= 32, "fgx_sort_by_code: kernel volume must be in [1, 32], got %d", V);
     FGX_CHECK_ARG(n < 0xFFFFFFFFull, "fgx_sort_by_code: too many rows");
     if (n == 0) return FGX_OK;
-    const bool own = n >= kOwnSortMin && n <= kOwnSortMax;
     const size_t need = fgx_sort_workspace_bytes(n);
     FGX_CHECK_ARG(binary && sorted_idx && workspace, "fgx_sort_by_code: null buffer");
     FGX_CHECK_ARG(workspace_bytes >= need, "fgx_sort_by_code: workspace of %zu bytes, need %zu", workspace_bytes, need);
@@ -532,12 +660,14 @@ int fgx_sort_by_code(const int32_t* binary, size_t n, int V, int64_t* sorted_idx
     phase_mark("mask sort", s);
     // With V < 32 every key is non-negative and only bits [0, V) can differ.
     const unsigned end_bit = V < 32 ? (unsigned)V : 32u;
-    if (own && V < 32) {
-        // (as unsigned numbers the keys then order like the int32 codes); the first pass numbers the rows itself and the
-        // last one writes the 64-bit indices
-        return radix_sort_pairs_u32((const uint32_t*)binary, nullptr, n, end_bit, ws, radix_layout(n), nullptr, nullptr, sorted_idx, s,
-                                    "fgx_sort_by_code");
+    if (n <= kRankSortMax) {
+        rank_sort_kernel<<<cdiv(n, 64), 64 * kRankSlices, 0, s>>>((const uint32_t*)binary, (uint32_t)n, V == 32 ? 0x80000000u : 0u, sorted_idx);
+        FGX_CHECK_LAUNCH("fgx_sort_by_code(rank)");
+        return FGX_OK;
     }
+    if (n <= kRsMaxItems)       // the first pass numbers the rows itself and the last one writes the 64-bit indices
+        return radix_sort_pairs_u32((const uint32_t*)binary, nullptr, n, end_bit, true, ws, radix_layout(n), nullptr, nullptr, sorted_idx,
+                                    s, "fgx_sort_by_code");
     const SortLayout L = sort_layout(n);
     int32_t* keys_out = (int32_t*)(ws + L.keys_out);
     uint32_t* vals_in = (uint32_t*)(ws + L.vals_in);
@@ -571,21 +701,17 @@ int fgx_locality_order_grid(const int32_t* coords, const int32_t* binary, size_t
     uint64_t* keys_a = (uint64_t*)(ws + L.keys_a);
     uint64_t* keys_b = (uint64_t*)(ws + L.keys_b);
     uint32_t* vals_a = (uint32_t*)(ws + L.vals_a);
-    uint32_t* vals_b = (uint32_t*)(ws + L.vals_b);
     const unsigned grid = cdiv(n, kBlock);
-    int rc = zorder_rank(coords, n, bits_per_axis, batch_bits, L, ws, vals_b, vals_a, s, "fgx_locality_order(keys)");
-    if (rc != FGX_OK) return rc;
-    if (chunk_rows == 1) {              // chunks of one rank: the curve's own order, nothing to sort inside them
-        widen_u32_i64_kernel<<<grid, kBlock, 0, s>>>(vals_b, order, n);
-        FGX_CHECK_LAUNCH("fgx_locality_order(widen)");
-        return FGX_OK;
-    }
+    const uint32_t* ranked = nullptr;
+    // (chunks of one rank: the curve's own order, nothing to sort inside them)
+    int rc = zorder_rank(coords, n, bits_per_axis, batch_bits, L, ws, &ranked, chunk_rows == 1 ? order : nullptr, s, "fgx_locality_order(keys)");
+    if (rc != FGX_OK || chunk_rows == 1) return rc;
     // (chunk, mask code) keys with the chunk right above the V code bits: the sort runs over the bits in use alone
-    chunk_code_key_kernel<<<grid, kBlock, 0, s>>>(vals_b, binary, n, (uint32_t)chunk_rows, V, keys_a);
+    chunk_code_key_kernel<<<grid, kBlock, 0, s>>>(ranked, binary, n, (uint32_t)chunk_rows, V, keys_a);
     FGX_CHECK_LAUNCH("fgx_locality_order(chunk keys)");
     const unsigned end_bit = (unsigned)V + (unsigned)bits_for((n - 1) / (size_t)chunk_rows);
     size_t temp_bytes = L.temp_bytes;
-    FGX_CHECK_HIP(rocprim::radix_sort_pairs(ws + L.temp, temp_bytes, keys_a, keys_b, vals_b, vals_a, n, 0u, end_bit, s));
+    FGX_CHECK_HIP(rocprim::radix_sort_pairs(ws + L.temp, temp_bytes, keys_a, keys_b, ranked, vals_a, n, 0u, end_bit, s));
     widen_u32_i64_kernel<<<grid, kBlock, 0, s>>>(vals_a, order, n);
     FGX_CHECK_LAUNCH("fgx_locality_order(widen)");
     return FGX_OK;
@@ -610,13 +736,8 @@ int fgx_zorder_rows(const int32_t* coords, size_t n, int bits_per_axis, int batc
     FGX_CHECK_ARG(((uintptr_t)workspace & 255) == 0, "fgx_zorder_rows: workspace must be 256-byte aligned");
     hipStream_t s = (hipStream_t)stream;
     char* ws = (char*)workspace;
-    uint32_t* vals_a = (uint32_t*)(ws + L.vals_a);
-    uint32_t* vals_b = (uint32_t*)(ws + L.vals_b);
-    int rc = zorder_rank(coords, n, bits_per_axis, batch_bits, L, ws, vals_b, vals_a, s, "fgx_zorder_rows(keys)");
-    if (rc != FGX_OK) return rc;
-    widen_u32_i64_kernel<<<cdiv(n, kBlock), kBlock, 0, s>>>(vals_b, order, n);
-    FGX_CHECK_LAUNCH("fgx_zorder_rows(widen)");
-    return FGX_OK;
+    const uint32_t* ranked = nullptr;
+    return zorder_rank(coords, n, bits_per_axis, batch_bits, L, ws, &ranked, order, s, "fgx_zorder_rows(keys)");
 }
 
 size_t fgx_pair_workspace_bytes(size_t n, int V) { return pair_layout(n, V > 0 ? V : 1).total; }
@@ -634,18 +755,17 @@ int fgx_pair_count(const int32_t* gray, size_t n, int V, uint32_t* seg, void* wo
         FGX_CHECK_ARG(((uintptr_t)workspace & 255) == 0, "fgx_pair_count: workspace must be 256-byte aligned");
     }
     char* ws = (char*)workspace;
-    uint32_t* counts = n ? (uint32_t*)(ws + L.counts) : nullptr;
-    uint32_t* offsets = n ? (uint32_t*)(ws + L.offsets) : nullptr;
     PhaseEnd phases{s};
     phase_mark("pair count", s);
+    uint32_t* totals = n ? (uint32_t*)(ws + L.totals) : nullptr;
     if (n > 0) {
-        pair_count_kernel<<<L.nblk, kPairThreads, 0, s>>>(gray, n, V, L.nblk, counts);
-        FGX_CHECK_LAUNCH("fgx_pair_count(count)");
-        size_t temp_bytes = L.temp_bytes;
-        FGX_CHECK_HIP(rocprim::exclusive_scan(ws + L.temp, temp_bytes, counts, offsets, 0u, (size_t)L.nblk * V,
-                                              rocprim::plus<uint32_t>(), s));
+        uint32_t* counts = (uint32_t*)(ws + L.counts);
+        const int rc = pair_counts(gray, n, V, counts, s);
+        if (rc != FGX_OK) return rc;
+        pair_scan_kernel<1><<<V, 256, 0, s>>>(counts, L.nblk, L.nblk, (uint32_t*)(ws + L.offsets), totals);
+        FGX_CHECK_LAUNCH("fgx_pair_count(scan)");
     }
-    pair_seg_kernel<<<1, 64, 0, s>>>(offsets, counts, V, n ? L.nblk : 0u, seg);
+    pair_seg_kernel<<<1, 64, 0, s>>>(totals, V, seg);
     FGX_CHECK_LAUNCH("fgx_pair_count(seg)");
     return FGX_OK;
 }
@@ -655,14 +775,12 @@ int fgx_pair_fill(const uint32_t* map, const int32_t* gray, size_t n, int V, con
     FGX_CHECK_ARG(V >= 1 && V <= 32, "fgx_pair_fill: kernel volume must be in [1, 32], got %d", V);
     if (n == 0) return FGX_OK;
     FGX_CHECK_ARG(map && gray && workspace && sig_i && sig_o, "fgx_pair_fill: null buffer");
-    PairLayout L = pair_layout(n, V);
-    const uint32_t* offsets = (const uint32_t*)((const char*)workspace + L.offsets);
-    size_t lds = ((size_t)kPairThreads * V + 2 * (kPairThreads / 64) * 32 + 32) * sizeof(uint32_t);
+    const PairLayout L = pair_layout(n, V);
+    const char* ws = (const char*)workspace;
     PhaseEnd phases{(hipStream_t)stream};
     phase_mark("pair fill", (hipStream_t)stream);
-    pair_fill_kernel<<<L.nblk, kPairThreads, lds, (hipStream_t)stream>>>(map, gray, n, V, L.nblk, offsets, sig_i, sig_o);
-    FGX_CHECK_LAUNCH("fgx_pair_fill");
-    return FGX_OK;
+    return pair_fill_launch(map, gray, n, V, (const uint32_t*)(ws + L.offsets), (const uint32_t*)(ws + L.totals), nullptr, sig_i, sig_o,
+                            (hipStream_t)stream);
 }
 
 size_t fgx_tile_workspace_bytes(size_t n, int block) { return tile_layout(n, block > 0 ? block : 1).total; }

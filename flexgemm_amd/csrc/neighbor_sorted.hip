@@ -400,7 +400,7 @@ int build_sorted(const int32_t* coords, size_t n, uint64_t vol, const SubmGeom& 
         FGX_CHECK_LAUNCH("fgx_subm_neighbor_map_sorted(keys)");
         phase_mark("key sort", s);
         const uint32_t *ks = nullptr, *vs = nullptr;
-        int rc = radix_sort_pairs_u32((const uint32_t*)keys_in, nullptr, n, end_bit, ws + L.radix, radix_layout(n), &ks, &vs, nullptr,
+        int rc = radix_sort_pairs_u32((const uint32_t*)keys_in, nullptr, n, end_bit, false, ws + L.radix, radix_layout(n), &ks, &vs, nullptr,
                                       s, "fgx_subm_neighbor_map_sorted(key sort)", flag);
         if (rc != FGX_OK) return rc;
         skeys = (const K*)ks;
