@@ -46,6 +46,10 @@ EXPORTS = [
     "fgx_spconv_neighbor_map_sorted_workspace_bytes", "fgx_spconv_neighbor_map_sorted",
     "fgx_serialize_encode", "fgx_serialize_decode", "fgx_serialize_reorder_workspace_bytes",
     "fgx_serialize_reorder_coords",
+    "fgx_grid_index_pays", "fgx_subm_neighbor_map_grid_workspace_bytes", "fgx_subm_neighbor_map_grid", "fgx_subm_cache_grid_workspace_bytes",
+    "fgx_subm_cache_build_grid", "fgx_spconv_neighbor_map_grid_workspace_bytes", "fgx_spconv_neighbor_map_grid",
+    "fgx_spconv_cache_grid_workspace_bytes", "fgx_spconv_cache_build_grid", "fgx_spconv_out_coords_grid_workspace_bytes",
+    "fgx_spconv_out_coords_grid_count", "fgx_spconv_out_coords_grid_emit",
 ]
 
 
@@ -104,7 +108,10 @@ def lib() -> C.CDLL:
                      "fgx_colsum_scratch_bytes", "fgx_spconv_out_coords_workspace_bytes",
                      "fgx_subm_neighbor_map_sorted_workspace_bytes", "fgx_wgrad_block_bounds_count", "fgx_wgrad_item_lists_count", "fgx_narrow_plan_bytes", "fgx_narrow_wgrad_scratch_bytes",
                      "fgx_spconv_neighbor_map_sorted_workspace_bytes", "fgx_serialize_reorder_workspace_bytes",
-                     "fgx_gather_item_order_workspace_bytes", "fgx_subm_cache_workspace_bytes", "fgx_wgrad_sweep_plan_bytes", "fgx_wgrad_sweep_scratch_bytes", "fgx_wgrad_sweep_giveup_words"):
+                     "fgx_gather_item_order_workspace_bytes", "fgx_subm_cache_workspace_bytes", "fgx_wgrad_sweep_plan_bytes", "fgx_wgrad_sweep_scratch_bytes", "fgx_wgrad_sweep_giveup_words",
+                     "fgx_subm_neighbor_map_grid_workspace_bytes", "fgx_subm_cache_grid_workspace_bytes",
+                     "fgx_spconv_neighbor_map_grid_workspace_bytes", "fgx_spconv_cache_grid_workspace_bytes",
+                     "fgx_spconv_out_coords_grid_workspace_bytes"):
             getattr(L, name).restype = C.c_size_t
         _lib = L
     return _lib

@@ -40,10 +40,12 @@ OUT_COORD_ALGO = SparseConv3dOutCoordAlgorithm.HASHMAP
 SERIALIZATION_MODE = SerializationMode.BXYZ
 
 
-# How the submanifold neighbor map is found (no counterpart in the reference, which always hashes; the map is the same
-# either way): "hash" = open-addressing table and probes, "sort" = radix sort of the flattened keys and windowed merges,
-# "auto" = "sort" once the searches outweigh the two sorts: from SORT_BUILDER_MIN_PROBES (voxel, kernel position)
-# questions on (131 072 voxels of a 3x3x3 kernel).
+# How the neighbor maps are found (no counterpart in the reference, which always hashes; the maps are the same either
+# way): "grid" = an index over the grid's cells (one word or one bit per cell), "hash" = open-addressing table and probes,
+# "sort" = radix sort of the flattened keys and windowed merges, "auto" = "grid" where the index is worth clearing
+# (fgx_grid_index_pays: the grid's bits are at most 16 MiB or 64 bytes per voxel), else "sort" once the searches outweigh
+# the two sorts: from SORT_BUILDER_MIN_PROBES (voxel, kernel position) questions on (131 072 voxels of a 3x3x3 kernel),
+# else "hash".  "grid" on a grid too large for it (512 MiB of bits) means what "auto" would take there.
 NEIGHBOR_MAP_BUILDER = "auto"
 SORT_BUILDER_MIN_PROBES = 27 * 131072
 # How the streaming GEMM's tiles are dealt to its persistent workgroups: "balanced" (by cost, every round of tiles dealt
@@ -86,8 +88,8 @@ def set_weight_panel_cache(enabled: bool, max_bytes: int = None):
 
 def set_neighbor_map_builder(builder: str):
     global NEIGHBOR_MAP_BUILDER
-    if builder not in ("auto", "hash", "sort"):
-        raise ValueError(f"unknown neighbor map builder {builder!r}; expected 'auto', 'hash' or 'sort'")
+    if builder not in ("auto", "grid", "hash", "sort"):
+        raise ValueError(f"unknown neighbor map builder {builder!r}; expected 'auto', 'grid', 'hash' or 'sort'")
     NEIGHBOR_MAP_BUILDER = builder
 
 

@@ -21,7 +21,7 @@ from .. import serialize
 from . import Algorithm, SerializationMode, SparseConv3dOutCoordAlgorithm
 from .submanifold_conv3d import (EMPTY, _IMPLICIT, _MASKED, _NO_SPLITK, SubMConv3dNeighborCache, _codes_and_order, _colsum,
                                  _gather_gemm, _gathered_rows, _grad_mode_of_the_caller, _gradients_possible, _pair_lists,
-                                 _relu_mask_apply, _require_cuda, _wgrad)
+                                 _pick_builder, _relu_mask_apply, _require_cuda, _wgrad, PAIR_LISTS_UNSIZED_MAX_BYTES)
 
 
 def _triple(x) -> Tuple[int, int, int]:
@@ -80,6 +80,58 @@ class SparseConv3dNeighborCache(SubMConv3dNeighborCache):
         return self[f"valid_kernel_bwd_seg_{block_size}"]
 
 
+def _maps_builder(m: int, l: int, v: int, shape, ks, st, pd, dl, with_bwd: bool) -> str:
+    """The builder of both maps: the grid index wants grids it fits (the output's too where the backward map is looked up
+    in it)."""
+    B, _, W, H, D = [int(s) for s in shape]
+    out_dims = _out_dims(shape, ks, st, pd, dl)
+    if (l > 0 and min(out_dims) > 0 and _pick_builder(m, v, B, (W, H, D)) == "grid"
+            and (not with_bwd or _pick_builder(l, v, B, out_dims) == "grid")):
+        return "grid"
+    if spconv.NEIGHBOR_MAP_BUILDER in ("hash", "sort"):
+        return spconv.NEIGHBOR_MAP_BUILDER
+    # (the sorted builder sorts the queries as well, with wider keys: it needs more questions to pay off)
+    return "sort" if l * v >= 4 * spconv.SORT_BUILDER_MIN_PROBES else "hash"
+
+
+def _build_cache_one_call(coords: torch.Tensor, out_coords: torch.Tensor, shape, ks, st, pd, dl, needs_grad: bool, bwd_order: bool):
+    """The masked algorithms' tables through fgx_spconv_cache_build_grid, every buffer allocated beforehand: a dict of them,
+    or None where the step-by-step path runs (no grid index, nothing to convolve, pair lists too large for their bound)."""
+    m, l = coords.shape[0], out_coords.shape[0]
+    v = ks[0] * ks[1] * ks[2]
+    if m == 0 or l == 0 or l * v >= 0xFFFFFFFF or (needs_grad and l * v * 8 > PAIR_LISTS_UNSIZED_MAX_BYTES):
+        return None
+    if _maps_builder(m, l, v, shape, ks, st, pd, dl, needs_grad) != "grid":
+        return None
+    B, _, W, H, D = [int(s) for s in shape]
+    dims = [C.c_int(x) for x in (B, W, H, D)]
+    out_dims = [C.c_int(x) for x in _out_dims(shape, ks, st, pd, dl)]
+    dev = coords.device
+    with torch.cuda.device(dev):
+        L = nat.lib()
+        t = {"nmap": torch.empty((l, v), dtype=torch.uint32, device=dev), "gray": torch.empty((l,), dtype=torch.int32, device=dev),
+             "binary": torch.empty((l,), dtype=torch.int32, device=dev), "order": torch.empty((l,), dtype=torch.int64, device=dev)}
+        if needs_grad:
+            t.update(nmap_bwd=torch.empty((m, v), dtype=torch.uint32, device=dev), seg=torch.empty((v + 1,), dtype=torch.uint32, device=dev),
+                     sig_i=torch.empty((l * v,), dtype=torch.uint32, device=dev), sig_o=torch.empty((l * v,), dtype=torch.uint32, device=dev))
+            if bwd_order:
+                t.update(gray_bwd=torch.empty((m,), dtype=torch.int32, device=dev), order_bwd=torch.empty((m,), dtype=torch.int64, device=dev))
+        ws = nat.workspace(L.fgx_spconv_cache_grid_workspace_bytes(nat.sz(m), nat.sz(l), *dims, *out_dims, C.c_int(v), C.c_int(int(needs_grad)),
+                                                                   C.c_int(int("order_bwd" in t))), dev)
+        nat.check(L.fgx_spconv_cache_build_grid(
+            nat.ptr(coords), nat.sz(m), nat.ptr(out_coords), nat.sz(l), *dims, *[C.c_int(x) for x in (*ks, *st, *pd, *dl)],
+            nat.ptr(ws), nat.sz(ws.numel()),
+            *[nat.ptr(t.get(k)) for k in ("nmap", "gray", "binary", "order", "nmap_bwd", "seg", "sig_i", "sig_o", "gray_bwd", "order_bwd")],
+            nat.stream()))
+        if needs_grad:
+            seg_pinned = torch.empty((v + 1,), dtype=torch.int32, pin_memory=True)
+            seg_pinned.copy_(t["seg"].view(torch.int32), non_blocking=True)
+            arrived = torch.cuda.Event()
+            arrived.record()
+            t["pairs"] = {"seg": t["seg"], "pending": (t["sig_i"], t["sig_o"], seg_pinned, arrived)}
+    return t
+
+
 def _build_maps(coords: torch.Tensor, out_coords: torch.Tensor, shape, kernel_size, stride, padding, dilation,
                 with_bwd: bool, with_codes: bool, hashmap_ratio: Optional[float] = None):
     """(map_fwd [L, V], map_bwd [M, V] | None, gray | None, binary | None), by hash probes or by sort and merge.
@@ -97,13 +149,20 @@ def _build_maps(coords: torch.Tensor, out_coords: torch.Tensor, shape, kernel_si
         gray = torch.empty((l,), dtype=torch.int32, device=dev)
         binary = torch.empty((l,), dtype=torch.int32, device=dev)
     B = int(shape[0])
-    builder = spconv.NEIGHBOR_MAP_BUILDER
-    if builder == "auto":
-        # (the generic builder sorts the queries as well, with wider keys: it needs more questions to pay off)
-        builder = "sort" if l * v >= 4 * spconv.SORT_BUILDER_MIN_PROBES else "hash"
+    builder = _maps_builder(m, l, v, shape, kernel_size, stride, padding, dilation, with_bwd)
     vol = B * W * H * D
     geom = [C.c_int(x) for x in (kw, kh, kd, stride[0], stride[1], stride[2], padding[0], padding[1], padding[2],
                                  dilation[0], dilation[1], dilation[2])]
+    if builder == "grid":
+        dims = [C.c_int(x) for x in (B, W, H, D)]
+        out_dims = [C.c_int(x) for x in _out_dims(shape, kernel_size, stride, padding, dilation)]
+        with torch.cuda.device(dev):
+            L = nat.lib()
+            ws = nat.workspace(L.fgx_spconv_neighbor_map_grid_workspace_bytes(nat.sz(m), nat.sz(l), *dims, *out_dims, C.c_int(1 if with_bwd else 0)), dev)
+            nat.check(L.fgx_spconv_neighbor_map_grid(
+                nat.ptr(coords), nat.sz(m), nat.ptr(out_coords), nat.sz(l), *dims, *geom, nat.ptr(ws), nat.sz(ws.numel()), nat.ptr(nmap),
+                nat.ptr(nmap_bwd), nat.ptr(gray), nat.ptr(binary), nat.stream()))
+        return nmap, nmap_bwd, gray, binary
     if builder == "sort" and kw * kh <= 128 and vol <= 2 ** 62:
         key_bits = 32 if vol <= 2 ** 32 else 64
         with torch.cuda.device(dev):
@@ -173,8 +232,20 @@ class SparseConv3dFunction(Function):
         vol = B * wo * ho * do
         if vol >= 2 ** 64 - 1:
             raise ValueError("The spatial size is too large. Require B*W*H*D < 2^64.")
-        key_bits = 32 if vol < 2 ** 32 - 1 else 64
         L = nat.lib()
+        geom = [C.c_int(x) for x in (B, W, H, D, *ks, *st, *pd, *dl)]
+        if m * v < 1 << 30 and spconv.NEIGHBOR_MAP_BUILDER in ("auto", "grid") and L.fgx_grid_index_pays(nat.sz(m), *[C.c_int(x) for x in (B, wo, ho, do)]):
+            out_dims = [C.c_int(x) for x in (B, wo, ho, do)]
+            with torch.cuda.device(dev):
+                ws = nat.workspace(L.fgx_spconv_out_coords_grid_workspace_bytes(*out_dims), dev)
+                count = torch.empty((1,), dtype=torch.int64, device=dev)
+                nat.check(L.fgx_spconv_out_coords_grid_count(nat.ptr(coords), nat.sz(m), *geom, nat.ptr(ws), nat.sz(ws.numel()), nat.ptr(count),
+                                                             nat.stream()))
+                total = int(count.item())      # the one host sync: sizes the result
+                out = torch.empty((total, 4), dtype=torch.int32, device=dev)
+                nat.check(L.fgx_spconv_out_coords_grid_emit(nat.ptr(ws), *out_dims, nat.sz(total), nat.ptr(out), nat.stream()))
+            return SparseConv3dFunction._serialized(out, mode, (B, W, H, D), (wo, ho, do))
+        key_bits = 32 if vol < 2 ** 32 - 1 else 64
         with torch.cuda.device(dev):
             ws = nat.workspace(L.fgx_spconv_out_coords_workspace_bytes(nat.sz(m), C.c_int(v), C.c_int(key_bits)), dev)
             count = torch.empty((1,), dtype=torch.int64, device=dev)
@@ -187,12 +258,17 @@ class SparseConv3dFunction(Function):
             out = torch.empty((total, 4), dtype=torch.int32, device=dev)
             nat.check(L.fgx_spconv_out_coords_decode(nat.ptr(ws), C.c_int(key_bits), nat.sz(total), C.c_int(wo), C.c_int(ho),
                                                      C.c_int(do), nat.ptr(out), nat.stream()))
-        if mode != SerializationMode.BXYZ:
-            bit_length = (max(W, H, D) - 1).bit_length()
-            if max(wo, ho, do) > (1 << bit_length):
-                raise ValueError("output grid exceeds the bits per axis of the input grid: curve codes would collide")
-            out = serialize.reorder_coords(out, bit_length, (B - 1).bit_length(), int(mode))
-        return out
+        return SparseConv3dFunction._serialized(out, mode, (B, W, H, D), (wo, ho, do))
+
+    @staticmethod
+    def _serialized(out: torch.Tensor, mode: int, grid, out_dims) -> torch.Tensor:
+        """Output coordinates in (b, x, y, z) order, re-sorted along the curve of `mode` (bits per axis: the input grid's)."""
+        if mode == SerializationMode.BXYZ:
+            return out
+        bit_length = (max(grid[1:]) - 1).bit_length()
+        if max(out_dims) > (1 << bit_length):
+            raise ValueError("output grid exceeds the bits per axis of the input grid: curve codes would collide")
+        return serialize.reorder_coords(out, bit_length, (grid[0] - 1).bit_length(), int(mode))
 
     @staticmethod
     def _get_output_coords_torch(
@@ -249,13 +325,23 @@ class SparseConv3dFunction(Function):
             nmap, nmap_bwd, _, _ = _build_maps(coords, out_coords, shape, ks, st, pd, dl, needs_grad, with_codes=False)
             return SparseConv3dNeighborCache(neighbor_map=nmap, neighbor_map_bwd=nmap_bwd, _n_in=coords.shape[0])
         assert v <= 32, "Currently, the max kernel volume is 32 because kernel mask is encoded as uint32"
+        irregular = any(s != 1 for s in st) or is_out_coords_given
+        t = _build_cache_one_call(coords, out_coords, shape, ks, st, pd, dl, needs_grad, irregular)
+        if t is not None:
+            cache = SparseConv3dNeighborCache(neighbor_map=t["nmap"], neighbor_map_bwd=t.get("nmap_bwd"), gray_code=t["gray"],
+                                              sorted_idx=t["order"], _n_in=coords.shape[0])
+            if needs_grad:
+                cache._attach_pairs(t["pairs"])
+                if irregular:
+                    cache["gray_code_bwd"], cache["sorted_idx_bwd"] = t["gray_bwd"], t["order_bwd"]
+            return cache
         nmap, nmap_bwd, gray, binary = _build_maps(coords, out_coords, shape, ks, st, pd, dl, needs_grad, with_codes=True)
         gray, binary, order = _codes_and_order(nmap, gray, binary)
         cache = SparseConv3dNeighborCache(neighbor_map=nmap, neighbor_map_bwd=nmap_bwd, gray_code=gray, sorted_idx=order,
                                           _n_in=coords.shape[0])
         if needs_grad:
             cache._attach_pairs(_pair_lists(nmap, gray))
-            if any(s != 1 for s in st) or is_out_coords_given:
+            if irregular:
                 # irregular backward masks: sort the input rows by theirs, as the reference does (:191-207); otherwise
                 # nearly every input reaches every kernel position and the input gradient runs unsorted
                 gray_b, _, order_b = _codes_and_order(nmap_bwd, None, None)

@@ -460,6 +460,21 @@ def _side_stream(dev: torch.device) -> torch.cuda.Stream:
     return _side_streams[key]
 
 
+GRID_BUILDER_MAX_VOLUME = 128            # kernel positions fgx_subm_neighbor_map_grid takes
+
+
+def _pick_builder(n: int, v: int, batch: int, dims) -> str:
+    """The builder NEIGHBOR_MAP_BUILDER stands for, for n rows asking v questions each on a batch x dims grid."""
+    builder = spconv.NEIGHBOR_MAP_BUILDER
+    if builder in ("auto", "grid") and n > 0 and v <= GRID_BUILDER_MAX_VOLUME:
+        L, args = nat.lib(), (nat.sz(n), C.c_int(batch), C.c_int(dims[0]), C.c_int(dims[1]), C.c_int(dims[2]))
+        if L.fgx_grid_index_pays(*args) or (builder == "grid" and L.fgx_subm_neighbor_map_grid_workspace_bytes(*args)):
+            return "grid"
+    if builder in ("auto", "grid"):
+        builder = "sort" if n * v >= spconv.SORT_BUILDER_MIN_PROBES else "hash"
+    return builder
+
+
 def _build_neighbor_map(coords: torch.Tensor, shape, kernel_size, dilation, with_codes: bool):
     n = coords.shape[0]
     B, _, W, H, D = [int(s) for s in shape]
@@ -471,10 +486,17 @@ def _build_neighbor_map(coords: torch.Tensor, shape, kernel_size, dilation, with
     if with_codes:
         gray = torch.empty((n,), dtype=torch.int32, device=dev)
         binary = torch.empty((n,), dtype=torch.int32, device=dev)
-    builder = spconv.NEIGHBOR_MAP_BUILDER
-    if builder == "auto":
-        builder = "sort" if n * v >= spconv.SORT_BUILDER_MIN_PROBES else "hash"
+    builder = _pick_builder(n, v, B, (W, H, D))
     vol = B * W * H * D
+    if builder == "grid":
+        with torch.cuda.device(dev):
+            L = nat.lib()
+            ws = nat.workspace(L.fgx_subm_neighbor_map_grid_workspace_bytes(nat.sz(n), C.c_int(B), C.c_int(W), C.c_int(H), C.c_int(D)), dev)
+            nat.check(L.fgx_subm_neighbor_map_grid(
+                nat.ptr(coords), nat.sz(n), C.c_int(B), C.c_int(W), C.c_int(H), C.c_int(D), C.c_int(kw), C.c_int(kh), C.c_int(kd),
+                C.c_int(int(dilation[0])), C.c_int(int(dilation[1])), C.c_int(int(dilation[2])), nat.ptr(ws), nat.sz(ws.numel()),
+                nat.ptr(nmap), nat.ptr(gray), nat.ptr(binary), nat.stream()))
+        return nmap, gray, binary
     if builder == "sort" and kw * kh <= 128 and vol <= 2 ** 63:
         key_bits = 32 if vol <= 2 ** 32 else 64
         with torch.cuda.device(dev):
@@ -508,7 +530,7 @@ def _build_neighbor_map(coords: torch.Tensor, shape, kernel_size, dilation, with
 
 
 def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, needs_grad: bool):
-    """The masked algorithms' neighbor cache through fgx_subm_cache_build: map, codes, mask sort and (needs_grad) the pair
+    """The masked algorithms' neighbor cache through fgx_subm_cache_build_grid or fgx_subm_cache_build: map, codes, mask sort and (needs_grad) the pair
     lists enqueued by one library call, with every buffer allocated beforehand -- the GPU does not wait for the host
     between the steps.  Returns (nmap, gray, binary, order, pairs or None), or None where the call does not apply (the
     hash builder's range, kernels beyond what the sorted builder takes, pair lists too large to allocate at their bound)
@@ -517,24 +539,18 @@ def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, ne
     B, _, W, H, D = [int(s) for s in shape]
     kw, kh, kd = [int(k) for k in kernel_size]
     v = kw * kh * kd
-    builder = spconv.NEIGHBOR_MAP_BUILDER
-    if builder == "auto":
-        builder = "sort" if n * v >= spconv.SORT_BUILDER_MIN_PROBES else "hash"
+    builder = _pick_builder(n, v, B, (W, H, D))
     vol = B * W * H * D
     bound = n * v
-    if builder != "sort" or n == 0 or v > 32 or kw * kh > 128 or vol > 2 ** 63 or bound >= 0xFFFFFFFF:
+    if builder not in ("grid", "sort") or n == 0 or v > 32 or kw * kh > 128 or vol > 2 ** 63 or bound >= 0xFFFFFFFF:
         return None
     if needs_grad and bound * 8 > PAIR_LISTS_UNSIZED_MAX_BYTES:
         return None
-    key_bits = 32 if vol <= 2 ** 32 else 64
     dev = coords.device
+    geom = [C.c_int(int(x)) for x in (B, W, H, D, kw, kh, kd, dilation[0], dilation[1], dilation[2])]
+    with_pairs = C.c_int(1 if needs_grad else 0)
     with torch.cuda.device(dev):
         L = nat.lib()
-        presorted = 2                       # (as in _build_neighbor_map)
-        if n > SORT_DECIDED_ON_DEVICE_MAX or key_bits != 32:
-            descents = torch.zeros((1,), dtype=torch.int32, device=dev)
-            nat.check(L.fgx_coords_key_order(nat.ptr(coords), nat.sz(n), C.c_int(W), C.c_int(H), C.c_int(D), nat.ptr(descents), nat.stream()))
-            presorted = 1 if int(descents.item()) == 0 else 0
         nmap = torch.empty((n, v), dtype=torch.uint32, device=dev)
         gray = torch.empty((n,), dtype=torch.int32, device=dev)
         binary = torch.empty((n,), dtype=torch.int32, device=dev)
@@ -544,13 +560,22 @@ def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, ne
             seg = torch.empty((v + 1,), dtype=torch.uint32, device=dev)
             buf_i = torch.empty((bound,), dtype=torch.uint32, device=dev)
             buf_o = torch.empty((bound,), dtype=torch.uint32, device=dev)
-        ws = nat.workspace(L.fgx_subm_cache_workspace_bytes(nat.sz(n), C.c_int(key_bits), C.c_int(kw), C.c_int(kh), C.c_int(kd),
-                                                            C.c_int(1 if needs_grad else 0)), dev)
-        nat.check(L.fgx_subm_cache_build(
-            nat.ptr(coords), nat.sz(n), C.c_int(B), C.c_int(W), C.c_int(H), C.c_int(D), C.c_int(kw), C.c_int(kh), C.c_int(kd),
-            C.c_int(int(dilation[0])), C.c_int(int(dilation[1])), C.c_int(int(dilation[2])), C.c_int(key_bits), C.c_int(presorted),
-            C.c_int(1 if needs_grad else 0), nat.ptr(ws), nat.sz(ws.numel()), nat.ptr(nmap), nat.ptr(gray), nat.ptr(binary),
-            nat.ptr(order), nat.ptr(seg), nat.ptr(buf_i), nat.ptr(buf_o), nat.stream()))
+        outs = [nat.ptr(t) for t in (nmap, gray, binary, order, seg, buf_i, buf_o)]
+        if builder == "grid":
+            ws = nat.workspace(L.fgx_subm_cache_grid_workspace_bytes(nat.sz(n), *geom[:4], C.c_int(v), with_pairs), dev)
+            nat.check(L.fgx_subm_cache_build_grid(nat.ptr(coords), nat.sz(n), *geom, with_pairs, nat.ptr(ws), nat.sz(ws.numel()), *outs,
+                                                  nat.stream()))
+        else:
+            key_bits = 32 if vol <= 2 ** 32 else 64
+            presorted = 2                   # (as in _build_neighbor_map)
+            if n > SORT_DECIDED_ON_DEVICE_MAX or key_bits != 32:
+                descents = torch.zeros((1,), dtype=torch.int32, device=dev)
+                nat.check(L.fgx_coords_key_order(nat.ptr(coords), nat.sz(n), C.c_int(W), C.c_int(H), C.c_int(D), nat.ptr(descents), nat.stream()))
+                presorted = 1 if int(descents.item()) == 0 else 0
+            ws = nat.workspace(L.fgx_subm_cache_workspace_bytes(nat.sz(n), C.c_int(key_bits), C.c_int(kw), C.c_int(kh), C.c_int(kd),
+                                                                with_pairs), dev)
+            nat.check(L.fgx_subm_cache_build(nat.ptr(coords), nat.sz(n), *geom, C.c_int(key_bits), C.c_int(presorted), with_pairs,
+                                             nat.ptr(ws), nat.sz(ws.numel()), *outs, nat.stream()))
         pairs = None
         if needs_grad:
             # the lists' length travels to pinned host memory behind an event; the cache cuts them to it when first asked

@@ -182,6 +182,23 @@ int fgx_subm_cache_build(const int32_t* coords, size_t n, int B, int W, int H, i
                          int32_t* gray, int32_t* binary, int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o,
                          fgx_stream_t stream);
 
+/* The submanifold map and the whole cache through an index over the grid's cells (a word per cell, or a bit per cell with
+ * running counts) instead of a hash table or a sort: same results, voxels given several times found under their smallest
+ * row.  fgx_grid_index_pays: 1 where the index fits and its clears are worth it for n voxels on this grid (the host's
+ * "auto" rule).  Workspace functions return 0 for a grid too large (512 MiB of bits); workspaces are 256-byte aligned.
+ * The map: kernel volumes up to 128, mask codes (gray / binary, both or neither) up to 32.  The cache: as
+ * fgx_subm_cache_build, without the sort's key_bits and presorted.
+ * Replaces: hashmap_build_submanifold_conv_neighbour_map and the same sequence of calls as fgx_subm_cache_build. */
+int fgx_grid_index_pays(size_t n, int B, int W, int H, int D);
+size_t fgx_subm_neighbor_map_grid_workspace_bytes(size_t n, int B, int W, int H, int D);
+int fgx_subm_neighbor_map_grid(const int32_t* coords, size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dw, int Dh,
+                               int Dd, void* workspace, size_t workspace_bytes, uint32_t* out_map, int32_t* gray, int32_t* binary,
+                               fgx_stream_t stream);
+size_t fgx_subm_cache_grid_workspace_bytes(size_t n, int B, int W, int H, int D, int V, int with_pairs);
+int fgx_subm_cache_build_grid(const int32_t* coords, size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dw, int Dh, int Dd,
+                              int with_pairs, void* workspace, size_t workspace_bytes, uint32_t* out_map, int32_t* gray, int32_t* binary,
+                              int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, fgx_stream_t stream);
+
 /* Per row-tile (block consecutive rows of the sorted order) OR of the masks.
  *   codes: tile_code[nb] <- OR mask, seg[nb+1] <- exclusive offsets of popcounts (seg[nb] = total);
  *   fill : valid_kernel[total] <- set-bit positions, ascending per tile.
@@ -524,6 +541,31 @@ int fgx_spconv_neighbor_map_sorted(const int32_t* in_coords, size_t n_in, const 
                                    int Pw, int Ph, int Pd, int Dw, int Dh, int Dd, int key_bits,
                                    void* workspace, size_t workspace_bytes, uint32_t* map_fwd, uint32_t* map_bwd,
                                    int32_t* gray, int32_t* binary, fgx_stream_t stream);
+
+/* The maps, and with the mask sort and the pair lists the whole cache, through an index over the cells of both grids (see
+ * fgx_subm_neighbor_map_grid).  map_bwd NULL: no backward map, and then no pair lists; gray_bwd / sorted_idx_bwd (both or
+ * neither): mask codes and mask order of the backward map's rows.  Output coordinates (fgx_spconv_out_coords_keys and
+ * _decode's list) as the set bits of a bit map over the output grid: _count leaves the bits in `workspace` and their number
+ * in `count` (DEVICE memory), _emit writes the coordinates.  Workspace functions return 0 for a grid too large.
+ * Replaces: the same reference functions as fgx_spconv_neighbor_map and fgx_spconv_out_coords_keys. */
+size_t fgx_spconv_neighbor_map_grid_workspace_bytes(size_t n_in, size_t n_out, int B, int W, int H, int D, int Wo, int Ho, int Do, int with_bwd);
+int fgx_spconv_neighbor_map_grid(const int32_t* in_coords, size_t n_in, const int32_t* out_coords, size_t n_out, int B, int W, int H, int D,
+                                 int Kw, int Kh, int Kd, int Sw, int Sh, int Sd, int Pw, int Ph, int Pd, int Dw, int Dh, int Dd,
+                                 void* workspace, size_t workspace_bytes, uint32_t* map_fwd, uint32_t* map_bwd, int32_t* gray,
+                                 int32_t* binary, fgx_stream_t stream);
+size_t fgx_spconv_cache_grid_workspace_bytes(size_t n_in, size_t n_out, int B, int W, int H, int D, int Wo, int Ho, int Do, int V,
+                                             int with_bwd, int with_bwd_order);
+int fgx_spconv_cache_build_grid(const int32_t* in_coords, size_t n_in, const int32_t* out_coords, size_t n_out, int B, int W, int H, int D,
+                                int Kw, int Kh, int Kd, int Sw, int Sh, int Sd, int Pw, int Ph, int Pd, int Dw, int Dh, int Dd,
+                                void* workspace, size_t workspace_bytes, uint32_t* map_fwd, int32_t* gray, int32_t* binary,
+                                int64_t* sorted_idx, uint32_t* map_bwd, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, int32_t* gray_bwd,
+                                int64_t* sorted_idx_bwd, fgx_stream_t stream);
+size_t fgx_spconv_out_coords_grid_workspace_bytes(int B, int Wo, int Ho, int Do);
+int fgx_spconv_out_coords_grid_count(const int32_t* coords, size_t n_in, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Sw, int Sh,
+                                     int Sd, int Pw, int Ph, int Pd, int Dw, int Dh, int Dd, void* workspace, size_t workspace_bytes,
+                                     uint64_t* count, fgx_stream_t stream);
+int fgx_spconv_out_coords_grid_emit(const void* workspace, int B, int Wo, int Ho, int Do, size_t count, int32_t* out_coords,
+                                    fgx_stream_t stream);
 
 /* ---- Space-filling-curve codes of voxel coordinates -----------------------------------------------------------
  * mode: 1 = z-order (Morton), 2 = Hilbert (the values of SerializationMode, flex_gemm/ops/spconv/__init__.py:20-24).

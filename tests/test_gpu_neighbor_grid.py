@@ -1,0 +1,118 @@
+"""Neighbor caches through the index over the grid's cells, and the sorts of the cache, against the CPU oracle (bit-exact)."""
+import ctypes as C
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+import flex_gemm
+from flex_gemm.ops.spconv import SparseConv3dFunction, SubMConv3dFunction
+from flexgemm_amd import _native as nat
+from flexgemm_amd.workloads import reference_test_shell
+from oracle import neighbor as nb
+from oracle import sparse_conv as sc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def grid_builder():
+    flex_gemm.ops.spconv.set_neighbor_map_builder("grid")
+    yield
+    flex_gemm.ops.spconv.set_neighbor_map_builder("auto")
+
+
+def _say(msg):
+    print(f"[case] {msg}", flush=True)
+    sys.stdout.flush()
+
+
+def _np(t):
+    return t.cpu().view(torch.int32).numpy().view(np.uint32) if t.dtype == torch.uint32 else t.cpu().numpy()
+
+
+def _voxels(dims, n, seed, order):
+    """n distinct voxels of a (B, W, H, D) grid, clustered so that most have neighbors, in scan or random order."""
+    rng = np.random.default_rng(seed)
+    cells = np.unique(rng.integers(0, max(int(np.prod(dims)) // 40, 1), 2 * n) + int(np.prod(dims)) // 2)[:n]
+    coords = np.stack(np.unravel_index(cells % int(np.prod(dims)), dims), 1).astype(np.int32)
+    coords = np.unique(coords, axis=0)
+    return coords if order == "scan" else coords[rng.permutation(len(coords))]
+
+
+# both forms of the index: a word per cell up to 2^23 cells, a bit per cell beyond (203^3 and 204^3 lie on either side);
+# long rows, cells that are no multiple of 128, fewer rows than a workgroup takes and one more than it takes
+@pytest.mark.parametrize("dims,n", [((1, 203, 203, 203), 5000), ((1, 204, 204, 204), 5000), ((3, 5, 7, 90001), 4097), ((2, 1, 3, 2000003), 65),
+                                    ((1, 300, 300, 300), 1), ((4, 11, 9, 13), 64)])
+@pytest.mark.parametrize("order", ["scan", "shuffled"])
+@pytest.mark.parametrize("dil", [(1, 1, 1), (2, 1, 3)])
+def test_subm_cache(gpu_device, dims, n, order, dil):
+    _say(f"grid cache dims={dims} n={n} {order} dilation={dil}")
+    coords = _voxels(dims, n, 7, order)
+    shape = torch.Size([dims[0], 0, *dims[1:]])
+    cache = SubMConv3dFunction._compute_neighbor_cache(torch.from_numpy(coords).to(gpu_device), shape, (3, 3, 3), dil, True)
+    ref = nb.neighbor_cache(coords, tuple(shape), (3, 3, 3), dil, needs_grad=True, blocks=(64,))
+    for field in ("neighbor_map", "gray_code", "sorted_idx", "valid_signal_seg", "valid_signal_i", "valid_signal_o"):
+        assert np.array_equal(_np(getattr(cache, field)), ref[field]), field
+
+
+@pytest.mark.parametrize("res", [32, 210])
+def test_subm_repeated_voxels_are_found_under_their_smallest_row(gpu_device, res):
+    _say(f"grid map with repeated voxels res={res}")
+    rng = np.random.default_rng(res)
+    base = reference_test_shell(32)
+    coords = np.concatenate([base, base[rng.choice(len(base), 300, replace=False)], base[:7], base[:7]])[rng.permutation(len(base) + 314)]
+    cache = SubMConv3dFunction._compute_neighbor_cache(torch.from_numpy(coords).to(gpu_device), torch.Size([1, 0, res, res, res]), (3, 3, 3),
+                                                       (1, 1, 1), False)
+    first = {}
+    for i, c in enumerate(map(tuple, coords)):
+        first.setdefault(c, i)
+    want = np.full((len(coords), 27), 0xFFFFFFFF, np.uint32)
+    for i, (b, x, y, z) in enumerate(coords):
+        for v in range(27):
+            want[i, v] = first.get((b, x + v // 9 - 1, y + v // 3 % 3 - 1, z + v % 3 - 1), 0xFFFFFFFF)
+        want[i, 13] = i
+    assert np.array_equal(_np(cache.neighbor_map), want)
+
+
+@pytest.mark.parametrize("dims,n", [((2, 40, 41, 39), 3000), ((1, 260, 250, 261), 4001), ((3, 5, 7, 90001), 700)])
+@pytest.mark.parametrize("geom", [((2, 2, 2), (2, 2, 2), (0, 0, 0), (1, 1, 1)), ((3, 3, 3), (2, 1, 3), (1, 0, 2), (1, 2, 1)),
+                                  ((1, 1, 5), (1, 1, 2), (0, 0, 1), (1, 1, 1))])
+def test_generic_convolution(gpu_device, dims, n, geom):
+    _say(f"grid conv dims={dims} n={n} geom={geom}")
+    coords = _voxels(dims, n, 3, "shuffled")
+    shape = torch.Size([dims[0], 0, *dims[1:]])
+    dev_coords = torch.from_numpy(coords).to(gpu_device)
+    out = SparseConv3dFunction._get_output_coords(dev_coords, shape, *geom)
+    want = sc.output_coords(coords, tuple(shape), *geom)
+    assert np.array_equal(out.cpu().numpy(), want)
+    if len(want) == 0:
+        return
+    cache = SparseConv3dFunction._compute_neighbor_cache(dev_coords, out, shape, *geom, True)
+    fwd, bwd = sc.neighbor_maps(coords, want, tuple(shape), *geom)
+    assert np.array_equal(_np(cache.neighbor_map), fwd)
+    assert np.array_equal(_np(cache.neighbor_map_bwd), bwd)
+    gray, binary = nb.gray_binary(fwd)
+    assert np.array_equal(_np(cache.gray_code), gray)
+    assert np.array_equal(_np(cache.sorted_idx), nb.sorted_idx_canonical(binary))
+    if any(s != 1 for s in geom[1]):
+        gray, binary = nb.gray_binary(bwd)
+        assert np.array_equal(_np(cache.gray_code_bwd), gray)
+        assert np.array_equal(_np(cache.sorted_idx_bwd), nb.sorted_idx_canonical(binary))
+
+
+# the rank sort's last size and the radix sort's first, the switch to long tiles, partial tiles; all code bits in use and few
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 16384, 16385, 786431, 786432, 1000003])
+@pytest.mark.parametrize("volume,distinct", [(27, 3000), (32, 1 << 32), (3, 8)])
+def test_mask_sort(gpu_device, n, volume, distinct):
+    _say(f"mask sort n={n} volume={volume} distinct={distinct}")
+    gen = torch.Generator(device=gpu_device).manual_seed(n)
+    lo, hi = (-(1 << 31), (1 << 31) - 1) if volume == 32 else (0, 1 << volume)
+    keys = torch.randint(lo, hi, (min(distinct, n),), generator=gen, device=gpu_device, dtype=torch.int64).to(torch.int32)
+    keys = keys[torch.randint(0, keys.shape[0], (n,), generator=gen, device=gpu_device)].contiguous()
+    order = torch.empty((n,), dtype=torch.int64, device=gpu_device)
+    L = nat.lib()
+    ws = nat.workspace(L.fgx_sort_workspace_bytes(nat.sz(n)), gpu_device)
+    nat.check(L.fgx_sort_by_code(nat.ptr(keys), nat.sz(n), C.c_int(volume), nat.ptr(order), nat.ptr(ws), nat.sz(ws.numel()), nat.stream()))
+    assert np.array_equal(order.cpu().numpy(), np.argsort(keys.cpu().numpy(), kind="stable"))
