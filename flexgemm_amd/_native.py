@@ -46,7 +46,7 @@ EXPORTS = [
     "fgx_spconv_neighbor_map_sorted_workspace_bytes", "fgx_spconv_neighbor_map_sorted",
     "fgx_serialize_encode", "fgx_serialize_decode", "fgx_serialize_reorder_workspace_bytes",
     "fgx_serialize_reorder_coords",
-    "fgx_grid_index_pays", "fgx_subm_neighbor_map_grid_workspace_bytes", "fgx_subm_neighbor_map_grid", "fgx_subm_cache_grid_workspace_bytes",
+    "fgx_tile_plan", "fgx_grid_index_pays", "fgx_subm_neighbor_map_grid_workspace_bytes", "fgx_subm_neighbor_map_grid", "fgx_subm_cache_grid_workspace_bytes",
     "fgx_subm_cache_build_grid", "fgx_spconv_neighbor_map_grid_workspace_bytes", "fgx_spconv_neighbor_map_grid",
     "fgx_spconv_cache_grid_workspace_bytes", "fgx_spconv_cache_build_grid", "fgx_spconv_out_coords_grid_workspace_bytes",
     "fgx_spconv_out_coords_grid_count", "fgx_spconv_out_coords_grid_emit",
@@ -115,6 +115,34 @@ def lib() -> C.CDLL:
             getattr(L, name).restype = C.c_size_t
         _lib = L
     return _lib
+
+
+_HOST_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "fgx_host.so")
+_host = None
+
+
+def host():
+    """The native host side of the operators (csrc/host/fgx_host.cpp), loaded and bound to the library once."""
+    global _host
+    if _host is None:
+        if not os.path.exists(_HOST_PATH):
+            raise NativeError(f"{_HOST_PATH} is missing: build it with `python -m flexgemm_amd.build`.  There is no fallback implementation.")
+        import importlib.util
+        import sys
+        from .ops import spconv
+        from .ops.spconv import submanifold_conv3d
+        spec = importlib.util.spec_from_file_location("fgx_host", _HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        lib()
+        module.bind(_LIB_PATH, submanifold_conv3d, spconv, sys.modules[__name__])
+        _host = module
+    return _host
+
+
+def raw_stream(t: torch.Tensor) -> int:
+    """Handle of the current stream of the tensor's device, as a number (what the native host side takes)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def check(rc: int) -> None:

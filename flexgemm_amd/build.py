@@ -17,6 +17,9 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG, "csrc")
 OUT_DIR = os.path.join(PKG, "_lib")
 LIB = os.path.join(OUT_DIR, "libflexgemm_hip.so")
+# the operators' host side: a Python extension over torch's C++ API (host code only: no kernels in it)
+HOST_SRC = os.path.join(CSRC, "host", "fgx_host.cpp")
+HOST_LIB = os.path.join(OUT_DIR, "fgx_host.so")
 # a caller of the C ABI without Python or torch, run by the GPU tests (tests/cabi_host/conv_host.cpp)
 HOST_CHECK_SRC = os.path.join(PKG, "..", "tests", "cabi_host", "conv_host.cpp")
 HOST_CHECK = os.path.join(OUT_DIR, "conv_host")
@@ -40,6 +43,18 @@ def _stale(target: str, deps) -> bool:
         return True
     t = os.path.getmtime(target)
     return any(os.path.getmtime(d) > t for d in deps)
+
+
+def _host_command():
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    includes = cpp_extension.include_paths() + [sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wno-unknown-pragmas", "-D__HIP_PLATFORM_AMD__",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DTORCH_EXTENSION_NAME=fgx_host", "-DNDEBUG"]
+            + [f for i in includes for f in ("-isystem", i)]
+            + [HOST_SRC, "-o", HOST_LIB, "-L", torch_lib, "-lc10", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lamdhip64", "-ldl"])
 
 
 def build(force: bool = False, verbose: bool = True, jobs: int = 4) -> str:
@@ -68,8 +83,19 @@ def build(force: bool = False, verbose: bool = True, jobs: int = 4) -> str:
         if verbose and warn:
             print(warn, flush=True)
 
+    def compile_host():
+        cmd = _host_command()
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"g++ failed on {HOST_SRC}:\n{r.stdout}\n{r.stderr}")
+
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
+        host = ex.submit(compile_host) if force or _stale(HOST_LIB, [HOST_SRC] + hdrs) else None
         list(ex.map(compile_one, todo))
+        if host is not None:
+            host.result()
     if force or todo or _stale(LIB, objs):
         cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-fno-gpu-rdc"] + objs + ["-o", LIB]
         if verbose:

@@ -174,7 +174,7 @@ extern "C" size_t fgx_subm_cache_grid_workspace_bytes(size_t n, int B, int W, in
 extern "C" int fgx_subm_cache_build_grid(const int32_t* coords, size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dw,
                                          int Dh, int Dd, int with_pairs, void* workspace, size_t workspace_bytes, uint32_t* out_map,
                                          int32_t* gray, int32_t* binary, int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i,
-                                         uint32_t* sig_o, fgx_stream_t stream) {
+                                         uint32_t* sig_o, uint32_t* seg_host, fgx_stream_t stream) {
     const char* who = "fgx_subm_cache_build_grid";
     FGX_CHECK_ARG(Kw > 0 && Kh > 0 && Kd > 0 && (long long)Kw * Kh * Kd <= 32 && (Kw & 1) && (Kh & 1) && (Kd & 1),
                   "%s: mask codes need odd kernel sizes and a volume <= 32, got (%d,%d,%d)", who, Kw, Kh, Kd);
@@ -200,7 +200,7 @@ extern "C" int fgx_subm_cache_build_grid(const int32_t* coords, size_t n, int B,
         int r = counted ? FGX_OK : pair_counts(gray, n, V, counts, on);
         if (r != FGX_OK) return r;
         return pair_lists_from_counts(out_map, gray, n, V, counts, cdiv(n, counted ? kPairSubRows : kPairRows), counted,
-                                      (uint32_t*)(ws + P.offsets), (uint32_t*)(ws + P.totals), seg, sig_i, sig_o, on);
+                                      (uint32_t*)(ws + P.offsets), (uint32_t*)(ws + P.totals), seg, seg_host, sig_i, sig_o, on);
     });
 }
 
@@ -215,7 +215,7 @@ extern "C" int fgx_spconv_cache_build_grid(const int32_t* in_coords, size_t n_in
                                            int D, int Kw, int Kh, int Kd, int Sw, int Sh, int Sd, int Pw, int Ph, int Pd, int Dw, int Dh,
                                            int Dd, void* workspace, size_t workspace_bytes, uint32_t* map_fwd, int32_t* gray,
                                            int32_t* binary, int64_t* sorted_idx, uint32_t* map_bwd, uint32_t* seg, uint32_t* sig_i,
-                                           uint32_t* sig_o, int32_t* gray_bwd, int64_t* sorted_idx_bwd, fgx_stream_t stream) {
+                                           uint32_t* sig_o, uint32_t* seg_host, int32_t* gray_bwd, int64_t* sorted_idx_bwd, fgx_stream_t stream) {
     const char* who = "fgx_spconv_cache_build_grid";
     int Wo, Ho, Do;
     int rc = fgx_spconv_out_dims(W, H, D, Kw, Kh, Kd, Sw, Sh, Sd, Pw, Ph, Pd, Dw, Dh, Dd, &Wo, &Ho, &Do);
@@ -244,7 +244,7 @@ extern "C" int fgx_spconv_cache_build_grid(const int32_t* in_coords, size_t n_in
     if (rc != FGX_OK) return rc;
     rc = sort_beside_pairs(n_out, V, binary, sorted_idx, ws + P.sort_ws, P.sort_bytes, bwd, s, who, [&](hipStream_t on) {
         return pair_lists_from_counts(map_fwd, gray, n_out, V, counts, cdiv(n_out, kPairSubRows), true, (uint32_t*)(ws + P.offsets),
-                                      (uint32_t*)(ws + P.totals), seg, sig_i, sig_o, on);
+                                      (uint32_t*)(ws + P.totals), seg, seg_host, sig_i, sig_o, on);
     });
     if (rc != FGX_OK || !order_bwd) return rc;
     return fgx_sort_by_code(binary_bwd, n_in, V, sorted_idx_bwd, ws + P.sort2_ws, P.sort2_bytes, stream);

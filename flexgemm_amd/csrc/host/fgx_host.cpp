@@ -1,0 +1,704 @@
+// Host side of the operators' hot path: tensors in, library calls out.
+//
+// A convolution call is a handful of kernel launches around buffers from torch's allocator and tables kept on the
+// caller's neighbor cache.  Doing that from Python costs more than the kernels do on small inputs (two 64-channel layers of
+// 3 716 voxels, forward and backward: 0.69 ms of host time for 0.23 ms of kernels), so it is done here: one call per
+// product or cache build, which allocates, fills in the tables the cache does not have yet -- as attributes of the Python
+// object, under the names its Python methods use -- and enqueues the kernels through the C ABI of flexgemm_hip.h.
+// Policy (algorithm, schedule, which kernel family) stays with the Python callers.
+#include <dlfcn.h>
+#include <hip/hip_runtime_api.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/pybind.h>
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+
+#include <memory>
+#include <mutex>
+#include <string>
+#include <vector>
+
+#include "../../../include/flexgemm_hip.h"
+
+namespace py = pybind11;
+using at::Tensor;
+
+namespace {
+
+// ---- the library -------------------------------------------------------------------------------------------------
+#define FGX_HOST_FUNCTIONS(X)                                                                                                     \
+    X(fgx_last_error) X(fgx_grid_index_pays) X(fgx_subm_neighbor_map_grid_workspace_bytes) X(fgx_subm_cache_grid_workspace_bytes) \
+    X(fgx_subm_cache_build_grid) X(fgx_spconv_cache_grid_workspace_bytes) X(fgx_spconv_cache_build_grid)                           \
+    X(fgx_spconv_out_dims) X(fgx_spconv_out_coords_grid_workspace_bytes) X(fgx_spconv_out_coords_grid_count)                       \
+    X(fgx_spconv_out_coords_grid_emit) X(fgx_tile_plan) X(fgx_gather_item_order) X(fgx_gather_item_order_workspace_bytes)          \
+    X(fgx_weight_panel_bytes) X(fgx_pack_weight) X(fgx_conv_scratch_bytes) X(fgx_conv_gather_gemm_act_mask)                        \
+    X(fgx_conv_gather_gemm_stream_act_mask) X(fgx_conv_gather_gemm_stream_groups) X(fgx_relu_mask_apply)                           \
+    X(fgx_colsum_scratch_bytes) X(fgx_colsum) X(fgx_wgrad_block_bounds_count) X(fgx_wgrad_block_bounds)                            \
+    X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
+    X(fgx_wgrad_sweep_plan_bytes) X(fgx_wgrad_sweep_plan) X(fgx_wgrad_sweep_scratch_bytes) X(fgx_conv_wgrad_sweep)                 \
+    X(fgx_serialize_encode) X(fgx_serialize_decode)
+
+struct Lib {
+#define X(name) decltype(&::name) name = nullptr;
+    FGX_HOST_FUNCTIONS(X)
+#undef X
+} L;
+
+// the Python modules whose switches the calls below read (looked up on every call: tests and users change them)
+PyObject* g_impl = nullptr;         // ops.spconv.submanifold_conv3d
+PyObject* g_spconv = nullptr;       // ops.spconv
+PyObject* g_native = nullptr;       // _native
+
+void bind(const std::string& path, py::module_ impl, py::module_ spconv, py::module_ native) {
+    void* lib = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
+    if (lib == nullptr) throw std::runtime_error(std::string("cannot load ") + path + ": " + dlerror());
+#define X(name)                                                                                                   \
+    L.name = (decltype(L.name))dlsym(lib, #name);                                                                 \
+    if (L.name == nullptr) throw std::runtime_error(path + " does not export " #name ": build the package again");
+    FGX_HOST_FUNCTIONS(X)
+#undef X
+    g_impl = impl.release().ptr();
+    g_spconv = spconv.release().ptr();
+    g_native = native.release().ptr();
+}
+
+void check(int rc) {
+    if (rc == 0) return;
+    const std::string msg = L.fgx_last_error();
+    if (rc == -1) throw py::value_error(msg);
+    if (rc == -3) {
+        PyErr_SetString(PyExc_NotImplementedError, msg.c_str());
+        throw py::error_already_set();
+    }
+    py::object err = py::reinterpret_borrow<py::object>(g_native).attr("NativeError");
+    PyErr_SetString(err.ptr(), msg.c_str());
+    throw py::error_already_set();
+}
+
+// ---- Python attributes ---------------------------------------------------------------------------------------------
+PyObject* module_get(PyObject* module, const char* name) {      // borrowed
+    PyObject* v = PyDict_GetItemString(PyModule_GetDict(module), name);
+    if (v == nullptr) throw py::attribute_error(name);
+    return v;
+}
+long module_int(PyObject* module, const char* name) { return PyLong_AsLong(module_get(module, name)); }
+
+// A neighbor cache: a Python object whose instance dictionary holds its tables.
+struct Cache {
+    py::object obj, dict;
+    explicit Cache(py::object o) : obj(std::move(o)), dict(obj.attr("__dict__")) {}
+    PyObject* find(const char* key) const { return PyDict_GetItemString(dict.ptr(), key); }        // borrowed, null if absent
+    PyObject* find(const std::string& key) const { return find(key.c_str()); }
+    bool has(const char* key) const { return find(key) != nullptr; }
+    bool tensor(const std::string& key, Tensor* out) const {
+        PyObject* v = find(key);
+        if (v == nullptr || !THPVariable_Check(v)) return false;
+        *out = THPVariable_Unpack(v);
+        return true;
+    }
+    Tensor need(const char* key) const {        // through the attribute, which may finish what is still in flight
+        Tensor t;
+        if (tensor(key, &t)) return t;
+        return obj.attr(key).cast<Tensor>();
+    }
+    void set(const std::string& key, py::handle value) const {
+        if (PyDict_SetItemString(dict.ptr(), key.c_str(), value.ptr()) != 0) throw py::error_already_set();
+    }
+    void set(const std::string& key, const Tensor& t) const { set(key, py::cast(t)); }
+};
+
+// ---- buffers ---------------------------------------------------------------------------------------------------------
+Tensor make(at::IntArrayRef sizes, at::ScalarType type, const at::Device& dev) {
+    return at::empty(sizes, at::TensorOptions().dtype(type).device(dev));
+}
+Tensor workspace(size_t bytes, const at::Device& dev) { return make({(int64_t)(bytes < 256 ? 256 : bytes)}, at::kByte, dev); }
+template <typename T = void>
+T* ptr(const Tensor& t) {
+    if (!t.defined()) return nullptr;
+    if (!t.is_contiguous()) throw py::value_error("a strided view was about to be passed as a plain pointer");    // the kernels assume dense rows
+    return (T*)t.data_ptr();
+}
+fgx_stream_t as_stream(int64_t s) { return (fgx_stream_t)(uintptr_t)s; }
+
+// ---- the segment table on its way to the host ------------------------------------------------------------------------
+// The pair lists' segment table is written to a pinned block by the kernel that fills the lists; the event behind it tells
+// when it has arrived.  Blocks are kept for the next cache (at most kIdleBlocks of them; one that may still be written is
+// not handed out), the rest is freed.
+struct SegBlock {
+    uint32_t* words = nullptr;
+    hipEvent_t event = nullptr;
+    int device = -1;
+};
+constexpr size_t kIdleBlocks = 64, kSegWords = 64;
+std::mutex g_blocks_mutex;
+std::vector<SegBlock> g_idle_blocks;
+
+void hip_check(hipError_t e, const char* what) {
+    if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
+}
+
+// (asking an event would break a capture some other thread is making in the strict mode)
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+bool capturing(int64_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    hip_check(hipStreamIsCapturing((hipStream_t)(uintptr_t)stream, &status), "hipStreamIsCapturing");
+    return status != hipStreamCaptureStatusNone;
+}
+
+SegBlock take_block(int device) {
+    const RelaxedCapture relaxed;
+    {
+        std::lock_guard<std::mutex> lock(g_blocks_mutex);
+        for (size_t i = 0; i < g_idle_blocks.size(); ++i)
+            if (g_idle_blocks[i].device == device && hipEventQuery(g_idle_blocks[i].event) == hipSuccess) {
+                const SegBlock b = g_idle_blocks[i];
+                g_idle_blocks[i] = g_idle_blocks.back();
+                g_idle_blocks.pop_back();
+                return b;
+            }
+    }
+    (void)hipGetLastError();        // (a query of an event still ahead leaves its answer behind as an error)
+    SegBlock b;
+    b.device = device;
+    hip_check(hipHostMalloc((void**)&b.words, kSegWords * sizeof(uint32_t), hipHostMallocPortable | hipHostMallocMapped), "hipHostMalloc");
+    hip_check(hipEventCreateWithFlags(&b.event, hipEventDisableTiming), "hipEventCreate");
+    return b;
+}
+
+void give_block(const SegBlock& b) {
+    {
+        std::lock_guard<std::mutex> lock(g_blocks_mutex);
+        if (g_idle_blocks.size() < kIdleBlocks) {
+            g_idle_blocks.push_back(b);
+            return;
+        }
+    }
+    const RelaxedCapture relaxed;
+    (void)hipEventSynchronize(b.event);
+    (void)hipEventDestroy(b.event);
+    (void)hipHostFree(b.words);
+}
+
+class SegHost {
+public:
+    SegHost(int device, int count) : block_(take_block(device)), count_(count) {}
+    ~SegHost() { give_block(block_); }
+    SegHost(const SegHost&) = delete;
+    SegHost& operator=(const SegHost&) = delete;
+    uint32_t* words() { return block_.words; }
+    void record(fgx_stream_t s) { hip_check(hipEventRecord(block_.event, (hipStream_t)s), "hipEventRecord"); }
+    void synchronize() {
+        py::gil_scoped_release nogil;
+        hip_check(hipEventSynchronize(block_.event), "hipEventSynchronize");
+    }
+    py::list tolist() const {
+        py::list out;
+        for (int i = 0; i < count_; ++i) out.append(py::int_(block_.words[i]));
+        return out;
+    }
+
+private:
+    SegBlock block_;
+    int count_;
+};
+
+// ---- neighbor caches ---------------------------------------------------------------------------------------------------
+// Tables of a submanifold convolution through the grid index, or None where it does not apply:
+// (neighbor_map, gray, binary, order, seg, sig_i, sig_o, SegHost), the last four None without gradients.
+py::object subm_cache(const Tensor& coords, const std::vector<int>& geom, bool needs_grad, bool forced, size_t max_pair_bytes, int64_t stream) {
+    const size_t n = (size_t)coords.size(0);
+    const int B = geom[0], W = geom[1], H = geom[2], D = geom[3], V = geom[4] * geom[5] * geom[6];
+    if (n == 0 || V > 32 || n * (size_t)V >= 0xFFFFFFFFull || (needs_grad && n * (size_t)V * 8 > max_pair_bytes)) return py::none();
+    if (needs_grad && capturing(stream)) return py::none();        // (nothing may wait for the segment table inside a capture)
+    if (!L.fgx_grid_index_pays(n, B, W, H, D) && !(forced && L.fgx_subm_neighbor_map_grid_workspace_bytes(n, B, W, H, D))) return py::none();
+    const at::Device dev = coords.device();
+    const c10::DeviceGuard guard(dev);
+    const int64_t rows = (int64_t)n, slots = rows * V;
+    Tensor nmap = make({rows, V}, at::kUInt32, dev), gray = make({rows}, at::kInt, dev), binary = make({rows}, at::kInt, dev);
+    Tensor order = make({rows}, at::kLong, dev), seg, sig_i, sig_o;
+    std::unique_ptr<SegHost> host;
+    if (needs_grad) {
+        seg = make({V + 1}, at::kUInt32, dev);
+        sig_i = make({slots}, at::kUInt32, dev);
+        sig_o = make({slots}, at::kUInt32, dev);
+        host = std::make_unique<SegHost>(dev.index(), V + 1);
+    }
+    Tensor ws = workspace(L.fgx_subm_cache_grid_workspace_bytes(n, B, W, H, D, V, needs_grad), dev);
+    check(L.fgx_subm_cache_build_grid(ptr<int32_t>(coords), n, B, W, H, D, geom[4], geom[5], geom[6], geom[7], geom[8], geom[9], needs_grad,
+                                      ptr(ws), (size_t)ws.numel(), ptr<uint32_t>(nmap), ptr<int32_t>(gray), ptr<int32_t>(binary),
+                                      ptr<int64_t>(order), ptr<uint32_t>(seg), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o),
+                                      host ? host->words() : nullptr, as_stream(stream)));
+    if (!host) return py::make_tuple(nmap, gray, binary, order, py::none(), py::none(), py::none(), py::none());
+    host->record(as_stream(stream));
+    return py::make_tuple(nmap, gray, binary, order, seg, sig_i, sig_o, std::move(host));
+}
+
+bool conv_grids_pay(size_t n_in, size_t n_out, int B, const int* in, const int* out, bool with_bwd) {
+    return L.fgx_grid_index_pays(n_in, B, in[0], in[1], in[2]) && (!with_bwd || L.fgx_grid_index_pays(n_out, B, out[0], out[1], out[2]));
+}
+
+// geom: B, W, H, D, kernel, stride, padding, dilation.  The dictionary of a generic convolution's tables, or None.
+py::object spconv_cache(const Tensor& coords, const Tensor& out_coords, const std::vector<int>& g, bool needs_grad, bool bwd_order,
+                        size_t max_pair_bytes, int64_t stream) {
+    const size_t m = (size_t)coords.size(0), l = (size_t)out_coords.size(0);
+    const int V = g[4] * g[5] * g[6];
+    if (m == 0 || l == 0 || V > 32 || l * (size_t)V >= 0xFFFFFFFFull || (needs_grad && l * (size_t)V * 8 > max_pair_bytes)) return py::none();
+    if (needs_grad && capturing(stream)) return py::none();        // (as in subm_cache)
+    int out[3];
+    check(L.fgx_spconv_out_dims(g[1], g[2], g[3], g[4], g[5], g[6], g[7], g[8], g[9], g[10], g[11], g[12], g[13], g[14], g[15], &out[0], &out[1], &out[2]));
+    if (out[0] < 1 || out[1] < 1 || out[2] < 1 || !conv_grids_pay(m, l, g[0], &g[1], out, needs_grad)) return py::none();
+    const at::Device dev = coords.device();
+    const c10::DeviceGuard guard(dev);
+    const int64_t rows = (int64_t)l;
+    Tensor nmap = make({rows, V}, at::kUInt32, dev), gray = make({rows}, at::kInt, dev), binary = make({rows}, at::kInt, dev);
+    Tensor order = make({rows}, at::kLong, dev), nmap_bwd, seg, sig_i, sig_o, gray_bwd, order_bwd;
+    std::unique_ptr<SegHost> host;
+    if (needs_grad) {
+        nmap_bwd = make({(int64_t)m, V}, at::kUInt32, dev);
+        seg = make({V + 1}, at::kUInt32, dev);
+        sig_i = make({rows * V}, at::kUInt32, dev);
+        sig_o = make({rows * V}, at::kUInt32, dev);
+        host = std::make_unique<SegHost>(dev.index(), V + 1);
+        if (bwd_order) {
+            gray_bwd = make({(int64_t)m}, at::kInt, dev);
+            order_bwd = make({(int64_t)m}, at::kLong, dev);
+        }
+    }
+    Tensor ws = workspace(L.fgx_spconv_cache_grid_workspace_bytes(m, l, g[0], g[1], g[2], g[3], out[0], out[1], out[2], V, needs_grad,
+                                                                  order_bwd.defined()), dev);
+    check(L.fgx_spconv_cache_build_grid(ptr<int32_t>(coords), m, ptr<int32_t>(out_coords), l, g[0], g[1], g[2], g[3], g[4], g[5], g[6], g[7], g[8],
+                                        g[9], g[10], g[11], g[12], g[13], g[14], g[15], ptr(ws), (size_t)ws.numel(), ptr<uint32_t>(nmap),
+                                        ptr<int32_t>(gray), ptr<int32_t>(binary), ptr<int64_t>(order), ptr<uint32_t>(nmap_bwd), ptr<uint32_t>(seg),
+                                        ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o), host ? host->words() : nullptr, ptr<int32_t>(gray_bwd),
+                                        ptr<int64_t>(order_bwd), as_stream(stream)));
+    py::dict t;
+    t["nmap"] = nmap;
+    t["gray"] = gray;
+    t["order"] = order;
+    if (needs_grad) {
+        host->record(as_stream(stream));
+        t["nmap_bwd"] = nmap_bwd;
+        if (bwd_order) {
+            t["gray_bwd"] = gray_bwd;
+            t["order_bwd"] = order_bwd;
+        }
+        t["pairs"] = py::dict(py::arg("seg") = seg, py::arg("pending") = py::make_tuple(sig_i, sig_o, py::cast(std::move(host))));
+    }
+    return std::move(t);
+}
+
+// Output coordinates in (b, x, y, z) order through the bit map of the output grid, or None where it does not apply.
+py::object out_coords(const Tensor& coords, const std::vector<int>& g, int64_t stream) {
+    const size_t m = (size_t)coords.size(0);
+    int out[3];
+    check(L.fgx_spconv_out_dims(g[1], g[2], g[3], g[4], g[5], g[6], g[7], g[8], g[9], g[10], g[11], g[12], g[13], g[14], g[15], &out[0], &out[1], &out[2]));
+    if (m * (size_t)g[4] * g[5] * g[6] >= (size_t)1 << 30 || !L.fgx_grid_index_pays(m, g[0], out[0], out[1], out[2])) return py::none();
+    const at::Device dev = coords.device();
+    const c10::DeviceGuard guard(dev);
+    Tensor ws = workspace(L.fgx_spconv_out_coords_grid_workspace_bytes(g[0], out[0], out[1], out[2]), dev);
+    SegHost host(dev.index(), 2);           // the number of coordinates, as one 64-bit word
+    check(L.fgx_spconv_out_coords_grid_count(ptr<int32_t>(coords), m, g[0], g[1], g[2], g[3], g[4], g[5], g[6], g[7], g[8], g[9], g[10], g[11],
+                                             g[12], g[13], g[14], g[15], ptr(ws), (size_t)ws.numel(), (uint64_t*)host.words(), as_stream(stream)));
+    host.record(as_stream(stream));
+    host.synchronize();                     // the one wait of the host: sizes the result
+    uint64_t total;
+    memcpy(&total, host.words(), sizeof(total));
+    Tensor result = make({(int64_t)total, 4}, at::kInt, dev);
+    check(L.fgx_spconv_out_coords_grid_emit(ptr(ws), g[0], out[0], out[1], out[2], (size_t)total, ptr<int32_t>(result), as_stream(stream)));
+    return py::cast(result);
+}
+
+// ---- tile tables -----------------------------------------------------------------------------------------------------
+struct Tiles {
+    Tensor order, code, plan_seg, plan_idx, plan_band;
+    std::string plan_key;
+};
+
+// Row order and tile masks of the masked schedule for tiles of `block` rows (own_order: the kernels' own row order).
+void tile_codes(const Cache& c, int block, bool own_order, int64_t stream, Tiles* t, bool for_plan) {
+    t->order = c.need(own_order ? "_tile_order" : "sorted_idx");
+    const std::string key = (own_order ? "_tile_code_" : "_mask_code_") + std::to_string(block);
+    if (c.tensor(key, &t->code) || for_plan) return;        // (the plan's call makes the masks on its way)
+    const Tensor gray = c.need("gray_code");
+    const int64_t n = gray.size(0);
+    t->code = make({(n + block - 1) / block}, at::kInt, gray.device());
+    check(L.fgx_tile_plan(ptr<int32_t>(gray), ptr<int64_t>(t->order), nullptr, (size_t)n, 1, block, 0, ptr<int32_t>(t->code), nullptr, nullptr,
+                          nullptr, nullptr, 1, 1, 1, nullptr, nullptr, as_stream(stream)));
+    c.set(key, t->code);
+}
+
+// How the tiles of a streaming GEMM are dealt: by cost ("balanced") or in the kernel's own order.
+// The locality order of short-row layers lives on neighboring tiles sharing an XCD (dealing them by cost alone: 0.32 -> 0.42
+// ms per launch at C = 32); with rows of 512 bytes and more balance wins whatever the number of tiles (-6 % per launch at
+// C = 256, -8 % at C = 1024); with shorter rows it wins while a workgroup has few tiles (C = 128, forward: 143 616 voxels
+// 0.120 -> 0.101 ms, 252 392 voxels 0.179 -> 0.155, 577 592 voxels 0.342 -> 0.320; 669 288 voxels, 10 rounds of items, and
+// 1 026 536 voxels, 16 rounds: no change).  With at most one item per workgroup there is nothing to even out; from there on
+// the dealt order pays (forward at 64 160 voxels: C = 256, two rounds of items, 0.158 -> 0.141 ms; C = 512, four rounds, 0.550
+// -> 0.512 ms; 15 192 voxels C = 1024, two rounds, 0.601 -> 0.568 ms).
+bool deal_items(const std::string& plan_key, int64_t tiles, int col_tiles, int groups, int slabs) {
+    std::string mode = py::reinterpret_borrow<py::object>(module_get(g_spconv, "GEMM_ITEM_ORDER")).cast<std::string>();
+    const int64_t items = tiles * col_tiles;
+    if (mode == "auto") {
+        const bool few_rounds = items <= module_int(g_impl, "ITEM_ORDER_ANY_ROW_MAX_ROUNDS") * groups;
+        mode = (slabs >= 4 || few_rounds) && plan_key.rfind("_plan_t_", 0) != 0 ? "balanced" : "default";
+    }
+    if (mode == "default" || items <= module_int(g_impl, "ITEM_ORDER_MIN_ROUNDS") * groups || groups > 1024) return false;
+    if (mode != "balanced") throw py::value_error("unknown GEMM_ITEM_ORDER '" + mode + "'; expected 'auto', 'balanced' or 'default'");
+    return true;
+}
+
+std::string items_key(const std::string& plan_key, int col_tiles, int groups, int slabs) {
+    return "_items_" + plan_key + "_" + std::to_string(col_tiles) + "_" + std::to_string(groups) + "_" + std::to_string(slabs);
+}
+
+Tensor item_order(const Cache& c, const std::string& plan_key, const Tensor& code, int col_tiles, int groups, int slabs, int64_t stream) {
+    Tensor item_at;
+    if (!deal_items(plan_key, code.size(0), col_tiles, groups, slabs)) return item_at;
+    const std::string key = items_key(plan_key, col_tiles, groups, slabs);
+    if (c.tensor(key, &item_at)) return item_at;
+    const size_t nb = (size_t)code.size(0);
+    item_at = make({code.size(0) * col_tiles}, at::kInt, code.device());
+    Tensor ws = workspace(L.fgx_gather_item_order_workspace_bytes(nb, col_tiles), code.device());
+    check(L.fgx_gather_item_order(ptr<int32_t>(code), nb, col_tiles, slabs, groups, ptr(ws), (size_t)ws.numel(), ptr<uint32_t>(item_at), as_stream(stream)));
+    c.set(key, item_at);
+    return item_at;
+}
+
+// The gather plan for tiles of `block` rows (dense: rows in their natural order, every tile all offsets), and with
+// col_tiles > 0 the item order of a launch over it; whatever is missing is made in one call.
+Tiles gather_plan(const Cache& c, int block, bool own_order, bool dense, int col_tiles, int groups, int slabs, Tensor* item_at, int64_t stream) {
+    Tiles t;
+    if (dense) {
+        py::tuple oc = c.obj.attr("_dense_tile_tables")(block);
+        t.order = oc[0].cast<Tensor>();
+        t.code = oc[1].cast<Tensor>();
+        t.plan_key = "_plan_d_" + std::to_string(block);
+    } else {
+        tile_codes(c, block, own_order, stream, &t, true);
+        t.plan_key = std::string(own_order ? "_plan_t_" : "_plan_m_") + std::to_string(block);
+    }
+    PyObject* kept = c.find(t.plan_key);
+    if (kept != nullptr) {
+        py::tuple p = py::reinterpret_borrow<py::tuple>(kept);
+        t.plan_seg = p[0].cast<Tensor>();
+        t.plan_idx = p[1].cast<Tensor>();
+        t.plan_band = p[2].cast<Tensor>();
+        if (item_at != nullptr) *item_at = item_order(c, t.plan_key, t.code, col_tiles, groups, slabs, stream);
+        return t;
+    }
+    const Tensor nmap = c.need("neighbor_map");
+    const at::Device dev = nmap.device();
+    const int64_t n = nmap.size(0), v = nmap.size(1), nb = (n + block - 1) / block;
+    const bool have_codes = t.code.defined();
+    Tensor gray;
+    if (!have_codes) {
+        gray = c.need("gray_code");
+        t.code = make({nb}, at::kInt, dev);
+    }
+    t.plan_seg = make({nb + 1}, at::kInt, dev);
+    const int64_t rows = nb * std::min<int64_t>(v, 32);       // the bound (every offset in every tile): no wait for the exact count
+    t.plan_idx = make({rows, block}, at::kUInt32, dev);
+    t.plan_band = make({rows}, at::kUInt32, dev);
+    Tensor items_ws;
+    if (item_at != nullptr && deal_items(t.plan_key, nb, col_tiles, groups, slabs)) {
+        *item_at = make({nb * col_tiles}, at::kInt, dev);
+        items_ws = workspace(L.fgx_gather_item_order_workspace_bytes((size_t)nb, col_tiles), dev);
+    }
+    check(L.fgx_tile_plan(ptr<int32_t>(gray), ptr<int64_t>(t.order), ptr<uint32_t>(nmap), (size_t)n, (int)v, block, have_codes, ptr<int32_t>(t.code),
+                          nullptr, ptr<int32_t>(t.plan_seg), ptr<uint32_t>(t.plan_idx), ptr<uint32_t>(t.plan_band), col_tiles > 0 ? col_tiles : 1,
+                          slabs > 0 ? slabs : 1, groups > 0 ? groups : 1, ptr<uint32_t>(items_ws),
+                          items_ws.defined() ? ptr<uint32_t>(*item_at) : nullptr, as_stream(stream)));
+    if (!have_codes) c.set((own_order ? "_tile_code_" : "_mask_code_") + std::to_string(block), t.code);
+    c.set(t.plan_key, py::make_tuple(t.plan_seg, t.plan_idx, t.plan_band));
+    if (items_ws.defined()) c.set(items_key(t.plan_key, col_tiles, groups, slabs), *item_at);
+    return t;
+}
+
+// ---- products --------------------------------------------------------------------------------------------------------
+struct Sched {
+    int tile_rows, tile_cols, slab_bytes, splitk, block_rows, stream;
+};
+
+Sched read_schedule(py::handle s) {
+    Py_buffer view;
+    if (PyObject_GetBuffer(s.ptr(), &view, PyBUF_SIMPLE) != 0) throw py::error_already_set();
+    Sched out;
+    const bool fits = view.len == (Py_ssize_t)sizeof(out);
+    if (fits) memcpy(&out, view.buf, sizeof(out));
+    PyBuffer_Release(&view);
+    if (!fits) throw py::value_error("not a schedule");
+    return out;
+}
+
+void mark(const char* name, const char* phase) {
+    PyObject* hook = PyDict_GetItemString(PyModule_GetDict(g_native), "EVENT_HOOK");
+    if (hook != nullptr && hook != Py_None) py::reinterpret_borrow<py::object>(hook)(name, phase);
+}
+
+int dtype_code(const Tensor& t) {
+    switch (t.scalar_type()) {
+        case at::kHalf: return FGX_F16;
+        case at::kBFloat16: return FGX_BF16;
+        case at::kFloat: return FGX_F32;
+        default: throw py::type_error("unsupported feature dtype; expected float16, bfloat16 or float32");
+    }
+}
+
+int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
+
+// The gather GEMM on the streaming or the tiled kernel.  mode 0 forward, 1 / 2 input gradient (see _gather_gemm); operands
+// dense, rows whole 16-byte pieces.  panel: a kept weight panel, or None to pack one.  stream_fits: the streaming kernel's
+// 32-bit offsets reach.  Returns (output, ReLU bit mask or None).
+py::tuple gather_gemm(const Tensor& src, const Tensor& weight, const c10::optional<Tensor>& bias, py::object cache_obj, int mode, int splitk,
+                      bool masked, bool own_order, int activation, bool want_mask, py::object sched_obj, const c10::optional<Tensor>& panel_kept,
+                      bool stream_fits, int64_t stream) {
+    const Cache c(std::move(cache_obj));
+    const Sched s = read_schedule(sched_obj);
+    const at::Device dev = src.device();
+    const c10::DeviceGuard guard(dev);
+    const int co = (int)weight.size(0), v = (int)weight.size(1), ci = (int)weight.size(2);
+    const int k = mode == 0 ? ci : co, cols = mode == 0 ? co : ci;
+    const Tensor nmap = c.need("neighbor_map");
+    const int64_t n = nmap.size(0);
+    const size_t n_src = (size_t)src.size(0);
+    const int code = dtype_code(src);
+    const int es = (int)src.element_size();
+    Tensor out = make({n, cols}, src.scalar_type(), dev), mask;
+    if (want_mask && activation == FGX_ACT_RELU && es == 2 && cols % 8 == 0) mask = make({n * cols / 8}, at::kByte, dev);
+    Tensor panel;
+    if (panel_kept.has_value()) {
+        panel = *panel_kept;
+    } else {
+        panel = workspace(L.fgx_weight_panel_bytes(code, mode, ci, co, v, s.slab_bytes, s.tile_cols), dev);
+        check(L.fgx_pack_weight(code, mode, ptr(weight), ci, co, v, s.slab_bytes, s.tile_cols, ptr(panel), as_stream(stream)));
+    }
+    const void* b = bias.has_value() ? ptr(*bias) : nullptr;
+    const char* name = mode == 0 ? "gather_gemm_fwd" : "gather_gemm_dgrad";
+    if (s.stream && stream_fits) {
+        int groups = 0;
+        check(L.fgx_conv_gather_gemm_stream_groups(code, cols, s.tile_rows, s.tile_cols, s.slab_bytes, &groups));
+        Tensor item_at;
+        const Tiles t = gather_plan(c, s.tile_rows, own_order, !masked, ceil_div(cols, s.tile_cols), groups, ceil_div((int64_t)k * es, s.slab_bytes),
+                                    &item_at, stream);
+        mark(name, "start");
+        check(L.fgx_conv_gather_gemm_stream_act_mask(code, ptr(src), ptr(panel), b, ptr<int64_t>(t.order), ptr<int32_t>(t.code),
+                                                     ptr<int32_t>(t.plan_seg), ptr<uint32_t>(t.plan_idx), ptr<uint32_t>(t.plan_band),
+                                                     (size_t)t.plan_idx.size(0), (size_t)n, n_src, k, cols, v, s.tile_rows, s.tile_cols,
+                                                     s.slab_bytes, ptr<uint32_t>(item_at), groups, activation, ptr(out), ptr<uint8_t>(mask),
+                                                     as_stream(stream)));
+        mark(name, "stop");
+    } else {
+        Tiles t;
+        if (masked) {
+            tile_codes(c, s.tile_rows, own_order, stream, &t, false);
+        } else {
+            py::tuple oc = c.obj.attr("_dense_tile_tables")(s.tile_rows);
+            t.order = oc[0].cast<Tensor>();
+            t.code = oc[1].cast<Tensor>();
+        }
+        Tensor scratch;
+        if (splitk > 1) scratch = workspace(L.fgx_conv_scratch_bytes((size_t)n, cols, splitk), dev);
+        mark(name, "start");
+        check(L.fgx_conv_gather_gemm_act_mask(code, ptr(src), ptr(panel), b, ptr<uint32_t>(nmap), ptr<int64_t>(t.order), ptr<int32_t>(t.code),
+                                              (size_t)n, k, cols, v, s.tile_rows, s.tile_cols, s.slab_bytes, splitk, ptr(scratch), activation,
+                                              ptr(out), ptr<uint8_t>(mask), as_stream(stream)));
+        mark(name, "stop");
+    }
+    return py::make_tuple(out, mask.defined() ? py::cast(mask) : py::none());
+}
+
+// [V + 1] words of the segment table on the host
+std::vector<uint32_t> seg_host(const Cache& c, int v) {
+    PyObject* kept = c.find("_valid_signal_seg_host");
+    py::sequence words = kept != nullptr ? py::reinterpret_borrow<py::sequence>(kept) : c.obj.attr("_seg_host")().cast<py::sequence>();
+    if ((int)py::len(words) != v + 1) throw py::value_error("valid_signal_seg does not fit the pair lists (V + 1 entries, the last one their length)");
+    std::vector<uint32_t> out((size_t)v + 1);
+    for (int i = 0; i <= v; ++i) out[i] = words[i].cast<uint32_t>();
+    return out;
+}
+
+Tensor wgrad_bounds(const Cache& c, const Tensor& sig_o, const std::vector<uint32_t>& seg, size_t n, int v, int block_rows, int64_t stream) {
+    const std::string key = "_wgrad_bounds_" + std::to_string(block_rows);
+    Tensor bounds;
+    if (c.tensor(key, &bounds)) return bounds;
+    const int64_t count = (int64_t)L.fgx_wgrad_block_bounds_count(n, v, block_rows);
+    bounds = make({std::max<int64_t>(count, 1)}, at::kUInt32, sig_o.device());
+    check(L.fgx_wgrad_block_bounds(ptr<uint32_t>(sig_o), seg.data(), n, v, block_rows, ptr<uint32_t>(bounds), as_stream(stream)));
+    c.set(key, bounds);
+    return bounds;
+}
+
+Tensor wgrad_item_lists(const Cache& c, const Tensor& bounds, size_t n, int v, int ci, int co, const Sched& s, int64_t stream) {
+    const std::string key = "_wgrad_lists_" + std::to_string(s.block_rows) + "_" + std::to_string(s.tile_rows) + "_" + std::to_string(s.tile_cols) +
+                            "_" + std::to_string(ci) + "_" + std::to_string(co);
+    Tensor lists;
+    if (PyObject* kept = c.find(key)) {
+        if (THPVariable_Check(kept)) lists = THPVariable_Unpack(kept);
+        return lists;                                   // (None: the library has none for the shape)
+    }
+    const size_t words = L.fgx_wgrad_item_lists_count(n, v, ci, co, s.tile_rows, s.tile_cols, s.block_rows);
+    if (words > 0) {
+        lists = make({(int64_t)words}, at::kUInt32, bounds.device());
+        check(L.fgx_wgrad_item_lists(ptr<uint32_t>(bounds), n, v, ci, co, s.tile_rows, s.tile_cols, s.block_rows, ptr<uint32_t>(lists), as_stream(stream)));
+        c.set(key, lists);
+    } else {
+        c.set(key, py::none());
+    }
+    return lists;
+}
+
+// [Co, V, Ci] weight gradient (and with with_bias the bias gradient) from the cache's pair lists; operands dense, rows whole
+// 16-byte pieces.  sweep_fits: what fgx_conv_wgrad_sweep takes (a schedule that asks for it runs block-major otherwise).
+py::tuple wgrad(const Tensor& grad, const Tensor& feats, py::object cache_obj, int v, bool with_bias, int bias_offset, py::object sched_obj,
+                int64_t stream) {
+    const Cache c(std::move(cache_obj));
+    Sched s = read_schedule(sched_obj);
+    const at::Device dev = feats.device();
+    const c10::DeviceGuard guard(dev);
+    const int64_t n = grad.size(0), n_in = feats.size(0);
+    const int co = (int)grad.size(1), ci = (int)feats.size(1), es = (int)feats.element_size();
+    const int code = dtype_code(feats);
+    const Tensor sig_i = c.need("valid_signal_i"), sig_o = c.need("valid_signal_o");
+    const std::vector<uint32_t> seg = seg_host(c, v);
+    const int64_t pairs = seg[v];
+    if (pairs > std::min(sig_i.numel(), sig_o.numel()))
+        throw py::value_error("valid_signal_seg does not fit the pair lists (V + 1 entries, the last one their length)");
+    if (s.stream == 2) {
+        // (the checks of the C entry point: 24-bit row numbers, operands and lists within its 32-bit byte offsets)
+        const double most = (double)0xFF000000u;
+        const bool fits = n > 0 && n <= (1 << 24) && n_in <= (1 << 24) && pairs > 0 && (double)n * co * es <= most && (double)n_in * ci * es <= most &&
+                          (double)pairs * 4 + 256 <= most;
+        if (!fits) {                                    // very long operands (and empty pair lists) take the block-major kernel
+            s.stream = 1;
+            s.block_rows = 12288;
+        }
+    }
+    Tensor gw = make({co, v, ci}, feats.scalar_type(), dev), gb;
+    if (with_bias) gb = make({co}, feats.scalar_type(), dev);
+    if (s.stream == 2) {
+        const std::string key = "_wgrad_sweep_plan_" + std::to_string(s.block_rows);
+        Tensor plan;
+        if (!c.tensor(key, &plan)) {
+            plan = workspace(L.fgx_wgrad_sweep_plan_bytes((size_t)n, (size_t)pairs, v, s.block_rows), dev);
+            check(L.fgx_wgrad_sweep_plan(ptr<uint32_t>(sig_o), seg.data(), (size_t)n, v, s.block_rows, ptr(plan), (size_t)plan.numel(), as_stream(stream)));
+            c.set(key, plan);
+        }
+        Tensor scratch = workspace(L.fgx_wgrad_sweep_scratch_bytes(ci, co), dev);
+        mark("wgrad", "start");
+        check(L.fgx_conv_wgrad_sweep(code, ptr(grad), ptr(feats), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o), seg.data(), ptr(plan), (size_t)n,
+                                     (size_t)n_in, ci, co, v, s.tile_rows, s.block_rows, (int)module_int(g_impl, "WGRAD_SWEEP_LEAD"),
+                                     (int)module_int(g_impl, "WGRAD_SWEEP_MAX_POLLS"), ptr(scratch), ptr(gw), ptr(gb), bias_offset, as_stream(stream)));
+    } else {
+        const Tensor bounds = wgrad_bounds(c, sig_o, seg, (size_t)n, v, s.block_rows, stream);
+        Tensor lists;
+        if (s.stream == 1 && PyObject_IsTrue(module_get(g_impl, "WGRAD_BALANCED_LISTS"))) lists = wgrad_item_lists(c, bounds, (size_t)n, v, ci, co, s, stream);
+        Tensor scratch = workspace(L.fgx_wgrad_scratch_bytes((size_t)n, v, ci, co, s.block_rows), dev);
+        mark("wgrad", "start");
+        check(L.fgx_conv_wgrad_lists(code, ptr(grad), ptr(feats), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o), seg.data(), ptr<uint32_t>(bounds),
+                                     ptr<uint32_t>(lists), (size_t)n, (size_t)n_in, ci, co, v, s.tile_rows, s.tile_cols, s.block_rows, s.stream,
+                                     ptr(scratch), ptr(gw), ptr(gb), bias_offset, as_stream(stream)));
+    }
+    mark("wgrad", "stop");
+    return py::make_tuple(gw, gb.defined() ? py::cast(gb) : py::none());
+}
+
+Tensor relu_mask_apply(const Tensor& grad, const Tensor& mask, int64_t stream) {
+    const c10::DeviceGuard guard(grad.device());
+    const Tensor g = grad.contiguous();
+    Tensor out = at::empty_like(g);
+    check(L.fgx_relu_mask_apply(dtype_code(g), ptr(g), ptr<uint8_t>(mask), (size_t)g.numel(), ptr(out), as_stream(stream)));
+    return out;
+}
+
+Tensor colsum(const Tensor& grad, int64_t stream) {
+    const c10::DeviceGuard guard(grad.device());
+    const int64_t n = grad.size(0), co = grad.size(1);
+    Tensor out = make({co}, grad.scalar_type(), grad.device());
+    Tensor scratch = workspace(L.fgx_colsum_scratch_bytes((size_t)n, (int)co), grad.device());
+    check(L.fgx_colsum(dtype_code(grad), ptr(grad), (size_t)n, (int)co, ptr(scratch), ptr(out), as_stream(stream)));
+    return out;
+}
+
+// ---- curve codes -----------------------------------------------------------------------------------------------------
+Tensor encode(const Tensor& coords, int mode, int bits, int code_bits, int64_t stream) {
+    const c10::DeviceGuard guard(coords.device());
+    const Tensor c = coords.contiguous();
+    Tensor codes = make({c.size(0)}, code_bits == 32 ? at::kInt : at::kLong, c.device());
+    check(L.fgx_serialize_encode(mode, ptr<int32_t>(c), (size_t)c.size(0), bits, code_bits, ptr(codes), as_stream(stream)));
+    return codes;
+}
+
+Tensor decode(const Tensor& codes, int mode, int bits, int code_bits, int64_t stream) {
+    const c10::DeviceGuard guard(codes.device());
+    const Tensor c = codes.contiguous();
+    Tensor coords = make({c.size(0), 4}, at::kInt, c.device());
+    check(L.fgx_serialize_decode(mode, ptr(c), (size_t)c.size(0), bits, code_bits, ptr<int32_t>(coords), as_stream(stream)));
+    return coords;
+}
+
+// ---- the Python methods of the cache that make tables by themselves ----------------------------------------------------
+py::tuple py_tile_codes(py::object cache_obj, int block, bool own_order, int64_t stream) {
+    const Cache c(std::move(cache_obj));
+    Tiles t;
+    const c10::DeviceGuard guard(c.need("neighbor_map").device());
+    tile_codes(c, block, own_order, stream, &t, false);
+    return py::make_tuple(t.order, t.code);
+}
+
+py::tuple py_gather_plan(py::object cache_obj, int block, bool own_order, bool dense, int64_t stream) {
+    const Cache c(std::move(cache_obj));
+    const c10::DeviceGuard guard(c.need("neighbor_map").device());
+    const Tiles t = gather_plan(c, block, own_order, dense, 0, 0, 0, nullptr, stream);
+    return py::make_tuple(t.order, t.code, t.plan_seg, t.plan_idx, t.plan_band, t.plan_key);
+}
+
+py::object py_item_order(py::object cache_obj, const std::string& plan_key, const Tensor& code, int col_tiles, int groups, int slabs, int64_t stream) {
+    const Cache c(std::move(cache_obj));
+    const c10::DeviceGuard guard(code.device());
+    const Tensor t = item_order(c, plan_key, code, col_tiles, groups, slabs, stream);
+    return t.defined() ? py::cast(t) : py::none();
+}
+
+py::object py_wgrad_bounds(py::object cache_obj, int block_rows, int64_t stream) {
+    const Cache c(std::move(cache_obj));
+    const Tensor nmap = c.need("neighbor_map"), sig_o = c.need("valid_signal_o");
+    const c10::DeviceGuard guard(nmap.device());
+    const int v = (int)nmap.size(1);
+    return py::cast(wgrad_bounds(c, sig_o, seg_host(c, v), (size_t)nmap.size(0), v, block_rows, stream));
+}
+
+py::object py_wgrad_item_lists(py::object cache_obj, int block_rows, int tile_rows, int tile_cols, int ci, int co, int64_t stream) {
+    const Tensor bounds = py_wgrad_bounds(cache_obj, block_rows, stream).cast<Tensor>();
+    const Cache c(std::move(cache_obj));
+    const Tensor nmap = c.need("neighbor_map");
+    const c10::DeviceGuard guard(nmap.device());
+    const Sched s{tile_rows, tile_cols, 0, 1, block_rows, 1};
+    const Tensor t = wgrad_item_lists(c, bounds, (size_t)nmap.size(0), (int)nmap.size(1), ci, co, s, stream);
+    return t.defined() ? py::cast(t) : py::none();
+}
+
+}  // namespace
+
+PYBIND11_MODULE(fgx_host, m) {
+    py::class_<SegHost>(m, "SegHost").def("synchronize", &SegHost::synchronize).def("tolist", &SegHost::tolist);
+    m.def("bind", &bind);
+    m.def("subm_cache", &subm_cache);
+    m.def("spconv_cache", &spconv_cache);
+    m.def("out_coords", &out_coords);
+    m.def("gather_gemm", &gather_gemm);
+    m.def("wgrad", &wgrad);
+    m.def("relu_mask_apply", &relu_mask_apply);
+    m.def("colsum", &colsum);
+    m.def("encode", &encode);
+    m.def("decode", &decode);
+    m.def("tile_codes", &py_tile_codes);
+    m.def("gather_plan", &py_gather_plan);
+    m.def("item_order", &py_item_order);
+    m.def("wgrad_bounds", &py_wgrad_bounds);
+    m.def("wgrad_item_lists", &py_wgrad_item_lists);
+}

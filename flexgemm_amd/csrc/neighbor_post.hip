@@ -253,7 +253,7 @@ __global__ void __launch_bounds__(kPairThreads) pair_fill_kernel(const uint32_t*
                                                                  const int32_t* __restrict__ gray, size_t n, int V,
                                                                  unsigned nblk, const uint32_t* __restrict__ offsets,
                                                                  const uint32_t* __restrict__ totals, uint32_t* __restrict__ seg,
-                                                                 uint32_t* __restrict__ sig_i, uint32_t* __restrict__ sig_o) {
+                                                                 uint32_t* __restrict__ seg_host, uint32_t* __restrict__ sig_i, uint32_t* __restrict__ sig_o) {
     extern __shared__ uint32_t lds[];
     constexpr int kWaves = kPairThreads / 64;
     uint32_t* rows = lds;                                    // [kPairThreads * V]
@@ -263,7 +263,10 @@ __global__ void __launch_bounds__(kPairThreads) pair_fill_kernel(const uint32_t*
     if (threadIdx.x < 64) {
         const uint32_t start = pair_segment(totals, V, (int)threadIdx.x);
         if (threadIdx.x < V) first[threadIdx.x] = start + offsets[(size_t)threadIdx.x * nblk + blockIdx.x];
-        if (seg != nullptr && blockIdx.x == 0 && threadIdx.x <= V) seg[threadIdx.x] = start;
+        if (seg != nullptr && blockIdx.x == 0 && threadIdx.x <= V) {
+            seg[threadIdx.x] = start;
+            if (seg_host != nullptr) seg_host[threadIdx.x] = start;
+        }
     }
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
@@ -318,8 +321,7 @@ __global__ void __launch_bounds__(kPairThreads) pair_fill_kernel(const uint32_t*
 // One wavefront per tile: OR of gray[sorted_idx[r]] over the tile's rows.
 __global__ void __launch_bounds__(kBlock) tile_or_kernel(const int32_t* __restrict__ gray,
                                                          const int64_t* __restrict__ sorted_idx, size_t n, int block,
-                                                         size_t num_tiles, int32_t* __restrict__ tile_code,
-                                                         uint32_t* __restrict__ popc) {
+                                                         size_t num_tiles, int32_t* __restrict__ tile_code) {
     const size_t tile = ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
     const int lane = threadIdx.x & 63;
     if (tile >= num_tiles) return;   // whole wavefronts leave together
@@ -328,15 +330,7 @@ __global__ void __launch_bounds__(kBlock) tile_or_kernel(const int32_t* __restri
     uint32_t code = 0;
     for (size_t r = lo + lane; r < hi; r += 64) code |= (uint32_t)gray[sorted_idx[r]];
     for (int off = 32; off > 0; off >>= 1) code |= (uint32_t)__shfl_xor((int)code, off, 64);
-    if (lane == 0) {
-        tile_code[tile] = (int32_t)code;
-        popc[tile] = (uint32_t)__popc(code);
-    }
-}
-
-// seg[0..nb) = exclusive offsets (already there from the scan), seg[nb] = total
-__global__ void tile_seg_tail_kernel(const uint32_t* __restrict__ popc, int32_t* __restrict__ seg, size_t num_tiles) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) seg[num_tiles] = seg[num_tiles - 1] + (int32_t)popc[num_tiles - 1];
+    if (lane == 0) tile_code[tile] = (int32_t)code;
 }
 
 __global__ void set_i32_kernel(int32_t* dst, int32_t value) {
@@ -354,16 +348,6 @@ __global__ void __launch_bounds__(kBlock) tile_fill_kernel(const int32_t* __rest
         *dst++ = __ffs((int)code) - 1;
         code &= code - 1;
     }
-}
-
-// Rows of the gather plan a tile contributes: one per offset present, and one (all rows missing) for a tile
-// without any, so that every tile owns at least one step of the streaming GEMM.
-__global__ void __launch_bounds__(kBlock) plan_count_kernel(const int32_t* __restrict__ tile_code, size_t num_tiles,
-                                                            uint32_t* __restrict__ cnt) {
-    size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    if (t >= num_tiles) return;
-    const int c = __popc((uint32_t)tile_code[t]);
-    cnt[t] = (uint32_t)(c > 0 ? c : 1);
 }
 
 // One workgroup per tile: plan_idx[seg[t] + k][r] = map[order[t * tile_rows + r]][k-th offset present in the tile]
@@ -443,71 +427,77 @@ __global__ void __launch_bounds__(kBlock) plan_fill_kernel(const uint32_t* __res
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Item order of the streaming GEMM (fgx_gather_item_order): one workgroup, no host round trip.
+// The tables over all row tiles, by one workgroup: where each tile's public offset list and its gather-plan rows start, and
+// the item order of the streaming GEMM.
 // ---------------------------------------------------------------------------------------------------------------
 // Items (row tile * col_tiles + column tile) cost about max(popcount(tile_code), 1) offsets each.  Workgroup slot q of
 // `groups` works through the positions q, q + groups, ... of the sequence written here.  Step 1 sorts the items by
-// cost, most expensive first (stable counting sort over the 33 possible popcounts: per-thread counts of a contiguous
-// chunk, one scan, one placement pass).  Step 2 deals them round by round: the incomplete last round takes the
-// cheapest items, every full round gives its most expensive item to the least loaded slot (rank of each slot's load by
-// counting).  Everything is deterministic.
+// cost, most expensive first (stable counting sort over the 33 possible popcounts: a wavefront counts, then places, a
+// contiguous piece 64 items at a time, equal costs found by ballots).  Step 2 deals them round by round: the incomplete
+// last round takes the cheapest items, every full round gives its most expensive item to the least loaded slot (rank of
+// each slot's load by counting).  Everything is deterministic.  One workgroup, so what bounds it is the length of its
+// dependent chains: the counting sort by one thread per piece with serial prefixes over 256 of them, and the ranks one
+// load at a time, took 0.040 ms for 1 306 items and 256 slots; this form and the two scans together 0.014.
 constexpr int kOrderThreads = 1024;     // also the largest number of slots
-constexpr int kCostBins = 33;
+constexpr int kOrderWaves = kOrderThreads / 64;
 
-__global__ void __launch_bounds__(kOrderThreads) item_order_kernel(const int32_t* __restrict__ tile_code, unsigned num_tiles,
-                                                                   unsigned col_tiles, unsigned slabs, unsigned groups,
-                                                                   uint32_t* __restrict__ sorted, uint32_t* __restrict__ item_at) {
-    __shared__ uint32_t count[kCostBins][kOrderThreads / 4];     // [bin][chunk owner]; 256 owners
-    __shared__ uint32_t bin_start[kCostBins];
-    __shared__ uint32_t load[kOrderThreads];
-    constexpr unsigned kOwners = kOrderThreads / 4;
-    const unsigned tid = threadIdx.x;
+__device__ __forceinline__ unsigned tile_cost_bin(uint32_t code) { return 32u - (unsigned)__popc(code); }   // 0 = most expensive
+
+__device__ void order_items(const int32_t* __restrict__ tile_code, unsigned num_tiles, unsigned col_tiles, unsigned slabs, unsigned groups,
+                            uint32_t* __restrict__ sorted, uint32_t* __restrict__ item_at) {
+    __shared__ uint32_t count[kOrderWaves][64];
+    __shared__ __attribute__((aligned(16))) uint32_t load[kOrderThreads];
+    const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const unsigned total = num_tiles * col_tiles;
-    auto bin_of = [&](unsigned item) -> unsigned {                // bin 0 = most expensive
-        const unsigned pc = (unsigned)__popc((uint32_t)tile_code[item / col_tiles]);
-        return 32u - pc;
-    };
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const unsigned piece = ((total + kOrderWaves - 1) / kOrderWaves + 63u) & ~63u;
+    const unsigned lo = wave * piece < total ? wave * piece : total, hi = lo + piece < total ? lo + piece : total;
+    auto bin_of = [&](unsigned item) -> unsigned { return tile_cost_bin((uint32_t)tile_code[col_tiles == 1 ? item : item / col_tiles]); };
     // ---- step 1: stable counting sort, cost descending ----
-    for (unsigned i = tid; i < kCostBins * kOwners; i += kOrderThreads) (&count[0][0])[i] = 0u;
-    __syncthreads();
-    const unsigned chunk = (total + kOwners - 1) / kOwners;
-    if (tid < kOwners) {
-        const unsigned lo = tid * chunk, hi = lo + chunk < total ? lo + chunk : total;
-        for (unsigned i = lo; i < hi; ++i) ++count[bin_of(i)][tid];
+    count[wave][lane] = 0u;
+    for (unsigned i0 = lo; i0 < hi; i0 += 64) {                   // (one wavefront: its LDS accesses stay in order)
+        const bool live = i0 + lane < hi;
+        const unsigned bin = live ? bin_of(i0 + lane) : 0u;
+        const unsigned long long peers = radix_peers(bin, 6, live);
+        if (live && lane == (unsigned)(__ffsll((long long)peers) - 1)) count[wave][bin] += (uint32_t)__popcll(peers);
     }
     __syncthreads();
-    if (tid < kCostBins) {                                        // per bin: exclusive prefix over the owners, total left in bin_start
-        uint32_t run = 0;
-        for (unsigned o = 0; o < kOwners; ++o) {
-            const uint32_t c = count[tid][o];
-            count[tid][o] = run;
-            run += c;
+    if (wave == 0) {                                              // lane = bin
+        uint32_t mine = 0u, before[kOrderWaves];
+#pragma unroll
+        for (int w = 0; w < kOrderWaves; ++w) {
+            before[w] = mine;
+            mine += count[w][lane];
         }
-        bin_start[tid] = run;
+        uint32_t incl = mine;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = (uint32_t)__shfl_up((int)incl, d, 64);
+            if ((int)lane >= d) incl += o;
+        }
+#pragma unroll
+        for (int w = 0; w < kOrderWaves; ++w) count[w][lane] = incl - mine + before[w];
     }
     __syncthreads();
-    if (tid == 0) {
-        uint32_t run = 0;
-        for (int b = 0; b < kCostBins; ++b) {
-            const uint32_t c = bin_start[b];
-            bin_start[b] = run;
-            run += c;
+    for (unsigned i0 = lo; i0 < hi; i0 += 64) {
+        const bool live = i0 + lane < hi;
+        const unsigned bin = live ? bin_of(i0 + lane) : 0u;
+        const unsigned long long peers = radix_peers(bin, 6, live);
+        const int leader = live ? __ffsll((long long)peers) - 1 : 0;
+        uint32_t first = 0u;
+        if (live && (int)lane == leader) {
+            first = count[wave][bin];
+            count[wave][bin] = first + (uint32_t)__popcll(peers);
         }
-    }
-    __syncthreads();
-    if (tid < kOwners) {
-        const unsigned lo = tid * chunk, hi = lo + chunk < total ? lo + chunk : total;
-        for (unsigned i = lo; i < hi; ++i) {
-            const unsigned b = bin_of(i);
-            sorted[bin_start[b] + count[b][tid]++] = i;
-        }
+        first = (uint32_t)__shfl((int)first, leader, 64);
+        if (live) sorted[first + (uint32_t)__popcll(peers & below)] = i0 + lane;
     }
     __threadfence_block();
     __syncthreads();
     // ---- step 2: deal the rounds ----
     const unsigned rounds = total / groups, rem = total % groups;
     auto cost_of = [&](unsigned item) -> uint32_t {
-        const unsigned pc = (unsigned)__popc((uint32_t)tile_code[item / col_tiles]);
+        const unsigned pc = 32u - bin_of(item);
         return (pc ? pc : 1u) * slabs + 3u;
     };
     uint32_t mine = 0;
@@ -516,14 +506,21 @@ __global__ void __launch_bounds__(kOrderThreads) item_order_kernel(const int32_t
         item_at[rounds * groups + tid] = item;
         mine = cost_of(item);
     }
+    const unsigned quads = (groups + 3u) / 4u;
     for (unsigned r = 0; r < rounds; ++r) {
-        if (tid < groups) load[tid] = mine;
+        load[tid] = tid < groups ? mine : 0xFFFFFFFFu;
         __syncthreads();
         if (tid < groups) {
-            unsigned rank = 0;                                    // slots with a smaller load come first, ties by slot number
-            for (unsigned q = 0; q < groups; ++q) {
-                const uint32_t other = load[q];
-                rank += (other < mine || (other == mine && q < tid)) ? 1u : 0u;
+            // slots with a smaller load come first, ties by slot number
+            unsigned rank = 0;
+            const uint4* load4 = reinterpret_cast<const uint4*>(load);
+#pragma unroll 8
+            for (unsigned q = 0; q < quads; ++q) {
+                const uint4 o = load4[q];
+                rank += (o.x < mine || (o.x == mine && 4 * q < tid)) ? 1u : 0u;
+                rank += (o.y < mine || (o.y == mine && 4 * q + 1 < tid)) ? 1u : 0u;
+                rank += (o.z < mine || (o.z == mine && 4 * q + 2 < tid)) ? 1u : 0u;
+                rank += (o.w < mine || (o.w == mine && 4 * q + 3 < tid)) ? 1u : 0u;
             }
             const unsigned item = sorted[r * groups + rank];      // rank 0 = least loaded slot <- most expensive item
             item_at[r * groups + tid] = item;
@@ -533,11 +530,36 @@ __global__ void __launch_bounds__(kOrderThreads) item_order_kernel(const int32_t
     }
 }
 
-size_t scan_temp_bytes(size_t count) {
-    size_t bytes = 0;
-    (void)rocprim::exclusive_scan(nullptr, bytes, (const uint32_t*)nullptr, (uint32_t*)nullptr, 0u, count ? count : 1,
-                                  rocprim::plus<uint32_t>(), (hipStream_t)0);
-    return bytes;
+// seg (optional): exclusive offsets of the tiles' public offset lists, plan_seg (optional): of their gather-plan rows, both with
+// the total at [num_tiles]; item_at (optional): the item order, `sorted` its workspace.
+__global__ void __launch_bounds__(kOrderThreads) tile_tables_kernel(const int32_t* __restrict__ tile_code, unsigned num_tiles,
+                                                                    int32_t* __restrict__ seg, int32_t* __restrict__ plan_seg,
+                                                                    unsigned col_tiles, unsigned slabs, unsigned groups,
+                                                                    uint32_t* __restrict__ sorted, uint32_t* __restrict__ item_at) {
+    __shared__ uint32_t part[kOrderWaves];
+    uint32_t at = 0u, plan_at = 0u;
+    if (seg != nullptr || plan_seg != nullptr) {
+        for (unsigned t0 = 0; t0 < num_tiles; t0 += kOrderThreads) {         // (uniform)
+            const unsigned t = t0 + threadIdx.x;
+            const uint32_t c = t < num_tiles ? (uint32_t)__popc((uint32_t)tile_code[t]) : 0u;
+            uint32_t all;
+            const uint32_t before = block_exclusive_sum<kOrderWaves>(c, part, &all);
+            // a tile without any offset has one plan row (all rows missing): every tile owns at least one step of the GEMM
+            uint32_t bare_all;
+            const uint32_t bare = block_exclusive_sum<kOrderWaves>(t < num_tiles && c == 0u ? 1u : 0u, part, &bare_all);
+            if (t < num_tiles) {
+                if (seg != nullptr) seg[t] = (int32_t)(at + before);
+                if (plan_seg != nullptr) plan_seg[t] = (int32_t)(plan_at + before + bare);
+            }
+            at += all;
+            plan_at += all + bare_all;
+        }
+        if (threadIdx.x == 0) {
+            if (seg != nullptr) seg[num_tiles] = (int32_t)at;
+            if (plan_seg != nullptr) plan_seg[num_tiles] = (int32_t)plan_at;
+        }
+    }
+    if (item_at != nullptr) order_items(tile_code, num_tiles, col_tiles, slabs, groups, sorted, item_at);
 }
 
 struct PairLayout {
@@ -558,27 +580,12 @@ PairLayout pair_layout(size_t n, int V) {
 }
 
 int pair_fill_launch(const uint32_t* map, const int32_t* gray, size_t n, int V, const uint32_t* offsets, const uint32_t* totals, uint32_t* seg,
-                     uint32_t* sig_i, uint32_t* sig_o, hipStream_t s) {
+                     uint32_t* seg_host, uint32_t* sig_i, uint32_t* sig_o, hipStream_t s) {
     const size_t lds = ((size_t)kPairThreads * V + 2 * (kPairThreads / 64) * 32 + 32) * sizeof(uint32_t);
     const unsigned nblk = cdiv(n, kPairRows);
-    pair_fill_kernel<<<nblk, kPairThreads, lds, s>>>(map, gray, n, V, nblk, offsets, totals, seg, sig_i, sig_o);
+    pair_fill_kernel<<<nblk, kPairThreads, lds, s>>>(map, gray, n, V, nblk, offsets, totals, seg, seg_host, sig_i, sig_o);
     FGX_CHECK_LAUNCH("fgx_pair_fill");
     return FGX_OK;
-}
-
-struct TileLayout {
-    size_t num_tiles, popc, temp, temp_bytes, total;
-};
-
-TileLayout tile_layout(size_t n, int block) {
-    TileLayout L{};
-    L.num_tiles = (n + block - 1) / block;
-    size_t off = 0;
-    L.popc = off; off = align_up(off + (L.num_tiles ? L.num_tiles : 1) * 4, 256);
-    L.temp_bytes = scan_temp_bytes(L.num_tiles);
-    L.temp = off; off = align_up(off + L.temp_bytes, 256);
-    L.total = off;
-    return L;
 }
 
 // Rows ranked along the Z-order curve (batch index above 3 * bits interleaved coordinate bits): a radix sort over the key
@@ -625,13 +632,14 @@ int pair_counts(const int32_t* gray, size_t n, int V, uint32_t* counts, hipStrea
 }
 
 int pair_lists_from_counts(const uint32_t* map, const int32_t* gray, size_t n, int V, const uint32_t* counts, size_t m, bool sub,
-                           uint32_t* offsets, uint32_t* totals, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, hipStream_t s) {
+                           uint32_t* offsets, uint32_t* totals, uint32_t* seg, uint32_t* seg_host, uint32_t* sig_i, uint32_t* sig_o,
+                           hipStream_t s) {
     const unsigned nblk = cdiv(n, kPairRows);
     phase_mark("pair fill", s);
     if (sub) pair_scan_kernel<kPairRows / kPairSubRows><<<V, 256, 0, s>>>(counts, m, nblk, offsets, totals);
     else pair_scan_kernel<1><<<V, 256, 0, s>>>(counts, m, nblk, offsets, totals);
     FGX_CHECK_LAUNCH("fgx_pair_count(scan)");
-    return pair_fill_launch(map, gray, n, V, offsets, totals, seg, sig_i, sig_o, s);
+    return pair_fill_launch(map, gray, n, V, offsets, totals, seg, seg_host, sig_i, sig_o, s);
 }
 
 }  // namespace fgx
@@ -779,37 +787,62 @@ int fgx_pair_fill(const uint32_t* map, const int32_t* gray, size_t n, int V, con
     const char* ws = (const char*)workspace;
     PhaseEnd phases{(hipStream_t)stream};
     phase_mark("pair fill", (hipStream_t)stream);
-    return pair_fill_launch(map, gray, n, V, (const uint32_t*)(ws + L.offsets), (const uint32_t*)(ws + L.totals), nullptr, sig_i, sig_o,
+    return pair_fill_launch(map, gray, n, V, (const uint32_t*)(ws + L.offsets), (const uint32_t*)(ws + L.totals), nullptr, nullptr, sig_i, sig_o,
                             (hipStream_t)stream);
 }
 
-size_t fgx_tile_workspace_bytes(size_t n, int block) { return tile_layout(n, block > 0 ? block : 1).total; }
+size_t fgx_tile_workspace_bytes(size_t n, int block) {
+    (void)n;
+    (void)block;
+    return 256;         // (the scans need none any more)
+}
 
 int fgx_tile_codes(const int32_t* gray, const int64_t* sorted_idx, size_t n, int block, int32_t* tile_code,
                    int32_t* seg, void* workspace, size_t workspace_bytes, fgx_stream_t stream) {
+    (void)workspace;
+    (void)workspace_bytes;
     FGX_CHECK_ARG(block >= 1, "fgx_tile_codes: tile size must be >= 1, got %d", block);
     FGX_CHECK_ARG(seg != nullptr, "fgx_tile_codes: null segment table");
+    return fgx_tile_plan(gray, sorted_idx, nullptr, n, 1, block, 0, tile_code, seg, nullptr, nullptr, nullptr, 1, 1, 1, nullptr, nullptr, stream);
+}
+
+int fgx_tile_plan(const int32_t* gray, const int64_t* order, const uint32_t* map, size_t n, int V, int tile_rows, int have_codes,
+                  int32_t* tile_code, int32_t* seg, int32_t* plan_seg, uint32_t* plan_idx, uint32_t* plan_band, int col_tiles, int slabs,
+                  int groups, uint32_t* item_ws, uint32_t* item_at, fgx_stream_t stream) {
+    FGX_CHECK_ARG(tile_rows >= 1 && V >= 1 && V <= 32, "fgx_tile_plan: bad shape tile_rows=%d V=%d", tile_rows, V);
     hipStream_t s = (hipStream_t)stream;
-    TileLayout L = tile_layout(n, block);
-    if (L.num_tiles == 0) {
-        set_i32_kernel<<<1, 64, 0, s>>>(seg, 0);
-        FGX_CHECK_LAUNCH("fgx_tile_codes(empty)");
+    const size_t num_tiles = (n + tile_rows - 1) / tile_rows;
+    FGX_CHECK_ARG(num_tiles <= 0x3FFFFFFu, "fgx_tile_plan: too many tiles");
+    PhaseEnd phases{s};
+    phase_mark("tile tables", s);
+    if (n == 0) {
+        for (int32_t* table : {seg, plan_seg})
+            if (table != nullptr) set_i32_kernel<<<1, 64, 0, s>>>(table, 0);
+        FGX_CHECK_LAUNCH("fgx_tile_plan(empty)");
         return FGX_OK;
     }
-    FGX_CHECK_ARG(gray && sorted_idx && tile_code && workspace, "fgx_tile_codes: null buffer");
-    FGX_CHECK_ARG(workspace_bytes >= L.total, "fgx_tile_codes: workspace of %zu bytes, need %zu", workspace_bytes, L.total);
-    FGX_CHECK_ARG(((uintptr_t)workspace & 255) == 0, "fgx_tile_codes: workspace must be 256-byte aligned");
-    char* ws = (char*)workspace;
-    uint32_t* popc = (uint32_t*)(ws + L.popc);
-    PhaseEnd phases{s};
-    phase_mark("tile masks", s);
-    tile_or_kernel<<<cdiv(L.num_tiles * 64, kBlock), kBlock, 0, s>>>(gray, sorted_idx, n, block, L.num_tiles, tile_code, popc);
-    FGX_CHECK_LAUNCH("fgx_tile_codes(or)");
-    size_t temp_bytes = L.temp_bytes;
-    FGX_CHECK_HIP(rocprim::exclusive_scan(ws + L.temp, temp_bytes, popc, (uint32_t*)seg, 0u, L.num_tiles,
-                                          rocprim::plus<uint32_t>(), s));
-    tile_seg_tail_kernel<<<1, 64, 0, s>>>(popc, seg, L.num_tiles);
-    FGX_CHECK_LAUNCH("fgx_tile_codes(tail)");
+    FGX_CHECK_ARG(tile_code && (have_codes || (gray && order)), "fgx_tile_plan: null buffer");
+    FGX_CHECK_ARG(plan_idx == nullptr || (map && order && plan_seg), "fgx_tile_plan: a gather plan needs the map, the order and its segment table");
+    FGX_CHECK_ARG(plan_band == nullptr || (plan_idx != nullptr && tile_rows <= 1024), "fgx_tile_plan: band masks need a plan and tile_rows <= 1024");
+    if (item_at != nullptr) {
+        FGX_CHECK_ARG(col_tiles >= 1 && slabs >= 1 && groups >= 1 && groups <= kOrderThreads && item_ws != nullptr,
+                      "fgx_tile_plan: bad item order col_tiles=%d slabs=%d groups=%d", col_tiles, slabs, groups);
+        FGX_CHECK_ARG(num_tiles * (size_t)col_tiles < 0x7FFFFFFFull, "fgx_tile_plan: too many items");
+    }
+    if (!have_codes) {
+        tile_or_kernel<<<cdiv(num_tiles * 64, kBlock), kBlock, 0, s>>>(gray, order, n, tile_rows, num_tiles, tile_code);
+        FGX_CHECK_LAUNCH("fgx_tile_plan(or)");
+    }
+    if (seg != nullptr || plan_seg != nullptr || item_at != nullptr) {
+        tile_tables_kernel<<<1, kOrderThreads, 0, s>>>(tile_code, (unsigned)num_tiles, seg, plan_seg, (unsigned)col_tiles, (unsigned)slabs,
+                                                       (unsigned)groups, item_ws, item_at);
+        FGX_CHECK_LAUNCH("fgx_tile_plan(tables)");
+    }
+    if (plan_idx != nullptr) {
+        phase_mark("gather plan fill", s);
+        plan_fill_kernel<<<(unsigned)num_tiles, kBlock, 0, s>>>(map, order, tile_code, plan_seg, n, V, tile_rows, plan_idx, plan_band);
+        FGX_CHECK_LAUNCH("fgx_tile_plan(plan)");
+    }
     return FGX_OK;
 }
 
@@ -824,29 +857,12 @@ int fgx_tile_fill(const int32_t* tile_code, const int32_t* seg, size_t num_tiles
 
 int fgx_gather_plan_count(const int32_t* tile_code, size_t num_tiles, int32_t* plan_seg, void* workspace,
                           size_t workspace_bytes, fgx_stream_t stream) {
+    (void)workspace;
+    (void)workspace_bytes;
     FGX_CHECK_ARG(plan_seg != nullptr, "fgx_gather_plan_count: null segment table");
-    hipStream_t s = (hipStream_t)stream;
-    if (num_tiles == 0) {
-        set_i32_kernel<<<1, 64, 0, s>>>(plan_seg, 0);
-        FGX_CHECK_LAUNCH("fgx_gather_plan_count(empty)");
-        return FGX_OK;
-    }
-    TileLayout L = tile_layout(num_tiles, 1);
-    FGX_CHECK_ARG(tile_code && workspace, "fgx_gather_plan_count: null buffer");
-    FGX_CHECK_ARG(workspace_bytes >= L.total, "fgx_gather_plan_count: workspace of %zu bytes, need %zu", workspace_bytes, L.total);
-    FGX_CHECK_ARG(((uintptr_t)workspace & 255) == 0, "fgx_gather_plan_count: workspace must be 256-byte aligned");
-    unsigned char* ws = (unsigned char*)workspace;
-    uint32_t* cnt = (uint32_t*)(ws + L.popc);
-    PhaseEnd phases{s};
-    phase_mark("gather plan count", s);
-    plan_count_kernel<<<cdiv(num_tiles, kBlock), kBlock, 0, s>>>(tile_code, num_tiles, cnt);
-    FGX_CHECK_LAUNCH("fgx_gather_plan_count(count)");
-    size_t temp_bytes = L.temp_bytes;
-    FGX_CHECK_HIP(rocprim::exclusive_scan(ws + L.temp, temp_bytes, cnt, (uint32_t*)plan_seg, 0u, num_tiles,
-                                          rocprim::plus<uint32_t>(), s));
-    tile_seg_tail_kernel<<<1, 64, 0, s>>>(cnt, plan_seg, num_tiles);
-    FGX_CHECK_LAUNCH("fgx_gather_plan_count(tail)");
-    return FGX_OK;
+    // (tiles of one row: as many tiles as rows)
+    return fgx_tile_plan(nullptr, nullptr, nullptr, num_tiles, 1, 1, 1, const_cast<int32_t*>(tile_code), nullptr, plan_seg, nullptr, nullptr, 1,
+                         1, 1, nullptr, nullptr, stream);
 }
 
 int fgx_gather_plan_fill(const uint32_t* map, const int64_t* order, const int32_t* tile_code, const int32_t* plan_seg,
@@ -882,8 +898,8 @@ int fgx_gather_item_order(const int32_t* tile_code, size_t num_tiles, int col_ti
     FGX_CHECK_ARG(workspace_bytes >= fgx_gather_item_order_workspace_bytes(num_tiles, col_tiles),
                   "fgx_gather_item_order: workspace of %zu bytes is too small", workspace_bytes);
     FGX_CHECK_ARG(((uintptr_t)workspace & 255) == 0, "fgx_gather_item_order: workspace must be 256-byte aligned");
-    item_order_kernel<<<1, kOrderThreads, 0, (hipStream_t)stream>>>(tile_code, (unsigned)num_tiles, (unsigned)col_tiles,
-                                                                    (unsigned)slabs, (unsigned)groups, (uint32_t*)workspace, item_at);
+    tile_tables_kernel<<<1, kOrderThreads, 0, (hipStream_t)stream>>>(tile_code, (unsigned)num_tiles, nullptr, nullptr, (unsigned)col_tiles,
+                                                                     (unsigned)slabs, (unsigned)groups, (uint32_t*)workspace, item_at);
     FGX_CHECK_LAUNCH("fgx_gather_item_order");
     return FGX_OK;
 }

@@ -37,20 +37,15 @@ def encode_seq(coords: torch.Tensor, shape: torch.Size, mode: Literal["z_order",
     bit_length = _bit_length(shape)
     total_bit_length = (int(shape[0]) - 1).bit_length() + 3 * bit_length
     if total_bit_length <= 32:
-        dtype, code_bits = torch.int32, 32
+        code_bits = 32
     elif total_bit_length <= 64:
-        dtype, code_bits = torch.int64, 64
+        code_bits = 64
     else:
         raise ValueError(f"Spatial dimensions are too large: {shape}")
     if not coords.is_cuda:
         raise NotImplementedError("encode_seq runs on the GPU only: move coords to the device")
     assert coords.dtype == torch.int32, "Unsupported coords dtype. Expect int32"
-    coords = coords.contiguous()
-    codes = torch.empty(coords.shape[0], dtype=dtype, device=coords.device)
-    with torch.cuda.device(coords.device):
-        nat.check(nat.lib().fgx_serialize_encode(C.c_int(code), nat.ptr(coords), nat.sz(coords.shape[0]), C.c_int(bit_length),
-                                                 C.c_int(code_bits), nat.ptr(codes), nat.stream()))
-    return codes
+    return nat.host().encode(coords, code, bit_length, code_bits, nat.raw_stream(coords))
 
 
 def decode_seq(code: torch.Tensor, shape: torch.Size, mode: Literal["z_order", "hilbert"] = "z_order") -> torch.Tensor:
@@ -66,12 +61,7 @@ def decode_seq(code: torch.Tensor, shape: torch.Size, mode: Literal["z_order", "
         raise RuntimeError("Unsupported input type")
     if not code.is_cuda:
         raise NotImplementedError("decode_seq runs on the GPU only: move the codes to the device")
-    code = code.contiguous()
-    coords = torch.empty((code.shape[0], 4), dtype=torch.int32, device=code.device)
-    with torch.cuda.device(code.device):
-        nat.check(nat.lib().fgx_serialize_decode(C.c_int(mode_code), nat.ptr(code), nat.sz(code.shape[0]), C.c_int(bit_length),
-                                                 C.c_int(code_bits), nat.ptr(coords), nat.stream()))
-    return coords
+    return nat.host().decode(code, mode_code, bit_length, code_bits, nat.raw_stream(code))
 
 
 def reorder_coords(coords: torch.Tensor, bit_length: int, batch_bits: int, mode_code: int) -> torch.Tensor:

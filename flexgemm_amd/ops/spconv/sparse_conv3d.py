@@ -97,39 +97,11 @@ def _maps_builder(m: int, l: int, v: int, shape, ks, st, pd, dl, with_bwd: bool)
 def _build_cache_one_call(coords: torch.Tensor, out_coords: torch.Tensor, shape, ks, st, pd, dl, needs_grad: bool, bwd_order: bool):
     """The masked algorithms' tables through fgx_spconv_cache_build_grid, every buffer allocated beforehand: a dict of them,
     or None where the step-by-step path runs (no grid index, nothing to convolve, pair lists too large for their bound)."""
-    m, l = coords.shape[0], out_coords.shape[0]
-    v = ks[0] * ks[1] * ks[2]
-    if m == 0 or l == 0 or l * v >= 0xFFFFFFFF or (needs_grad and l * v * 8 > PAIR_LISTS_UNSIZED_MAX_BYTES):
-        return None
-    if _maps_builder(m, l, v, shape, ks, st, pd, dl, needs_grad) != "grid":
+    if spconv.NEIGHBOR_MAP_BUILDER not in ("auto", "grid"):
         return None
     B, _, W, H, D = [int(s) for s in shape]
-    dims = [C.c_int(x) for x in (B, W, H, D)]
-    out_dims = [C.c_int(x) for x in _out_dims(shape, ks, st, pd, dl)]
-    dev = coords.device
-    with torch.cuda.device(dev):
-        L = nat.lib()
-        t = {"nmap": torch.empty((l, v), dtype=torch.uint32, device=dev), "gray": torch.empty((l,), dtype=torch.int32, device=dev),
-             "binary": torch.empty((l,), dtype=torch.int32, device=dev), "order": torch.empty((l,), dtype=torch.int64, device=dev)}
-        if needs_grad:
-            t.update(nmap_bwd=torch.empty((m, v), dtype=torch.uint32, device=dev), seg=torch.empty((v + 1,), dtype=torch.uint32, device=dev),
-                     sig_i=torch.empty((l * v,), dtype=torch.uint32, device=dev), sig_o=torch.empty((l * v,), dtype=torch.uint32, device=dev))
-            if bwd_order:
-                t.update(gray_bwd=torch.empty((m,), dtype=torch.int32, device=dev), order_bwd=torch.empty((m,), dtype=torch.int64, device=dev))
-        ws = nat.workspace(L.fgx_spconv_cache_grid_workspace_bytes(nat.sz(m), nat.sz(l), *dims, *out_dims, C.c_int(v), C.c_int(int(needs_grad)),
-                                                                   C.c_int(int("order_bwd" in t))), dev)
-        nat.check(L.fgx_spconv_cache_build_grid(
-            nat.ptr(coords), nat.sz(m), nat.ptr(out_coords), nat.sz(l), *dims, *[C.c_int(x) for x in (*ks, *st, *pd, *dl)],
-            nat.ptr(ws), nat.sz(ws.numel()),
-            *[nat.ptr(t.get(k)) for k in ("nmap", "gray", "binary", "order", "nmap_bwd", "seg", "sig_i", "sig_o", "gray_bwd", "order_bwd")],
-            nat.stream()))
-        if needs_grad:
-            seg_pinned = torch.empty((v + 1,), dtype=torch.int32, pin_memory=True)
-            seg_pinned.copy_(t["seg"].view(torch.int32), non_blocking=True)
-            arrived = torch.cuda.Event()
-            arrived.record()
-            t["pairs"] = {"seg": t["seg"], "pending": (t["sig_i"], t["sig_o"], seg_pinned, arrived)}
-    return t
+    return nat.host().spconv_cache(coords, out_coords, [B, W, H, D, *ks, *st, *pd, *dl], needs_grad, bwd_order, PAIR_LISTS_UNSIZED_MAX_BYTES,
+                                   nat.raw_stream(coords))
 
 
 def _build_maps(coords: torch.Tensor, out_coords: torch.Tensor, shape, kernel_size, stride, padding, dilation,
@@ -233,18 +205,10 @@ class SparseConv3dFunction(Function):
         if vol >= 2 ** 64 - 1:
             raise ValueError("The spatial size is too large. Require B*W*H*D < 2^64.")
         L = nat.lib()
-        geom = [C.c_int(x) for x in (B, W, H, D, *ks, *st, *pd, *dl)]
-        if m * v < 1 << 30 and spconv.NEIGHBOR_MAP_BUILDER in ("auto", "grid") and L.fgx_grid_index_pays(nat.sz(m), *[C.c_int(x) for x in (B, wo, ho, do)]):
-            out_dims = [C.c_int(x) for x in (B, wo, ho, do)]
-            with torch.cuda.device(dev):
-                ws = nat.workspace(L.fgx_spconv_out_coords_grid_workspace_bytes(*out_dims), dev)
-                count = torch.empty((1,), dtype=torch.int64, device=dev)
-                nat.check(L.fgx_spconv_out_coords_grid_count(nat.ptr(coords), nat.sz(m), *geom, nat.ptr(ws), nat.sz(ws.numel()), nat.ptr(count),
-                                                             nat.stream()))
-                total = int(count.item())      # the one host sync: sizes the result
-                out = torch.empty((total, 4), dtype=torch.int32, device=dev)
-                nat.check(L.fgx_spconv_out_coords_grid_emit(nat.ptr(ws), *out_dims, nat.sz(total), nat.ptr(out), nat.stream()))
-            return SparseConv3dFunction._serialized(out, mode, (B, W, H, D), (wo, ho, do))
+        if spconv.NEIGHBOR_MAP_BUILDER in ("auto", "grid") and not torch.cuda.is_current_stream_capturing():
+            out = nat.host().out_coords(coords, [B, W, H, D, *ks, *st, *pd, *dl], nat.raw_stream(coords))
+            if out is not None:
+                return SparseConv3dFunction._serialized(out, mode, (B, W, H, D), (wo, ho, do))
         key_bits = 32 if vol < 2 ** 32 - 1 else 64
         with torch.cuda.device(dev):
             ws = nat.workspace(L.fgx_spconv_out_coords_workspace_bytes(nat.sz(m), C.c_int(v), C.c_int(key_bits)), dev)
@@ -331,7 +295,8 @@ class SparseConv3dFunction(Function):
             cache = SparseConv3dNeighborCache(neighbor_map=t["nmap"], neighbor_map_bwd=t.get("nmap_bwd"), gray_code=t["gray"],
                                               sorted_idx=t["order"], _n_in=coords.shape[0])
             if needs_grad:
-                cache._attach_pairs(t["pairs"])
+                seg, (sig_i, sig_o, arriving) = t["pairs"]["seg"], t["pairs"]["pending"]
+                cache._attach_pairs({"seg": seg, "pending": (sig_i, sig_o, arriving, arriving)})
                 if irregular:
                     cache["gray_code_bwd"], cache["sorted_idx_bwd"] = t["gray_bwd"], t["order_bwd"]
             return cache

@@ -79,7 +79,7 @@ class SubMConv3dNeighborCache:
     def _finish_pairs(self):
         buf_i, buf_o, seg_pinned, arrived = self.__dict__.pop("_pending_pairs")
         arrived.synchronize()
-        seg_host = [x & 0xFFFFFFFF for x in seg_pinned.tolist()]
+        seg_host = [x & 0xFFFFFFFF for x in seg_pinned.tolist()]    # (int32 words, or the numbers of a native block)
         total = seg_host[-1]
         self["valid_signal_i"], self["valid_signal_o"] = buf_i[:total], buf_o[:total]
         self["_valid_signal_seg_host"] = seg_host
@@ -94,24 +94,15 @@ class SubMConv3dNeighborCache:
         if private:
             self._ensure_tile_order()
         use_private = private and hasattr(self, "_tile_order")
-        order = self["_tile_order"] if use_private else self["sorted_idx"]
-        key = f"_tile_code_{block_size}" if use_private else f"_mask_code_{block_size}"
+        order, code = nat.host().tile_codes(self, block_size, use_private, nat.raw_stream(self["gray_code"]))
         seg_key = f"_tile_seg_{block_size}" if use_private else f"valid_kernel_seg_{block_size}"
-        if not hasattr(self, key):
-            gray = self["gray_code"]
-            n = gray.shape[0]
-            nb = (n + block_size - 1) // block_size
-            code = torch.empty((nb,), dtype=torch.int32, device=gray.device)
-            seg = torch.empty((nb + 1,), dtype=torch.int32, device=gray.device)
-            with torch.cuda.device(gray.device):
-                L = nat.lib()
-                ws_bytes = L.fgx_tile_workspace_bytes(nat.sz(n), C.c_int(block_size))
-                ws = nat.workspace(ws_bytes, gray.device)
-                nat.check(L.fgx_tile_codes(nat.ptr(gray), nat.ptr(order), nat.sz(n), C.c_int(block_size),
-                                           nat.ptr(code), nat.ptr(seg), nat.ptr(ws), nat.sz(ws.numel()), nat.stream()))
-            setattr(self, key, code)
+        if not hasattr(self, seg_key):
+            seg = torch.empty((code.shape[0] + 1,), dtype=torch.int32, device=code.device)
+            with torch.cuda.device(code.device):
+                nat.check(nat.lib().fgx_tile_plan(None, None, None, nat.sz(code.shape[0]), C.c_int(1), C.c_int(1), C.c_int(1), nat.ptr(code),
+                                                  nat.ptr(seg), None, None, None, C.c_int(1), C.c_int(1), C.c_int(1), None, None, nat.stream()))
             setattr(self, seg_key, seg)
-        return order, getattr(self, key), getattr(self, seg_key)
+        return order, code, getattr(self, seg_key)
 
     def _dense_tile_tables(self, block_size: int):
         """(order, tile_code) of the non-masked schedule (reference: ..._fwd_implicit_gemm.py:18-89): rows in their
@@ -134,65 +125,15 @@ class SubMConv3dNeighborCache:
         for the streaming GEMM: per tile and offset present in it, the tile's source rows as one contiguous run and the
         mask of its 32-row bands that hold any.  Built once per tile size and kept with the cache; the lists are
         allocated at their bound (every offset present in every tile), plan_seg[-1] rows of them are used."""
-        if dense:
-            order, code = self._dense_tile_tables(block_size)
-            key = f"_plan_d_{block_size}"
-        else:
-            order, code, _ = self._tile_tables(block_size, private)
-            use_private = private and hasattr(self, "_tile_order")
-            key = f"_plan_{'t' if use_private else 'm'}_{block_size}"
-        if not hasattr(self, key):
-            nmap = self["neighbor_map"]
-            n, v = nmap.shape
-            nb = code.shape[0]
-            dev = nmap.device
-            seg = torch.empty((nb + 1,), dtype=torch.int32, device=dev)
-            with torch.cuda.device(dev):
-                L = nat.lib()
-                ws = nat.workspace(L.fgx_tile_workspace_bytes(nat.sz(nb), C.c_int(1)), dev)
-                nat.check(L.fgx_gather_plan_count(nat.ptr(code), nat.sz(nb), nat.ptr(seg), nat.ptr(ws), nat.sz(ws.numel()),
-                                                  nat.stream()))
-                rows = nb * min(v, 32)       # the bound (every offset in every tile): no wait for the exact count
-                plan_idx = torch.empty((rows, block_size), dtype=torch.uint32, device=dev)
-                plan_band = torch.empty((rows,), dtype=torch.uint32, device=dev)
-                nat.check(L.fgx_gather_plan_fill(nat.ptr(nmap), nat.ptr(order), nat.ptr(code), nat.ptr(seg), nat.sz(n),
-                                                 C.c_int(v), C.c_int(block_size), nat.ptr(plan_idx), nat.ptr(plan_band),
-                                                 nat.stream()))
-            setattr(self, key, (seg, plan_idx, plan_band))
-        return (order, code) + getattr(self, key) + (key,)
+        if private and not dense:
+            self._ensure_tile_order()
+        return nat.host().gather_plan(self, block_size, private and not dense and hasattr(self, "_tile_order"), dense,
+                                      nat.raw_stream(self["neighbor_map"]))
 
     def _item_order(self, plan_key: str, code: torch.Tensor, col_tiles: int, groups: int, slabs: int):
         """uint32 device tensor for fgx_conv_gather_gemm_stream's item_at (or None): the tiles dealt to the persistent
         workgroups by cost, built on the device (no read-back) once per plan and shape and kept with the cache."""
-        mode = spconv.GEMM_ITEM_ORDER
-        nb = code.shape[0]
-        if mode == "auto":
-            # the locality order of short-row layers lives on neighboring tiles sharing an XCD (dealing them by cost
-            # alone: 0.32 -> 0.42 ms per launch at C = 32); with rows of 512 bytes and more balance wins whatever the
-            # number of tiles (-6 % per launch at C = 256, -8 % at C = 1024); with shorter rows it wins while a workgroup
-            # has few tiles (C = 128, forward: 143 616 voxels 0.120 -> 0.101 ms, 252 392 voxels 0.179 -> 0.155, 577 592
-            # voxels 0.342 -> 0.320; 669 288 voxels, 10 rounds of items, and 1 026 536 voxels, 16 rounds: no change), and the ordering kernel takes
-            # ~3 us per round of items and neighbor cache
-            few_rounds = nb * col_tiles <= ITEM_ORDER_ANY_ROW_MAX_ROUNDS * groups
-            mode = "balanced" if (slabs >= 4 or few_rounds) and not plan_key.startswith("_plan_t_") else "default"
-        # with at most one item per workgroup there is nothing to even out; from there on the dealt order pays (forward at
-        # 64 160 voxels: C = 256, two rounds of items, 0.158 -> 0.141 ms; C = 512, four rounds, 0.550 -> 0.512 ms;
-        # 15 192 voxels C = 1024, two rounds, 0.601 -> 0.568 ms)
-        if mode == "default" or nb * col_tiles <= ITEM_ORDER_MIN_ROUNDS * groups or groups > 1024:
-            return None
-        if mode != "balanced":
-            raise ValueError(f"unknown GEMM_ITEM_ORDER {spconv.GEMM_ITEM_ORDER!r}; expected 'auto', 'balanced' or 'default'")
-        key = f"_items_{plan_key}_{col_tiles}_{groups}_{slabs}"
-        if not hasattr(self, key):
-            dev = code.device
-            item_at = torch.empty((nb * col_tiles,), dtype=torch.int32, device=dev)
-            with torch.cuda.device(dev):
-                L = nat.lib()
-                ws = nat.workspace(L.fgx_gather_item_order_workspace_bytes(nat.sz(nb), C.c_int(col_tiles)), dev)
-                nat.check(L.fgx_gather_item_order(nat.ptr(code), nat.sz(nb), C.c_int(col_tiles), C.c_int(slabs), C.c_int(groups),
-                                                  nat.ptr(ws), nat.sz(ws.numel()), nat.ptr(item_at), nat.stream()))
-            setattr(self, key, item_at)
-        return getattr(self, key)
+        return nat.host().item_order(self, plan_key, code, col_tiles, groups, slabs, nat.raw_stream(code))
 
     def compute_kernel_idx(self, block_size: int):
         """Fill `valid_kernel_{B}` / `valid_kernel_seg_{B}` (reference: submanifold_conv3d.py:20-23,
@@ -271,38 +212,12 @@ class SubMConv3dNeighborCache:
     def _wgrad_bounds(self, block_rows: int):
         """First pair of every (offset, voxel block) for wgrad's blocks of `block_rows` rows: a function of the pair lists
         alone, so it is made once per block size and kept."""
-        key = f"_wgrad_bounds_{block_rows}"
-        if not hasattr(self, key):
-            sig_o = self["valid_signal_o"]
-            n, v = self["neighbor_map"].shape
-            seg_host = self._seg_host()
-            L = nat.lib()
-            count = L.fgx_wgrad_block_bounds_count(nat.sz(n), C.c_int(v), C.c_int(block_rows))
-            bounds = torch.empty((max(int(count), 1),), dtype=torch.uint32, device=sig_o.device)
-            with torch.cuda.device(sig_o.device):
-                nat.check(L.fgx_wgrad_block_bounds(nat.ptr(sig_o), (C.c_uint32 * (v + 1))(*seg_host), nat.sz(n), C.c_int(v),
-                                                   C.c_int(block_rows), nat.ptr(bounds), nat.stream()))
-            setattr(self, key, bounds)
-        return getattr(self, key)
+        return nat.host().wgrad_bounds(self, block_rows, nat.raw_stream(self["neighbor_map"]))
 
     def _wgrad_item_lists(self, block_rows: int, tile_rows: int, tile_cols: int, ci: int, co: int):
         """Balanced work lists of the streaming weight gradient (fgx_wgrad_item_lists) for one block size, tile shape and
         channel counts, made on the device from the block table and kept; None where the library has none for the shape."""
-        key = f"_wgrad_lists_{block_rows}_{tile_rows}_{tile_cols}_{ci}_{co}"
-        if not hasattr(self, key):
-            bounds = self._wgrad_bounds(block_rows)
-            n, v = self["neighbor_map"].shape
-            L = nat.lib()
-            lists = None
-            with torch.cuda.device(bounds.device):
-                words = int(L.fgx_wgrad_item_lists_count(nat.sz(n), C.c_int(v), C.c_int(ci), C.c_int(co), C.c_int(tile_rows),
-                                                         C.c_int(tile_cols), C.c_int(block_rows)))
-                if words > 0:
-                    lists = torch.empty((words,), dtype=torch.uint32, device=bounds.device)
-                    nat.check(L.fgx_wgrad_item_lists(nat.ptr(bounds), nat.sz(n), C.c_int(v), C.c_int(ci), C.c_int(co), C.c_int(tile_rows),
-                                                     C.c_int(tile_cols), C.c_int(block_rows), nat.ptr(lists), nat.stream()))
-            setattr(self, key, lists)
-        return getattr(self, key)
+        return nat.host().wgrad_item_lists(self, block_rows, tile_rows, tile_cols, ci, co, nat.raw_stream(self["neighbor_map"]))
 
     def _wgrad_sweep_plan(self, sub_rows: int):
         """Step lists of the paced wgrad sweep (fgx_wgrad_sweep_plan): a function of the pair lists and the sub-block
@@ -539,10 +454,16 @@ def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, ne
     B, _, W, H, D = [int(s) for s in shape]
     kw, kh, kd = [int(k) for k in kernel_size]
     v = kw * kh * kd
+    if spconv.NEIGHBOR_MAP_BUILDER in ("auto", "grid"):
+        built = nat.host().subm_cache(coords, [B, W, H, D, kw, kh, kd, int(dilation[0]), int(dilation[1]), int(dilation[2])], needs_grad,
+                                      spconv.NEIGHBOR_MAP_BUILDER == "grid", PAIR_LISTS_UNSIZED_MAX_BYTES, nat.raw_stream(coords))
+        if built is not None:
+            nmap, gray, binary, order, seg, sig_i, sig_o, arriving = built
+            return nmap, gray, binary, order, ({"seg": seg, "pending": (sig_i, sig_o, arriving, arriving)} if needs_grad else None)
     builder = _pick_builder(n, v, B, (W, H, D))
     vol = B * W * H * D
     bound = n * v
-    if builder not in ("grid", "sort") or n == 0 or v > 32 or kw * kh > 128 or vol > 2 ** 63 or bound >= 0xFFFFFFFF:
+    if builder != "sort" or n == 0 or v > 32 or kw * kh > 128 or vol > 2 ** 63 or bound >= 0xFFFFFFFF:
         return None
     if needs_grad and bound * 8 > PAIR_LISTS_UNSIZED_MAX_BYTES:
         return None
@@ -561,21 +482,16 @@ def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, ne
             buf_i = torch.empty((bound,), dtype=torch.uint32, device=dev)
             buf_o = torch.empty((bound,), dtype=torch.uint32, device=dev)
         outs = [nat.ptr(t) for t in (nmap, gray, binary, order, seg, buf_i, buf_o)]
-        if builder == "grid":
-            ws = nat.workspace(L.fgx_subm_cache_grid_workspace_bytes(nat.sz(n), *geom[:4], C.c_int(v), with_pairs), dev)
-            nat.check(L.fgx_subm_cache_build_grid(nat.ptr(coords), nat.sz(n), *geom, with_pairs, nat.ptr(ws), nat.sz(ws.numel()), *outs,
-                                                  nat.stream()))
-        else:
-            key_bits = 32 if vol <= 2 ** 32 else 64
-            presorted = 2                   # (as in _build_neighbor_map)
-            if n > SORT_DECIDED_ON_DEVICE_MAX or key_bits != 32:
-                descents = torch.zeros((1,), dtype=torch.int32, device=dev)
-                nat.check(L.fgx_coords_key_order(nat.ptr(coords), nat.sz(n), C.c_int(W), C.c_int(H), C.c_int(D), nat.ptr(descents), nat.stream()))
-                presorted = 1 if int(descents.item()) == 0 else 0
-            ws = nat.workspace(L.fgx_subm_cache_workspace_bytes(nat.sz(n), C.c_int(key_bits), C.c_int(kw), C.c_int(kh), C.c_int(kd),
-                                                                with_pairs), dev)
-            nat.check(L.fgx_subm_cache_build(nat.ptr(coords), nat.sz(n), *geom, C.c_int(key_bits), C.c_int(presorted), with_pairs,
-                                             nat.ptr(ws), nat.sz(ws.numel()), *outs, nat.stream()))
+        key_bits = 32 if vol <= 2 ** 32 else 64
+        presorted = 2                       # (as in _build_neighbor_map)
+        if n > SORT_DECIDED_ON_DEVICE_MAX or key_bits != 32:
+            descents = torch.zeros((1,), dtype=torch.int32, device=dev)
+            nat.check(L.fgx_coords_key_order(nat.ptr(coords), nat.sz(n), C.c_int(W), C.c_int(H), C.c_int(D), nat.ptr(descents), nat.stream()))
+            presorted = 1 if int(descents.item()) == 0 else 0
+        ws = nat.workspace(L.fgx_subm_cache_workspace_bytes(nat.sz(n), C.c_int(key_bits), C.c_int(kw), C.c_int(kh), C.c_int(kd),
+                                                            with_pairs), dev)
+        nat.check(L.fgx_subm_cache_build(nat.ptr(coords), nat.sz(n), *geom, C.c_int(key_bits), C.c_int(presorted), with_pairs,
+                                         nat.ptr(ws), nat.sz(ws.numel()), *outs, nat.stream()))
         pairs = None
         if needs_grad:
             # the lists' length travels to pinned host memory behind an event; the cache cuts them to it when first asked
@@ -602,16 +518,6 @@ def _panel_nbytes(code: int, mode: int, ci: int, co: int, v: int, slab_bytes: in
     if key not in _pure_answers:
         _pure_answers[key] = int(nat.lib().fgx_weight_panel_bytes(C.c_int(code), C.c_int(mode), C.c_int(ci), C.c_int(co), C.c_int(v),
                                                                    C.c_int(slab_bytes), C.c_int(tile_cols)))
-    return _pure_answers[key]
-
-
-def _stream_groups(code: int, cols: int, tile_rows: int, tile_cols: int, slab_bytes: int, dev: torch.device) -> int:
-    key = ("groups", code, cols, tile_rows, tile_cols, slab_bytes, dev.index)
-    if key not in _pure_answers:
-        groups = C.c_int(0)
-        nat.check(nat.lib().fgx_conv_gather_gemm_stream_groups(C.c_int(code), C.c_int(cols), C.c_int(tile_rows), C.c_int(tile_cols),
-                                                               C.c_int(slab_bytes), C.byref(groups)))
-        _pure_answers[key] = groups.value
     return _pure_answers[key]
 
 
@@ -723,19 +629,21 @@ def _gather_gemm(src: torch.Tensor, weight_cvk: torch.Tensor, bias: Optional[tor
     if masked:
         cache._ensure_sorted()
     private = masked and _locality_applies(cache, n, k * src.element_size())
-    out = torch.empty((n, cols), dtype=dt, device=dev)
     if n == 0:
-        return out
-    L = nat.lib()
+        return torch.empty((n, cols), dtype=dt, device=dev)
     code = nat.DTYPE_CODE[dt]
-    name = "gather_gemm_fwd" if mode == 0 else "gather_gemm_dgrad"
-    mask = None
-    if relu_mask_out is not None and activation == nat.ACT_RELU and src.element_size() == 2 and cols % 8 == 0:
-        mask = torch.empty((n * cols // 8,), dtype=torch.uint8, device=dev)
-        relu_mask_out.append(mask)
-    with torch.cuda.device(dev):
-        panel = _weight_panel(weight_owner, weight_cvk, code, mode, sched, dev)
-        if _narrow_applies(cache, src, k, cols, v, n, n_src, sched):
+    want_mask = relu_mask_out is not None and activation == nat.ACT_RELU
+    narrow = _narrow_applies(cache, src, k, cols, v, n, n_src, sched)
+    panel = None
+    if narrow or (spconv.WEIGHT_PANEL_CACHE and weight_owner is not None):
+        with torch.cuda.device(dev):
+            panel = _weight_panel(weight_owner, weight_cvk, code, mode, sched, dev)
+    if narrow:
+        L = nat.lib()
+        name = "gather_gemm_fwd" if mode == 0 else "gather_gemm_dgrad"
+        out = torch.empty((n, cols), dtype=dt, device=dev)
+        mask = torch.empty((n * cols // 8,), dtype=torch.uint8, device=dev) if want_mask and cols % 8 == 0 else None
+        with torch.cuda.device(dev):
             plan = cache._narrow_plan()
             nat.mark(name, "start")
             nat.check(L.fgx_conv_narrow_gemm(
@@ -743,48 +651,20 @@ def _gather_gemm(src: torch.Tensor, weight_cvk: torch.Tensor, bias: Optional[tor
                 nat.sz(n), nat.sz(n_src), C.c_int(k), C.c_int(cols), C.c_int(v), C.c_int(activation), nat.ptr(out), nat.ptr(mask),
                 nat.stream()))
             nat.mark(name, "stop")
-            return out
-        if sched.stream and _stream_fits(n, n_src, k * src.element_size()):
-            order, tile_code, plan_seg, plan_idx, plan_band, plan_key = cache._gather_plan(sched.tile_rows, private,
-                                                                                           dense=not masked)
-            groups = _stream_groups(code, cols, int(sched.tile_rows), int(sched.tile_cols), int(sched.slab_bytes), dev)
-            item_at = cache._item_order(plan_key, tile_code, -(-cols // sched.tile_cols), groups,
-                                        -(-(k * src.element_size()) // sched.slab_bytes))
-            nat.mark(name, "start")
-            nat.check(L.fgx_conv_gather_gemm_stream_act_mask(
-                C.c_int(code), nat.ptr(src), nat.ptr(panel), nat.ptr(bias), nat.ptr(order), nat.ptr(tile_code),
-                nat.ptr(plan_seg), nat.ptr(plan_idx), nat.ptr(plan_band), nat.sz(plan_idx.shape[0]), nat.sz(n), nat.sz(n_src),
-                C.c_int(k), C.c_int(cols), C.c_int(v),
-                C.c_int(sched.tile_rows), C.c_int(sched.tile_cols), C.c_int(sched.slab_bytes), nat.ptr(item_at),
-                C.c_int(groups), C.c_int(activation), nat.ptr(out), nat.ptr(mask), nat.stream()))
-            nat.mark(name, "stop")
-            return out
-        if masked:
-            order, tile_code, _ = cache._tile_tables(sched.tile_rows, private)
-        else:
-            order, tile_code = cache._dense_tile_tables(sched.tile_rows)
-        scratch = None
-        if splitk > 1:
-            scratch = nat.workspace(L.fgx_conv_scratch_bytes(nat.sz(n), C.c_int(cols), C.c_int(splitk)), dev)
-        nat.mark(name, "start")
-        nat.check(L.fgx_conv_gather_gemm_act_mask(
-            C.c_int(code), nat.ptr(src), nat.ptr(panel), nat.ptr(bias), nat.ptr(cache["neighbor_map"]),
-            nat.ptr(order), nat.ptr(tile_code), nat.sz(n), C.c_int(k), C.c_int(cols), C.c_int(v),
-            C.c_int(sched.tile_rows), C.c_int(sched.tile_cols), C.c_int(sched.slab_bytes), C.c_int(splitk),
-            nat.ptr(scratch), C.c_int(activation), nat.ptr(out), nat.ptr(mask), nat.stream()))
-        nat.mark(name, "stop")
+    else:
+        if private:
+            cache._ensure_tile_order()
+        out, mask = nat.host().gather_gemm(src, weight_cvk, bias, cache, mode, splitk, masked, private and hasattr(cache, "_tile_order"), activation,
+                                           want_mask, sched, panel, _stream_fits(n, n_src, k * src.element_size()), nat.raw_stream(src))
+    if mask is not None:
+        relu_mask_out.append(mask)
     return out
 
 
 def _relu_mask_apply(grad_output: torch.Tensor, mask: torch.Tensor) -> torch.Tensor:
     """grad_output where the forward pass's bit mask says the activated output was positive, zero elsewhere
     (fgx_relu_mask_apply: one pass that reads an eighth of a byte per element beside the gradient)."""
-    g = grad_output.contiguous()
-    out = torch.empty_like(g)
-    with torch.cuda.device(g.device):
-        nat.check(nat.lib().fgx_relu_mask_apply(C.c_int(nat.DTYPE_CODE[g.dtype]), nat.ptr(g), nat.ptr(mask), nat.sz(g.numel()),
-                                                nat.ptr(out), nat.stream()))
-    return out
+    return nat.host().relu_mask_apply(grad_output, mask, nat.raw_stream(grad_output))
 
 
 def _narrow_applies(cache, src: torch.Tensor, k: int, cols: int, v: int, n: int, n_src: int, sched) -> bool:
@@ -913,47 +793,8 @@ def _wgrad(grad_output: torch.Tensor, feats: torch.Tensor, cache, v: int, with_b
             gb = gb[:co].contiguous() if with_bias else None
         return (gw, gb) if with_bias else gw
     cache._ensure_pairs()
-    seg_host = cache._seg_host()
-    if len(seg_host) != v + 1 or seg_host[-1] > min(cache["valid_signal_i"].numel(), cache["valid_signal_o"].numel()):
-        raise ValueError("valid_signal_seg does not fit the pair lists (V + 1 entries, the last one their length)")
-    seg_arr = (C.c_uint32 * (v + 1))(*seg_host)
     sched = nat.table_lookup(nat.PASS_WGRAD, dt, n, cip, cop, v)
-    gw = torch.empty((cop, v, cip), dtype=dt, device=dev)
-    gb = torch.empty((cop,), dtype=dt, device=dev) if with_bias else None
-    L = nat.lib()
-    code = nat.DTYPE_CODE[dt]
-    if sched.stream == 2 and not _sweep_fits(n, n_in, cip, cop, f.element_size(), seg_host[-1]):
-        # very long operands (and empty pair lists) take the block-major kernel
-        sched.stream, sched.block_rows = 1, 12288
-    if sched.stream == 2:
-        plan = cache._wgrad_sweep_plan(sched.block_rows)
-        with torch.cuda.device(dev):
-            scratch = nat.workspace(L.fgx_wgrad_sweep_scratch_bytes(C.c_int(cip), C.c_int(cop)), dev)
-            nat.mark("wgrad", "start")
-            nat.check(L.fgx_conv_wgrad_sweep(
-                C.c_int(code), nat.ptr(g), nat.ptr(f), nat.ptr(cache["valid_signal_i"]), nat.ptr(cache["valid_signal_o"]),
-                seg_arr, nat.ptr(plan), nat.sz(n), nat.sz(n_in), C.c_int(cip), C.c_int(cop), C.c_int(v), C.c_int(sched.tile_rows),
-                C.c_int(sched.block_rows), C.c_int(WGRAD_SWEEP_LEAD), C.c_int(WGRAD_SWEEP_MAX_POLLS), nat.ptr(scratch), nat.ptr(gw),
-                nat.ptr(gb), C.c_int(bias_offset), nat.stream()))
-            nat.mark("wgrad", "stop")
-        if cip != ci or cop != co:
-            gw = gw[:co, :, :ci].contiguous()
-            gb = gb[:co].contiguous() if with_bias else None
-        return (gw, gb) if with_bias else gw
-    bounds = cache._wgrad_bounds(sched.block_rows)
-    lists = None
-    if sched.stream == 1 and WGRAD_BALANCED_LISTS:
-        lists = cache._wgrad_item_lists(sched.block_rows, sched.tile_rows, sched.tile_cols, cip, cop)
-    with torch.cuda.device(dev):
-        scratch = nat.workspace(L.fgx_wgrad_scratch_bytes(nat.sz(n), C.c_int(v), C.c_int(cip), C.c_int(cop),
-                                                          C.c_int(sched.block_rows)), dev)
-        nat.mark("wgrad", "start")
-        nat.check(L.fgx_conv_wgrad_lists(
-            C.c_int(code), nat.ptr(g), nat.ptr(f), nat.ptr(cache["valid_signal_i"]), nat.ptr(cache["valid_signal_o"]),
-            seg_arr, nat.ptr(bounds), nat.ptr(lists), nat.sz(n), nat.sz(n_in), C.c_int(cip), C.c_int(cop), C.c_int(v), C.c_int(sched.tile_rows), C.c_int(sched.tile_cols),
-            C.c_int(sched.block_rows), C.c_int(sched.stream), nat.ptr(scratch), nat.ptr(gw), nat.ptr(gb), C.c_int(bias_offset),
-            nat.stream()))
-        nat.mark("wgrad", "stop")
+    gw, gb = nat.host().wgrad(g, f, cache, v, with_bias, bias_offset, sched, nat.raw_stream(f))
     if cip != ci or cop != co:
         gw = gw[:co, :, :ci].contiguous()
         gb = gb[:co].contiguous() if with_bias else None
@@ -961,14 +802,7 @@ def _wgrad(grad_output: torch.Tensor, feats: torch.Tensor, cache, v: int, with_b
 
 
 def _colsum(grad_output: torch.Tensor) -> torch.Tensor:
-    n, co = grad_output.shape
-    out = torch.empty((co,), dtype=grad_output.dtype, device=grad_output.device)
-    L = nat.lib()
-    with torch.cuda.device(grad_output.device):
-        scratch = nat.workspace(L.fgx_colsum_scratch_bytes(nat.sz(n), C.c_int(co)), grad_output.device)
-        nat.check(L.fgx_colsum(C.c_int(nat.DTYPE_CODE[grad_output.dtype]), nat.ptr(grad_output), nat.sz(n), C.c_int(co),
-                               nat.ptr(scratch), nat.ptr(out), nat.stream()))
-    return out
+    return nat.host().colsum(grad_output, nat.raw_stream(grad_output))
 
 
 def _gathered_rows(src: torch.Tensor, nmap: torch.Tensor) -> torch.Tensor:

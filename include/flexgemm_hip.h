@@ -187,7 +187,8 @@ int fgx_subm_cache_build(const int32_t* coords, size_t n, int B, int W, int H, i
  * row.  fgx_grid_index_pays: 1 where the index fits and its clears are worth it for n voxels on this grid (the host's
  * "auto" rule).  Workspace functions return 0 for a grid too large (512 MiB of bits); workspaces are 256-byte aligned.
  * The map: kernel volumes up to 128, mask codes (gray / binary, both or neither) up to 32.  The cache: as
- * fgx_subm_cache_build, without the sort's key_bits and presorted.
+ * fgx_subm_cache_build, without the sort's key_bits and presorted; seg_host (optional): pinned host memory that receives the
+ * segment table as well (valid once the stream has passed the call).
  * Replaces: hashmap_build_submanifold_conv_neighbour_map and the same sequence of calls as fgx_subm_cache_build. */
 int fgx_grid_index_pays(size_t n, int B, int W, int H, int D);
 size_t fgx_subm_neighbor_map_grid_workspace_bytes(size_t n, int B, int W, int H, int D);
@@ -197,7 +198,8 @@ int fgx_subm_neighbor_map_grid(const int32_t* coords, size_t n, int B, int W, in
 size_t fgx_subm_cache_grid_workspace_bytes(size_t n, int B, int W, int H, int D, int V, int with_pairs);
 int fgx_subm_cache_build_grid(const int32_t* coords, size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dw, int Dh, int Dd,
                               int with_pairs, void* workspace, size_t workspace_bytes, uint32_t* out_map, int32_t* gray, int32_t* binary,
-                              int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, fgx_stream_t stream);
+                              int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, uint32_t* seg_host,
+                              fgx_stream_t stream);
 
 /* Per row-tile (block consecutive rows of the sorted order) OR of the masks.
  *   codes: tile_code[nb] <- OR mask, seg[nb+1] <- exclusive offsets of popcounts (seg[nb] = total);
@@ -380,6 +382,14 @@ size_t fgx_gather_item_order_workspace_bytes(size_t num_tiles, int col_tiles);
 int fgx_gather_item_order(const int32_t* tile_code, size_t num_tiles, int col_tiles, int slabs, int groups,
                           void* workspace, size_t workspace_bytes, uint32_t* item_at, fgx_stream_t stream);
 
+/* The tile tables above in one call, every output but tile_code optional (NULL): the tiles' masks (have_codes != 0: given),
+ * the public offset lists' starts (seg), the gather plan (plan_seg, plan_idx, plan_band) and the item order (item_at, with
+ * item_ws of fgx_gather_item_order_workspace_bytes bytes).  gray may be NULL with given masks, map without a plan.
+ * Replaces: the same post-pass as fgx_tile_codes (flex_gemm/kernels/cuda/spconv/migemm_neighmap_pp.cu:330-368). */
+int fgx_tile_plan(const int32_t* gray, const int64_t* order, const uint32_t* map, size_t n, int V, int tile_rows, int have_codes,
+                  int32_t* tile_code, int32_t* seg, int32_t* plan_seg, uint32_t* plan_idx, uint32_t* plan_band, int col_tiles, int slabs,
+                  int groups, uint32_t* item_ws, uint32_t* item_at, fgx_stream_t stream);
+
 /* grad_weight[co, v, ci] = sum over pairs k in [seg[v], seg[v+1]) of grad_out[sig_o[k], co] * feats[sig_i[k], ci].
  * seg_host is the HOST copy of valid_signal_seg (V+1 entries); sig_o must ascend inside every segment (it does
  * when it comes from fgx_pair_fill).  The voxels are cut into blocks of `block_rows` rows; every (block, offset)
@@ -558,8 +568,8 @@ size_t fgx_spconv_cache_grid_workspace_bytes(size_t n_in, size_t n_out, int B, i
 int fgx_spconv_cache_build_grid(const int32_t* in_coords, size_t n_in, const int32_t* out_coords, size_t n_out, int B, int W, int H, int D,
                                 int Kw, int Kh, int Kd, int Sw, int Sh, int Sd, int Pw, int Ph, int Pd, int Dw, int Dh, int Dd,
                                 void* workspace, size_t workspace_bytes, uint32_t* map_fwd, int32_t* gray, int32_t* binary,
-                                int64_t* sorted_idx, uint32_t* map_bwd, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, int32_t* gray_bwd,
-                                int64_t* sorted_idx_bwd, fgx_stream_t stream);
+                                int64_t* sorted_idx, uint32_t* map_bwd, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, uint32_t* seg_host,
+                                int32_t* gray_bwd, int64_t* sorted_idx_bwd, fgx_stream_t stream);
 size_t fgx_spconv_out_coords_grid_workspace_bytes(int B, int Wo, int Ho, int Do);
 int fgx_spconv_out_coords_grid_count(const int32_t* coords, size_t n_in, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Sw, int Sh,
                                      int Sd, int Pw, int Ph, int Pd, int Dw, int Dh, int Dd, void* workspace, size_t workspace_bytes,
