@@ -437,9 +437,10 @@ __global__ void __launch_bounds__(kBlock) plan_fill_kernel(const uint32_t* __res
 // last round takes the cheapest items, every full round gives its most expensive item to the least loaded slot (rank of
 // each slot's load by counting).  Everything is deterministic.  One workgroup, so what bounds it is the length of its
 // dependent chains: the counting sort by one thread per piece with serial prefixes over 256 of them, and the ranks one
-// load at a time, took 0.040 ms for 1 306 items and 256 slots; this form and the two scans together 0.014.
+// load at a time, took 0.040 ms for 1 306 items and 256 slots; this form, the scans of 1 306 tiles included, 0.017.
 constexpr int kOrderThreads = 1024;     // also the largest number of slots
 constexpr int kOrderWaves = kOrderThreads / 64;
+constexpr unsigned kOrderInLds = 8192;  // items whose sorted list stays in LDS
 
 __device__ __forceinline__ unsigned tile_cost_bin(uint32_t code) { return 32u - (unsigned)__popc(code); }   // 0 = most expensive
 
@@ -490,41 +491,45 @@ __device__ void order_items(const int32_t* __restrict__ tile_code, unsigned num_
             count[wave][bin] = first + (uint32_t)__popcll(peers);
         }
         first = (uint32_t)__shfl((int)first, leader, 64);
-        if (live) sorted[first + (uint32_t)__popcll(peers & below)] = i0 + lane;
+        if (live) sorted[first + (uint32_t)__popcll(peers & below)] = bin << 26 | (i0 + lane);      // (the item, its cost above it)
     }
     __threadfence_block();
     __syncthreads();
     // ---- step 2: deal the rounds ----
+    // A slot's standing is its load above its number, so that one compare orders two slots; loads are kept within 21 bits.
     const unsigned rounds = total / groups, rem = total % groups;
-    auto cost_of = [&](unsigned item) -> uint32_t {
-        const unsigned pc = 32u - bin_of(item);
-        return (pc ? pc : 1u) * slabs + 3u;
+    unsigned scale = 0;
+    while ((((unsigned long long)(rounds + 1) * (32u * slabs + 3u)) >> scale) >= (1ull << 21)) ++scale;
+    auto cost_of = [&](uint32_t entry) -> uint32_t {
+        const unsigned pc = 32u - (entry >> 26);
+        return ((pc ? pc : 1u) * slabs + 3u) >> scale;
     };
-    uint32_t mine = 0;
-    if (tid < rem) {                                              // cheapest items: the positions of the last round
-        const unsigned item = sorted[total - rem + tid];
-        item_at[rounds * groups + tid] = item;
-        mine = cost_of(item);
+    // P threads per slot share the counting
+    const unsigned P = groups <= kOrderThreads / 4 ? 4u : (groups <= kOrderThreads / 2 ? 2u : 1u);
+    const unsigned slot = tid / P, part = tid % P;
+    uint32_t mine = slot;
+    if (slot < rem) {                                             // cheapest items: the positions of the last round
+        const uint32_t entry = sorted[total - rem + slot];
+        if (part == 0) item_at[rounds * groups + slot] = entry & 0x3FFFFFFu;
+        mine += cost_of(entry) << 10;
     }
     const unsigned quads = (groups + 3u) / 4u;
     for (unsigned r = 0; r < rounds; ++r) {
-        load[tid] = tid < groups ? mine : 0xFFFFFFFFu;
+        if (part == 0) load[slot] = slot < groups ? mine : 0xFFFFFFFFu;
         __syncthreads();
-        if (tid < groups) {
-            // slots with a smaller load come first, ties by slot number
-            unsigned rank = 0;
-            const uint4* load4 = reinterpret_cast<const uint4*>(load);
-#pragma unroll 8
-            for (unsigned q = 0; q < quads; ++q) {
-                const uint4 o = load4[q];
-                rank += (o.x < mine || (o.x == mine && 4 * q < tid)) ? 1u : 0u;
-                rank += (o.y < mine || (o.y == mine && 4 * q + 1 < tid)) ? 1u : 0u;
-                rank += (o.z < mine || (o.z == mine && 4 * q + 2 < tid)) ? 1u : 0u;
-                rank += (o.w < mine || (o.w == mine && 4 * q + 3 < tid)) ? 1u : 0u;
-            }
-            const unsigned item = sorted[r * groups + rank];      // rank 0 = least loaded slot <- most expensive item
-            item_at[r * groups + tid] = item;
-            mine += cost_of(item);
+        unsigned rank = 0;
+        const uint4* load4 = reinterpret_cast<const uint4*>(load);
+#pragma unroll 4
+        for (unsigned q = part; q < quads; q += P) {
+            const uint4 o = load4[q];
+            rank += (o.x < mine ? 1u : 0u) + (o.y < mine ? 1u : 0u) + (o.z < mine ? 1u : 0u) + (o.w < mine ? 1u : 0u);
+        }
+        if (P >= 2) rank += (unsigned)__shfl_xor((int)rank, 1, 64);
+        if (P >= 4) rank += (unsigned)__shfl_xor((int)rank, 2, 64);
+        if (slot < groups) {
+            const uint32_t entry = sorted[r * groups + rank];     // rank 0 = least loaded slot <- most expensive item
+            if (part == 0) item_at[r * groups + slot] = entry & 0x3FFFFFFu;
+            mine += cost_of(entry) << 10;
         }
         __syncthreads();
     }
@@ -537,6 +542,7 @@ __global__ void __launch_bounds__(kOrderThreads) tile_tables_kernel(const int32_
                                                                     unsigned col_tiles, unsigned slabs, unsigned groups,
                                                                     uint32_t* __restrict__ sorted, uint32_t* __restrict__ item_at) {
     __shared__ uint32_t part[kOrderWaves];
+    __shared__ uint32_t sorted_lds[kOrderInLds];
     uint32_t at = 0u, plan_at = 0u;
     if (seg != nullptr || plan_seg != nullptr) {
         for (unsigned t0 = 0; t0 < num_tiles; t0 += kOrderThreads) {         // (uniform)
@@ -559,7 +565,8 @@ __global__ void __launch_bounds__(kOrderThreads) tile_tables_kernel(const int32_
             if (plan_seg != nullptr) plan_seg[num_tiles] = (int32_t)plan_at;
         }
     }
-    if (item_at != nullptr) order_items(tile_code, num_tiles, col_tiles, slabs, groups, sorted, item_at);
+    if (item_at != nullptr)
+        order_items(tile_code, num_tiles, col_tiles, slabs, groups, num_tiles * col_tiles <= kOrderInLds ? sorted_lds : sorted, item_at);
 }
 
 struct PairLayout {
@@ -827,7 +834,7 @@ int fgx_tile_plan(const int32_t* gray, const int64_t* order, const uint32_t* map
     if (item_at != nullptr) {
         FGX_CHECK_ARG(col_tiles >= 1 && slabs >= 1 && groups >= 1 && groups <= kOrderThreads && item_ws != nullptr,
                       "fgx_tile_plan: bad item order col_tiles=%d slabs=%d groups=%d", col_tiles, slabs, groups);
-        FGX_CHECK_ARG(num_tiles * (size_t)col_tiles < 0x7FFFFFFFull, "fgx_tile_plan: too many items");
+        FGX_CHECK_ARG(num_tiles * (size_t)col_tiles < ((size_t)1 << 26), "fgx_tile_plan: too many items");
     }
     if (!have_codes) {
         tile_or_kernel<<<cdiv(num_tiles * 64, kBlock), kBlock, 0, s>>>(gray, order, n, tile_rows, num_tiles, tile_code);
@@ -893,7 +900,7 @@ int fgx_gather_item_order(const int32_t* tile_code, size_t num_tiles, int col_ti
                   groups);
     const size_t total = num_tiles * (size_t)col_tiles;
     if (total == 0) return FGX_OK;
-    FGX_CHECK_ARG(total < 0x7FFFFFFFull, "fgx_gather_item_order: too many items");
+    FGX_CHECK_ARG(total < ((size_t)1 << 26), "fgx_gather_item_order: too many items");
     FGX_CHECK_ARG(tile_code && workspace && item_at, "fgx_gather_item_order: null buffer");
     FGX_CHECK_ARG(workspace_bytes >= fgx_gather_item_order_workspace_bytes(num_tiles, col_tiles),
                   "fgx_gather_item_order: workspace of %zu bytes is too small", workspace_bytes);
