@@ -140,11 +140,6 @@ def host():
     return _host
 
 
-def raw_stream(t: torch.Tensor) -> int:
-    """Handle of the current stream of the tensor's device, as a number (what the native host side takes)."""
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
-
-
 def check(rc: int) -> None:
     if rc != 0:
         msg = lib().fgx_last_error().decode("utf-8", "replace")

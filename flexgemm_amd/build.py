@@ -54,7 +54,7 @@ def _host_command():
     return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wno-unknown-pragmas", "-D__HIP_PLATFORM_AMD__",
              f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DTORCH_EXTENSION_NAME=fgx_host", "-DNDEBUG"]
             + [f for i in includes for f in ("-isystem", i)]
-            + [HOST_SRC, "-o", HOST_LIB, "-L", torch_lib, "-lc10", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lamdhip64", "-ldl"])
+            + [HOST_SRC, "-o", HOST_LIB, "-L", torch_lib, "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lamdhip64", "-ldl"])
 
 
 def build(force: bool = False, verbose: bool = True, jobs: int = 4) -> str:

@@ -8,7 +8,13 @@
 // Policy (algorithm, schedule, which kernel family) stays with the Python callers.
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/grad_mode.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/utils/pybind.h>
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
@@ -16,6 +22,8 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <tuple>
+#include <unordered_map>
 #include <vector>
 
 #include "../../../include/flexgemm_hip.h"
@@ -36,7 +44,7 @@ namespace {
     X(fgx_colsum_scratch_bytes) X(fgx_colsum) X(fgx_wgrad_block_bounds_count) X(fgx_wgrad_block_bounds)                            \
     X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
     X(fgx_wgrad_sweep_plan_bytes) X(fgx_wgrad_sweep_plan) X(fgx_wgrad_sweep_scratch_bytes) X(fgx_conv_wgrad_sweep)                 \
-    X(fgx_serialize_encode) X(fgx_serialize_decode)
+    X(fgx_serialize_encode) X(fgx_serialize_decode) X(fgx_table_lookup)
 
 struct Lib {
 #define X(name) decltype(&::name) name = nullptr;
@@ -48,6 +56,7 @@ struct Lib {
 PyObject* g_impl = nullptr;         // ops.spconv.submanifold_conv3d
 PyObject* g_spconv = nullptr;       // ops.spconv
 PyObject* g_native = nullptr;       // _native
+PyObject* g_table_lookup = nullptr; // _native.table_lookup as it was at binding
 
 void bind(const std::string& path, py::module_ impl, py::module_ spconv, py::module_ native) {
     void* lib = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
@@ -60,6 +69,7 @@ void bind(const std::string& path, py::module_ impl, py::module_ spconv, py::mod
     g_impl = impl.release().ptr();
     g_spconv = spconv.release().ptr();
     g_native = native.release().ptr();
+    g_table_lookup = PyDict_GetItemString(PyModule_GetDict(g_native), "table_lookup");
 }
 
 void check(int rc) {
@@ -119,6 +129,8 @@ T* ptr(const Tensor& t) {
     return (T*)t.data_ptr();
 }
 fgx_stream_t as_stream(int64_t s) { return (fgx_stream_t)(uintptr_t)s; }
+// handle of the current stream of the tensor's device
+int64_t stream_of(const Tensor& t) { return (int64_t)(uintptr_t)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
 // ---- the segment table on its way to the host ------------------------------------------------------------------------
 // The pair lists' segment table is written to a pinned block by the kernel that fills the lists; the event behind it tells
@@ -210,7 +222,8 @@ private:
 // ---- neighbor caches ---------------------------------------------------------------------------------------------------
 // Tables of a submanifold convolution through the grid index, or None where it does not apply:
 // (neighbor_map, gray, binary, order, seg, sig_i, sig_o, SegHost), the last four None without gradients.
-py::object subm_cache(const Tensor& coords, const std::vector<int>& geom, bool needs_grad, bool forced, size_t max_pair_bytes, int64_t stream) {
+py::object subm_cache(const Tensor& coords, const std::vector<int>& geom, bool needs_grad, bool forced, size_t max_pair_bytes) {
+    const int64_t stream = stream_of(coords);
     const size_t n = (size_t)coords.size(0);
     const int B = geom[0], W = geom[1], H = geom[2], D = geom[3], V = geom[4] * geom[5] * geom[6];
     if (n == 0 || V > 32 || n * (size_t)V >= 0xFFFFFFFFull || (needs_grad && n * (size_t)V * 8 > max_pair_bytes)) return py::none();
@@ -244,7 +257,8 @@ bool conv_grids_pay(size_t n_in, size_t n_out, int B, const int* in, const int* 
 
 // geom: B, W, H, D, kernel, stride, padding, dilation.  The dictionary of a generic convolution's tables, or None.
 py::object spconv_cache(const Tensor& coords, const Tensor& out_coords, const std::vector<int>& g, bool needs_grad, bool bwd_order,
-                        size_t max_pair_bytes, int64_t stream) {
+                        size_t max_pair_bytes) {
+    const int64_t stream = stream_of(coords);
     const size_t m = (size_t)coords.size(0), l = (size_t)out_coords.size(0);
     const int V = g[4] * g[5] * g[6];
     if (m == 0 || l == 0 || V > 32 || l * (size_t)V >= 0xFFFFFFFFull || (needs_grad && l * (size_t)V * 8 > max_pair_bytes)) return py::none();
@@ -293,7 +307,9 @@ py::object spconv_cache(const Tensor& coords, const Tensor& out_coords, const st
 }
 
 // Output coordinates in (b, x, y, z) order through the bit map of the output grid, or None where it does not apply.
-py::object out_coords(const Tensor& coords, const std::vector<int>& g, int64_t stream) {
+py::object out_coords(const Tensor& coords, const std::vector<int>& g) {
+    const int64_t stream = stream_of(coords);
+    if (capturing(stream)) return py::none();              // (the count is waited for)
     const size_t m = (size_t)coords.size(0);
     int out[3];
     check(L.fgx_spconv_out_dims(g[1], g[2], g[3], g[4], g[5], g[6], g[7], g[8], g[9], g[10], g[11], g[12], g[13], g[14], g[15], &out[0], &out[1], &out[2]));
@@ -451,48 +467,138 @@ int dtype_code(const Tensor& t) {
 
 int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
-// The gather GEMM on the streaming or the tiled kernel.  mode 0 forward, 1 / 2 input gradient (see _gather_gemm); operands
-// dense, rows whole 16-byte pieces.  panel: a kept weight panel, or None to pack one.  stream_fits: the streaming kernel's
-// 32-bit offsets reach.  Returns (output, ReLU bit mask or None).
-py::tuple gather_gemm(const Tensor& src, const Tensor& weight, const c10::optional<Tensor>& bias, py::object cache_obj, int mode, int splitk,
-                      bool masked, bool own_order, int activation, bool want_mask, py::object sched_obj, const c10::optional<Tensor>& panel_kept,
-                      bool stream_fits, int64_t stream) {
-    const Cache c(std::move(cache_obj));
-    const Sched s = read_schedule(sched_obj);
+// The schedule of a pass and shape (fgx_table_lookup; answers are pure functions of the key and remembered).  Python's
+// table_lookup is asked instead when somebody has replaced it: that is how schedules are forced.
+py::object python_schedule(int pass, const Tensor& like, int64_t n, int ci, int co, int v) {
+    return py::reinterpret_borrow<py::object>(module_get(g_native, "table_lookup"))(
+        pass, py::cast(like).attr("dtype"), n, ci, co, v);
+}
+
+Sched schedule(int pass, const Tensor& like, int64_t n, int ci, int co, int v) {
+    if (module_get(g_native, "table_lookup") != g_table_lookup) return read_schedule(python_schedule(pass, like, n, ci, co, v));
+    struct Key {
+        int pass, code, ci, co, v;
+        int64_t n;
+        bool operator==(const Key& o) const { return pass == o.pass && code == o.code && ci == o.ci && co == o.co && v == o.v && n == o.n; }
+    };
+    struct Hash {
+        size_t operator()(const Key& k) const {
+            uint64_t h = (uint64_t)k.n * 0x9E3779B97F4A7C15ull;
+            for (int x : {k.pass, k.code, k.ci, k.co, k.v}) h = (h ^ (uint64_t)x) * 0x9E3779B97F4A7C15ull + (h >> 29);
+            return (size_t)h;
+        }
+    };
+    static std::unordered_map<Key, Sched, Hash> known;      // (guarded by the interpreter lock, like all callers here)
+    const Key key{pass, dtype_code(like), ci, co, v, n};
+    auto it = known.find(key);
+    if (it == known.end()) {
+        fgx_schedule got;
+        static_assert(sizeof(got) == sizeof(Sched), "the schedule's fields");
+        check(L.fgx_table_lookup(pass, key.code, (size_t)n, ci, co, v, &got));
+        Sched s;
+        memcpy(&s, &got, sizeof(s));
+        if (known.size() > 4096) known.clear();
+        it = known.emplace(key, s).first;
+    }
+    return it->second;
+}
+
+py::object impl_function(const char* name) { return py::reinterpret_borrow<py::object>(module_get(g_impl, name)); }
+
+// Whether the resident-row kernels for narrow layers could run at all; the Python policy decides when they do.
+bool narrow_shape(const Cache& c, int es, int k, int cols, int v, int64_t n) {
+    if (es != 2 || k < 8 || k > 32 || k % 8 || cols < 8 || cols > 32 || cols % 8 || v > 27) return false;
+    return c.has("_narrow_plan_buf") || n >= module_int(g_impl, "NARROW_RESIDENT_MIN_ROWS") ||
+           py::reinterpret_borrow<py::object>(module_get(g_spconv, "NARROW_RESIDENT")).cast<std::string>() != "auto";
+}
+
+Tensor pad_columns(const Tensor& t, int64_t multiple) {
+    const int64_t pad = (multiple - t.size(-1) % multiple) % multiple;
+    return pad ? at::constant_pad_nd(t, {0, pad}) : t;
+}
+
+struct Product {
+    Tensor out, mask;
+};
+
+// mode 0: out = conv(src) with weight [Co, V, Ci] (+ bias), mode 1: input gradient from src = grad_output through the same
+// map with the offsets mirrored, mode 2: through a map of its own, offsets as they are.  One row per row of the cache's
+// neighbor_map.  masked: mask-sorted schedule (else natural row order, all offsets per tile).  want_mask: also one bit per
+// output, "greater than zero", where the kernels can (ReLU, 16-bit type, a multiple of 8 columns).  panel: a kept weight
+// panel, or undefined to pack one.
+Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, int mode, bool allow_splitk, bool masked, int activation,
+                       bool want_mask, const Tensor& panel_kept, int64_t stream) {
     const at::Device dev = src.device();
     const c10::DeviceGuard guard(dev);
-    const int co = (int)weight.size(0), v = (int)weight.size(1), ci = (int)weight.size(2);
-    const int k = mode == 0 ? ci : co, cols = mode == 0 ? co : ci;
-    const Tensor nmap = c.need("neighbor_map");
-    const int64_t n = nmap.size(0);
-    const size_t n_src = (size_t)src.size(0);
     const int code = dtype_code(src);
-    const int es = (int)src.element_size();
-    Tensor out = make({n, cols}, src.scalar_type(), dev), mask;
-    if (want_mask && activation == FGX_ACT_RELU && es == 2 && cols % 8 == 0) mask = make({n * cols / 8}, at::kByte, dev);
-    Tensor panel;
-    if (panel_kept.has_value()) {
-        panel = *panel_kept;
-    } else {
+    if (weight.scalar_type() != src.scalar_type() || (bias.defined() && bias.scalar_type() != src.scalar_type()))
+        throw py::type_error("features, weight and bias must share one dtype");
+    const int es = (int)src.element_size(), v = (int)weight.size(1);
+    const Tensor nmap = c.need("neighbor_map");
+    const int64_t n = nmap.size(0), n_src = src.size(0);
+    const int cols = (int)weight.size(mode == 0 ? 0 : 2);
+    Product p;
+    if (n_src == 0) {                       // nothing to gather: the bias alone
+        p.out = at::zeros({n, cols}, src.options());
+        if (bias.defined()) p.out = p.out + bias;
+        if (activation == FGX_ACT_RELU) p.out = at::relu(p.out);
+        return p;
+    }
+    const int align = 16 / es;
+    if (weight.size(mode == 0 ? 2 : 0) % align) {       // rows must be whole 16-byte pieces
+        src = pad_columns(src, align);
+        weight = mode == 0 ? pad_columns(weight, align) : at::constant_pad_nd(weight, {0, 0, 0, 0, 0, (align - weight.size(0) % align) % align});
+    }
+    src = src.contiguous();
+    weight = weight.contiguous();
+    if (bias.defined()) bias = bias.contiguous();
+    const int co = (int)weight.size(0), ci = (int)weight.size(2), k = mode == 0 ? ci : co;
+    const int64_t row_bytes = (int64_t)k * es;
+    if (masked && !(c.has("gray_code") && c.has("sorted_idx"))) c.obj.attr("_ensure_sorted")();
+    const int pass = mode == 0 ? 0 : 1;
+    const Sched s = schedule(pass, src, n, ci, co, v);
+    bool own_order = false;
+    if (masked && row_bytes <= module_int(g_impl, "LOCALITY_MAX_ROW_BYTES") && (c.has("_tile_order") || n >= module_int(g_impl, "LOCALITY_MIN_ROWS")) &&
+        impl_function("_locality_applies")(c.obj, n, row_bytes).cast<bool>()) {
+        c.obj.attr("_ensure_tile_order")();
+        own_order = c.has("_tile_order");
+    }
+    if (n == 0) {
+        p.out = make({n, cols}, src.scalar_type(), dev);
+        return p;
+    }
+    Tensor panel = panel_kept;
+    if (!panel.defined()) {
         panel = workspace(L.fgx_weight_panel_bytes(code, mode, ci, co, v, s.slab_bytes, s.tile_cols), dev);
         check(L.fgx_pack_weight(code, mode, ptr(weight), ci, co, v, s.slab_bytes, s.tile_cols, ptr(panel), as_stream(stream)));
     }
-    const void* b = bias.has_value() ? ptr(*bias) : nullptr;
+    if (narrow_shape(c, es, k, cols, v, n) &&
+        impl_function("_narrow_applies")(c.obj, src, k, cols, v, n, n_src, python_schedule(pass, src, n, ci, co, v)).cast<bool>()) {
+        py::tuple got = impl_function("_narrow_gemm")(src, panel, bias.defined() ? py::cast(bias) : py::none(), c.obj, mode, k, cols, v, activation, want_mask);
+        p.out = got[0].cast<Tensor>();
+        if (!got[1].is_none()) p.mask = got[1].cast<Tensor>();
+        return p;
+    }
+    p.out = make({n, cols}, src.scalar_type(), dev);
+    if (want_mask && activation == FGX_ACT_RELU && es == 2 && cols % 8 == 0) p.mask = make({n * cols / 8}, at::kByte, dev);
+    const void* b = ptr(bias);
     const char* name = mode == 0 ? "gather_gemm_fwd" : "gather_gemm_dgrad";
-    if (s.stream && stream_fits) {
+    // the streaming kernel addresses its operands with 32-bit byte offsets
+    const double most = (double)0xFF000000u;
+    if (s.stream && (double)n_src * row_bytes <= most && (double)n * 8 <= most && (double)n * 27 * 4 * 2 <= most) {
         int groups = 0;
         check(L.fgx_conv_gather_gemm_stream_groups(code, cols, s.tile_rows, s.tile_cols, s.slab_bytes, &groups));
         Tensor item_at;
-        const Tiles t = gather_plan(c, s.tile_rows, own_order, !masked, ceil_div(cols, s.tile_cols), groups, ceil_div((int64_t)k * es, s.slab_bytes),
-                                    &item_at, stream);
+        const Tiles t = gather_plan(c, s.tile_rows, own_order, !masked, ceil_div(cols, s.tile_cols), groups, ceil_div(row_bytes, s.slab_bytes), &item_at,
+                                    stream);
         mark(name, "start");
         check(L.fgx_conv_gather_gemm_stream_act_mask(code, ptr(src), ptr(panel), b, ptr<int64_t>(t.order), ptr<int32_t>(t.code),
                                                      ptr<int32_t>(t.plan_seg), ptr<uint32_t>(t.plan_idx), ptr<uint32_t>(t.plan_band),
-                                                     (size_t)t.plan_idx.size(0), (size_t)n, n_src, k, cols, v, s.tile_rows, s.tile_cols,
-                                                     s.slab_bytes, ptr<uint32_t>(item_at), groups, activation, ptr(out), ptr<uint8_t>(mask),
+                                                     (size_t)t.plan_idx.size(0), (size_t)n, (size_t)n_src, k, cols, v, s.tile_rows, s.tile_cols,
+                                                     s.slab_bytes, ptr<uint32_t>(item_at), groups, activation, ptr(p.out), ptr<uint8_t>(p.mask),
                                                      as_stream(stream)));
-        mark(name, "stop");
     } else {
+        const int splitk = allow_splitk ? s.splitk : 1;
         Tiles t;
         if (masked) {
             tile_codes(c, s.tile_rows, own_order, stream, &t, false);
@@ -506,10 +612,17 @@ py::tuple gather_gemm(const Tensor& src, const Tensor& weight, const c10::option
         mark(name, "start");
         check(L.fgx_conv_gather_gemm_act_mask(code, ptr(src), ptr(panel), b, ptr<uint32_t>(nmap), ptr<int64_t>(t.order), ptr<int32_t>(t.code),
                                               (size_t)n, k, cols, v, s.tile_rows, s.tile_cols, s.slab_bytes, splitk, ptr(scratch), activation,
-                                              ptr(out), ptr<uint8_t>(mask), as_stream(stream)));
-        mark(name, "stop");
+                                              ptr(p.out), ptr<uint8_t>(p.mask), as_stream(stream)));
     }
-    return py::make_tuple(out, mask.defined() ? py::cast(mask) : py::none());
+    mark(name, "stop");
+    return p;
+}
+
+py::tuple gather_gemm(const Tensor& src, const Tensor& weight, const c10::optional<Tensor>& bias, py::object cache, int mode, bool allow_splitk,
+                      bool masked, int activation, bool want_mask, const c10::optional<Tensor>& panel) {
+    const Product p = gather_product(src, weight, bias.value_or(Tensor()), Cache(std::move(cache)), mode, allow_splitk, masked, activation, want_mask,
+                                     panel.value_or(Tensor()), stream_of(src));
+    return py::make_tuple(p.out, p.mask.defined() ? py::cast(p.mask) : py::none());
 }
 
 // [V + 1] words of the segment table on the host
@@ -552,59 +665,85 @@ Tensor wgrad_item_lists(const Cache& c, const Tensor& bounds, size_t n, int v, i
     return lists;
 }
 
-// [Co, V, Ci] weight gradient (and with with_bias the bias gradient) from the cache's pair lists; operands dense, rows whole
-// 16-byte pieces.  sweep_fits: what fgx_conv_wgrad_sweep takes (a schedule that asks for it runs block-major otherwise).
-py::tuple wgrad(const Tensor& grad, const Tensor& feats, py::object cache_obj, int v, bool with_bias, int bias_offset, py::object sched_obj,
-                int64_t stream) {
-    const Cache c(std::move(cache_obj));
-    Sched s = read_schedule(sched_obj);
+struct WeightGrads {
+    Tensor weight, bias;
+};
+
+// [Co, V, Ci] weight gradient (and with with_bias the bias gradient) from the cache's pair lists: grad has one row per row of
+// the cache's map, feats one per row the map points at.  bias_offset names an offset whose pairs hold every row of grad exactly
+// once (-1: none), which lets the streaming kernel sum the rows it loads anyway.
+WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool with_bias, int bias_offset, int64_t stream) {
     const at::Device dev = feats.device();
     const c10::DeviceGuard guard(dev);
-    const int64_t n = grad.size(0), n_in = feats.size(0);
-    const int co = (int)grad.size(1), ci = (int)feats.size(1), es = (int)feats.element_size();
     const int code = dtype_code(feats);
-    const Tensor sig_i = c.need("valid_signal_i"), sig_o = c.need("valid_signal_o");
-    const std::vector<uint32_t> seg = seg_host(c, v);
-    const int64_t pairs = seg[v];
-    if (pairs > std::min(sig_i.numel(), sig_o.numel()))
-        throw py::value_error("valid_signal_seg does not fit the pair lists (V + 1 entries, the last one their length)");
-    if (s.stream == 2) {
-        // (the checks of the C entry point: 24-bit row numbers, operands and lists within its 32-bit byte offsets)
-        const double most = (double)0xFF000000u;
-        const bool fits = n > 0 && n <= (1 << 24) && n_in <= (1 << 24) && pairs > 0 && (double)n * co * es <= most && (double)n_in * ci * es <= most &&
-                          (double)pairs * 4 + 256 <= most;
-        if (!fits) {                                    // very long operands (and empty pair lists) take the block-major kernel
-            s.stream = 1;
-            s.block_rows = 12288;
-        }
-    }
-    Tensor gw = make({co, v, ci}, feats.scalar_type(), dev), gb;
-    if (with_bias) gb = make({co}, feats.scalar_type(), dev);
-    if (s.stream == 2) {
-        const std::string key = "_wgrad_sweep_plan_" + std::to_string(s.block_rows);
-        Tensor plan;
-        if (!c.tensor(key, &plan)) {
-            plan = workspace(L.fgx_wgrad_sweep_plan_bytes((size_t)n, (size_t)pairs, v, s.block_rows), dev);
-            check(L.fgx_wgrad_sweep_plan(ptr<uint32_t>(sig_o), seg.data(), (size_t)n, v, s.block_rows, ptr(plan), (size_t)plan.numel(), as_stream(stream)));
-            c.set(key, plan);
-        }
-        Tensor scratch = workspace(L.fgx_wgrad_sweep_scratch_bytes(ci, co), dev);
-        mark("wgrad", "start");
-        check(L.fgx_conv_wgrad_sweep(code, ptr(grad), ptr(feats), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o), seg.data(), ptr(plan), (size_t)n,
-                                     (size_t)n_in, ci, co, v, s.tile_rows, s.block_rows, (int)module_int(g_impl, "WGRAD_SWEEP_LEAD"),
-                                     (int)module_int(g_impl, "WGRAD_SWEEP_MAX_POLLS"), ptr(scratch), ptr(gw), ptr(gb), bias_offset, as_stream(stream)));
+    const int64_t n = grad.size(0), n_in = feats.size(0), true_ci = feats.size(1), true_co = grad.size(1);
+    const int es = (int)feats.element_size(), align = 16 / es;
+    feats = pad_columns(feats, align).contiguous();
+    grad = pad_columns(grad, align).contiguous();
+    const int ci = (int)feats.size(1), co = (int)grad.size(1);
+    WeightGrads w;
+    if (n > 0 && narrow_shape(c, es, ci, co, v, n) && impl_function("_narrow_wgrad_applies")(c.obj, feats, ci, co, v, n, n_in).cast<bool>()) {
+        py::tuple got = impl_function("_narrow_wgrad")(grad, feats, c.obj, v, with_bias);
+        w.weight = got[0].cast<Tensor>();
+        if (with_bias) w.bias = got[1].cast<Tensor>();
     } else {
-        const Tensor bounds = wgrad_bounds(c, sig_o, seg, (size_t)n, v, s.block_rows, stream);
-        Tensor lists;
-        if (s.stream == 1 && PyObject_IsTrue(module_get(g_impl, "WGRAD_BALANCED_LISTS"))) lists = wgrad_item_lists(c, bounds, (size_t)n, v, ci, co, s, stream);
-        Tensor scratch = workspace(L.fgx_wgrad_scratch_bytes((size_t)n, v, ci, co, s.block_rows), dev);
-        mark("wgrad", "start");
-        check(L.fgx_conv_wgrad_lists(code, ptr(grad), ptr(feats), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o), seg.data(), ptr<uint32_t>(bounds),
-                                     ptr<uint32_t>(lists), (size_t)n, (size_t)n_in, ci, co, v, s.tile_rows, s.tile_cols, s.block_rows, s.stream,
-                                     ptr(scratch), ptr(gw), ptr(gb), bias_offset, as_stream(stream)));
+        if (!(c.has("valid_signal_seg") && (c.has("valid_signal_i") || c.has("_pending_pairs")))) c.obj.attr("_ensure_pairs")();
+        const Tensor sig_i = c.need("valid_signal_i"), sig_o = c.need("valid_signal_o");
+        const std::vector<uint32_t> seg = seg_host(c, v);
+        const int64_t pairs = seg[v];
+        if (pairs > std::min(sig_i.numel(), sig_o.numel()))
+            throw py::value_error("valid_signal_seg does not fit the pair lists (V + 1 entries, the last one their length)");
+        Sched s = schedule(2, feats, n, ci, co, v);
+        if (s.stream == 2) {
+            // (the checks of the C entry point: 24-bit row numbers, operands and lists within its 32-bit byte offsets)
+            const double most = (double)0xFF000000u;
+            const bool fits = n > 0 && n <= (1 << 24) && n_in <= (1 << 24) && pairs > 0 && (double)n * co * es <= most &&
+                              (double)n_in * ci * es <= most && (double)pairs * 4 + 256 <= most;
+            if (!fits) {                                // very long operands (and empty pair lists) take the block-major kernel
+                s.stream = 1;
+                s.block_rows = 12288;
+            }
+        }
+        w.weight = make({co, v, ci}, feats.scalar_type(), dev);
+        if (with_bias) w.bias = make({co}, feats.scalar_type(), dev);
+        if (s.stream == 2) {
+            const std::string key = "_wgrad_sweep_plan_" + std::to_string(s.block_rows);
+            Tensor plan;
+            if (!c.tensor(key, &plan)) {
+                plan = workspace(L.fgx_wgrad_sweep_plan_bytes((size_t)n, (size_t)pairs, v, s.block_rows), dev);
+                check(L.fgx_wgrad_sweep_plan(ptr<uint32_t>(sig_o), seg.data(), (size_t)n, v, s.block_rows, ptr(plan), (size_t)plan.numel(),
+                                             as_stream(stream)));
+                c.set(key, plan);
+            }
+            Tensor scratch = workspace(L.fgx_wgrad_sweep_scratch_bytes(ci, co), dev);
+            mark("wgrad", "start");
+            check(L.fgx_conv_wgrad_sweep(code, ptr(grad), ptr(feats), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o), seg.data(), ptr(plan), (size_t)n,
+                                         (size_t)n_in, ci, co, v, s.tile_rows, s.block_rows, (int)module_int(g_impl, "WGRAD_SWEEP_LEAD"),
+                                         (int)module_int(g_impl, "WGRAD_SWEEP_MAX_POLLS"), ptr(scratch), ptr(w.weight), ptr(w.bias), bias_offset,
+                                         as_stream(stream)));
+        } else {
+            const Tensor bounds = wgrad_bounds(c, sig_o, seg, (size_t)n, v, s.block_rows, stream);
+            Tensor lists;
+            if (s.stream == 1 && PyObject_IsTrue(module_get(g_impl, "WGRAD_BALANCED_LISTS")))
+                lists = wgrad_item_lists(c, bounds, (size_t)n, v, ci, co, s, stream);
+            Tensor scratch = workspace(L.fgx_wgrad_scratch_bytes((size_t)n, v, ci, co, s.block_rows), dev);
+            mark("wgrad", "start");
+            check(L.fgx_conv_wgrad_lists(code, ptr(grad), ptr(feats), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o), seg.data(), ptr<uint32_t>(bounds),
+                                         ptr<uint32_t>(lists), (size_t)n, (size_t)n_in, ci, co, v, s.tile_rows, s.tile_cols, s.block_rows, s.stream,
+                                         ptr(scratch), ptr(w.weight), ptr(w.bias), bias_offset, as_stream(stream)));
+        }
+        mark("wgrad", "stop");
     }
-    mark("wgrad", "stop");
-    return py::make_tuple(gw, gb.defined() ? py::cast(gb) : py::none());
+    if (ci != true_ci || co != true_co) {
+        w.weight = w.weight.slice(0, 0, true_co).slice(2, 0, true_ci).contiguous();
+        if (with_bias) w.bias = w.bias.slice(0, 0, true_co).contiguous();
+    }
+    return w;
+}
+
+py::tuple wgrad(const Tensor& grad, const Tensor& feats, py::object cache, int v, bool with_bias, int bias_offset) {
+    const WeightGrads w = weight_grads(grad, feats, Cache(std::move(cache)), v, with_bias, bias_offset, stream_of(feats));
+    return py::make_tuple(w.weight, w.bias.defined() ? py::cast(w.bias) : py::none());
 }
 
 Tensor relu_mask_apply(const Tensor& grad, const Tensor& mask, int64_t stream) {
@@ -624,61 +763,209 @@ Tensor colsum(const Tensor& grad, int64_t stream) {
     return out;
 }
 
+// ---- the differentiable operators --------------------------------------------------------------------------------------
+// What one call of an operator is: kept by its node for the backward pass.
+struct Call {
+    bool generic = false;               // sparse_conv3d: an input gradient through a map of its own
+    bool masked = true, splitk = true;  // the algorithm's schedule
+};
+
+// A Python object held where the interpreter lock may not be.
+struct Held {
+    PyObject* obj = nullptr;
+    ~Held() { drop(); }
+    void take(py::handle h) {
+        obj = h.ptr();
+        Py_INCREF(obj);
+    }
+    void drop() {
+        if (obj != nullptr && Py_IsInitialized()) {
+            const py::gil_scoped_acquire gil;
+            Py_CLEAR(obj);
+        }
+    }
+};
+
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+struct ConvBackward : public torch::autograd::Node {
+    Call call;
+    Held cache;
+    SavedVariable feats, weight, output;
+    Tensor mask;                        // the ReLU's derivative, one bit per output
+    bool relu = false, has_bias = false;
+
+    std::string name() const override { return call.generic ? "SparseConv3dBackward" : "SubMConv3dBackward"; }
+    void release_variables() override {
+        feats.reset_data();
+        weight.reset_data();
+        output.reset_data();
+        mask.reset();
+    }
+
+    variable_list apply(variable_list&& grads) override {
+        try {
+            return gradients(std::move(grads));
+        } catch (py::error_already_set& e) {        // keep the Python error's type on its way through the engine's thread
+            const py::gil_scoped_acquire gil;
+            e.restore();
+            python_error err;
+            err.persist();
+            throw err;
+        }
+    }
+
+    variable_list gradients(variable_list&& grads) {
+        variable_list result(has_bias ? 3 : 2);
+        if (!grads[0].defined()) return result;
+        const bool need_f = task_should_compute_output(0), need_w = task_should_compute_output(1);
+        const bool need_b = has_bias && task_should_compute_output(2);
+        const at::NoGradGuard no_grad;
+        const Tensor f = feats.unpack(), w = weight.unpack();
+        const py::gil_scoped_acquire gil;
+        if (cache.obj == nullptr) throw std::runtime_error("Trying to backward through the graph a second time");
+        const Cache c(py::reinterpret_borrow<py::object>(cache.obj));
+        const int64_t stream = stream_of(f);
+        Tensor grad = grads[0];
+        if (relu && mask.defined()) grad = relu_mask_apply(grad, mask, stream);
+        else if (relu) grad = at::where(output.unpack(shared_from_this()).gt(0), grad, at::zeros({}, grad.options()));
+        grad = grad.contiguous();
+        const int64_t co = w.size(0), kw = w.size(1), kh = w.size(2), kd = w.size(3), ci = w.size(4), v = kw * kh * kd;
+        if (need_f) {
+            const Tensor wv = w.reshape({co, v, ci});
+            if (call.generic) {
+                const Cache view(c.obj.attr("_bwd_view")());
+                // mask-sorted walk only where the cache carries the backward order
+                result[0] = gather_product(grad, wv, Tensor(), view, 2, call.splitk, call.masked && view.has("sorted_idx"), FGX_ACT_NONE, false, Tensor(),
+                                           stream).out;
+            } else {
+                result[0] = gather_product(grad, wv, Tensor(), c, 1, call.splitk, call.masked, FGX_ACT_NONE, false, Tensor(), stream).out;
+            }
+        }
+        if (need_w) {
+            // odd submanifold kernel: the centre offset pairs every voxel with itself, so the bias gradient rides along
+            const bool odd = kw % 2 && kh % 2 && kd % 2 && !call.generic;
+            const int centre = odd && PyObject_IsTrue(module_get(g_spconv, "FUSE_DBIAS")) ? (int)(v / 2) : -1;
+            const bool with_bias = need_b && !call.generic;
+            WeightGrads g = weight_grads(grad, f, c, (int)v, with_bias, with_bias ? centre : -1, stream);
+            result[1] = g.weight.reshape({co, kw, kh, kd, ci});
+            if (with_bias) result[2] = g.bias;
+        }
+        if (need_b && !result[2].defined()) result[2] = colsum(grad, stream);
+        return result;
+    }
+};
+
+void require(bool ok, const std::string& what) {
+    if (ok) return;
+    PyErr_SetString(PyExc_AssertionError, what.c_str());
+    throw py::error_already_set();
+}
+
+// One layer: its output, with a node behind it when gradients are recorded.  cache: the neighbor cache of its coordinates.
+Tensor convolve(const Tensor& feats, py::object cache_obj, const Tensor& weight, const c10::optional<Tensor>& bias_opt, bool relu, bool generic,
+                bool masked, bool splitk) {
+    const Tensor bias = bias_opt.value_or(Tensor());
+    const bool has_bias = bias.defined();
+    const bool record = at::GradMode::is_enabled() && (feats.requires_grad() || weight.requires_grad() || (has_bias && bias.requires_grad()));
+    require(weight.dim() == 5 && feats.dim() == 2, "features are [N, C], weights [Co, Kw, Kh, Kd, Ci]");
+    const int64_t co = weight.size(0), v = weight.size(1) * weight.size(2) * weight.size(3), ci = weight.size(4);
+    require(feats.size(1) == ci, "Input channels (" + std::to_string(feats.size(1)) + ") should match weight channels (" + std::to_string(ci) + ")");
+    require(feats.is_contiguous(), "Input features should be contiguous");
+    const Cache c(std::move(cache_obj));
+    int64_t expected = c.need("neighbor_map").size(0);
+    if (generic) {                      // rows of the input the maps were made for (absent on a hand-made cache)
+        expected = feats.size(0);
+        Tensor bwd;
+        if (PyObject* m = c.find("_n_in")) {
+            if (m != Py_None) expected = PyLong_AsLongLong(m);
+        } else if (c.tensor("neighbor_map_bwd", &bwd)) {
+            expected = bwd.size(0);
+        }
+    }
+    require(feats.size(0) == expected, std::to_string(feats.size(0)) + " feature rows for a neighbor cache of " + std::to_string(expected) + " voxels");
+    const bool bits = relu && record && PyObject_IsTrue(module_get(g_spconv, "RELU_BIT_MASK"));
+    Product p;
+    {
+        const at::NoGradGuard no_grad;
+        p = gather_product(feats, weight.reshape({co, v, ci}), bias, c, 0, splitk, masked, relu ? FGX_ACT_RELU : FGX_ACT_NONE, bits, Tensor(),
+                           stream_of(feats));
+    }
+    if (!record) return p.out;
+    auto node = std::make_shared<ConvBackward>();
+    node->set_next_edges(has_bias ? torch::autograd::collect_next_edges(feats, weight, bias) : torch::autograd::collect_next_edges(feats, weight));
+    node->call.generic = generic;
+    node->call.masked = masked;
+    node->call.splitk = splitk;
+    node->cache.take(c.obj);
+    node->relu = relu;
+    node->has_bias = has_bias;
+    node->feats = SavedVariable(feats, false);
+    node->weight = SavedVariable(weight, false);
+    node->mask = p.mask;
+    torch::autograd::set_history(p.out, node);
+    if (relu && !p.mask.defined()) node->output = SavedVariable(p.out, true);
+    return p.out;
+}
+
 // ---- curve codes -----------------------------------------------------------------------------------------------------
-Tensor encode(const Tensor& coords, int mode, int bits, int code_bits, int64_t stream) {
+Tensor encode(const Tensor& coords, int mode, int bits, int code_bits) {
     const c10::DeviceGuard guard(coords.device());
     const Tensor c = coords.contiguous();
     Tensor codes = make({c.size(0)}, code_bits == 32 ? at::kInt : at::kLong, c.device());
-    check(L.fgx_serialize_encode(mode, ptr<int32_t>(c), (size_t)c.size(0), bits, code_bits, ptr(codes), as_stream(stream)));
+    check(L.fgx_serialize_encode(mode, ptr<int32_t>(c), (size_t)c.size(0), bits, code_bits, ptr(codes), as_stream(stream_of(c))));
     return codes;
 }
 
-Tensor decode(const Tensor& codes, int mode, int bits, int code_bits, int64_t stream) {
+Tensor decode(const Tensor& codes, int mode, int bits, int code_bits) {
     const c10::DeviceGuard guard(codes.device());
     const Tensor c = codes.contiguous();
     Tensor coords = make({c.size(0), 4}, at::kInt, c.device());
-    check(L.fgx_serialize_decode(mode, ptr(c), (size_t)c.size(0), bits, code_bits, ptr<int32_t>(coords), as_stream(stream)));
+    check(L.fgx_serialize_decode(mode, ptr(c), (size_t)c.size(0), bits, code_bits, ptr<int32_t>(coords), as_stream(stream_of(c))));
     return coords;
 }
 
 // ---- the Python methods of the cache that make tables by themselves ----------------------------------------------------
-py::tuple py_tile_codes(py::object cache_obj, int block, bool own_order, int64_t stream) {
+py::tuple py_tile_codes(py::object cache_obj, int block, bool own_order) {
     const Cache c(std::move(cache_obj));
     Tiles t;
-    const c10::DeviceGuard guard(c.need("neighbor_map").device());
-    tile_codes(c, block, own_order, stream, &t, false);
+    const Tensor nmap = c.need("neighbor_map");
+    const c10::DeviceGuard guard(nmap.device());
+    tile_codes(c, block, own_order, stream_of(nmap), &t, false);
     return py::make_tuple(t.order, t.code);
 }
 
-py::tuple py_gather_plan(py::object cache_obj, int block, bool own_order, bool dense, int64_t stream) {
+py::tuple py_gather_plan(py::object cache_obj, int block, bool own_order, bool dense) {
     const Cache c(std::move(cache_obj));
-    const c10::DeviceGuard guard(c.need("neighbor_map").device());
-    const Tiles t = gather_plan(c, block, own_order, dense, 0, 0, 0, nullptr, stream);
+    const Tensor nmap = c.need("neighbor_map");
+    const c10::DeviceGuard guard(nmap.device());
+    const Tiles t = gather_plan(c, block, own_order, dense, 0, 0, 0, nullptr, stream_of(nmap));
     return py::make_tuple(t.order, t.code, t.plan_seg, t.plan_idx, t.plan_band, t.plan_key);
 }
 
-py::object py_item_order(py::object cache_obj, const std::string& plan_key, const Tensor& code, int col_tiles, int groups, int slabs, int64_t stream) {
+py::object py_item_order(py::object cache_obj, const std::string& plan_key, const Tensor& code, int col_tiles, int groups, int slabs) {
     const Cache c(std::move(cache_obj));
     const c10::DeviceGuard guard(code.device());
-    const Tensor t = item_order(c, plan_key, code, col_tiles, groups, slabs, stream);
+    const Tensor t = item_order(c, plan_key, code, col_tiles, groups, slabs, stream_of(code));
     return t.defined() ? py::cast(t) : py::none();
 }
 
-py::object py_wgrad_bounds(py::object cache_obj, int block_rows, int64_t stream) {
+py::object py_wgrad_bounds(py::object cache_obj, int block_rows) {
     const Cache c(std::move(cache_obj));
     const Tensor nmap = c.need("neighbor_map"), sig_o = c.need("valid_signal_o");
     const c10::DeviceGuard guard(nmap.device());
     const int v = (int)nmap.size(1);
-    return py::cast(wgrad_bounds(c, sig_o, seg_host(c, v), (size_t)nmap.size(0), v, block_rows, stream));
+    return py::cast(wgrad_bounds(c, sig_o, seg_host(c, v), (size_t)nmap.size(0), v, block_rows, stream_of(nmap)));
 }
 
-py::object py_wgrad_item_lists(py::object cache_obj, int block_rows, int tile_rows, int tile_cols, int ci, int co, int64_t stream) {
-    const Tensor bounds = py_wgrad_bounds(cache_obj, block_rows, stream).cast<Tensor>();
+py::object py_wgrad_item_lists(py::object cache_obj, int block_rows, int tile_rows, int tile_cols, int ci, int co) {
+    const Tensor bounds = py_wgrad_bounds(cache_obj, block_rows).cast<Tensor>();
     const Cache c(std::move(cache_obj));
     const Tensor nmap = c.need("neighbor_map");
     const c10::DeviceGuard guard(nmap.device());
     const Sched s{tile_rows, tile_cols, 0, 1, block_rows, 1};
-    const Tensor t = wgrad_item_lists(c, bounds, (size_t)nmap.size(0), (int)nmap.size(1), ci, co, s, stream);
+    const Tensor t = wgrad_item_lists(c, bounds, (size_t)nmap.size(0), (int)nmap.size(1), ci, co, s, stream_of(nmap));
     return t.defined() ? py::cast(t) : py::none();
 }
 
@@ -690,10 +977,11 @@ PYBIND11_MODULE(fgx_host, m) {
     m.def("subm_cache", &subm_cache);
     m.def("spconv_cache", &spconv_cache);
     m.def("out_coords", &out_coords);
+    m.def("convolve", &convolve);
     m.def("gather_gemm", &gather_gemm);
     m.def("wgrad", &wgrad);
-    m.def("relu_mask_apply", &relu_mask_apply);
-    m.def("colsum", &colsum);
+    m.def("relu_mask_apply", [](const Tensor& grad, const Tensor& mask) { return relu_mask_apply(grad, mask, stream_of(grad)); });
+    m.def("colsum", [](const Tensor& grad) { return colsum(grad, stream_of(grad)); });
     m.def("encode", &encode);
     m.def("decode", &decode);
     m.def("tile_codes", &py_tile_codes);

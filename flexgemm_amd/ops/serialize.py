@@ -45,7 +45,7 @@ def encode_seq(coords: torch.Tensor, shape: torch.Size, mode: Literal["z_order",
     if not coords.is_cuda:
         raise NotImplementedError("encode_seq runs on the GPU only: move coords to the device")
     assert coords.dtype == torch.int32, "Unsupported coords dtype. Expect int32"
-    return nat.host().encode(coords, code, bit_length, code_bits, nat.raw_stream(coords))
+    return nat.host().encode(coords, code, bit_length, code_bits)
 
 
 def decode_seq(code: torch.Tensor, shape: torch.Size, mode: Literal["z_order", "hilbert"] = "z_order") -> torch.Tensor:
@@ -61,7 +61,7 @@ def decode_seq(code: torch.Tensor, shape: torch.Size, mode: Literal["z_order", "
         raise RuntimeError("Unsupported input type")
     if not code.is_cuda:
         raise NotImplementedError("decode_seq runs on the GPU only: move the codes to the device")
-    return nat.host().decode(code, mode_code, bit_length, code_bits, nat.raw_stream(code))
+    return nat.host().decode(code, mode_code, bit_length, code_bits)
 
 
 def reorder_coords(coords: torch.Tensor, bit_length: int, batch_bits: int, mode_code: int) -> torch.Tensor:

@@ -20,8 +20,8 @@ from .. import spconv, utils
 from .. import serialize
 from . import Algorithm, SerializationMode, SparseConv3dOutCoordAlgorithm
 from .submanifold_conv3d import (EMPTY, _IMPLICIT, _MASKED, _NO_SPLITK, SubMConv3dNeighborCache, _codes_and_order, _colsum,
-                                 _gather_gemm, _gathered_rows, _grad_mode_of_the_caller, _gradients_possible, _pair_lists,
-                                 _pick_builder, _relu_mask_apply, _require_cuda, _wgrad, PAIR_LISTS_UNSIZED_MAX_BYTES)
+                                 _gather_gemm, _gathered_rows, _grad_mode_of_the_caller, _gradients_possible, _native_call, _pair_lists,
+                                 _pick_builder, _records_gradients, _relu_mask_apply, _require_cuda, _wgrad, PAIR_LISTS_UNSIZED_MAX_BYTES)
 
 
 def _triple(x) -> Tuple[int, int, int]:
@@ -100,8 +100,7 @@ def _build_cache_one_call(coords: torch.Tensor, out_coords: torch.Tensor, shape,
     if spconv.NEIGHBOR_MAP_BUILDER not in ("auto", "grid"):
         return None
     B, _, W, H, D = [int(s) for s in shape]
-    return nat.host().spconv_cache(coords, out_coords, [B, W, H, D, *ks, *st, *pd, *dl], needs_grad, bwd_order, PAIR_LISTS_UNSIZED_MAX_BYTES,
-                                   nat.raw_stream(coords))
+    return nat.host().spconv_cache(coords, out_coords, [B, W, H, D, *ks, *st, *pd, *dl], needs_grad, bwd_order, PAIR_LISTS_UNSIZED_MAX_BYTES)
 
 
 def _build_maps(coords: torch.Tensor, out_coords: torch.Tensor, shape, kernel_size, stride, padding, dilation,
@@ -205,8 +204,8 @@ class SparseConv3dFunction(Function):
         if vol >= 2 ** 64 - 1:
             raise ValueError("The spatial size is too large. Require B*W*H*D < 2^64.")
         L = nat.lib()
-        if spconv.NEIGHBOR_MAP_BUILDER in ("auto", "grid") and not torch.cuda.is_current_stream_capturing():
-            out = nat.host().out_coords(coords, [B, W, H, D, *ks, *st, *pd, *dl], nat.raw_stream(coords))
+        if spconv.NEIGHBOR_MAP_BUILDER in ("auto", "grid"):
+            out = nat.host().out_coords(coords, [B, W, H, D, *ks, *st, *pd, *dl])
             if out is not None:
                 return SparseConv3dFunction._serialized(out, mode, (B, W, H, D), (wo, ho, do))
         key_bits = 32 if vol < 2 ** 32 - 1 else 64
@@ -492,6 +491,24 @@ class SparseConv3dFunction(Function):
         return grad_input, None, None, None, grad_weight, grad_bias, None, None, None, None, None
 
 
+def _convolve(feats, coords, shape, weight, bias, neighbor_cache, out_coords, stride, padding, dilation, relu: bool):
+    """(output, output coordinates, cache): see the submanifold operator's _convolve."""
+    if not _native_call(feats):
+        with _grad_mode_of_the_caller():
+            return SparseConv3dFunction.apply(feats, coords, shape, neighbor_cache, weight, bias, out_coords, stride, padding, dilation, relu)
+    algo = spconv.ALGORITHM
+    assert feats.shape[-1] == weight.shape[-1], f"Input channels ({feats.shape[-1]}) should match weight channels ({weight.shape[-1]})"
+    given = out_coords is not None
+    kernel = tuple(weight.shape[1:4])
+    if not given:
+        out_coords = SparseConv3dFunction._get_output_coords(coords, shape, kernel, stride, padding, dilation)
+    if neighbor_cache is None:
+        neighbor_cache = SparseConv3dFunction._compute_neighbor_cache(coords, out_coords, shape, kernel, stride, padding, dilation,
+                                                                      _records_gradients(feats, weight, bias), given)
+    out = nat.host().convolve(feats, neighbor_cache, weight, bias, relu, True, algo in _MASKED, algo not in _NO_SPLITK)
+    return out, out_coords, neighbor_cache
+
+
 def sparse_conv3d(
     feats: torch.Tensor,
     coords: torch.Tensor,
@@ -522,9 +539,7 @@ def sparse_conv3d(
     Returns:
         (out_feats [M, Co], out_coords [M, 4], neighbor_cache)
     """
-    with _grad_mode_of_the_caller():
-        return SparseConv3dFunction.apply(feats, coords, shape, neighbor_cache, weight, bias, out_coords, stride, padding,
-                                          dilation)
+    return _convolve(feats, coords, shape, weight, bias, neighbor_cache, out_coords, stride, padding, dilation, False)
 
 
 def sparse_conv3d_relu(
@@ -542,6 +557,4 @@ def sparse_conv3d_relu(
     """relu(sparse_conv3d(...)) with the clamp done in the GEMM's epilogue (no counterpart in the reference; same
     arguments and return values as sparse_conv3d).  Differentiable: backward masks the incoming gradient with the sign
     of the saved output and runs the usual passes."""
-    with _grad_mode_of_the_caller():
-        return SparseConv3dFunction.apply(feats, coords, shape, neighbor_cache, weight, bias, out_coords, stride, padding,
-                                          dilation, True)
+    return _convolve(feats, coords, shape, weight, bias, neighbor_cache, out_coords, stride, padding, dilation, True)

@@ -94,7 +94,7 @@ class SubMConv3dNeighborCache:
         if private:
             self._ensure_tile_order()
         use_private = private and hasattr(self, "_tile_order")
-        order, code = nat.host().tile_codes(self, block_size, use_private, nat.raw_stream(self["gray_code"]))
+        order, code = nat.host().tile_codes(self, block_size, use_private)
         seg_key = f"_tile_seg_{block_size}" if use_private else f"valid_kernel_seg_{block_size}"
         if not hasattr(self, seg_key):
             seg = torch.empty((code.shape[0] + 1,), dtype=torch.int32, device=code.device)
@@ -127,13 +127,12 @@ class SubMConv3dNeighborCache:
         allocated at their bound (every offset present in every tile), plan_seg[-1] rows of them are used."""
         if private and not dense:
             self._ensure_tile_order()
-        return nat.host().gather_plan(self, block_size, private and not dense and hasattr(self, "_tile_order"), dense,
-                                      nat.raw_stream(self["neighbor_map"]))
+        return nat.host().gather_plan(self, block_size, private and not dense and hasattr(self, "_tile_order"), dense)
 
     def _item_order(self, plan_key: str, code: torch.Tensor, col_tiles: int, groups: int, slabs: int):
         """uint32 device tensor for fgx_conv_gather_gemm_stream's item_at (or None): the tiles dealt to the persistent
         workgroups by cost, built on the device (no read-back) once per plan and shape and kept with the cache."""
-        return nat.host().item_order(self, plan_key, code, col_tiles, groups, slabs, nat.raw_stream(code))
+        return nat.host().item_order(self, plan_key, code, col_tiles, groups, slabs)
 
     def compute_kernel_idx(self, block_size: int):
         """Fill `valid_kernel_{B}` / `valid_kernel_seg_{B}` (reference: submanifold_conv3d.py:20-23,
@@ -212,12 +211,12 @@ class SubMConv3dNeighborCache:
     def _wgrad_bounds(self, block_rows: int):
         """First pair of every (offset, voxel block) for wgrad's blocks of `block_rows` rows: a function of the pair lists
         alone, so it is made once per block size and kept."""
-        return nat.host().wgrad_bounds(self, block_rows, nat.raw_stream(self["neighbor_map"]))
+        return nat.host().wgrad_bounds(self, block_rows)
 
     def _wgrad_item_lists(self, block_rows: int, tile_rows: int, tile_cols: int, ci: int, co: int):
         """Balanced work lists of the streaming weight gradient (fgx_wgrad_item_lists) for one block size, tile shape and
         channel counts, made on the device from the block table and kept; None where the library has none for the shape."""
-        return nat.host().wgrad_item_lists(self, block_rows, tile_rows, tile_cols, ci, co, nat.raw_stream(self["neighbor_map"]))
+        return nat.host().wgrad_item_lists(self, block_rows, tile_rows, tile_cols, ci, co)
 
     def _wgrad_sweep_plan(self, sub_rows: int):
         """Step lists of the paced wgrad sweep (fgx_wgrad_sweep_plan): a function of the pair lists and the sub-block
@@ -456,7 +455,7 @@ def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, ne
     v = kw * kh * kd
     if spconv.NEIGHBOR_MAP_BUILDER in ("auto", "grid"):
         built = nat.host().subm_cache(coords, [B, W, H, D, kw, kh, kd, int(dilation[0]), int(dilation[1]), int(dilation[2])], needs_grad,
-                                      spconv.NEIGHBOR_MAP_BUILDER == "grid", PAIR_LISTS_UNSIZED_MAX_BYTES, nat.raw_stream(coords))
+                                      spconv.NEIGHBOR_MAP_BUILDER == "grid", PAIR_LISTS_UNSIZED_MAX_BYTES)
         if built is not None:
             nmap, gray, binary, order, seg, sig_i, sig_o, arriving = built
             return nmap, gray, binary, order, ({"seg": seg, "pending": (sig_i, sig_o, arriving, arriving)} if needs_grad else None)
@@ -595,76 +594,43 @@ def _gather_gemm(src: torch.Tensor, weight_cvk: torch.Tensor, bias: Optional[tor
     activation: nat.ACT_RELU clamps (sum + bias) at zero in the kernel's epilogue.  relu_mask_out: a list; where the kernels
     can (ReLU, 16-bit type, a multiple of 8 output columns) they also write one bit per output, "greater than zero", and
     the uint8 tensor [n * cols / 8] holding them is appended to the list."""
-    co, v, ci = weight_cvk.shape
-    n = cache["neighbor_map"].shape[0]
-    n_src = src.shape[0]
-    dt = src.dtype
-    if dt not in nat.DTYPE_CODE:
-        raise TypeError(f"unsupported feature dtype {dt}; expected float16, bfloat16 or float32")
-    if weight_cvk.dtype != dt or (bias is not None and bias.dtype != dt):
-        raise TypeError("features, weight and bias must share one dtype")
-    k_true, cols = (ci, co) if mode == 0 else (co, ci)
-    dev = src.device
-    if n_src == 0:      # nothing to gather: the bias alone
-        out = torch.zeros((n, cols), dtype=dt, device=dev)
-        out = out if bias is None else out + bias
-        return torch.relu(out) if activation == nat.ACT_RELU else out
-    # rows must be whole 16-byte chunks: zero-pad the contraction dimension when they are not
-    align = 16 // src.element_size()
-    if k_true % align:
-        src = _pad_cols(src, align)
-        weight_owner = None             # the padded copy is made per call: nothing to key a kept panel on
-        if mode == 0:
-            weight_cvk = _pad_cols(weight_cvk, align)
-        else:
-            weight_cvk = torch.nn.functional.pad(weight_cvk, (0, 0, 0, 0, 0, (-co) % align))
-        co, v, ci = weight_cvk.shape
-    k = ci if mode == 0 else co
-    src = src.contiguous()
-    weight_cvk = weight_cvk.contiguous()
-    if bias is not None:
-        bias = bias.contiguous()        # the kernels read it with stride 1 (a view such as a column of a matrix has another)
-    sched = nat.table_lookup(nat.PASS_FWD if mode == 0 else nat.PASS_DGRAD, dt, n, ci, co, v)
-    splitk = sched.splitk if allow_splitk else 1
-    if masked:
-        cache._ensure_sorted()
-    private = masked and _locality_applies(cache, n, k * src.element_size())
-    if n == 0:
-        return torch.empty((n, cols), dtype=dt, device=dev)
-    code = nat.DTYPE_CODE[dt]
-    want_mask = relu_mask_out is not None and activation == nat.ACT_RELU
-    narrow = _narrow_applies(cache, src, k, cols, v, n, n_src, sched)
     panel = None
-    if narrow or (spconv.WEIGHT_PANEL_CACHE and weight_owner is not None):
-        with torch.cuda.device(dev):
-            panel = _weight_panel(weight_owner, weight_cvk, code, mode, sched, dev)
-    if narrow:
-        L = nat.lib()
-        name = "gather_gemm_fwd" if mode == 0 else "gather_gemm_dgrad"
-        out = torch.empty((n, cols), dtype=dt, device=dev)
-        mask = torch.empty((n * cols // 8,), dtype=torch.uint8, device=dev) if want_mask and cols % 8 == 0 else None
-        with torch.cuda.device(dev):
-            plan = cache._narrow_plan()
-            nat.mark(name, "start")
-            nat.check(L.fgx_conv_narrow_gemm(
-                C.c_int(code), nat.ptr(src), nat.ptr(panel), nat.ptr(bias), nat.ptr(cache["neighbor_map"]), nat.ptr(plan),
-                nat.sz(n), nat.sz(n_src), C.c_int(k), C.c_int(cols), C.c_int(v), C.c_int(activation), nat.ptr(out), nat.ptr(mask),
-                nat.stream()))
-            nat.mark(name, "stop")
-    else:
-        if private:
-            cache._ensure_tile_order()
-        out, mask = nat.host().gather_gemm(src, weight_cvk, bias, cache, mode, splitk, masked, private and hasattr(cache, "_tile_order"), activation,
-                                           want_mask, sched, panel, _stream_fits(n, n_src, k * src.element_size()), nat.raw_stream(src))
+    if weight_owner is not None and spconv.WEIGHT_PANEL_CACHE and weight_cvk.shape[2 if mode == 0 else 0] % (16 // src.element_size()) == 0:
+        # (the padded copy of another width is made per call: nothing to key a kept panel on)
+        co, v, ci = weight_cvk.shape
+        if src.dtype in nat.DTYPE_CODE and weight_cvk.dtype == src.dtype and src.shape[0] > 0 and cache["neighbor_map"].shape[0] > 0:
+            sched = nat.table_lookup(nat.PASS_FWD if mode == 0 else nat.PASS_DGRAD, src.dtype, cache["neighbor_map"].shape[0], ci, co, v)
+            with torch.cuda.device(src.device):
+                panel = _weight_panel(weight_owner, weight_cvk.contiguous(), nat.DTYPE_CODE[src.dtype], mode, sched, src.device)
+    out, mask = nat.host().gather_gemm(src, weight_cvk, bias, cache, mode, allow_splitk, masked, activation, relu_mask_out is not None, panel)
     if mask is not None:
         relu_mask_out.append(mask)
     return out
 
 
+def _narrow_gemm(src: torch.Tensor, panel: torch.Tensor, bias: Optional[torch.Tensor], cache, mode: int, k: int, cols: int, v: int,
+                 activation: int, want_mask: bool):
+    """(output, ReLU bit mask or None) of the gather GEMM on the resident-row kernel (_narrow_applies has agreed)."""
+    n = cache["neighbor_map"].shape[0]
+    L = nat.lib()
+    name = "gather_gemm_fwd" if mode == 0 else "gather_gemm_dgrad"
+    out = torch.empty((n, cols), dtype=src.dtype, device=src.device)
+    mask = torch.empty((n * cols // 8,), dtype=torch.uint8, device=src.device) if want_mask and activation == nat.ACT_RELU else None
+    with torch.cuda.device(src.device):
+        plan = cache._narrow_plan()
+        nat.mark(name, "start")
+        nat.check(L.fgx_conv_narrow_gemm(
+            C.c_int(nat.DTYPE_CODE[src.dtype]), nat.ptr(src), nat.ptr(panel), nat.ptr(bias), nat.ptr(cache["neighbor_map"]), nat.ptr(plan),
+            nat.sz(n), nat.sz(src.shape[0]), C.c_int(k), C.c_int(cols), C.c_int(v), C.c_int(activation), nat.ptr(out), nat.ptr(mask),
+            nat.stream()))
+        nat.mark(name, "stop")
+    return out, mask
+
+
 def _relu_mask_apply(grad_output: torch.Tensor, mask: torch.Tensor) -> torch.Tensor:
     """grad_output where the forward pass's bit mask says the activated output was positive, zero elsewhere
     (fgx_relu_mask_apply: one pass that reads an eighth of a byte per element beside the gradient)."""
-    return nat.host().relu_mask_apply(grad_output, mask, nat.raw_stream(grad_output))
+    return nat.host().relu_mask_apply(grad_output, mask)
 
 
 def _narrow_applies(cache, src: torch.Tensor, k: int, cols: int, v: int, n: int, n_src: int, sched) -> bool:
@@ -768,41 +734,29 @@ def _wgrad(grad_output: torch.Tensor, feats: torch.Tensor, cache, v: int, with_b
     that map, feats one per row the map points at.  with_bias: also the bias gradient (column sums of grad_output),
     returned as a second value; bias_offset names an offset whose pairs hold every row of grad_output exactly once (the
     centre of a submanifold convolution), which lets the streaming kernel sum the rows it loads anyway."""
-    n_in, ci = feats.shape
-    n, co = grad_output.shape
-    dt = feats.dtype
-    dev = feats.device
-    align = 16 // feats.element_size()
-    f = _pad_cols(feats, align).contiguous()
-    g = _pad_cols(grad_output, align).contiguous()
-    cip, cop = f.shape[1], g.shape[1]
-    if _narrow_wgrad_applies(cache, f, cip, cop, v, n, n_in):
-        # narrow layers on a cache that has the resident-row plan: the chunk's rows gathered in LDS (fgx_conv_narrow_wgrad)
-        L = nat.lib()
-        gw = torch.empty((cop, v, cip), dtype=dt, device=dev)
-        with torch.cuda.device(dev):
-            scratch = nat.workspace(L.fgx_narrow_wgrad_scratch_bytes(C.c_int(v)), dev)
-            nat.mark("wgrad", "start")
-            nat.check(L.fgx_conv_narrow_wgrad(C.c_int(nat.DTYPE_CODE[dt]), nat.ptr(g), nat.ptr(f), nat.ptr(cache._narrow_plan()),
-                                              nat.sz(n), nat.sz(n_in), C.c_int(cip), C.c_int(cop), C.c_int(v), nat.ptr(scratch),
-                                              nat.ptr(gw), nat.stream()))
-            gb = _colsum(g) if with_bias else None
-            nat.mark("wgrad", "stop")
-        if cip != ci or cop != co:
-            gw = gw[:co, :, :ci].contiguous()
-            gb = gb[:co].contiguous() if with_bias else None
-        return (gw, gb) if with_bias else gw
-    cache._ensure_pairs()
-    sched = nat.table_lookup(nat.PASS_WGRAD, dt, n, cip, cop, v)
-    gw, gb = nat.host().wgrad(g, f, cache, v, with_bias, bias_offset, sched, nat.raw_stream(f))
-    if cip != ci or cop != co:
-        gw = gw[:co, :, :ci].contiguous()
-        gb = gb[:co].contiguous() if with_bias else None
+    gw, gb = nat.host().wgrad(grad_output, feats, cache, v, with_bias, bias_offset)
     return (gw, gb) if with_bias else gw
 
 
+def _narrow_wgrad(g: torch.Tensor, f: torch.Tensor, cache, v: int, with_bias: bool):
+    """(weight gradient, bias gradient or None) of a narrow layer on a cache that has the resident-row plan: the chunk's rows
+    gathered in LDS (fgx_conv_narrow_wgrad; _narrow_wgrad_applies has agreed)."""
+    L = nat.lib()
+    n, n_in, ci, co = g.shape[0], f.shape[0], f.shape[1], g.shape[1]
+    gw = torch.empty((co, v, ci), dtype=f.dtype, device=f.device)
+    with torch.cuda.device(f.device):
+        scratch = nat.workspace(L.fgx_narrow_wgrad_scratch_bytes(C.c_int(v)), f.device)
+        nat.mark("wgrad", "start")
+        nat.check(L.fgx_conv_narrow_wgrad(C.c_int(nat.DTYPE_CODE[f.dtype]), nat.ptr(g), nat.ptr(f), nat.ptr(cache._narrow_plan()),
+                                          nat.sz(n), nat.sz(n_in), C.c_int(ci), C.c_int(co), C.c_int(v), nat.ptr(scratch),
+                                          nat.ptr(gw), nat.stream()))
+        gb = _colsum(g) if with_bias else None
+        nat.mark("wgrad", "stop")
+    return gw, gb
+
+
 def _colsum(grad_output: torch.Tensor) -> torch.Tensor:
-    return nat.host().colsum(grad_output, nat.raw_stream(grad_output))
+    return nat.host().colsum(grad_output)
 
 
 def _gathered_rows(src: torch.Tensor, nmap: torch.Tensor) -> torch.Tensor:
@@ -1047,6 +1001,30 @@ class SubMConv3dFunction(Function):
         return grad_input, None, None, None, grad_weight, grad_bias, None, None
 
 
+def _native_call(feats: torch.Tensor) -> bool:
+    """Whether an operator call goes through the native host side, autograd node included (the implicit algorithms on the
+    GPU); the Python functions serve the others and calls that keep weight panels with their weights."""
+    return feats.is_cuda and not spconv.WEIGHT_PANEL_CACHE and spconv.ALGORITHM in _IMPLICIT
+
+
+def _records_gradients(feats: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
+    return torch.is_grad_enabled() and (feats.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad))
+
+
+def _convolve(feats, coords, shape, weight, bias, neighbor_cache, dilation, relu: bool):
+    """(output, cache) of a submanifold layer: the cache built when the caller has none, the product and its autograd node
+    made natively (nat.host().convolve)."""
+    if not _native_call(feats):
+        with _grad_mode_of_the_caller():
+            return SubMConv3dFunction.apply(feats, coords, shape, neighbor_cache, weight, bias, dilation, relu)
+    algo = spconv.ALGORITHM
+    if neighbor_cache is None:
+        assert feats.shape[-1] == weight.shape[-1], f"Input channels ({feats.shape[-1]}) should match weight channels ({weight.shape[-1]})"
+        neighbor_cache = SubMConv3dFunction._compute_neighbor_cache(coords, shape, tuple(weight.shape[1:4]), dilation,
+                                                                    _records_gradients(feats, weight, bias))
+    return nat.host().convolve(feats, neighbor_cache, weight, bias, relu, False, algo in _MASKED, algo not in _NO_SPLITK), neighbor_cache
+
+
 def sparse_submanifold_conv3d(
     feats: torch.Tensor,
     coords: torch.Tensor,
@@ -1072,8 +1050,7 @@ def sparse_submanifold_conv3d(
     Returns:
         (output [N, Co], neighbor_cache)
     """
-    with _grad_mode_of_the_caller():
-        return SubMConv3dFunction.apply(feats, coords, shape, neighbor_cache, weight, bias, dilation)
+    return _convolve(feats, coords, shape, weight, bias, neighbor_cache, dilation, False)
 
 
 def sparse_submanifold_conv3d_relu(
@@ -1088,5 +1065,4 @@ def sparse_submanifold_conv3d_relu(
     """relu(sparse_submanifold_conv3d(...)) with the clamp done in the GEMM's epilogue: the output is written once,
     already activated (no counterpart in the reference; same arguments and return values as sparse_submanifold_conv3d).
     Differentiable: backward masks the incoming gradient with the sign of the saved output and runs the usual passes."""
-    with _grad_mode_of_the_caller():
-        return SubMConv3dFunction.apply(feats, coords, shape, neighbor_cache, weight, bias, dilation, True)
+    return _convolve(feats, coords, shape, weight, bias, neighbor_cache, dilation, True)
