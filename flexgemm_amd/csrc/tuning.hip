@@ -41,7 +41,73 @@ int pick_cols(int c) { return c > 64 ? 128 : (c > 32 ? 64 : 32); }
 
 size_t round_up(size_t x, size_t m) { return (x + m - 1) / m * m; }
 
+// fp32: the matrix units take 32-bit operands at a sixteenth of the 16-bit rate, so every pass is bound by what is multiplied --
+// padding and idle CUs included -- long before loads count, and the choice is the one with the least of both.
+//
+// Weight gradient: 64 x 64 tiles, or 32 x 32 where those pad at least 28 % less (a 32 x 32 tile multiplies at about that
+// much less: 64 160 voxels x 64 channels 0.169 against 0.122 ms), over voxel blocks short enough for about 2000 items of the
+// larger tile: an item is (block, offset, tile), and with fewer the centre offset's items alone decide the time.
+// Measured (ms; before: 128 x 128 tiles over blocks of 4096 rows and more):  96 channels, 38 720 voxels 0.513 -> 0.202;
+// 155 096 voxels 1.08 -> 0.66;  128 channels, 3 840 voxels 0.275 -> 0.038;  166 232 voxels 0.81 -> 0.60;  64 channels,
+// 15 192 voxels 0.096 -> 0.045;  16 channels, 669 288 voxels 0.75 -> 0.45.  From 1024 x 1024 channels on, where partial products
+// must stay few and blocks are long, the 128 x 128 tile of the general rule is ahead (42 608 voxels: 9.5 ms against 10.3).
+bool rule_wgrad_f32(size_t n, int Ci, int Co, int V, fgx_schedule* out) {
+    if ((size_t)Ci * Co >= (size_t)1024 * 1024) return false;
+    auto padded = [&](int t) { return (double)cdiv(Ci, t) * t * cdiv(Co, t) * t; };
+    const int t = padded(32) < 0.72 * padded(64) ? 32 : 64;
+    const double tiles = (double)cdiv(Ci, t) * cdiv(Co, t);
+    const double ideal = (double)n * V * tiles / (t == 64 ? 2000.0 : 4000.0);
+    size_t rows = V * tiles < 400 ? 512 : 1024;
+    while (rows < 4096 && ideal > 1.42 * rows) rows *= 2;
+    const double per_block = 4.0 * V * (double)Co * Ci;            // partial products stay below 256 MiB
+    while ((double)cdiv(n ? n : 1, rows) * per_block > 268435456.0 && rows < ((size_t)1 << 29)) rows *= 2;
+    if (n > rows) rows = round_up(cdiv(n, cdiv(n, rows)), 64);       // even blocks
+    *out = fgx_schedule{t, t, 64, 1, (int)rows, 0};
+    return true;
+}
+
+// Gather GEMM: what a CU multiplies, in columns of 256-row tiles, under each choice.
+//   streaming kernel, tiles of 256 x c: whole items per CU, c columns each, at a rate that falls a little with c; a lone
+//   32-column item leaves the matrix units waiting for its loads half as long again;
+//   tiled kernel with K split until the pieces even out: the columns of all tiles over the CUs, at about 0.72 of the rate.
+// Measured forward (ms; before: 128-column tiles from 65 columns on):  38 720 voxels, 96 channels 0.285 -> 0.159;  40 -> 200
+// channels 0.270 -> 0.173;  155 096 voxels, 96 channels 0.606 -> 0.437;  24 488 voxels, 320 channels 1.37 -> 0.87;  101 304
+// voxels, 48 channels 0.141 -> 0.109;  64 160 voxels, 32 channels 0.058 -> 0.045;  tiled: 8 624 voxels, 96 channels 0.108 ->
+// 0.069, 512 channels 1.52 -> 0.99;  38 720 voxels, 160 -> 24 channels 0.200 -> 0.118;  344 voxels, 128 channels 0.043 -> 0.028.
+void rule_gemm_f32(size_t n, int K, int cols, int V, fgx_schedule* out) {
+    const size_t row_bytes = (size_t)K * 4;
+    const int slab = row_bytes >= 128 ? 128 : 64;
+    const double row_tiles = cdiv(n ? n : 1, 256);
+    const int wide = cdiv(cols, 64) * 64;
+    const bool narrow = cdiv(cols, 32) * 32 < wide;
+    double best = row_tiles * (narrow ? cdiv(cols, 32) * 32 : wide) / kCUs / 0.72;
+    *out = fgx_schedule{narrow && n < 1024 ? 32 : 64, narrow ? 32 : 64, 64, 1, 0, 0};
+    if (cdiv(cols, 128) * 128 == wide && row_bytes >= 1024 && cdiv(n ? n : 1, 128) * cdiv(cols, 128) >= 32) out->tile_rows = out->tile_cols = 128;
+    {
+        const size_t tiles = (size_t)cdiv(n ? n : 1, out->tile_rows) * cdiv(cols, out->tile_cols);
+        const int steps = V * (int)cdiv(row_bytes, (size_t)64);
+        int s = 1;
+        while (tiles * s < (s < 8 ? 1500u : 300u) && s < 16 && 12 * s <= steps) s *= 2;
+        out->splitk = s;
+    }
+    if (row_bytes < 64) return;
+    struct Shape { int rows, cols, slab; double rate; };
+    const Shape shapes[] = {{128, 256, 128, 1.08}, {256, 128, 128, 1.0}, {256, 64, slab, 0.98}, {256, 32, 64, 0.92}};
+    for (const Shape& sh : shapes) {
+        if (sh.slab > (int)align_up(row_bytes, 64) || (sh.cols == 256 && cols <= 128) || !stream_lds_fits(sh.rows, sh.cols, sh.slab, cols)) continue;
+        const size_t items = (size_t)cdiv(n ? n : 1, sh.rows) * cdiv(cols, sh.cols);
+        const double each = sh.cols * sh.rows / 256.0 / sh.rate;
+        const double time = cdiv(items, (size_t)kCUs) * each * (sh.cols == 32 && items <= (size_t)kCUs ? 1.5 : 1.0);
+        if (time < best) {
+            best = time;
+            *out = fgx_schedule{sh.rows, sh.cols, sh.slab, 1, 0, 1};
+        }
+    }
+}
+
 void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* out) {
+    if (es == 4 && pass_kind != 2) return rule_gemm_f32(n, pass_kind == 0 ? Ci : Co, pass_kind == 0 ? Co : Ci, V, out);
+    if (es == 4 && rule_wgrad_f32(n, Ci, Co, V, out)) return;
     if (pass_kind == 2) {
         // wgrad: tiles over (Co, Ci) and voxel blocks; an item is (block, offset, tile), every item costs an exposed
         // epilogue and a partial product, and the fp32 partial products (blocks x V x Co x Ci) stay below 256 MiB.
