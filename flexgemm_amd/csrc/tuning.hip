@@ -130,6 +130,17 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
             out->block_rows = 2048;
             return;
         }
+        // 33 ... 64 channels on one side and over 192 on the other, or over 128 of many voxels: three and more 64 x 64 tiles.  The tiled kernel over short
+        // blocks is ahead of the streaming one, whose workgroups walk one tile's pairs at a time (256 -> 64 channels, 38 720
+        // voxels: 0.057 against 0.071 ms; 64 -> 160 channels, 228 816 voxels: 0.178 against 0.219).
+        if (out->stream == 1 && t == 64 && (Ci > 192 || Co > 192 || ((Ci > 128 || Co > 128) && n >= 98304)) && n >= 12288) {
+            out->stream = 0;
+            size_t rows = n >= 98304 ? 4096 : 2048;
+            const double per_block = 4.0 * V * (double)Co * Ci;
+            while ((double)cdiv(n, rows) * per_block > 268435456.0 && rows < ((size_t)1 << 29)) rows *= 2;
+            out->block_rows = (int)round_up(cdiv(n, cdiv(n, rows)), 64);
+            return;
+        }
         // Streaming kernel with balanced work lists (fgx_wgrad_item_lists): a launch takes as long as its most loaded
         // workgroup, and the lists even the loads out as far as the items allow -- the largest item is the centre
         // offset of a voxel block (one pair per row), the mean load is about 0.45 V pairs per voxel x tiles / CUs.
@@ -172,9 +183,15 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
                 out->tile_rows = shapes[i].rows;
                 out->tile_cols = shapes[i].cols;
                 const bool fills = 2 * (size_t)V * tiles * nb >= 3 * (size_t)kCUs;
-                if (last && !fills) {                           // nothing fills the chip: blocks down to 2048 rows
-                    const size_t most_short = n > 2048 ? cdiv(n, (size_t)2048) : 1;
+                if (last && !fills) {
+                    // nothing fills the chip: blocks down to 1024 rows (64 channels, 3 840 voxels: 0.020 -> 0.016 ms), 2048 where
+                    // the tile splits its pairs over the wavefronts itself or two short blocks would be all (1 976 voxels,
+                    // 64 -> 384 channels: 0.020 ms, one block 0.016)
+                    const size_t least = (slices == 4 || n < 3072) ? 2048 : 1024;
+                    const size_t most_short = n > least ? cdiv(n, least) : 1;
+                    const size_t filling = cdiv((size_t)3 * kCUs, (size_t)2 * V * tiles);
                     nb = wanted < most_short ? wanted : most_short;
+                    if (nb > filling) nb = filling;
                 }
                 if (last || fills) break;
             }
@@ -220,62 +237,69 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
         return;
     }
     const int cols = pass_kind == 0 ? Co : Ci;
-    out->tile_cols = pick_cols(cols);
-    out->tile_rows = n >= 4096 ? 128 : (n >= 1024 ? 64 : 32);
-    if (out->tile_rows == 64 && out->tile_cols == 128) out->tile_rows = 128;
-    if (out->tile_rows == 32 && out->tile_cols != 32) out->tile_rows = out->tile_cols == 64 ? 64 : 128;
-    // narrow outputs with fewer 128-row tiles than CUs: 64-row tiles before any split of K (15 192 voxels, C = 64: 0.036 ->
-    // 0.030 ms)
-    if (out->tile_rows == 128 && out->tile_cols == 64 && (size_t)cdiv(n, 128) * cdiv(cols, 64) < (size_t)kCUs) out->tile_rows = 64;
+    const int K = pass_kind == 0 ? Ci : Co;
+    const size_t row_bytes = (size_t)K * es;
+    // Tiled kernel: 64 x 64 tiles (one of 32 columns where there are no more), 128 x 128 once splits of four go round with
+    // those; K split until the CUs have one to three pieces each, as many as the tile's size leaves room for.  A piece's partial
+    // sums are written and read again, so more than eight only of a long K.  (848 voxels: 8 splits against 16, C = 32 0.015 ->
+    // 0.013 ms; C = 80 128 x 128 in 16 splits 0.022, these 0.016; 3 840 voxels, C = 128: 0.030 -> 0.026 in 4; 13 488 voxels,
+    // C = 128: 128 x 128 in 4 0.042, 64 x 64 0.053; 15 192 voxels, 320 -> 16 channels in 2 0.060, in 4 0.044.)
+    // A long K keeps the larger tile, which reads half as much per product: 256 channels and more
+    // (848 voxels, 256 -> 768 channels: 0.042 ms, 64 x 64 0.062; 1 976 voxels, 256 channels: 0.034 and 0.038).
+    out->tile_rows = (cols > 32 || n >= 1024) ? 64 : 32;
+    out->tile_cols = cols > 32 ? 64 : 32;
+    const bool long_k = row_bytes >= 512 && n >= 256;
+    if (cols > 64 && (long_k || (size_t)cdiv(n, 128) * cdiv(cols, 128) >= (size_t)kCUs / 4)) out->tile_rows = out->tile_cols = 128;
+    else if (cols > 32 && cols <= 64 && (size_t)cdiv(n, 128) >= 2 * (size_t)kCUs) out->tile_rows = 128;
     out->block_rows = 0;
     out->stream = 0;
     out->slab_bytes = 64;
-    // split K only when the tiles cannot fill the chip (reference: candidates start at #SM / blocks)
-    size_t tiles = (size_t)cdiv(n, out->tile_rows) * cdiv(cols, out->tile_cols);
+    const size_t tiles = (size_t)cdiv(n ? n : 1, out->tile_rows) * cdiv(cols, out->tile_cols);
     int s = 1;
-    while (tiles * s < (size_t)kCUs && s < 16) s *= 2;
+    const size_t steps = (size_t)V * cdiv(row_bytes, (size_t)64);
+    for (; s < (steps >= 160 ? 16 : 8); s *= 2) {
+        size_t pieces = cols <= 32 ? 700 : kCUs;
+        if (out->tile_cols == 64 && (s < 4 ? steps >= 54 : (s < 8 && steps >= 320))) pieces = 450;
+        if (tiles * s >= pieces) break;
+    }
     out->splitk = s;
-    // persistent streaming kernel (256-row tiles): rows of at least 64 bytes -- 128-byte K-slabs from 128 bytes on, 64-byte
-    // ones below, where 32 output columns get a tile of their own.  With 128-byte slabs it is ahead of the tiled kernel
-    // as soon as there is an item for a little under half of the CUs (measured: 120 items 10 % ahead, 64 items 13 %
-    // behind); the short-row form, two workgroups per CU, keeps the bar of two items per CU.
-    const int K = pass_kind == 0 ? Ci : Co;
-    const size_t row_bytes = (size_t)K * es;
-    // 16-bit rows of 128 ... 255 bytes (64 ... 127 channels) also take the 64-byte slabs: their rings leave room for two
-    // workgroups per CU, which is worth more than the longer pieces (measured forward, C = 64: 143 616 / 252 392 / 577 592 /
-    // 1 026 536 voxels -5 / -22 / -7 / -12 %; C = 80 and 96: -2 ... -5 %; from 256 bytes on the 128-byte slabs are ahead,
-    // C = 128: 0.049 against 0.056 ms at 64 160 voxels)
-    // ... given two items per CU to keep both workgroups busy (64 160 voxels, 251 items: 0.028 ms on 128-byte slabs, 0.031 on
-    // 64-byte ones)
-    const bool short_slabs = es == 2 && row_bytes >= 128 && row_bytes < 256 &&
+    // Persistent streaming kernel: rows of at least 64 bytes; 64-byte K-slabs below 128 bytes, 128-byte ones from there on.
+    // 16-bit rows of 128 ... 255 bytes (64 ... 127 channels) also take the 64-byte slabs while one column tile holds the outputs:
+    // their rings leave room for two workgroups per CU, which is worth more than the longer pieces (measured forward, C = 64:
+    // 143 616 / 252 392 / 577 592 / 1 026 536 voxels -5 / -22 / -7 / -12 %; C = 80 and 96: -2 ... -5 %; from 256 bytes on the
+    // 128-byte slabs are ahead, C = 128: 0.049 against 0.056 ms at 64 160 voxels) ... given two items per CU to keep both
+    // workgroups busy (64 160 voxels, 251 items: 0.028 ms on 128-byte slabs, 0.031 on 64-byte ones)
+    const bool short_slabs = row_bytes >= 128 && row_bytes < 256 && cols <= 128 &&
                              (size_t)cdiv(n, 256) * cdiv(cols, cols > 64 ? 128 : 64) >= 2 * (size_t)kCUs;
     const int slab = (row_bytes >= 128 && !short_slabs) ? 128 : 64;
-    int scols = cols > 64 ? 128 : ((cols > 32 || row_bytes >= 128) ? 64 : 32);
-    const size_t enough = row_bytes >= 128 ? (size_t)kCUs * 7 / 16 : 2 * (size_t)kCUs;
-    if (row_bytes >= 64 && (slab == 64 || cols >= 64) && (size_t)cdiv(n, 256) * cdiv(cols, scols) >= enough &&
-        stream_lds_fits(256, scols, slab, cols)) {      // (from ~1900 output columns on the staged bias no longer fits)
-        out->tile_rows = 256;
-        out->tile_cols = scols;
-        out->slab_bytes = slab;
-        out->splitk = 1;
-        out->stream = 1;
-        // 129 ... 256 output columns on 128-byte slabs: one tile of 128 rows x 256 columns instead of two of 256 x 128 -- the
-        // same bytes loaded per product, every row gathered once instead of twice, and 128-row tiles pad less (measured,
-        // C = 256: -6 % at 15 192 voxels, -5 % at 252 392, -2 % at 1 026 536; C = 160 and 192 at 252 392 voxels: -8 %, -7 %;
-        // beyond 256 columns the 256-row tile stays ahead)
-        if (slab == 128 && cols > 128 && cols <= 256 && stream_lds_fits(128, 256, slab, cols)) {
-            out->tile_rows = 128;
-            out->tile_cols = 256;
+    // The tile by what a CU multiplies and loads: whole items per CU, each its columns (of 256 rows) at the tile's rate.  One
+    // tile of 128 rows x 256 columns gathers every row once for the same bytes per product as 256 x 128, and pads less;
+    // 64-column tiles read a gathered row from L2 more often but even out a chip that larger ones fill 1.3 times or less than
+    // half (measured forward: 42 608 voxels C = 192, 128 x 256 0.084 ms, 256 x 64 0.078; 8 624 voxels C = 384 0.131 ms in two
+    // K splits, 0.096 on 256 x 64; 15 192 voxels C = 128 0.043 -> 0.039; 64 -> 160 channels at 228 816 voxels 256 x 128 on 64-byte
+    // slabs 0.135, 128 x 256 0.104; 38 720 voxels C = 48 tiled 0.038, 256 x 64 0.027).
+    // An item for half of the CUs is enough (15 192 voxels, 120 items: 384 -> 80 channels 0.087 ms, tiled 0.070; 160 -> 128
+    // 0.052 and 0.044), for five eighths where the outputs are up to 32 columns, with little to multiply, and on rows of
+    // 1 KiB, which the tiled kernel below splits well (1 976 voxels, C = 1024: 128 items 0.232 ms, tiled 0.166).
+    struct Shape { int rows, cols, slab; double rate; };
+    const Shape shapes[] = {{128, 256, 128, 1.0}, {256, 128, slab, 0.95}, {256, 64, slab, 0.6}, {256, 32, 64, 0.5}};
+    double best = 0.0;
+    for (const Shape& sh : shapes) {
+        if (row_bytes < 64 || sh.slab > (int)align_up(row_bytes, 64)) continue;
+        if (sh.cols == 256 ? cols <= 128 || slab != 128 : (sh.cols == 128 ? cols <= 64 : (sh.cols == 64 ? cols <= 32 : cols > 32 || row_bytes >= 256))) continue;
+        // (from ~1900 output columns on the staged bias does not fit beside the rings of the 256 x 128 tile; the other shapes,
+        // whose rings leave a little more room, are no help under a weight that wide)
+        if (!stream_lds_fits(sh.rows, sh.cols, sh.slab, cols) || (cols > 128 && !stream_lds_fits(256, 128, slab, cols))) continue;
+        const size_t items = (size_t)cdiv(n ? n : 1, sh.rows) * cdiv(cols, sh.cols);
+        if (items < (size_t)kCUs * (sh.cols == 32 || row_bytes >= 1024 ? 5 : 4) / 8) continue;
+        const double time = cdiv(items, (size_t)kCUs) * (sh.cols * sh.rows / 256.0 / sh.rate);
+        if (best == 0.0 || time < best) {
+            best = time;
+            *out = fgx_schedule{sh.rows, sh.cols, sh.slab, 1, 0, 1};
         }
-        // Half a chip's worth of items or fewer: tiles of 64 columns make twice as many, and a gathered row read twice
-        // from L2 costs less than idle CUs (measured forward: 15 192 voxels C = 256, 119 items, 0.074 -> 0.064 ms; 3 840
-        // voxels C = 1024, 120 items, 0.270 -> 0.223 ms).
-        if (slab == 128 && out->tile_cols >= 128 &&
-            (size_t)cdiv(n, out->tile_rows) * cdiv(cols, out->tile_cols) <= (size_t)kCUs / 2 && stream_lds_fits(256, 64, slab, cols)) {
-            out->tile_rows = 256;
-            out->tile_cols = 64;
-        }
-    } else if (es == 2 && row_bytes >= 1024 && cols >= 128) {
+    }
+    if (out->stream) return;
+    if (row_bytes >= 1024 && cols >= 128) {
         // Too few tiles to stream and rows of 1 KiB or more (512 channels of a 16-bit type): a few hundred or thousand voxels
         // under a weight of tens of megabytes.  The tiled kernel on 256 x 128 tiles and 128-byte slabs, with as many K
         // splits as give every CU one workgroup, keeps more of the weight in flight than 128 x 128 tiles on 64-byte slabs
