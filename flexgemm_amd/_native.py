@@ -37,7 +37,7 @@ EXPORTS = [
     "fgx_conv_gather_gemm_stream_groups", "fgx_gather_item_order_workspace_bytes", "fgx_gather_item_order",
     "fgx_wgrad_scratch_bytes", "fgx_wgrad_block_bounds_count", "fgx_wgrad_block_bounds", "fgx_conv_wgrad",
     "fgx_wgrad_item_lists_count", "fgx_wgrad_item_lists", "fgx_conv_wgrad_lists",
-    "fgx_zorder_rows", "fgx_narrow_plan_bytes", "fgx_narrow_plan", "fgx_conv_narrow_gemm", "fgx_narrow_wgrad_scratch_bytes", "fgx_conv_narrow_wgrad",
+    "fgx_zorder_rows", "fgx_narrow_plan_bytes", "fgx_narrow_plan", "fgx_narrow_plan_walk", "fgx_conv_narrow_gemm", "fgx_narrow_wgrad_scratch_bytes", "fgx_conv_narrow_wgrad",
     "fgx_wgrad_sweep_plan_bytes", "fgx_wgrad_sweep_plan", "fgx_wgrad_sweep_scratch_bytes", "fgx_conv_wgrad_sweep",
     "fgx_wgrad_sweep_giveup_words", "fgx_wgrad_sweep_reduce",
     "fgx_colsum_scratch_bytes", "fgx_colsum", "fgx_colsum_static_prepare", "fgx_colsum_static_max_cols", "fgx_colsum_static",
@@ -46,7 +46,7 @@ EXPORTS = [
     "fgx_spconv_neighbor_map_sorted_workspace_bytes", "fgx_spconv_neighbor_map_sorted",
     "fgx_serialize_encode", "fgx_serialize_decode", "fgx_serialize_reorder_workspace_bytes",
     "fgx_serialize_reorder_coords",
-    "fgx_tile_plan", "fgx_grid_index_pays", "fgx_subm_neighbor_map_grid_workspace_bytes", "fgx_subm_neighbor_map_grid", "fgx_subm_cache_grid_workspace_bytes",
+    "fgx_tile_plan", "fgx_grid_index_pays", "fgx_grid_index_walks", "fgx_subm_neighbor_map_grid_workspace_bytes", "fgx_subm_neighbor_map_grid", "fgx_subm_cache_grid_workspace_bytes",
     "fgx_subm_cache_build_grid", "fgx_spconv_neighbor_map_grid_workspace_bytes", "fgx_spconv_neighbor_map_grid",
     "fgx_spconv_cache_grid_workspace_bytes", "fgx_spconv_cache_build_grid", "fgx_spconv_out_coords_grid_workspace_bytes",
     "fgx_spconv_out_coords_grid_count", "fgx_spconv_out_coords_grid_emit",

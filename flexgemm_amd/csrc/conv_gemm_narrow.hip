@@ -35,7 +35,8 @@ constexpr int kNarrowHash = 1024;                // hash table of the plan build
 // ------------------------------------------------------------------------------------------------
 __global__ void __launch_bounds__(64) narrow_plan_header_kernel(uint32_t* __restrict__ header) { header[threadIdx.x] = 0u; }
 
-__global__ void __launch_bounds__(256) narrow_plan_kernel(const uint32_t* __restrict__ nmap, const int64_t* __restrict__ order,
+template <typename Order>
+__global__ void __launch_bounds__(256) narrow_plan_kernel(const uint32_t* __restrict__ nmap, const Order* __restrict__ order,
                                                           uint32_t n, int V, int own_rows, unsigned char* __restrict__ plan) {
     __shared__ uint32_t keys[kNarrowHash];
     __shared__ uint16_t slot_of[kNarrowHash];
@@ -434,6 +435,22 @@ int launch_narrow(const void* src, const void* panel, const void* bias, const ui
     return FGX_OK;
 }
 
+template <typename Order>
+int make_narrow_plan(const uint32_t* map, const Order* order, size_t n, int V, int same_rows, void* plan, hipStream_t s) {
+    FGX_CHECK_ARG(V >= 1 && V <= kNarrowMaxV, "fgx_narrow_plan: bad kernel volume %d", V);
+    FGX_CHECK_ARG(n < 0xFFFFFFFFull, "fgx_narrow_plan: too many rows");
+    if (n == 0) return FGX_OK;
+    FGX_CHECK_ARG(map && plan, "fgx_narrow_plan: null buffer");
+    FGX_CHECK_ARG(((uintptr_t)plan & 15) == 0, "fgx_narrow_plan: plan must be 16-byte aligned");
+    FGX_CHECK_ARG(fgx_narrow_plan_bytes(n, V) < 0xFF000000ull, "fgx_narrow_plan: plan of %zu rows passes the 32-bit offset range", n);
+    const unsigned chunks = (unsigned)((n + kNarrowRows - 1) / kNarrowRows);
+    narrow_plan_header_kernel<<<1, 64, 0, s>>>((uint32_t*)plan);
+    FGX_CHECK_LAUNCH("fgx_narrow_plan(header)");
+    narrow_plan_kernel<<<chunks, 256, 0, s>>>(map, order, (uint32_t)n, V, same_rows ? 1 : 0, (unsigned char*)plan);
+    FGX_CHECK_LAUNCH("fgx_narrow_plan");
+    return FGX_OK;
+}
+
 }  // namespace
 }  // namespace fgx
 
@@ -447,18 +464,11 @@ size_t fgx_narrow_plan_bytes(size_t n, int V) {
 }
 
 int fgx_narrow_plan(const uint32_t* map, const int64_t* order, size_t n, int V, int same_rows, void* plan, fgx_stream_t stream) {
-    FGX_CHECK_ARG(V >= 1 && V <= kNarrowMaxV, "fgx_narrow_plan: bad kernel volume %d", V);
-    FGX_CHECK_ARG(n < 0xFFFFFFFFull, "fgx_narrow_plan: too many rows");
-    if (n == 0) return FGX_OK;
-    FGX_CHECK_ARG(map && plan, "fgx_narrow_plan: null buffer");
-    FGX_CHECK_ARG(((uintptr_t)plan & 15) == 0, "fgx_narrow_plan: plan must be 16-byte aligned");
-    FGX_CHECK_ARG(fgx_narrow_plan_bytes(n, V) < 0xFF000000ull, "fgx_narrow_plan: plan of %zu rows passes the 32-bit offset range", n);
-    const unsigned chunks = (unsigned)((n + kNarrowRows - 1) / kNarrowRows);
-    narrow_plan_header_kernel<<<1, 64, 0, (hipStream_t)stream>>>((uint32_t*)plan);
-    FGX_CHECK_LAUNCH("fgx_narrow_plan(header)");
-    narrow_plan_kernel<<<chunks, 256, 0, (hipStream_t)stream>>>(map, order, (uint32_t)n, V, same_rows ? 1 : 0, (unsigned char*)plan);
-    FGX_CHECK_LAUNCH("fgx_narrow_plan");
-    return FGX_OK;
+    return make_narrow_plan(map, order, n, V, same_rows, plan, (hipStream_t)stream);
+}
+
+int fgx_narrow_plan_walk(const uint32_t* map, const uint32_t* walk, size_t n, int V, void* plan, fgx_stream_t stream) {
+    return make_narrow_plan(map, walk, n, V, 1, plan, (hipStream_t)stream);
 }
 
 int fgx_conv_narrow_gemm(int dtype, const void* src, const void* panel, const void* bias, const uint32_t* map, const void* plan,

@@ -35,7 +35,7 @@ namespace {
 
 // ---- the library -------------------------------------------------------------------------------------------------
 #define FGX_HOST_FUNCTIONS(X)                                                                                                     \
-    X(fgx_last_error) X(fgx_grid_index_pays) X(fgx_subm_neighbor_map_grid_workspace_bytes) X(fgx_subm_cache_grid_workspace_bytes) \
+    X(fgx_last_error) X(fgx_grid_index_pays) X(fgx_grid_index_walks) X(fgx_subm_neighbor_map_grid_workspace_bytes) X(fgx_subm_cache_grid_workspace_bytes) \
     X(fgx_subm_cache_build_grid) X(fgx_spconv_cache_grid_workspace_bytes) X(fgx_spconv_cache_build_grid)                           \
     X(fgx_spconv_out_dims) X(fgx_spconv_out_coords_grid_workspace_bytes) X(fgx_spconv_out_coords_grid_count)                       \
     X(fgx_spconv_out_coords_grid_emit) X(fgx_tile_plan) X(fgx_gather_item_order) X(fgx_gather_item_order_workspace_bytes)          \
@@ -221,7 +221,8 @@ private:
 
 // ---- neighbor caches ---------------------------------------------------------------------------------------------------
 // Tables of a submanifold convolution through the grid index, or None where it does not apply:
-// (neighbor_map, gray, binary, order, seg, sig_i, sig_o, SegHost), the last four None without gradients.
+// (neighbor_map, gray, binary, order, walk, seg, sig_i, sig_o, SegHost), the last four None without gradients; walk: the rows in the
+// order of the index's cells, for the plan of narrow layers, or None.
 py::object subm_cache(const Tensor& coords, const std::vector<int>& geom, bool needs_grad, bool forced, size_t max_pair_bytes) {
     const int64_t stream = stream_of(coords);
     const size_t n = (size_t)coords.size(0);
@@ -241,14 +242,17 @@ py::object subm_cache(const Tensor& coords, const std::vector<int>& geom, bool n
         sig_o = make({slots}, at::kUInt32, dev);
         host = std::make_unique<SegHost>(dev.index(), V + 1);
     }
+    Tensor walk;
+    if (rows >= module_int(g_impl, "NARROW_RESIDENT_MIN_ROWS") && L.fgx_grid_index_walks(n, B, W, H, D)) walk = make({rows}, at::kUInt32, dev);
     Tensor ws = workspace(L.fgx_subm_cache_grid_workspace_bytes(n, B, W, H, D, V, needs_grad), dev);
     check(L.fgx_subm_cache_build_grid(ptr<int32_t>(coords), n, B, W, H, D, geom[4], geom[5], geom[6], geom[7], geom[8], geom[9], needs_grad,
                                       ptr(ws), (size_t)ws.numel(), ptr<uint32_t>(nmap), ptr<int32_t>(gray), ptr<int32_t>(binary),
                                       ptr<int64_t>(order), ptr<uint32_t>(seg), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o),
-                                      host ? host->words() : nullptr, as_stream(stream)));
-    if (!host) return py::make_tuple(nmap, gray, binary, order, py::none(), py::none(), py::none(), py::none());
+                                      host ? host->words() : nullptr, ptr<uint32_t>(walk), as_stream(stream)));
+    py::object walk_out = walk.defined() ? py::cast(walk) : py::none();
+    if (!host) return py::make_tuple(nmap, gray, binary, order, walk_out, py::none(), py::none(), py::none(), py::none());
     host->record(as_stream(stream));
-    return py::make_tuple(nmap, gray, binary, order, seg, sig_i, sig_o, std::move(host));
+    return py::make_tuple(nmap, gray, binary, order, walk_out, seg, sig_i, sig_o, std::move(host));
 }
 
 bool conv_grids_pay(size_t n_in, size_t n_out, int B, const int* in, const int* out, bool with_bwd) {

@@ -24,12 +24,13 @@ constexpr int count_rows(size_t blocks) { return blocks > kCountLongFrom ? kCoun
 
 static_assert(kRowsPerGroup == kPairSubRows, "the map kernel counts pairs by its own rows");
 
-// [zero, zero + zero_pieces) := 0 and [fill, fill + fill_pieces) := all ones, 16 bytes at a time
-__global__ void __launch_bounds__(256) clear_kernel(uint4* __restrict__ zero, size_t zero_pieces, uint4* __restrict__ fill, size_t fill_pieces) {
+// [zero, zero + zero_pieces) := 0, 16 bytes at a time, and the words of fill := all ones
+__global__ void __launch_bounds__(256) clear_kernel(uint4* __restrict__ zero, size_t zero_pieces, uint4* __restrict__ fill, size_t fill_words) {
     const size_t stride = (size_t)gridDim.x * 256;
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < zero_pieces; i += stride) zero[i] = make_uint4(0u, 0u, 0u, 0u);
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < fill_pieces; i += stride)
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < fill_words / 4; i += stride)
         fill[i] = make_uint4(FGX_EMPTY32, FGX_EMPTY32, FGX_EMPTY32, FGX_EMPTY32);
+    if (blockIdx.x == 0 && threadIdx.x < (fill_words & 3)) ((uint32_t*)(fill + fill_words / 4))[threadIdx.x] = FGX_EMPTY32;
 }
 
 __device__ __forceinline__ bool in_grid(const GridIndex& g, int b, int x, int y, int z) {
@@ -58,12 +59,21 @@ __device__ __forceinline__ void or_word(uint32_t* __restrict__ words, size_t wor
     if (set && (lane == 0 || before != w)) atomicOr(&words[word], set);
 }
 
-__global__ void __launch_bounds__(256) set_bits_kernel(const int32_t* __restrict__ coords, size_t n, GridIndex g, uint32_t* __restrict__ words) {
+// steps_back (a word): how many of the sampled rows come before the row in front of them (every `every`-th workgroup looks)
+__global__ void __launch_bounds__(256) set_bits_kernel(const int32_t* __restrict__ coords, size_t n, GridIndex g, uint32_t* __restrict__ words,
+                                                       unsigned every, uint32_t* __restrict__ steps_back) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     const int4 c = i < n ? reinterpret_cast<const int4*>(coords)[i] : make_int4(-1, 0, 0, 0);
     const bool in = in_grid(g, c.x, c.y, c.z, c.w);
-    const size_t cell = in ? grid_cell(g, c.x, c.y, c.z, c.w) : 0;
-    or_word(words, cell >> 5, in ? 1u << (cell & 31u) : 0u);
+    const GridPlace<false> p = grid_place<false>(g, c.x, c.y, c.z, c.w);
+    or_word(words, (size_t)p.brick * 4 + (p.at >> 5), in ? 1u << (p.at & 31u) : 0u);
+    if (blockIdx.x % every == 0u) {
+        const int lane = threadIdx.x & 63;
+        const size_t cell = in ? grid_cell(g, c.x, c.y, c.z, c.w) : 0;
+        const uint32_t lo = (uint32_t)__shfl_up((int)(uint32_t)cell, 1, 64), hi = (uint32_t)__shfl_up((int)(uint32_t)(cell >> 32), 1, 64);
+        const unsigned long long back = __ballot(in && lane > 0 && cell < (((size_t)hi << 32) | lo));
+        if (back != 0ull && lane == 0) atomicAdd(steps_back, (uint32_t)__popcll(back));
+    }
 }
 
 __device__ __forceinline__ uint32_t state_load(const uint32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -101,10 +111,10 @@ __device__ __forceinline__ uint32_t lookback(uint32_t* state, unsigned tile, uin
 
 // counts[block] = set bits before the block, in one pass over the bits.  state[tiles] is the ticket; total (optional): all
 // set bits.  A wavefront counts 64 * ROWS consecutive blocks.
-template <int ROWS>
+template <int ROWS, typename Total>
 __global__ void __launch_bounds__(kCountThreads) count_bits_kernel(const ulonglong2* __restrict__ bits, size_t blocks, unsigned tiles,
                                                                    uint32_t* __restrict__ state, uint32_t* __restrict__ counts,
-                                                                   uint64_t* __restrict__ total) {
+                                                                   Total* __restrict__ total) {
     constexpr int kWaves = kCountThreads / 64;
     __shared__ uint32_t wave_sum[kWaves];
     __shared__ uint32_t tile_lds, before_lds;
@@ -142,7 +152,7 @@ __global__ void __launch_bounds__(kCountThreads) count_bits_kernel(const ulonglo
         const uint32_t before = lookback(state, tile, sum);
         if (lane == 0) {
             before_lds = before;
-            if (tile == tiles - 1 && total != nullptr) *total = (uint64_t)(before + sum);
+            if (tile == tiles - 1 && total != nullptr) *total = (Total)(before + sum);
         }
     }
     __syncthreads();
@@ -163,11 +173,12 @@ __global__ void __launch_bounds__(256) place_rows_kernel(const int32_t* __restri
     const int4 c = reinterpret_cast<const int4*>(coords)[i];
     uint32_t loser = (uint32_t)i;
     if (in_grid(g, c.x, c.y, c.z, c.w)) {
-        const size_t cell = grid_cell(g, c.x, c.y, c.z, c.w);
-        const ulonglong2 w = g.bits[cell >> 7];
-        const unsigned at = (unsigned)cell & 127u;
-        const unsigned long long below = (at & 64u ? w.y : w.x) & ((1ull << (at & 63u)) - 1ull);
-        const uint32_t rank = g.counts[cell >> 7] + (uint32_t)__popcll(below) + (at & 64u ? (uint32_t)__popcll(w.x) : 0u);
+        const GridPlace<false> p = grid_place<false>(g, c.x, c.y, c.z, c.w);
+        const uint32_t rank = g.counts[p.brick] + bits_before(g.bits[p.brick], p.at);
+        if ((size_t)g.order[0] == n) {           // as many cells as rows: nobody loses
+            rows[rank] = (uint32_t)i;
+            return;
+        }
         const uint32_t had = atomicMin(&rows[rank], (uint32_t)i);
         loser = had == FGX_EMPTY32 ? FGX_EMPTY32 : (had > (uint32_t)i ? had : (uint32_t)i);
     }
@@ -211,12 +222,12 @@ __device__ __forceinline__ bool target(int c, int k, int K, int S, int P, int Di
     return ok && (unsigned)t < (unsigned)extent;
 }
 
-// map[row][v] for kRowsPerGroup rows (`walk`: which rows, in an order whose neighbors ask for neighboring cells; nullptr: as they
-// come).  A wavefront asks the questions of one kernel column (kx, ky) for all of them, KD along z (0: g.Kd).  `own` (kConvBwd):
+// map[row][v] for kRowsPerGroup rows (`walk`: an index of the queries whose row order makes neighbors ask for neighboring cells;
+// without rows, or where the voxels come in scan order anyway and their map rows then lie side by side: as they come).  A wavefront asks the questions of one kernel column (kx, ky) for all of them, KD along z (0: g.Kd).  `own` (kConvBwd):
 // the index of the queries themselves -- a row that is not the one its cell is known by gets an empty map row.  counts
 // (rows as they come only): set mask bits per offset of every group, [V][gridDim.x].
 template <bool DENSE, int MODE, int KD>
-__global__ void map_kernel(const int32_t* __restrict__ coords, const uint32_t* __restrict__ walk, size_t n, GridIndex index, GridIndex own,
+__global__ void map_kernel(const int32_t* __restrict__ coords, GridIndex walk, size_t n, GridIndex index, GridIndex own,
                            int own_dense, QueryGeom g, uint32_t* __restrict__ out_map, int32_t* __restrict__ gray, int32_t* __restrict__ binary,
                            uint32_t* __restrict__ counts) {
     extern __shared__ uint32_t lds[];
@@ -233,14 +244,13 @@ __global__ void map_kernel(const int32_t* __restrict__ coords, const uint32_t* _
         uint32_t id = FGX_EMPTY32;
         int4 c = make_int4(-1, 0, 0, 0);
         if (tid < cnt) {
-            id = walk != nullptr ? walk[p0 + tid] : (uint32_t)(p0 + tid);
+            id = walk.rows != nullptr && !grid_in_scan_order(walk, n) ? walk.rows[p0 + tid] : (uint32_t)(p0 + tid);
             c = reinterpret_cast<const int4*>(coords)[id];
             if constexpr (MODE == kConvBwd) {
                 bool known = in_grid(own, c.x, c.y, c.z, c.w);
-                if (known) {
-                    const size_t cell = grid_cell(own, c.x, c.y, c.z, c.w);
-                    known = (own_dense ? grid_find<true>(own, cell) : grid_find<false>(own, cell)) == id;
-                }
+                if (known)
+                    known = (own_dense ? grid_find<true>(own, grid_place<true>(own, c.x, c.y, c.z, c.w))
+                                       : grid_find<false>(own, grid_place<false>(own, c.x, c.y, c.z, c.w))) == id;
                 if (!known) c.x = -1;
             }
         }
@@ -260,12 +270,12 @@ __global__ void map_kernel(const int32_t* __restrict__ coords, const uint32_t* _
         const bool x_ok = target<MODE>(c.y, kx, g.Kw, g.Sw, g.Pw, g.Dw, index.W, &x);
         const bool y_ok = target<MODE>(c.z, ky, g.Kh, g.Sh, g.Ph, g.Dh, index.H, &y);
         const bool column = batch_ok && x_ok && y_ok;
-        const size_t cell0 = column ? grid_cell(index, c.x, x, y, 0) : 0;
+        const GridPlace<DENSE> at = place_bx<DENSE>(index, c.x, x) + place_y<DENSE>(index, y);
         uint32_t found = 0u;
         auto ask = [&](int kz) {
             int z;
             uint32_t value = FGX_EMPTY32;
-            if (target<MODE>(c.w, kz, g.Kd, g.Sd, g.Pd, g.Dd, index.D, &z) && column) value = grid_find<DENSE>(index, cell0 + (size_t)z);
+            if (target<MODE>(c.w, kz, g.Kd, g.Sd, g.Pd, g.Dd, index.D, &z) && column) value = grid_find<DENSE>(index, at + place_z<DENSE>(index, z));
             if (MODE == kSubm && r * kd + kz == V / 2) value = id;       // the middle entry is the voxel itself, found or not
             return value;
         };
@@ -311,9 +321,10 @@ __global__ void map_kernel(const int32_t* __restrict__ coords, const uint32_t* _
 // questions) before it needs the first answer, and nothing waits for other wavefronts.  What bounds it is the latency of
 // three dependent reads (row, bits, row number) against what a CU holds in flight: one column per wavefront, as above, took
 // 0.261 ms for 2 667 120 voxels of a surface in scan order (3x3x3, map and codes, 331 MB read and written), this form
-// 0.136 (sort and merge: 0.331).  In random order the scattered 108-byte rows bound it (0.283 ms; a plain scatter: 0.26).  Dilations along z beyond 63 go to the general kernel: here a column's cells lie in at most two blocks of bits.
+// 0.136 (sort and merge: 0.331).  In random order the scattered 108-byte rows bound it (0.283 ms; a plain scatter: 0.26).  In
+// the `bits` form a column's cells have to lie in two bricks: columns longer than 32 cells go to the general kernel.
 template <bool DENSE, int MODE, int K>
-__global__ void __launch_bounds__(64) cube_map_kernel(const int32_t* __restrict__ coords, const uint32_t* __restrict__ walk, size_t n,
+__global__ void __launch_bounds__(64) cube_map_kernel(const int32_t* __restrict__ coords, GridIndex walk, size_t n,
                                                       GridIndex index, GridIndex own, int own_dense, QueryGeom g, uint32_t* __restrict__ out_map,
                                                       int32_t* __restrict__ gray, int32_t* __restrict__ binary, uint32_t* __restrict__ counts) {
     constexpr int V = K * K * K, PITCH = V | 1;
@@ -325,25 +336,37 @@ __global__ void __launch_bounds__(64) cube_map_kernel(const int32_t* __restrict_
     uint32_t id = FGX_EMPTY32;
     int4 c = make_int4(-1, 0, 0, 0);
     if (lane < cnt) {
-        id = walk != nullptr ? walk[p0 + lane] : (uint32_t)(p0 + lane);
+        id = walk.rows != nullptr && !grid_in_scan_order(walk, n) ? walk.rows[p0 + lane] : (uint32_t)(p0 + lane);
         c = reinterpret_cast<const int4*>(coords)[id];
         if constexpr (MODE == kConvBwd) {
             bool known = in_grid(own, c.x, c.y, c.z, c.w);
-            if (known) {
-                const size_t cell = grid_cell(own, c.x, c.y, c.z, c.w);
-                known = (own_dense ? grid_find<true>(own, cell) : grid_find<false>(own, cell)) == id;
-            }
+            if (known)
+                known = (own_dense ? grid_find<true>(own, grid_place<true>(own, c.x, c.y, c.z, c.w))
+                                   : grid_find<false>(own, grid_place<false>(own, c.x, c.y, c.z, c.w))) == id;
             if (!known) c.x = -1;
         }
     }
     id_lds[lane] = id;
     const bool batch_ok = (unsigned)c.x < (unsigned)index.B;
     bool y_ok[K], z_ok[K];
-    int yt[K], zt[K];
+    GridPlace<DENSE> yp[K], zp[K];
+    uint32_t z_first = 0u, z_last = 0u;         // (`bits` form: bricks of the first and the last cell along z inside the grid)
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        y_ok[k] = target<MODE>(c.z, k, K, g.Sh, g.Ph, g.Dh, index.H, &yt[k]);
-        z_ok[k] = target<MODE>(c.w, k, K, g.Sd, g.Pd, g.Dd, index.D, &zt[k]);
+        int t;
+        y_ok[k] = target<MODE>(c.z, k, K, g.Sh, g.Ph, g.Dh, index.H, &t);
+        yp[k] = place_y<DENSE>(index, t);
+        z_ok[k] = target<MODE>(c.w, k, K, g.Sd, g.Pd, g.Dd, index.D, &t);
+        zp[k] = place_z<DENSE>(index, t);
+        if constexpr (!DENSE) {
+            if (z_ok[k]) z_last = zp[k].brick;
+        }
+    }
+    if constexpr (!DENSE) {
+        z_first = z_last;
+#pragma unroll
+        for (int k = K - 1; k >= 0; --k)
+            if (z_ok[k]) z_first = zp[k].brick;
     }
     uint32_t mask = 0u;
 #pragma unroll
@@ -351,53 +374,42 @@ __global__ void __launch_bounds__(64) cube_map_kernel(const int32_t* __restrict_
         int xt;
         const bool x_ok = target<MODE>(c.y, kx, K, g.Sw, g.Pw, g.Dw, index.W, &xt) && batch_ok;
         uint32_t value[K][K];
+        const GridPlace<DENSE> xp = place_bx<DENSE>(index, c.x, xt);
         if constexpr (DENSE || MODE == kConvBwd) {
 #pragma unroll
-            for (int ky = 0; ky < K; ++ky) {
-                const bool column = x_ok && y_ok[ky];
-                const size_t cell0 = column ? grid_cell(index, c.x, xt, yt[ky], 0) : 0;
+            for (int ky = 0; ky < K; ++ky)
 #pragma unroll
                 for (int kz = 0; kz < K; ++kz)
-                    value[ky][kz] = column && z_ok[kz] ? grid_find<DENSE>(index, cell0 + (size_t)zt[kz]) : FGX_EMPTY32;
-            }
+                    value[ky][kz] = x_ok && y_ok[ky] && z_ok[kz] ? grid_find<DENSE>(index, xp + yp[ky] + zp[kz]) : FGX_EMPTY32;
         } else {
-            // the column's cells ascend along z and span less than 128: they lie in the block of the first one inside the
-            // grid or in that of the last one
-            const int z_first = zt[0] < 0 ? 0 : (zt[0] < index.D ? zt[0] : index.D - 1);
-            const int z_last = zt[K - 1] < 0 ? 0 : (zt[K - 1] < index.D ? zt[K - 1] : index.D - 1);
+            // the column's cells ascend along z and span at most 32: they lie in the brick of the first one inside the grid or in
+            // that of the last one
             ulonglong2 wa[K], wb[K];
             uint32_t na[K], nb[K];
-            size_t cell0[K], block_a[K];
 #pragma unroll
             for (int ky = 0; ky < K; ++ky) {
                 const bool column = x_ok && y_ok[ky];
-                cell0[ky] = column ? grid_cell(index, c.x, xt, yt[ky], 0) : 0;
-                block_a[ky] = column ? (cell0[ky] + (size_t)z_first) >> 7 : 0;
-                const size_t block_b = column ? (cell0[ky] + (size_t)z_last) >> 7 : 0;
-                wa[ky] = index.bits[block_a[ky]];
-                na[ky] = index.counts[block_a[ky]];
+                const uint32_t brick_a = column ? xp.brick + yp[ky].brick + z_first : 0u;
+                wa[ky] = index.bits[brick_a];
+                na[ky] = index.counts[brick_a];
                 wb[ky] = make_ulonglong2(0ull, 0ull);
                 nb[ky] = 0u;
-                if (block_b != block_a[ky]) {
-                    wb[ky] = index.bits[block_b];
-                    nb[ky] = index.counts[block_b];
+                if (column && z_last != z_first) {
+                    wb[ky] = index.bits[xp.brick + yp[ky].brick + z_last];
+                    nb[ky] = index.counts[xp.brick + yp[ky].brick + z_last];
                 }
             }
 #pragma unroll
             for (int ky = 0; ky < K; ++ky) {
-                const bool column = x_ok && y_ok[ky];
                 uint32_t rank[K];
                 bool have[K];
 #pragma unroll
                 for (int kz = 0; kz < K; ++kz) {
-                    const size_t cell = cell0[ky] + (size_t)(z_ok[kz] ? zt[kz] : 0);
-                    const bool in_a = (cell >> 7) == block_a[ky];
-                    const unsigned long long lo = in_a ? wa[ky].x : wb[ky].x, hi = in_a ? wa[ky].y : wb[ky].y;
-                    const bool upper = (cell & 64u) != 0;
-                    const unsigned long long word = upper ? hi : lo;
-                    const unsigned at = (unsigned)cell & 63u;
-                    have[kz] = column && z_ok[kz] && ((word >> at) & 1ull);
-                    rank[kz] = (in_a ? na[ky] : nb[ky]) + (upper ? (uint32_t)__popcll(lo) : 0u) + (uint32_t)__popcll(word & ((1ull << at) - 1ull));
+                    const bool in_a = zp[kz].brick == z_first;
+                    const ulonglong2 w = make_ulonglong2(in_a ? wa[ky].x : wb[ky].x, in_a ? wa[ky].y : wb[ky].y);
+                    const uint32_t at = (xp.at + yp[ky].at + zp[kz].at) & 127u;
+                    have[kz] = x_ok && y_ok[ky] && z_ok[kz] && (((at & 64u ? w.y : w.x) >> (at & 63u)) & 1ull);
+                    rank[kz] = (in_a ? na[ky] : nb[ky]) + bits_before(w, at);
                 }
 #pragma unroll
                 for (int kz = 0; kz < K; ++kz) value[ky][kz] = have[kz] ? index.rows[rank[kz]] : FGX_EMPTY32;
@@ -443,11 +455,11 @@ __global__ void __launch_bounds__(64) cube_map_kernel(const int32_t* __restrict_
 }
 
 template <bool DENSE, int MODE>
-int launch_map(const int32_t* coords, const uint32_t* walk, size_t n, const GridIndex& index, const GridIndex& own, bool own_dense,
+int launch_map(const int32_t* coords, const GridIndex& walk, size_t n, const GridIndex& index, const GridIndex& own, bool own_dense,
                const QueryGeom& g, uint32_t* out_map, int32_t* gray, int32_t* binary, uint32_t* counts, hipStream_t s, const char* what) {
     const unsigned grid = cdiv(n, kRowsPerGroup);
     const int R = g.Kw * g.Kh;
-    const bool cube = g.Kw == g.Kh && g.Kh == g.Kd && g.Dd < 64;
+    const bool cube = g.Kw == g.Kh && g.Kh == g.Kd && (DENSE || MODE == kConvBwd || g.Dd * (g.Kd - 1) <= 32);
     if (cube && g.Kd == 3) {
         cube_map_kernel<DENSE, MODE, 3><<<grid, 64, 0, s>>>(coords, walk, n, index, own, own_dense ? 1 : 0, g, out_map, gray, binary, counts);
     } else if (MODE != kSubm && cube && g.Kd == 2) {
@@ -540,16 +552,17 @@ int check_query(const char* who, int Kw, int Kh, int Kd) {
     return FGX_OK;
 }
 
-int launch_clear(void* zero, size_t zero_bytes, void* fill, size_t fill_bytes, hipStream_t s, const char* what) {
-    const size_t most = zero_bytes > fill_bytes ? zero_bytes : fill_bytes;
+int launch_clear(void* zero, size_t zero_bytes, uint32_t* fill, size_t fill_words, hipStream_t s, const char* what) {
+    const size_t most = zero_bytes > fill_words * 4 ? zero_bytes : fill_words * 4;
     unsigned grid = cdiv(most / 16 + 1, 256);
     if (grid > 4096u) grid = 4096u;
-    clear_kernel<<<grid, 256, 0, s>>>((uint4*)zero, zero_bytes / 16, (uint4*)fill, fill_bytes / 16);
+    clear_kernel<<<grid, 256, 0, s>>>((uint4*)zero, zero_bytes / 16, (uint4*)fill, fill_words);
     FGX_CHECK_LAUNCH(what);
     return FGX_OK;
 }
 
-int launch_count(const char* ws, const GridIndexLayout& L, uint64_t* total, hipStream_t s, const char* what) {
+template <typename Total>
+int launch_count(const char* ws, const GridIndexLayout& L, Total* total, hipStream_t s, const char* what) {
     const ulonglong2* bits = (const ulonglong2*)(ws + L.bits);
     uint32_t* state = (uint32_t*)(ws + L.state);
     uint32_t* counts = (uint32_t*)(ws + L.counts);
@@ -560,19 +573,32 @@ int launch_count(const char* ws, const GridIndexLayout& L, uint64_t* total, hipS
     return FGX_OK;
 }
 
-bool bits_layout(size_t n_rows, int B, int W, int H, int D, GridIndexLayout* out) {
+// Bit map of a grid: in bricks and cubes of 2^shift bricks each way (the index), or cells in their order (`in_order`: the output
+// coordinates, which leave in that order).  The cubes are the largest whose padding adds no more than a quarter to the bricks'.
+bool bits_layout(size_t n_rows, int B, int W, int H, int D, bool in_order, GridIndexLayout* out) {
     GridIndexLayout L{};
     if (B < 1 || W < 1 || H < 1 || D < 1) return false;
     const double cells = (double)B * W * H * D;
     if (cells > 8.0 * (double)kBitsMaxBytes || n_rows >= ((size_t)1 << 30)) return false;
     L.cells = (size_t)B * W * H * D;
     L.blocks = (L.cells + 127) / 128;
+    if (!in_order) {
+        const double bricks = (double)B * cdiv(W, 2) * cdiv(H, 2) * cdiv(D, 32);
+        for (L.shift = 3;; --L.shift) {
+            const uint32_t e = 2u << L.shift;
+            const double padded = (double)B * cdiv(W, e) * cdiv(H, e) * cdiv(D, 32) * (double)(1u << (2 * L.shift));
+            if (L.shift > 0 && padded > 1.25 * bricks) continue;
+            if (padded > (double)kBitsMaxBytes / 16.0) return false;
+            L.blocks = (size_t)padded;
+            break;
+        }
+    }
     L.tiles = cdiv(L.blocks, (size_t)kCountThreads * count_rows(L.blocks));
     size_t off = 0;
     L.bits = off;
     off = align_up(off + L.blocks * 16, 256);
     L.state = off;
-    off = align_up(off + (L.tiles + 2) * 4, 256);       // the tiles' words, the ticket, the number of losers
+    off = align_up(off + (L.tiles + 4) * 4, 256);       // the tiles' words, the ticket, the number of losers, GridIndex::order
     L.zero_bytes = off;
     L.counts = off;
     off = align_up(off + L.blocks * 4, 256);
@@ -587,9 +613,9 @@ bool bits_layout(size_t n_rows, int B, int W, int H, int D, GridIndexLayout* out
 
 bool grid_index_plan(size_t n, int B, int W, int H, int D, GridIndexLayout* out) {
     GridIndexLayout L{};
-    if (!bits_layout(n, B, W, H, D, &L)) return false;
+    if (!bits_layout(n, B, W, H, D, false, &L)) return false;
     if (L.cells <= kDenseMaxCells) {
-        L = GridIndexLayout{true, L.cells, 0, 0, 0, 0, 0, 0, align_up(L.cells * 4, 256), 0};
+        L = GridIndexLayout{true, L.cells, 0, 0, 0, 0, 0, 0, align_up(L.cells * 4, 256), 0, 0};
     }
     *out = L;
     return true;
@@ -598,12 +624,12 @@ bool grid_index_plan(size_t n, int B, int W, int H, int D, GridIndexLayout* out)
 bool grid_index_pays(size_t n, int B, int W, int H, int D) {
     GridIndexLayout L;
     if (!grid_index_plan(n, B, W, H, D, &L)) return false;
-    const size_t bytes = L.cells / 8;
+    const size_t bytes = L.blocks * 16;
     return L.dense || bytes <= kBitsAlwaysMaxBytes || bytes <= n * kBitsBytesPerVoxel;
 }
 
-int grid_index_build(const int32_t* coords, size_t n, int B, int W, int H, int D, const GridIndexLayout& L, void* workspace, GridIndex* out,
-                     hipStream_t s, const char* what) {
+int grid_index_build(const int32_t* coords, size_t n, int B, int W, int H, int D, const GridIndexLayout& L, void* workspace, uint32_t* walk,
+                     GridIndex* out, hipStream_t s, const char* what) {
     char* ws = (char*)workspace;
     GridIndex g{};
     g.B = B;
@@ -613,18 +639,25 @@ int grid_index_build(const int32_t* coords, size_t n, int B, int W, int H, int D
     const unsigned grid = cdiv(n, 256);
     if (L.dense) {
         uint32_t* cells = (uint32_t*)ws;
-        int rc = launch_clear(nullptr, 0, cells, L.total, s, what);
+        int rc = launch_clear(nullptr, 0, cells, L.cells, s, what);
         if (rc != FGX_OK) return rc;
         g.cells = cells;
         if (n) insert_cells_kernel<<<grid, 256, 0, s>>>(coords, n, g, cells);
         FGX_CHECK_LAUNCH(what);
     } else {
-        uint32_t* rows = (uint32_t*)(ws + L.rows);
-        int rc = launch_clear(ws, L.zero_bytes, rows, L.total - L.rows, s, what);
+        const uint32_t e = 2u << L.shift;
+        g.shift = L.shift;
+        g.step_y = (1u << (2 * L.shift)) * cdiv(D, 32);
+        g.step_x = g.step_y * cdiv(H, e);
+        g.step_b = g.step_x * cdiv(W, e);
+        uint32_t* rows = walk != nullptr ? walk : (uint32_t*)(ws + L.rows);
+        int rc = launch_clear(ws, L.zero_bytes, rows, n, s, what);
         if (rc != FGX_OK) return rc;
-        if (n) set_bits_kernel<<<grid, 256, 0, s>>>(coords, n, g, (uint32_t*)(ws + L.bits));
+        uint32_t* order = (uint32_t*)(ws + L.state) + L.tiles + 2;
+        g.order = order;
+        if (n) set_bits_kernel<<<grid, 256, 0, s>>>(coords, n, g, (uint32_t*)(ws + L.bits), cdiv(grid, kOrderSamples), order + 1);
         FGX_CHECK_LAUNCH(what);
-        rc = launch_count(ws, L, nullptr, s, what);
+        rc = launch_count<uint32_t>(ws, L, order, s, what);
         if (rc != FGX_OK) return rc;
         g.bits = (const ulonglong2*)(ws + L.bits);
         g.counts = (const uint32_t*)(ws + L.counts);
@@ -637,18 +670,18 @@ int grid_index_build(const int32_t* coords, size_t n, int B, int W, int H, int D
 }
 
 int subm_map_grid(const int32_t* coords, size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dw, int Dh, int Dd,
-                  const GridIndexLayout& L, void* workspace, uint32_t* out_map, int32_t* gray, int32_t* binary, uint32_t* counts,
+                  const GridIndexLayout& L, void* workspace, uint32_t* walk, uint32_t* out_map, int32_t* gray, int32_t* binary, uint32_t* counts,
                   bool* counted, hipStream_t s) {
     GridIndex index;
     phase_mark("grid index", s);
-    int rc = grid_index_build(coords, n, B, W, H, D, L, workspace, &index, s, "fgx_subm_neighbor_map_grid(index)");
+    int rc = grid_index_build(coords, n, B, W, H, D, L, workspace, walk, &index, s, "fgx_subm_neighbor_map_grid(index)");
     if (rc != FGX_OK) return rc;
     phase_mark("grid map", s);
     const QueryGeom g{Kw, Kh, Kd, Kw * Kh * Kd, 1, 1, 1, 0, 0, 0, Dw, Dh, Dd};
     if (counted) *counted = L.dense && counts != nullptr;
     if (L.dense)
-        return launch_map<true, kSubm>(coords, nullptr, n, index, index, true, g, out_map, gray, binary, counts, s, "fgx_subm_neighbor_map_grid");
-    return launch_map<false, kSubm>(coords, index.rows, n, index, index, false, g, out_map, gray, binary, nullptr, s, "fgx_subm_neighbor_map_grid");
+        return launch_map<true, kSubm>(coords, GridIndex{}, n, index, index, true, g, out_map, gray, binary, counts, s, "fgx_subm_neighbor_map_grid");
+    return launch_map<false, kSubm>(coords, index, n, index, index, false, g, out_map, gray, binary, nullptr, s, "fgx_subm_neighbor_map_grid");
 }
 
 bool conv_maps_plan(size_t n_in, size_t n_out, int B, int W, int H, int D, int Wo, int Ho, int Do, bool with_bwd, ConvMapsLayout* P) {
@@ -669,16 +702,16 @@ int conv_maps_grid(const int32_t* in_coords, size_t n_in, const int32_t* out_coo
     char* ws = (char*)workspace;
     GridIndex in, out{};
     phase_mark("grid index", s);
-    int rc = grid_index_build(in_coords, n_in, B, W, H, D, P.in, ws, &in, s, what);
-    if (rc == FGX_OK && map_bwd != nullptr) rc = grid_index_build(out_coords, n_out, B, Wo, Ho, Do, P.out, ws + P.out_at, &out, s, what);
+    int rc = grid_index_build(in_coords, n_in, B, W, H, D, P.in, ws, nullptr, &in, s, what);
+    if (rc == FGX_OK && map_bwd != nullptr) rc = grid_index_build(out_coords, n_out, B, Wo, Ho, Do, P.out, ws + P.out_at, nullptr, &out, s, what);
     if (rc != FGX_OK) return rc;
     phase_mark("grid map", s);
     const QueryGeom g{k[0], k[1], k[2], k[0] * k[1] * k[2], k[3], k[4], k[5], k[6], k[7], k[8], k[9], k[10], k[11]};
     if (n_out > 0)
-        rc = P.in.dense ? launch_map<true, kConvFwd>(out_coords, nullptr, n_out, in, in, true, g, map_fwd, gray, binary, counts, s, what)
-                        : launch_map<false, kConvFwd>(out_coords, nullptr, n_out, in, in, false, g, map_fwd, gray, binary, counts, s, what);
+        rc = P.in.dense ? launch_map<true, kConvFwd>(out_coords, GridIndex{}, n_out, in, in, true, g, map_fwd, gray, binary, counts, s, what)
+                        : launch_map<false, kConvFwd>(out_coords, GridIndex{}, n_out, in, in, false, g, map_fwd, gray, binary, counts, s, what);
     if (rc != FGX_OK || map_bwd == nullptr || n_in == 0) return rc;
-    const uint32_t* walk = P.in.dense ? nullptr : in.rows;
+    const GridIndex walk = P.in.dense ? GridIndex{} : in;
     return P.out.dense ? launch_map<true, kConvBwd>(in_coords, walk, n_in, out, in, P.in.dense, g, map_bwd, gray_bwd, binary_bwd, nullptr, s, what)
                        : launch_map<false, kConvBwd>(in_coords, walk, n_in, out, in, P.in.dense, g, map_bwd, gray_bwd, binary_bwd, nullptr, s, what);
 }
@@ -690,6 +723,11 @@ using namespace fgx;
 extern "C" {
 
 int fgx_grid_index_pays(size_t n, int B, int W, int H, int D) { return grid_index_pays(n, B, W, H, D) ? 1 : 0; }
+
+int fgx_grid_index_walks(size_t n, int B, int W, int H, int D) {
+    GridIndexLayout L;
+    return grid_index_plan(n, B, W, H, D, &L) && !L.dense ? 1 : 0;
+}
 
 size_t fgx_subm_neighbor_map_grid_workspace_bytes(size_t n, int B, int W, int H, int D) {
     GridIndexLayout L;
@@ -711,7 +749,7 @@ int fgx_subm_neighbor_map_grid(const int32_t* coords, size_t n, int B, int W, in
     FGX_CHECK_ARG((((uintptr_t)coords & 15) | ((uintptr_t)workspace & 255)) == 0, "%s: coords must be 16-byte, workspace 256-byte aligned", who);
     FGX_CHECK_ARG(workspace_bytes >= L.total, "%s: workspace of %zu bytes, need %zu", who, workspace_bytes, L.total);
     PhaseEnd phases{(hipStream_t)stream};
-    return subm_map_grid(coords, n, B, W, H, D, Kw, Kh, Kd, Dw, Dh, Dd, L, workspace, out_map, gray, binary, nullptr, nullptr, (hipStream_t)stream);
+    return subm_map_grid(coords, n, B, W, H, D, Kw, Kh, Kd, Dw, Dh, Dd, L, workspace, nullptr, out_map, gray, binary, nullptr, nullptr, (hipStream_t)stream);
 }
 
 size_t fgx_spconv_neighbor_map_grid_workspace_bytes(size_t n_in, size_t n_out, int B, int W, int H, int D, int Wo, int Ho, int Do, int with_bwd) {
@@ -746,7 +784,7 @@ int fgx_spconv_neighbor_map_grid(const int32_t* in_coords, size_t n_in, const in
 
 size_t fgx_spconv_out_coords_grid_workspace_bytes(int B, int Wo, int Ho, int Do) {
     GridIndexLayout L;
-    return bits_layout(0, B, Wo, Ho, Do, &L) ? L.total : 0;
+    return bits_layout(0, B, Wo, Ho, Do, true, &L) ? L.total : 0;
 }
 
 int fgx_spconv_out_coords_grid_count(const int32_t* coords, size_t n_in, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Sw, int Sh,
@@ -757,7 +795,7 @@ int fgx_spconv_out_coords_grid_count(const int32_t* coords, size_t n_in, int B, 
     int rc = fgx_spconv_out_dims(W, H, D, Kw, Kh, Kd, Sw, Sh, Sd, Pw, Ph, Pd, Dw, Dh, Dd, &Wo, &Ho, &Do);
     if (rc != FGX_OK) return rc;
     GridIndexLayout L;
-    FGX_CHECK_ARG(bits_layout(0, B, Wo, Ho, Do, &L), "%s: no bit map over an output grid of %d x %d x %d x %d cells", who, B, Wo, Ho, Do);
+    FGX_CHECK_ARG(bits_layout(0, B, Wo, Ho, Do, true, &L), "%s: no bit map over an output grid of %d x %d x %d x %d cells", who, B, Wo, Ho, Do);
     FGX_CHECK_ARG(coords && n_in > 0 && workspace && count, "%s: null buffer", who);
     FGX_CHECK_ARG((double)n_in * Kw * Kh * Kd < (double)(1u << 30), "%s: too many candidates", who);
     FGX_CHECK_ARG((((uintptr_t)coords & 15) | ((uintptr_t)workspace & 255)) == 0, "%s: coords must be 16-byte, workspace 256-byte aligned", who);
@@ -780,7 +818,7 @@ int fgx_spconv_out_coords_grid_count(const int32_t* coords, size_t n_in, int B, 
 int fgx_spconv_out_coords_grid_emit(const void* workspace, int B, int Wo, int Ho, int Do, size_t count, int32_t* out_coords, fgx_stream_t stream) {
     const char* who = "fgx_spconv_out_coords_grid_emit";
     GridIndexLayout L;
-    FGX_CHECK_ARG(bits_layout(0, B, Wo, Ho, Do, &L), "%s: no bit map over an output grid of %d x %d x %d x %d cells", who, B, Wo, Ho, Do);
+    FGX_CHECK_ARG(bits_layout(0, B, Wo, Ho, Do, true, &L), "%s: no bit map over an output grid of %d x %d x %d x %d cells", who, B, Wo, Ho, Do);
     if (count == 0) return FGX_OK;
     FGX_CHECK_ARG(workspace && out_coords && ((uintptr_t)out_coords & 15) == 0, "%s: null or misaligned buffer", who);
     const char* ws = (const char*)workspace;

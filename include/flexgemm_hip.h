@@ -188,9 +188,11 @@ int fgx_subm_cache_build(const int32_t* coords, size_t n, int B, int W, int H, i
  * "auto" rule).  Workspace functions return 0 for a grid too large (512 MiB of bits); workspaces are 256-byte aligned.
  * The map: kernel volumes up to 128, mask codes (gray / binary, both or neither) up to 32.  The cache: as
  * fgx_subm_cache_build, without the sort's key_bits and presorted; seg_host (optional): pinned host memory that receives the
- * segment table as well (valid once the stream has passed the call).
+ * segment table as well (valid once the stream has passed the call); walk (optional, where fgx_grid_index_walks is 1): the rows
+ * in the order of the index's cells, a space-filling curve, for fgx_narrow_plan_walk.
  * Replaces: hashmap_build_submanifold_conv_neighbour_map and the same sequence of calls as fgx_subm_cache_build. */
 int fgx_grid_index_pays(size_t n, int B, int W, int H, int D);
+int fgx_grid_index_walks(size_t n, int B, int W, int H, int D);
 size_t fgx_subm_neighbor_map_grid_workspace_bytes(size_t n, int B, int W, int H, int D);
 int fgx_subm_neighbor_map_grid(const int32_t* coords, size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dw, int Dh,
                                int Dd, void* workspace, size_t workspace_bytes, uint32_t* out_map, int32_t* gray, int32_t* binary,
@@ -199,7 +201,7 @@ size_t fgx_subm_cache_grid_workspace_bytes(size_t n, int B, int W, int H, int D,
 int fgx_subm_cache_build_grid(const int32_t* coords, size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dw, int Dh, int Dd,
                               int with_pairs, void* workspace, size_t workspace_bytes, uint32_t* out_map, int32_t* gray, int32_t* binary,
                               int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, uint32_t* seg_host,
-                              fgx_stream_t stream);
+                              uint32_t* walk, fgx_stream_t stream);
 
 /* Per row-tile (block consecutive rows of the sorted order) OR of the masks.
  *   codes: tile_code[nb] <- OR mask, seg[nb+1] <- exclusive offsets of popcounts (seg[nb] = total);
@@ -355,6 +357,8 @@ int fgx_conv_gather_gemm_stream_groups(int dtype, int cols, int tile_rows, int t
  * (..._fwd_masked_implicit_gemm.py:20-100). */
 size_t fgx_narrow_plan_bytes(size_t n, int V);
 int fgx_narrow_plan(const uint32_t* map, const int64_t* order, size_t n, int V, int same_rows, void* plan, fgx_stream_t stream);
+/* ... of a submanifold map (same_rows = 1) along the 32-bit row order fgx_subm_cache_build_grid leaves as `walk`. */
+int fgx_narrow_plan_walk(const uint32_t* map, const uint32_t* walk, size_t n, int V, void* plan, fgx_stream_t stream);
 int fgx_conv_narrow_gemm(int dtype, const void* src, const void* panel, const void* bias, const uint32_t* map, const void* plan,
                          size_t n, size_t n_src, int K, int cols, int V, int activation, void* out, uint8_t* relu_mask,
                          fgx_stream_t stream);

@@ -7,9 +7,10 @@ import pytest
 import torch
 
 import flex_gemm
-from flex_gemm.ops.spconv import SparseConv3dFunction, SubMConv3dFunction
+from flex_gemm.ops.spconv import SparseConv3dFunction, SubMConv3dFunction, sparse_submanifold_conv3d
 from flexgemm_amd import _native as nat
 from flexgemm_amd.workloads import reference_test_shell
+from oracle import explicit_gemm as eg
 from oracle import neighbor as nb
 from oracle import sparse_conv as sc
 
@@ -116,3 +117,28 @@ def test_mask_sort(gpu_device, n, volume, distinct):
     ws = nat.workspace(L.fgx_sort_workspace_bytes(nat.sz(n)), gpu_device)
     nat.check(L.fgx_sort_by_code(nat.ptr(keys), nat.sz(n), C.c_int(volume), nat.ptr(order), nat.ptr(ws), nat.sz(ws.numel()), nat.stream()))
     assert np.array_equal(order.cpu().numpy(), np.argsort(keys.cpu().numpy(), kind="stable"))
+
+
+# the index's row order as the narrow layers' plan: first product of a fresh cache, rows in scan and random order, with and without
+# voxels given twice, a grid whose columns need no padding and one whose do, a last chunk that is not full
+@pytest.mark.parametrize("res,order,twice", [(256, "scan", 0), (256, "shuffled", 0), (205, "shuffled", 90), (230, "scan", 1)])
+def test_narrow_layer_on_a_fresh_grid_cache(gpu_device, res, order, twice):
+    _say(f"narrow layer on a fresh grid cache res={res} {order} twice={twice}")
+    rng = np.random.default_rng(res)
+    coords = reference_test_shell(96) + np.array([0, 50, 3, 101], np.int32)
+    coords = np.concatenate([coords, coords[:twice]])
+    if order == "shuffled":
+        coords = coords[rng.permutation(len(coords))]
+    n, c = len(coords), 16
+    gen = torch.Generator().manual_seed(res)
+    feats, grad = torch.randn(n, c, generator=gen).half(), torch.randn(n, c, generator=gen).half()
+    weight = (torch.randn(c, 3, 3, 3, c, generator=gen) / (27 * c) ** 0.5).half()
+    dev = gpu_device
+    f, w = feats.to(dev).requires_grad_(True), weight.to(dev).requires_grad_(True)
+    out, cache = sparse_submanifold_conv3d(f, torch.from_numpy(coords).to(dev), torch.Size([1, c, res, res, res]), w)
+    out.backward(grad.to(dev))
+    assert np.array_equal(np.sort(_np(cache["_cell_walk"])), np.arange(n)) and hasattr(cache, "_narrow_plan_buf")
+    nmap = cache.neighbor_map.cpu().view(torch.int32)
+    ref_gi, ref_gw, _ = eg.backward(grad.double(), feats.double(), nmap, weight.double())
+    for got, ref in ((out, eg.forward(feats.double(), nmap, weight.double())), (f.grad, ref_gi), (w.grad, ref_gw)):
+        assert eg.max_rel_err(got.detach().cpu(), ref) < 1e-2
