@@ -796,16 +796,16 @@ using torch::autograd::variable_list;
 struct ConvBackward : public torch::autograd::Node {
     Call call;
     Held cache;
-    SavedVariable feats, weight, output;
-    Tensor mask;                        // the ReLU's derivative, one bit per output
-    bool relu = false, has_bias = false;
+    SavedVariable feats, weight, bias, output;      // (the bias only to refuse one that was changed in place)
+    SavedVariable mask;                 // the ReLU's derivative, one bit per output
+    bool relu = false, has_bias = false, has_mask = false;
 
     std::string name() const override { return call.generic ? "SparseConv3dBackward" : "SubMConv3dBackward"; }
     void release_variables() override {
         feats.reset_data();
         weight.reset_data();
         output.reset_data();
-        mask.reset();
+        mask.reset_data();
     }
 
     variable_list apply(variable_list&& grads) override {
@@ -815,6 +815,7 @@ struct ConvBackward : public torch::autograd::Node {
             const py::gil_scoped_acquire gil;
             e.restore();
             python_error err;
+        bias.reset_data();
             err.persist();
             throw err;
         }
@@ -826,16 +827,19 @@ struct ConvBackward : public torch::autograd::Node {
         const bool need_f = task_should_compute_output(0), need_w = task_should_compute_output(1);
         const bool need_b = has_bias && task_should_compute_output(2);
         const at::NoGradGuard no_grad;
-        const Tensor f = feats.unpack(), w = weight.unpack();
         const py::gil_scoped_acquire gil;
         if (cache.obj == nullptr) throw std::runtime_error("Trying to backward through the graph a second time");
         const Cache c(py::reinterpret_borrow<py::object>(cache.obj));
         const int64_t stream = stream_of(f);
         Tensor grad = grads[0];
-        if (relu && mask.defined()) grad = relu_mask_apply(grad, mask, stream);
-        else if (relu) grad = at::where(output.unpack(shared_from_this()).gt(0), grad, at::zeros({}, grad.options()));
+        if (has_mask) grad = relu_mask_apply(grad, m, stream);
+        else if (relu) grad = at::where(y.gt(0), grad, at::zeros({}, grad.options()));
         grad = grad.contiguous();
         const int64_t co = w.size(0), kw = w.size(1), kh = w.size(2), kd = w.size(3), ci = w.size(4), v = kw * kh * kd;
+        // (before anything else: a hook of the saved tensors may run the caller's code here)
+        const Tensor f = feats.unpack(), w = weight.unpack(), m = has_mask ? mask.unpack() : Tensor();
+        const Tensor y = relu && !has_mask ? output.unpack(shared_from_this()) : Tensor();
+        if (has_bias) (void)bias.unpack();
         if (need_f) {
             const Tensor wv = w.reshape({co, v, ci});
             if (call.generic) {
@@ -897,7 +901,8 @@ Tensor convolve(const Tensor& feats, py::object cache_obj, const Tensor& weight,
                            stream_of(feats));
     }
     if (!record) return p.out;
-    auto node = std::make_shared<ConvBackward>();
+    // (deleteNode: a long chain of layers is taken down without a stack frame per layer)
+    const std::shared_ptr<ConvBackward> node(new ConvBackward(), torch::autograd::deleteNode);
     node->set_next_edges(has_bias ? torch::autograd::collect_next_edges(feats, weight, bias) : torch::autograd::collect_next_edges(feats, weight));
     node->call.generic = generic;
     node->call.masked = masked;
@@ -907,7 +912,9 @@ Tensor convolve(const Tensor& feats, py::object cache_obj, const Tensor& weight,
     node->has_bias = has_bias;
     node->feats = SavedVariable(feats, false);
     node->weight = SavedVariable(weight, false);
-    node->mask = p.mask;
+    if (has_bias) node->bias = SavedVariable(bias, false);
+    node->has_mask = p.mask.defined();
+    if (node->has_mask) node->mask = SavedVariable(p.mask, false);
     torch::autograd::set_history(p.out, node);
     if (relu && !p.mask.defined()) node->output = SavedVariable(p.out, true);
     return p.out;

@@ -14,7 +14,7 @@ import weakref
 from typing import Optional, Tuple
 
 import torch
-from torch.autograd import Function
+from torch.autograd import Function, forward_ad
 
 from ... import _native as nat
 from .. import spconv, utils
@@ -1015,8 +1015,10 @@ class SubMConv3dFunction(Function):
 
 def _native_call(feats: torch.Tensor) -> bool:
     """Whether an operator call goes through the native host side, autograd node included (the implicit algorithms on the
-    GPU); the Python functions serve the others and calls that keep weight panels with their weights."""
-    return feats.is_cuda and not spconv.WEIGHT_PANEL_CACHE and spconv.ALGORITHM in _IMPLICIT
+    GPU); the Python functions serve the others, calls that keep weight panels with their weights, and calls under forward-mode
+    differentiation, a function transform or a tracer, which autograd answers for a Python function (most of them with an error)."""
+    return (feats.is_cuda and not spconv.WEIGHT_PANEL_CACHE and spconv.ALGORITHM in _IMPLICIT and forward_ad._current_level < 0
+            and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None)
 
 
 def _records_gradients(feats: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:

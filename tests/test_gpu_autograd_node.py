@@ -1,0 +1,81 @@
+"""The operators' native autograd node under what autograd offers around a node: hooks of the saved tensors, recomputation,
+refusal of what it does not differentiate, graphs thousands of layers deep."""
+import pytest
+import torch
+from torch.autograd import forward_ad
+from torch.utils.checkpoint import checkpoint
+
+import flex_gemm
+from flexgemm_amd.workloads import reference_test_shell
+
+spconv = flex_gemm.ops.spconv
+pytestmark = pytest.mark.gpu
+
+
+def _layer(device, relu, c=32):
+    gen = torch.Generator(device=device).manual_seed(5)
+    coords = torch.from_numpy(reference_test_shell(16)).to(device)
+    shape = torch.Size([1, c, 16, 16, 16])
+    feats = torch.randn(coords.shape[0], c, generator=gen, device=device).half().requires_grad_()
+    weight = (torch.randn(c, 3, 3, 3, c, generator=gen, device=device) / 30).half().requires_grad_()
+    bias = torch.randn(c, generator=gen, device=device).half().requires_grad_()
+    op = spconv.sparse_submanifold_conv3d_relu if relu else spconv.sparse_submanifold_conv3d
+    cache = op(feats, coords, shape, weight, bias)[1]
+    return lambda f, w, b: op(f, coords, shape, w, b, cache)[0], (feats, weight, bias)
+
+
+def _same(a, b):
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("relu,saved", [(False, 3), (True, 4)])
+def test_saved_tensor_hooks_see_every_saved_tensor(gpu_device, relu, saved):
+    layer, leaves = _layer(gpu_device, relu)
+    out = layer(*leaves)
+    up = torch.ones_like(out)
+    plain = torch.autograd.grad(out, leaves, up)
+    packed = []
+
+    def pack(t):
+        packed.append(t.shape)
+        return t.cpu()
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.to(gpu_device)):
+        out = layer(*leaves)
+    _same(torch.autograd.grad(out, leaves, up), plain)
+    assert len(packed) == saved
+
+
+@pytest.mark.parametrize("relu", [False, True])
+def test_recomputed_in_the_backward_pass(gpu_device, relu):
+    layer, leaves = _layer(gpu_device, relu)
+    out = layer(*leaves)
+    up = torch.ones_like(out)
+    plain = torch.autograd.grad(out, leaves, up)
+    again = checkpoint(lambda *a: layer(*a), *leaves, use_reentrant=False)
+    _same(torch.autograd.grad(again, leaves, up), plain)
+
+
+def test_what_is_not_differentiated_is_refused(gpu_device):
+    layer, (feats, weight, bias) = _layer(gpu_device, False)
+    with forward_ad.dual_level(), pytest.raises((NotImplementedError, RuntimeError)):
+        layer(forward_ad.make_dual(feats.detach(), torch.ones_like(feats)), weight, bias)
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda f: layer(f, weight.detach(), bias.detach()).float().sum())(feats.detach())
+    out = layer(feats, weight, bias)
+    torch.autograd.grad(out, feats, torch.ones_like(out))
+    with pytest.raises(RuntimeError, match="second time"):
+        torch.autograd.grad(out, feats, torch.ones_like(out))
+    for changed in (weight, bias):
+        out = layer(feats, weight, bias)
+        with torch.no_grad():
+            changed.add_(1)
+        with pytest.raises(RuntimeError, match="inplace"):
+            torch.autograd.grad(out, feats, torch.ones_like(out))
+
+
+def test_a_chain_of_many_layers_is_freed(gpu_device):
+    layer, (h, weight, bias) = _layer(gpu_device, False, c=8)
+    for _ in range(20000):
+        h = layer(h, weight, bias)
+    del h
