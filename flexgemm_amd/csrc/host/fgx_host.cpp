@@ -804,6 +804,7 @@ struct ConvBackward : public torch::autograd::Node {
     void release_variables() override {
         feats.reset_data();
         weight.reset_data();
+        bias.reset_data();
         output.reset_data();
         mask.reset_data();
     }
@@ -815,7 +816,6 @@ struct ConvBackward : public torch::autograd::Node {
             const py::gil_scoped_acquire gil;
             e.restore();
             python_error err;
-        bias.reset_data();
             err.persist();
             throw err;
         }
@@ -826,6 +826,10 @@ struct ConvBackward : public torch::autograd::Node {
         if (!grads[0].defined()) return result;
         const bool need_f = task_should_compute_output(0), need_w = task_should_compute_output(1);
         const bool need_b = has_bias && task_should_compute_output(2);
+        // (before anything else: a hook of the saved tensors may run the caller's code here)
+        const Tensor f = feats.unpack(), w = weight.unpack(), m = has_mask ? mask.unpack() : Tensor();
+        const Tensor y = relu && !has_mask ? output.unpack(shared_from_this()) : Tensor();
+        if (has_bias) (void)bias.unpack();
         const at::NoGradGuard no_grad;
         const py::gil_scoped_acquire gil;
         if (cache.obj == nullptr) throw std::runtime_error("Trying to backward through the graph a second time");
@@ -836,10 +840,6 @@ struct ConvBackward : public torch::autograd::Node {
         else if (relu) grad = at::where(y.gt(0), grad, at::zeros({}, grad.options()));
         grad = grad.contiguous();
         const int64_t co = w.size(0), kw = w.size(1), kh = w.size(2), kd = w.size(3), ci = w.size(4), v = kw * kh * kd;
-        // (before anything else: a hook of the saved tensors may run the caller's code here)
-        const Tensor f = feats.unpack(), w = weight.unpack(), m = has_mask ? mask.unpack() : Tensor();
-        const Tensor y = relu && !has_mask ? output.unpack(shared_from_this()) : Tensor();
-        if (has_bias) (void)bias.unpack();
         if (need_f) {
             const Tensor wv = w.reshape({co, v, ci});
             if (call.generic) {
