@@ -120,6 +120,37 @@ __global__ void __launch_bounds__(256) pack_weight_transpose_kernel(const uint16
 // ------------------------------------------------------------------------------------------------
 // Gather GEMM
 // ------------------------------------------------------------------------------------------------
+// Where the multiplicand of the gathered rows is read from: `lines` lines of one (offset, K-slab), line_stride bytes apart.
+//   columns (TR = false): a line is an output column, its K values side by side -- a panel of fgx_pack_weight, or the
+//     weight itself for the forward product;
+//   transposed (TR = true): a line is a K value, its columns side by side -- the weight itself for an input gradient.
+// Reading the weight itself takes out the pack launch and two of the three passes over the weight: 848 voxels, 1024 channels,
+// forward 0.097 -> 0.080 ms, input gradient 0.105 -> 0.078; 64 channels 0.0135 -> 0.0115; 9 744 voxels, 128 channels 0.037 -> 0.035;
+// none of 190 shapes from 192 to 38 720 voxels and 8 to 1024 channels slower (fp32 among them).
+struct BOperand {
+    const unsigned char* base;
+    long long v_stride, slab_stride;
+    int line_stride;
+    int lines;
+};
+
+using i16x4 = short __attribute__((ext_vector_type(4)));
+// Transposing LDS read: in a group of 16 lanes, lane s names 4 adjacent columns of K row s / 4 and receives 4 K values of column s.
+// Inline assembly, because the compiler would drain the loads into LDS in front of its builtin; lds_wait ties the results to
+// the wait.
+__device__ __forceinline__ i16x4 lds_read_tr16(const unsigned char* p) {
+    const uint32_t addr = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)p;
+    i16x4 r;
+    asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(r) : "v"(addr));
+    return r;
+}
+template <int N>
+__device__ __forceinline__ void lds_wait(i16x4 (&r)[N]) {
+    static_assert(N % 4 == 0, "results come in fours");
+#pragma unroll
+    for (int i = 0; i < N; i += 4) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[i]), "+v"(r[i + 1]), "+v"(r[i + 2]), "+v"(r[i + 3]));
+}
+
 template <typename Tag, int BM, int BN, int WAVES_M, int WAVES_N, int S, int CH>
 struct GemmCfg {
     using T = typename Tag::type;
@@ -135,6 +166,9 @@ struct GemmCfg {
     static constexpr int A_PER = (A_INST + NW - 1) / NW, B_PER = (B_INST + NW - 1) / NW;  // row loads per wavefront and step
     static constexpr int IDX_INST = (BM + 63) / 64;                  // wave-wide loads per index column
     static constexpr int LPS = A_PER + B_PER + 1;                    // + one index load
+    static constexpr int TCH = BN * ES / 16;                         // 16-byte pieces of a transposed line: [SK][BN] in place of [BN][SK]
+    static constexpr int TR_LINES_PER_INST = 64 / TCH;
+    static constexpr int tr_key(int line) { return TCH >= 16 ? 4 * (line & 3) : (TCH >= 8 ? 2 * (line & 3) : 0); }   // 4 lines of a read, 4 bank groups
     static constexpr int STAGE_BYTES = (BM + BN) * SLAB;
     static constexpr int IDX_SLOT_BYTES = IDX_INST * 256;
     static constexpr int OUT_PITCH = WN * ES + 16;                   // epilogue band: 32 rows of a wave tile
@@ -148,12 +182,12 @@ struct GemmCfg {
     static constexpr size_t lds_bytes = (size_t)RING_BYTES + (size_t)kIdxSlots * IDX_SLOT_BYTES + 1024 + (size_t)BM * 4 + 32 * 4;
 };
 
-template <typename Tag, int BM, int BN, int WAVES_M, int WAVES_N, int S, int CH>
+template <typename Tag, int BM, int BN, int WAVES_M, int WAVES_N, int S, int CH, bool TR>
 __global__ void __launch_bounds__(64 * WAVES_M * WAVES_N)
-gather_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Tag::type* __restrict__ panel,
+gather_gemm_kernel(const typename Tag::type* __restrict__ src, BOperand b,
                    const typename Tag::type* __restrict__ bias, const uint32_t* __restrict__ map,
                    const int64_t* __restrict__ sorted_idx, const int32_t* __restrict__ tile_code, uint32_t n, int K,
-                   int cols, int cols_pad, int V, int splitk, unsigned row_tiles, unsigned col_tiles,
+                   int cols, int V, int splitk, unsigned row_tiles, unsigned col_tiles, int by_columns,
                    float* __restrict__ partial, int act, typename Tag::type* __restrict__ out,
                    uint8_t* __restrict__ relu_mask) {
     using C = GemmCfg<Tag, BM, BN, WAVES_M, WAVES_N, S, CH>;
@@ -162,13 +196,14 @@ gather_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
     constexpr int kSlabBytes = C::SLAB, kChunks = CH;
 
     // XCD-aware tile order: workgroups are dealt round-robin to the 8 XCDs, so give each XCD a
-    // contiguous run of tiles (all column tiles of a row tile share their gathered rows -> same L2).
+    // contiguous run of tiles: all column tiles of a row tile, which share their gathered rows -> same L2, or (by_columns,
+    // a weight larger than the rows) all row tiles of a column tile, which share the weight's columns.
     const unsigned total_tiles = row_tiles * col_tiles;
     const unsigned per_xcd = (total_tiles + kXcds - 1) / kXcds;
     const unsigned logical = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
     if (logical >= total_tiles) return;
-    const unsigned row_tile = logical / col_tiles;
-    const unsigned col_tile = logical % col_tiles;
+    const unsigned row_tile = by_columns ? logical % row_tiles : logical / col_tiles;
+    const unsigned col_tile = by_columns ? logical / row_tiles : logical % col_tiles;
     const int kid = blockIdx.y;
 
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
@@ -222,7 +257,6 @@ gather_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
 
     const size_t row_bytes = (size_t)K * sizeof(T);
     const unsigned char* src_b = (const unsigned char*)src;
-    const unsigned char* panel_b = (const unsigned char*)panel;
     const unsigned char* zero_b = g_zero_block;
     const int sub_row = lane / kChunks, pch = lane % kChunks;
     const bool ragged = (row_bytes % kSlabBytes) != 0;   // last slab of a row is partly past the row end
@@ -253,8 +287,8 @@ gather_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
 
     // ---- row stream: runs S-1 steps ahead of the multiply stream and keeps per-lane source pointers that
     // advance by one slab per step; they are re-derived only when the offset changes ----
-    int a_row[C::A_PER], a_choff[C::A_PER], a_inc[C::A_PER], b_off[C::B_PER];
-    bool a_mine[C::A_PER], b_mine[C::B_PER];
+    int a_row[C::A_PER], a_choff[C::A_PER], a_inc[C::A_PER], b_off[C::B_PER], b_at[C::B_PER];
+    bool a_mine[C::A_PER], b_mine[C::B_PER], b_real[C::B_PER];
     const unsigned char* a_ptr[C::A_PER];
 #pragma unroll
     for (int i = 0; i < C::A_PER; ++i) {
@@ -269,12 +303,21 @@ gather_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
     for (int i = 0; i < C::B_PER; ++i) {
         const int inst = i * C::NW + wave;
         b_mine[i] = C::B_INST % C::NW == 0 || inst < C::B_INST;          // wave-uniform
-        const int col = (b_mine[i] ? inst : 0) * C::ROWS_PER_INST + sub_row;
-        b_off[i] = col * kSlabBytes + ((pch ^ swz_key<CH>(col)) << 4);
+        if constexpr (TR) {                                              // b_at: the K value inside the slab
+            b_at[i] = (b_mine[i] ? inst : 0) * C::TR_LINES_PER_INST + lane / C::TCH;
+            const int piece = (lane % C::TCH) ^ C::tr_key(b_at[i]);
+            b_off[i] = b_at[i] * b.line_stride + (piece << 4);
+            b_real[i] = b_mine[i] && (int)col_tile * BN + piece * (16 / C::ES) < cols;
+        } else {                                                         // b_at: the byte inside the slab
+            const int col = (b_mine[i] ? inst : 0) * C::ROWS_PER_INST + sub_row;
+            b_at[i] = (pch ^ swz_key<CH>(col)) << 4;
+            b_off[i] = col * b.line_stride + b_at[i];
+            b_real[i] = b_mine[i] && (int)col_tile * BN + col < b.lines;
+        }
     }
-    const size_t b_slab_stride = (size_t)cols_pad * kSlabBytes;
-    const unsigned char* b_ptr = zero_b;   // panel slice of the row stream's (offset, slab), column tile applied
-    size_t b_inc = 0;
+    const unsigned char* b_tile = b.base + (TR ? (size_t)col_tile * BN * C::ES : (size_t)col_tile * BN * (size_t)b.line_stride);
+    const unsigned char* b_ptr = zero_b;   // lines of the row stream's (offset, slab), column tile applied
+    long long b_inc = 0;
     int is_step = step_lo;                 // next step to enqueue
     int is_vi = slabs > 0 ? step_lo / slabs : 0;
     int is_slab = step_lo - is_vi * slabs;
@@ -295,8 +338,8 @@ gather_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
                 a_ptr[i] = real ? src_b + off : zero_b;
                 a_inc[i] = real ? kSlabBytes : 0;
             }
-            b_ptr = live ? panel_b + (((size_t)v * slabs + is_slab) * cols_pad + (size_t)col_tile * BN) * kSlabBytes : zero_b;
-            b_inc = live ? b_slab_stride : 0;
+            b_ptr = live ? b_tile + v * b.v_stride + is_slab * b.slab_stride : zero_b;
+            b_inc = live ? b.slab_stride : 0;
             is_fresh = false;
         }
         const bool tail = ragged && is_slab == slabs - 1;   // wave-uniform
@@ -310,7 +353,8 @@ gather_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
         }
 #pragma unroll
         for (int i = 0; i < C::B_PER; ++i) {
-            const unsigned char* p = (b_inc != 0 && b_mine[i]) ? b_ptr + b_off[i] : zero_b;
+            const bool past = tail && (TR ? is_slab * C::SK + b_at[i] >= K : (size_t)(is_slab * kSlabBytes + b_at[i]) >= row_bytes);
+            const unsigned char* p = (b_inc != 0 && b_real[i] && !past) ? b_ptr + b_off[i] : zero_b;
             unsigned char* dst = b_mine[i] ? stage + BM * kSlabBytes + (i * C::NW + wave) * 1024 : dump;
             __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(dst), 16, 0, 0);
         }
@@ -340,13 +384,22 @@ gather_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
 
     const int g = lane >> 5;        // lane group inside the MFMA fragment
     const int l32 = lane & 31;
+    constexpr int TB = kChunks * C::TN;                           // transposing reads of a step: two per fragment
+    const int s16 = lane & 15, half = (lane >> 4) & 1;
     int a_frag[kChunks / 2][C::TM], b_frag[kChunks / 2][C::TN];   // byte offsets of this lane's fragments in a stage
 #pragma unroll
     for (int kk = 0; kk < kChunks / 2; ++kk) {
 #pragma unroll
         for (int i = 0; i < C::TM; ++i) a_frag[kk][i] = swz<CH>(wave_m * C::WM + i * 32 + l32, kk * 2 + g);
 #pragma unroll
-        for (int j = 0; j < C::TN; ++j) b_frag[kk][j] = BM * kSlabBytes + swz<CH>(wave_n * C::WN + j * 32 + l32, kk * 2 + g);
+        for (int j = 0; j < C::TN; ++j) {
+            if constexpr (TR) {
+                const int line = kk * 16 + g * 8 + (s16 >> 2), byte = (wave_n * C::WN + j * 32 + half * 16 + (s16 & 3) * 4) * C::ES;
+                b_frag[kk][j] = BM * kSlabBytes + line * (C::TCH * 16) + (((byte >> 4) ^ C::tr_key(line)) << 4) + (byte & 15);
+            } else {
+                b_frag[kk][j] = BM * kSlabBytes + swz<CH>(wave_n * C::WN + j * 32 + l32, kk * 2 + g);
+            }
+        }
     }
     int cur_stage = 0;
     for (int step = step_lo; step < step_hi; ++step) {
@@ -360,12 +413,28 @@ gather_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
         const unsigned char* cur = ring + cur_stage * C::STAGE_BYTES;
         cur_stage = cur_stage + 1 == S ? 0 : cur_stage + 1;
         u32x4 af[kChunks / 2][C::TM], bf[kChunks / 2][C::TN];
+        i16x4 tr[TR ? TB : 4];
 #pragma unroll
         for (int kk = 0; kk < kChunks / 2; ++kk) {
 #pragma unroll
             for (int i = 0; i < C::TM; ++i) af[kk][i] = *(const u32x4*)(cur + a_frag[kk][i]);
 #pragma unroll
-            for (int j = 0; j < C::TN; ++j) bf[kk][j] = *(const u32x4*)(cur + b_frag[kk][j]);
+            for (int j = 0; j < C::TN; ++j) {
+                if constexpr (TR) {                 // (K rows 4 apart share a key)
+                    tr[(kk * C::TN + j) * 2] = lds_read_tr16(cur + b_frag[kk][j]);
+                    tr[(kk * C::TN + j) * 2 + 1] = lds_read_tr16(cur + b_frag[kk][j] + 4 * C::TCH * 16);
+                } else {
+                    bf[kk][j] = *(const u32x4*)(cur + b_frag[kk][j]);
+                }
+            }
+        }
+        if constexpr (TR) {
+            lds_wait(tr);
+#pragma unroll
+            for (int kk = 0; kk < kChunks / 2; ++kk)
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j)
+                    bf[kk][j] = __builtin_bit_cast(u32x4, __builtin_shufflevector(tr[(kk * C::TN + j) * 2], tr[(kk * C::TN + j) * 2 + 1], 0, 1, 2, 3, 4, 5, 6, 7));
         }
 #pragma unroll
         for (int kk = 0; kk < kChunks / 2; ++kk)
@@ -570,13 +639,13 @@ __global__ void __launch_bounds__(256) colsum_final_kernel(const float* __restri
 int elem_size(int dtype) { return dtype == FGX_F32 ? 4 : 2; }
 bool dtype_ok(int dtype) { return dtype == FGX_F16 || dtype == FGX_BF16 || dtype == FGX_F32; }
 
-template <typename Tag, int BM, int BN, int WAVES_M, int WAVES_N, int S, int CH>
-int launch_gemm(const void* src, const void* panel, const void* bias, const uint32_t* map, const int64_t* sorted_idx,
-                const int32_t* tile_code, size_t n, int K, int cols, int cols_pad, int V, int splitk, void* scratch,
+template <typename Tag, int BM, int BN, int WAVES_M, int WAVES_N, int S, int CH, bool TR>
+int launch_gemm(const void* src, const BOperand& b, const void* bias, const uint32_t* map, const int64_t* sorted_idx,
+                const int32_t* tile_code, size_t n, int K, int cols, int V, int splitk, void* scratch,
                 int act, void* out, uint8_t* relu_mask, hipStream_t s) {
     using C = GemmCfg<Tag, BM, BN, WAVES_M, WAVES_N, S, CH>;
     using T = typename Tag::type;
-    auto kern = gather_gemm_kernel<Tag, BM, BN, WAVES_M, WAVES_N, S, CH>;
+    auto kern = gather_gemm_kernel<Tag, BM, BN, WAVES_M, WAVES_N, S, CH, TR>;
     constexpr size_t lds = C::lds_bytes;
     static_assert(lds <= 160 * 1024, "tile does not fit the 160 KiB LDS");
     static thread_local bool lds_raised = false;   // raise the dynamic LDS limit once per thread and instantiation
@@ -588,8 +657,11 @@ int launch_gemm(const void* src, const void* panel, const void* bias, const uint
     const unsigned total = row_tiles * col_tiles;
     const unsigned grid_x = cdiv(total, kXcds) * kXcds;
     dim3 grid(grid_x, splitk, 1);
-    kern<<<grid, C::NT, lds, s>>>((const T*)src, (const T*)panel, (const T*)bias, map, sorted_idx, tile_code, (uint32_t)n, K,
-                                  cols, cols_pad, V, splitk, row_tiles, col_tiles, (float*)scratch, act, (T*)out,
+    // the larger operand is the one that should cross to one XCD only (848 voxels, 1024 channels, a 57 MB weight: all eight XCDs
+    // read half of it, 0.084 ms; an eighth each, 0.067).  fp32 multiplies sixteen times as long and keeps the rows' order.
+    const int by_columns = sizeof(T) == 2 && (size_t)V * cols > n;
+    kern<<<grid, C::NT, lds, s>>>((const T*)src, b, (const T*)bias, map, sorted_idx, tile_code, (uint32_t)n, K,
+                                  cols, V, splitk, row_tiles, col_tiles, by_columns, (float*)scratch, act, (T*)out,
                                   splitk > 1 ? nullptr : relu_mask);
     FGX_CHECK_LAUNCH("fgx_conv_gather_gemm");
     if (splitk > 1) {
@@ -602,14 +674,14 @@ int launch_gemm(const void* src, const void* panel, const void* bias, const uint
     return FGX_OK;
 }
 
-template <typename Tag>
-int dispatch_tile(int tile_rows, int tile_cols, int slab_bytes, const void* src, const void* panel, const void* bias,
+template <typename Tag, bool TR>
+int dispatch_tile(int tile_rows, int tile_cols, int slab_bytes, const void* src, const BOperand& b, const void* bias,
                   const uint32_t* map, const int64_t* sorted_idx, const int32_t* tile_code, size_t n, int K, int cols,
-                  int cols_pad, int V, int splitk, void* scratch, int act, void* out, uint8_t* relu_mask, hipStream_t s) {
+                  int V, int splitk, void* scratch, int act, void* out, uint8_t* relu_mask, hipStream_t s) {
 #define FGX_TILE(BM, BN, WMv, WNv, Sv, CHv)                                                                        \
     if (tile_rows == BM && tile_cols == BN && slab_bytes == CHv * 16)                                              \
-        return launch_gemm<Tag, BM, BN, WMv, WNv, Sv, CHv>(src, panel, bias, map, sorted_idx, tile_code, n, K, cols, \
-                                                           cols_pad, V, splitk, scratch, act, out, relu_mask, s);
+        return launch_gemm<Tag, BM, BN, WMv, WNv, Sv, CHv, TR>(src, b, bias, map, sorted_idx, tile_code, n, K, cols, \
+                                                               V, splitk, scratch, act, out, relu_mask, s);
     FGX_TILE(256, 128, 2, 2, 3, 4)
     FGX_TILE(256, 128, 4, 2, 3, 8)
     FGX_TILE(128, 128, 2, 2, 3, 4)
@@ -621,6 +693,55 @@ int dispatch_tile(int tile_rows, int tile_cols, int slab_bytes, const void* src,
 #undef FGX_TILE
     set_error("fgx_conv_gather_gemm: no kernel for tile %dx%d with %d-byte slabs", tile_rows, tile_cols, slab_bytes);
     return FGX_ERR_UNSUPPORTED;
+}
+
+// mode: of the weight that `b` is (as in fgx_pack_weight), or -1 for a panel
+int gather_gemm_checked(const char* who, int mode, int dtype, const void* src, const void* b, const void* bias, const uint32_t* map,
+                        const int64_t* sorted_idx, const int32_t* tile_code, size_t n, int K, int cols, int V, int tile_rows, int tile_cols,
+                        int slab_bytes, int splitk, void* scratch, int act, void* out, uint8_t* relu_mask, hipStream_t s) {
+    FGX_CHECK_ARG(act == FGX_ACT_NONE || act == FGX_ACT_RELU, "%s: unknown activation %d", who, act);
+    FGX_CHECK_ARG(relu_mask == nullptr || (act == FGX_ACT_RELU && dtype != FGX_F32 && cols % 8 == 0),
+                  "%s: a ReLU mask needs the ReLU epilogue, a 16-bit type and a multiple of 8 columns (got %d)", who, cols);
+    FGX_CHECK_ARG(dtype_ok(dtype), "%s: unknown dtype %d", who, dtype);
+    FGX_CHECK_ARG(K > 0 && cols > 0 && V >= 1 && V <= 32, "%s: bad shape K=%d cols=%d V=%d", who, K, cols, V);
+    FGX_CHECK_ARG(splitk >= 1 && splitk <= 1024, "%s: splitk %d out of range", who, splitk);
+    FGX_CHECK_ARG(n < 0xFFFFFFFFull, "%s: too many rows", who);
+    if (n == 0) return FGX_OK;
+    const int es = elem_size(dtype);
+    FGX_CHECK_ARG(((size_t)K * es) % 16 == 0, "%s: source row of %d elements is not a multiple of 16 bytes", who, K);
+    FGX_CHECK_ARG(src && b && map && sorted_idx && tile_code && out, "%s: null buffer", who);
+    FGX_CHECK_ARG((((uintptr_t)src | (uintptr_t)b) & 15) == 0, "%s: src and %s must be 16-byte aligned", who, mode < 0 ? "panel" : "weight");
+    FGX_CHECK_ARG(splitk == 1 || scratch != nullptr, "%s: split-K needs a scratch buffer", who);
+    FGX_CHECK_ARG(tile_rows > 0 && tile_cols > 0 && slab_bytes > 0 && cdiv(n, tile_rows) <= 0x7FFFFFu, "%s: too many row tiles", who);
+    BOperand op;
+    op.base = (const unsigned char*)b;
+    if (mode < 0) {
+        const int cols_pad = (int)align_up((size_t)cols, (size_t)tile_cols);
+        op.line_stride = slab_bytes;
+        op.slab_stride = (long long)cols_pad * slab_bytes;
+        op.v_stride = op.slab_stride * (long long)cdiv((size_t)K * es, (size_t)slab_bytes);
+        op.lines = cols_pad;
+    } else {                                                // [Co][V][Ci]
+        const int Ci = mode == 0 ? K : cols;
+        op.line_stride = V * Ci * es;
+        op.slab_stride = mode == 0 ? (long long)slab_bytes : (long long)(slab_bytes / es) * op.line_stride;
+        op.v_stride = (long long)Ci * es;
+        op.lines = mode == 0 ? cols : K;
+        if (mode == 1) {                                    // mirrored offsets
+            op.base += (V - 1) * op.v_stride;
+            op.v_stride = -op.v_stride;
+        }
+    }
+#define FGX_DISPATCH(Tag, TR) \
+    dispatch_tile<Tag, TR>(tile_rows, tile_cols, slab_bytes, src, op, bias, map, sorted_idx, tile_code, n, K, cols, V, splitk, scratch, act, out, \
+                           relu_mask, s)
+    if (mode > 0) return dtype == FGX_F16 ? FGX_DISPATCH(F16, true) : FGX_DISPATCH(BF16, true);
+    switch (dtype) {
+        case FGX_F16: return FGX_DISPATCH(F16, false);
+        case FGX_BF16: return FGX_DISPATCH(BF16, false);
+        default: return FGX_DISPATCH(F32, false);
+    }
+#undef FGX_DISPATCH
 }
 
 // both column-sum kernels on `s`, partial sums in `scratch` (kColsumSlices x cols floats)
@@ -731,28 +852,25 @@ int fgx_conv_gather_gemm_act_mask(int dtype, const void* src, const void* panel,
                                   const int64_t* sorted_idx, const int32_t* tile_code, size_t n, int K, int cols, int V,
                                   int tile_rows, int tile_cols, int slab_bytes, int splitk, void* scratch, int activation,
                                   void* out, uint8_t* relu_mask, fgx_stream_t stream) {
-    FGX_CHECK_ARG(activation == FGX_ACT_NONE || activation == FGX_ACT_RELU, "fgx_conv_gather_gemm: unknown activation %d", activation);
-    FGX_CHECK_ARG(relu_mask == nullptr || (activation == FGX_ACT_RELU && dtype != FGX_F32 && cols % 8 == 0),
-                  "fgx_conv_gather_gemm: a ReLU mask needs the ReLU epilogue, a 16-bit type and a multiple of 8 columns (got %d)", cols);
-    const int act = activation;
-    FGX_CHECK_ARG(dtype_ok(dtype), "fgx_conv_gather_gemm: unknown dtype %d", dtype);
-    FGX_CHECK_ARG(K > 0 && cols > 0 && V >= 1 && V <= 32, "fgx_conv_gather_gemm: bad shape K=%d cols=%d V=%d", K, cols, V);
-    FGX_CHECK_ARG(splitk >= 1 && splitk <= 1024, "fgx_conv_gather_gemm: splitk %d out of range", splitk);
-    FGX_CHECK_ARG(n < 0xFFFFFFFFull, "fgx_conv_gather_gemm: too many rows");
-    if (n == 0) return FGX_OK;
+    return gather_gemm_checked("fgx_conv_gather_gemm", -1, dtype, src, panel, bias, map, sorted_idx, tile_code, n, K, cols, V, tile_rows, tile_cols,
+                               slab_bytes, splitk, scratch, activation, out, relu_mask, (hipStream_t)stream);
+}
+
+int fgx_conv_gather_gemm_weight_pays(int dtype, int mode, int Ci, int Co, int V) {
+    if (!dtype_ok(dtype) || mode < 0 || mode > 2 || Ci <= 0 || Co <= 0 || V <= 0) return 0;
     const int es = elem_size(dtype);
-    FGX_CHECK_ARG(((size_t)K * es) % 16 == 0, "fgx_conv_gather_gemm: source row of %d elements is not a multiple of 16 bytes", K);
-    FGX_CHECK_ARG(src && panel && map && sorted_idx && tile_code && out, "fgx_conv_gather_gemm: null buffer");
-    FGX_CHECK_ARG((((uintptr_t)src | (uintptr_t)panel) & 15) == 0, "fgx_conv_gather_gemm: src and panel must be 16-byte aligned");
-    FGX_CHECK_ARG(splitk == 1 || scratch != nullptr, "fgx_conv_gather_gemm: split-K needs a scratch buffer");
-    FGX_CHECK_ARG(cdiv(n, tile_rows) <= 0x7FFFFFu, "fgx_conv_gather_gemm: too many row tiles");
-    const int cols_pad = (int)align_up((size_t)cols, (size_t)tile_cols);
-    hipStream_t s = (hipStream_t)stream;
-    switch (dtype) {
-        case FGX_F16: return dispatch_tile<F16>(tile_rows, tile_cols, slab_bytes, src, panel, bias, map, sorted_idx, tile_code, n, K, cols, cols_pad, V, splitk, scratch, act, out, relu_mask, s);
-        case FGX_BF16: return dispatch_tile<BF16>(tile_rows, tile_cols, slab_bytes, src, panel, bias, map, sorted_idx, tile_code, n, K, cols, cols_pad, V, splitk, scratch, act, out, relu_mask, s);
-        default: return dispatch_tile<F32>(tile_rows, tile_cols, slab_bytes, src, panel, bias, map, sorted_idx, tile_code, n, K, cols, cols_pad, V, splitk, scratch, act, out, nullptr, s);
-    }
+    if ((es == 4 && mode != 0) || Ci % (16 / es) != 0 || Co % (16 / es) != 0) return 0;
+    return (size_t)V * Ci * Co * es < ((size_t)1 << 31);       // (lines are addressed with 32-bit offsets)
+}
+
+int fgx_conv_gather_gemm_weight(int dtype, int mode, const void* src, const void* weight, const void* bias, const uint32_t* map,
+                                const int64_t* sorted_idx, const int32_t* tile_code, size_t n, int Ci, int Co, int V,
+                                int tile_rows, int tile_cols, int slab_bytes, int splitk, void* scratch, int activation,
+                                void* out, uint8_t* relu_mask, fgx_stream_t stream) {
+    FGX_CHECK_ARG(fgx_conv_gather_gemm_weight_pays(dtype, mode, Ci, Co, V), "fgx_conv_gather_gemm_weight: dtype %d, mode %d, Ci=%d Co=%d V=%d takes a panel",
+                  dtype, mode, Ci, Co, V);
+    return gather_gemm_checked("fgx_conv_gather_gemm_weight", mode, dtype, src, weight, bias, map, sorted_idx, tile_code, n, mode == 0 ? Ci : Co,
+                               mode == 0 ? Co : Ci, V, tile_rows, tile_cols, slab_bytes, splitk, scratch, activation, out, relu_mask, (hipStream_t)stream);
 }
 
 int fgx_relu_mask_apply(int dtype, const void* grad, const uint8_t* relu_mask, size_t numel, void* out, fgx_stream_t stream) {

@@ -40,6 +40,7 @@ namespace {
     X(fgx_spconv_out_dims) X(fgx_spconv_out_coords_grid_workspace_bytes) X(fgx_spconv_out_coords_grid_count)                       \
     X(fgx_spconv_out_coords_grid_emit) X(fgx_tile_plan) X(fgx_gather_item_order) X(fgx_gather_item_order_workspace_bytes)          \
     X(fgx_weight_panel_bytes) X(fgx_pack_weight) X(fgx_conv_scratch_bytes) X(fgx_conv_gather_gemm_act_mask)                        \
+    X(fgx_conv_gather_gemm_weight_pays) X(fgx_conv_gather_gemm_weight)                                                             \
     X(fgx_conv_gather_gemm_stream_act_mask) X(fgx_conv_gather_gemm_stream_groups) X(fgx_relu_mask_apply)                           \
     X(fgx_colsum_scratch_bytes) X(fgx_colsum) X(fgx_wgrad_block_bounds_count) X(fgx_wgrad_block_bounds)                            \
     X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
@@ -571,13 +572,20 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
         p.out = make({n, cols}, src.scalar_type(), dev);
         return p;
     }
+    // the streaming kernel addresses its operands with 32-bit byte offsets
+    const double most = (double)0xFF000000u;
+    const bool streams = s.stream && (double)n_src * row_bytes <= most && (double)n * 8 <= most && (double)n * 27 * 4 * 2 <= most;
+    const bool narrow = narrow_shape(c, es, k, cols, v, n) &&
+                        impl_function("_narrow_applies")(c.obj, src, k, cols, v, n, n_src, python_schedule(pass, src, n, ci, co, v)).cast<bool>();
     Tensor panel = panel_kept;
-    if (!panel.defined()) {
+    // the tiled kernel reads the weight itself where it can
+    const bool direct = !panel.defined() && !narrow && !streams && ((uintptr_t)weight.data_ptr() & 15) == 0 &&
+                        L.fgx_conv_gather_gemm_weight_pays(code, mode, ci, co, v);
+    if (!direct && !panel.defined()) {
         panel = workspace(L.fgx_weight_panel_bytes(code, mode, ci, co, v, s.slab_bytes, s.tile_cols), dev);
         check(L.fgx_pack_weight(code, mode, ptr(weight), ci, co, v, s.slab_bytes, s.tile_cols, ptr(panel), as_stream(stream)));
     }
-    if (narrow_shape(c, es, k, cols, v, n) &&
-        impl_function("_narrow_applies")(c.obj, src, k, cols, v, n, n_src, python_schedule(pass, src, n, ci, co, v)).cast<bool>()) {
+    if (narrow) {
         py::tuple got = impl_function("_narrow_gemm")(src, panel, bias.defined() ? py::cast(bias) : py::none(), c.obj, mode, k, cols, v, activation, want_mask);
         p.out = got[0].cast<Tensor>();
         if (!got[1].is_none()) p.mask = got[1].cast<Tensor>();
@@ -587,9 +595,7 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
     if (want_mask && activation == FGX_ACT_RELU && es == 2 && cols % 8 == 0) p.mask = make({n * cols / 8}, at::kByte, dev);
     const void* b = ptr(bias);
     const char* name = mode == 0 ? "gather_gemm_fwd" : "gather_gemm_dgrad";
-    // the streaming kernel addresses its operands with 32-bit byte offsets
-    const double most = (double)0xFF000000u;
-    if (s.stream && (double)n_src * row_bytes <= most && (double)n * 8 <= most && (double)n * 27 * 4 * 2 <= most) {
+    if (streams) {
         int groups = 0;
         check(L.fgx_conv_gather_gemm_stream_groups(code, cols, s.tile_rows, s.tile_cols, s.slab_bytes, &groups));
         Tensor item_at;
@@ -614,9 +620,14 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
         Tensor scratch;
         if (splitk > 1) scratch = workspace(L.fgx_conv_scratch_bytes((size_t)n, cols, splitk), dev);
         mark(name, "start");
-        check(L.fgx_conv_gather_gemm_act_mask(code, ptr(src), ptr(panel), b, ptr<uint32_t>(nmap), ptr<int64_t>(t.order), ptr<int32_t>(t.code),
-                                              (size_t)n, k, cols, v, s.tile_rows, s.tile_cols, s.slab_bytes, splitk, ptr(scratch), activation,
-                                              ptr(p.out), ptr<uint8_t>(p.mask), as_stream(stream)));
+        if (direct)
+            check(L.fgx_conv_gather_gemm_weight(code, mode, ptr(src), ptr(weight), b, ptr<uint32_t>(nmap), ptr<int64_t>(t.order), ptr<int32_t>(t.code),
+                                                (size_t)n, ci, co, v, s.tile_rows, s.tile_cols, s.slab_bytes, splitk, ptr(scratch), activation,
+                                                ptr(p.out), ptr<uint8_t>(p.mask), as_stream(stream)));
+        else
+            check(L.fgx_conv_gather_gemm_act_mask(code, ptr(src), ptr(panel), b, ptr<uint32_t>(nmap), ptr<int64_t>(t.order), ptr<int32_t>(t.code),
+                                                  (size_t)n, k, cols, v, s.tile_rows, s.tile_cols, s.slab_bytes, splitk, ptr(scratch), activation,
+                                                  ptr(p.out), ptr<uint8_t>(p.mask), as_stream(stream)));
     }
     mark(name, "stop");
     return p;

@@ -281,6 +281,16 @@ int fgx_conv_gather_gemm_act_mask(int dtype, const void* src, const void* panel,
                                   const uint32_t* map, const int64_t* sorted_idx, const int32_t* tile_code,
                                   size_t n, int K, int cols, int V, int tile_rows, int tile_cols, int slab_bytes, int splitk,
                                   void* scratch, int activation, void* out, uint8_t* relu_mask, fgx_stream_t stream);
+
+/* The same product with the multiplicand read from the weight itself ([Co, V, Ci], dense, 16-byte aligned) instead of a packed
+ * panel.  mode as in fgx_pack_weight; src rows have Ci elements in mode 0 and Co in the others.  16-bit types in all modes,
+ * fp32 in mode 0; Ci and Co whole 16-byte pieces, the weight under 2 GiB: fgx_conv_gather_gemm_weight_pays says whether a
+ * shape is taken (1) or needs a panel (0). */
+int fgx_conv_gather_gemm_weight_pays(int dtype, int mode, int Ci, int Co, int V);
+int fgx_conv_gather_gemm_weight(int dtype, int mode, const void* src, const void* weight, const void* bias,
+                                const uint32_t* map, const int64_t* sorted_idx, const int32_t* tile_code, size_t n,
+                                int Ci, int Co, int V, int tile_rows, int tile_cols, int slab_bytes, int splitk,
+                                void* scratch, int activation, void* out, uint8_t* relu_mask, fgx_stream_t stream);
 /* out[i] = bit i of relu_mask ? grad[i] : 0 for i < numel (a multiple of 8; 16-bit types; grad and out 16-byte aligned,
  * out may be grad): the gradient of a fused ReLU from the mask its forward pass wrote.  One pass, numel / 8 bytes of mask
  * read beside the gradient.  No counterpart in the reference. */
