@@ -663,7 +663,7 @@ Tensor wgrad_bounds(const Cache& c, const Tensor& sig_o, const std::vector<uint3
     return bounds;
 }
 
-Tensor wgrad_item_lists(const Cache& c, const Tensor& bounds, size_t n, int v, int ci, int co, const Sched& s, int64_t stream) {
+Tensor wgrad_item_lists(const Cache& c, const Tensor& bounds, size_t n, int v, int ci, int co, const Sched& s, bool only_if_they_pay, int64_t stream) {
     const std::string key = "_wgrad_lists_" + std::to_string(s.block_rows) + "_" + std::to_string(s.tile_rows) + "_" + std::to_string(s.tile_cols) +
                             "_" + std::to_string(ci) + "_" + std::to_string(co);
     Tensor lists;
@@ -672,6 +672,10 @@ Tensor wgrad_item_lists(const Cache& c, const Tensor& bounds, size_t n, int v, i
         return lists;                                   // (None: the library has none for the shape)
     }
     const size_t words = L.fgx_wgrad_item_lists_count(n, v, ci, co, s.tile_rows, s.tile_cols, s.block_rows);
+    // with no more items than workgroups there is nothing to even out, and the fixed interleave hands out one item each
+    // (3 716 voxels, 64 channels: 108 items; making their lists took 18 us beside a weight gradient of 12)
+    const size_t items = (size_t)v * ceil_div(co, s.tile_rows) * ceil_div(ci, s.tile_cols) * (size_t)ceil_div((int64_t)n, s.block_rows);
+    if (only_if_they_pay && words > 0 && items <= words - 4 - items) return lists;
     if (words > 0) {
         lists = make({(int64_t)words}, at::kUInt32, bounds.device());
         check(L.fgx_wgrad_item_lists(ptr<uint32_t>(bounds), n, v, ci, co, s.tile_rows, s.tile_cols, s.block_rows, ptr<uint32_t>(lists), as_stream(stream)));
@@ -742,7 +746,7 @@ WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool 
             const Tensor bounds = wgrad_bounds(c, sig_o, seg, (size_t)n, v, s.block_rows, stream);
             Tensor lists;
             if (s.stream == 1 && PyObject_IsTrue(module_get(g_impl, "WGRAD_BALANCED_LISTS")))
-                lists = wgrad_item_lists(c, bounds, (size_t)n, v, ci, co, s, stream);
+                lists = wgrad_item_lists(c, bounds, (size_t)n, v, ci, co, s, true, stream);
             Tensor scratch = workspace(L.fgx_wgrad_scratch_bytes((size_t)n, v, ci, co, s.block_rows), dev);
             mark("wgrad", "start");
             check(L.fgx_conv_wgrad_lists(code, ptr(grad), ptr(feats), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o), seg.data(), ptr<uint32_t>(bounds),
@@ -989,7 +993,7 @@ py::object py_wgrad_item_lists(py::object cache_obj, int block_rows, int tile_ro
     const Tensor nmap = c.need("neighbor_map");
     const c10::DeviceGuard guard(nmap.device());
     const Sched s{tile_rows, tile_cols, 0, 1, block_rows, 1};
-    const Tensor t = wgrad_item_lists(c, bounds, (size_t)nmap.size(0), (int)nmap.size(1), ci, co, s, stream_of(nmap));
+    const Tensor t = wgrad_item_lists(c, bounds, (size_t)nmap.size(0), (int)nmap.size(1), ci, co, s, false, stream_of(nmap));
     return t.defined() ? py::cast(t) : py::none();
 }
 
