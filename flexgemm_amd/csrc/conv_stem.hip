@@ -1,0 +1,532 @@
+// The convolutions of a network's first layers (16-bit types, 8 or 16 channels on the gathered side, kernels of 17 ... 27 offsets):
+// all offsets of a voxel side by side are one row of a matrix.  First the weight gradient:
+//
+//   grad_weight[co][v][ci] = sum over rows r with a neighbor at offset v of grad_out[r][co] * feats[map[r][v]][ci]
+//
+// As products per offset (wgrad_gemm.hip) every (row, offset) pair fetches a grad_out row of 2 * Co bytes for 16 or 32 bytes
+// of features, and the 32-wide tile multiplies mostly padding.  Here the features of a row's V neighbors lie next to each other
+// in LDS (a missing neighbor: zeros), [rows][V * Ci], and one product with the rows' own grad_out gives every offset at
+// once: grad_out is read once per 64 of its columns, the pair lists not at all.  What bounds it are the 16-byte gathers, one
+// per (row, offset): 64 rows a step take 1.4 us of a CU, 1 792 pieces at about 0.6 per clock.  A last piece per row holds a one: its column is the bias gradient.
+// A workgroup keeps all accumulators over its contiguous run of rows and writes one partial product; a second kernel adds the
+// partial products in workgroup order (same bits on every run).
+#include "wgrad_device.h"
+
+namespace fgx {
+namespace {
+
+__device__ __attribute__((aligned(256))) unsigned char g_zero_block_s[256];
+// the piece (16 bytes) that starts with a one
+__device__ __attribute__((aligned(256))) uint16_t g_one_f16[8] = {0x3C00, 0, 0, 0, 0, 0, 0, 0};
+__device__ __attribute__((aligned(256))) uint16_t g_one_bf16[8] = {0x3F80, 0, 0, 0, 0, 0, 0, 0};
+
+constexpr int kStemWaves = 8, kStemThreads = 64 * kStemWaves, kStemStages = 3, kStemIdxSlots = 4;
+constexpr int kStemMaxV = 27, kStemCols = 64;
+
+// P: 16-byte pieces of a feature row (Ci = 8 P)
+template <int P>
+struct StemCfg {
+    static constexpr int ROWS = 64 / P;                        // rows of a step
+    static constexpr int PIECES = 28 * P;                      // of an LDS row: the offsets', the ones, padding
+    static constexpr int N = PIECES * 8, NT = N / 32;          // columns of the product, in tiles of 32
+    static constexpr int NT_PER = (NT + 3) / 4;                // ... per wavefront (4 share them, 2 the rows of the product)
+    static constexpr int ROWB = PIECES * 16;
+    static constexpr int F_BYTES = ROWS * ROWB, G_BYTES = ROWS * kStemCols * 2;
+    static constexpr int F_INST = F_BYTES / 1024, G_INST = G_BYTES / 1024;
+    static constexpr int PER = (F_INST + G_INST + kStemWaves - 1) / kStemWaves;    // row loads per wavefront and step
+    static constexpr int LPS = PER + 1;                        // + one load of map words
+    static constexpr int IDX_BYTES = ROWS * kStemMaxV * 4;
+    static constexpr int IDX_SLOT = (IDX_BYTES + 1023) / 1024 * 1024;
+    static constexpr int STAGE = F_BYTES + G_BYTES;
+    static constexpr size_t LDS = (size_t)kStemStages * STAGE + kStemIdxSlots * IDX_SLOT + 1024;
+    static_assert(IDX_SLOT / 1024 <= kStemWaves && F_BYTES % 1024 == 0, "one load of map words per wavefront");
+    static_assert(NT_PER % 2 == 0, "fragments are waited for in fours");
+    static_assert(LDS <= 160 * 1024, "LDS");
+    // XOR key on the 16-byte pieces of a grad_out row (8 of them): four rows of a transposing read on distinct banks.  Rows of
+    // the feature side are 448 bytes (or 896) apart: 7 * 64 bytes put any four on distinct banks by themselves (two and two).
+    static constexpr int key(int row) { return 2 * (row & 3); }
+};
+
+// Map words of step j: ROWS * V of them in a row, 16 bytes per lane; past the map's end, and in the steps after the last one, zeros
+// that nobody reads.
+template <int P>
+__device__ __forceinline__ void stem_issue_idx(const uint32_t* map, unsigned long long map_bytes, unsigned lo, int nsteps, int j, int V, int wave,
+                                               int lane, unsigned char* slot, unsigned char* dump, const unsigned char* zero_b) {
+    using C = StemCfg<P>;
+    const unsigned long long at = (unsigned long long)(lo + (unsigned)j) * (unsigned)(C::ROWS * V * 4) + (unsigned)(wave * 1024 + lane * 16);
+    const bool real = j < nsteps && wave * 1024 + lane * 16 < C::ROWS * V * 4 && at + 16 <= map_bytes;
+    const unsigned char* p = real ? (const unsigned char*)map + at : zero_b;
+    unsigned char* dst = wave * 1024 < C::IDX_SLOT ? slot + wave * 1024 : dump;
+    __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(dst), 16, 0, 0);
+}
+
+// Where piece `at` of row `row` of a step comes from.  WHOLE: a step with all its rows; the last one has `rows`, and its map
+// rows are read where they are (16 bytes of them may end past the map).
+template <int P, bool WHOLE>
+__device__ __forceinline__ const unsigned char* stem_piece(const unsigned char* feats, const uint32_t* map, const uint32_t* words,
+                                                           const unsigned char* one_b, const unsigned char* zero_b, unsigned long long base,
+                                                           int row, int rows, int at, int V) {
+    const int v = at / P, part = at - v * P;
+    if (!WHOLE && row >= rows) return zero_b;
+    if (v < V) {
+        const uint32_t m = WHOLE ? words[row * V + v] : map[(base + (unsigned)row) * (unsigned)V + (unsigned)v];
+        return m != FGX_EMPTY32 ? feats + (size_t)m * (16 * P) + part * 16 : zero_b;
+    }
+    return at == StemCfg<P>::PIECES - 1 ? one_b : zero_b;
+}
+
+template <typename Tag, int P>
+__global__ void __launch_bounds__(kStemThreads)
+stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Tag::type* __restrict__ feats, const uint32_t* __restrict__ map,
+                  uint32_t n, int V, int Co, unsigned steps_total, unsigned groups, float* __restrict__ partial) {
+    using C = StemCfg<P>;
+    constexpr int S = kStemStages;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    unsigned char* ring = lds;                                 // [S][features | grad_out]
+    unsigned char* idx_ring = lds + S * C::STAGE;              // [kStemIdxSlots] map rows
+    unsigned char* dump = idx_ring + kStemIdxSlots * C::IDX_SLOT;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_m = wave & 1, wave_n = wave >> 1;
+    const int g = lane >> 5, l32 = lane & 31, s16 = lane & 15, mb = (lane >> 4) & 1;
+    const int m0 = (int)blockIdx.y * kStemCols;
+
+    // workgroups of one XCD take neighboring runs of steps
+    const unsigned per_xcd = (groups + kXcds - 1) / kXcds;
+    const unsigned group = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+    if (group >= groups) return;
+    const unsigned lo = (unsigned)((unsigned long long)steps_total * group / groups);
+    const unsigned hi = (unsigned)((unsigned long long)steps_total * (group + 1) / groups);
+    const int nsteps = (int)(hi - lo);
+
+    const unsigned char* gout_b = (const unsigned char*)gout;
+    const unsigned char* feats_b = (const unsigned char*)feats;
+    const unsigned char* one_b = (const unsigned char*)(__is_same(typename Tag::type, _Float16) ? g_one_f16 : g_one_bf16);
+    const unsigned char* zero_b = g_zero_block_s;
+    const unsigned long long map_bytes = (unsigned long long)n * V * 4;
+
+    auto issue_idx = [&](int j) {
+        stem_issue_idx<P>(map, map_bytes, lo, nsteps, j, V, wave, lane, idx_ring + (j & (kStemIdxSlots - 1)) * C::IDX_SLOT, dump, zero_b);
+    };
+    auto issue_rows_of = [&](int j, auto whole) {
+        constexpr bool WHOLE = decltype(whole)::value;
+        unsigned char* stage = ring + (j % S) * C::STAGE;
+        const uint32_t* words = (const uint32_t*)(idx_ring + (j & (kStemIdxSlots - 1)) * C::IDX_SLOT);
+        const unsigned long long base = (unsigned long long)(lo + (unsigned)j) * C::ROWS;
+        const int rows = WHOLE ? C::ROWS : (j < nsteps && base < n ? (int)(n - base) : 0);
+#pragma unroll
+        for (int i = 0; i < C::PER; ++i) {
+            const int inst = i * kStemWaves + wave;            // wave-uniform
+            const unsigned char* p = zero_b;
+            unsigned char* dst = dump;
+            if (inst < C::F_INST) {
+                const int piece = inst * 64 + lane;
+                const int row = piece / C::PIECES;
+                dst = stage + inst * 1024;
+                p = stem_piece<P, WHOLE>(feats_b, map, words, one_b, zero_b, base, row, rows, piece - row * C::PIECES, V);
+            } else if (inst < C::F_INST + C::G_INST) {
+                const int piece = (inst - C::F_INST) * 64 + lane;
+                const int row = piece >> 3, c = ((piece & 7) ^ C::key(row)) * 8;       // first column
+                dst = stage + C::F_BYTES + (inst - C::F_INST) * 1024;
+                if ((WHOLE || row < rows) && m0 + c < Co) p = gout_b + ((base + (unsigned)row) * (unsigned)Co + (unsigned)(m0 + c)) * 2;
+            }
+            __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(dst), 16, 0, 0);
+        }
+    };
+    auto issue_rows = [&](int j) {
+        if (j < nsteps && (unsigned long long)(lo + (unsigned)j + 1) * C::ROWS <= n) issue_rows_of(j, std::true_type{});
+        else issue_rows_of(j, std::false_type{});
+    };
+
+    f32x16 acc[C::NT_PER];
+#pragma unroll
+    for (int t = 0; t < C::NT_PER; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
+
+#pragma unroll
+    for (int j = 0; j < S - 1; ++j) issue_idx(j);
+    wait_vmcnt<0>();
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < S - 1; ++j) {
+        issue_rows(j);
+        issue_idx(j + S - 1);
+    }
+
+    constexpr int NK = C::ROWS / 16;
+    for (int k = 0; k < nsteps; ++k) {
+        wait_vmcnt<(S - 2) * C::LPS>();                        // rows of step k and the map words of step k + S - 1 have landed
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();                          // ... everybody's; the stage of step k - 1 is free
+        asm volatile("" ::: "memory");
+        issue_rows(k + S - 1);
+        issue_idx(k + 2 * (S - 1));
+        const unsigned char* f_cur = ring + (k % S) * C::STAGE;
+        const unsigned char* g_cur = f_cur + C::F_BYTES;
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk) {
+            const int row = kk * 16 + g * 8 + (s16 >> 2);      // (see wgrad_gemm.hip on the transposing read)
+            i16x4 fr[2 * C::NT_PER + 4];                       // (two of them fill the last group of four)
+            {
+                const int byte = (wave_m * 32 + mb * 16 + (s16 & 3) * 4) * 2;
+                const unsigned char* at = g_cur + row * (kStemCols * 2) + (((byte >> 4) ^ C::key(row)) << 4) + (byte & 15);
+                fr[0] = lds_read_tr16(at);
+                fr[1] = lds_read_tr16(at + 4 * kStemCols * 2);
+            }
+#pragma unroll
+            for (int t = 0; t < C::NT_PER; ++t) {
+                const int tile = wave_n * C::NT_PER + t < C::NT ? wave_n * C::NT_PER + t : 0;
+                const unsigned char* at = f_cur + row * C::ROWB + (tile * 32 + mb * 16 + (s16 & 3) * 4) * 2;
+                fr[2 + 2 * t] = lds_read_tr16(at);
+                fr[3 + 2 * t] = lds_read_tr16(at + 4 * C::ROWB);
+            }
+            fr[2 + 2 * C::NT_PER] = fr[3 + 2 * C::NT_PER] = i16x4{0, 0, 0, 0};
+            lds_wait_all(fr);
+            const i16x8 af = __builtin_shufflevector(fr[0], fr[1], 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+            for (int t = 0; t < C::NT_PER; ++t) {
+                const i16x8 bf = __builtin_shufflevector(fr[2 + 2 * t], fr[3 + 2 * t], 0, 1, 2, 3, 4, 5, 6, 7);
+                mma16<Tag>(acc[t], af, bf);
+            }
+        }
+    }
+    wait_vmcnt<0>();                                           // the loads of the steps past the end
+
+    // partial[column tile][group][64][N]
+    float* dst = partial + ((size_t)blockIdx.y * groups + group) * ((size_t)kStemCols * C::N);
+#pragma unroll
+    for (int t = 0; t < C::NT_PER; ++t) {
+        const int tile = wave_n * C::NT_PER + t;
+        if (tile >= C::NT) continue;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int m = wave_m * 32 + (e >> 2) * 8 + g * 4 + (e & 3);
+            dst[(size_t)m * C::N + tile * 32 + l32] = acc[t][e];
+        }
+    }
+}
+
+// grad_weight and grad_bias: 32 columns of blockDim.z rows of the product per workgroup, blockDim.y threads per element each adding
+// every blockDim.y-th partial product, their sums added in order.  An infinity or NaN in grad_out times the zeros of a missing neighbor is NaN where the
+// sum over the pairs has no such term: an element that comes out like that is summed again over its pairs alone.
+template <typename T>
+__global__ void __launch_bounds__(1024) stem_reduce_kernel(const float* __restrict__ partial, unsigned groups, int V, int Ci, int Co, int N,
+                                                           const T* __restrict__ gout, const T* __restrict__ feats,
+                                                           const uint32_t* __restrict__ map, uint32_t n, T* __restrict__ gw, T* __restrict__ gb) {
+    __shared__ float sums[32][33];                             // [rows * slices][32]
+    const int c = threadIdx.x, slices = blockDim.y, slice = threadIdx.y, at = threadIdx.z * slices;
+    const int col = blockIdx.x * 32 + c, co = blockIdx.y * blockDim.z + threadIdx.z;
+    const size_t per = (size_t)kStemCols * N;
+    const float* src = partial + (size_t)(co / kStemCols) * groups * per + (size_t)(co % kStemCols) * N + col;
+    float s = 0.f;
+    unsigned b = co < Co ? slice : groups;
+    for (; b + 3 * slices < groups; b += 4 * slices) {
+        const float x0 = src[b * per], x1 = src[(b + slices) * per], x2 = src[(b + 2 * slices) * per], x3 = src[(b + 3 * slices) * per];
+        s += x0; s += x1; s += x2; s += x3;
+    }
+    for (; b < groups; b += slices) s += src[b * per];
+    sums[at + slice][c] = s;
+    __syncthreads();
+    float r = sums[at][c];
+    for (int q = 1; q < slices; ++q) r += sums[at + q][c];
+    const bool again = co < Co && col < V * Ci && !(fabsf(r) < __builtin_inff());
+    if (__syncthreads_or(again)) {
+        __syncthreads();                                       // (the sums have been read)
+        s = 0.f;
+        if (again) {
+            const int v = col / Ci, ci = col - v * Ci;
+            for (size_t row = slice; row < n; row += slices) {
+                const uint32_t m = map[row * V + v];
+                if (m != FGX_EMPTY32) s += (float)gout[row * Co + co] * (float)feats[(size_t)m * Ci + ci];
+            }
+        }
+        sums[at + slice][c] = s;
+        __syncthreads();
+        if (again) {
+            r = sums[at][c];
+            for (int q = 1; q < slices; ++q) r += sums[at + q][c];
+        }
+    }
+    if (slice != 0 || co >= Co) return;
+    if (col < V * Ci) gw[(size_t)co * V * Ci + col] = from_float<T>(r);
+    else if (gb != nullptr && col == N - 8) gb[co] = from_float<T>(r);
+}
+
+// Forward product and input gradient of such layers (8 or 16 channels on the gathered side): the neighbors' features of a row lie
+// side by side as in the weight gradient, and one product with the weight, [V * K] x [columns], replaces V products that fill
+// a quarter (8 channels) or half of a K-slab.  The wavefronts keep the weight in registers over the workgroup's run of rows; the
+// piece with the one multiplies the bias.  Rows are walked as they come, nothing of the mask sort is read.
+template <int P>
+struct StemGemmCfg {
+    using W = StemCfg<P>;
+    static constexpr int COLS = 128;                           // output columns of a workgroup: four tiles of 32, one per wavefront column
+    static constexpr int RT = W::ROWS / 32;                    // row tiles of a step
+    static constexpr int KK = W::PIECES / 2;                   // products of a tile: 16 K values each
+    static constexpr int PER = (W::F_INST + kStemWaves - 1) / kStemWaves;
+    static constexpr int LPS = PER + 1;
+    static constexpr int STAGES = 4, IDX_SLOTS = 2 * (STAGES - 1);     // (a slot is written again once its step's rows are on their way)
+    static constexpr size_t LDS = (size_t)STAGES * W::F_BYTES + IDX_SLOTS * W::IDX_SLOT + 1024;
+    static_assert(LDS <= 160 * 1024, "LDS");
+    // XOR key on the low bits of a row's piece numbers: 16 rows' reads of one piece fall on distinct banks (rows are 28 or 56 pieces)
+    static __device__ __forceinline__ int key(int row) { return P == 1 ? (row >> 2) & 3 : (row >> 1) & 7; }
+};
+
+// mode as in fgx_pack_weight: 0 weight [cols][V][K], 1 / 2 weight [K][V][cols] with mirrored offsets / as they are
+template <typename Tag, int P>
+__global__ void __launch_bounds__(kStemThreads)
+stem_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Tag::type* __restrict__ weight,
+                 const typename Tag::type* __restrict__ bias, const uint32_t* __restrict__ map, uint32_t n, int V, int cols, int mode,
+                 unsigned steps_total, unsigned groups, int relu, typename Tag::type* __restrict__ out, uint8_t* __restrict__ relu_mask) {
+    using C = StemCfg<P>;
+    using G = StemGemmCfg<P>;
+    using T = typename Tag::type;
+    constexpr int S = G::STAGES;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    unsigned char* ring = lds;                                 // [S][rows' features]
+    unsigned char* idx_ring = lds + S * C::F_BYTES;
+    unsigned char* dump = idx_ring + G::IDX_SLOTS * C::IDX_SLOT;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int g = lane >> 5, l32 = lane & 31;
+    const int ct = wave & 3, rt = wave >> 2;                   // column and row tile of this wavefront
+    const int c0 = (int)blockIdx.y * G::COLS + ct * 32;
+    const bool multiplies = rt < G::RT && c0 < cols;
+
+    const unsigned per_xcd = (groups + kXcds - 1) / kXcds;
+    const unsigned group = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+    if (group >= groups) return;
+    const unsigned lo = (unsigned)((unsigned long long)steps_total * group / groups);
+    const unsigned hi = (unsigned)((unsigned long long)steps_total * (group + 1) / groups);
+    const int nsteps = (int)(hi - lo);
+
+    // the weight's fragments: lane l32 is a column, a piece its 8 consecutive K values
+    i16x8 wf[G::KK];
+#pragma unroll
+    for (int kk = 0; kk < G::KK; ++kk) {
+        i16x8 f = {0, 0, 0, 0, 0, 0, 0, 0};
+        const int at = kk * 2 + g, v = at / P, part = at - v * P, col = c0 + l32;
+        if (multiplies && col < cols) {
+            if (v < V && mode == 0) {
+                f = *reinterpret_cast<const i16x8*>((const short*)weight + ((size_t)col * V + v) * (8 * P) + part * 8);
+            } else if (v < V) {
+                const int from = mode == 1 ? V - 1 - v : v;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) f[e] = ((const short*)weight)[((size_t)(part * 8 + e) * V + from) * cols + col];
+            } else if (at == C::PIECES - 1 && bias != nullptr) {
+                f[0] = ((const short*)bias)[col];
+            }
+        }
+        wf[kk] = f;
+    }
+
+    const unsigned char* src_b = (const unsigned char*)src;
+    const unsigned char* one_b = (const unsigned char*)(__is_same(T, _Float16) ? g_one_f16 : g_one_bf16);
+    const unsigned char* zero_b = g_zero_block_s;
+    const unsigned long long map_bytes = (unsigned long long)n * V * 4;
+    auto issue_idx = [&](int j) {
+        stem_issue_idx<P>(map, map_bytes, lo, nsteps, j, V, wave, lane, idx_ring + (j % G::IDX_SLOTS) * C::IDX_SLOT, dump, zero_b);
+    };
+    auto issue_rows_of = [&](int j, auto whole) {
+        constexpr bool WHOLE = decltype(whole)::value;
+        unsigned char* stage = ring + (j % S) * C::F_BYTES;
+        const uint32_t* words = (const uint32_t*)(idx_ring + (j % G::IDX_SLOTS) * C::IDX_SLOT);
+        const unsigned long long base = (unsigned long long)(lo + (unsigned)j) * C::ROWS;
+        const int rows = WHOLE ? C::ROWS : (j < nsteps && base < n ? (int)(n - base) : 0);
+#pragma unroll
+        for (int i = 0; i < G::PER; ++i) {
+            const int inst = i * kStemWaves + wave;            // wave-uniform
+            const unsigned char* p = zero_b;
+            unsigned char* dst = dump;
+            if (inst < C::F_INST) {
+                const int piece = inst * 64 + lane;
+                const int row = piece / C::PIECES, at = (piece - row * C::PIECES) ^ G::key(row);
+                dst = stage + inst * 1024;
+                p = stem_piece<P, WHOLE>(src_b, map, words, one_b, zero_b, base, row, rows, at, V);
+            }
+            __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(dst), 16, 0, 0);
+        }
+    };
+    auto issue_rows = [&](int j) {
+        if (j < nsteps && (unsigned long long)(lo + (unsigned)j + 1) * C::ROWS <= n) issue_rows_of(j, std::true_type{});
+        else issue_rows_of(j, std::false_type{});
+    };
+
+#pragma unroll
+    for (int j = 0; j < S - 1; ++j) issue_idx(j);
+    wait_vmcnt<0>();
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < S - 1; ++j) {
+        issue_rows(j);
+        issue_idx(j + S - 1);
+    }
+    const int frag_row = rt * 32 + l32;
+    for (int k = 0; k < nsteps; ++k) {
+        // rows of step k and the map words of step k + S - 1 have landed (stores count as well: the wait is only stricter)
+        wait_vmcnt<(S - 2) * G::LPS>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        issue_rows(k + S - 1);
+        issue_idx(k + 2 * (S - 1));
+        if (!multiplies) continue;
+        const unsigned char* row_at = ring + (k % S) * C::F_BYTES + frag_row * C::ROWB;
+        f32x16 acc;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < G::KK; ++kk) {
+            const i16x8 rf = *reinterpret_cast<const i16x8*>(row_at + (((kk * 2 + g) ^ G::key(frag_row)) << 4));
+            mma16<Tag>(acc, wf[kk], rf);                       // [column][row]: a lane ends up with columns of one row
+        }
+        // element e of lane l: column 8 * (e / 4) + 4 * (l / 32) + e % 4, row l % 32
+        const unsigned long long row = (unsigned long long)(lo + (unsigned)k) * C::ROWS + (unsigned)frag_row;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            using T4 = T __attribute__((ext_vector_type(4)));
+            T4 four;
+            uint32_t bits = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float x = acc[q * 4 + e];
+                four[e] = from_float<T>(relu ? fmaxf(x, 0.f) : x);
+                bits |= (uint32_t)((float)four[e] > 0.f) << e;
+            }
+            const uint32_t high = (uint32_t)__shfl_xor((int)bits, 32, 64);
+            const int col = c0 + q * 8 + g * 4;
+            if (row >= n || col >= cols) continue;             // (cols is a multiple of 8)
+            *reinterpret_cast<T4*>(out + row * (unsigned)cols + col) = four;
+            if (relu_mask != nullptr && g == 0) relu_mask[(row * (unsigned)cols + col) >> 3] = (uint8_t)(bits | high << 4);
+        }
+    }
+    wait_vmcnt<0>();
+}
+
+// Workgroups per 64 columns of grad_out: the chip full, and at least four steps each -- a partial product of 57 KB (Ci = 16: 115)
+// is written and read for every one.
+unsigned stem_groups(size_t n, int Ci, int Co) {
+    const size_t runs = cdiv(n, 4 * (64 / (Ci / 8)));
+    const unsigned col_tiles = cdiv(Co, kStemCols);
+    const size_t most = col_tiles >= 256 ? 1 : 256 / col_tiles;
+    return (unsigned)(runs < most ? (runs ? runs : 1) : most);
+}
+
+template <typename Tag, int P>
+int stem_launch(const void* gout, const void* feats, const uint32_t* map, size_t n, int Co, int V, float* scratch, void* gw, void* gb, hipStream_t s) {
+    using C = StemCfg<P>;
+    using T = typename Tag::type;
+    auto kern = stem_wgrad_kernel<Tag, P>;
+    static thread_local bool lds_raised = false;
+    if (!lds_raised) {
+        FGX_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS));
+        lds_raised = true;
+    }
+    const unsigned groups = stem_groups(n, 8 * P, Co), col_tiles = cdiv(Co, kStemCols);
+    const dim3 grid(cdiv(groups, kXcds) * kXcds, col_tiles);
+    kern<<<grid, kStemThreads, C::LDS, s>>>((const T*)gout, (const T*)feats, map, (uint32_t)n, V, Co, cdiv(n, C::ROWS), groups, scratch);
+    FGX_CHECK_LAUNCH("fgx_conv_wgrad_stem");
+    unsigned slices = 1;
+    while (slices < 32 && slices * 8 < groups) slices *= 2;
+    const unsigned rows = slices >= 8 ? 1 : 8 / slices;
+    stem_reduce_kernel<T><<<dim3(C::N / 32, cdiv(Co, rows)), dim3(32, slices, rows), 0, s>>>(scratch, groups, V, 8 * P, Co, C::N, (const T*)gout, (const T*)feats, map, (uint32_t)n,
+                                                                 (T*)gw, (T*)gb);
+    FGX_CHECK_LAUNCH("fgx_conv_wgrad_stem(reduce)");
+    return FGX_OK;
+}
+
+template <typename Tag, int P>
+int stem_gemm_launch(int mode, const void* src, const void* weight, const void* bias, const uint32_t* map, size_t n, int cols, int V, int relu,
+                     void* out, uint8_t* relu_mask, hipStream_t s) {
+    using C = StemCfg<P>;
+    using G = StemGemmCfg<P>;
+    using T = typename Tag::type;
+    auto kern = stem_gemm_kernel<Tag, P>;
+    static thread_local bool lds_raised = false;
+    if (!lds_raised) {
+        FGX_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)G::LDS));
+        lds_raised = true;
+    }
+    const unsigned steps = cdiv(n, C::ROWS), col_tiles = cdiv(cols, G::COLS);
+    const unsigned most = col_tiles >= 256 ? 1 : 256 / col_tiles, groups = steps < most ? steps : most;
+    const dim3 grid(cdiv(groups, kXcds) * kXcds, col_tiles);
+    kern<<<grid, kStemThreads, G::LDS, s>>>((const T*)src, (const T*)weight, (const T*)bias, map, (uint32_t)n, V, cols, mode, steps, groups, relu,
+                                            (T*)out, relu_mask);
+    FGX_CHECK_LAUNCH("fgx_conv_gemm_stem");
+    return FGX_OK;
+}
+
+bool stem_wgrad_takes(int dtype, size_t n, int Ci, int Co, int V) {
+    return (dtype == FGX_F16 || dtype == FGX_BF16) && (Ci == 8 || Ci == 16) && Co > 0 && Co % 8 == 0 && Co <= 65535 && V >= 17 && V <= kStemMaxV &&
+           n > 0 && n < 0xFFFFFFFFull;
+}
+
+bool stem_gemm_takes(int dtype, size_t n, int K, int cols, int V) {
+    return (dtype == FGX_F16 || dtype == FGX_BF16) && (K == 8 || K == 16) && cols > 0 && cols % 8 == 0 && cols <= 65535 * 128 && V >= 17 &&
+           V <= kStemMaxV && n > 0 && n < 0xFFFFFFFFull;
+}
+
+}  // namespace
+}  // namespace fgx
+
+using namespace fgx;
+
+extern "C" {
+
+// Weight gradient, ms: 424 000 voxels 6 (padded to 8) -> 48 channels 0.132 on the streaming kernel, 0.043 here; 143 616 voxels
+// 8 -> 64 0.053 and 0.023, 16 -> 64 0.057 and 0.036; 848 voxels 8 -> 48 0.013 and 0.011.  With 16 channels and few voxels the partial
+// products weigh as much as the pairs: level up to 64 columns, behind over more (15 192 voxels 16 -> 128 0.027 and 0.028).
+int fgx_wgrad_stem_pays(int dtype, size_t n, int Ci, int Co, int V) {
+    return stem_wgrad_takes(dtype, n, Ci, Co, V) && (Ci == 8 || Co <= 64 || n >= 24576);
+}
+
+size_t fgx_wgrad_stem_scratch_bytes(size_t n, int Ci, int Co) {
+    if ((Ci != 8 && Ci != 16) || Co <= 0) return 0;
+    return (size_t)stem_groups(n, Ci, Co) * cdiv(Co, kStemCols) * kStemCols * (size_t)(28 * Ci) * sizeof(float);
+}
+
+int fgx_conv_wgrad_stem(int dtype, const void* grad_out, const void* feats, const uint32_t* map, size_t n, int Ci, int Co, int V, void* scratch,
+                        void* grad_weight, void* grad_bias, fgx_stream_t stream) {
+    FGX_CHECK_ARG(stem_wgrad_takes(dtype, n, Ci, Co, V), "fgx_conv_wgrad_stem: dtype %d, n=%zu, Ci=%d, Co=%d, V=%d is not for this kernel", dtype, n,
+                  Ci, Co, V);
+    FGX_CHECK_ARG(grad_out && feats && map && scratch && grad_weight, "fgx_conv_wgrad_stem: null buffer");
+    FGX_CHECK_ARG((((uintptr_t)grad_out | (uintptr_t)feats | (uintptr_t)map | (uintptr_t)scratch) & 15) == 0,
+                  "fgx_conv_wgrad_stem: grad_out, feats, map and scratch must be 16-byte aligned");
+    hipStream_t s = (hipStream_t)stream;
+    if (dtype == FGX_F16)
+        return Ci == 8 ? stem_launch<F16, 1>(grad_out, feats, map, n, Co, V, (float*)scratch, grad_weight, grad_bias, s)
+                       : stem_launch<F16, 2>(grad_out, feats, map, n, Co, V, (float*)scratch, grad_weight, grad_bias, s);
+    return Ci == 8 ? stem_launch<BF16, 1>(grad_out, feats, map, n, Co, V, (float*)scratch, grad_weight, grad_bias, s)
+                   : stem_launch<BF16, 2>(grad_out, feats, map, n, Co, V, (float*)scratch, grad_weight, grad_bias, s);
+}
+
+// Forward, ms (the tiled kernel, this one): 424 000 voxels 6 -> 48 channels 0.090 and 0.066; 143 616 voxels 8 -> 128 0.049 and 0.025, 16 ->
+// 128 0.050 and 0.038; 15 192 voxels 8 -> 64 0.019 and 0.008; 192 voxels 0.010 and 0.007; level at 624 264 voxels 16 -> 64.  An input gradient
+// fetches its fragments of the weight one value at a time: 3 us more per launch, and the streaming kernel keeps 16 channels of
+// many voxels up to 64 columns (143 616 voxels 0.040 and 0.047; 96 columns 0.052 and 0.048).
+int fgx_conv_gemm_stem_pays(int dtype, int mode, size_t n, int K, int cols, int V) {
+    if (mode < 0 || mode > 2 || !stem_gemm_takes(dtype, n, K, cols, V)) return 0;
+    return mode == 0 || (K == 8 ? n >= 768 : n >= 3072 && cols >= 96);
+}
+
+int fgx_conv_gemm_stem(int dtype, int mode, const void* src, const void* weight, const void* bias, const uint32_t* map, size_t n, int Ci, int Co,
+                       int V, int activation, void* out, uint8_t* relu_mask, fgx_stream_t stream) {
+    FGX_CHECK_ARG(mode >= 0 && mode <= 2, "fgx_conv_gemm_stem: mode must be 0 (forward), 1 (dgrad, mirrored offsets) or 2 (dgrad)");
+    const int K = mode == 0 ? Ci : Co, cols = mode == 0 ? Co : Ci;
+    FGX_CHECK_ARG(stem_gemm_takes(dtype, n, K, cols, V), "fgx_conv_gemm_stem: dtype %d, n=%zu, K=%d, cols=%d, V=%d is not for this kernel", dtype, n, K,
+                  cols, V);
+    FGX_CHECK_ARG(activation == FGX_ACT_NONE || activation == FGX_ACT_RELU, "fgx_conv_gemm_stem: unknown activation %d", activation);
+    FGX_CHECK_ARG(relu_mask == nullptr || activation == FGX_ACT_RELU, "fgx_conv_gemm_stem: a ReLU mask needs the ReLU epilogue");
+    FGX_CHECK_ARG(src && weight && map && out, "fgx_conv_gemm_stem: null buffer");
+    FGX_CHECK_ARG((((uintptr_t)src | (uintptr_t)weight | (uintptr_t)map | (uintptr_t)out) & 15) == 0,
+                  "fgx_conv_gemm_stem: src, weight, map and out must be 16-byte aligned");
+    const int relu = activation == FGX_ACT_RELU;
+    hipStream_t s = (hipStream_t)stream;
+    if (dtype == FGX_F16)
+        return K == 8 ? stem_gemm_launch<F16, 1>(mode, src, weight, bias, map, n, cols, V, relu, out, relu_mask, s)
+                      : stem_gemm_launch<F16, 2>(mode, src, weight, bias, map, n, cols, V, relu, out, relu_mask, s);
+    return K == 8 ? stem_gemm_launch<BF16, 1>(mode, src, weight, bias, map, n, cols, V, relu, out, relu_mask, s)
+                  : stem_gemm_launch<BF16, 2>(mode, src, weight, bias, map, n, cols, V, relu, out, relu_mask, s);
+}
+
+}  // extern "C"

@@ -43,7 +43,7 @@ namespace {
     X(fgx_conv_gather_gemm_weight_pays) X(fgx_conv_gather_gemm_weight)                                                             \
     X(fgx_conv_gather_gemm_stream_act_mask) X(fgx_conv_gather_gemm_stream_groups) X(fgx_relu_mask_apply)                           \
     X(fgx_colsum_scratch_bytes) X(fgx_colsum) X(fgx_wgrad_block_bounds_count) X(fgx_wgrad_block_bounds)                            \
-    X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
+    X(fgx_conv_gemm_stem_pays) X(fgx_conv_gemm_stem) X(fgx_wgrad_stem_pays) X(fgx_wgrad_stem_scratch_bytes) X(fgx_conv_wgrad_stem) X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
     X(fgx_wgrad_sweep_plan_bytes) X(fgx_wgrad_sweep_plan) X(fgx_wgrad_sweep_scratch_bytes) X(fgx_conv_wgrad_sweep)                 \
     X(fgx_serialize_encode) X(fgx_serialize_decode) X(fgx_table_lookup)
 
@@ -479,8 +479,11 @@ py::object python_schedule(int pass, const Tensor& like, int64_t n, int ci, int 
         pass, py::cast(like).attr("dtype"), n, ci, co, v);
 }
 
+// Nobody has replaced the schedules: a forced one names the kernels that take schedules, not the first layers'.
+bool schedules_are_ours() { return module_get(g_native, "table_lookup") == g_table_lookup; }
+
 Sched schedule(int pass, const Tensor& like, int64_t n, int ci, int co, int v) {
-    if (module_get(g_native, "table_lookup") != g_table_lookup) return read_schedule(python_schedule(pass, like, n, ci, co, v));
+    if (!schedules_are_ours()) return read_schedule(python_schedule(pass, like, n, ci, co, v));
     struct Key {
         int pass, code, ci, co, v;
         int64_t n;
@@ -507,6 +510,8 @@ Sched schedule(int pass, const Tensor& like, int64_t n, int ci, int co, int v) {
     }
     return it->second;
 }
+
+bool aligned(const Tensor& t) { return ((uintptr_t)t.data_ptr() & 15) == 0; }
 
 py::object impl_function(const char* name) { return py::reinterpret_borrow<py::object>(module_get(g_impl, name)); }
 
@@ -559,6 +564,18 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
     if (bias.defined()) bias = bias.contiguous();
     const int co = (int)weight.size(0), ci = (int)weight.size(2), k = mode == 0 ? ci : co;
     const int64_t row_bytes = (int64_t)k * es;
+    // a network's first layers: all offsets of a row in one product, no row order or tile tables
+    if (n > 0 && !panel_kept.defined() && L.fgx_conv_gemm_stem_pays(code, mode, (size_t)n, k, cols, v) && !narrow_shape(c, es, k, cols, v, n) &&
+        schedules_are_ours() && aligned(src) && aligned(weight)) {
+        const char* name = mode == 0 ? "gather_gemm_fwd" : "gather_gemm_dgrad";
+        p.out = make({n, cols}, src.scalar_type(), dev);
+        if (want_mask && activation == FGX_ACT_RELU) p.mask = make({n * cols / 8}, at::kByte, dev);
+        mark(name, "start");
+        check(L.fgx_conv_gemm_stem(code, mode, ptr(src), ptr(weight), ptr(bias), ptr<uint32_t>(nmap), (size_t)n, ci, co, v, activation, ptr(p.out),
+                                   ptr<uint8_t>(p.mask), as_stream(stream)));
+        mark(name, "stop");
+        return p;
+    }
     if (masked && !(c.has("gray_code") && c.has("sorted_idx"))) c.obj.attr("_ensure_sorted")();
     const int pass = mode == 0 ? 0 : 1;
     const Sched s = schedule(pass, src, n, ci, co, v);
@@ -578,10 +595,9 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
     const bool narrow = narrow_shape(c, es, k, cols, v, n) &&
                         impl_function("_narrow_applies")(c.obj, src, k, cols, v, n, n_src, python_schedule(pass, src, n, ci, co, v)).cast<bool>();
     Tensor panel = panel_kept;
-    // the tiled kernel reads the weight itself where it can
-    // (fp32 rows that end inside a 64-byte slab keep their panel, whose lines
-    // all start on one: 716 voxels, 296 channels, three layers: 0.269 ms, direct 0.272 ... 0.278)
-    const bool direct = !panel.defined() && !narrow && !streams && ((uintptr_t)weight.data_ptr() & 15) == 0 && (es == 2 || (int64_t)ci * es % 64 == 0) &&
+    // the tiled kernel reads the weight itself where it can; fp32 rows that end inside a 64-byte slab keep their panel, whose lines
+    // all start on one (716 voxels, 296 channels, three layers: 0.269 ms, direct 0.272 ... 0.278)
+    const bool direct = !panel.defined() && !narrow && !streams && aligned(weight) && (es == 2 || (int64_t)ci * es % 64 == 0) &&
                         L.fgx_conv_gather_gemm_weight_pays(code, mode, ci, co, v);
     if (!direct && !panel.defined()) {
         panel = workspace(L.fgx_weight_panel_bytes(code, mode, ci, co, v, s.slab_bytes, s.tile_cols), dev);
@@ -707,6 +723,15 @@ WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool 
         py::tuple got = impl_function("_narrow_wgrad")(grad, feats, c.obj, v, with_bias);
         w.weight = got[0].cast<Tensor>();
         if (with_bias) w.bias = got[1].cast<Tensor>();
+    } else if (L.fgx_wgrad_stem_pays(code, (size_t)n, ci, co, v) && n_in > 0 && schedules_are_ours() && aligned(feats) && aligned(grad)) {
+        const Tensor nmap = c.need("neighbor_map");
+        Tensor scratch = workspace(L.fgx_wgrad_stem_scratch_bytes((size_t)n, ci, co), dev);
+        w.weight = make({co, v, ci}, feats.scalar_type(), dev);
+        if (with_bias) w.bias = make({co}, feats.scalar_type(), dev);
+        mark("wgrad", "start");
+        check(L.fgx_conv_wgrad_stem(code, ptr(grad), ptr(feats), ptr<uint32_t>(nmap), (size_t)n, ci, co, v, ptr(scratch), ptr(w.weight), ptr(w.bias),
+                                    as_stream(stream)));
+        mark("wgrad", "stop");
     } else {
         if (!(c.has("valid_signal_seg") && (c.has("valid_signal_i") || c.has("_pending_pairs")))) c.obj.attr("_ensure_pairs")();
         const Tensor sig_i = c.need("valid_signal_i"), sig_o = c.need("valid_signal_o");

@@ -387,6 +387,21 @@ size_t fgx_narrow_wgrad_scratch_bytes(int V);
 int fgx_conv_narrow_wgrad(int dtype, const void* grad_out, const void* feats, const void* plan, size_t n, size_t n_src, int Ci,
                           int Co, int V, void* scratch, void* grad_weight, fgx_stream_t stream);
 
+/* Forward product and input gradient of a network's first layers: K (Ci in mode 0, Co in modes 1 and 2, modes as in
+ * fgx_pack_weight) of 8 or 16, 16-bit types, V of 17 ... 27, a multiple of 8 columns.  Reads the neighbor map [n, V] row by row and
+ * the weight itself; no row order, tile masks or panel.  fgx_conv_gemm_stem_pays says where it is the faster kernel. */
+int fgx_conv_gemm_stem_pays(int dtype, int mode, size_t n, int K, int cols, int V);
+int fgx_conv_gemm_stem(int dtype, int mode, const void* src, const void* weight, const void* bias, const uint32_t* map, size_t n,
+                       int Ci, int Co, int V, int activation, void* out, uint8_t* relu_mask, fgx_stream_t stream);
+
+/* The weight gradient of a network's first layers: Ci of 8 or 16, 16-bit types, V of 17 ... 27, Co a multiple of 8, straight from
+ * the neighbor map ([n, V], row r of grad_out its row r) without pair lists.  grad_bias (optional) comes with it.
+ * fgx_wgrad_stem_pays says where it is the faster kernel.  scratch: fgx_wgrad_stem_scratch_bytes bytes; buffers 16-byte aligned. */
+int fgx_wgrad_stem_pays(int dtype, size_t n, int Ci, int Co, int V);
+size_t fgx_wgrad_stem_scratch_bytes(size_t n, int Ci, int Co);
+int fgx_conv_wgrad_stem(int dtype, const void* grad_out, const void* feats, const uint32_t* map, size_t n, int Ci, int Co, int V,
+                        void* scratch, void* grad_weight, void* grad_bias, fgx_stream_t stream);
+
 /* item_at for fgx_conv_gather_gemm_stream, made on the device from the tile codes: items sorted by cost (offsets per
  * row tile x `slabs` K-slabs + an epilogue), the incomplete last round of `groups` positions filled with the cheapest,
  * every full round dealt most-expensive-item to least-loaded-slot.  One workgroup, deterministic, no read-back;
