@@ -132,6 +132,7 @@ struct BOperand {
     long long v_stride, slab_stride;
     int line_stride;
     int lines;
+    int ends_inside;        // the last K-slab may end inside a line (a panel is padded to whole slabs)
 };
 
 using i16x4 = short __attribute__((ext_vector_type(4)));
@@ -343,6 +344,7 @@ gather_gemm_kernel(const typename Tag::type* __restrict__ src, BOperand b,
             is_fresh = false;
         }
         const bool tail = ragged && is_slab == slabs - 1;   // wave-uniform
+        const bool b_tail = tail && b.ends_inside != 0;
 #pragma unroll
         for (int i = 0; i < C::A_PER; ++i) {
             const unsigned char* p = a_ptr[i];
@@ -353,7 +355,7 @@ gather_gemm_kernel(const typename Tag::type* __restrict__ src, BOperand b,
         }
 #pragma unroll
         for (int i = 0; i < C::B_PER; ++i) {
-            const bool past = tail && (TR ? is_slab * C::SK + b_at[i] >= K : (size_t)(is_slab * kSlabBytes + b_at[i]) >= row_bytes);
+            const bool past = b_tail && (TR ? is_slab * C::SK + b_at[i] >= K : (size_t)(is_slab * kSlabBytes + b_at[i]) >= row_bytes);
             const unsigned char* p = (b_inc != 0 && b_real[i] && !past) ? b_ptr + b_off[i] : zero_b;
             unsigned char* dst = b_mine[i] ? stage + BM * kSlabBytes + (i * C::NW + wave) * 1024 : dump;
             __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(dst), 16, 0, 0);
@@ -756,12 +758,14 @@ int gather_gemm_checked(const char* who, int mode, int dtype, const void* src, c
         op.slab_stride = (long long)cols_pad * slab_bytes;
         op.v_stride = op.slab_stride * (long long)cdiv((size_t)K * es, (size_t)slab_bytes);
         op.lines = cols_pad;
+        op.ends_inside = 0;
     } else {                                                // [Co][V][Ci]
         const int Ci = mode == 0 ? K : cols;
         op.line_stride = V * Ci * es;
         op.slab_stride = mode == 0 ? (long long)slab_bytes : (long long)(slab_bytes / es) * op.line_stride;
         op.v_stride = (long long)Ci * es;
         op.lines = mode == 0 ? cols : K;
+        op.ends_inside = 1;
         if (mode == 1) {                                    // mirrored offsets
             op.base += (V - 1) * op.v_stride;
             op.v_stride = -op.v_stride;
@@ -894,7 +898,7 @@ int fgx_conv_gather_gemm_act_mask(int dtype, const void* src, const void* panel,
 int fgx_conv_gather_gemm_weight_pays(int dtype, int mode, int Ci, int Co, int V) {
     if (!dtype_ok(dtype) || mode < 0 || mode > 2 || Ci <= 0 || Co <= 0 || V <= 0) return 0;
     const int es = elem_size(dtype);
-    if ((es == 4 && mode != 0) || Ci % (16 / es) != 0 || Co % (16 / es) != 0) return 0;
+    if ((es == 4 && mode != 0) || Ci % (16 / es) != 0 || (mode != 0 && Co % (16 / es) != 0)) return 0;
     return (size_t)V * Ci * Co * es < ((size_t)1 << 31);       // (lines are addressed with 32-bit offsets)
 }
 

@@ -595,10 +595,8 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
     const bool narrow = narrow_shape(c, es, k, cols, v, n) &&
                         impl_function("_narrow_applies")(c.obj, src, k, cols, v, n, n_src, python_schedule(pass, src, n, ci, co, v)).cast<bool>();
     Tensor panel = panel_kept;
-    // the tiled kernel reads the weight itself where it can; fp32 rows that end inside a 64-byte slab keep their panel, whose lines
-    // all start on one (716 voxels, 296 channels, three layers: 0.269 ms, direct 0.272 ... 0.278)
-    const bool direct = !panel.defined() && !narrow && !streams && aligned(weight) && (es == 2 || (int64_t)ci * es % 64 == 0) &&
-                        L.fgx_conv_gather_gemm_weight_pays(code, mode, ci, co, v);
+    // the tiled kernel reads the weight itself where it can
+    const bool direct = !panel.defined() && !narrow && !streams && aligned(weight) && L.fgx_conv_gather_gemm_weight_pays(code, mode, ci, co, v);
     if (!direct && !panel.defined()) {
         panel = workspace(L.fgx_weight_panel_bytes(code, mode, ci, co, v, s.slab_bytes, s.tile_cols), dev);
         check(L.fgx_pack_weight(code, mode, ptr(weight), ci, co, v, s.slab_bytes, s.tile_cols, ptr(panel), as_stream(stream)));

@@ -284,7 +284,7 @@ int fgx_conv_gather_gemm_act_mask(int dtype, const void* src, const void* panel,
 
 /* The same product with the multiplicand read from the weight itself ([Co, V, Ci], dense, 16-byte aligned) instead of a packed
  * panel.  mode as in fgx_pack_weight; src rows have Ci elements in mode 0 and Co in the others.  16-bit types in all modes,
- * fp32 in mode 0; Ci and Co whole 16-byte pieces, the weight under 2 GiB: fgx_conv_gather_gemm_weight_pays says whether a
+ * fp32 in mode 0; Ci (and Co but in mode 0) whole 16-byte pieces, the weight under 2 GiB: fgx_conv_gather_gemm_weight_pays says whether a
  * shape is taken (1) or needs a panel (0). */
 int fgx_conv_gather_gemm_weight_pays(int dtype, int mode, int Ci, int Co, int V);
 int fgx_conv_gather_gemm_weight(int dtype, int mode, const void* src, const void* weight, const void* bias,
