@@ -182,7 +182,19 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
                 nb = wanted < most ? wanted : most;
                 out->tile_rows = shapes[i].rows;
                 out->tile_cols = shapes[i].cols;
-                const bool fills = 2 * (size_t)V * tiles * nb >= 3 * (size_t)kCUs;
+                // How many items fill the chip: of 128 x 128 tiles a few more than CUs (324 items: 3 840 voxels, 256 -> 768 channels
+                // 0.050 ms, 64 x 64 tiles 0.083; 848 voxels 0.031 and 0.038), of the larger ones half as many again.
+                const bool square = shapes[i].rows == 128 && shapes[i].cols == 128;
+                bool fills = (size_t)V * tiles * nb >= (square ? (size_t)kCUs * 5 / 4 : (size_t)kCUs * 3 / 2);
+                if (square && !fills && n > 4096 && n <= 8192 && 10 * tiles * 4 <= (size_t)11 * cdiv(Co, 64) * cdiv(Ci, 64)) {
+                    // ... in blocks of 1024 rows before smaller tiles, where they pad no more than those (5 816 voxels, 256 channels
+                    // 0.051 -> 0.043 ms; 192 channels, padded to 256, 0.035 -> 0.045: not there)
+                    const size_t most_short = cdiv(n, (size_t)1024), nb_short = wanted < most_short ? wanted : most_short;
+                    if ((size_t)V * tiles * nb_short >= (size_t)kCUs * 5 / 4) {
+                        nb = nb_short;
+                        fills = true;
+                    }
+                }
                 if (last && !fills) {
                     // nothing fills the chip: blocks down to 1024 rows (64 channels, 3 840 voxels: 0.020 -> 0.016 ms), 2048 where
                     // the tile splits its pairs over the wavefronts itself or two short blocks would be all (1 976 voxels,
@@ -259,6 +271,9 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
     const size_t steps = (size_t)V * cdiv(row_bytes, (size_t)64);
     for (; s < (steps >= 160 ? 16 : 8); s *= 2) {
         size_t pieces = cols <= 32 ? 700 : kCUs;
+        // (128 x 128 tiles under a long K: two pieces for a CU rather than one and a half; 5 816 voxels, 256 channels in 4 splits 0.053 ms, in 8
+        // 0.048; 1 976 voxels, 256 -> 768 0.054 and 0.049; not from 1.6 on: 13 488 voxels, 192 -> 96 0.044 and 0.051)
+        if (out->tile_rows == 128 && out->tile_cols == 128 && steps >= 160) pieces = 400;
         if (out->tile_cols == 64 && (s < 4 ? steps >= 54 : (s < 8 && steps >= 320))) pieces = 450;
         if (tiles * s >= pieces) break;
     }
@@ -299,7 +314,8 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
         }
     }
     if (out->stream) return;
-    if (row_bytes >= 1024 && cols >= 128) {
+    // (not for a single tile of rows under a small weight: 192 voxels, 768 -> 256 channels 0.030 ms, 64 x 64 tiles 0.024)
+    if (row_bytes >= 1024 && cols >= 128 && !(n < 256 && (size_t)K * cols < (size_t)512 * 512)) {
         // Too few tiles to stream and rows of 1 KiB or more (512 channels of a 16-bit type): a few hundred or thousand voxels
         // under a weight of tens of megabytes.  The tiled kernel on 256 x 128 tiles and 128-byte slabs, with as many K
         // splits as give every CU one workgroup, keeps more of the weight in flight than 128 x 128 tiles on 64-byte slabs

@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("dtype, res, ci, co", [
     (torch.float32, 8, 24, 40), (torch.float32, 24, 320, 96), (torch.float32, 32, 33, 512), (torch.float32, 64, 96, 24), (torch.float32, 100, 7, 33),
     (torch.float16, 16, 80, 200), (torch.bfloat16, 16, 300, 136), (torch.float16, 32, 320, 16), (torch.bfloat16, 40, 40, 72),
-    (torch.float16, 48, 24, 384), (torch.bfloat16, 60, 128, 96), (torch.float16, 64, 264, 56), (torch.float16, 100, 48, 24), (torch.bfloat16, 100, 40, 200),
+    (torch.float16, 8, 768, 256), (torch.bfloat16, 32, 768, 256), (torch.float16, 40, 72, 512), (torch.bfloat16, 24, 256, 768), (torch.float16, 48, 24, 384), (torch.bfloat16, 60, 128, 96), (torch.float16, 64, 264, 56), (torch.float16, 100, 48, 24), (torch.bfloat16, 100, 40, 200),
 ])
 def test_rule_schedules_match_oracle(gpu_device, dtype, res, ci, co):
     coords = reference_test_shell(res)
