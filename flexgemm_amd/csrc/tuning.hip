@@ -272,8 +272,9 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
     for (; s < (steps >= 160 ? 16 : 8); s *= 2) {
         size_t pieces = cols <= 32 ? 700 : kCUs;
         // (128 x 128 tiles under a long K: two pieces for a CU rather than one and a half; 5 816 voxels, 256 channels in 4 splits 0.053 ms, in 8
-        // 0.048; 1 976 voxels, 256 -> 768 0.054 and 0.049; not from 1.6 on: 13 488 voxels, 192 -> 96 0.044 and 0.051)
-        if (out->tile_rows == 128 && out->tile_cols == 128 && steps >= 160) pieces = 400;
+        // 0.048; 1 976 voxels, 768 <- 256 0.054 and 0.049; not from 1.6 on: 13 488 voxels, 320 <- 96 0.062 and 0.067.  Input gradients
+        // alone: other splits round a forward sum differently, and a ReLU behind it then falls on its other side now and then)
+        if (pass_kind != 0 && out->tile_rows == 128 && out->tile_cols == 128 && steps >= 160) pieces = 400;
         if (out->tile_cols == 64 && (s < 4 ? steps >= 54 : (s < 8 && steps >= 320))) pieces = 450;
         if (tiles * s >= pieces) break;
     }
@@ -314,8 +315,8 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
         }
     }
     if (out->stream) return;
-    // (not for a single tile of rows under a small weight: 192 voxels, 768 -> 256 channels 0.030 ms, 64 x 64 tiles 0.024)
-    if (row_bytes >= 1024 && cols >= 128 && !(n < 256 && (size_t)K * cols < (size_t)512 * 512)) {
+    // (not for an input gradient of a single tile of rows under a small weight: 192 voxels, 256 <- 768 channels 0.029 ms, 64 x 64 tiles 0.023)
+    if (row_bytes >= 1024 && cols >= 128 && !(pass_kind != 0 && n < 256 && (size_t)K * cols < (size_t)512 * 512)) {
         // Too few tiles to stream and rows of 1 KiB or more (512 channels of a 16-bit type): a few hundred or thousand voxels
         // under a weight of tens of megabytes.  The tiled kernel on 256 x 128 tiles and 128-byte slabs, with as many K
         // splits as give every CU one workgroup, keeps more of the weight in flight than 128 x 128 tiles on 64-byte slabs
