@@ -566,7 +566,7 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
     const int64_t row_bytes = (int64_t)k * es;
     // a network's first layers: all offsets of a row in one product, no row order or tile tables
     if (n > 0 && !panel_kept.defined() && L.fgx_conv_gemm_stem_pays(code, mode, (size_t)n, k, cols, v) && !narrow_shape(c, es, k, cols, v, n) &&
-        schedules_are_ours() && aligned(src) && aligned(weight)) {
+        schedules_are_ours() && aligned(src) && aligned(weight) && aligned(nmap)) {
         const char* name = mode == 0 ? "gather_gemm_fwd" : "gather_gemm_dgrad";
         p.out = make({n, cols}, src.scalar_type(), dev);
         if (want_mask && activation == FGX_ACT_RELU) p.mask = make({n * cols / 8}, at::kByte, dev);
@@ -721,7 +721,8 @@ WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool 
         py::tuple got = impl_function("_narrow_wgrad")(grad, feats, c.obj, v, with_bias);
         w.weight = got[0].cast<Tensor>();
         if (with_bias) w.bias = got[1].cast<Tensor>();
-    } else if (L.fgx_wgrad_stem_pays(code, (size_t)n, ci, co, v) && n_in > 0 && schedules_are_ours() && aligned(feats) && aligned(grad)) {
+    } else if (L.fgx_wgrad_stem_pays(code, (size_t)n, ci, co, v) && n_in > 0 && schedules_are_ours() && aligned(feats) && aligned(grad) &&
+               aligned(c.need("neighbor_map"))) {
         const Tensor nmap = c.need("neighbor_map");
         Tensor scratch = workspace(L.fgx_wgrad_stem_scratch_bytes((size_t)n, ci, co), dev);
         w.weight = make({co, v, ci}, feats.scalar_type(), dev);

@@ -125,3 +125,31 @@ def test_products_against_the_sum_over_neighbors(gpu_device, n, k, cols, v, mode
     assert torch.equal(relu, got.clamp(min=0))
     on = (bits[:, None] >> torch.arange(8, device=gpu_device)) & 1
     assert torch.equal(on.bool().reshape(n, cols), relu > 0)
+
+
+def test_a_map_that_starts_between_16_byte_pieces(gpu_device):
+    """A hand-made cache whose neighbor map is a row slice of a larger one (rows of 108 bytes): dense, but not on a 16-byte
+    boundary, which these kernels' loads need.  The layer runs on the other kernels then."""
+    coords = torch.from_numpy(reference_test_shell(20)).to(gpu_device)
+    gen = torch.Generator(device=gpu_device).manual_seed(4)
+    n, ci, co = coords.shape[0], 8, 40
+    nmap = spconv.SubMConv3dFunction._compute_neighbor_cache(coords, torch.Size([1, ci, 20, 20, 20]), (3, 3, 3), (1, 1, 1), False).neighbor_map
+    larger = torch.zeros(n + 1, 27, dtype=torch.int32, device=gpu_device)
+    larger[1:] = nmap.view(torch.int32)
+    cache = spconv.SubMConv3dNeighborCache(neighbor_map=larger[1:].view(torch.uint32))
+    assert cache.neighbor_map.is_contiguous() and cache.neighbor_map.data_ptr() % 16
+    feats = torch.randn(n, ci, generator=gen, device=gpu_device).half().requires_grad_()
+    weight = (torch.randn(co, 3, 3, 3, ci, generator=gen, device=gpu_device) / 9).half().requires_grad_()
+    out, _ = spconv.sparse_submanifold_conv3d(feats, coords, torch.Size([1, ci, 20, 20, 20]), weight, None, cache)
+    up = torch.randn(out.shape, generator=gen, device=gpu_device).half()
+    gf, gw = torch.autograd.grad(out, (feats, weight), up)
+    m = nmap.cpu().to(torch.int64)
+    w = weight.detach().cpu().double().view(co, 27, ci)
+
+    def through(src, wt):           # [n, v, k] x [cols, v, k]
+        rows = torch.cat([src.detach().cpu().double(), torch.zeros(1, src.shape[1], dtype=torch.float64)])
+        return rows[torch.where(m == 0xFFFFFFFF, n, m)].reshape(n, -1) @ wt.reshape(wt.shape[0], -1).t()
+
+    want = (through(feats, w), through(up, w.flip(1).permute(2, 1, 0)), _pairs(nmap, feats.detach(), up)[0])
+    for got, ref in zip((out.detach(), gf, gw.view(co, 27, ci)), want):
+        assert (got.cpu().double() - ref).abs().max() <= 2.0 ** -11 * ref.abs().max() + 1e-3
