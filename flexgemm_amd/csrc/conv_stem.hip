@@ -80,6 +80,8 @@ __global__ void __launch_bounds__(kStemThreads)
 stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Tag::type* __restrict__ feats, const uint32_t* __restrict__ map,
                   uint32_t n, int V, int Co, unsigned steps_total, unsigned groups, float* __restrict__ partial) {
     using C = StemCfg<P>;
+    using T = typename Tag::type;
+    using T4 = T __attribute__((ext_vector_type(4)));
     constexpr int S = kStemStages;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     unsigned char* ring = lds;                                 // [S][features | grad_out]
@@ -105,10 +107,10 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
     const unsigned char* zero_b = g_zero_block_s;
     const unsigned long long map_bytes = (unsigned long long)n * V * 4;
 
-    auto issue_idx = [&](int j) {
+    auto issue_idx = [&](int j) __attribute__((always_inline)) {
         stem_issue_idx<P>(map, map_bytes, lo, nsteps, j, V, wave, lane, idx_ring + (j & (kStemIdxSlots - 1)) * C::IDX_SLOT, dump, zero_b);
     };
-    auto issue_rows_of = [&](int j, auto whole) {
+    auto issue_rows_of = [&](int j, auto whole) __attribute__((always_inline)) {
         constexpr bool WHOLE = decltype(whole)::value;
         unsigned char* stage = ring + (j % S) * C::STAGE;
         const uint32_t* words = (const uint32_t*)(idx_ring + (j & (kStemIdxSlots - 1)) * C::IDX_SLOT);
@@ -133,65 +135,100 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
             __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(dst), 16, 0, 0);
         }
     };
-    auto issue_rows = [&](int j) {
+    auto issue_rows = [&](int j) __attribute__((always_inline)) {
         if (j < nsteps && (unsigned long long)(lo + (unsigned)j + 1) * C::ROWS <= n) issue_rows_of(j, std::true_type{});
         else issue_rows_of(j, std::false_type{});
     };
 
     f32x16 acc[C::NT_PER];
+    // APART: rows of grad_out that are not finite are added pair by pair (wgrad_device.h).  424 000 voxels 8 -> 48 channels, with the
+    // reduction: all finite 0.081 ms as without the second run, one row in a thousand infinite 0.175, every value 1.1 (the
+    // sums that are not finite taken again over all rows, by the reduction: 8.2 and 8.8).
+    auto run = [&](auto apart_rows) __attribute__((always_inline)) {
+        constexpr bool APART = decltype(apart_rows)::value;
 #pragma unroll
-    for (int t = 0; t < C::NT_PER; ++t)
+        for (int t = 0; t < C::NT_PER; ++t)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
+            for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
 
 #pragma unroll
-    for (int j = 0; j < S - 1; ++j) issue_idx(j);
-    wait_vmcnt<0>();
-    __syncthreads();
+        for (int j = 0; j < S - 1; ++j) issue_idx(j);
+        wait_vmcnt<0>();
+        __syncthreads();
 #pragma unroll
-    for (int j = 0; j < S - 1; ++j) {
-        issue_rows(j);
-        issue_idx(j + S - 1);
-    }
+        for (int j = 0; j < S - 1; ++j) {
+            issue_rows(j);
+            issue_idx(j + S - 1);
+        }
 
-    constexpr int NK = C::ROWS / 16;
-    for (int k = 0; k < nsteps; ++k) {
-        wait_vmcnt<(S - 2) * C::LPS>();                        // rows of step k and the map words of step k + S - 1 have landed
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();                          // ... everybody's; the stage of step k - 1 is free
-        asm volatile("" ::: "memory");
-        issue_rows(k + S - 1);
-        issue_idx(k + 2 * (S - 1));
-        const unsigned char* f_cur = ring + (k % S) * C::STAGE;
-        const unsigned char* g_cur = f_cur + C::F_BYTES;
+        constexpr int NK = C::ROWS / 16;
+        for (int k = 0; k < nsteps; ++k) {
+            wait_vmcnt<(S - 2) * C::LPS>();                        // rows of step k and the map words of step k + S - 1 have landed
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();                          // ... everybody's; the stage of step k - 1 is free
+            asm volatile("" ::: "memory");
+            issue_rows(k + S - 1);
+            issue_idx(k + 2 * (S - 1));
+            const unsigned char* f_cur = ring + (k % S) * C::STAGE;
+            const unsigned char* g_cur = f_cur + C::F_BYTES;
 #pragma unroll
-        for (int kk = 0; kk < NK; ++kk) {
-            const int row = kk * 16 + g * 8 + (s16 >> 2);      // (see wgrad_gemm.hip on the transposing read)
-            i16x4 fr[2 * C::NT_PER + 4];                       // (two of them fill the last group of four)
-            {
-                const int byte = (wave_m * 32 + mb * 16 + (s16 & 3) * 4) * 2;
-                const unsigned char* at = g_cur + row * (kStemCols * 2) + (((byte >> 4) ^ C::key(row)) << 4) + (byte & 15);
-                fr[0] = lds_read_tr16(at);
-                fr[1] = lds_read_tr16(at + 4 * kStemCols * 2);
-            }
+            for (int kk = 0; kk < NK; ++kk) {
+                const int row = kk * 16 + g * 8 + (s16 >> 2);      // (see wgrad_gemm.hip on the transposing read)
+                i16x4 fr[2 * C::NT_PER + 4];                       // (two of them fill the last group of four)
+                {
+                    const int byte = (wave_m * 32 + mb * 16 + (s16 & 3) * 4) * 2;
+                    const unsigned char* at = g_cur + row * (kStemCols * 2) + (((byte >> 4) ^ C::key(row)) << 4) + (byte & 15);
+                    fr[0] = lds_read_tr16(at);
+                    fr[1] = lds_read_tr16(at + 4 * kStemCols * 2);
+                }
 #pragma unroll
-            for (int t = 0; t < C::NT_PER; ++t) {
-                const int tile = wave_n * C::NT_PER + t < C::NT ? wave_n * C::NT_PER + t : 0;
-                const unsigned char* at = f_cur + row * C::ROWB + (tile * 32 + mb * 16 + (s16 & 3) * 4) * 2;
-                fr[2 + 2 * t] = lds_read_tr16(at);
-                fr[3 + 2 * t] = lds_read_tr16(at + 4 * C::ROWB);
-            }
-            fr[2 + 2 * C::NT_PER] = fr[3 + 2 * C::NT_PER] = i16x4{0, 0, 0, 0};
-            lds_wait_all(fr);
-            const i16x8 af = __builtin_shufflevector(fr[0], fr[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                for (int t = 0; t < C::NT_PER; ++t) {
+                    const int tile = wave_n * C::NT_PER + t < C::NT ? wave_n * C::NT_PER + t : 0;
+                    const unsigned char* at = f_cur + row * C::ROWB + (tile * 32 + mb * 16 + (s16 & 3) * 4) * 2;
+                    fr[2 + 2 * t] = lds_read_tr16(at);
+                    fr[3 + 2 * t] = lds_read_tr16(at + 4 * C::ROWB);
+                }
+                fr[2 + 2 * C::NT_PER] = fr[3 + 2 * C::NT_PER] = i16x4{0, 0, 0, 0};
+                lds_wait_all(fr);
+                i16x8 af = __builtin_shufflevector(fr[0], fr[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                uint32_t apart = 0u;
+                if constexpr (APART) {
+                    apart = nonfinite_rows<Tag>(af);
+                    drop_rows(af, apart, g);
+                }
 #pragma unroll
-            for (int t = 0; t < C::NT_PER; ++t) {
-                const i16x8 bf = __builtin_shufflevector(fr[2 + 2 * t], fr[3 + 2 * t], 0, 1, 2, 3, 4, 5, 6, 7);
-                mma16<Tag>(acc[t], af, bf);
+                for (int t = 0; t < C::NT_PER; ++t) {
+                    i16x8 bf = __builtin_shufflevector(fr[2 + 2 * t], fr[3 + 2 * t], 0, 1, 2, 3, 4, 5, 6, 7);
+                    if constexpr (APART) drop_rows(bf, apart, g);
+                    mma16<Tag>(acc[t], af, bf);
+                }
+                while (APART && apart) {
+                    const int row = kk * 16 + __ffs((int)apart) - 1;
+                    apart &= apart - 1u;
+                    // (a row past the end is zeros and never comes here)
+                    const uint32_t* neighbors = map + ((unsigned long long)(lo + (unsigned)k) * C::ROWS + (unsigned)row) * (unsigned)V;
+                    T4 gv[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        gv[q] = *reinterpret_cast<const T4*>(g_cur + row * (kStemCols * 2) + (((wave_m * 4 + q) ^ C::key(row)) << 4) + g * 8);
+#pragma unroll
+                    for (int t = 0; t < C::NT_PER; ++t) {
+                        const int col = (wave_n * C::NT_PER + t) * 32 + l32, v = col / (8 * P);
+                        if (col >= C::N || (v < V ? neighbors[v] == FGX_EMPTY32 : col < C::N - 8)) continue;
+                        const float x = (float)*reinterpret_cast<const T*>(f_cur + row * C::ROWB + col * 2);
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) acc[t][e] += (float)gv[e >> 2][e & 3] * x;
+                    }
+                }
             }
         }
-    }
-    wait_vmcnt<0>();                                           // the loads of the steps past the end
+        wait_vmcnt<0>();                                           // the loads of the steps past the end
+    };
+    run(std::false_type{});
+    bool finite = true;
+#pragma unroll
+    for (int t = 0; t < C::NT_PER; ++t) finite = finite && all_finite(acc[t]);
+    if (__syncthreads_or(!finite)) run(std::true_type{});
 
     // partial[column tile][group][64][N]
     float* dst = partial + ((size_t)blockIdx.y * groups + group) * ((size_t)kStemCols * C::N);
@@ -208,12 +245,10 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
 }
 
 // grad_weight and grad_bias: 32 columns of blockDim.z rows of the product per workgroup, blockDim.y threads per element each adding
-// every blockDim.y-th partial product, their sums added in order.  An infinity or NaN in grad_out times the zeros of a missing neighbor is NaN where the
-// sum over the pairs has no such term: an element that comes out like that is summed again over its pairs alone.
+// every blockDim.y-th partial product, their sums added in order.
 template <typename T>
 __global__ void __launch_bounds__(1024) stem_reduce_kernel(const float* __restrict__ partial, unsigned groups, int V, int Ci, int Co, int N,
-                                                           const T* __restrict__ gout, const T* __restrict__ feats,
-                                                           const uint32_t* __restrict__ map, uint32_t n, T* __restrict__ gw, T* __restrict__ gb) {
+                                                           T* __restrict__ gw, T* __restrict__ gb) {
     __shared__ float sums[32][33];                             // [rows * slices][32]
     const int c = threadIdx.x, slices = blockDim.y, slice = threadIdx.y, at = threadIdx.z * slices;
     const int col = blockIdx.x * 32 + c, co = blockIdx.y * blockDim.z + threadIdx.z;
@@ -230,24 +265,6 @@ __global__ void __launch_bounds__(1024) stem_reduce_kernel(const float* __restri
     __syncthreads();
     float r = sums[at][c];
     for (int q = 1; q < slices; ++q) r += sums[at + q][c];
-    const bool again = co < Co && col < V * Ci && !(fabsf(r) < __builtin_inff());
-    if (__syncthreads_or(again)) {
-        __syncthreads();                                       // (the sums have been read)
-        s = 0.f;
-        if (again) {
-            const int v = col / Ci, ci = col - v * Ci;
-            for (size_t row = slice; row < n; row += slices) {
-                const uint32_t m = map[row * V + v];
-                if (m != FGX_EMPTY32) s += (float)gout[row * Co + co] * (float)feats[(size_t)m * Ci + ci];
-            }
-        }
-        sums[at + slice][c] = s;
-        __syncthreads();
-        if (again) {
-            r = sums[at][c];
-            for (int q = 1; q < slices; ++q) r += sums[at + q][c];
-        }
-    }
     if (slice != 0 || co >= Co) return;
     if (col < V * Ci) gw[(size_t)co * V * Ci + col] = from_float<T>(r);
     else if (gb != nullptr && col == N - 8) gb[co] = from_float<T>(r);
@@ -429,8 +446,7 @@ int stem_launch(const void* gout, const void* feats, const uint32_t* map, size_t
     unsigned slices = 1;
     while (slices < 32 && slices * 8 < groups) slices *= 2;
     const unsigned rows = slices >= 8 ? 1 : 8 / slices;
-    stem_reduce_kernel<T><<<dim3(C::N / 32, cdiv(Co, rows)), dim3(32, slices, rows), 0, s>>>(scratch, groups, V, 8 * P, Co, C::N, (const T*)gout, (const T*)feats, map, (uint32_t)n,
-                                                                 (T*)gw, (T*)gb);
+    stem_reduce_kernel<T><<<dim3(C::N / 32, cdiv(Co, rows)), dim3(32, slices, rows), 0, s>>>(scratch, groups, V, 8 * P, Co, C::N, (T*)gw, (T*)gb);
     FGX_CHECK_LAUNCH("fgx_conv_wgrad_stem(reduce)");
     return FGX_OK;
 }

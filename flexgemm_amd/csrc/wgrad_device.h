@@ -85,6 +85,35 @@ template <> __device__ __forceinline__ void mma16<BF16>(f32x16& acc, const i16x8
 }
 template <> __device__ __forceinline__ void mma16<F32>(f32x16&, const i16x8&, const i16x8&) {}
 
+// Rows of grad_out with an infinity or a NaN, for the kernels that multiply a missing neighbor as zeros: 0 * infinity is NaN
+// where the sum over the pairs has no such term.  A workgroup whose sums come out finite met none; one with a sum that is not goes
+// over its rows again, leaves such rows out of the matrix product and adds their pairs one by one.
+__device__ __forceinline__ bool all_finite(const f32x16& a) {
+    bool ok = true;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) ok = ok && fabsf(a[e]) < __builtin_inff();
+    return ok;
+}
+constexpr uint32_t exponent16(F16) { return 0x7C00u; }
+constexpr uint32_t exponent16(BF16) { return 0x7F80u; }
+// the rows of the wavefront's fragment (bit 8 * half + j: element j of a lane of that half) where some lane has one
+template <typename Tag>
+__device__ __forceinline__ uint32_t nonfinite_rows(const i16x8& f) {
+    constexpr uint32_t E = exponent16(Tag{});
+    uint32_t rows = 0u;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const unsigned long long have = __ballot(((uint32_t)(uint16_t)f[j] & E) == E);
+        rows |= ((have & 0xFFFFFFFFull) ? 1u : 0u) << j | ((have >> 32) ? 1u : 0u) << (8 + j);
+    }
+    return rows;
+}
+__device__ __forceinline__ void drop_rows(i16x8& f, uint32_t rows, int half) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        if ((rows >> (8 * half + j)) & 1u) f[j] = 0;
+}
+
 // eight ones in the 16-bit type, as a fragment
 template <typename Tag> __device__ __forceinline__ i16x8 ones16() {
     constexpr short one = sizeof(typename Tag::type) == 2 && __is_same(typename Tag::type, _Float16) ? (short)0x3C00 : (short)0x3F80;

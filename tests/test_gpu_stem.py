@@ -153,3 +153,50 @@ def test_a_map_that_starts_between_16_byte_pieces(gpu_device):
     want = (through(feats, w), through(up, w.flip(1).permute(2, 1, 0)), _pairs(nmap, feats.detach(), up)[0])
     for got, ref in zip((out.detach(), gf, gw.view(co, 27, ci)), want):
         assert (got.cpu().double() - ref).abs().max() <= 2.0 ** -11 * ref.abs().max() + 1e-3
+
+
+def _same_classes(got, want):
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got == float("inf"), want == float("inf"))
+    assert torch.equal(got == -float("inf"), want == -float("inf"))
+
+
+# rows with an infinity or NaN among the last of a step, alone in theirs, side by side, over an infinite or zero feature
+@pytest.mark.parametrize("ci,co,v,dtype", [(8, 16, 27, torch.float16), (8, 72, 17, torch.bfloat16), (16, 48, 27, torch.bfloat16),
+                                           (16, 136, 25, torch.float16)])
+def test_infinities_of_many_kinds_stay_with_their_pairs(gpu_device, ci, co, v, dtype):
+    print(f"[case] {ci}->{co} v={v} {dtype}", flush=True)
+    n = 20011
+    nmap, feats, grad = _case(gpu_device, n, ci, co, v, dtype, seed=5)
+    inf, nan = float("inf"), float("nan")
+    feats[100, 1], feats[101, 2], feats[102, 3] = inf, -inf, 0.0
+    m = nmap.view(torch.int32)
+    m[64, 3], m[65, 4], m[66, 5], m[70, 3] = 100, 101, 102, 102
+    grad[64, 0], grad[65, 1], grad[66, 2], grad[70, 3], grad[n - 1, 4], grad[n - 2, 4], grad[63, 5], grad[5000, 6] = inf, inf, -inf, nan, inf, -inf, -inf, inf
+    grad[200:264, 7] = inf
+    want_w, want_b = _pairs(nmap, feats, grad)
+    gw, gb = _run(nmap, feats, grad)
+    for got, want in ((gw.cpu().double(), want_w), (gb.cpu().double(), want_b)):
+        _same_classes(got, want)
+        ok = want.isfinite()
+        # one rounding to the type, sums as in test_against_the_sum_over_pairs
+        assert (got - want)[ok].abs().max() <= 2.0 ** (-11 if dtype == torch.float16 else -8) * want[ok].abs().max() + n ** 0.5 * 2.0 ** -21
+
+
+def test_a_step_that_overflows_everywhere_takes_no_longer(gpu_device):
+    """Every element of the gradient infinite, as a step of mixed-precision training with too large a loss scale leaves it."""
+    nmap, feats, grad = _case(gpu_device, 200003, 8, 48, 27, torch.bfloat16)
+
+    def fastest(g):
+        best = float("inf")
+        for _ in range(4):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            _run(nmap, feats, g)
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        return best
+
+    usual, overflown = fastest(grad), fastest(torch.full_like(grad, float("inf")))
+    print(f"[case] {usual:.3f} ms, overflown {overflown:.3f} ms", flush=True)
+    assert overflown < 20 * usual
