@@ -14,7 +14,8 @@
 //           more in scan order at 400 000 voxels, where four times as many words are set.)
 //           Map rows are walked in cell order when the voxels come in no order of their own.
 // A voxel given several times is found under its smallest row number, and voxels outside the grid are not found; the `bits`
-// form lists the rows that lost their cell behind the others, so that its walk visits every row once.
+// form lists the rows that lost their cell behind the others (in row order where the walk is the caller's), so that its walk
+// visits every row once.
 //
 // Against the hash table (hash_build.hip) a question is one or two reads of a few neighboring lines instead of a probe at a
 // pseudo-random place; against sort and merge (neighbor_sorted.hip) nothing is sorted.
@@ -44,7 +45,7 @@ struct GridIndexLayout {
     bool dense;
     size_t cells;                   // B * W * H * D
     size_t blocks, tiles;           // `bits` form: 128-bit blocks, tiles of the count
-    size_t bits, counts, state, rows, total;        // byte offsets; [bits, state + state bytes) is cleared to 0, rows to EMPTY
+    size_t bits, counts, state, losers, rows, total;        // byte offsets; [bits, losers + its bytes) is cleared to 0, rows to EMPTY
     size_t zero_bytes;
     uint32_t shift;                 // as in GridIndex
 };

@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(256) set_bits_kernel(const int32_t* __restrict
 __device__ __forceinline__ uint32_t state_load(const uint32_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void state_store(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
-// Sum of the tiles before `tile`, by one whole wavefront; the tile's own sum is made known to the tiles after it first, the
+// Single-pass prefix sums with decoupled look-back (Merrill and Garland, 2016): sum of the tiles before `tile`, by one whole wavefront; the tile's own sum is made known to the tiles after it first, the
 // running total last.  A word says what it holds (kLookbackSum / kLookbackTotal) in the bits above its value, so one relaxed
 // load is enough.  Tiles are numbered in the order their workgroups started (a ticket), so every tile waited for is running.
 __device__ __forceinline__ uint32_t lookback(uint32_t* state, unsigned tile, uint32_t sum) {
@@ -165,7 +165,8 @@ __global__ void __launch_bounds__(kCountThreads) count_bits_kernel(const ulonglo
     }
 }
 
-// rows[rank of the voxel's cell] = the smallest row of that cell; the rows that lose (and those outside the grid) from the end
+// rows[rank of the voxel's cell] = the smallest row of that cell.  losers (optional): the rows that lose (and those outside the grid)
+// from the end, in no fixed order
 __global__ void __launch_bounds__(256) place_rows_kernel(const int32_t* __restrict__ coords, size_t n, GridIndex g, uint32_t* __restrict__ rows,
                                                          uint32_t* __restrict__ losers) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -183,7 +184,51 @@ __global__ void __launch_bounds__(256) place_rows_kernel(const int32_t* __restri
         loser = had == FGX_EMPTY32 ? FGX_EMPTY32 : (had > (uint32_t)i ? had : (uint32_t)i);
     }
     // every row but the cell's smallest loses exactly once, so these places and the ranks together are the n rows
-    if (loser != FGX_EMPTY32) rows[n - 1 - atomicAdd(losers, 1u)] = loser;
+    if (losers != nullptr && loser != FGX_EMPTY32) rows[n - 1 - atomicAdd(losers, 1u)] = loser;
+}
+
+// The rows that lost their cell (and those outside the grid) behind the others in row order: a walk that outlives the build is the
+// chunks and the summation order of the narrow layers, and has to be a function of the coordinates.  One pass, tiles of rows by
+// decoupled look-back; nobody loses in most builds, and then it is a launch that returns at once.
+constexpr int kLoserThreads = 512, kLoserRows = 8;                  // rows per thread
+__global__ void __launch_bounds__(kLoserThreads) list_losers_kernel(const int32_t* __restrict__ coords, size_t n, GridIndex g, uint32_t* __restrict__ state,
+                                                                    uint32_t* rows) {
+    if ((size_t)g.order[0] == n) return;
+    __shared__ uint32_t wave_sum[kLoserThreads / 64];
+    __shared__ uint32_t tile_lds, before_lds;
+    if (threadIdx.x == 0) tile_lds = atomicAdd(&state[gridDim.x], 1u);
+    __syncthreads();
+    const unsigned tile = tile_lds;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const size_t base = ((size_t)tile * (kLoserThreads / 64) + wave) * (64 * kLoserRows) + lane;       // a wavefront's rows are consecutive
+    unsigned long long loses[kLoserRows];
+    uint32_t mine = 0u;
+#pragma unroll
+    for (int r = 0; r < kLoserRows; ++r) {
+        const size_t i = base + (size_t)r * 64;
+        const int4 c = i < n ? reinterpret_cast<const int4*>(coords)[i] : make_int4(-1, 0, 0, 0);
+        const bool in = in_grid(g, c.x, c.y, c.z, c.w);
+        const bool kept = in && grid_find<false>(g, grid_place<false>(g, c.x, c.y, c.z, c.w)) == (uint32_t)i;
+        loses[r] = __ballot(i < n && !kept);
+        mine += (uint32_t)__popcll(loses[r]);
+    }
+    if (lane == 0) wave_sum[wave] = mine;
+    __syncthreads();
+    if (wave == 0) {
+        uint32_t sum = 0u;
+#pragma unroll
+        for (int w = 0; w < kLoserThreads / 64; ++w) sum += wave_sum[w];
+        const uint32_t before = lookback(state, tile, sum);
+        if (lane == 0) before_lds = before;
+    }
+    __syncthreads();
+    size_t at = (size_t)g.order[0] + before_lds;
+    for (int w = 0; w < wave; ++w) at += wave_sum[w];
+#pragma unroll
+    for (int r = 0; r < kLoserRows; ++r) {
+        if ((loses[r] >> lane) & 1ull) rows[at + (size_t)__popcll(loses[r] & ((1ull << lane) - 1ull))] = (uint32_t)(base + (size_t)r * 64);
+        at += (size_t)__popcll(loses[r]);
+    }
 }
 
 enum { kSubm = 0, kConvFwd = 1, kConvBwd = 2 };
@@ -599,6 +644,8 @@ bool bits_layout(size_t n_rows, int B, int W, int H, int D, bool in_order, GridI
     off = align_up(off + L.blocks * 16, 256);
     L.state = off;
     off = align_up(off + (L.tiles + 4) * 4, 256);       // the tiles' words, the ticket, the number of losers, GridIndex::order
+    L.losers = off;
+    off = align_up(off + ((size_t)cdiv(n_rows, kLoserThreads * kLoserRows) + 1) * 4, 256);          // ... and of the tiles of rows, their ticket
     L.zero_bytes = off;
     L.counts = off;
     off = align_up(off + L.blocks * 4, 256);
@@ -615,7 +662,7 @@ bool grid_index_plan(size_t n, int B, int W, int H, int D, GridIndexLayout* out)
     GridIndexLayout L{};
     if (!bits_layout(n, B, W, H, D, false, &L)) return false;
     if (L.cells <= kDenseMaxCells) {
-        L = GridIndexLayout{true, L.cells, 0, 0, 0, 0, 0, 0, align_up(L.cells * 4, 256), 0, 0};
+        L = GridIndexLayout{true, L.cells, 0, 0, 0, 0, 0, 0, 0, align_up(L.cells * 4, 256), 0, 0};
     }
     *out = L;
     return true;
@@ -662,8 +709,12 @@ int grid_index_build(const int32_t* coords, size_t n, int B, int W, int H, int D
         g.bits = (const ulonglong2*)(ws + L.bits);
         g.counts = (const uint32_t*)(ws + L.counts);
         g.rows = rows;
-        if (n) place_rows_kernel<<<grid, 256, 0, s>>>(coords, n, g, rows, (uint32_t*)(ws + L.state) + L.tiles + 1);
+        if (n) place_rows_kernel<<<grid, 256, 0, s>>>(coords, n, g, rows, walk != nullptr ? nullptr : (uint32_t*)(ws + L.state) + L.tiles + 1);
         FGX_CHECK_LAUNCH(what);
+        if (n && walk != nullptr) {
+            list_losers_kernel<<<cdiv(n, kLoserThreads * kLoserRows), kLoserThreads, 0, s>>>(coords, n, g, (uint32_t*)(ws + L.losers), rows);
+            FGX_CHECK_LAUNCH(what);
+        }
     }
     *out = g;
     return FGX_OK;

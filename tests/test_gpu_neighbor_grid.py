@@ -142,3 +142,29 @@ def test_narrow_layer_on_a_fresh_grid_cache(gpu_device, res, order, twice):
     ref_gi, ref_gw, _ = eg.backward(grad.double(), feats.double(), nmap, weight.double())
     for got, ref in ((out, eg.forward(feats.double(), nmap, weight.double())), (f.grad, ref_gi), (w.grad, ref_gw)):
         assert eg.max_rel_err(got.detach().cpu(), ref) < 1e-2
+
+
+# voxels given several times and voxels outside the grid have no cell of their own: they follow the others in row order, so that
+# every build of the same coordinates gives the same walk (and with it the same chunks and sums of the narrow layers)
+@pytest.mark.parametrize("twice,outside", [(0, 0), (1, 0), (0, 3), (5000, 700), (34000, 0)])
+def test_walk_is_a_function_of_the_coordinates(gpu_device, twice, outside):
+    res = 230
+    _say(f"walk order twice={twice} outside={outside}")
+    rng = np.random.default_rng(twice + outside)
+    base = reference_test_shell(96) + np.array([0, 50, 3, 101], np.int32)
+    coords = np.concatenate([base, base[rng.integers(0, len(base), twice)], base[:outside]])
+    coords[len(coords) - outside:, 1 + rng.integers(0, 3)] += rng.choice(np.array([-res, res], np.int32), outside)
+    coords = np.ascontiguousarray(coords[rng.permutation(len(coords))])
+    n = len(coords)
+    dev = torch.from_numpy(coords).to(gpu_device)
+    shape = torch.Size([1, 0, res, res, res])
+    walks = [_np(SubMConv3dFunction._compute_neighbor_cache(dev, shape, (3, 3, 3), (1, 1, 1), False)["_cell_walk"]) for _ in range(4)]
+    inside = ((coords >= 0) & (coords < np.array([1, res, res, res]))).all(1)
+    first = {}
+    for i in np.nonzero(inside)[0]:
+        first.setdefault(tuple(coords[i]), i)
+    losers = np.setdiff1d(np.arange(n), np.fromiter(first.values(), np.int64))
+    assert np.array_equal(np.sort(walks[0]), np.arange(n))
+    assert np.array_equal(walks[0][n - len(losers):], losers)
+    for walk in walks[1:]:
+        assert np.array_equal(walk, walks[0])
