@@ -519,10 +519,12 @@ int fgx_conv_wgrad_stem(int dtype, const void* grad_out, const void* feats, cons
 // Forward, ms (the tiled kernel, this one): 424 000 voxels 6 -> 48 channels 0.090 and 0.066; 143 616 voxels 8 -> 128 0.049 and 0.025, 16 ->
 // 128 0.050 and 0.038; 15 192 voxels 8 -> 64 0.019 and 0.008; 192 voxels 0.010 and 0.007; level at 624 264 voxels 16 -> 64.  An input gradient
 // fetches its fragments of the weight one value at a time: 3 us more per launch, and the streaming kernel keeps 16 channels of
-// many voxels up to 64 columns (143 616 voxels 0.040 and 0.047; 96 columns 0.052 and 0.048).
+// many voxels up to 64 columns (143 616 voxels 0.040 and 0.047; 96 columns 0.052 and 0.048).  Forward, 16 channels, up to 32 columns (general
+// kernels, this one): 98 408 voxels 0.028 and 0.026, 427 872 0.085 and 0.087, 2 667 120 0.425 and 0.504.
 int fgx_conv_gemm_stem_pays(int dtype, int mode, size_t n, int K, int cols, int V) {
     if (mode < 0 || mode > 2 || !stem_gemm_takes(dtype, n, K, cols, V)) return 0;
-    return mode == 0 || (K == 8 ? n >= 768 : n >= 3072 && cols >= 96);
+    if (mode == 0) return K == 8 || cols > 32 || n < 262144;
+    return K == 8 ? n >= 768 : n >= 3072 && cols >= 96;
 }
 
 int fgx_conv_gemm_stem(int dtype, int mode, const void* src, const void* weight, const void* bias, const uint32_t* map, size_t n, int Ci, int Co,

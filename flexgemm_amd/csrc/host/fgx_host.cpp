@@ -564,9 +564,15 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
     if (bias.defined()) bias = bias.contiguous();
     const int co = (int)weight.size(0), ci = (int)weight.size(2), k = mode == 0 ? ci : co;
     const int64_t row_bytes = (int64_t)k * es;
+    const int pass = mode == 0 ? 0 : 1;
     // a network's first layers: all offsets of a row in one product, no row order or tile tables
-    if (n > 0 && !panel_kept.defined() && L.fgx_conv_gemm_stem_pays(code, mode, (size_t)n, k, cols, v) && !narrow_shape(c, es, k, cols, v, n) &&
-        schedules_are_ours() && aligned(src) && aligned(weight) && aligned(nmap)) {
+    const bool stem = n > 0 && !panel_kept.defined() && L.fgx_conv_gemm_stem_pays(code, mode, (size_t)n, k, cols, v) && schedules_are_ours() &&
+                      aligned(src) && aligned(weight) && aligned(nmap);
+    // Up to 32 channels on both sides: the resident-row kernel where it runs at once or the cache has earned its plan (38 720 voxels, 8 ->
+    // 32 channels: 0.014 ms, 0.010 without; 98 408 voxels 0.015 and 0.016, 427 872 voxels 0.033 and 0.046, 16 -> 32 0.034 and 0.087).
+    const bool narrow = n > 0 && narrow_shape(c, es, k, cols, v, n) &&
+                        impl_function("_narrow_applies")(c.obj, src, k, cols, v, n, n_src, python_schedule(pass, src, n, ci, co, v)).cast<bool>();
+    if (stem && !narrow) {
         const char* name = mode == 0 ? "gather_gemm_fwd" : "gather_gemm_dgrad";
         p.out = make({n, cols}, src.scalar_type(), dev);
         if (want_mask && activation == FGX_ACT_RELU) p.mask = make({n * cols / 8}, at::kByte, dev);
@@ -577,7 +583,6 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
         return p;
     }
     if (masked && !(c.has("gray_code") && c.has("sorted_idx"))) c.obj.attr("_ensure_sorted")();
-    const int pass = mode == 0 ? 0 : 1;
     const Sched s = schedule(pass, src, n, ci, co, v);
     bool own_order = false;
     if (masked && row_bytes <= module_int(g_impl, "LOCALITY_MAX_ROW_BYTES") && (c.has("_tile_order") || n >= module_int(g_impl, "LOCALITY_MIN_ROWS")) &&
@@ -592,8 +597,6 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
     // the streaming kernel addresses its operands with 32-bit byte offsets
     const double most = (double)0xFF000000u;
     const bool streams = s.stream && (double)n_src * row_bytes <= most && (double)n * 8 <= most && (double)n * 27 * 4 * 2 <= most;
-    const bool narrow = narrow_shape(c, es, k, cols, v, n) &&
-                        impl_function("_narrow_applies")(c.obj, src, k, cols, v, n, n_src, python_schedule(pass, src, n, ci, co, v)).cast<bool>();
     Tensor panel = panel_kept;
     // the tiled kernel reads the weight itself where it can
     const bool direct = !panel.defined() && !narrow && !streams && aligned(weight) && L.fgx_conv_gather_gemm_weight_pays(code, mode, ci, co, v);

@@ -200,3 +200,26 @@ def test_a_step_that_overflows_everywhere_takes_no_longer(gpu_device):
     usual, overflown = fastest(grad), fastest(torch.full_like(grad, float("inf")))
     print(f"[case] {usual:.3f} ms, overflown {overflown:.3f} ms", flush=True)
     assert overflown < 20 * usual
+
+
+# a first layer with up to 32 columns and more rows than the resident-row kernel asks for: grids that have no cell order, and the
+# generic convolution, whose cache has no coordinates, take these kernels at once (nothing of a tile schedule is made)
+@pytest.mark.parametrize("generic", [False, True])
+@pytest.mark.parametrize("ci,co", [(8, 32), (16, 24)])
+def test_narrow_first_layers_without_a_cell_order(gpu_device, generic, ci, co):
+    res = 100 if generic else 160
+    coords = torch.from_numpy(reference_test_shell(res)).to(gpu_device)
+    gen = torch.Generator(device=gpu_device).manual_seed(6)
+    feats = torch.randn(coords.shape[0], ci, generator=gen, device=gpu_device).half()
+    weight = (torch.randn(co, 3, 3, 3, ci, generator=gen, device=gpu_device) / 9).half()
+    shape = torch.Size([1, ci, res, res, res])
+    with torch.no_grad():
+        if generic:
+            out, _, cache = spconv.sparse_conv3d(feats, coords, shape, weight, None, padding=(1, 1, 1))
+        else:
+            out, cache = spconv.sparse_submanifold_conv3d(feats, coords, shape, weight)
+    assert out.shape[0] >= 32768 and not any(k.startswith(("_plan_", "_mask_code_", "_narrow_plan_buf")) for k in vars(cache))
+    m = cache.neighbor_map[::97].cpu().to(torch.int64)
+    rows = torch.cat([feats.cpu().double(), torch.zeros(1, ci, dtype=torch.float64)])
+    want = rows[torch.where(m == 0xFFFFFFFF, len(feats), m)].reshape(len(m), -1) @ weight.cpu().double().reshape(co, -1).t()
+    assert ((out[::97].cpu().double() - want).abs() <= 2.0 ** -11 * want.abs() + 1e-4).all()
