@@ -368,7 +368,7 @@ bool deal_items(const std::string& plan_key, int64_t tiles, int col_tiles, int g
         const bool few_rounds = items <= module_int(g_impl, "ITEM_ORDER_ANY_ROW_MAX_ROUNDS") * groups;
         mode = (slabs >= 4 || few_rounds) && plan_key.rfind("_plan_t_", 0) != 0 ? "balanced" : "default";
     }
-    if (mode == "default" || items <= module_int(g_impl, "ITEM_ORDER_MIN_ROUNDS") * groups || groups > 1024 || items >= (1 << 26)) return false;
+    if (mode == "default" || items <= module_int(g_impl, "ITEM_ORDER_MIN_ROUNDS") * groups || groups > 1024 || items >= 0x7FFFFFFF) return false;
     if (mode != "balanced") throw py::value_error("unknown GEMM_ITEM_ORDER '" + mode + "'; expected 'auto', 'balanced' or 'default'");
     return true;
 }

@@ -336,19 +336,19 @@ __global__ void __launch_bounds__(kPairThreads) pair_fill_kernel(const uint32_t*
     }
 }
 
-// One wavefront per tile: OR of gray[sorted_idx[r]] over the tile's rows.
+// One wavefront per tile and turn: OR of gray[sorted_idx[r]] over the tile's rows.
 __global__ void __launch_bounds__(kBlock) tile_or_kernel(const int32_t* __restrict__ gray,
                                                          const int64_t* __restrict__ sorted_idx, size_t n, int block,
                                                          size_t num_tiles, int32_t* __restrict__ tile_code) {
-    const size_t tile = ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
     const int lane = threadIdx.x & 63;
-    if (tile >= num_tiles) return;   // whole wavefronts leave together
-    const size_t lo = tile * (size_t)block;
-    const size_t hi = lo + (size_t)block < n ? lo + (size_t)block : n;
-    uint32_t code = 0;
-    for (size_t r = lo + lane; r < hi; r += 64) code |= (uint32_t)gray[sorted_idx[r]];
-    for (int off = 32; off > 0; off >>= 1) code |= (uint32_t)__shfl_xor((int)code, off, 64);
-    if (lane == 0) tile_code[tile] = (int32_t)code;
+    for (size_t tile = ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 6; tile < num_tiles; tile += (size_t)gridDim.x * (kBlock / 64)) {
+        const size_t lo = tile * (size_t)block;
+        const size_t hi = lo + (size_t)block < n ? lo + (size_t)block : n;
+        uint32_t code = 0;
+        for (size_t r = lo + lane; r < hi; r += 64) code |= (uint32_t)gray[sorted_idx[r]];
+        for (int off = 32; off > 0; off >>= 1) code |= (uint32_t)__shfl_xor((int)code, off, 64);
+        if (lane == 0) tile_code[tile] = (int32_t)code;
+    }
 }
 
 __global__ void set_i32_kernel(int32_t* dst, int32_t value) {
@@ -462,6 +462,9 @@ constexpr unsigned kOrderInLds = 8192;  // items whose sorted list stays in LDS
 
 __device__ __forceinline__ unsigned tile_cost_bin(uint32_t code) { return 32u - (unsigned)__popc(code); }   // 0 = most expensive
 
+// A sorted item carries its cost above 26 bits of its number; WIDE: more items than that, whose cost is looked up again.
+constexpr unsigned kItemBits = 26;
+template <bool WIDE>
 __device__ void order_items(const int32_t* __restrict__ tile_code, unsigned num_tiles, unsigned col_tiles, unsigned slabs, unsigned groups,
                             uint32_t* __restrict__ sorted, uint32_t* __restrict__ item_at) {
     __shared__ uint32_t count[kOrderWaves][64];
@@ -509,7 +512,7 @@ __device__ void order_items(const int32_t* __restrict__ tile_code, unsigned num_
             count[wave][bin] = first + (uint32_t)__popcll(peers);
         }
         first = (uint32_t)__shfl((int)first, leader, 64);
-        if (live) sorted[first + (uint32_t)__popcll(peers & below)] = bin << 26 | (i0 + lane);      // (the item, its cost above it)
+        if (live) sorted[first + (uint32_t)__popcll(peers & below)] = WIDE ? i0 + lane : bin << kItemBits | (i0 + lane);
     }
     __threadfence_block();
     __syncthreads();
@@ -518,8 +521,9 @@ __device__ void order_items(const int32_t* __restrict__ tile_code, unsigned num_
     const unsigned rounds = total / groups, rem = total % groups;
     unsigned scale = 0;
     while ((((unsigned long long)(rounds + 1) * (32u * slabs + 3u)) >> scale) >= (1ull << 21)) ++scale;
+    auto item_of = [](uint32_t entry) -> uint32_t { return WIDE ? entry : entry & ((1u << kItemBits) - 1u); };
     auto cost_of = [&](uint32_t entry) -> uint32_t {
-        const unsigned pc = 32u - (entry >> 26);
+        const unsigned pc = 32u - (WIDE ? bin_of(entry) : entry >> kItemBits);
         return ((pc ? pc : 1u) * slabs + 3u) >> scale;
     };
     // P threads per slot share the counting
@@ -528,7 +532,7 @@ __device__ void order_items(const int32_t* __restrict__ tile_code, unsigned num_
     uint32_t mine = slot;
     if (slot < rem) {                                             // cheapest items: the positions of the last round
         const uint32_t entry = sorted[total - rem + slot];
-        if (part == 0) item_at[rounds * groups + slot] = entry & 0x3FFFFFFu;
+        if (part == 0) item_at[rounds * groups + slot] = item_of(entry);
         mine += cost_of(entry) << 10;
     }
     const unsigned quads = (groups + 3u) / 4u;
@@ -546,11 +550,28 @@ __device__ void order_items(const int32_t* __restrict__ tile_code, unsigned num_
         if (P >= 4) rank += (unsigned)__shfl_xor((int)rank, 2, 64);
         if (slot < groups) {
             const uint32_t entry = sorted[r * groups + rank];     // rank 0 = least loaded slot <- most expensive item
-            if (part == 0) item_at[r * groups + slot] = entry & 0x3FFFFFFu;
+            if (part == 0) item_at[r * groups + slot] = item_of(entry);
             mine += cost_of(entry) << 10;
         }
         __syncthreads();
     }
+}
+
+struct TilePrefix {
+    uint32_t at, plan_at;           // offsets, gather-plan rows
+};
+// sums of `mine` over the threads before this one, and (*all) over the workgroup's
+__device__ __forceinline__ TilePrefix tile_prefix(const TilePrefix& mine, uint32_t (*part)[kOrderWaves], TilePrefix* all) {
+    TilePrefix before;
+    before.at = block_exclusive_sum<kOrderWaves>(mine.at, part[0], &all->at);
+    before.plan_at = block_exclusive_sum<kOrderWaves>(mine.plan_at, part[1], &all->plan_at);
+    return before;
+}
+
+// (a tile without any offset has one plan row, all rows missing: every tile owns at least one step of the GEMM)
+__device__ __forceinline__ TilePrefix tile_counts(const int32_t* __restrict__ tile_code, unsigned t, unsigned num_tiles) {
+    const uint32_t c = t < num_tiles ? (uint32_t)__popc((uint32_t)tile_code[t]) : 0u;
+    return TilePrefix{c, t < num_tiles && c == 0u ? 1u : c};
 }
 
 // seg (optional): exclusive offsets of the tiles' public offset lists, plan_seg (optional): of their gather-plan rows, both with
@@ -559,32 +580,96 @@ __global__ void __launch_bounds__(kOrderThreads) tile_tables_kernel(const int32_
                                                                     int32_t* __restrict__ seg, int32_t* __restrict__ plan_seg,
                                                                     unsigned col_tiles, unsigned slabs, unsigned groups,
                                                                     uint32_t* __restrict__ sorted, uint32_t* __restrict__ item_at) {
-    __shared__ uint32_t part[kOrderWaves];
+    __shared__ uint32_t part[2][kOrderWaves];
     __shared__ uint32_t sorted_lds[kOrderInLds];
-    uint32_t at = 0u, plan_at = 0u;
     if (seg != nullptr || plan_seg != nullptr) {
+        TilePrefix run{0u, 0u}, all;
         for (unsigned t0 = 0; t0 < num_tiles; t0 += kOrderThreads) {         // (uniform)
             const unsigned t = t0 + threadIdx.x;
-            const uint32_t c = t < num_tiles ? (uint32_t)__popc((uint32_t)tile_code[t]) : 0u;
-            uint32_t all;
-            const uint32_t before = block_exclusive_sum<kOrderWaves>(c, part, &all);
-            // a tile without any offset has one plan row (all rows missing): every tile owns at least one step of the GEMM
-            uint32_t bare_all;
-            const uint32_t bare = block_exclusive_sum<kOrderWaves>(t < num_tiles && c == 0u ? 1u : 0u, part, &bare_all);
+            const TilePrefix before = tile_prefix(tile_counts(tile_code, t, num_tiles), part, &all);
             if (t < num_tiles) {
-                if (seg != nullptr) seg[t] = (int32_t)(at + before);
-                if (plan_seg != nullptr) plan_seg[t] = (int32_t)(plan_at + before + bare);
+                if (seg != nullptr) seg[t] = (int32_t)(run.at + before.at);
+                if (plan_seg != nullptr) plan_seg[t] = (int32_t)(run.plan_at + before.plan_at);
             }
-            at += all;
-            plan_at += all + bare_all;
+            run.at += all.at;
+            run.plan_at += all.plan_at;
         }
         if (threadIdx.x == 0) {
-            if (seg != nullptr) seg[num_tiles] = (int32_t)at;
-            if (plan_seg != nullptr) plan_seg[num_tiles] = (int32_t)plan_at;
+            if (seg != nullptr) seg[num_tiles] = (int32_t)run.at;
+            if (plan_seg != nullptr) plan_seg[num_tiles] = (int32_t)run.plan_at;
         }
     }
-    if (item_at != nullptr)
-        order_items(tile_code, num_tiles, col_tiles, slabs, groups, num_tiles * col_tiles <= kOrderInLds ? sorted_lds : sorted, item_at);
+    if (item_at == nullptr) return;
+    if ((unsigned long long)num_tiles * col_tiles < (1ull << kItemBits))
+        order_items<false>(tile_code, num_tiles, col_tiles, slabs, groups, num_tiles * col_tiles <= kOrderInLds ? sorted_lds : sorted, item_at);
+    else
+        order_items<true>(tile_code, num_tiles, col_tiles, slabs, groups, sorted, item_at);
+}
+
+// The segment tables of many tiles, in chunks: a chunk's sums are left in its last entries of the tables, one workgroup adds them up
+// there, and every chunk then writes its own entries from what it finds there.  One workgroup for all tiles takes
+// 1.45 us per 1024 of them (8 192 tiles 13.1 us, 10 419 17.6, 83 350 120, 2 667 120 4 079); the chunks' three launches take 13.3 us for
+// 10 419, 14.7 for 83 350, 32 for 2 667 120.
+constexpr unsigned kOneScanTiles = 8192, kScanChunk = 4096;
+
+__global__ void __launch_bounds__(kOrderThreads) tile_sums_kernel(const int32_t* __restrict__ tile_code, unsigned num_tiles, int32_t* seg,
+                                                                  int32_t* plan_seg) {
+    __shared__ uint32_t part[2][kOrderWaves];
+    const unsigned t0 = blockIdx.x * kScanChunk, last = (num_tiles - t0 < kScanChunk ? num_tiles : t0 + kScanChunk) - 1u;
+    TilePrefix mine{0u, 0u}, all;
+#pragma unroll
+    for (unsigned r = 0; r < kScanChunk; r += kOrderThreads) {
+        const TilePrefix c = tile_counts(tile_code, t0 + r + threadIdx.x, num_tiles);
+        mine.at += c.at;
+        mine.plan_at += c.plan_at;
+    }
+    tile_prefix(mine, part, &all);
+    if (threadIdx.x == 0) {
+        if (seg != nullptr) seg[last] = (int32_t)all.at;
+        if (plan_seg != nullptr) plan_seg[last] = (int32_t)all.plan_at;
+    }
+}
+
+__global__ void __launch_bounds__(kOrderThreads) chunk_scan_kernel(unsigned num_tiles, unsigned chunks, int32_t* seg,
+                                                                   int32_t* plan_seg) {
+    __shared__ uint32_t part[2][kOrderWaves];
+    TilePrefix run{0u, 0u};
+    for (unsigned b0 = 0; b0 < chunks; b0 += kOrderThreads) {                // (uniform)
+        const unsigned b = b0 + threadIdx.x;
+        const unsigned last = b + 1 < chunks ? (b + 1) * kScanChunk - 1u : num_tiles - 1u;
+        TilePrefix mine{0u, 0u}, all;
+        if (b < chunks && seg != nullptr) mine.at = (uint32_t)seg[last];
+        if (b < chunks && plan_seg != nullptr) mine.plan_at = (uint32_t)plan_seg[last];
+        const TilePrefix before = tile_prefix(mine, part, &all);
+        if (b < chunks && seg != nullptr) seg[last] = (int32_t)(run.at + before.at);
+        if (b < chunks && plan_seg != nullptr) plan_seg[last] = (int32_t)(run.plan_at + before.plan_at);
+        run.at += all.at;
+        run.plan_at += all.plan_at;
+    }
+    if (threadIdx.x == 0) {
+        if (seg != nullptr) seg[num_tiles] = (int32_t)run.at;
+        if (plan_seg != nullptr) plan_seg[num_tiles] = (int32_t)run.plan_at;
+    }
+}
+
+__global__ void __launch_bounds__(kOrderThreads) chunk_tables_kernel(const int32_t* __restrict__ tile_code, unsigned num_tiles, int32_t* seg,
+                                                                     int32_t* plan_seg) {
+    __shared__ uint32_t part[2][kOrderWaves];
+    const unsigned t0 = blockIdx.x * kScanChunk, last = (num_tiles - t0 < kScanChunk ? num_tiles : t0 + kScanChunk) - 1u;
+    TilePrefix run{seg != nullptr ? (uint32_t)seg[last] : 0u, plan_seg != nullptr ? (uint32_t)plan_seg[last] : 0u};
+#pragma unroll
+    for (unsigned r = 0; r < kScanChunk; r += kOrderThreads) {
+        const unsigned t = t0 + r + threadIdx.x;
+        const TilePrefix c = tile_counts(tile_code, t, num_tiles);
+        TilePrefix all;
+        const TilePrefix before = tile_prefix(c, part, &all);               // (its barriers: the chunk's sum has been read)
+        if (t < num_tiles) {
+            if (seg != nullptr) seg[t] = (int32_t)(run.at + before.at);
+            if (plan_seg != nullptr) plan_seg[t] = (int32_t)(run.plan_at + before.plan_at);
+        }
+        run.at += all.at;
+        run.plan_at += all.plan_at;
+    }
 }
 
 struct PairLayout {
@@ -839,7 +924,7 @@ int fgx_tile_plan(const int32_t* gray, const int64_t* order, const uint32_t* map
     FGX_CHECK_ARG(tile_rows >= 1 && V >= 1 && V <= 32, "fgx_tile_plan: bad shape tile_rows=%d V=%d", tile_rows, V);
     hipStream_t s = (hipStream_t)stream;
     const size_t num_tiles = (n + tile_rows - 1) / tile_rows;
-    FGX_CHECK_ARG(num_tiles <= 0x3FFFFFFu, "fgx_tile_plan: too many tiles");
+    FGX_CHECK_ARG(num_tiles <= 0x7FFFFFFFu, "fgx_tile_plan: too many tiles");
     PhaseEnd phases{s};
     phase_mark("tile tables", s);
     if (n == 0) {
@@ -854,15 +939,25 @@ int fgx_tile_plan(const int32_t* gray, const int64_t* order, const uint32_t* map
     if (item_at != nullptr) {
         FGX_CHECK_ARG(col_tiles >= 1 && slabs >= 1 && groups >= 1 && groups <= kOrderThreads && item_ws != nullptr,
                       "fgx_tile_plan: bad item order col_tiles=%d slabs=%d groups=%d", col_tiles, slabs, groups);
-        FGX_CHECK_ARG(num_tiles * (size_t)col_tiles < ((size_t)1 << 26), "fgx_tile_plan: too many items");
+        FGX_CHECK_ARG(num_tiles * (size_t)col_tiles < 0x7FFFFFFFull, "fgx_tile_plan: too many items");
     }
     if (!have_codes) {
-        tile_or_kernel<<<cdiv(num_tiles * 64, kBlock), kBlock, 0, s>>>(gray, order, n, tile_rows, num_tiles, tile_code);
+        const size_t groups_or = cdiv(num_tiles, (size_t)(kBlock / 64)), most = (size_t)0xFFFFFFFFu / kBlock;       // (of one launch)
+        tile_or_kernel<<<(unsigned)(groups_or < most ? groups_or : most), kBlock, 0, s>>>(gray, order, n, tile_rows, num_tiles, tile_code);
         FGX_CHECK_LAUNCH("fgx_tile_plan(or)");
     }
-    if (seg != nullptr || plan_seg != nullptr || item_at != nullptr) {
-        tile_tables_kernel<<<1, kOrderThreads, 0, s>>>(tile_code, (unsigned)num_tiles, seg, plan_seg, (unsigned)col_tiles, (unsigned)slabs,
-                                                       (unsigned)groups, item_ws, item_at);
+    bool scans = seg != nullptr || plan_seg != nullptr;
+    if (scans && num_tiles > kOneScanTiles) {
+        const unsigned chunks = cdiv(num_tiles, kScanChunk);
+        tile_sums_kernel<<<chunks, kOrderThreads, 0, s>>>(tile_code, (unsigned)num_tiles, seg, plan_seg);
+        chunk_scan_kernel<<<1, kOrderThreads, 0, s>>>((unsigned)num_tiles, chunks, seg, plan_seg);
+        chunk_tables_kernel<<<chunks, kOrderThreads, 0, s>>>(tile_code, (unsigned)num_tiles, seg, plan_seg);
+        FGX_CHECK_LAUNCH("fgx_tile_plan(chunks)");
+        scans = false;
+    }
+    if (scans || item_at != nullptr) {
+        tile_tables_kernel<<<1, kOrderThreads, 0, s>>>(tile_code, (unsigned)num_tiles, scans ? seg : nullptr, scans ? plan_seg : nullptr,
+                                                       (unsigned)col_tiles, (unsigned)slabs, (unsigned)groups, item_ws, item_at);
         FGX_CHECK_LAUNCH("fgx_tile_plan(tables)");
     }
     if (plan_idx != nullptr) {
@@ -920,7 +1015,7 @@ int fgx_gather_item_order(const int32_t* tile_code, size_t num_tiles, int col_ti
                   groups);
     const size_t total = num_tiles * (size_t)col_tiles;
     if (total == 0) return FGX_OK;
-    FGX_CHECK_ARG(total < ((size_t)1 << 26), "fgx_gather_item_order: too many items");
+    FGX_CHECK_ARG(total < 0x7FFFFFFFull, "fgx_gather_item_order: too many items");
     FGX_CHECK_ARG(tile_code && workspace && item_at, "fgx_gather_item_order: null buffer");
     FGX_CHECK_ARG(workspace_bytes >= fgx_gather_item_order_workspace_bytes(num_tiles, col_tiles),
                   "fgx_gather_item_order: workspace of %zu bytes is too small", workspace_bytes);
