@@ -94,6 +94,14 @@ __device__ __forceinline__ bool all_finite(const f32x16& a) {
     for (int e = 0; e < 16; ++e) ok = ok && fabsf(a[e]) < __builtin_inff();
     return ok;
 }
+// whether nothing that is added changes the sum any more: NaN in every element with a column below `cols` and a row below `rows`
+// (element e of lane l: row first_row + 8 * (e / 4) + 4 * (l / 32) + e % 4, column first_col + l % 32)
+__device__ __forceinline__ bool all_nan(const f32x16& a, int lane, int first_row, int rows, int first_col, int cols) {
+    bool nan = true;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) nan = nan && (a[e] != a[e] || first_row + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3) >= rows);
+    return nan || first_col + (lane & 31) >= cols;
+}
 constexpr uint32_t exponent16(F16) { return 0x7C00u; }
 constexpr uint32_t exponent16(BF16) { return 0x7F80u; }
 // the rows of the wavefront's fragment (bit 8 * half + j: element j of a lane of that half) where some lane has one

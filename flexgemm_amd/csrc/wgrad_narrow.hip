@@ -15,6 +15,10 @@
 // chunks of the workgroup; offsets from V on multiply zeros) and walks the chunk's 128 rows in eight k-steps of 16; the
 // grad_out fragment of a k-step is read once for the eight offsets.  At the end every workgroup writes its partial
 // products, and a second kernel adds them in workgroup order (fixed order: same bits on every run).
+// An infinity or NaN in grad_out times the row of zeros is NaN where the sum over the pairs has no term: a workgroup whose sums are not
+// all finite goes over its chunks again and adds such rows of grad_out pair by pair, until every sum is NaN (wgrad_device.h).  2.67 M
+// voxels, 32 channels: all finite 0.240 ms (0.236 without the second pass), one row in a thousand infinite 0.75, every value 0.95; most
+// where no sum ends as NaN, 6.1.
 // A plan with an overflowing chunk (more distinct sources than slots) is not for this kernel: the caller looks at the
 // plan's header and takes the block-major kernel then.
 #include "wgrad_device.h"
@@ -27,7 +31,7 @@ constexpr int kNwMult = 4, kNwLoad = 4, kNwThreads = 64 * (kNwMult + kNwLoad);
 constexpr int kNwTaps = 8;                                                       // offsets per multiplier
 constexpr int kNwGoutBytes = kNarrowRows * 64;                                   // the chunk's grad_out rows
 constexpr int kNwBufferBytes = kNarrowRowBufPad + kNwGoutBytes + kNarrowTableBytes;
-constexpr size_t kNwLdsBytes = 2 * (size_t)kNwBufferBytes;
+constexpr size_t kNwLdsBytes = 2 * (size_t)kNwBufferBytes + 16;                  // ... and the word that asks for a second pass
 constexpr int kNwSrcGroups = kNarrowSlots / 16 / kNwLoad;                        // 7 wave-wide row loads per loader
 constexpr int kNwOutGroups = kNarrowRows / 16 / kNwLoad;                         // 2
 constexpr int kNwIds = kNwSrcGroups + kNwOutGroups;
@@ -37,10 +41,14 @@ __global__ void __launch_bounds__(kNwThreads)
 narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Tag::type* __restrict__ feats,
                     const unsigned char* __restrict__ plan, uint32_t chunks, uint32_t plan_bytes, uint32_t gout_bytes,
                     uint32_t feats_bytes, int V, int Ci, int Co, float* __restrict__ partial) {
+    using T = typename Tag::type;
+    using T4 = T __attribute__((ext_vector_type(4)));
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    volatile uint32_t& again = *reinterpret_cast<volatile uint32_t*>(lds + 2 * kNwBufferBytes);       // some sum is not finite
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool loader = wave >= kNwMult;
+    if (tid == 0) again = 0u;
     const int src_row_bytes = Ci * 2, out_row_bytes = Co * 2;
 
     // chunks of this workgroup: XCD x owns the x-th eighth, its workgroups interleave
@@ -114,93 +122,138 @@ narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename 
     // The two roles run loops of their own (with the same number of barriers): the multipliers' accumulators then take
     // no registers from the loaders and the other way round.
     if (loader) {
-        if (first < range_hi) {
-            fetch_ids(first);
-            enqueue(first, 0);
-            if (first + per_round < range_hi) fetch_ids(first + per_round);
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-            int b = 0;
-            for (unsigned chunk = first; chunk < range_hi; chunk += per_round, b ^= 1) {
-                const unsigned next = chunk + per_round;
-                const bool enqueues = next < range_hi, fetches = next + per_round < range_hi;
-                if (enqueues) {
-                    enqueue(next, b ^ 1);
-                    if (fetches) fetch_ids(next + per_round);
-                }
-                if (fetches) wait_vmcnt<kNwIds>();
-                else wait_vmcnt<0>();
+        for (int pass = 0; pass < 2; ++pass) {
+            if (first < range_hi) {
+                fetch_ids(first);
+                enqueue(first, 0);
+                if (first + per_round < range_hi) fetch_ids(first + per_round);
+                __builtin_amdgcn_s_waitcnt(0);
                 __syncthreads();
+                int b = 0;
+                for (unsigned chunk = first; chunk < range_hi; chunk += per_round, b ^= 1) {
+                    const unsigned next = chunk + per_round;
+                    const bool enqueues = next < range_hi, fetches = next + per_round < range_hi;
+                    if (enqueues) {
+                        enqueue(next, b ^ 1);
+                        if (fetches) fetch_ids(next + per_round);
+                    }
+                    if (fetches) wait_vmcnt<kNwIds>();
+                    else wait_vmcnt<0>();
+                    __syncthreads();
+                }
             }
+            if (pass == 0) __syncthreads();
+            if (again == 0u) break;
         }
         return;
     }
     f32x16 acc[kNwTaps];
+    auto run = [&](auto apart_rows) __attribute__((always_inline)) {
+        constexpr bool APART = decltype(apart_rows)::value;
 #pragma unroll
-    for (int t = 0; t < kNwTaps; ++t)
+        for (int t = 0; t < kNwTaps; ++t)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
-    if (first < range_hi) {
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        int b = 0;
-        for (unsigned chunk = first; chunk < range_hi; chunk += per_round, b ^= 1) {
-            const unsigned char* buf = lds + (size_t)b * kNwBufferBytes;
-            const unsigned char* gbuf = buf + kNarrowRowBufPad;
-            const unsigned char* table = gbuf + kNwGoutBytes;
-            // grad_out rows sit in the slots of their chunk row numbers: row r = kk * 16 + g * 8 + q (+ 4) has the
-            // piece key (g * 2 (+ 1)) & 3, whatever kk
-            const uint32_t g_lo = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)gbuf +
-                                  (uint32_t)((g * 8 + q) * 64) + ((cpiece ^ (uint32_t)((g * 2) & 3)) << 4) + cw;
-            const uint32_t g_hi = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)gbuf +
-                                  (uint32_t)((g * 8 + q + 4) * 64) + ((cpiece ^ (uint32_t)((g * 2 + 1) & 3)) << 4) + cw;
-            const uint32_t row_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)buf + cw;
-#pragma unroll 1
-            for (int kk = 0; kk < kNarrowRows / 16; ++kk) {
-                // the table entries of this lane's two rows for the wavefront's eight offsets: 16 bytes each
-                const int r0 = kk * 16 + g * 8 + q;
-                const u32x4 e_lo = *reinterpret_cast<const u32x4*>(table + r0 * (kNarrowTableStride * 2) + mw * 16);
-                const u32x4 e_hi = *reinterpret_cast<const u32x4*>(table + (r0 + 4) * (kNarrowTableStride * 2) + mw * 16);
-                i16x4 gfr[2], ffr[16];                                       // grad_out (lo, hi); eight offsets (lo, hi)
-                gfr[0] = lds_read_tr16_at<0>(g_lo + (uint32_t)(kk * 16 * 64));
-                gfr[1] = lds_read_tr16_at<0>(g_hi + (uint32_t)(kk * 16 * 64));
-                auto at = [&](const u32x4& e, int t) -> uint32_t {
-                    const uint32_t word = e[t >> 1];
-                    const uint32_t off = (t & 1) ? word >> 16 : word & 0xFFFFu;
-                    return row_base + (off ^ (cpiece << 4));
-                };
-#pragma unroll
-                for (int t = 0; t < 6; ++t) {                                // (at most 15 reads are counted in flight)
-                    ffr[t * 2] = lds_read_tr16_at<0>(at(e_lo, t));
-                    ffr[t * 2 + 1] = lds_read_tr16_at<0>(at(e_hi, t));
-                }
-                // every fragment register is tied to the wait: the compiler must not touch one before it
-                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(gfr[0]), "+v"(gfr[1]));
-                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[0]), "+v"(ffr[1]), "+v"(ffr[2]), "+v"(ffr[3]));
-                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[4]), "+v"(ffr[5]), "+v"(ffr[6]), "+v"(ffr[7]));
-                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[8]), "+v"(ffr[9]), "+v"(ffr[10]), "+v"(ffr[11]));
-#pragma unroll
-                for (int t = 6; t < 8; ++t) {
-                    ffr[t * 2] = lds_read_tr16_at<0>(at(e_lo, t));
-                    ffr[t * 2 + 1] = lds_read_tr16_at<0>(at(e_hi, t));
-                }
-                const i16x8 gf = __builtin_shufflevector(gfr[0], gfr[1], 0, 1, 2, 3, 4, 5, 6, 7);
-#pragma unroll
-                for (int t = 0; t < 6; ++t) {
-                    const i16x8 ff = __builtin_shufflevector(ffr[t * 2], ffr[t * 2 + 1], 0, 1, 2, 3, 4, 5, 6, 7);
-                    mma16<Tag>(acc[t], gf, ff);
-                }
-                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[12]), "+v"(ffr[13]), "+v"(ffr[14]), "+v"(ffr[15]));
-#pragma unroll
-                for (int t = 6; t < 8; ++t) {
-                    const i16x8 ff = __builtin_shufflevector(ffr[t * 2], ffr[t * 2 + 1], 0, 1, 2, 3, 4, 5, 6, 7);
-                    mma16<Tag>(acc[t], gf, ff);
-                }
-            }
+            for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
+        if (first < range_hi) {
             __builtin_amdgcn_s_waitcnt(0);
             __syncthreads();
+            int b = 0;
+            bool done = false;                                                   // (second pass) every sum is NaN
+            for (unsigned chunk = first; chunk < range_hi; chunk += per_round, b ^= 1) {
+                const unsigned char* buf = lds + (size_t)b * kNwBufferBytes;
+                const unsigned char* gbuf = buf + kNarrowRowBufPad;
+                const unsigned char* table = gbuf + kNwGoutBytes;
+                // grad_out rows sit in the slots of their chunk row numbers: row r = kk * 16 + g * 8 + q (+ 4) has the
+                // piece key (g * 2 (+ 1)) & 3, whatever kk
+                const uint32_t g_lo = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)gbuf +
+                                      (uint32_t)((g * 8 + q) * 64) + ((cpiece ^ (uint32_t)((g * 2) & 3)) << 4) + cw;
+                const uint32_t g_hi = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)gbuf +
+                                      (uint32_t)((g * 8 + q + 4) * 64) + ((cpiece ^ (uint32_t)((g * 2 + 1) & 3)) << 4) + cw;
+                const uint32_t row_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)buf + cw;
+#pragma unroll 1
+                for (int kk = 0; kk < kNarrowRows / 16 && !done; ++kk) {
+                    // the table entries of this lane's two rows for the wavefront's eight offsets: 16 bytes each
+                    const int r0 = kk * 16 + g * 8 + q;
+                    const u32x4 e_lo = *reinterpret_cast<const u32x4*>(table + r0 * (kNarrowTableStride * 2) + mw * 16);
+                    const u32x4 e_hi = *reinterpret_cast<const u32x4*>(table + (r0 + 4) * (kNarrowTableStride * 2) + mw * 16);
+                    i16x4 gfr[2], ffr[16];                                       // grad_out (lo, hi); eight offsets (lo, hi)
+                    gfr[0] = lds_read_tr16_at<0>(g_lo + (uint32_t)(kk * 16 * 64));
+                    gfr[1] = lds_read_tr16_at<0>(g_hi + (uint32_t)(kk * 16 * 64));
+                    auto entry = [](const u32x4& e, int t) -> uint32_t { return (t & 1) ? e[t >> 1] >> 16 : e[t >> 1] & 0xFFFFu; };
+                    auto at = [&](const u32x4& e, int t) -> uint32_t { return row_base + (entry(e, t) ^ (cpiece << 4)); };
+#pragma unroll
+                    for (int t = 0; t < 6; ++t) {                                // (at most 15 reads are counted in flight)
+                        ffr[t * 2] = lds_read_tr16_at<0>(at(e_lo, t));
+                        ffr[t * 2 + 1] = lds_read_tr16_at<0>(at(e_hi, t));
+                    }
+                    // every fragment register is tied to the wait: the compiler must not touch one before it
+                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(gfr[0]), "+v"(gfr[1]));
+                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[0]), "+v"(ffr[1]), "+v"(ffr[2]), "+v"(ffr[3]));
+                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[4]), "+v"(ffr[5]), "+v"(ffr[6]), "+v"(ffr[7]));
+                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[8]), "+v"(ffr[9]), "+v"(ffr[10]), "+v"(ffr[11]));
+#pragma unroll
+                    for (int t = 6; t < 8; ++t) {
+                        ffr[t * 2] = lds_read_tr16_at<0>(at(e_lo, t));
+                        ffr[t * 2 + 1] = lds_read_tr16_at<0>(at(e_hi, t));
+                    }
+                    i16x8 gf = __builtin_shufflevector(gfr[0], gfr[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                    uint32_t apart = 0u;
+                    if constexpr (APART) {
+                        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[12]), "+v"(ffr[13]), "+v"(ffr[14]), "+v"(ffr[15]));
+                        apart = nonfinite_rows<Tag>(gf);
+                        if (apart) drop_rows(gf, apart, g);
+                    }
+#pragma unroll
+                    for (int t = 0; t < 6; ++t) {
+                        i16x8 ff = __builtin_shufflevector(ffr[t * 2], ffr[t * 2 + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+                        if (APART && apart) drop_rows(ff, apart, g);
+                        mma16<Tag>(acc[t], gf, ff);
+                    }
+                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[12]), "+v"(ffr[13]), "+v"(ffr[14]), "+v"(ffr[15]));
+#pragma unroll
+                    for (int t = 6; t < 8; ++t) {
+                        i16x8 ff = __builtin_shufflevector(ffr[t * 2], ffr[t * 2 + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+                        if (APART && apart) drop_rows(ff, apart, g);
+                        mma16<Tag>(acc[t], gf, ff);
+                    }
+                    while (APART && apart) {
+                        const int r = kk * 16 + __ffs((int)apart) - 1;
+                        apart &= apart - 1u;
+                        T4 gv[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            gv[e] = *reinterpret_cast<const T4*>(gbuf + r * 64 + (((uint32_t)e ^ narrow_piece_key((uint32_t)r)) << 4) + g * 8);
+                        const u32x4 entries = *reinterpret_cast<const u32x4*>(table + r * (kNarrowTableStride * 2) + mw * 16);
+                        T x[kNwTaps];                                            // (all reads in flight together; a missing neighbor's: zeros)
+#pragma unroll
+                        for (int t = 0; t < kNwTaps; ++t)
+                            x[t] = *reinterpret_cast<const T*>(buf + (entry(entries, t) ^ ((uint32_t)((lane & 31) >> 3) << 4)) + (lane & 7) * 2);
+#pragma unroll
+                        for (int t = 0; t < kNwTaps; ++t) {
+                            if (__builtin_amdgcn_readfirstlane((int)entry(entries, t)) >> 6 == (int)kNarrowZeroSlot) continue;
+#pragma unroll
+                            for (int e = 0; e < 16; ++e) acc[t][e] += (float)gv[e >> 2][e & 3] * (float)x[t];
+                        }
+                    }
+                }
+                if constexpr (APART) {
+                    bool nan = true;
+#pragma unroll
+                    for (int t = 0; t < kNwTaps; ++t) nan = nan && (mw * kNwTaps + t >= V || all_nan(acc[t], lane, 0, Co, 0, Ci));
+                    done = __all(nan);
+                }
+                __builtin_amdgcn_s_waitcnt(0);
+                __syncthreads();
+            }
         }
-    }
+    };
+    run(std::false_type{});
+    bool finite = true;
+#pragma unroll
+    for (int t = 0; t < kNwTaps; ++t) finite = finite && (mw * kNwTaps + t >= V || all_finite(acc[t]));
+    if (__any(!finite) && lane == 0) again = 1u;
+    __syncthreads();                                                             // (the loaders' after their first pass)
+    if (again != 0u) run(std::true_type{});
     // partial[workgroup][v][co][ci] (32 x 32 per offset): accumulator element e of lane (l32, g) is co = (e >> 2) * 8 +
     // g * 4 + (e & 3), ci = l32
     {

@@ -168,3 +168,35 @@ def test_walk_is_a_function_of_the_coordinates(gpu_device, twice, outside):
     assert np.array_equal(walks[0][n - len(losers):], losers)
     for walk in walks[1:]:
         assert np.array_equal(walk, walks[0])
+
+
+# an infinity or NaN in the upstream gradient reaches the weight gradient through its own pairs alone, not as its product with the
+# zeros that stand for a missing neighbor
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("ci,co", [(16, 16), (24, 32)])
+def test_narrow_weight_gradient_with_infinities(gpu_device, dtype, ci, co):
+    _say(f"narrow weight gradient with infinities {ci}->{co} {dtype}")
+    res = 210
+    coords = torch.from_numpy(reference_test_shell(96) + np.array([0, 50, 3, 101], np.int32)).to(gpu_device)
+    n, inf = len(coords), float("inf")
+    gen = torch.Generator(device=gpu_device).manual_seed(ci)
+    feats = torch.randn(n, ci, generator=gen, device=gpu_device).to(dtype)
+    feats[500, 1], feats[501, 2], feats[502, 3] = inf, -inf, 0.0
+    weight = torch.randn(co, 3, 3, 3, ci, generator=gen, device=gpu_device).to(dtype).requires_grad_()
+    bias = torch.randn(co, generator=gen, device=gpu_device).to(dtype).requires_grad_()
+    out, cache = sparse_submanifold_conv3d(feats, coords, torch.Size([1, ci, res, res, res]), weight, bias)
+    up = torch.randn(n, co, generator=gen, device=gpu_device).to(dtype)
+    up[500, 0], up[501, 1], up[502, 2], up[3000, 3], up[n - 1, 4], up[n - 2, 4] = inf, -inf, inf, float("nan"), inf, -inf
+    up[7000:7300, 5] = -inf
+    gw, gb = torch.autograd.grad(out, (weight, bias), up)
+    assert cache["_narrow_overflows"] == 0
+    m, f, g = cache.neighbor_map.cpu().to(torch.int64), feats.cpu().double(), up.cpu().double()
+    want = []
+    for v in range(27):
+        rows = (m[:, v] != 0xFFFFFFFF).nonzero()[:, 0]
+        want.append(g[rows].t() @ f[m[rows, v]])
+    for got, ref in ((gw.detach().cpu().double().view(co, 27, ci), torch.stack(want, 1)), (gb.detach().cpu().double(), g.sum(0))):
+        assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got == inf, ref == inf) and torch.equal(got == -inf, ref == -inf)
+        ok = ref.isfinite()
+        # one rounding to the type of fp32 sums over n rows (random signs: their error grows with the root)
+        assert ok.any() and (got - ref)[ok].abs().max() <= 2.0 ** (-11 if dtype == torch.float16 else -8) * ref[ok].abs().max() + n ** 0.5 * 2.0 ** -21
