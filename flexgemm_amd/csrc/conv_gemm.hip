@@ -31,6 +31,7 @@
 #include <atomic>
 
 #include "gemm_device.h"
+#include "lds_read.h"
 
 namespace fgx {
 namespace {
@@ -134,23 +135,6 @@ struct BOperand {
     int lines;
     int ends_inside;        // the last K-slab may end inside a line (a panel is padded to whole slabs)
 };
-
-using i16x4 = short __attribute__((ext_vector_type(4)));
-// Transposing LDS read: in a group of 16 lanes, lane s names 4 adjacent columns of K row s / 4 and receives 4 K values of column s.
-// Inline assembly, because the compiler would drain the loads into LDS in front of its builtin; lds_wait ties the results to
-// the wait.
-__device__ __forceinline__ i16x4 lds_read_tr16(const unsigned char* p) {
-    const uint32_t addr = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)p;
-    i16x4 r;
-    asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(r) : "v"(addr));
-    return r;
-}
-template <int N>
-__device__ __forceinline__ void lds_wait(i16x4 (&r)[N]) {
-    static_assert(N % 4 == 0, "results come in fours");
-#pragma unroll
-    for (int i = 0; i < N; i += 4) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[i]), "+v"(r[i + 1]), "+v"(r[i + 2]), "+v"(r[i + 3]));
-}
 
 template <typename Tag, int BM, int BN, int WAVES_M, int WAVES_N, int S, int CH>
 struct GemmCfg {
@@ -431,7 +415,7 @@ gather_gemm_kernel(const typename Tag::type* __restrict__ src, BOperand b,
             }
         }
         if constexpr (TR) {
-            lds_wait(tr);
+            lds_wait_all(tr);
 #pragma unroll
             for (int kk = 0; kk < kChunks / 2; ++kk)
 #pragma unroll

@@ -703,6 +703,14 @@ Tensor wgrad_item_lists(const Cache& c, const Tensor& bounds, size_t n, int v, i
     return lists;
 }
 
+// What fgx_conv_wgrad_sweep accepts (the checks of the C entry point): it multiplies row numbers with 24-bit multiplies and addresses
+// both operands and the pair lists with 32-bit byte offsets.
+bool sweep_fits(int64_t n, int64_t n_in, int64_t ci, int64_t co, int es, int64_t pairs) {
+    const double most = (double)0xFF000000u;
+    return n > 0 && n <= (1 << 24) && n_in <= (1 << 24) && pairs > 0 && (double)n * co * es <= most && (double)n_in * ci * es <= most &&
+           (double)pairs * 4 + 256 <= most;
+}
+
 struct WeightGrads {
     Tensor weight, bias;
 };
@@ -742,15 +750,9 @@ WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool 
         if (pairs > std::min(sig_i.numel(), sig_o.numel()))
             throw py::value_error("valid_signal_seg does not fit the pair lists (V + 1 entries, the last one their length)");
         Sched s = schedule(2, feats, n, ci, co, v);
-        if (s.stream == 2) {
-            // (the checks of the C entry point: 24-bit row numbers, operands and lists within its 32-bit byte offsets)
-            const double most = (double)0xFF000000u;
-            const bool fits = n > 0 && n <= (1 << 24) && n_in <= (1 << 24) && pairs > 0 && (double)n * co * es <= most &&
-                              (double)n_in * ci * es <= most && (double)pairs * 4 + 256 <= most;
-            if (!fits) {                                // very long operands (and empty pair lists) take the block-major kernel
-                s.stream = 1;
-                s.block_rows = 12288;
-            }
+        if (s.stream == 2 && !sweep_fits(n, n_in, ci, co, es, pairs)) {      // very long operands (and empty pair lists) take the block-major kernel
+            s.stream = 1;
+            s.block_rows = 12288;
         }
         w.weight = make({co, v, ci}, feats.scalar_type(), dev);
         if (with_bias) w.bias = make({co}, feats.scalar_type(), dev);
@@ -876,7 +878,6 @@ struct ConvBackward : public torch::autograd::Node {
         if (has_bias) (void)bias.unpack();
         const at::NoGradGuard no_grad;
         const py::gil_scoped_acquire gil;
-        if (cache.obj == nullptr) throw std::runtime_error("Trying to backward through the graph a second time");
         const Cache c(py::reinterpret_borrow<py::object>(cache.obj));
         const int64_t stream = stream_of(f);
         Tensor grad = grads[0];
@@ -1035,6 +1036,7 @@ PYBIND11_MODULE(fgx_host, m) {
     m.def("convolve", &convolve);
     m.def("gather_gemm", &gather_gemm);
     m.def("wgrad", &wgrad);
+    m.def("sweep_fits", &sweep_fits);
     m.def("relu_mask_apply", [](const Tensor& grad, const Tensor& mask) { return relu_mask_apply(grad, mask, stream_of(grad)); });
     m.def("colsum", [](const Tensor& grad) { return colsum(grad, stream_of(grad)); });
     m.def("encode", &encode);

@@ -1,9 +1,10 @@
-// Device-side pieces shared by the weight-gradient kernels (wgrad_gemm.hip, wgrad_sweep.hip): vector types, the
-// transposing LDS read with its hand-placed waits, the MFMA wrappers, buffer resources.
+// Device-side pieces shared by the weight-gradient kernels (wgrad_gemm.hip, wgrad_sweep.hip, wgrad_narrow.hip, conv_stem.hip): vector
+// types, the MFMA wrappers, buffer resources, rows that are not finite.
 #pragma once
 #include <type_traits>
 
 #include "fgx_common.h"
+#include "lds_read.h"
 
 namespace fgx {
 namespace {
@@ -12,7 +13,6 @@ using f16x8 = _Float16 __attribute__((ext_vector_type(8)));
 using bf16x8 = __bf16 __attribute__((ext_vector_type(8)));
 using f32x16 = float __attribute__((ext_vector_type(16)));
 using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
-using i16x4 = short __attribute__((ext_vector_type(4)));
 using i16x8 = short __attribute__((ext_vector_type(8)));
 
 struct F16 { using type = _Float16; };
@@ -49,32 +49,6 @@ __device__ __forceinline__ void wait_vmcnt() {
 struct SegTable {
     uint32_t seg[kMaxV + 1];   // pair offsets per kernel offset
 };
-
-// Transposing LDS read, issued as inline assembly: through the compiler builtin every such read is preceded by a
-// conservative s_waitcnt vmcnt(0) (the compiler cannot tell it apart from the LDS areas the in-flight direct-to-LDS
-// loads are filling), which would drain the whole ring each step.  The price is that the result must be waited
-// for by hand: lds_wait_all() below ties the fragment registers to an s_waitcnt lgkmcnt(0).
-__device__ __forceinline__ i16x4 lds_read_tr16(const unsigned char* p) {
-    const uint32_t addr = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)p;
-    i16x4 r;
-    asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(r) : "v"(addr));
-    return r;
-}
-// the same with the address given as an LDS byte address plus a constant that goes into the instruction's offset field
-template <int OFFSET>
-__device__ __forceinline__ i16x4 lds_read_tr16_at(uint32_t addr) {
-    static_assert(OFFSET >= 0 && OFFSET < 65536, "the offset field is 16 bits wide");
-    i16x4 r;
-    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(r) : "v"(addr), "n"(OFFSET));
-    return r;
-}
-template <int N>
-__device__ __forceinline__ void lds_wait_all(i16x4 (&r)[N]) {
-    static_assert(N % 4 == 0, "fragments come in groups of four registers pairs");
-#pragma unroll
-    for (int i = 0; i < N; i += 4)
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(r[i]), "+v"(r[i + 1]), "+v"(r[i + 2]), "+v"(r[i + 3]));
-}
 
 template <typename Tag> __device__ __forceinline__ void mma16(f32x16& acc, const i16x8& a, const i16x8& b);
 template <> __device__ __forceinline__ void mma16<F16>(f32x16& acc, const i16x8& a, const i16x8& b) {

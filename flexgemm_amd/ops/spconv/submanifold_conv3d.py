@@ -506,12 +506,6 @@ def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, ne
     return nmap, gray, binary, order, None, pairs
 
 
-def _pad_cols(t: torch.Tensor, mult: int) -> torch.Tensor:
-    c = t.shape[-1]
-    pad = (-c) % mult
-    return t if pad == 0 else torch.nn.functional.pad(t, (0, pad))
-
-
 _panel_bytes_kept = 0       # bytes of weight panels kept with their weights (all devices)
 _pure_answers: dict = {}    # answers of the library's size / occupancy queries, which depend on their arguments alone
 
@@ -702,17 +696,9 @@ def _narrow_wgrad_applies(cache, f: torch.Tensor, ci: int, co: int, v: int, n: i
     return cache["_narrow_overflows"] == 0
 
 
-def _stream_fits(n: int, n_src: int, row_bytes: int) -> bool:
-    """The streaming kernel addresses its operands with 32-bit byte offsets."""
-    return n_src * row_bytes <= 0xFF000000 and n * 8 <= 0xFF000000 and n * 27 * 4 * 2 <= 0xFF000000
-
-
 def _sweep_fits(n: int, n_in: int, ci: int, co: int, elem_bytes: int, n_pairs: int) -> bool:
-    """What fgx_conv_wgrad_sweep accepts: it multiplies row numbers with 24-bit multiplies and addresses both operands
-    and the pair lists with 32-bit byte offsets below 0xFF000000 (the checks of the C entry point, restated)."""
-    return (0 < n <= (1 << 24) and n_in <= (1 << 24) and n_pairs > 0
-            and n * co * elem_bytes <= 0xFF000000 and n_in * ci * elem_bytes <= 0xFF000000
-            and n_pairs * 4 + 256 <= 0xFF000000)
+    """Whether the weight gradient of a sweep schedule runs on the sweep (what fgx_conv_wgrad_sweep accepts)."""
+    return nat.host().sweep_fits(n, n_in, ci, co, elem_bytes, n_pairs)
 
 
 # Fewest rows from which NARROW_RESIDENT = "auto" takes the resident-row kernel.
