@@ -527,6 +527,15 @@ Tensor pad_columns(const Tensor& t, int64_t multiple) {
     return pad ? at::constant_pad_nd(t, {0, pad}) : t;
 }
 
+// What a kernel would otherwise find out by reading past a buffer or on another device.
+void require_map(const Tensor& nmap, int64_t v) {
+    if (nmap.dim() != 2 || nmap.size(1) != v)
+        throw py::value_error("a neighbor cache of " + std::to_string(nmap.dim() == 2 ? nmap.size(1) : 0) + " kernel positions for a weight of " + std::to_string(v));
+}
+void require_on(const at::Device& dev, const Tensor& t, const char* what) {
+    if (t.defined() && t.device() != dev) throw py::value_error(std::string(what) + " is on " + t.device().str() + ", the features on " + dev.str());
+}
+
 struct Product {
     Tensor out, mask;
 };
@@ -545,8 +554,14 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
         throw py::type_error("features, weight and bias must share one dtype");
     const int es = (int)src.element_size(), v = (int)weight.size(1);
     const Tensor nmap = c.need("neighbor_map");
+    require_map(nmap, v);
+    require_on(dev, nmap, "the neighbor cache");
+    require_on(dev, weight, "the weight");
+    require_on(dev, bias, "the bias");
     const int64_t n = nmap.size(0), n_src = src.size(0);
     const int cols = (int)weight.size(mode == 0 ? 0 : 2);
+    if (bias.defined() && bias.numel() != cols)
+        throw py::value_error("a bias of " + std::to_string(bias.numel()) + " values for " + std::to_string(cols) + " output channels");
     Product p;
     if (n_src == 0) {                       // nothing to gather: the bias alone
         p.out = at::zeros({n, cols}, src.options());
@@ -722,6 +737,14 @@ WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool 
     const at::Device dev = feats.device();
     const c10::DeviceGuard guard(dev);
     const int code = dtype_code(feats);
+    {
+        const Tensor nmap = c.need("neighbor_map");
+        require_map(nmap, v);
+        require_on(dev, nmap, "the neighbor cache");
+        require_on(dev, grad, "the upstream gradient");
+        if (grad.size(0) != nmap.size(0))
+            throw py::value_error(std::to_string(grad.size(0)) + " gradient rows for a neighbor cache of " + std::to_string(nmap.size(0)) + " rows");
+    }
     const int64_t n = grad.size(0), n_in = feats.size(0), true_ci = feats.size(1), true_co = grad.size(1);
     const int es = (int)feats.element_size(), align = 16 / es;
     feats = pad_columns(feats, align).contiguous();
@@ -876,6 +899,9 @@ struct ConvBackward : public torch::autograd::Node {
         const Tensor f = feats.unpack(), w = weight.unpack(), m = has_mask ? mask.unpack() : Tensor();
         const Tensor y = relu && !has_mask ? output.unpack(shared_from_this()) : Tensor();
         if (has_bias) (void)bias.unpack();
+        for (const Tensor* t : {&f, &w, &m, &y})             // (... and may leave one where the kernels cannot read it)
+            if (t->defined() && t->device() != grads[0].device())
+                throw std::invalid_argument("a saved tensor of " + name() + " is on " + t->device().str() + ", the gradient on " + grads[0].device().str());
         const at::NoGradGuard no_grad;
         const py::gil_scoped_acquire gil;
         const Cache c(py::reinterpret_borrow<py::object>(cache.obj));

@@ -6,6 +6,7 @@ from torch.autograd import forward_ad
 from torch.utils.checkpoint import checkpoint
 
 import flex_gemm
+from flexgemm_amd.ops.spconv import submanifold_conv3d as impl
 from flexgemm_amd.workloads import reference_test_shell
 
 spconv = flex_gemm.ops.spconv
@@ -79,3 +80,31 @@ def test_a_chain_of_many_layers_is_freed(gpu_device):
     for _ in range(20000):
         h = layer(h, weight, bias)
     del h
+
+
+@pytest.mark.parametrize("c", [8, 64])
+def test_arguments_that_do_not_fit_the_cache_are_refused(gpu_device, c):
+    """On the host, before a kernel runs: the kernels would read past the map or the bias, or another device's memory."""
+    coords = torch.from_numpy(reference_test_shell(16)).to(gpu_device)
+    shape = torch.Size([1, c, 16, 16, 16])
+    feats = torch.zeros(len(coords), c, dtype=torch.half, device=gpu_device)
+    weight = torch.zeros(c, 3, 3, 3, c, dtype=torch.half, device=gpu_device)
+    cache = spconv.sparse_submanifold_conv3d(feats, coords, shape, weight)[1]
+
+    def call(w, b=None):
+        return spconv.sparse_submanifold_conv3d(feats, coords, shape, w, b, cache)
+
+    for other in (torch.zeros(c, 3, 3, 1, c).half().to(gpu_device), weight.cpu()):
+        with pytest.raises(ValueError):
+            call(other)
+    for bias in (torch.zeros(c - 1, dtype=torch.half, device=gpu_device), torch.zeros(c, dtype=torch.half)):
+        with pytest.raises(ValueError):
+            call(weight, bias)
+    with pytest.raises(ValueError):
+        impl._wgrad(feats[:-1], feats, cache, 27)
+    w = weight.clone().requires_grad_()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t):          # (kept on the host and left there)
+        out = call(w)[0]
+    with pytest.raises((ValueError, RuntimeError), match="saved tensor"):
+        torch.autograd.grad(out, w, torch.ones_like(out))
+    torch.autograd.grad(call(w)[0], w, torch.ones_like(out))
