@@ -170,6 +170,26 @@ def test_walk_is_a_function_of_the_coordinates(gpu_device, twice, outside):
         assert np.array_equal(walk, walks[0])
 
 
+# the index's two forms: such a voxel is nobody's neighbor, finds the voxels that are its own neighbors, and is its own middle entry
+@pytest.mark.parametrize("res", [40, 210])
+def test_voxels_outside_the_grid(gpu_device, res):
+    _say(f"voxels outside the grid res={res}")
+    rng = np.random.default_rng(res)
+    coords = np.concatenate([reference_test_shell(40), [[0, -1, 5, 5], [0, res, 6, 6], [0, 5, -7, 5], [0, 8, 8, res], [0, 8, res + 900, 8], [1, 5, 5, 5],
+                                                        [-1, 5, 5, 5], [0, 20, 0, -1]]]).astype(np.int32)
+    coords = np.ascontiguousarray(coords[rng.permutation(len(coords))])
+    inside = ((coords >= 0) & (coords < np.array([1, res, res, res]))).all(1)
+    at = {tuple(c): i for i, c in enumerate(coords) if inside[i]}
+    want = np.full((len(coords), 27), 0xFFFFFFFF, np.uint32)
+    for i, (b, x, y, z) in enumerate(coords):
+        for v in range(27):
+            want[i, v] = at.get((b, x + v // 9 - 1, y + v // 3 % 3 - 1, z + v % 3 - 1), 0xFFFFFFFF)
+        want[i, 13] = i
+    cache = SubMConv3dFunction._compute_neighbor_cache(torch.from_numpy(coords).to(gpu_device), torch.Size([1, 0, res, res, res]), (3, 3, 3),
+                                                       (1, 1, 1), False)
+    assert np.array_equal(_np(cache.neighbor_map), want)
+
+
 # an infinity or NaN in the upstream gradient reaches the weight gradient through its own pairs alone, not as its product with the
 # zeros that stand for a missing neighbor
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
