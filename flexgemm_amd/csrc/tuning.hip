@@ -271,9 +271,11 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
     const size_t steps = (size_t)V * cdiv(row_bytes, (size_t)64);
     for (; s < (steps >= 160 ? 16 : 8); s *= 2) {
         size_t pieces = cols <= 32 ? 700 : kCUs;
-        // (128 x 128 tiles under a long K: two pieces for a CU rather than one and a half; 5 816 voxels, 256 channels in 4 splits 0.053 ms, in 8
-        // 0.048; 1 976 voxels, 768 <- 256 0.054 and 0.049; not from 1.6 on: 13 488 voxels, 320 <- 96 0.062 and 0.067.  Input gradients
-        // alone: other splits round a forward sum differently, and a ReLU behind it then falls on its other side now and then)
+        // (input gradients on 128 x 128 tiles under a long K: two pieces for a CU rather than one and a half; 5 816 voxels, 256 channels in 4
+        // splits 0.051 ms, in 8 0.045; 384 -> 256 0.067 and 0.057; not from 1.6 on: 13 488 voxels, 96 <- 320 0.059 and 0.064.  The forward
+        // pass would gain as much -- 5 816 voxels, 256 channels 0.050 and 0.046, 1 976 voxels, 256 -> 768 0.051 and 0.047 -- and does
+        // without it: another split rounds a forward sum differently, so that a ReLU behind it changes sides here and there, and
+        // results stay those of the splits it has had.)
         if (pass_kind != 0 && out->tile_rows == 128 && out->tile_cols == 128 && steps >= 160) pieces = 400;
         if (out->tile_cols == 64 && (s < 4 ? steps >= 54 : (s < 8 && steps >= 320))) pieces = 450;
         if (tiles * s >= pieces) break;
