@@ -884,10 +884,17 @@ struct ConvBackward : public torch::autograd::Node {
         } catch (py::error_already_set& e) {        // keep the Python error's type on its way through the engine's thread
             const py::gil_scoped_acquire gil;
             e.restore();
-            python_error err;
-            err.persist();
-            throw err;
+            throw_persistent();
+        } catch (py::builtin_exception& e) {        // (py::value_error and its like, which become one only in pybind's hands)
+            const py::gil_scoped_acquire gil;
+            e.set_error();
+            throw_persistent();
         }
+    }
+    [[noreturn]] static void throw_persistent() {
+        python_error err;
+        err.persist();
+        throw err;
     }
 
     variable_list gradients(variable_list&& grads) {
@@ -901,7 +908,7 @@ struct ConvBackward : public torch::autograd::Node {
         if (has_bias) (void)bias.unpack();
         for (const Tensor* t : {&f, &w, &m, &y})             // (... and may leave one where the kernels cannot read it)
             if (t->defined() && t->device() != grads[0].device())
-                throw std::invalid_argument("a saved tensor of " + name() + " is on " + t->device().str() + ", the gradient on " + grads[0].device().str());
+                throw py::value_error("a saved tensor of " + name() + " is on " + t->device().str() + ", the gradient on " + grads[0].device().str());
         const at::NoGradGuard no_grad;
         const py::gil_scoped_acquire gil;
         const Cache c(py::reinterpret_borrow<py::object>(cache.obj));
