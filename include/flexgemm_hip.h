@@ -189,7 +189,8 @@ int fgx_subm_cache_build(const int32_t* coords, size_t n, int B, int W, int H, i
  * The map: kernel volumes up to 128, mask codes (gray / binary, both or neither) up to 32.  The cache: as
  * fgx_subm_cache_build, without the sort's key_bits and presorted; seg_host (optional): pinned host memory that receives the
  * segment table as well (valid once the stream has passed the call); walk (optional, where fgx_grid_index_walks is 1): the rows
- * in the order of the index's cells, a space-filling curve, for fgx_narrow_plan_walk.
+ * in the order of the index's cells, a space-filling curve, then the rows without a cell of their own (given again, or outside the
+ * grid) in row order, for fgx_narrow_plan_walk.
  * Replaces: hashmap_build_submanifold_conv_neighbour_map and the same sequence of calls as fgx_subm_cache_build. */
 int fgx_grid_index_pays(size_t n, int B, int W, int H, int D);
 int fgx_grid_index_walks(size_t n, int B, int W, int H, int D);
@@ -379,7 +380,7 @@ int fgx_conv_narrow_gemm(int dtype, const void* src, const void* panel, const vo
  * fgx_conv_wgrad fetches two rows per pair), the gather happens in the transposing LDS reads.  Every workgroup keeps the
  * accumulators of all V offsets over its chunks and writes one partial product; a second kernel adds the partial
  * products in workgroup order (same bits on every run; against fgx_conv_wgrad the sums differ by fp32 rounding of a
- * different order).  The plan must have been made with same_rows = 1 and must have NO overflowing chunk: the first
+ * different order; an infinity or NaN of grad_out counts for its own pairs, as there).  The plan must have been made with same_rows = 1 and must have NO overflowing chunk: the first
  * uint32 of the plan counts them -- read it back once per plan and call fgx_conv_wgrad instead when it is not 0.
  * scratch: fgx_narrow_wgrad_scratch_bytes(V) bytes, 16-byte aligned.  The bias gradient is not made here (fgx_colsum).
  * No counterpart in the reference (..._bwd_masked_implicit_gemm_splitk.py:108-182 gathers both operands per pair). */
@@ -389,13 +390,15 @@ int fgx_conv_narrow_wgrad(int dtype, const void* grad_out, const void* feats, co
 
 /* Forward product and input gradient of a network's first layers: K (Ci in mode 0, Co in modes 1 and 2, modes as in
  * fgx_pack_weight) of 8 or 16, 16-bit types, V of 17 ... 27, a multiple of 8 columns.  Reads the neighbor map [n, V] row by row and
- * the weight itself; no row order, tile masks or panel.  fgx_conv_gemm_stem_pays says where it is the faster kernel. */
+ * the weight itself; no row order, tile masks or panel.  src, weight, map and out 16-byte aligned.  fgx_conv_gemm_stem_pays says where
+ * it is the faster kernel. */
 int fgx_conv_gemm_stem_pays(int dtype, int mode, size_t n, int K, int cols, int V);
 int fgx_conv_gemm_stem(int dtype, int mode, const void* src, const void* weight, const void* bias, const uint32_t* map, size_t n,
                        int Ci, int Co, int V, int activation, void* out, uint8_t* relu_mask, fgx_stream_t stream);
 
 /* The weight gradient of a network's first layers: Ci of 8 or 16, 16-bit types, V of 17 ... 27, Co a multiple of 8, straight from
- * the neighbor map ([n, V], row r of grad_out its row r) without pair lists.  grad_bias (optional) comes with it.
+ * the neighbor map ([n, V], row r of grad_out its row r) without pair lists: sums over the pairs, an infinity or NaN of grad_out included.
+ * grad_bias (optional) comes with it.
  * fgx_wgrad_stem_pays says where it is the faster kernel.  scratch: fgx_wgrad_stem_scratch_bytes bytes; buffers 16-byte aligned. */
 int fgx_wgrad_stem_pays(int dtype, size_t n, int Ci, int Co, int V);
 size_t fgx_wgrad_stem_scratch_bytes(size_t n, int Ci, int Co);
