@@ -328,7 +328,19 @@ struct WStreamCfg {
     static constexpr int LPS = A_PER + B_PER;
     static constexpr int A_BYTES = P * ROWB_A, B_BYTES = P * ROWB_B, STAGE_BYTES = A_BYTES + B_BYTES;
     static constexpr int IDX_SLOT_BYTES = 2 * P * 4;               // sig_o x P | sig_i x P
-    static constexpr size_t lds_bytes = (size_t)S * STAGE_BYTES + (size_t)kWsIdxSlots * IDX_SLOT_BYTES;
+    static constexpr int RING_BYTES = S * STAGE_BYTES + kWsIdxSlots * IDX_SLOT_BYTES;
+    // Epilogue band of a multiplier, behind the rings: as many of a 32-row accumulator's rows (32, 16, 8 or 4) as what the rings
+    // leave of the 160 KiB holds, in the output type (`es` bytes an element).
+    static constexpr int band_pitch(int es) { return WN * es + 16; }
+    static constexpr int band_rows(int es) {
+        int rows = 32;
+        while (rows * band_pitch(es) * NW > 160 * 1024 - RING_BYTES) rows /= 2;
+        return rows;
+    }
+    static constexpr int band_bytes(int es) { return band_rows(es) * band_pitch(es); }
+    static constexpr int BAND_BYTES = band_bytes(ES) > band_bytes(4) ? band_bytes(ES) : band_bytes(4);
+    static constexpr size_t lds_bytes = (size_t)RING_BYTES + (size_t)NW * BAND_BYTES;
+    static_assert(band_rows(4) >= 1024 / (WN * 4) && band_rows(ES) >= 1024 / (WN * ES), "a wave-wide store takes its rows from one band");
     static_assert(ES == 2, "the streaming kernel handles 16-bit types");
     static_assert(S == 3 || S == 4, "the loaders' wait is written for rings of three or four stages");
     static_assert(kWsIdxAhead > S - 1 && lds_bytes <= 160 * 1024, "index loads run ahead of the row loads; the ring fits LDS");
@@ -354,6 +366,7 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     unsigned char* ring = lds_raw;                                              // [S][A rows | B rows]
     uint32_t* idx_ring = (uint32_t*)(ring + S * C::STAGE_BYTES);                // [kWsIdxSlots][o x P | i x P]
+    unsigned char* bands = ring + C::RING_BYTES;                                // [NW][BAND_BYTES]
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -656,7 +669,7 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
     #pragma unroll
                         for (int j = 0; j < C::TN; ++j) {
                             const i16x8 bf = __builtin_shufflevector(fr[kk & 1][(C::TM + j) * 2], fr[kk & 1][(C::TM + j) * 2 + 1], 0, 1, 2, 3, 4, 5, 6, 7);
-                            mma16<Tag>(acc[i][j], af, bf);
+                            mma16<Tag>(acc[i][j], bf, af);       // transposed tile
                         }
                     }
                 });
@@ -668,26 +681,54 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
         } else {
             run_steps(std::false_type{});
         }
-        // partial[b][v][co][ci], fp32
+        // partial[b][v][co][ci], fp32 -- or, with a single voxel block, straight into grad_weight[co][v][ci].  The products were
+        // taken with the operands swapped: element e of lane l is row l % 32 (co) and column 8 * (e / 4) + 4 * (l / 32) + e % 4 (ci), so four
+        // neighbors of an output row lie in one lane.  They go through the wavefront's band in LDS and leave as 16-byte pieces,
+        // whole lines of an output row side by side.  (Stored element by element the tile took 64 address computations, conversions and
+        // 64-byte stores of a wavefront that has its SIMD's matrix unit to itself, longer than the products of an item of few
+        // pairs: 864 voxels x 1024 channels, 1728 items of 6 steps, 77 -> 50 us.)
         const unsigned co_tile = tile % co_tiles, ci_tile = tile / co_tiles;
         const int m0 = (int)co_tile * BM, n0 = (int)ci_tile * BN;
-        float* dst = partial + (((size_t)b * C::SLICES + (C::KSPLIT ? mw : 0)) * V + v) * ((size_t)Co * Ci);
-        typename Tag::type* out = direct ? direct + (size_t)v * Ci : nullptr;      // single voxel block: no partial products
+        auto write_tile = [&](auto* dst, size_t row_stride, bool pieces_ok) {
+            using O = std::remove_pointer_t<decltype(dst)>;
+            using O4 = O __attribute__((ext_vector_type(4)));
+            constexpr int OS = (int)sizeof(O), PITCH = C::band_pitch(OS), ROWS = C::band_rows(OS), PARTS = 32 / ROWS;
+            constexpr int PIECES = C::WN * OS / 16, RPP = 64 / PIECES;      // 16-byte pieces of a band row, rows of a wave-wide store
+            unsigned char* band = bands + mw * C::BAND_BYTES;
+            const int piece = lane % PIECES, ci = n0 + wave_n * C::WN + piece * (16 / OS);
 #pragma unroll
-        for (int j = 0; j < C::TN; ++j) {
-            const int ci = n0 + wave_n * C::WN + j * 32 + l32;
-            if (ci >= Ci) continue;
+            for (int ih = 0; ih < C::TM * PARTS; ++ih) {
+                const int i = ih / PARTS, h = ih % PARTS;
+                if (PARTS == 1 || l32 / ROWS == h) {
 #pragma unroll
-            for (int i = 0; i < C::TM; ++i)
+                    for (int j = 0; j < C::TN; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    int co = m0 + wave_m * C::WM + i * 32 + (e >> 2) * 8 + g * 4 + (e & 3);
-                    if (co < Co) {
-                        if (out) out[(size_t)co * V * Ci + ci] = from_float<typename Tag::type>(acc[i][j][e]);
-                        else dst[(size_t)co * Ci + ci] = acc[i][j][e];
+                        for (int q = 0; q < 4; ++q) {
+                            O4 four;
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) four[e] = (O)acc[i][j][q * 4 + e];
+                            *(O4*)(band + (l32 - h * ROWS) * PITCH + (j * 32 + q * 8 + g * 4) * OS) = four;
+                        }
+                }
+                // (written and read by the same wavefront: program order suffices)
+#pragma unroll
+                for (int pass = 0; pass < ROWS / RPP; ++pass) {
+                    const int r = pass * RPP + lane / PIECES;
+                    const int co = m0 + wave_m * C::WM + i * 32 + h * ROWS + r;
+                    const unsigned char* sp = band + r * PITCH + piece * 16;
+                    O* dp = dst + (size_t)co * row_stride + ci;
+                    if (co >= Co || ci >= Ci) continue;
+                    if (pieces_ok) {
+                        *(u32x4*)dp = *(const u32x4*)sp;
+                    } else {
+                        for (int t = 0; t < 16 / OS && ci + t < Ci; ++t) dp[t] = ((const O*)sp)[t];
                     }
                 }
-        }
+            }
+        };
+        if (direct) write_tile(direct + (size_t)v * Ci, (size_t)V * Ci, (((uintptr_t)direct | (uintptr_t)(Ci * ES)) & 15) == 0);
+        else write_tile(partial + (((size_t)b * C::SLICES + (C::KSPLIT ? mw : 0)) * V + v) * ((size_t)Co * Ci), (size_t)Ci,
+                        (((uintptr_t)partial | (uintptr_t)(Ci * 4)) & 15) == 0);
         if (do_bias && l32 == 0) {                  // bias_partial[block * SLICES + slice][co]
             float* bdst = bias_partial + ((size_t)b * C::SLICES + (C::KSPLIT ? mw : 0)) * Co;
 #pragma unroll
