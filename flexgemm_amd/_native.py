@@ -32,7 +32,8 @@ EXPORTS = [
     "fgx_tile_workspace_bytes", "fgx_tile_codes", "fgx_tile_fill",
     "fgx_table_lookup", "fgx_weight_panel_bytes", "fgx_pack_weight",
     "fgx_conv_scratch_bytes", "fgx_conv_gather_gemm", "fgx_conv_gather_gemm_act", "fgx_conv_gather_gemm_act_mask", "fgx_conv_gather_gemm_weight_pays",
-    "fgx_conv_gather_gemm_weight",
+    "fgx_conv_gather_gemm_weight", "fgx_conv_gemm_pairs_pays", "fgx_pair_plan_words", "fgx_pair_plan", "fgx_conv_gemm_pairs_scratch_bytes",
+    "fgx_conv_gemm_pairs",
     "fgx_relu_mask_apply", "fgx_conv_gather_gemm_stream_act_mask",
     "fgx_gather_plan_count", "fgx_gather_plan_fill", "fgx_conv_gather_gemm_stream", "fgx_conv_gather_gemm_stream_act",
     "fgx_conv_gather_gemm_stream_groups", "fgx_gather_item_order_workspace_bytes", "fgx_gather_item_order",
@@ -106,7 +107,7 @@ def lib() -> C.CDLL:
         L = C.CDLL(_LIB_PATH)
         L.fgx_last_error.restype = C.c_char_p
         for name in ("fgx_sort_workspace_bytes", "fgx_locality_workspace_bytes", "fgx_pair_workspace_bytes", "fgx_tile_workspace_bytes",
-                     "fgx_weight_panel_bytes", "fgx_conv_scratch_bytes", "fgx_wgrad_scratch_bytes",
+                     "fgx_weight_panel_bytes", "fgx_conv_scratch_bytes", "fgx_wgrad_scratch_bytes", "fgx_pair_plan_words", "fgx_conv_gemm_pairs_scratch_bytes",
                      "fgx_colsum_scratch_bytes", "fgx_spconv_out_coords_workspace_bytes",
                      "fgx_subm_neighbor_map_sorted_workspace_bytes", "fgx_wgrad_block_bounds_count", "fgx_wgrad_item_lists_count", "fgx_narrow_plan_bytes", "fgx_narrow_wgrad_scratch_bytes",
                      "fgx_spconv_neighbor_map_sorted_workspace_bytes", "fgx_serialize_reorder_workspace_bytes",

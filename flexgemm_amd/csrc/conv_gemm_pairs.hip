@@ -1,0 +1,562 @@
+// Gather GEMM of few voxels under wide weights, offset by offset over the pairs that exist (forward and dgrad, gfx950).
+//
+//   partial[p, :] = src[in(p), :] x W_v          for the pairs p = (r, v) of one offset v after the other
+//   out[r, :]     = sum over v of partial[pair(r, v), :] (+ bias)
+//
+// The masked kernels multiply a tile of output rows with every offset that any of its rows has.  A few hundred or thousand voxels
+// of a surface have nearly as many masks as voxels, so a tile carries almost all offsets and 2 to 2.5 rows are multiplied per
+// pair (864 voxels of a thick shell: 0.42 of the rows of a 256-row tile have the offset; 3 758 voxels 0.51; 41 700 voxels 0.58).  Here the rows
+// of a tile are 128 pairs of ONE offset: 0.89 and 0.96 of what is multiplied exists.  What that costs is the partial sums, 4 bytes
+// per pair and output column written and read once, which the 256 MB memory-side cache holds for as many voxels as this
+// pays for.  The product itself has no masks, bands or index stream left: a tile's source rows are known before its first step.
+//
+// fgx_pair_plan lists the pairs: per offset how many, their source rows in row order, and for each (row, offset) its place in the
+// offset's list.  Nothing is read back: the launch covers the most tiles there can be, and a workgroup finds its tile -- or that
+// there is none for it -- from the counts.
+#include "gemm_device.h"
+#include "lds_read.h"
+
+namespace fgx {
+namespace {
+
+constexpr int kPairRows = 128;                      // pairs of a tile
+constexpr int kPairMaxV = 32;
+constexpr uint32_t kOobOffset = 0xFF000000u;        // buffer offset no operand reaches: the load returns zeros
+
+using rsrc_t = __amdgpu_buffer_rsrc_t;
+__device__ __forceinline__ rsrc_t make_rsrc(const void* p, uint32_t bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
+}
+
+constexpr int kPairChunk = 256;     // rows a workgroup of the plan places
+
+// plan: counts[kPairMaxV] | place[n][V] | rows[V][n] | the chunks' counts [chunks][kPairMaxV] (while it is made)
+__host__ __device__ inline size_t pair_place_at() { return kPairMaxV; }
+__host__ __device__ inline size_t pair_rows_at(size_t n, int V) { return kPairMaxV + n * (size_t)V; }
+__host__ __device__ inline size_t pair_chunks_at(size_t n, int V) { return kPairMaxV + 2 * n * (size_t)V; }
+
+// Up to kPairColumnRows rows in one launch: a workgroup per offset, four words of its column in flight per thread, one barrier to hand
+// the wavefronts' counts round.  It waits for the scattered words (a wave-wide load takes 64 lines): 864 rows 4.2 us, 3 758 rows 8.2.
+constexpr int kPairColumnRows = 4096;
+__global__ void __launch_bounds__(1024) pair_plan_columns_kernel(const uint32_t* __restrict__ map, uint32_t n, int V, uint32_t* __restrict__ plan) {
+    __shared__ uint32_t counts[64];             // of (quarter of the rows, wavefront)
+    const int v = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t m[4];
+    unsigned long long have[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t r = q * 1024 + threadIdx.x;
+        m[q] = r < n ? map[(size_t)r * V + v] : FGX_EMPTY32;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        have[q] = __ballot(m[q] != FGX_EMPTY32);
+        if (lane == 0) counts[q * 16 + wave] = (uint32_t)__popcll(have[q]);
+    }
+    __syncthreads();
+    const uint32_t mine = counts[lane];
+    uint32_t to = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+        const uint32_t other = (uint32_t)__shfl_up((int)to, d, 64);
+        if (lane >= d) to += other;
+    }
+    uint32_t* place = plan + pair_place_at();
+    uint32_t* rows = plan + pair_rows_at(n, V) + (size_t)v * n;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t r = q * 1024 + threadIdx.x;
+        const uint32_t at = (uint32_t)__shfl((int)(to - mine), q * 16 + wave, 64) + (uint32_t)__popcll(have[q] & ((1ull << lane) - 1ull));
+        if (r < n) place[(size_t)r * V + v] = m[q] != FGX_EMPTY32 ? at : FGX_EMPTY32;
+        if (m[q] != FGX_EMPTY32) rows[at] = m[q];
+    }
+    if (threadIdx.x == 63) plan[v] = to;
+}
+
+// More rows: a workgroup takes kPairChunk of them through LDS, a thread a row, so the map comes in and the places go out as whole
+// lines; a launch of its own counts the chunks first (COUNT).  38 407 rows 12.6 us (column by column in chunks of 4096: 22.6), 3 758 rows 10.9.
+template <bool COUNT, int VC>
+__global__ void __launch_bounds__(kPairChunk) pair_plan_kernel(const uint32_t* __restrict__ map, uint32_t n, int v_arg, uint32_t* __restrict__ plan) {
+    constexpr int kWaves = kPairChunk / 64, VM = VC > 0 ? VC : kPairMaxV;
+    extern __shared__ uint32_t words[];                         // [kPairChunk][V]
+    __shared__ uint32_t counts[kPairMaxV][kWaves], before[kPairMaxV];
+    const int V = VC > 0 ? VC : v_arg;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    uint32_t* chunks = plan + pair_chunks_at(n, V);
+    const uint32_t base = blockIdx.x * (uint32_t)kPairChunk, here = n - base < (uint32_t)kPairChunk ? n - base : (uint32_t)kPairChunk;
+    const uint32_t* from = map + (size_t)base * V;
+    {
+        uint32_t w[VM];
+#pragma unroll
+        for (int i = 0; i < VM; ++i) w[i] = i < V && i * kPairChunk + tid < (int)here * V ? from[i * kPairChunk + tid] : FGX_EMPTY32;
+#pragma unroll
+        for (int i = 0; i < VM; ++i)
+            if (i < V) words[i * kPairChunk + tid] = w[i];      // (rows past the end: no neighbors)
+    }
+    if constexpr (!COUNT) {                                     // pairs of the chunks before this one, 8 threads on each offset
+        static_assert(kPairChunk == 8 * kPairMaxV, "a thread for every eighth of an offset's chunks");
+        const int v = tid >> 3;
+        uint32_t sum = 0;
+        for (uint32_t c0 = 0; c0 < blockIdx.x; c0 += 64) {      // (eight loads in flight)
+#pragma unroll
+            for (uint32_t q = 0; q < 64; q += 8) {
+                const uint32_t c = c0 + q + (uint32_t)(tid & 7);
+                sum += v < V && c < blockIdx.x ? chunks[(size_t)c * kPairMaxV + v] : 0u;
+            }
+        }
+#pragma unroll
+        for (int d = 4; d > 0; d /= 2) sum += (uint32_t)__shfl_xor((int)sum, d, 64);
+        if ((tid & 7) == 0) before[v] = sum;
+    }
+    __syncthreads();
+    uint32_t m[VM];
+#pragma unroll
+    for (int v = 0; v < VM; ++v) m[v] = v < V ? words[tid * V + v] : FGX_EMPTY32;
+    uint32_t have_mine = 0;
+#pragma unroll
+    for (int v = 0; v < VM; ++v) {
+        const uint32_t c = (uint32_t)__popcll(__ballot(m[v] != FGX_EMPTY32));
+        have_mine = lane == v ? c : have_mine;
+    }
+    if (lane < VM) counts[lane][wave] = have_mine;
+    __syncthreads();
+    if (tid < V) {                                              // up to each wavefront, and all of them
+        uint32_t to = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            const uint32_t c = counts[tid][w];
+            if constexpr (!COUNT) counts[tid][w] = before[tid] + to;
+            to += c;
+        }
+        if constexpr (COUNT) chunks[(size_t)blockIdx.x * kPairMaxV + tid] = to;
+        else if (blockIdx.x == gridDim.x - 1) plan[tid] = before[tid] + to;
+    }
+    if constexpr (!COUNT) {
+        __syncthreads();
+        uint32_t* rows = plan + pair_rows_at(n, V);
+#pragma unroll
+        for (int v = 0; v < VM; ++v) {
+            if (v >= V) break;
+            const unsigned long long have = __ballot(m[v] != FGX_EMPTY32);
+            const uint32_t at = counts[v][wave] + (uint32_t)__popcll(have & ((1ull << lane) - 1ull));
+            if (m[v] != FGX_EMPTY32) rows[(size_t)v * n + at] = m[v];
+            words[tid * V + v] = m[v] != FGX_EMPTY32 ? at : FGX_EMPTY32;
+        }
+        __syncthreads();
+        uint32_t* place = plan + pair_place_at() + (size_t)base * V;
+#pragma unroll
+        for (int i = 0; i < VM; ++i)
+            if (i < V && i * kPairChunk + tid < (int)here * V) place[i * kPairChunk + tid] = words[i * kPairChunk + tid];
+    }
+}
+
+// Lane v < 32 of a wavefront holds offset v's number of pairs: the pairs and the tiles of the offsets up to and with it (lanes above: nothing).
+__device__ __forceinline__ void scan_counts(const uint32_t* __restrict__ plan, int V, int lane, uint32_t& pairs, uint32_t& tiles, uint32_t& count) {
+    count = lane < V ? plan[lane] : 0u;
+    pairs = count;
+    tiles = (count + kPairRows - 1) / kPairRows;
+#pragma unroll
+    for (int d = 1; d < kPairMaxV; d *= 2) {
+        const uint32_t p = (uint32_t)__shfl_up((int)pairs, d, 64), t = (uint32_t)__shfl_up((int)tiles, d, 64);
+        if (lane >= d) {
+            pairs += p;
+            tiles += t;
+        }
+    }
+}
+
+// Where the weight is read from: as in the tiled gather GEMM, lines of one (offset, K-slab).
+//   TR = false: a line is an output column, its K values side by side;  TR = true: a line is a K value, its columns side by side.
+struct PairWeight {
+    const unsigned char* base;
+    uint32_t bytes, v_stride, slab_stride, line_stride;
+    int mirrored;           // offset v multiplies the weight of V - 1 - v
+};
+
+template <typename Tag, bool TR, int BN_, int WAVES_M>
+struct PairCfg {
+    using T = typename Tag::type;
+    static constexpr int ES = (int)sizeof(T), CH = 8, SLAB = 128, SK = SLAB / ES;
+    static constexpr int BM = kPairRows, BN = BN_, NW = 4, NT = 256, WAVES_N = NW / WAVES_M;
+    static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, TM = WM / 32, TN = WN / 32;
+    static constexpr int A_PER = BM / 8 / NW;                       // a wave-wide load covers 8 rows of 128 bytes
+    static constexpr int LCOLS = BN == 96 ? 128 : BN;               // columns of a transposed line in LDS: whole loads of whole lines
+    static constexpr int TCH = LCOLS * ES / 16, LINES = 64 / TCH;   // 16-byte pieces of a transposed line, lines a load covers
+    static constexpr int B_PER = TR ? SK / LINES / NW : BN / 8 / NW;
+    static constexpr int LPS = A_PER + B_PER;
+    static constexpr int STAGE = (BM + (TR ? LCOLS : BN)) * SLAB, S = 2;
+    static constexpr int tr_key(int line) { return ES != 2 ? 0 : (TCH >= 16 ? 4 * (line & 3) : 2 * (line & 3)); }   // 4 lines of a transposing read, 4 bank groups
+    static constexpr int PITCH = WN * 4 + 16;                       // epilogue band of a wavefront: 32 rows of WN sums
+    static constexpr size_t lds_bytes = S * STAGE;
+    static_assert(NW * 32 * PITCH <= S * STAGE, "the epilogue bands lie in the ring");
+    static_assert(2 * lds_bytes <= 160 * 1024, "two workgroups share a CU: one multiplies while the other waits for LDS");
+};
+
+// One tile of 128 pairs x 128 columns per workgroup, four wavefronts of 64 x 64, K in slabs of 128 bytes through two stages: a
+// stage's fragments are taken into registers, the loads two slabs on go out into it, and the products run meanwhile.  Two
+// workgroups per CU cover each other's barriers.  XCD x takes the x-th eighth of the (column tile, row tile) list, so a part of
+// the weight -- the larger operand here -- crosses to one XCD only.
+// 864 voxels x 1024 channels (11 022 pairs, 57 MB of weight) 44 us, 513 TFLOP/s; 3 758 voxels 146 us, 695 TFLOP/s.  Tiles of 128 x 256 and 256 x 128 on
+// eight wavefronts, rings of three to five slabs, slabs of 64 bytes, and loads by wavefronts of their own in a persistent workgroup came out between
+// 0.9 and 1.2 of that time, ahead only for the second, behind for everything smaller.
+template <typename Tag, bool TR, int BN, int WAVES_M>
+__global__ void __launch_bounds__(256, 2)
+pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const uint32_t* __restrict__ plan, uint32_t n, int K, int cols,
+                 int V, uint32_t src_bytes, float* __restrict__ partial) {
+    using C = PairCfg<Tag, TR, BN, WAVES_M>;
+    constexpr int CH = C::CH;
+    extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_m = wave / C::WAVES_N, wave_n = wave % C::WAVES_N;
+
+    uint32_t pairs_to, tiles_to, count;
+    scan_counts(plan, V, lane, pairs_to, tiles_to, count);
+    const uint32_t row_tiles = (uint32_t)__builtin_amdgcn_readlane((int)tiles_to, kPairMaxV - 1);
+    const uint32_t total = row_tiles * ((cols + C::BN - 1) / C::BN), per_xcd = (total + kXcds - 1) / kXcds;
+    const uint32_t logical = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+    if (blockIdx.x / kXcds >= per_xcd || logical >= total) return;      // whole workgroup
+    const uint32_t col_tile = logical / row_tiles, row_tile = logical % row_tiles;
+    const int v = __builtin_amdgcn_readfirstlane(__popc((uint32_t)__ballot(tiles_to <= row_tile)));
+    const uint32_t have = (uint32_t)__builtin_amdgcn_readlane((int)count, v);
+    const uint32_t first = (row_tile - ((uint32_t)__builtin_amdgcn_readlane((int)tiles_to, v) - (have + C::BM - 1) / C::BM)) * C::BM;
+    const uint32_t live = have - first < (uint32_t)C::BM ? have - first : (uint32_t)C::BM;              // pairs of this tile
+    const size_t pair0 = (size_t)((uint32_t)__builtin_amdgcn_readlane((int)pairs_to, v) - have + first);
+    const int col0 = (int)col_tile * C::BN;
+
+    const rsrc_t src_rs = make_rsrc(src, src_bytes), b_rs = make_rsrc(b.base, b.bytes);
+    const uint32_t* rows = plan + pair_rows_at(n, V) + (size_t)v * n + first;
+    const uint32_t row_bytes = (uint32_t)K * C::ES;
+    const int slabs = (int)((row_bytes + C::SLAB - 1) / C::SLAB);
+    const bool ragged = row_bytes % C::SLAB != 0;
+
+    uint32_t a_off[C::A_PER], a_at[C::A_PER], b_off[C::B_PER], b_at[C::B_PER];      // ..._at: byte (TR: K value) inside the slab
+#pragma unroll
+    for (int i = 0; i < C::A_PER; ++i) {
+        const uint32_t r = (uint32_t)((i * C::NW + wave) * 8 + lane / 8);
+        a_at[i] = (uint32_t)(((lane & 7) ^ swz_key<CH>((int)r)) << 4);
+        a_off[i] = r < live ? rows[r] * row_bytes + a_at[i] : kOobOffset;
+    }
+    const int wv = b.mirrored ? V - 1 - v : v;
+#pragma unroll
+    for (int i = 0; i < C::B_PER; ++i) {
+        if constexpr (TR) {
+            const int line = (i * C::NW + wave) * C::LINES + lane / C::TCH;
+            const int piece = (lane % C::TCH) ^ C::tr_key(line);
+            b_at[i] = (uint32_t)line;
+            b_off[i] = piece * (16 / C::ES) < BN && col0 + piece * (16 / C::ES) < cols ? (uint32_t)line * b.line_stride + (uint32_t)(col0 * C::ES + (piece << 4)) : kOobOffset;
+        } else {
+            const int col = (i * C::NW + wave) * 8 + lane / 8;
+            b_at[i] = (uint32_t)(((lane & 7) ^ swz_key<CH>(col)) << 4);
+            b_off[i] = col0 + col < cols ? (uint32_t)(col0 + col) * b.line_stride + b_at[i] : kOobOffset;
+        }
+    }
+    uint32_t b_soff = (uint32_t)wv * b.v_stride;
+    auto issue = [&](int slab) {
+        unsigned char* stage = ring + (slab & 1) * C::STAGE;
+        const bool tail = ragged && slab == slabs - 1;
+        const uint32_t a_soff = (uint32_t)slab * C::SLAB;
+#pragma unroll
+        for (int i = 0; i < C::A_PER; ++i) {
+            const uint32_t vo = tail && a_soff + a_at[i] >= row_bytes ? kOobOffset : a_off[i];
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(src_rs, FGX_LDS_PTR(stage + (i * C::NW + wave) * 1024), 16, vo, a_soff, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < C::B_PER; ++i) {
+            const bool past = tail && (TR ? slab * C::SK + (int)b_at[i] >= K : a_soff + b_at[i] >= row_bytes);
+            const uint32_t vo = past ? kOobOffset : b_off[i];
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(b_rs, FGX_LDS_PTR(stage + C::BM * C::SLAB + (i * C::NW + wave) * 1024), 16, vo, b_soff, 0, 0);
+        }
+        b_soff += b.slab_stride;
+    };
+
+    const int g = lane >> 5, l32 = lane & 31, s16 = lane & 15, half = (lane >> 4) & 1;
+    int a_frag[CH / 2][C::TM], b_frag[CH / 2][C::TN];
+#pragma unroll
+    for (int kk = 0; kk < CH / 2; ++kk)
+#pragma unroll
+        for (int i = 0; i < C::TM; ++i) a_frag[kk][i] = swz<CH>(wave_m * C::WM + i * 32 + l32, kk * 2 + g);
+#pragma unroll
+    for (int kk = 0; kk < CH / 2; ++kk)
+#pragma unroll
+        for (int i = 0; i < C::TN; ++i) {
+            if constexpr (TR && C::ES == 2) {
+                const int line = kk * 16 + g * 8 + (s16 >> 2), byte = (wave_n * C::WN + i * 32 + half * 16 + (s16 & 3) * 4) * C::ES;
+                b_frag[kk][i] = C::BM * C::SLAB + line * (C::TCH * 16) + (((byte >> 4) ^ C::tr_key(line)) << 4) + (byte & 15);
+            } else if constexpr (TR) {
+                b_frag[kk][i] = C::BM * C::SLAB + (kk * 8 + g * 4) * (C::TCH * 16) + (wave_n * C::WN + i * 32 + l32) * C::ES;
+            } else {
+                b_frag[kk][i] = C::BM * C::SLAB + swz<CH>(wave_n * C::WN + i * 32 + l32, kk * 2 + g);
+            }
+        }
+    f32x16 acc[C::TM][C::TN];
+#pragma unroll
+    for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+        for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+    issue(0);
+    if (slabs > 1) issue(1);
+    for (int s = 0; s < slabs; ++s) {
+        if (s + 1 < slabs) wait_vmcnt<C::LPS>();        // all but the newest slab's loads have landed
+        else wait_vmcnt<0>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const unsigned char* cur = ring + (s & 1) * C::STAGE;
+        u32x4 af[CH / 2][C::TM], bf[CH / 2][C::TN];
+        i16x4 tr[TR && C::ES == 2 ? CH * C::TN : 4];
+#pragma unroll
+        for (int kk = 0; kk < CH / 2; ++kk) {
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i) af[kk][i] = *(const u32x4*)(cur + a_frag[kk][i]);
+#pragma unroll
+            for (int j = 0; j < C::TN; ++j) {
+                if constexpr (TR && C::ES == 2) {       // (K rows 4 apart share a key)
+                    tr[(kk * C::TN + j) * 2] = lds_read_tr16(cur + b_frag[kk][j]);
+                    tr[(kk * C::TN + j) * 2 + 1] = lds_read_tr16(cur + b_frag[kk][j] + 4 * C::TCH * 16);
+                } else if constexpr (TR) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) bf[kk][j][e] = *(const uint32_t*)(cur + b_frag[kk][j] + e * C::TCH * 16);
+                } else {
+                    bf[kk][j] = *(const u32x4*)(cur + b_frag[kk][j]);
+                }
+            }
+        }
+        if constexpr (TR && C::ES == 2) {
+            lds_wait_all(tr);
+#pragma unroll
+            for (int kk = 0; kk < CH / 2; ++kk)
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j)
+                    bf[kk][j] = __builtin_bit_cast(u32x4, __builtin_shufflevector(tr[(kk * C::TN + j) * 2], tr[(kk * C::TN + j) * 2 + 1], 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+        if (s + 2 < slabs) {
+            // every wavefront's fragments are in registers before the stage is written again
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            issue(s + 2);
+        }
+#pragma unroll
+        for (int kk = 0; kk < CH / 2; ++kk)
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j) mma<Tag>(acc[i][j], bf[kk][j], af[kk][i]);      // transposed tile
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();           // the ring is reused below
+    asm volatile("" ::: "memory");
+
+    // element e of lane l: pair l % 32, column 8 * (e / 4) + 4 * (l / 32) + e % 4.  Through the wavefront's band in LDS, out as 16-byte
+    // pieces of 256 bytes a pair.
+    unsigned char* band = ring + wave * 32 * C::PITCH;
+    constexpr int QUADS = C::WN / 4;            // 16-byte pieces of a band row
+#pragma unroll
+    for (int i = 0; i < C::TM; ++i) {
+#pragma unroll
+        for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 four = {acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
+                *(f32x4*)(band + l32 * C::PITCH + (j * 32 + q * 8 + g * 4) * 4) = four;
+            }
+        // (written and read by the same wavefront: program order suffices)
+#pragma unroll
+        for (int pass = 0; pass < 32 * QUADS / 64; ++pass) {
+            const int r = (pass * 64 + lane) / QUADS, quad = (pass * 64 + lane) % QUADS, col = col0 + wave_n * C::WN + quad * 4;
+            const uint32_t row = (uint32_t)(wave_m * C::WM + i * 32 + r);
+            if (row < live && col < cols) *(f32x4*)(partial + (pair0 + row) * cols + col) = *(const f32x4*)(band + r * C::PITCH + quad * 16);
+        }
+    }
+}
+
+// out[r] = act(sum over the offsets of row r, in order, of its partial sums + bias): tpr = min(cols / 4, 256) threads a row, four columns
+// each, four partial sums in flight.  It waits for memory: 45 MB
+// of sums in 9.5 us (4.7 TB/s).
+template <typename T>
+__global__ void __launch_bounds__(256) pair_reduce_kernel(const float* __restrict__ partial, const uint32_t* __restrict__ plan, uint32_t n, int cols,
+                                                          int V, const T* __restrict__ bias, int act, T* __restrict__ out,
+                                                          uint8_t* __restrict__ relu_mask) {
+    using Out = T __attribute__((ext_vector_type(4)));
+    __shared__ uint32_t pair_of[256 / 8][kPairMaxV];
+    __shared__ int pairs[256 / 8];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int quads = cols / 4, tpr = quads < 256 ? quads : 256;
+    const int rows = 256 / tpr < 32 ? 256 / tpr : 32;
+    uint32_t pairs_to, tiles_to, count;
+    scan_counts(plan, V, lane, pairs_to, tiles_to, count);
+    const uint32_t* place = plan + pair_place_at();
+    const uint32_t r0 = blockIdx.x * (uint32_t)rows;
+    for (int i = wave; i < rows; i += 4) {
+        const uint32_t at = r0 + i < n && lane < V ? place[(size_t)(r0 + i) * V + lane] : FGX_EMPTY32;
+        const unsigned long long have = __ballot(at != FGX_EMPTY32);
+        if (at != FGX_EMPTY32) pair_of[i][__popcll(have & ((1ull << lane) - 1ull))] = pairs_to - count + at;
+        if (lane == 0) pairs[i] = __popcll(have);
+    }
+    __syncthreads();
+    const int mine = (int)threadIdx.x / tpr;
+    const uint32_t r = r0 + mine;
+    if (mine >= rows || r >= n) return;
+    const int m = pairs[mine];
+    const f32x4* from = (const f32x4*)partial;
+    for (int c = (int)threadIdx.x % tpr; c < quads; c += tpr) {
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        int u = 0;
+        for (; u + 4 <= m; u += 4) {
+            f32x4 x[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) x[q] = from[(size_t)pair_of[mine][u + q] * quads + c];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) s += x[q];
+        }
+        for (; u < m; ++u) s += from[(size_t)pair_of[mine][u] * quads + c];
+        Out rounded;
+        uint32_t bits = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float bv = bias != nullptr ? to_float<T>(bias[c * 4 + e]) : 0.f;
+            rounded[e] = from_float<T>(activate(s[e] + bv, act));
+            bits |= (uint32_t)(to_float<T>(rounded[e]) > 0.f) << e;
+        }
+        const size_t i = (size_t)r * quads + c;
+        ((Out*)out)[i] = rounded;
+        if (relu_mask != nullptr) {
+            const uint32_t other = (uint32_t)__shfl_xor((int)bits, 1, 64);
+            if ((i & 1) == 0) relu_mask[i >> 1] = (uint8_t)(bits | other << 4);
+        }
+    }
+}
+
+size_t most_tiles(size_t n, int V) { return (size_t)V * cdiv(n, kPairRows); }
+
+template <typename Tag, bool TR, int BN, int WAVES_M>
+int launch_gemm(const void* src, const PairWeight& b, const uint32_t* plan, size_t n, size_t n_src, int K, int cols, int V, float* partial, hipStream_t s) {
+    using C = PairCfg<Tag, TR, BN, WAVES_M>;
+    using T = typename Tag::type;
+    const unsigned grid = cdiv(most_tiles(n, V) * cdiv(cols, BN), kXcds) * kXcds;
+    pair_gemm_kernel<Tag, TR, BN, WAVES_M><<<grid, C::NT, C::lds_bytes, s>>>((const T*)src, b, plan, (uint32_t)n, K, cols, V,
+                                                                   (uint32_t)(n_src * (size_t)K * sizeof(T)), partial);
+    FGX_CHECK_LAUNCH("fgx_conv_gemm_pairs");
+    return FGX_OK;
+}
+
+template <typename Tag, bool TR>
+int launch_pairs(const void* src, const PairWeight& b, const void* bias, const uint32_t* plan, size_t n, size_t n_src, int K, int cols, int V,
+                 float* partial, int act, void* out, uint8_t* relu_mask, hipStream_t s) {
+    using T = typename Tag::type;
+    // Columns of a tile.  fp32 is bound by what it multiplies: 96 where that pads less, else 64, whose smaller pieces even out better (96
+    // channels, 38 407 voxels 0.140 ms, 64 columns 0.165; 512 channels, 3 758 voxels 0.244, 128 columns 0.260).  16-bit types load half as much per product
+    // with 128: those unless they pad by a sixth or leave CUs without a tile (864 voxels: 256 channels 64 columns 16.4 us, 128 16.8; 288 channels
+    // 18.1 and 19.3; 512 channels 24.5 and 22.9; 3 758 voxels, 1024 channels 217 and 177).
+    int rc;
+    if constexpr (sizeof(T) == 4) {
+        rc = cdiv(cols, 96) * 96 < cdiv(cols, 64) * 64 ? launch_gemm<Tag, TR, 96, 4>(src, b, plan, n, n_src, K, cols, V, partial, s)
+                                                       : launch_gemm<Tag, TR, 64, 2>(src, b, plan, n, n_src, K, cols, V, partial, s);
+    } else {
+        const size_t tiles = (size_t)V * cdiv(n * 9, 20 * kPairRows) * cdiv(cols, 128);     // (a little under half of a row's offsets exist)
+        const bool narrow = tiles < 224 || cdiv(cols, 128) * 128 * 6 > cdiv(cols, 64) * 64 * 7;
+        rc = narrow ? launch_gemm<Tag, TR, 64, 2>(src, b, plan, n, n_src, K, cols, V, partial, s)
+                    : launch_gemm<Tag, TR, 128, 2>(src, b, plan, n, n_src, K, cols, V, partial, s);
+    }
+    if (rc != FGX_OK) return rc;
+    const int quads = cols / 4, tpr = quads < 256 ? quads : 256, rows = 256 / tpr < 32 ? 256 / tpr : 32;
+    pair_reduce_kernel<T><<<cdiv(n, rows), 256, 0, s>>>(partial, plan, (uint32_t)n, cols, V, (const T*)bias, act, (T*)out, relu_mask);
+    FGX_CHECK_LAUNCH("fgx_conv_gemm_pairs(sums)");
+    return FGX_OK;
+}
+
+}  // namespace
+}  // namespace fgx
+
+using namespace fgx;
+
+extern "C" {
+
+// Where the products of the pairs and their sums are ahead of the masked kernels (all per call, ms; the plan takes 4 to 13 us, once per
+// map, in the place of tile masks or a gather plan).
+// 16-bit, up to 9 000 rows, where the streaming kernel takes over (864 voxels: C = 1024 0.083 -> 0.053, 512 0.034 -> 0.023, 256 0.025 -> 0.016,
+// 128 0.0146 -> 0.0116;  2 047 voxels: 1024 0.134 -> 0.102, 256 0.031 -> 0.024, 128 0.0195 -> 0.0160;  3 758: 1024 0.236 -> 0.177, 512 0.076 ->
+// 0.064, 128 0.0246 and 0.0232;  8 589: 512 0.180 -> 0.140, 256 0.067 -> 0.057;  11 813: 512 0.148 and 0.205).  The sums are
+// traffic per output column, so a short row pays up to fewer voxels (8 589 voxels: 256 -> 64 channels 0.038 -> 0.024, 64 -> 256 0.028 and 0.045), as
+// do the widest layers, whose sums outgrow the memory-side cache first (5 914 voxels, C = 1024: 0.296 and 0.290).
+// fp32 multiplies a sixteenth as fast, and what is not multiplied counts for more (864 voxels: 1024 0.52 -> 0.24, 256 0.058 -> 0.031, 64 0.016 ->
+// 0.012;  8 589: 256 0.34 -> 0.155, 128 0.095 -> 0.057;  15 467: 512 1.37 -> 0.92, 96 0.110 -> 0.067, 64 0.056 -> 0.041;  38 407: 256 0.97 -> 0.68, 160 0.42 -> 0.36,
+// 96 0.156 -> 0.142, 64 0.091 -> 0.078, 32 0.046 and 0.052;  41 700, 288: 1.01 -> 0.78;  101 586, 192: 0.91 and 0.94).
+// The sums at most 1 GiB at their bound.
+int fgx_conv_gemm_pairs_pays(int dtype, int mode, size_t n, int Ci, int Co, int V) {
+    if (mode < 0 || mode > 2 || V < 1 || V > kPairMaxV || Ci <= 0 || Co <= 0 || n == 0) return 0;
+    const int es = dtype == FGX_F32 ? 4 : 2, K = mode == 0 ? Ci : Co, cols = mode == 0 ? Co : Ci;
+    if (Ci % (16 / es) != 0 || Co % (16 / es) != 0 || (size_t)V * Ci * Co * es >= ((size_t)1 << 31)) return 0;
+    if (n > 65536 || fgx_conv_gemm_pairs_scratch_bytes(n, cols, V) > ((size_t)1 << 30)) return 0;
+    if (es == 4) return K >= 64 ? n <= 45000 : K >= 32 && n <= 4000;
+    if (cols < 64 || cols > 2 * K) return 0;
+    return n <= ((size_t)K * cols >= (size_t)768 * 768 ? 5000u : K >= 256 ? 9000u : K >= 96 ? 2500u : K >= 64 ? 300u : 0u);
+}
+
+size_t fgx_pair_plan_words(size_t n, int V) {
+    return V >= 1 && V <= kPairMaxV ? pair_chunks_at(n, V) + (size_t)cdiv(n, kPairChunk) * kPairMaxV : 0;
+}
+
+int fgx_pair_plan(const uint32_t* map, size_t n, int V, uint32_t* plan, fgx_stream_t stream) {
+    FGX_CHECK_ARG(V >= 1 && V <= kPairMaxV && n < ((size_t)1 << 26), "fgx_pair_plan: %zu rows, V=%d out of range", n, V);
+    FGX_CHECK_ARG(plan != nullptr && (n == 0 || map != nullptr), "fgx_pair_plan: null buffer");
+    if (n <= (size_t)kPairColumnRows) {
+        pair_plan_columns_kernel<<<V, 1024, 0, (hipStream_t)stream>>>(map, (uint32_t)n, V, plan);
+        FGX_CHECK_LAUNCH("fgx_pair_plan");
+        return FGX_OK;
+    }
+    const unsigned chunks = cdiv(n, kPairChunk);
+    const size_t lds = (size_t)kPairChunk * V * sizeof(uint32_t);
+#define FGX_PLAN(VC)                                                                                                                \
+    do {                                                                                                                            \
+        pair_plan_kernel<true, VC><<<chunks, kPairChunk, lds, (hipStream_t)stream>>>(map, (uint32_t)n, V, plan);    \
+        pair_plan_kernel<false, VC><<<chunks, kPairChunk, lds, (hipStream_t)stream>>>(map, (uint32_t)n, V, plan);                   \
+    } while (0)
+    if (V == 27) FGX_PLAN(27);
+    else if (V == 8) FGX_PLAN(8);
+    else FGX_PLAN(0);
+#undef FGX_PLAN
+    FGX_CHECK_LAUNCH("fgx_pair_plan");
+    return FGX_OK;
+}
+
+size_t fgx_conv_gemm_pairs_scratch_bytes(size_t n, int cols, int V) { return n * (size_t)V * (size_t)(cols > 0 ? cols : 0) * sizeof(float); }
+
+int fgx_conv_gemm_pairs(int dtype, int mode, const void* src, const void* weight, const void* bias, const uint32_t* plan, size_t n, size_t n_src,
+                        int Ci, int Co, int V, void* scratch, int activation, void* out, uint8_t* relu_mask, fgx_stream_t stream) {
+    FGX_CHECK_ARG(activation == FGX_ACT_NONE || activation == FGX_ACT_RELU, "fgx_conv_gemm_pairs: unknown activation %d", activation);
+    FGX_CHECK_ARG(dtype == FGX_F16 || dtype == FGX_BF16 || dtype == FGX_F32, "fgx_conv_gemm_pairs: unknown dtype %d", dtype);
+    FGX_CHECK_ARG(mode >= 0 && mode <= 2 && V >= 1 && V <= kPairMaxV && Ci > 0 && Co > 0, "fgx_conv_gemm_pairs: bad shape, mode %d Ci=%d Co=%d V=%d",
+                  mode, Ci, Co, V);
+    const int es = dtype == FGX_F32 ? 4 : 2, K = mode == 0 ? Ci : Co, cols = mode == 0 ? Co : Ci;
+    FGX_CHECK_ARG(Ci % (16 / es) == 0 && Co % (16 / es) == 0, "fgx_conv_gemm_pairs: rows of %d and %d elements are not whole 16-byte pieces", Ci, Co);
+    FGX_CHECK_ARG(relu_mask == nullptr || (activation == FGX_ACT_RELU && es == 2), "fgx_conv_gemm_pairs: a ReLU mask needs the ReLU and a 16-bit type");
+    if (n == 0) return FGX_OK;
+    FGX_CHECK_ARG(src && weight && plan && scratch && out, "fgx_conv_gemm_pairs: null buffer");
+    FGX_CHECK_ARG((((uintptr_t)src | (uintptr_t)weight | (uintptr_t)scratch | (uintptr_t)out) & 15) == 0, "fgx_conv_gemm_pairs: buffers must be 16-byte aligned");
+    const size_t weight_bytes = (size_t)V * Ci * Co * es, src_bytes = n_src * (size_t)K * es;
+    FGX_CHECK_ARG(weight_bytes < ((size_t)1 << 31) && src_bytes <= kOobOffset && n * (size_t)V < 0xFFFFFFFFull && n < 0x7FFFFFFFull &&
+                      most_tiles(n, V) * cdiv(cols, 64) < 0x7FFFFFF0ull,
+                  "fgx_conv_gemm_pairs: an operand exceeds the 32-bit offset range");
+    PairWeight b;                                           // [Co][V][Ci]
+    b.base = (const unsigned char*)weight;
+    b.bytes = (uint32_t)weight_bytes;
+    b.v_stride = (uint32_t)(Ci * es);
+    b.line_stride = (uint32_t)((size_t)V * Ci * es);
+    b.slab_stride = mode == 0 ? 128u : (uint32_t)(128 / es) * b.line_stride;
+    b.mirrored = mode == 1;
+    hipStream_t s = (hipStream_t)stream;
+#define FGX_PAIRS(Tag)                                                                                                                              \
+    return mode == 0 ? launch_pairs<Tag, false>(src, b, bias, plan, n, n_src, K, cols, V, (float*)scratch, activation, out, relu_mask, s)           \
+                     : launch_pairs<Tag, true>(src, b, bias, plan, n, n_src, K, cols, V, (float*)scratch, activation, out, relu_mask, s)
+    if (dtype == FGX_F16) FGX_PAIRS(F16);
+    if (dtype == FGX_BF16) FGX_PAIRS(BF16);
+    FGX_PAIRS(F32);
+#undef FGX_PAIRS
+}
+
+}  // extern "C"

@@ -40,7 +40,7 @@ namespace {
     X(fgx_spconv_out_dims) X(fgx_spconv_out_coords_grid_workspace_bytes) X(fgx_spconv_out_coords_grid_count)                       \
     X(fgx_spconv_out_coords_grid_emit) X(fgx_tile_plan) X(fgx_gather_item_order) X(fgx_gather_item_order_workspace_bytes)          \
     X(fgx_weight_panel_bytes) X(fgx_pack_weight) X(fgx_conv_scratch_bytes) X(fgx_conv_gather_gemm_act_mask)                        \
-    X(fgx_conv_gather_gemm_weight_pays) X(fgx_conv_gather_gemm_weight)                                                             \
+    X(fgx_conv_gather_gemm_weight_pays) X(fgx_conv_gather_gemm_weight) X(fgx_conv_gemm_pairs_pays) X(fgx_pair_plan_words) X(fgx_pair_plan) X(fgx_conv_gemm_pairs_scratch_bytes) X(fgx_conv_gemm_pairs)                                                             \
     X(fgx_conv_gather_gemm_stream_act_mask) X(fgx_conv_gather_gemm_stream_groups) X(fgx_relu_mask_apply)                           \
     X(fgx_colsum_scratch_bytes) X(fgx_colsum) X(fgx_wgrad_block_bounds_count) X(fgx_wgrad_block_bounds)                            \
     X(fgx_conv_gemm_stem_pays) X(fgx_conv_gemm_stem) X(fgx_wgrad_stem_pays) X(fgx_wgrad_stem_scratch_bytes) X(fgx_conv_wgrad_stem) X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
@@ -594,6 +594,27 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
         mark(name, "start");
         check(L.fgx_conv_gemm_stem(code, mode, ptr(src), ptr(weight), ptr(bias), ptr<uint32_t>(nmap), (size_t)n, ci, co, v, activation, ptr(p.out),
                                    ptr<uint8_t>(p.mask), as_stream(stream)));
+        mark(name, "stop");
+        return p;
+    }
+    // few voxels under a wide weight: the pairs' products and their sums, from a plan of the map that every layer on it shares (none is made
+    // inside a capture, which would hold it)
+    if (masked && allow_splitk && n > 0 && !narrow && !panel_kept.defined() && L.fgx_conv_gemm_pairs_pays(code, mode, (size_t)n, ci, co, v) &&
+        schedules_are_ours() && aligned(src) && aligned(weight) && (double)n_src * row_bytes <= (double)0xFF000000u &&
+        (c.has("_pair_plan") || !capturing(stream))) {
+        Tensor plan;
+        if (!c.tensor("_pair_plan", &plan)) {
+            plan = make({(int64_t)L.fgx_pair_plan_words((size_t)n, v)}, at::kUInt32, dev);
+            check(L.fgx_pair_plan(ptr<uint32_t>(nmap), (size_t)n, v, ptr<uint32_t>(plan), as_stream(stream)));
+            c.set("_pair_plan", plan);
+        }
+        Tensor scratch = workspace(L.fgx_conv_gemm_pairs_scratch_bytes((size_t)n, cols, v), dev);
+        p.out = make({n, cols}, src.scalar_type(), dev);
+        if (want_mask && activation == FGX_ACT_RELU && es == 2) p.mask = make({n * cols / 8}, at::kByte, dev);
+        const char* name = mode == 0 ? "gather_gemm_fwd" : "gather_gemm_dgrad";
+        mark(name, "start");
+        check(L.fgx_conv_gemm_pairs(code, mode, ptr(src), ptr(weight), ptr(bias), ptr<uint32_t>(plan), (size_t)n, (size_t)n_src, ci, co, v, ptr(scratch),
+                                    activation, ptr(p.out), ptr<uint8_t>(p.mask), as_stream(stream)));
         mark(name, "stop");
         return p;
     }

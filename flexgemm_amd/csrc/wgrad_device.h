@@ -39,6 +39,7 @@ constexpr int kItemListHeader = 4;
 
 #define FGX_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 #define FGX_GLOBAL_PTR(p) ((const __attribute__((address_space(1))) void*)(p))
+#define FGX_CONST_PTR(p) ((const __attribute__((address_space(4))) uint32_t*)(uintptr_t)(p))      // words no launch in flight writes
 
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {

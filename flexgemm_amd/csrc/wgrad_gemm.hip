@@ -389,12 +389,16 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
     if (lists) lists += kItemListHeader;
     const unsigned range_end = lists ? total_items : ((xcd + 1) * per_xcd < total_items ? (xcd + 1) * per_xcd : total_items);
     const uint32_t* chain = lists ? lists + gridDim.x : nullptr;
-    auto after = [&](unsigned item) -> unsigned { return chain ? chain[item] : item + stride; };
+    // (through the scalar cache: as a vector load, which the compiler picks because of the loads into LDS in between, the next
+    // link would be waited for with every row load that is in flight)
+    auto after = [&](unsigned item) -> unsigned {
+        return chain ? *(FGX_CONST_PTR(chain) + __builtin_amdgcn_readfirstlane(item)) : item + stride;
+    };
 
     struct Walk {
         unsigned item;
         uint32_t k, k_hi;       // next pair to hand out, end of the item's pairs
-        unsigned b, v, tile;
+        unsigned b, v, co_tile, ci_tile;
         bool live;
     };
     auto seek = [&](Walk& w) {                      // settle on the first non-empty item at or after w.item
@@ -408,7 +412,9 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
                 w.k_hi = hi;
                 w.b = b;
                 w.v = v;
-                w.tile = within % tiles;
+                const unsigned tile = within % tiles;
+                w.co_tile = tile % co_tiles;
+                w.ci_tile = tile / co_tiles;
                 w.live = true;
                 return;
             }
@@ -450,7 +456,7 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
             b_chb[i] = (uint32_t)(((lane % C::CH_B) ^ C::key_b(b_row[i])) * 16);
         }
         Walk f = first, r = first;                  // index stream, row stream
-        unsigned f_step = 0, r_step = 0;            // steps handed out so far (ring positions)
+        unsigned f_step = 0, r_step = 0, r_stage = 0;       // steps handed out so far (index ring positions), row ring position
         auto issue_idx = [&]() -> int {             // index loads of the index stream's next step
             if (!f.live) return 0;
             int ops = 0;
@@ -486,10 +492,10 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
         auto prep_rows = [&]() {
             pr_live = r.live;
             if (!r.live) return;
-            pr_stage = r_step % S;
+            pr_stage = r_stage;
+            r_stage = r_stage + 1 == S ? 0 : r_stage + 1;
             const uint32_t* slot_p = idx_ring + (r_step & (kWsIdxSlots - 1)) * (2 * P);
-            const unsigned co_tile = r.tile % co_tiles, ci_tile = r.tile / co_tiles;
-            const uint32_t m0b = co_tile * (uint32_t)(BM * ES), n0b = ci_tile * (uint32_t)(BN * ES);
+            const uint32_t m0b = r.co_tile * (uint32_t)(BM * ES), n0b = r.ci_tile * (uint32_t)(BN * ES);
             const uint32_t left = r.k_hi - r.k;                                   // pairs left in the item
             const bool ragged = left < (uint32_t)P || m0b + BM * ES > rowb_o || n0b + BN * ES > rowb_i;   // uniform
 #pragma unroll
@@ -600,9 +606,9 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
     const uint32_t ring_addr = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)ring;
     constexpr int RK = 2 * (C::TM + C::TN);         // LDS reads per k-block
     Walk m = first;
-    unsigned step = 0;
+    uint32_t stage_at = ring_addr;
     while (m.live) {
-        const unsigned b = m.b, v = m.v, tile = m.tile;
+        const unsigned b = m.b, v = m.v;
         const int nsteps = (int)((m.k_hi - m.k + P - 1) / P);
         f32x16 acc[C::TM][C::TN];
 #pragma unroll
@@ -615,7 +621,7 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
         // the grad_out fragments are multiplied by a fragment of ones as well, so every column of bacc is the sum.  Only
         // the wavefronts of the first column of wave tiles do it, for the first Ci-tile.
         // (not with 128 x 64 or 64 x 128 wave tiles: the extra accumulators do not fit the register budget; the host then sums apart)
-        const bool do_bias = C::TM * C::TN <= 4 && bias_partial != nullptr && (int)v == bias_offset && wave_n == 0 && tile < co_tiles;
+        const bool do_bias = C::TM * C::TN <= 4 && bias_partial != nullptr && (int)v == bias_offset && wave_n == 0 && m.ci_tile == 0;
         f32x16 bacc[C::TM];
 #pragma unroll
         for (int i = 0; i < C::TM; ++i)
@@ -628,8 +634,8 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
                 asm volatile("" ::: "memory");
                 __builtin_amdgcn_s_barrier();           // the loaders saw this step's rows land
                 asm volatile("" ::: "memory");
-                const uint32_t cur = ring_addr + (step % S) * (uint32_t)C::STAGE_BYTES;
-                ++step;
+                const uint32_t cur = stage_at;
+                stage_at = cur == ring_addr + (S - 1) * (uint32_t)C::STAGE_BYTES ? ring_addr : cur + (uint32_t)C::STAGE_BYTES;
                 // Transposing read: in a 16-lane group, lane s supplies the address of 4 adjacent channels of pair row
                 // (s / 4) and receives the 4 pair values of channel (group base + s).  Lanes 0-15 / 16-31 cover fragment
                 // rows 0-15 / 16-31, the two wave halves take pair rows [0, 8) / [8, 16) of the k-block.  The reads of
@@ -687,8 +693,7 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
         // whole lines of an output row side by side.  (Stored element by element the tile took 64 address computations, conversions and
         // 64-byte stores of a wavefront that has its SIMD's matrix unit to itself, longer than the products of an item of few
         // pairs: 864 voxels x 1024 channels, 1728 items of 6 steps, 77 -> 50 us.)
-        const unsigned co_tile = tile % co_tiles, ci_tile = tile / co_tiles;
-        const int m0 = (int)co_tile * BM, n0 = (int)ci_tile * BN;
+        const int m0 = (int)m.co_tile * BM, n0 = (int)m.ci_tile * BN;
         auto write_tile = [&](auto* dst, size_t row_stride, bool pieces_ok) {
             using O = std::remove_pointer_t<decltype(dst)>;
             using O4 = O __attribute__((ext_vector_type(4)));

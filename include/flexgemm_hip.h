@@ -292,6 +292,20 @@ int fgx_conv_gather_gemm_weight(int dtype, int mode, const void* src, const void
                                 const uint32_t* map, const int64_t* sorted_idx, const int32_t* tile_code, size_t n,
                                 int Ci, int Co, int V, int tile_rows, int tile_cols, int slab_bytes, int splitk,
                                 void* scratch, int activation, void* out, uint8_t* relu_mask, fgx_stream_t stream);
+
+/* Few voxels under a wide weight (conv_gemm_pairs.hip): the products offset by offset over the pairs that exist, their fp32 sums
+ * added per output row in offset order.  fgx_pair_plan lists the pairs of a map [n][V], V <= 32, into plan[fgx_pair_plan_words]; a plan serves
+ * every layer on the map.  weight [Co][V][Ci] and mode as in fgx_conv_gather_gemm_weight (all types, all modes); Ci and Co whole 16-byte
+ * pieces, the weight under 2 GiB, src under 4 GB; src, weight, scratch and out 16-byte aligned.  scratch:
+ * fgx_conv_gemm_pairs_scratch_bytes (only the sums of existing pairs are written).  fgx_conv_gemm_pairs_pays: whether the operators take it. */
+int fgx_conv_gemm_pairs_pays(int dtype, int mode, size_t n, int Ci, int Co, int V);
+size_t fgx_pair_plan_words(size_t n, int V);
+int fgx_pair_plan(const uint32_t* map, size_t n, int V, uint32_t* plan, fgx_stream_t stream);
+size_t fgx_conv_gemm_pairs_scratch_bytes(size_t n, int cols, int V);
+int fgx_conv_gemm_pairs(int dtype, int mode, const void* src, const void* weight, const void* bias, const uint32_t* plan,
+                        size_t n, size_t n_src, int Ci, int Co, int V, void* scratch, int activation, void* out,
+                        uint8_t* relu_mask, fgx_stream_t stream);
+
 /* out[i] = bit i of relu_mask ? grad[i] : 0 for i < numel (a multiple of 8; 16-bit types; grad and out 16-byte aligned,
  * out may be grad): the gradient of a fused ReLU from the mask its forward pass wrote.  One pass, numel / 8 bytes of mask
  * read beside the gradient.  No counterpart in the reference. */

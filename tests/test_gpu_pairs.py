@@ -1,0 +1,122 @@
+"""The gather GEMM over pairs (conv_gemm_pairs.hip): its plan against the map, its products against the definition in 64 bits, at
+the edges of its tiles and of what takes it."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import flex_gemm
+from flexgemm_amd import _native as nat
+from flexgemm_amd.workloads import reference_test_shell
+
+spconv = flex_gemm.ops.spconv
+pytestmark = pytest.mark.gpu
+EMPTY = 0xFFFFFFFF
+
+
+def _plan(nmap):
+    n, v = nmap.shape
+    plan = torch.full((nat.lib().fgx_pair_plan_words(nat.sz(n), C.c_int(v)),), 0x55555555, dtype=torch.int32, device=nmap.device)
+    nat.check(nat.lib().fgx_pair_plan(nat.ptr(nmap), nat.sz(n), C.c_int(v), nat.ptr(plan), nat.stream()))
+    return plan
+
+
+def _map(n, n_src, v, density, seed):
+    """A random map; offset 0 holds every row, the last offset (of several) none."""
+    rng = np.random.default_rng(seed)
+    m = rng.integers(0, n_src, size=(n, v), dtype=np.uint32)
+    m[rng.random((n, v)) >= density] = EMPTY
+    m[:, 0] = rng.integers(0, n_src, size=n)
+    if v > 1:
+        m[:, -1] = EMPTY
+    return m
+
+
+@pytest.mark.parametrize("n,v", [(1, 1), (1, 27), (63, 8), (1024, 27), (1025, 32), (4096, 27), (4097, 27), (66000, 27), (300000, 2), (5000, 8), (5000, 32)])
+def test_plan_lists_the_pairs_in_row_order(gpu_device, n, v):
+    m = _map(n, n, v, 0.4, n + v)
+    plan = _plan(torch.from_numpy(m.view(np.int32)).view(torch.uint32).to(gpu_device)).cpu().numpy().view(np.uint32)
+    counts, place, rows = plan[:32], plan[32:32 + n * v].reshape(n, v), plan[32 + n * v:32 + 2 * n * v].reshape(v, n)
+    for o in range(v):
+        have = np.flatnonzero(m[:, o] != EMPTY)
+        assert counts[o] == len(have)
+        assert np.array_equal(rows[o, :len(have)], m[have, o]) and np.array_equal(place[have, o], np.arange(len(have)))
+        assert (place[m[:, o] == EMPTY, o] == EMPTY).all()
+
+
+# 1 ... 129 pairs: one tile and a tile of one pair more; channels of one 16-byte piece, ending inside a slab, a tile, a 32-column block and
+# on their edges; one offset, 27, the most
+@pytest.mark.parametrize("n,n_src,v", [(1, 3, 1), (127, 50, 27), (128, 200, 8), (129, 129, 27), (700, 300, 32), (2600, 2600, 27)])
+@pytest.mark.parametrize("ci,co", [(8, 8), (64, 64), (72, 136), (264, 96), (128, 200), (40, 296)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_products_match_the_definition(gpu_device, n, n_src, v, ci, co, dtype):
+    print(f"[case] n={n} n_src={n_src} v={v} {ci}->{co} {dtype}", flush=True)
+    gen = torch.Generator(device=gpu_device).manual_seed(n + ci)
+    m = torch.from_numpy(_map(n, n_src, v, 0.45, n).view(np.int32)).to(gpu_device)
+    plan = _plan(m.view(torch.uint32))
+    L = nat.lib()
+    room = torch.full((co * v * ci + 4096,), float("nan"), dtype=dtype, device=gpu_device)      # what lies around the weight must not matter
+    weight = room[2048:2048 + co * v * ci].view(co, v, ci)
+    weight.copy_(torch.randn(co, v, ci, generator=gen, device=gpu_device) / 8)
+    for mode in (0, 1, 2):
+        k, cols = (ci, co) if mode == 0 else (co, ci)
+        src = torch.randn(n_src, k, generator=gen, device=gpu_device).to(dtype)
+        bias = torch.randn(cols, generator=gen, device=gpu_device).to(dtype) if mode == 0 else None
+        relu = mode == 0 and dtype != torch.float32
+        out = torch.full((n, cols), float("nan"), dtype=dtype, device=gpu_device)
+        mask = torch.zeros((n * cols // 8,), dtype=torch.uint8, device=gpu_device) if relu else None
+        scratch = torch.full((L.fgx_conv_gemm_pairs_scratch_bytes(nat.sz(n), C.c_int(cols), C.c_int(v)) // 4,), float("nan"), device=gpu_device)
+        nat.check(L.fgx_conv_gemm_pairs(C.c_int(nat.DTYPE_CODE[dtype]), C.c_int(mode), nat.ptr(src), nat.ptr(weight), nat.ptr(bias), nat.ptr(plan), nat.sz(n),
+                                        nat.sz(n_src), C.c_int(ci), C.c_int(co), C.c_int(v), nat.ptr(scratch), C.c_int(1 if relu else 0), nat.ptr(out),
+                                        nat.ptr(mask), nat.stream()))
+        want = torch.zeros(n, cols, dtype=torch.float64, device=gpu_device)
+        size = torch.zeros_like(want)           # sum of the magnitudes that are added
+        for o in range(v):
+            have = (m[:, o] != -1).nonzero()[:, 0]
+            if not len(have):
+                continue
+            w = (weight[:, o] if mode == 0 else weight[:, v - 1 - o if mode == 1 else o].T).double().T.contiguous()
+            rows = src[m[have, o].long()].double()
+            want[have] += rows @ w
+            size[have] += rows.abs() @ w.abs()
+        if bias is not None:
+            want += bias.double()
+            size += bias.double().abs()
+        if relu:
+            want = want.clamp(min=0)
+        # one rounding to the result's type, and at most (K + V) roundings of the running sums to 24 bits
+        unit = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}[dtype]
+        bound = unit * want.abs() + (k + v) * 2.0 ** -24 * size + 1e-7
+        assert ((out.double() - want).abs() <= bound).all(), mode
+        if relu:
+            bits = (out > 0).view(-1, 8).to(torch.int32)
+            assert torch.equal(mask.to(torch.int32), (bits << torch.arange(8, device=gpu_device, dtype=torch.int32)).sum(1).to(torch.int32))
+
+
+@pytest.mark.parametrize("dtype,c", [(torch.float16, 128), (torch.float32, 64)])
+def test_operator_takes_it_and_agrees_with_the_masked_kernels(gpu_device, monkeypatch, dtype, c):
+    """One plan per map, shared by all layers and both directions; a capture before there is one runs the masked kernels."""
+    gen = torch.Generator(device=gpu_device).manual_seed(5)
+    coords = torch.from_numpy(reference_test_shell(16)).to(gpu_device)
+    n = coords.shape[0]
+    assert nat.lib().fgx_conv_gemm_pairs_pays(C.c_int(nat.DTYPE_CODE[dtype]), C.c_int(0), nat.sz(n), C.c_int(c), C.c_int(c), C.c_int(27))
+    shape = torch.Size([1, c, 16, 16, 16])
+    weight = (torch.randn(c, 3, 3, 3, c, generator=gen, device=gpu_device) / 50).to(dtype).requires_grad_(True)
+    feats = torch.randn(n, c, generator=gen, device=gpu_device).to(dtype).requires_grad_(True)
+
+    def step():
+        out, cache = spconv.sparse_submanifold_conv3d(feats, coords, shape, weight, None, None)
+        return out, torch.autograd.grad(out, feats, torch.ones_like(out))[0], cache
+
+    out, grad, cache = step()
+    plan = cache.__dict__["_pair_plan"]
+    again, _ = spconv.sparse_submanifold_conv3d(feats, coords, shape, weight, None, cache)
+    assert cache.__dict__["_pair_plan"] is plan and torch.equal(out, again)
+    real = nat.table_lookup
+    monkeypatch.setattr(nat, "table_lookup", lambda *a, **k: real(*a, **k))         # (a table of the caller's keeps every shape on it)
+    want, want_grad, masked_cache = step()
+    assert "_pair_plan" not in masked_cache.__dict__
+    unit = {torch.float16: 2.0 ** -10, torch.float32: 1e-5}[dtype]
+    for a, b in ((out, want), (grad, want_grad)):
+        assert (a - b).abs().max() <= unit * b.abs().max()
