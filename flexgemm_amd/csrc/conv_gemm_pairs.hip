@@ -476,25 +476,26 @@ using namespace fgx;
 
 extern "C" {
 
-// Where the products of the pairs and their sums are ahead of the masked kernels (all per call, ms; the plan takes 4 to 13 us, once per
-// map, in the place of tile masks or a gather plan).
-// 16-bit, up to 9 000 rows, where the streaming kernel takes over (864 voxels: C = 1024 0.083 -> 0.053, 512 0.034 -> 0.023, 256 0.025 -> 0.016,
-// 128 0.0146 -> 0.0116;  2 047 voxels: 1024 0.134 -> 0.102, 256 0.031 -> 0.024, 128 0.0195 -> 0.0160;  3 758: 1024 0.236 -> 0.177, 512 0.076 ->
-// 0.064, 128 0.0246 and 0.0232;  8 589: 512 0.180 -> 0.140, 256 0.067 -> 0.057;  11 813: 512 0.148 and 0.205).  The sums are
-// traffic per output column, so a short row pays up to fewer voxels (8 589 voxels: 256 -> 64 channels 0.038 -> 0.024, 64 -> 256 0.028 and 0.045), as
-// do the widest layers, whose sums outgrow the memory-side cache first (5 914 voxels, C = 1024: 0.296 and 0.290).
+// Where the products of the pairs and their sums are ahead of the masked kernels by more than a plan used once costs (4 us for 864 rows, 8 for
+// 3 758, 13 for 38 407, of which the tile masks or gather plan that it replaces take 3 to 15).  ms per call:
+// 16-bit, up to 6 500 rows, from where on the tiles pad less and the streaming kernel sets in (864 voxels: C = 1024 0.083 -> 0.053, 512 0.034 ->
+// 0.023, 256 0.025 -> 0.016, but 128 0.0146 -> 0.0116;  2 047 voxels: 1024 0.134 -> 0.102, 256 0.031 -> 0.024;  3 758: 1024 0.236 -> 0.177, 512
+// 0.076 -> 0.064;  training steps of four layers, 512 channels: 5 914 voxels 1.40 -> 1.20, 7 840 voxels 1.48 -> 1.52).  The sums are traffic per
+// output column, so rows that are short beside the outputs do not pay (8 589 voxels: 256 -> 64 channels 0.038 -> 0.024, 64 -> 256 0.028 -> 0.045), and the
+// widest layers, whose sums outgrow the memory-side cache first, only up to 5 000 (5 914 voxels, C = 1024: 0.296 and 0.290).
 // fp32 multiplies a sixteenth as fast, and what is not multiplied counts for more (864 voxels: 1024 0.52 -> 0.24, 256 0.058 -> 0.031, 64 0.016 ->
 // 0.012;  8 589: 256 0.34 -> 0.155, 128 0.095 -> 0.057;  15 467: 512 1.37 -> 0.92, 96 0.110 -> 0.067, 64 0.056 -> 0.041;  38 407: 256 0.97 -> 0.68, 160 0.42 -> 0.36,
-// 96 0.156 -> 0.142, 64 0.091 -> 0.078, 32 0.046 and 0.052;  41 700, 288: 1.01 -> 0.78;  101 586, 192: 0.91 and 0.94).
+// 96 0.156 -> 0.142, 64 0.091 -> 0.078, 32 0.046 -> 0.052;  41 700, 288: 1.01 -> 0.78;  101 586, 192: 0.91 -> 0.94).
 // The sums at most 1 GiB at their bound.
 int fgx_conv_gemm_pairs_pays(int dtype, int mode, size_t n, int Ci, int Co, int V) {
     if (mode < 0 || mode > 2 || V < 1 || V > kPairMaxV || Ci <= 0 || Co <= 0 || n == 0) return 0;
     const int es = dtype == FGX_F32 ? 4 : 2, K = mode == 0 ? Ci : Co, cols = mode == 0 ? Co : Ci;
     if (Ci % (16 / es) != 0 || Co % (16 / es) != 0 || (size_t)V * Ci * Co * es >= ((size_t)1 << 31)) return 0;
     if (n > 65536 || fgx_conv_gemm_pairs_scratch_bytes(n, cols, V) > ((size_t)1 << 30)) return 0;
-    if (es == 4) return K >= 64 ? n <= 45000 : K >= 32 && n <= 4000;
-    if (cols < 64 || cols > 2 * K) return 0;
-    return n <= ((size_t)K * cols >= (size_t)768 * 768 ? 5000u : K >= 256 ? 9000u : K >= 96 ? 2500u : K >= 64 ? 300u : 0u);
+    if (es == 4) return K >= 64 && n <= 45000;
+    if (K < 256 || cols < 64 || cols > 2 * K) return 0;
+    const size_t area = (size_t)K * cols;
+    return n <= (area >= (size_t)512 * 512 && area < (size_t)768 * 768 ? 6500u : 5000u);
 }
 
 size_t fgx_pair_plan_words(size_t n, int V) {

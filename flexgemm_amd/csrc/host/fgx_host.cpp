@@ -544,9 +544,9 @@ struct Product {
 // map with the offsets mirrored, mode 2: through a map of its own, offsets as they are.  One row per row of the cache's
 // neighbor_map.  masked: mask-sorted schedule (else natural row order, all offsets per tile).  want_mask: also one bit per
 // output, "greater than zero", where the kernels can (ReLU, 16-bit type, a multiple of 8 columns).  panel: a kept weight
-// panel, or undefined to pack one.
+// panel, or undefined to pack one.  pairs: whether the product over pairs may be taken.
 Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, int mode, bool allow_splitk, bool masked, int activation,
-                       bool want_mask, const Tensor& panel_kept, int64_t stream) {
+                       bool want_mask, const Tensor& panel_kept, int64_t stream, bool pairs) {
     const at::Device dev = src.device();
     const c10::DeviceGuard guard(dev);
     const int code = dtype_code(src);
@@ -599,7 +599,7 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
     }
     // few voxels under a wide weight: the pairs' products and their sums, from a plan of the map that every layer on it shares (none is made
     // inside a capture, which would hold it)
-    if (masked && allow_splitk && n > 0 && !narrow && !panel_kept.defined() && L.fgx_conv_gemm_pairs_pays(code, mode, (size_t)n, ci, co, v) &&
+    if (pairs && masked && allow_splitk && n > 0 && !narrow && !panel_kept.defined() && L.fgx_conv_gemm_pairs_pays(code, mode, (size_t)n, ci, co, v) &&
         schedules_are_ours() && aligned(src) && aligned(weight) && (double)n_src * row_bytes <= (double)0xFF000000u &&
         (c.has("_pair_plan") || !capturing(stream))) {
         Tensor plan;
@@ -691,7 +691,7 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
 py::tuple gather_gemm(const Tensor& src, const Tensor& weight, const c10::optional<Tensor>& bias, py::object cache, int mode, bool allow_splitk,
                       bool masked, int activation, bool want_mask, const c10::optional<Tensor>& panel) {
     const Product p = gather_product(src, weight, bias.value_or(Tensor()), Cache(std::move(cache)), mode, allow_splitk, masked, activation, want_mask,
-                                     panel.value_or(Tensor()), stream_of(src));
+                                     panel.value_or(Tensor()), stream_of(src), !want_mask);
     return py::make_tuple(p.out, p.mask.defined() ? py::cast(p.mask) : py::none());
 }
 
@@ -941,13 +941,14 @@ struct ConvBackward : public torch::autograd::Node {
         const int64_t co = w.size(0), kw = w.size(1), kh = w.size(2), kd = w.size(3), ci = w.size(4), v = kw * kh * kd;
         if (need_f) {
             const Tensor wv = w.reshape({co, v, ci});
+            const bool pairs = !relu || f.element_size() == 4 || co >= 256;      // (a plan for input gradients alone: 4 us)
             if (call.generic) {
                 const Cache view(c.obj.attr("_bwd_view")());
                 // mask-sorted walk only where the cache carries the backward order
                 result[0] = gather_product(grad, wv, Tensor(), view, 2, call.splitk, call.masked && view.has("sorted_idx"), FGX_ACT_NONE, false, Tensor(),
-                                           stream).out;
+                                           stream, pairs).out;
             } else {
-                result[0] = gather_product(grad, wv, Tensor(), c, 1, call.splitk, call.masked, FGX_ACT_NONE, false, Tensor(), stream).out;
+                result[0] = gather_product(grad, wv, Tensor(), c, 1, call.splitk, call.masked, FGX_ACT_NONE, false, Tensor(), stream, pairs).out;
             }
         }
         if (need_w) {
@@ -992,12 +993,16 @@ Tensor convolve(const Tensor& feats, py::object cache_obj, const Tensor& weight,
         }
     }
     require(feats.size(0) == expected, std::to_string(feats.size(0)) + " feature rows for a neighbor cache of " + std::to_string(expected) + " voxels");
+    // A 16-bit forward pass that trains through the ReLU keeps the order of sums it has always had: another one rounds an output
+    // differently here and there, and from layer to layer more sums near zero change sides (four layers of 512 channels: gradients 0.7 % off).
+    // So does a narrow one, where the operator with the ReLU and one followed by it agree bit for bit.
+    const bool pairs = !record || feats.element_size() == 4 || (!relu && co >= 128);
     const bool bits = relu && record && PyObject_IsTrue(module_get(g_spconv, "RELU_BIT_MASK"));
     Product p;
     {
         const at::NoGradGuard no_grad;
         p = gather_product(feats, weight.reshape({co, v, ci}), bias, c, 0, splitk, masked, relu ? FGX_ACT_RELU : FGX_ACT_NONE, bits, Tensor(),
-                           stream_of(feats));
+                           stream_of(feats), pairs);
     }
     if (!record) return p.out;
     // (deleteNode: a long chain of layers is taken down without a stack frame per layer)

@@ -94,9 +94,9 @@ def test_products_match_the_definition(gpu_device, n, n_src, v, ci, co, dtype):
             assert torch.equal(mask.to(torch.int32), (bits << torch.arange(8, device=gpu_device, dtype=torch.int32)).sum(1).to(torch.int32))
 
 
-@pytest.mark.parametrize("dtype,c", [(torch.float16, 128), (torch.float32, 64)])
+@pytest.mark.parametrize("dtype,c", [(torch.float16, 256), (torch.float32, 64)])
 def test_operator_takes_it_and_agrees_with_the_masked_kernels(gpu_device, monkeypatch, dtype, c):
-    """One plan per map, shared by all layers and both directions; a capture before there is one runs the masked kernels."""
+    """One plan per map, shared by all layers and both directions."""
     gen = torch.Generator(device=gpu_device).manual_seed(5)
     coords = torch.from_numpy(reference_test_shell(16)).to(gpu_device)
     n = coords.shape[0]
