@@ -50,7 +50,7 @@ EXPORTS = [
     "fgx_serialize_encode", "fgx_serialize_decode", "fgx_serialize_reorder_workspace_bytes",
     "fgx_serialize_reorder_coords",
     "fgx_tile_plan", "fgx_grid_index_pays", "fgx_grid_index_walks", "fgx_subm_neighbor_map_grid_workspace_bytes", "fgx_subm_neighbor_map_grid", "fgx_subm_cache_grid_workspace_bytes",
-    "fgx_subm_cache_build_grid", "fgx_spconv_neighbor_map_grid_workspace_bytes", "fgx_spconv_neighbor_map_grid",
+    "fgx_subm_cache_build_grid", "fgx_cache_post_workspace_bytes", "fgx_cache_post", "fgx_spconv_neighbor_map_grid_workspace_bytes", "fgx_spconv_neighbor_map_grid",
     "fgx_spconv_cache_grid_workspace_bytes", "fgx_spconv_cache_build_grid", "fgx_spconv_out_coords_grid_workspace_bytes",
     "fgx_spconv_out_coords_grid_count", "fgx_spconv_out_coords_grid_emit",
 ]
@@ -107,7 +107,7 @@ def lib() -> C.CDLL:
         L = C.CDLL(_LIB_PATH)
         L.fgx_last_error.restype = C.c_char_p
         for name in ("fgx_sort_workspace_bytes", "fgx_locality_workspace_bytes", "fgx_pair_workspace_bytes", "fgx_tile_workspace_bytes",
-                     "fgx_weight_panel_bytes", "fgx_conv_scratch_bytes", "fgx_wgrad_scratch_bytes", "fgx_pair_plan_words", "fgx_conv_gemm_pairs_scratch_bytes",
+                     "fgx_weight_panel_bytes", "fgx_conv_scratch_bytes", "fgx_wgrad_scratch_bytes", "fgx_pair_plan_words", "fgx_conv_gemm_pairs_scratch_bytes", "fgx_cache_post_workspace_bytes",
                      "fgx_colsum_scratch_bytes", "fgx_spconv_out_coords_workspace_bytes",
                      "fgx_subm_neighbor_map_sorted_workspace_bytes", "fgx_wgrad_block_bounds_count", "fgx_wgrad_item_lists_count", "fgx_narrow_plan_bytes", "fgx_narrow_wgrad_scratch_bytes",
                      "fgx_spconv_neighbor_map_sorted_workspace_bytes", "fgx_serialize_reorder_workspace_bytes",

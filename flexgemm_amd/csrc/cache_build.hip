@@ -49,12 +49,12 @@ CacheLayout cache_layout(size_t n, int key_bits, int Kw, int Kh, int V, int with
     return L;
 }
 
-// The mask sort on `s` and, with_pairs, the pair lists (enqueued by `lists` on the stream it is given) -- beside it on the second
+// The mask sort on `s` (none without sorted_idx) and, with_pairs, the pair lists (enqueued by `lists` on the stream it is given) -- beside it on the second
 // stream for many rows, outside a capture (which would have to own that stream); `s` waits for both.
 template <typename Lists>
 int sort_beside_pairs(size_t n, int V, const int32_t* binary, int64_t* sorted_idx, void* sort_ws, size_t sort_bytes, bool with_pairs,
                       hipStream_t s, const char* who, Lists lists) {
-    bool two_streams = with_pairs && n >= kTwoStreamsMinRows;
+    bool two_streams = with_pairs && sorted_idx != nullptr && n >= kTwoStreamsMinRows;
     if (two_streams) {
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         FGX_CHECK_HIP(hipStreamIsCapturing(s, &capturing));
@@ -76,7 +76,7 @@ int sort_beside_pairs(size_t n, int V, const int32_t* binary, int64_t* sorted_id
         }
     }
     // the mask sort first: it is the longer of the two chains
-    rc = fgx_sort_by_code(binary, n, V, sorted_idx, sort_ws, sort_bytes, (fgx_stream_t)s);
+    if (sorted_idx != nullptr) rc = fgx_sort_by_code(binary, n, V, sorted_idx, sort_ws, sort_bytes, (fgx_stream_t)s);
     if (rc == FGX_OK && with_pairs) {
         hipError_t e = two_streams ? hipStreamWaitEvent(side, map_made, 0) : hipSuccess;
         if (e != hipSuccess) rc = fail_hip(e, who);
@@ -186,7 +186,7 @@ extern "C" int fgx_subm_cache_build_grid(const int32_t* coords, size_t n, int B,
     GridIndexLayout G;
     FGX_CHECK_ARG(grid_index_plan(n, B, W, H, D, &G), "%s: no index over a grid of %d x %d x %d x %d cells and %zu voxels", who, B, W, H, D, n);
     const PostLayout P = post_layout(G.total, n, V, with_pairs != 0, 0);
-    FGX_CHECK_ARG(coords && workspace && out_map && gray && binary && sorted_idx, "%s: null buffer", who);
+    FGX_CHECK_ARG(coords && workspace && out_map && gray && binary, "%s: null buffer", who);
     FGX_CHECK_ARG(!with_pairs || (sig_i && sig_o), "%s: null pair list", who);
     FGX_CHECK_ARG((((uintptr_t)coords & 15) | ((uintptr_t)workspace & 255)) == 0, "%s: coords must be 16-byte, workspace 256-byte aligned", who);
     FGX_CHECK_ARG(workspace_bytes >= P.total, "%s: workspace of %zu bytes, need %zu", who, workspace_bytes, P.total);
@@ -202,6 +202,29 @@ extern "C" int fgx_subm_cache_build_grid(const int32_t* coords, size_t n, int B,
         if (r != FGX_OK) return r;
         return pair_lists_from_counts(out_map, gray, n, V, counts, cdiv(n, counted ? kPairSubRows : kPairRows), counted,
                                       (uint32_t*)(ws + P.offsets), (uint32_t*)(ws + P.totals), seg, seg_host, sig_i, sig_o, on);
+    });
+}
+
+extern "C" size_t fgx_cache_post_workspace_bytes(size_t n, int V, int with_pairs) {
+    return V >= 1 && V <= 32 ? post_layout(0, n, V, with_pairs != 0, 0).total : 0;
+}
+
+extern "C" int fgx_cache_post(const uint32_t* map, const int32_t* gray, const int32_t* binary, size_t n, int V, int with_pairs, void* workspace,
+                              size_t workspace_bytes, int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, uint32_t* seg_host,
+                              fgx_stream_t stream) {
+    const char* who = "fgx_cache_post";
+    FGX_CHECK_ARG(V >= 1 && V <= 32 && n > 0 && n * (size_t)V < 0xFFFFFFFFull, "%s: %zu rows of %d offsets out of range", who, n, V);
+    const PostLayout P = post_layout(0, n, V, with_pairs != 0, 0);
+    FGX_CHECK_ARG(map && gray && binary && workspace && (!with_pairs || (seg && sig_i && sig_o)), "%s: null buffer", who);
+    FGX_CHECK_ARG(((uintptr_t)workspace & 255) == 0 && workspace_bytes >= P.total, "%s: workspace of %zu bytes, need %zu, 256-byte aligned", who,
+                  workspace_bytes, P.total);
+    char* ws = (char*)workspace;
+    hipStream_t s = (hipStream_t)stream;
+    PhaseEnd phases{s};
+    return sort_beside_pairs(n, V, binary, sorted_idx, ws + P.sort_ws, P.sort_bytes, with_pairs != 0, s, who, [&](hipStream_t on) {
+        const int r = pair_counts(gray, n, V, (uint32_t*)(ws + P.counts), on);
+        return r != FGX_OK ? r : pair_lists_from_counts(map, gray, n, V, (uint32_t*)(ws + P.counts), cdiv(n, kPairRows), false, (uint32_t*)(ws + P.offsets),
+                                                        (uint32_t*)(ws + P.totals), seg, seg_host, sig_i, sig_o, on);
     });
 }
 

@@ -36,7 +36,7 @@ namespace {
 // ---- the library -------------------------------------------------------------------------------------------------
 #define FGX_HOST_FUNCTIONS(X)                                                                                                     \
     X(fgx_last_error) X(fgx_grid_index_pays) X(fgx_grid_index_walks) X(fgx_subm_neighbor_map_grid_workspace_bytes) X(fgx_subm_cache_grid_workspace_bytes) \
-    X(fgx_subm_cache_build_grid) X(fgx_spconv_cache_grid_workspace_bytes) X(fgx_spconv_cache_build_grid)                           \
+    X(fgx_subm_cache_build_grid) X(fgx_cache_post_workspace_bytes) X(fgx_cache_post) X(fgx_spconv_cache_grid_workspace_bytes) X(fgx_spconv_cache_build_grid)                           \
     X(fgx_spconv_out_dims) X(fgx_spconv_out_coords_grid_workspace_bytes) X(fgx_spconv_out_coords_grid_count)                       \
     X(fgx_spconv_out_coords_grid_emit) X(fgx_tile_plan) X(fgx_gather_item_order) X(fgx_gather_item_order_workspace_bytes)          \
     X(fgx_weight_panel_bytes) X(fgx_pack_weight) X(fgx_conv_scratch_bytes) X(fgx_conv_gather_gemm_act_mask)                        \
@@ -116,6 +116,9 @@ struct Cache {
         if (PyDict_SetItemString(dict.ptr(), key.c_str(), value.ptr()) != 0) throw py::error_already_set();
     }
     void set(const std::string& key, const Tensor& t) const { set(key, py::cast(t)); }
+    void drop(const char* key) const {
+        if (has(key) && PyDict_DelItemString(dict.ptr(), key) != 0) throw py::error_already_set();
+    }
 };
 
 // ---- buffers ---------------------------------------------------------------------------------------------------------
@@ -221,10 +224,81 @@ private:
 };
 
 // ---- neighbor caches ---------------------------------------------------------------------------------------------------
+// The layer a cache is built for.
+struct Layer {
+    int code;                       // dtype (-1: one the kernels do not take)
+    int64_t ci, co;
+    bool record, input_grad, weight_grad, relu, splitk;
+};
+struct Needs {
+    bool order = true, lists = true;
+};
+
+bool schedules_are_ours();
+std::string narrow_mode() { return py::reinterpret_borrow<py::object>(module_get(g_spconv, "NARROW_RESIDENT")).cast<std::string>(); }
+// a 16-bit forward pass that trains through the ReLU, or is narrow, keeps the masked kernels' order of sums (see convolve)
+bool pairs_forward(bool record, int es, bool relu, int64_t co) { return !record || es == 4 || (!relu && co >= 128); }
+bool pairs_backward(int es, bool relu, int64_t co) { return !relu || es == 4 || co >= 256; }
+
+// What of the mask order and the pair lists the kernels of this layer read (a guess that errs towards "all of it": what a pass finds missing
+// it makes).  The resident-row kernels walk the cells of the index, first layers the map, the products over pairs a plan of
+// their own; so of the tables of 2 667 120 voxels under 32 channels 0.26 ms of sorts and 0.19 ms of lists were never read, of 434 000 voxels under a
+// first layer 0.05 and 0.03 of 0.27.
+Needs layer_needs(const Layer& l, int64_t n, int v, bool walks) {
+    Needs needs;
+    if (!schedules_are_ours()) return needs;
+    const int es = l.code == FGX_F32 ? 4 : 2, align = 16 / es;
+    const int ci = (int)((l.ci + align - 1) / align * align), co = (int)((l.co + align - 1) / align * align);
+    const bool resident = es == 2 && walks && v <= 27 && ci <= 32 && l.co <= 32 && l.co % 8 == 0 && n >= module_int(g_impl, "NARROW_RESIDENT_MIN_ROWS") &&
+                          narrow_mode() != "off";
+    const bool forward = resident || L.fgx_conv_gemm_stem_pays(l.code, 0, (size_t)n, ci, (int)l.co, v) ||
+                         (l.splitk && pairs_forward(l.record, es, l.relu, l.co) && L.fgx_conv_gemm_pairs_pays(l.code, 0, (size_t)n, ci, (int)l.co, v));
+    const bool backward = !l.record || !l.input_grad || (resident && l.ci % 8 == 0) || L.fgx_conv_gemm_stem_pays(l.code, 1, (size_t)n, co, (int)l.ci, v) ||
+                          (l.splitk && pairs_backward(es, l.relu, l.co) && L.fgx_conv_gemm_pairs_pays(l.code, 1, (size_t)n, (int)l.ci, co, v));
+    needs.order = !(forward && backward);
+    needs.lists = l.record && l.weight_grad && !resident && !L.fgx_wgrad_stem_pays(l.code, (size_t)n, ci, co, v);
+    return needs;
+}
+
+// The mask order and / or the pair lists of a cache that was built without them.
+void cache_post(const Cache& c, bool order, bool lists) {
+    const Tensor nmap = c.need("neighbor_map"), gray = c.need("gray_code"), binary = c.need("_binary_code");
+    const at::Device dev = nmap.device();
+    const c10::DeviceGuard guard(dev);
+    const int64_t stream = stream_of(nmap), n = nmap.size(0);
+    const int v = (int)nmap.size(1);
+    Tensor sorted, seg, sig_i, sig_o;
+    std::unique_ptr<SegHost> host;
+    if (order) sorted = make({n}, at::kLong, dev);
+    if (lists) {
+        seg = make({v + 1}, at::kUInt32, dev);
+        sig_i = make({n * v}, at::kUInt32, dev);
+        sig_o = make({n * v}, at::kUInt32, dev);
+        host = std::make_unique<SegHost>(dev.index(), v + 1);
+    }
+    Tensor ws = workspace(L.fgx_cache_post_workspace_bytes((size_t)n, v, lists), dev);
+    check(L.fgx_cache_post(ptr<uint32_t>(nmap), ptr<int32_t>(gray), ptr<int32_t>(binary), (size_t)n, v, lists, ptr(ws), (size_t)ws.numel(),
+                           ptr<int64_t>(sorted), ptr<uint32_t>(seg), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o), host ? host->words() : nullptr,
+                           as_stream(stream)));
+    if (order) {
+        c.set("sorted_idx", sorted);
+        c.drop("_order_left_out");
+    }
+    if (lists) {
+        host->record(as_stream(stream));
+        const py::object arriving = py::cast(std::move(host));
+        c.set("valid_signal_seg", seg);
+        c.set("_pending_pairs", py::make_tuple(sig_i, sig_o, arriving, arriving));
+        c.drop("_lists_left_out");
+    }
+}
+
 // Tables of a submanifold convolution through the grid index, or None where it does not apply:
 // (neighbor_map, gray, binary, order, walk, seg, sig_i, sig_o, SegHost), the last four None without gradients; walk: the rows in the
-// order of the index's cells, for the plan of narrow layers, or None.
-py::object subm_cache(const Tensor& coords, const std::vector<int>& geom, bool needs_grad, bool forced, size_t max_pair_bytes) {
+// order of the index's cells, for the plan of narrow layers, or None.  layer (dtype code, ci, co, record, input_grad, weight_grad, relu, splitk):
+// the layer that asks, whose kernels may read neither the order nor the lists; those are None then.
+py::object subm_cache(const Tensor& coords, const std::vector<int>& geom, bool needs_grad, bool forced, size_t max_pair_bytes,
+                      const c10::optional<std::tuple<int, int64_t, int64_t, bool, bool, bool, bool, bool>>& layer) {
     const int64_t stream = stream_of(coords);
     const size_t n = (size_t)coords.size(0);
     const int B = geom[0], W = geom[1], H = geom[2], D = geom[3], V = geom[4] * geom[5] * geom[6];
@@ -234,26 +308,35 @@ py::object subm_cache(const Tensor& coords, const std::vector<int>& geom, bool n
     const at::Device dev = coords.device();
     const c10::DeviceGuard guard(dev);
     const int64_t rows = (int64_t)n, slots = rows * V;
+    const bool walks = rows >= module_int(g_impl, "NARROW_RESIDENT_MIN_ROWS") && L.fgx_grid_index_walks(n, B, W, H, D);
+    Needs needs;
+    if (layer && std::get<0>(*layer) >= 0) {
+        const auto& [code, ci, co, record, input_grad, weight_grad, relu, splitk] = *layer;
+        needs = layer_needs(Layer{code, ci, co, record, input_grad, weight_grad, relu, splitk}, rows, V, walks);
+    }
+    const bool lists = needs_grad && needs.lists;
     Tensor nmap = make({rows, V}, at::kUInt32, dev), gray = make({rows}, at::kInt, dev), binary = make({rows}, at::kInt, dev);
-    Tensor order = make({rows}, at::kLong, dev), seg, sig_i, sig_o;
+    Tensor order, seg, sig_i, sig_o;
     std::unique_ptr<SegHost> host;
-    if (needs_grad) {
+    if (needs.order) order = make({rows}, at::kLong, dev);
+    if (lists) {
         seg = make({V + 1}, at::kUInt32, dev);
         sig_i = make({slots}, at::kUInt32, dev);
         sig_o = make({slots}, at::kUInt32, dev);
         host = std::make_unique<SegHost>(dev.index(), V + 1);
     }
     Tensor walk;
-    if (rows >= module_int(g_impl, "NARROW_RESIDENT_MIN_ROWS") && L.fgx_grid_index_walks(n, B, W, H, D)) walk = make({rows}, at::kUInt32, dev);
-    Tensor ws = workspace(L.fgx_subm_cache_grid_workspace_bytes(n, B, W, H, D, V, needs_grad), dev);
-    check(L.fgx_subm_cache_build_grid(ptr<int32_t>(coords), n, B, W, H, D, geom[4], geom[5], geom[6], geom[7], geom[8], geom[9], needs_grad,
+    if (walks) walk = make({rows}, at::kUInt32, dev);
+    Tensor ws = workspace(L.fgx_subm_cache_grid_workspace_bytes(n, B, W, H, D, V, lists), dev);
+    check(L.fgx_subm_cache_build_grid(ptr<int32_t>(coords), n, B, W, H, D, geom[4], geom[5], geom[6], geom[7], geom[8], geom[9], lists,
                                       ptr(ws), (size_t)ws.numel(), ptr<uint32_t>(nmap), ptr<int32_t>(gray), ptr<int32_t>(binary),
                                       ptr<int64_t>(order), ptr<uint32_t>(seg), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o),
                                       host ? host->words() : nullptr, ptr<uint32_t>(walk), as_stream(stream)));
     py::object walk_out = walk.defined() ? py::cast(walk) : py::none();
-    if (!host) return py::make_tuple(nmap, gray, binary, order, walk_out, py::none(), py::none(), py::none(), py::none());
+    const py::object order_out = order.defined() ? py::cast(order) : py::none();
+    if (!host) return py::make_tuple(nmap, gray, binary, order_out, walk_out, py::none(), py::none(), py::none(), py::none());
     host->record(as_stream(stream));
-    return py::make_tuple(nmap, gray, binary, order, walk_out, seg, sig_i, sig_o, std::move(host));
+    return py::make_tuple(nmap, gray, binary, order_out, walk_out, seg, sig_i, sig_o, std::move(host));
 }
 
 bool conv_grids_pay(size_t n_in, size_t n_out, int B, const int* in, const int* out, bool with_bwd) {
@@ -618,10 +701,11 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
         mark(name, "stop");
         return p;
     }
-    if (masked && !(c.has("gray_code") && c.has("sorted_idx"))) c.obj.attr("_ensure_sorted")();
+    if (masked && !narrow && c.has("_order_left_out")) cache_post(c, true, false);
+    if (masked && !narrow && !(c.has("gray_code") && c.has("sorted_idx"))) c.obj.attr("_ensure_sorted")();
     const Sched s = schedule(pass, src, n, ci, co, v);
     bool own_order = false;
-    if (masked && row_bytes <= module_int(g_impl, "LOCALITY_MAX_ROW_BYTES") && (c.has("_tile_order") || n >= module_int(g_impl, "LOCALITY_MIN_ROWS")) &&
+    if (masked && !narrow && row_bytes <= module_int(g_impl, "LOCALITY_MAX_ROW_BYTES") && (c.has("_tile_order") || n >= module_int(g_impl, "LOCALITY_MIN_ROWS")) &&
         impl_function("_locality_applies")(c.obj, n, row_bytes).cast<bool>()) {
         c.obj.attr("_ensure_tile_order")();
         own_order = c.has("_tile_order");
@@ -941,7 +1025,7 @@ struct ConvBackward : public torch::autograd::Node {
         const int64_t co = w.size(0), kw = w.size(1), kh = w.size(2), kd = w.size(3), ci = w.size(4), v = kw * kh * kd;
         if (need_f) {
             const Tensor wv = w.reshape({co, v, ci});
-            const bool pairs = !relu || f.element_size() == 4 || co >= 256;      // (a plan for input gradients alone: 4 us)
+            const bool pairs = pairs_backward((int)f.element_size(), relu, co);      // (a plan for input gradients alone: 4 us)
             if (call.generic) {
                 const Cache view(c.obj.attr("_bwd_view")());
                 // mask-sorted walk only where the cache carries the backward order
@@ -996,7 +1080,13 @@ Tensor convolve(const Tensor& feats, py::object cache_obj, const Tensor& weight,
     // A 16-bit forward pass that trains through the ReLU keeps the order of sums it has always had: another one rounds an output
     // differently here and there, and from layer to layer more sums near zero change sides (four layers of 512 channels: gradients 0.7 % off).
     // So does a narrow one, where the operator with the ReLU and one followed by it agree bit for bit.
-    const bool pairs = !record || feats.element_size() == 4 || (!relu && co >= 128);
+    const bool pairs = pairs_forward(record, (int)feats.element_size(), relu, co);
+    // lists that the layer the cache was built for does not read and this one's weight gradient will: on their way from here on, so that
+    // the backward pass does not wait for their length
+    if (record && weight.requires_grad() && c.has("_lists_left_out") && !capturing(stream_of(feats))) {
+        const Layer l{dtype_code(feats), ci, co, true, feats.requires_grad(), true, relu, splitk};
+        if (layer_needs(l, feats.size(0), (int)v, c.has("_cell_walk")).lists) cache_post(c, false, true);
+    }
     const bool bits = relu && record && PyObject_IsTrue(module_get(g_spconv, "RELU_BIT_MASK"));
     Product p;
     {
@@ -1090,6 +1180,7 @@ PYBIND11_MODULE(fgx_host, m) {
     py::class_<SegHost>(m, "SegHost").def("synchronize", &SegHost::synchronize).def("tolist", &SegHost::tolist);
     m.def("bind", &bind);
     m.def("subm_cache", &subm_cache);
+    m.def("cache_post", [](py::object cache, bool order, bool lists) { cache_post(Cache(std::move(cache)), order, lists); });
     m.def("spconv_cache", &spconv_cache);
     m.def("out_coords", &out_coords);
     m.def("convolve", &convolve);

@@ -60,8 +60,17 @@ class SubMConv3dNeighborCache:
     # (one entry per slot of the map) and cut to L when somebody first reads them or the host copy of the segment
     # table, which by then has long arrived.  (__getattr__ is only asked for names that are not there yet.)
     _PENDING = ("valid_signal_i", "valid_signal_o", "_valid_signal_seg_host")
+    # A cache that a layer builds for itself leaves out the mask order and the pair lists where that layer's kernels read neither
+    # (`_order_left_out`, `_lists_left_out`); whoever asks first, a layer with other kernels or a reader of the fields, has them made.
 
     def __getattr__(self, name):
+        if name == "sorted_idx" and "_order_left_out" in self.__dict__:
+            nat.host().cache_post(self, True, False)
+            return self.__dict__[name]
+        if (name in SubMConv3dNeighborCache._PENDING or name == "valid_signal_seg") and "_lists_left_out" in self.__dict__:
+            nat.host().cache_post(self, False, True)
+            if name == "valid_signal_seg":
+                return self.__dict__[name]
         if name in SubMConv3dNeighborCache._PENDING and "_pending_pairs" in self.__dict__:
             self._finish_pairs()
             return self.__dict__[name]
@@ -447,10 +456,11 @@ def _build_neighbor_map(coords: torch.Tensor, shape, kernel_size, dilation, with
     return nmap, gray, binary
 
 
-def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, needs_grad: bool):
+def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, needs_grad: bool, layer: Optional[tuple] = None):
     """The masked algorithms' neighbor cache through fgx_subm_cache_build_grid or fgx_subm_cache_build: map, codes, mask sort and (needs_grad) the pair
     lists enqueued by one library call, with every buffer allocated beforehand -- the GPU does not wait for the host
-    between the steps.  Returns (nmap, gray, binary, order, walk of the grid index or None, pairs or None), or None where the call does not apply (the
+    between the steps.  layer: the layer the cache is for, (dtype code or -1, ci, co, records gradients, the input's, the weight's, relu, split K), whose kernels may not
+    need all of it.  Returns (nmap, gray, binary, order or None, walk of the grid index or None, pairs or None), or None where the call does not apply (the
     hash builder's range, kernels beyond what the sorted builder takes, pair lists too large to allocate at their bound)
     and the step-by-step path runs."""
     n = coords.shape[0]
@@ -459,10 +469,10 @@ def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, ne
     v = kw * kh * kd
     if spconv.NEIGHBOR_MAP_BUILDER in ("auto", "grid"):
         built = nat.host().subm_cache(coords, [B, W, H, D, kw, kh, kd, int(dilation[0]), int(dilation[1]), int(dilation[2])], needs_grad,
-                                      spconv.NEIGHBOR_MAP_BUILDER == "grid", PAIR_LISTS_UNSIZED_MAX_BYTES)
+                                      spconv.NEIGHBOR_MAP_BUILDER == "grid", PAIR_LISTS_UNSIZED_MAX_BYTES, layer)
         if built is not None:
             nmap, gray, binary, order, walk, seg, sig_i, sig_o, arriving = built
-            return nmap, gray, binary, order, walk, ({"seg": seg, "pending": (sig_i, sig_o, arriving, arriving)} if needs_grad else None)
+            return nmap, gray, binary, order, walk, ({"seg": seg, "pending": (sig_i, sig_o, arriving, arriving)} if seg is not None else None)
     builder = _pick_builder(n, v, B, (W, H, D))
     vol = B * W * H * D
     bound = n * v
@@ -772,9 +782,10 @@ class SubMConv3dFunction(Function):
         kernel_size: Tuple[int, int, int],
         dilation: Tuple[int, int, int],
         needs_grad: bool,
+        layer: Optional[tuple] = None,
     ) -> SubMConv3dNeighborCache:
         """Build the neighbor tables for `coords` under the current algorithm
-        (reference: submanifold_conv3d.py:46-107)."""
+        (reference: submanifold_conv3d.py:46-107).  layer: as in _build_cache_one_call."""
         assert coords.is_contiguous(), "Coords should be contiguous"
         assert coords.dtype in [torch.int32], "Unsupported coords dtype. Expect int32"
         algo = spconv.ALGORITHM
@@ -792,18 +803,24 @@ class SubMConv3dFunction(Function):
             # pair lists wgrad needs are derived from it on first use
             nmap, _, _ = _build_neighbor_map(coords, shape, kernel_size, dilation, with_codes=False)
             return SubMConv3dNeighborCache(neighbor_map=nmap)
-        built = _build_cache_one_call(coords, shape, kernel_size, dilation, needs_grad) if CACHE_BUILD_ONE_CALL else None
+        built = _build_cache_one_call(coords, shape, kernel_size, dilation, needs_grad, layer) if CACHE_BUILD_ONE_CALL else None
         if built is not None:
             nmap, gray, binary, order, walk, pairs = built
-            cache = SubMConv3dNeighborCache(neighbor_map=nmap, gray_code=gray, sorted_idx=order)
+            cache = SubMConv3dNeighborCache(neighbor_map=nmap, gray_code=gray)
+            if order is not None:
+                cache["sorted_idx"] = order
+            else:
+                cache["_order_left_out"] = True
             cache["_coords"] = coords
             cache["_needs_grad"] = bool(needs_grad)
             cache["_grid"] = (int(shape[0]), tuple(int(d) for d in shape[2:]))
             cache["_binary_code"] = binary
             if walk is not None:
                 cache["_cell_walk"] = walk
-            if needs_grad:
+            if pairs is not None:
                 cache._attach_pairs(pairs)
+            elif needs_grad:
+                cache["_lists_left_out"] = True
             return cache
         nmap, gray, binary = _build_neighbor_map(coords, shape, kernel_size, dilation, with_codes=True)
         # The pair lists and the mask sort both start from the map and its codes and need nothing of each other: the lists
@@ -1020,8 +1037,9 @@ def _convolve(feats, coords, shape, weight, bias, neighbor_cache, dilation, relu
     algo = spconv.ALGORITHM
     if neighbor_cache is None:
         assert feats.shape[-1] == weight.shape[-1], f"Input channels ({feats.shape[-1]}) should match weight channels ({weight.shape[-1]})"
-        neighbor_cache = SubMConv3dFunction._compute_neighbor_cache(coords, shape, tuple(weight.shape[1:4]), dilation,
-                                                                    _records_gradients(feats, weight, bias))
+        records = _records_gradients(feats, weight, bias)
+        layer = (nat.DTYPE_CODE.get(feats.dtype, -1), feats.shape[-1], weight.shape[0], records, feats.requires_grad, weight.requires_grad, relu, algo not in _NO_SPLITK)
+        neighbor_cache = SubMConv3dFunction._compute_neighbor_cache(coords, shape, tuple(weight.shape[1:4]), dilation, records, layer)
     return nat.host().convolve(feats, neighbor_cache, weight, bias, relu, False, algo in _MASKED, algo not in _NO_SPLITK), neighbor_cache
 
 

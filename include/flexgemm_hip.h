@@ -190,7 +190,8 @@ int fgx_subm_cache_build(const int32_t* coords, size_t n, int B, int W, int H, i
  * fgx_subm_cache_build, without the sort's key_bits and presorted; seg_host (optional): pinned host memory that receives the
  * segment table as well (valid once the stream has passed the call); walk (optional, where fgx_grid_index_walks is 1): the rows
  * in the order of the index's cells, a space-filling curve, then the rows without a cell of their own (given again, or outside the
- * grid) in row order, for fgx_narrow_plan_walk.
+ * grid) in row order, for fgx_narrow_plan_walk.  sorted_idx may be NULL: no mask order now.  fgx_cache_post makes what was left out
+ * from the map and its codes: the order (sorted_idx not NULL) and, with_pairs, the pair lists.
  * Replaces: hashmap_build_submanifold_conv_neighbour_map and the same sequence of calls as fgx_subm_cache_build. */
 int fgx_grid_index_pays(size_t n, int B, int W, int H, int D);
 int fgx_grid_index_walks(size_t n, int B, int W, int H, int D);
@@ -199,6 +200,10 @@ int fgx_subm_neighbor_map_grid(const int32_t* coords, size_t n, int B, int W, in
                                int Dd, void* workspace, size_t workspace_bytes, uint32_t* out_map, int32_t* gray, int32_t* binary,
                                fgx_stream_t stream);
 size_t fgx_subm_cache_grid_workspace_bytes(size_t n, int B, int W, int H, int D, int V, int with_pairs);
+size_t fgx_cache_post_workspace_bytes(size_t n, int V, int with_pairs);
+int fgx_cache_post(const uint32_t* map, const int32_t* gray, const int32_t* binary, size_t n, int V, int with_pairs, void* workspace,
+                   size_t workspace_bytes, int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, uint32_t* seg_host,
+                   fgx_stream_t stream);
 int fgx_subm_cache_build_grid(const int32_t* coords, size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dw, int Dh, int Dd,
                               int with_pairs, void* workspace, size_t workspace_bytes, uint32_t* out_map, int32_t* gray, int32_t* binary,
                               int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, uint32_t* seg_host,
