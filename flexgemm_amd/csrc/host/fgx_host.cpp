@@ -44,6 +44,7 @@ namespace {
     X(fgx_conv_gather_gemm_stream_act_mask) X(fgx_conv_gather_gemm_stream_groups) X(fgx_relu_mask_apply)                           \
     X(fgx_colsum_scratch_bytes) X(fgx_colsum) X(fgx_wgrad_block_bounds_count) X(fgx_wgrad_block_bounds)                            \
     X(fgx_conv_gemm_stem_pays) X(fgx_conv_gemm_stem) X(fgx_wgrad_stem_pays) X(fgx_wgrad_stem_scratch_bytes) X(fgx_conv_wgrad_stem) X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
+    X(fgx_conv_wgrad_split_scratch_bytes) X(fgx_conv_wgrad_split)                                                                  \
     X(fgx_wgrad_sweep_plan_bytes) X(fgx_wgrad_sweep_plan) X(fgx_wgrad_sweep_scratch_bytes) X(fgx_conv_wgrad_sweep)                 \
     X(fgx_serialize_encode) X(fgx_serialize_decode) X(fgx_table_lookup)
 
@@ -902,13 +903,20 @@ WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool 
         } else {
             const Tensor bounds = wgrad_bounds(c, sig_o, seg, (size_t)n, v, s.block_rows, stream);
             Tensor lists;
-            if (s.stream == 1 && PyObject_IsTrue(module_get(g_impl, "WGRAD_BALANCED_LISTS")))
+            const size_t split = s.stream == 1 && code == FGX_F32 && s.tile_rows == s.tile_cols
+                                     ? L.fgx_conv_wgrad_split_scratch_bytes((size_t)n, (size_t)n_in, (uint32_t)pairs, v, ci, co, s.tile_rows, s.block_rows) : 0;
+            if (s.stream == 1 && code != FGX_F32 && PyObject_IsTrue(module_get(g_impl, "WGRAD_BALANCED_LISTS")))
                 lists = wgrad_item_lists(c, bounds, (size_t)n, v, ci, co, s, true, stream);
-            Tensor scratch = workspace(L.fgx_wgrad_scratch_bytes((size_t)n, v, ci, co, s.block_rows), dev);
+            Tensor scratch = workspace(split ? split : L.fgx_wgrad_scratch_bytes((size_t)n, v, ci, co, s.block_rows), dev);
             mark("wgrad", "start");
-            check(L.fgx_conv_wgrad_lists(code, ptr(grad), ptr(feats), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o), seg.data(), ptr<uint32_t>(bounds),
-                                         ptr<uint32_t>(lists), (size_t)n, (size_t)n_in, ci, co, v, s.tile_rows, s.tile_cols, s.block_rows, s.stream,
-                                         ptr(scratch), ptr(w.weight), ptr(w.bias), bias_offset, as_stream(stream)));
+            if (split)
+                check(L.fgx_conv_wgrad_split(ptr(grad), ptr(feats), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o), seg.data(), ptr<uint32_t>(bounds),
+                                             (size_t)n, (size_t)n_in, ci, co, v, s.tile_rows, s.block_rows, ptr(scratch), ptr(w.weight), ptr(w.bias),
+                                             as_stream(stream)));
+            else
+                check(L.fgx_conv_wgrad_lists(code, ptr(grad), ptr(feats), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o), seg.data(), ptr<uint32_t>(bounds),
+                                             ptr<uint32_t>(lists), (size_t)n, (size_t)n_in, ci, co, v, s.tile_rows, s.tile_cols, s.block_rows, s.stream,
+                                             ptr(scratch), ptr(w.weight), ptr(w.bias), bias_offset, as_stream(stream)));
         }
         mark("wgrad", "stop");
     }

@@ -27,6 +27,7 @@
 // fp32 partial product; a second kernel adds an offset's partials in block order (deterministic) and
 // casts to the output type.  The per-(offset, block) pair ranges are found by a small binary-search
 // kernel over sig_o.
+#include <numeric>
 #include <type_traits>
 
 #include "wgrad_device.h"
@@ -291,7 +292,7 @@ wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Tag::ty
 }
 
 // ------------------------------------------------------------------------------------------------
-// Streaming variant (16-bit types): one persistent workgroup per CU, specialised wavefronts.
+// Streaming variant: one persistent workgroup per CU, specialised wavefronts.
 // ------------------------------------------------------------------------------------------------
 // Four wavefronts multiply (2 x 2 over the Co x Ci tile), four more only enqueue loads: issuing a vector-memory
 // instruction blocks its wavefront while the address pipeline is busy, and a step's gathers keep that pipeline busy
@@ -307,6 +308,7 @@ constexpr int kWsIdxSlots = 8;
 constexpr int kWsIdxAhead = 4;       // index loads run this many steps ahead of the row loads (> kWsStages - 1)
 constexpr int kWsLoaders = 4;
 constexpr int kWsPairs = 64;         // pairs per step
+constexpr unsigned kSplitMaxUnits = 2048;       // fp32: (block, offset) pairs of the even split, whose running cost stands in LDS
 template <typename Tag, int BM, int BN>
 struct WStreamCfg {
     using T = typename Tag::type;
@@ -317,14 +319,15 @@ struct WStreamCfg {
     static constexpr bool KSPLIT = BM == 32 && BN == 32;
     static constexpr int SLICES = KSPLIT ? 4 : 1;                  // partial products per (voxel block, offset, tile)
     // (a 256 x 128 tile's stages are 48 KiB: three of them fit, with the same 64-pair steps)
-    static constexpr int P = KSPLIT ? 4 * kWsPairs : kWsPairs, S = BM * BN > 128 * 128 ? 3 : kWsStages;
+    static constexpr int P = KSPLIT ? 4 * kWsPairs : kWsPairs, S = (BM + BN) * ES > 512 ? 3 : kWsStages;
     static constexpr int NW = 4, NL = kWsLoaders, NT = 64 * (NW + NL);
-    static constexpr int WM = KSPLIT ? BM : BM / 2, WN = KSPLIT ? BN : BN / 2, TM = WM / 32, TN = WN / 32;
+    // fp32 multiplies in 16 x 16 tiles: a 96 x 96 tile then has nine of them for each of the four multipliers
+    static constexpr int MT = ES == 2 ? 32 : 16;
+    static constexpr int WM = KSPLIT ? BM : BM / 2, WN = KSPLIT ? BN : BN / 2, TM = WM / MT, TN = WN / MT;
     static constexpr int IDX_PER = P / 64;                         // wave-wide index loads per operand and step
     static constexpr int ROWB_A = BM * ES, ROWB_B = BN * ES;
     static constexpr int CH_A = ROWB_A / 16, CH_B = ROWB_B / 16;
-    static constexpr int RPI_A = 64 / CH_A, RPI_B = 64 / CH_B;
-    static constexpr int A_PER = P / RPI_A / NL, B_PER = P / RPI_B / NL;
+    static constexpr int A_PER = P * CH_A / 64 / NL, B_PER = P * CH_B / 64 / NL;
     static constexpr int LPS = A_PER + B_PER;
     static constexpr int A_BYTES = P * ROWB_A, B_BYTES = P * ROWB_B, STAGE_BYTES = A_BYTES + B_BYTES;
     static constexpr int IDX_SLOT_BYTES = 2 * P * 4;               // sig_o x P | sig_i x P
@@ -339,18 +342,154 @@ struct WStreamCfg {
     }
     static constexpr int band_bytes(int es) { return band_rows(es) * band_pitch(es); }
     static constexpr int BAND_BYTES = band_bytes(ES) > band_bytes(4) ? band_bytes(ES) : band_bytes(4);
-    static constexpr size_t lds_bytes = (size_t)RING_BYTES + (size_t)NW * BAND_BYTES;
-    static_assert(band_rows(4) >= 1024 / (WN * 4) && band_rows(ES) >= 1024 / (WN * ES), "a wave-wide store takes its rows from one band");
-    static_assert(ES == 2, "the streaming kernel handles 16-bit types");
+    // (fp32 tiles leave straight from the registers: behind the rings stands the running cost of the even split)
+    static constexpr size_t lds_bytes = (size_t)RING_BYTES + (ES == 4 ? (size_t)(kSplitMaxUnits + 1) * 4 : (size_t)NW * BAND_BYTES);
+    static_assert(ES == 4 || (band_rows(4) >= 1024 / (WN * 4) && band_rows(ES) >= 1024 / (WN * ES)), "a wave-wide store takes its rows from one band");
+    static_assert(!KSPLIT || ES == 2, "the pair-splitting tile is for 16-bit types");
     static_assert(S == 3 || S == 4, "the loaders' wait is written for rings of three or four stages");
     static_assert(kWsIdxAhead > S - 1 && lds_bytes <= 160 * 1024, "index loads run ahead of the row loads; the ring fits LDS");
     static_assert(IDX_PER == 1 || IDX_PER == NL, "index loads: one loader per operand, or every loader a quarter of both");
-    static_assert(WM % 32 == 0 && WN % 32 == 0, "wave tile must be a multiple of 32x32");
-    static_assert(P % (RPI_A * NL) == 0 && P % (RPI_B * NL) == 0, "every loader issues the same row loads");
+    static_assert(WM % MT == 0 && WN % MT == 0, "wave tile must be a multiple of the matrix unit's");
+    static_assert(P * CH_A % (64 * NL) == 0 && P * CH_B % (64 * NL) == 0, "every loader issues the same row loads");
     static_assert(2 * (LPS + 1) < 64, "outstanding loads exceed the vmcnt range");
-    static constexpr int key_a(int row) { return CH_A >= 16 ? 4 * (row & 3) : (CH_A >= 8 ? 2 * (row & 3) : 0); }
-    static constexpr int key_b(int row) { return CH_B >= 16 ? 4 * (row & 3) : (CH_B >= 8 ? 2 * (row & 3) : 0); }
+    // fp32 fragments are four pair rows of 16 columns: rows that start on the same banks (all of them, or every second one where a row
+    // is half a bank line longer) put them into different quarters of the line
+    static constexpr int key(int ch, int row) {
+        return ES == 4 ? (ch % 16 == 0 ? 4 * (row & 3) : 4 * ((row >> 1) & 1)) : (ch >= 16 ? 4 * (row & 3) : (ch >= 8 ? 2 * (row & 3) : 0));
+    }
+    static constexpr int key_a(int row) { return key(CH_A, row); }
+    static constexpr int key_b(int row) { return key(CH_B, row); }
 };
+
+// fp32 multipliers of the streaming kernel: a wavefront's WM x WN part of the tile in 16 x 16 products over four pairs at a time (lane l
+// holds row l / 16 of the four and column l % 16), transposed, so that element e of lane l is row l % 16 (co) and column
+// 4 * (l / 16) + e (ci): a lane stores 16 bytes of an output row, four lanes 64.
+// Bound by the matrix units, whose fp32 rate is a sixteenth of the 16-bit one: a lone workgroup keeps them busy 82 % of the time at
+// 96 x 96, 64 % at 64 x 64 (a step's barrier and first reads take about a thousand cycles beside 4608 and 2048 of products).
+// 96 x 96 because it is the widest tile whose three stages of 64 pairs fit LDS; two stages of 128 x 128 run at 88 %, but were no
+// faster where both fit (41 700 voxels, 128 channels: 0.172 ms each).  Reading fragments four k-blocks ahead was 4 % slower.
+template <typename C, typename W, typename Seek, typename After>
+__device__ __forceinline__ void multiply_f32(const unsigned char* ring, W m, const Seek& seek, const After& after, int wave_m, int wave_n,
+                                             unsigned group, float* partial) {
+    const int lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
+    int a_off[C::TM], b_off[C::TN];                 // of the first four pairs; 16-byte pieces swizzled by the row, whose key repeats every four
+#pragma unroll
+    for (int i = 0; i < C::TM; ++i) {
+        const int byte = (wave_m * C::WM + i * 16 + l16) * 4;
+        a_off[i] = q * C::ROWB_A + (((byte >> 4) ^ C::key_a(q)) << 4) + (byte & 15);
+    }
+#pragma unroll
+    for (int j = 0; j < C::TN; ++j) {
+        const int byte = (wave_n * C::WN + j * 16 + l16) * 4;
+        b_off[j] = C::A_BYTES + q * C::ROWB_B + (((byte >> 4) ^ C::key_b(q)) << 4) + (byte & 15);
+    }
+    using f32x4 = float __attribute__((ext_vector_type(4)));
+    // A running sum loses about a unit in the last place of itself with every addition: it is folded into a second one every 256
+    // pairs, so that a segment may be long (error against 64-bit sums, 96 channels: 667 763 voxels 3.5e-7, tiled kernel 9.8e-7).
+    constexpr int kFoldSteps = 256 / C::P;
+    int stage = 0;
+    while (m.live) {
+        const int nsteps = (int)((m.k_hi - m.k + C::P - 1) / C::P);
+        f32x4 acc[C::TM][C::TN], sum[C::TM][C::TN];
+#pragma unroll
+        for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+            for (int j = 0; j < C::TN; ++j) acc[i][j] = sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int s = 0; s < nsteps; ++s) {
+            if (s && s % kFoldSteps == 0) {
+#pragma unroll
+                for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < C::TN; ++j) {
+                        sum[i][j] += acc[i][j];
+                        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+            }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();           // the loaders saw this step's rows land
+            asm volatile("" ::: "memory");
+            const unsigned char* cur = ring + stage * C::STAGE_BYTES;
+            stage = stage + 1 == C::S ? 0 : stage + 1;
+#pragma unroll
+            for (int kb = 0; kb < C::P / 4; ++kb) {
+                float af[C::TM], bf[C::TN];
+#pragma unroll
+                for (int i = 0; i < C::TM; ++i) af[i] = *(const float*)(cur + a_off[i] + kb * 4 * C::ROWB_A);
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j) bf[j] = *(const float*)(cur + b_off[j] + kb * 4 * C::ROWB_B);
+#pragma unroll
+                for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < C::TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j], af[i], acc[i][j], 0, 0, 0);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // done reading this stage
+        }
+        float* dst = partial + ((size_t)group + m.item) * (4 * C::WM * C::WN);     // the segment's slot: a whole tile
+#pragma unroll
+        for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+            for (int j = 0; j < C::TN; ++j)
+                *(f32x4*)(dst + (wave_m * C::WM + i * 16 + l16) * (2 * C::WN) + wave_n * C::WN + j * 16 + q * 4) = sum[i][j] + acc[i][j];
+        m.k = m.k_hi;
+        m.item = after(m.item);
+        seek(m);
+    }
+}
+
+// ---- even split of the fp32 streaming kernel ----
+// The pairs of all (tile, voxel block, offset) items, one after the other, cut into as many runs of equal cost as there are
+// workgroups: nothing to even out, no lists to make (balanced lists of 648 items: 83 us beside a product of 96), and a workgroup
+// and an item have at most one segment in common, which goes to partial product `run + item`.  An item counts kSplitItemCost
+// pairs for its epilogue; cuts inside an item fall on whole steps.
+constexpr uint32_t kSplitItemCost = 64;
+constexpr unsigned kSplitMaxGroups = 256;       // workgroups at most: one per CU
+
+// pre[u] = cost of the units before u (pre[units]: of all); by the workgroup's first wavefront
+__device__ __forceinline__ void split_prefix(const uint32_t* __restrict__ bounds, unsigned V, unsigned nb, uint32_t* pre) {
+    const unsigned lane = threadIdx.x & 63, units = nb * V;
+    uint32_t before = 0;
+    if (lane == 0) pre[0] = 0;
+    for (unsigned u0 = 0; u0 < units; u0 += 64) {
+        const unsigned u = u0 + lane;
+        uint32_t cost = 0;
+        if (u < units) {
+            const unsigned at = u % V * (nb + 1) + u / V;
+            const uint32_t cnt = bounds[at + 1] - bounds[at];
+            cost = cnt ? cnt + kSplitItemCost : 0u;
+        }
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const uint32_t o = __shfl_up(cost, d);
+            cost += lane >= (unsigned)d ? o : 0u;
+        }
+        if (u < units) pre[u + 1] = before + cost;
+        before += __shfl(cost, 63);
+    }
+}
+
+// where run `w` of `runs` starts: (item << 32) | pairs of the item before it
+__device__ __forceinline__ uint64_t split_cut(unsigned w, unsigned runs, const uint32_t* __restrict__ bounds, unsigned V, unsigned nb,
+                                              unsigned tiles, const uint32_t* pre) {
+    const unsigned units = nb * V;
+    const uint32_t total = pre[units], c = (uint32_t)((uint64_t)total * tiles * w / runs);
+    if (total == 0 || w >= runs) return (uint64_t)(units * tiles) << 32;
+    const unsigned tile = c / total;
+    const uint32_t at_cost = c - tile * total;
+    unsigned lo = 0, hi = units;                // first unit that ends behind it
+    while (lo < hi) {
+        const unsigned mid = (lo + hi) / 2;
+        if (pre[mid + 1] <= at_cost) lo = mid + 1;
+        else hi = mid;
+    }
+    const unsigned at = lo % V * (nb + 1) + lo / V;
+    const uint32_t cnt = bounds[at + 1] - bounds[at], in = at_cost - pre[lo];
+    uint32_t k = in <= kSplitItemCost ? 0u : (in - kSplitItemCost + 32) / 64 * 64;
+    if (k >= cnt) {
+        k = 0;
+        ++lo;
+    }
+    return ((uint64_t)(tile * units + lo) << 32) | k;
+}
 
 template <typename Tag, int BM, int BN>
 __global__ void __launch_bounds__(64 * (4 + kWsLoaders))
@@ -359,7 +498,7 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
                     const uint32_t* __restrict__ bounds, int V, int Ci, int Co, unsigned nb, unsigned co_tiles,
                     unsigned ci_tiles, uint32_t n_pairs, uint32_t gout_bytes, uint32_t feats_bytes,
                     float* __restrict__ partial, typename Tag::type* __restrict__ direct,
-                    float* __restrict__ bias_partial, int bias_offset, const uint32_t* __restrict__ lists) {
+                    float* __restrict__ bias_partial, int bias_offset, const uint32_t* __restrict__ lists, unsigned run_copies, unsigned run_step) {
     using C = WStreamCfg<Tag, BM, BN>;
     constexpr int ES = C::ES, S = C::S, P = C::P;
 
@@ -387,11 +526,26 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
     // the wrong size does not)
     if (lists && !(lists[0] == gridDim.x && lists[1] == total_items && lists[2] == tiles && lists[3] == kItemListMagic)) lists = nullptr;
     if (lists) lists += kItemListHeader;
-    const unsigned range_end = lists ? total_items : ((xcd + 1) * per_xcd < total_items ? (xcd + 1) * per_xcd : total_items);
+    unsigned range_end = lists ? total_items : ((xcd + 1) * per_xcd < total_items ? (xcd + 1) * per_xcd : total_items);
     const uint32_t* chain = lists ? lists + gridDim.x : nullptr;
+    // fp32: this workgroup's run of the even split.  Runs at the same place of their tiles read the same rows: they are dealt one
+    // after the other (run_copies of them exactly, the next ones run_step runs on), so that an XCD has them at the same time.
+    const unsigned place = xcd * stride + slot, spread = ES == 4 ? gridDim.x / run_copies : 1u;
+    const unsigned group = ES == 4 ? place / run_copies * run_step % spread + place % run_copies * spread : 0u;
+    uint64_t run_lo = 0, run_hi = 0;
+    if constexpr (ES == 4) {
+        uint32_t* pre = (uint32_t*)bands;
+        if (wave == 0) split_prefix(bounds, (unsigned)V, nb, pre);
+        __syncthreads();
+        const uint64_t cut = split_cut(group + (lane & 1), gridDim.x, bounds, (unsigned)V, nb, tiles, pre);
+        run_lo = ((uint64_t)__builtin_amdgcn_readlane((int)(cut >> 32), 0) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)cut, 0);
+        run_hi = ((uint64_t)__builtin_amdgcn_readlane((int)(cut >> 32), 1) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)cut, 1);
+        range_end = (unsigned)(run_hi >> 32) + ((uint32_t)run_hi ? 1u : 0u);
+    }
     // (through the scalar cache: as a vector load, which the compiler picks because of the loads into LDS in between, the next
     // link would be waited for with every row load that is in flight)
     auto after = [&](unsigned item) -> unsigned {
+        if constexpr (ES == 4) return item + 1;
         return chain ? *(FGX_CONST_PTR(chain) + __builtin_amdgcn_readfirstlane(item)) : item + stride;
     };
 
@@ -404,15 +558,20 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
     auto seek = [&](Walk& w) {                      // settle on the first non-empty item at or after w.item
         w.live = false;
         while (w.item < range_end) {
-            const unsigned b = w.item / per_block, within = w.item % per_block;
-            const unsigned v = within / tiles;
-            const uint32_t lo = bounds[v * (nb + 1) + b], hi = bounds[v * (nb + 1) + b + 1];
+            // 16-bit: block-major (block, offset, tile); fp32: (tile, block, offset)
+            const unsigned unit = ES == 4 ? w.item % (nb * V) : w.item / tiles;
+            const unsigned tile = ES == 4 ? w.item / (nb * V) : w.item % tiles;
+            const unsigned b = unit / V, v = unit % V;
+            uint32_t lo = bounds[v * (nb + 1) + b], hi = bounds[v * (nb + 1) + b + 1];
+            if constexpr (ES == 4) {
+                if (w.item == (unsigned)(run_hi >> 32)) hi = lo + (uint32_t)run_hi;
+                if (w.item == (unsigned)(run_lo >> 32)) lo += (uint32_t)run_lo;
+            }
             if (lo < hi) {
                 w.k = lo;
                 w.k_hi = hi;
                 w.b = b;
                 w.v = v;
-                const unsigned tile = within % tiles;
                 w.co_tile = tile % co_tiles;
                 w.ci_tile = tile / co_tiles;
                 w.live = true;
@@ -429,7 +588,7 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
         }
     };
     Walk first;
-    first.item = lists ? lists[blockIdx.x] : xcd * per_xcd + slot;
+    first.item = ES == 4 ? (unsigned)(run_lo >> 32) : lists ? lists[blockIdx.x] : xcd * per_xcd + slot;
     seek(first);
     if (!first.live) return;                        // whole workgroup: nothing to do
 
@@ -447,13 +606,15 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
         uint32_t a_chb[C::A_PER], b_chb[C::B_PER];          // byte column inside the tile, swizzle applied
 #pragma unroll
         for (int i = 0; i < C::A_PER; ++i) {
-            a_row[i] = (i * C::NL + lw) * C::RPI_A + lane / C::CH_A;
-            a_chb[i] = (uint32_t)(((lane % C::CH_A) ^ C::key_a(a_row[i])) * 16);
+            const int piece = (i * C::NL + lw) * 64 + lane;     // of the operand's stage
+            a_row[i] = piece / C::CH_A;
+            a_chb[i] = (uint32_t)(((piece % C::CH_A) ^ C::key_a(a_row[i])) * 16);
         }
 #pragma unroll
         for (int i = 0; i < C::B_PER; ++i) {
-            b_row[i] = (i * C::NL + lw) * C::RPI_B + lane / C::CH_B;
-            b_chb[i] = (uint32_t)(((lane % C::CH_B) ^ C::key_b(b_row[i])) * 16);
+            const int piece = (i * C::NL + lw) * 64 + lane;
+            b_row[i] = piece / C::CH_B;
+            b_chb[i] = (uint32_t)(((piece % C::CH_B) ^ C::key_b(b_row[i])) * 16);
         }
         Walk f = first, r = first;                  // index stream, row stream
         unsigned f_step = 0, r_step = 0, r_stage = 0;       // steps handed out so far (index ring positions), row ring position
@@ -580,6 +741,9 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
     // multipliers
     // =================================================================================================
     __syncthreads();                                // the loaders' prologue barrier
+    if constexpr (ES == 4) {
+        multiply_f32<C>(ring, first, seek, after, wave_m, wave_n, group, partial);
+    } else {
     const int s16 = lane & 15, mb = (lane >> 4) & 1;
     constexpr int NK = P / 16 / C::SLICES;          // k-blocks (16 pair rows) this wavefront multiplies per step
     const int kk0 = C::KSPLIT ? mw * NK : 0;        // ... starting at this one
@@ -747,6 +911,7 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
         m.k = m.k_hi;                               // on to the next non-empty item
         m.item = after(m.item);
         seek(m);
+    }
     }
 }
 
@@ -1319,7 +1484,7 @@ int launch_wgrad_stream(const void* gout, const void* feats, const uint32_t* sig
         kern<<<groups, C::NT, C::lds_bytes, s>>>((const T*)gout, (const T*)feats, sig_i, sig_o, bounds, V, Ci, Co, L.nb, co_tiles,
                                                  ci_tiles, tab.seg[V], (uint32_t)(n * (size_t)Co * sizeof(T)),
                                                  (uint32_t)(n_in * (size_t)Ci * sizeof(T)), partial, direct ? (T*)gw : nullptr,
-                                                 bias_partial, bias.offset, lists);
+                                                 bias_partial, bias.offset, lists, 1u, 1u);
         FGX_CHECK_LAUNCH("fgx_conv_wgrad(stream)");
         if (bias_partial) {
             bias_reduce_kernel<T><<<cdiv((size_t)Co, 32), 1024, 0, s>>>(bias_partial, bounds + (size_t)bias.offset * (L.nb + 1),
@@ -1331,7 +1496,7 @@ int launch_wgrad_stream(const void* gout, const void* feats, const uint32_t* sig
     return launch_reduce<T>(partial, bounds, V, Ci, Co, L.nb * C::SLICES, (unsigned)C::SLICES, (T*)gw, s);
 }
 
-// the streaming kernel: 16-bit types, tiles of 128x128 or 64x64, operands addressable with 32-bit offsets
+// the streaming kernel: 16-bit types, the tiles that exist, operands addressable with 32-bit offsets
 template <typename Tag>
 bool stream_ok(int tile_rows, int tile_cols, size_t n, size_t n_in, int Ci, int Co, uint32_t n_pairs) {
     if (sizeof(typename Tag::type) != 2) return false;
@@ -1381,7 +1546,140 @@ int dispatch_wgrad(int tile_rows, int tile_cols, const void* gout, const void* f
 
 using namespace fgx;
 
+namespace fgx {
+namespace {
+
+// grad_weight of one (offset, tile) from the segments' partial products: every workgroup finds the slots of its tile in the order
+// of the pairs (the cuts are those of the product), then a thread adds up one 16-byte piece.  Bound by reading the slots.
+__global__ void __launch_bounds__(256) split_reduce_kernel(const float* __restrict__ partial, const uint32_t* __restrict__ bounds, unsigned V,
+                                                           unsigned nb, unsigned co_tiles, unsigned ci_tiles, unsigned groups, int tile, int Ci,
+                                                           int Co, float* __restrict__ gw) {
+    __shared__ uint32_t pre[kSplitMaxUnits + 1];
+    __shared__ uint64_t cut[kSplitMaxGroups + 1];
+    __shared__ uint32_t slots[kSplitMaxGroups + kSplitMaxUnits];
+    __shared__ uint32_t count;
+    const unsigned tiles = co_tiles * ci_tiles, v = blockIdx.x / tiles, t = blockIdx.x % tiles, tid = threadIdx.x;
+    if (tid < 64) split_prefix(bounds, V, nb, pre);
+    __syncthreads();
+    for (unsigned w = tid; w <= groups; w += 256) cut[w] = split_cut(w, groups, bounds, V, nb, tiles, pre);
+    __syncthreads();
+    if (tid < 64) {
+        uint32_t before = 0;
+        for (unsigned b0 = 0; b0 < nb; b0 += 64) {
+            const unsigned b = b0 + tid;
+            const unsigned item = (t * nb + b) * V + v;
+            const uint64_t start = (uint64_t)item << 32, end = (uint64_t)(item + 1) << 32;
+            unsigned w0 = 0, mine = 0;
+            const bool any = b < nb && bounds[v * (nb + 1) + b] < bounds[v * (nb + 1) + b + 1];
+            if (any) {
+                unsigned hi = groups;                       // the last workgroup that starts at or before the item
+                while (w0 + 1 < hi) {
+                    const unsigned mid = (w0 + hi) / 2;
+                    if (cut[mid] <= start) w0 = mid;
+                    else hi = mid;
+                }
+                for (unsigned w = w0; w < groups && cut[w] < end; ++w) mine += cut[w] < cut[w + 1] && cut[w + 1] > start;
+            }
+            uint32_t upto = mine;
+#pragma unroll
+            for (int d = 1; d < 64; d *= 2) {
+                const uint32_t o = __shfl_up(upto, d);
+                upto += tid >= (unsigned)d ? o : 0u;
+            }
+            uint32_t at = before + upto - mine;
+            if (any)
+                for (unsigned w = w0; w < groups && cut[w] < end; ++w)
+                    if (cut[w] < cut[w + 1] && cut[w + 1] > start) slots[at++] = w + item;
+            before += __shfl(upto, 63);
+        }
+        if (tid == 0) count = before;
+    }
+    __syncthreads();
+    using f32x4 = float __attribute__((ext_vector_type(4)));
+    const int piece = (int)(blockIdx.y * 256 + tid), per_row = tile / 4;
+    if (piece >= tile * per_row) return;
+    const int co = (int)(t % co_tiles) * tile + piece / per_row, ci = (int)(t / co_tiles) * tile + piece % per_row * 4;
+    if (co >= Co || ci >= Ci) return;
+    const size_t size = (size_t)tile * tile;
+    const float* src = partial + (size_t)piece * 4;
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    unsigned i = 0;
+    for (; i + 8 <= count; i += 8) {
+        f32x4 x[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) x[k] = *(const f32x4*)(src + slots[i + k] * size);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) sum += x[k];
+    }
+    for (; i < count; ++i) sum += *(const f32x4*)(src + slots[i] * size);
+    float* dst = gw + ((size_t)co * V + v) * Ci + ci;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dst[e] = sum[e];
+}
+
+template <int TILE>
+int launch_wgrad_split(const void* gout, const void* feats, const uint32_t* sig_i, const uint32_t* sig_o, const uint32_t* bounds, uint32_t pairs,
+                       size_t n, size_t n_in, int V, int Ci, int Co, unsigned nb, unsigned groups, float* partial, float* gw, hipStream_t s) {
+    using C = WStreamCfg<F32, TILE, TILE>;
+    const unsigned co_tiles = cdiv(Co, TILE), ci_tiles = cdiv(Ci, TILE);
+    auto kern = wgrad_stream_kernel<F32, TILE, TILE>;
+    static thread_local bool lds_raised = false;
+    if (!lds_raised) {
+        FGX_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::lds_bytes));
+        lds_raised = true;
+    }
+    // run w starts at (w * tiles mod groups) / groups of a tile: `copies` runs at every such place, and the place after the first
+    // belongs to run `step`
+    const unsigned tiles = co_tiles * ci_tiles;
+    const unsigned copies = std::gcd(tiles, groups), spread = groups / copies;
+    unsigned step = 1;
+    while (spread > 1 && (size_t)step * (tiles / copies) % spread != 1) ++step;
+    kern<<<groups, C::NT, C::lds_bytes, s>>>((const float*)gout, (const float*)feats, sig_i, sig_o, bounds, V, Ci, Co, nb, co_tiles, ci_tiles, pairs,
+                                             (uint32_t)(n * (size_t)Co * 4), (uint32_t)(n_in * (size_t)Ci * 4), partial, nullptr, nullptr, -1, nullptr, copies, step);
+    FGX_CHECK_LAUNCH("fgx_conv_wgrad_split");
+    split_reduce_kernel<<<dim3((unsigned)V * co_tiles * ci_tiles, TILE * TILE / 4 / 256), 256, 0, s>>>(partial, bounds, (unsigned)V, nb, co_tiles,
+                                                                                                      ci_tiles, groups, TILE, Ci, Co, gw);
+    FGX_CHECK_LAUNCH("fgx_conv_wgrad_split(reduce)");
+    return FGX_OK;
+}
+
+}  // namespace
+}  // namespace fgx
+
 extern "C" {
+
+size_t fgx_conv_wgrad_split_scratch_bytes(size_t n, size_t n_in, uint32_t n_pairs, int V, int Ci, int Co, int tile, int block_rows) {
+    if (V < 1 || V > kMaxV || Ci <= 0 || Co <= 0 || Ci % 4 || Co % 4 || block_rows <= 0 || n == 0 || !(tile == 64 || tile == 96)) return 0;
+    const size_t nb = cdiv(n, (size_t)block_rows), units = nb * V, tiles = (size_t)cdiv(Co, tile) * cdiv(Ci, tile);
+    if (units > kSplitMaxUnits || units * tiles > (size_t)1 << 20) return 0;
+    if (((double)n_pairs + (double)units * kSplitItemCost) * tiles >= 4294967296.0) return 0;         // costs are 32-bit numbers
+    if ((double)n * Co * 4 > (double)kOobOffset || (double)n_in * Ci * 4 > (double)kOobOffset || (double)n_pairs * 4 + 256 > (double)kOobOffset) return 0;
+    return align_up((kSplitMaxGroups + units * tiles) * tile * tile * 4, 256) + fgx_colsum_scratch_bytes(n, Co);
+}
+
+int fgx_conv_wgrad_split(const void* grad_out, const void* feats, const uint32_t* sig_i, const uint32_t* sig_o, const uint32_t* seg_host,
+                         const uint32_t* block_bounds, size_t n, size_t n_in, int Ci, int Co, int V, int tile, int block_rows, void* scratch,
+                         void* grad_weight, void* grad_bias, fgx_stream_t stream) {
+    FGX_CHECK_ARG(seg_host && V >= 1 && V <= kMaxV, "fgx_conv_wgrad_split: bad V=%d or no segment table", V);
+    for (int v = 0; v < V; ++v) FGX_CHECK_ARG(seg_host[v + 1] >= seg_host[v], "fgx_conv_wgrad_split: segment table is not monotone");
+    const size_t bytes = fgx_conv_wgrad_split_scratch_bytes(n, n_in, seg_host[V], V, Ci, Co, tile, block_rows);
+    FGX_CHECK_ARG(bytes > 0, "fgx_conv_wgrad_split: not for this shape (fgx_conv_wgrad_split_scratch_bytes says 0)");
+    FGX_CHECK_ARG(grad_out && feats && sig_i && sig_o && block_bounds && scratch && grad_weight, "fgx_conv_wgrad_split: null buffer");
+    FGX_CHECK_ARG((((uintptr_t)grad_out | (uintptr_t)feats) & 15) == 0, "fgx_conv_wgrad_split: grad_out and feats must be 16-byte aligned");
+    FGX_CHECK_ARG(((uintptr_t)scratch & 255) == 0, "fgx_conv_wgrad_split: scratch must be 256-byte aligned");
+    unsigned groups = 0;
+    int rc = stream_groups(&groups);
+    if (rc != FGX_OK) return rc;
+    if (groups > kSplitMaxGroups) groups = kSplitMaxGroups;
+    const unsigned nb = (unsigned)cdiv(n, (size_t)block_rows);
+    if (grad_bias) {
+        rc = fgx_colsum(FGX_F32, grad_out, n, Co, (char*)scratch + (bytes - fgx_colsum_scratch_bytes(n, Co)), grad_bias, stream);
+        if (rc != FGX_OK) return rc;
+    }
+    auto launch = tile == 96 ? launch_wgrad_split<96> : launch_wgrad_split<64>;
+    return launch(grad_out, feats, sig_i, sig_o, block_bounds, seg_host[V], n, n_in, V, Ci, Co, nb, groups, (float*)scratch, (float*)grad_weight,
+                  (hipStream_t)stream);
+}
 
 size_t fgx_wgrad_scratch_bytes(size_t n, int V, int Ci, int Co, int block_rows) {
     if (V < 1 || V > kMaxV || Ci <= 0 || Co <= 0 || block_rows <= 0) return 0;
@@ -1474,6 +1772,8 @@ int fgx_conv_wgrad_lists(int dtype, const void* grad_out, const void* feats, con
     }
     const bool stream_f16 = streaming && any && dtype == FGX_F16 && stream_ok<F16>(tile_rows, tile_cols, n, n_in, Ci, Co, tab.seg[V]);
     const bool stream_bf16 = streaming && any && dtype == FGX_BF16 && stream_ok<BF16>(tile_rows, tile_cols, n, n_in, Ci, Co, tab.seg[V]);
+    if (streaming && dtype == FGX_F32 && tile_rows == 96 && tile_cols == 96)
+        tile_rows = tile_cols = 32;         // a schedule for fgx_conv_wgrad_split, whose tile no other kernel has
     Layout L = layout(any ? n : 0, V, Ci, Co, block_rows, (stream_f16 || stream_bf16) && tile_rows == 32 ? 4 : 1);
     // 32-bit byte offsets into grad_out / feats are enough below 4 GiB
     const bool small = (double)n * Co * es < 4294967296.0 && (double)n_in * Ci * es < 4294967296.0;
