@@ -547,6 +547,35 @@ __global__ void __launch_bounds__(256) splitk_reduce4_kernel(const f32x4* __rest
     }
 }
 
+// Rows widened with zeros or cut, in units of U, PER of them (16 bytes) a thread where the new rows are whole pieces.  Bound by the
+// launch for the few hundred thousand rows that have such channel counts: one pass where a fill and a strided copy take two (a
+// training step of 6 -> 48 channels over three 192^3 shells had three fills and four copies of 3.9 and 4.7 us: 0.181 ms, now 0.167).
+template <typename U, int PER>
+__global__ void __launch_bounds__(256) copy_columns_kernel(const U* __restrict__ src, size_t pieces, unsigned src_cols, unsigned pieces_per_row,
+                                                           U* __restrict__ dst) {
+    struct alignas(sizeof(U) * PER) Piece { U u[PER]; };
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < pieces; i += (size_t)gridDim.x * 256) {
+        const size_t row = pieces >> 32 ? i / pieces_per_row : (uint32_t)i / pieces_per_row;
+        const unsigned c0 = (unsigned)(i - row * pieces_per_row) * PER;
+        const U* from = src + row * src_cols;
+        Piece p;
+#pragma unroll
+        for (int e = 0; e < PER; ++e) p.u[e] = c0 + e < src_cols ? from[c0 + e] : U(0);
+        ((Piece*)dst)[i] = p;
+    }
+}
+
+template <typename U>
+void launch_copy_columns(const void* src, size_t rows, size_t src_bytes, void* dst, size_t dst_bytes, hipStream_t s) {
+    constexpr int PER = 16 / (int)sizeof(U);
+    const bool whole = dst_bytes % 16 == 0 && ((uintptr_t)dst & 15) == 0;
+    const size_t per_row = dst_bytes / (whole ? 16 : sizeof(U)), pieces = rows * per_row;
+    unsigned grid = cdiv(pieces, 256);
+    if (grid > 16384u) grid = 16384u;
+    if (whole) copy_columns_kernel<U, PER><<<grid, 256, 0, s>>>((const U*)src, pieces, (unsigned)(src_bytes / sizeof(U)), (unsigned)per_row, (U*)dst);
+    else copy_columns_kernel<U, 1><<<grid, 256, 0, s>>>((const U*)src, pieces, (unsigned)(src_bytes / sizeof(U)), (unsigned)per_row, (U*)dst);
+}
+
 // out[8 i .. 8 i + 7] = grad[...] where bit t of mask[i] is set, else 0 (16-bit elements: one 16-byte piece per lane)
 __global__ void __launch_bounds__(256) relu_mask_apply_kernel(const u32x4* __restrict__ grad, const uint8_t* __restrict__ mask,
                                                               size_t pieces, u32x4* __restrict__ out) {
@@ -907,6 +936,20 @@ int fgx_relu_mask_apply(int dtype, const void* grad, const uint8_t* relu_mask, s
     if (grid > 16384u) grid = 16384u;
     relu_mask_apply_kernel<<<grid, 256, 0, (hipStream_t)stream>>>((const u32x4*)grad, relu_mask, pieces, (u32x4*)out);
     FGX_CHECK_LAUNCH("fgx_relu_mask_apply");
+    return FGX_OK;
+}
+
+int fgx_copy_columns(int elem_bytes, const void* src, size_t rows, int src_cols, void* dst, int dst_cols, fgx_stream_t stream) {
+    FGX_CHECK_ARG((elem_bytes == 2 || elem_bytes == 4) && src_cols > 0 && dst_cols > 0, "fgx_copy_columns: %d -> %d columns of %d bytes", src_cols,
+                  dst_cols, elem_bytes);
+    FGX_CHECK_ARG(rows < ((size_t)1 << 36), "fgx_copy_columns: too many rows");
+    if (rows == 0) return FGX_OK;
+    FGX_CHECK_ARG(src && dst, "fgx_copy_columns: null buffer");
+    FGX_CHECK_ARG((((uintptr_t)src | (uintptr_t)dst) & (elem_bytes - 1)) == 0, "fgx_copy_columns: elements are not aligned");
+    const size_t sb = (size_t)src_cols * elem_bytes, db = (size_t)dst_cols * elem_bytes;
+    if (((sb | db) & 3) == 0 && (((uintptr_t)src | (uintptr_t)dst) & 3) == 0) launch_copy_columns<uint32_t>(src, rows, sb, dst, db, (hipStream_t)stream);
+    else launch_copy_columns<uint16_t>(src, rows, sb, dst, db, (hipStream_t)stream);
+    FGX_CHECK_LAUNCH("fgx_copy_columns");
     return FGX_OK;
 }
 

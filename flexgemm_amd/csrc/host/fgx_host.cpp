@@ -41,7 +41,7 @@ namespace {
     X(fgx_spconv_out_coords_grid_emit) X(fgx_tile_plan) X(fgx_gather_item_order) X(fgx_gather_item_order_workspace_bytes)          \
     X(fgx_weight_panel_bytes) X(fgx_pack_weight) X(fgx_conv_scratch_bytes) X(fgx_conv_gather_gemm_act_mask)                        \
     X(fgx_conv_gather_gemm_weight_pays) X(fgx_conv_gather_gemm_weight) X(fgx_conv_gemm_pairs_pays) X(fgx_pair_plan_words) X(fgx_pair_plan) X(fgx_conv_gemm_pairs_scratch_bytes) X(fgx_conv_gemm_pairs)                                                             \
-    X(fgx_conv_gather_gemm_stream_act_mask) X(fgx_conv_gather_gemm_stream_groups) X(fgx_relu_mask_apply)                           \
+    X(fgx_conv_gather_gemm_stream_act_mask) X(fgx_conv_gather_gemm_stream_groups) X(fgx_relu_mask_apply) X(fgx_copy_columns)       \
     X(fgx_colsum_scratch_bytes) X(fgx_colsum) X(fgx_wgrad_block_bounds_count) X(fgx_wgrad_block_bounds)                            \
     X(fgx_conv_gemm_stem_pays) X(fgx_conv_gemm_stem) X(fgx_wgrad_stem_pays) X(fgx_wgrad_stem_scratch_bytes) X(fgx_conv_wgrad_stem) X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
     X(fgx_conv_wgrad_split_scratch_bytes) X(fgx_conv_wgrad_split)                                                                  \
@@ -606,9 +606,26 @@ bool narrow_shape(const Cache& c, int es, int k, int cols, int v, int64_t n) {
            py::reinterpret_borrow<py::object>(module_get(g_spconv, "NARROW_RESIDENT")).cast<std::string>() != "auto";
 }
 
-Tensor pad_columns(const Tensor& t, int64_t multiple) {
-    const int64_t pad = (multiple - t.size(-1) % multiple) % multiple;
-    return pad ? at::constant_pad_nd(t, {0, pad}) : t;
+// A contiguous tensor of rows of `cols` elements as one of `sizes` with rows of `out_cols`: filled up with zeros, or cut.
+Tensor copy_columns(const Tensor& t, int64_t rows, int64_t cols, at::IntArrayRef sizes, int64_t out_cols, int64_t stream) {
+    Tensor out = make(sizes, t.scalar_type(), t.device());
+    if (rows > 0) check(L.fgx_copy_columns((int)t.element_size(), ptr(t), (size_t)rows, (int)cols, ptr(out), (int)out_cols, as_stream(stream)));
+    return out;
+}
+
+// `dim` (the last one, or the first of a contiguous tensor) filled up with zeros to a multiple
+Tensor pad_to(const Tensor& t, int64_t dim, int64_t multiple, int64_t stream) {
+    const int64_t size = t.size(dim), padded = (size + multiple - 1) / multiple * multiple;
+    if (padded == size) return t;
+    std::vector<int64_t> sizes = t.sizes().vec();
+    sizes[dim] = padded;
+    const int64_t rows = dim == 0 ? 1 : t.numel() / std::max<int64_t>(size, 1), cols = dim == 0 ? t.numel() : size;
+    if (cols == 0 || (dim == 0 ? cols / size * padded : padded) > INT32_MAX) {          // (no elements, or past the kernel's 32-bit widths)
+        std::vector<int64_t> pad(2 * (t.dim() - dim), 0);
+        pad.back() = padded - size;
+        return at::constant_pad_nd(t, pad);
+    }
+    return copy_columns(t.contiguous(), rows, cols, sizes, dim == 0 ? cols / size * padded : padded, stream);
 }
 
 // What a kernel would otherwise find out by reading past a buffer or on another device.
@@ -655,8 +672,8 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
     }
     const int align = 16 / es;
     if (weight.size(mode == 0 ? 2 : 0) % align) {       // rows must be whole 16-byte pieces
-        src = pad_columns(src, align);
-        weight = mode == 0 ? pad_columns(weight, align) : at::constant_pad_nd(weight, {0, 0, 0, 0, 0, (align - weight.size(0) % align) % align});
+        src = pad_to(src, 1, align, stream);
+        weight = pad_to(weight, mode == 0 ? 2 : 0, align, stream);
     }
     src = src.contiguous();
     weight = weight.contiguous();
@@ -853,8 +870,8 @@ WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool 
     }
     const int64_t n = grad.size(0), n_in = feats.size(0), true_ci = feats.size(1), true_co = grad.size(1);
     const int es = (int)feats.element_size(), align = 16 / es;
-    feats = pad_columns(feats, align).contiguous();
-    grad = pad_columns(grad, align).contiguous();
+    feats = pad_to(feats, 1, align, stream).contiguous();
+    grad = pad_to(grad, 1, align, stream).contiguous();
     const int ci = (int)feats.size(1), co = (int)grad.size(1);
     WeightGrads w;
     if (n > 0 && narrow_shape(c, es, ci, co, v, n) && impl_function("_narrow_wgrad_applies")(c.obj, feats, ci, co, v, n, n_in).cast<bool>()) {
@@ -921,7 +938,8 @@ WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool 
         mark("wgrad", "stop");
     }
     if (ci != true_ci || co != true_co) {
-        w.weight = w.weight.slice(0, 0, true_co).slice(2, 0, true_ci).contiguous();
+        w.weight = w.weight.slice(0, 0, true_co).contiguous();              // (a view: whole rows)
+        if (ci != true_ci) w.weight = copy_columns(w.weight, true_co * v, ci, {true_co, v, true_ci}, true_ci, stream);
         if (with_bias) w.bias = w.bias.slice(0, 0, true_co).contiguous();
     }
     return w;

@@ -317,6 +317,10 @@ int fgx_conv_gemm_pairs(int dtype, int mode, const void* src, const void* weight
  * read beside the gradient.  No counterpart in the reference. */
 int fgx_relu_mask_apply(int dtype, const void* grad, const uint8_t* relu_mask, size_t numel, void* out, fgx_stream_t stream);
 
+/* dst[r][c] = c < src_cols ? src[r][c] : 0 for c < dst_cols: rows filled up with zeros to whole 16-byte pieces, or cut back to what the
+ * caller's tensors have.  elem_bytes 2 or 4; src and dst must not overlap.  One pass. */
+int fgx_copy_columns(int elem_bytes, const void* src, size_t rows, int src_cols, void* dst, int dst_cols, fgx_stream_t stream);
+
 /* Gather plan of a row order for tiles of `tile_rows` rows: for tile t and the k-th offset v present in it
  * (the set bits of tile_code[t], ascending; a tile whose code is 0 gets one row with every neighbor missing),
  *   plan_idx[(plan_seg[t] + k) * tile_rows + r] = map[order[t * tile_rows + r], v]     (0xFFFFFFFF for rows past n),
