@@ -368,82 +368,6 @@ __global__ void __launch_bounds__(kBlock) tile_fill_kernel(const int32_t* __rest
     }
 }
 
-// One workgroup per tile: plan_idx[seg[t] + k][r] = map[order[t * tile_rows + r]][k-th offset present in the tile]
-// (EMPTY for rows past the end); plan_band[seg[t] + k] (optional) has bit b set when rows [32 b, 32 b + 32) of the
-// tile hold at least one present neighbor for that offset.
-__global__ void __launch_bounds__(kBlock) plan_fill_kernel(const uint32_t* __restrict__ map,
-                                                           const int64_t* __restrict__ order,
-                                                           const int32_t* __restrict__ tile_code,
-                                                           const int32_t* __restrict__ seg, size_t n, int V, int tile_rows,
-                                                           uint32_t* __restrict__ plan_idx, uint32_t* __restrict__ plan_band) {
-    __shared__ uint32_t bands[32];
-    __shared__ uint32_t stage[kBlock * 32];      // kBlock map rows of V <= 32 words
-    __shared__ int64_t src_row[kBlock];          // which map row each of them is (-1: past the end)
-    const size_t t = blockIdx.x;
-    uint32_t code = (uint32_t)tile_code[t];
-    size_t slot = (size_t)seg[t];
-    if (code == 0) {
-        for (int r = threadIdx.x; r < tile_rows; r += kBlock) plan_idx[slot * tile_rows + r] = FGX_EMPTY32;
-        if (plan_band != nullptr && threadIdx.x == 0) plan_band[slot] = 0u;
-        return;
-    }
-    if (threadIdx.x < 32) bands[threadIdx.x] = 0u;
-    const int lane = threadIdx.x & 63;
-    for (int r0 = 0; r0 < tile_rows; r0 += kBlock) {
-        // The rows of this tile sit wherever the mask order put them.  A half-wave fetches one whole row (V consecutive
-        // words: one or two cache lines per request) into LDS; each thread then walks its own row there.  One thread
-        // per row reading straight from memory would ask for 64 different cache lines with every load instruction.
-        __syncthreads();                         // the previous chunk's rows have been consumed; bands[] is cleared
-        {
-            const size_t row = t * (size_t)tile_rows + r0 + threadIdx.x;
-            src_row[threadIdx.x] = (r0 + (int)threadIdx.x < tile_rows && row < n) ? order[row] : (int64_t)-1;
-        }
-        __syncthreads();
-        for (int i0 = 0; i0 < kBlock * 32; i0 += 8 * kBlock) {       // eight loads in flight per thread
-            uint32_t t8[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int i = i0 + q * kBlock + threadIdx.x;
-                const int64_t src = src_row[i >> 5];
-                t8[q] = ((i & 31) < V && src >= 0) ? map[(size_t)src * V + (i & 31)] : FGX_EMPTY32;
-            }
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int i = i0 + q * kBlock + threadIdx.x;
-                if ((i & 31) < V) stage[(i >> 5) * V + (i & 31)] = t8[q];
-            }
-        }
-        __syncthreads();
-        const int r = r0 + threadIdx.x;
-        const uint32_t* mrow = src_row[threadIdx.x] >= 0 ? stage + threadIdx.x * V : nullptr;
-        uint32_t c = code;
-        size_t s = slot;
-        int k = 0;
-        while (c) {
-            const int v = __ffs((int)c) - 1;
-            c &= c - 1;
-            const uint32_t m = mrow ? mrow[v] : FGX_EMPTY32;
-            if (r < tile_rows) plan_idx[s * tile_rows + r] = m;
-            if (plan_band != nullptr) {
-                const unsigned long long live = __ballot(m != FGX_EMPTY32);    // all 64 lanes take part
-                if (lane == 0) {
-                    const int b0 = (r0 + (int)(threadIdx.x & ~63u)) >> 5;          // band of this wavefront's lanes 0-31
-                    uint32_t bits = ((live & 0xFFFFFFFFull) ? 1u : 0u) << (b0 & 31);
-                    bits |= ((live >> 32) ? 1u : 0u) << ((b0 + 1) & 31);
-                    if (bits) atomicOr(&bands[k], bits);
-                }
-            }
-            ++s;
-            ++k;
-        }
-    }
-    if (plan_band != nullptr) {
-        __syncthreads();
-        const int cnt = __popc(code);
-        if ((int)threadIdx.x < cnt) plan_band[slot + threadIdx.x] = bands[threadIdx.x];
-    }
-}
-
 // ---------------------------------------------------------------------------------------------------------------
 // The tables over all row tiles, by one workgroup: where each tile's public offset list and its gather-plan rows start, and
 // the item order of the streaming GEMM.
@@ -464,15 +388,16 @@ __device__ __forceinline__ unsigned tile_cost_bin(uint32_t code) { return 32u - 
 
 // A sorted item carries its cost above 26 bits of its number; WIDE: more items than that, whose cost is looked up again.
 constexpr unsigned kItemBits = 26;
-template <bool WIDE>
+template <bool WIDE, int THREADS>
 __device__ void order_items(const int32_t* __restrict__ tile_code, unsigned num_tiles, unsigned col_tiles, unsigned slabs, unsigned groups,
                             uint32_t* __restrict__ sorted, uint32_t* __restrict__ item_at) {
-    __shared__ uint32_t count[kOrderWaves][64];
-    __shared__ __attribute__((aligned(16))) uint32_t load[kOrderThreads];
+    constexpr int WAVES = THREADS / 64;
+    __shared__ uint32_t count[WAVES][64];
+    __shared__ __attribute__((aligned(16))) uint32_t load[THREADS];
     const unsigned tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const unsigned total = num_tiles * col_tiles;
     const unsigned long long below = (1ull << lane) - 1ull;
-    const unsigned piece = ((total + kOrderWaves - 1) / kOrderWaves + 63u) & ~63u;
+    const unsigned piece = ((total + WAVES - 1) / WAVES + 63u) & ~63u;
     const unsigned lo = wave * piece < total ? wave * piece : total, hi = lo + piece < total ? lo + piece : total;
     auto bin_of = [&](unsigned item) -> unsigned { return tile_cost_bin((uint32_t)tile_code[col_tiles == 1 ? item : item / col_tiles]); };
     // ---- step 1: stable counting sort, cost descending ----
@@ -485,9 +410,9 @@ __device__ void order_items(const int32_t* __restrict__ tile_code, unsigned num_
     }
     __syncthreads();
     if (wave == 0) {                                              // lane = bin
-        uint32_t mine = 0u, before[kOrderWaves];
+        uint32_t mine = 0u, before[WAVES];
 #pragma unroll
-        for (int w = 0; w < kOrderWaves; ++w) {
+        for (int w = 0; w < WAVES; ++w) {
             before[w] = mine;
             mine += count[w][lane];
         }
@@ -498,7 +423,7 @@ __device__ void order_items(const int32_t* __restrict__ tile_code, unsigned num_
             if ((int)lane >= d) incl += o;
         }
 #pragma unroll
-        for (int w = 0; w < kOrderWaves; ++w) count[w][lane] = incl - mine + before[w];
+        for (int w = 0; w < WAVES; ++w) count[w][lane] = incl - mine + before[w];
     }
     __syncthreads();
     for (unsigned i0 = lo; i0 < hi; i0 += 64) {
@@ -527,7 +452,7 @@ __device__ void order_items(const int32_t* __restrict__ tile_code, unsigned num_
         return ((pc ? pc : 1u) * slabs + 3u) >> scale;
     };
     // P threads per slot share the counting
-    const unsigned P = groups <= kOrderThreads / 4 ? 4u : (groups <= kOrderThreads / 2 ? 2u : 1u);
+    const unsigned P = groups <= THREADS / 4 ? 4u : (groups <= THREADS / 2 ? 2u : 1u);
     const unsigned slot = tid / P, part = tid % P;
     uint32_t mine = slot;
     if (slot < rem) {                                             // cheapest items: the positions of the last round
@@ -601,9 +526,9 @@ __global__ void __launch_bounds__(kOrderThreads) tile_tables_kernel(const int32_
     }
     if (item_at == nullptr) return;
     if ((unsigned long long)num_tiles * col_tiles < (1ull << kItemBits))
-        order_items<false>(tile_code, num_tiles, col_tiles, slabs, groups, num_tiles * col_tiles <= kOrderInLds ? sorted_lds : sorted, item_at);
+        order_items<false, kOrderThreads>(tile_code, num_tiles, col_tiles, slabs, groups, num_tiles * col_tiles <= kOrderInLds ? sorted_lds : sorted, item_at);
     else
-        order_items<true>(tile_code, num_tiles, col_tiles, slabs, groups, sorted, item_at);
+        order_items<true, kOrderThreads>(tile_code, num_tiles, col_tiles, slabs, groups, sorted, item_at);
 }
 
 // The segment tables of many tiles, in chunks: a chunk's sums are left in its last entries of the tables, one workgroup adds them up
@@ -671,6 +596,137 @@ __global__ void __launch_bounds__(kOrderThreads) chunk_tables_kernel(const int32
         run.plan_at += all.plan_at;
     }
 }
+
+// ---------------------------------------------------------------------------------------------------------------
+// One workgroup per tile: plan_idx[plan_seg[t] + k][r] = map[order[t * tile_rows + r]][k-th offset present in the tile]
+// (EMPTY for rows past the end); plan_band[plan_seg[t] + k] (optional) has bit b set when rows [32 b, 32 b + 32) of the
+// tile hold at least one present neighbor for that offset.
+//
+// The tile's rows sit wherever the mask order put them: a half-wave fetches one whole row (V consecutive words: one or two cache
+// lines per request) into LDS, and kFillThreads / R threads share a row's offsets.  Bound by latency: with 256 threads a tile, each
+// of them walking all offsets of its row, 1 306 tiles of 128 rows took 18.4 us.  512 threads and no more LDS than the rows need
+// put four tiles on a CU at a time (1024 threads, two tiles: 29 us with the tables below).
+//
+// TABLES: a workgroup adds up the counts of the tiles before its own itself (and leaves them in seg and plan_seg), and the first one
+// (item_at) deals the item order beside them.  One workgroup that scanned and dealt before the others could start took 15.7 us for
+// 1 306 tiles: tables and fill 34.1 -> 17.8 us (and for the two maps of a 2 x 2 x 2 stride over a 256^3 shell 34.0 -> 18.3).  Up to
+// kFillScanTiles tiles: the additions are quadratic.
+// ---------------------------------------------------------------------------------------------------------------
+constexpr int kFillThreads = 512, kFillRows = 256;
+constexpr unsigned kFillScanTiles = 4096;
+
+template <bool TABLES>
+__global__ void __launch_bounds__(kFillThreads) plan_fill_kernel(const uint32_t* __restrict__ map, const int64_t* __restrict__ order,
+                                                                 const int32_t* __restrict__ tile_code, size_t num_tiles, size_t n, int V,
+                                                                 int tile_rows, int R, int32_t* __restrict__ seg, int32_t* __restrict__ plan_seg,
+                                                                 uint32_t* __restrict__ plan_idx, uint32_t* __restrict__ plan_band,
+                                                                 unsigned col_tiles, unsigned slabs, unsigned groups, uint32_t* __restrict__ sorted,
+                                                                 uint32_t* __restrict__ item_at) {
+    extern __shared__ uint32_t stage[];              // R map rows of V words; the item order's sorted list in the workgroup that makes it
+    __shared__ int64_t src_row[kFillRows];           // which map row each of them is (-1: past the end)
+    __shared__ uint32_t bands[32], offsets[32];
+    const int tid = threadIdx.x, lane = tid & 63;
+    size_t t = blockIdx.x;
+    if constexpr (TABLES) {
+        if (item_at != nullptr) {
+            if (t == 0) {
+                order_items<false, kFillThreads>(tile_code, (unsigned)num_tiles, col_tiles, slabs, groups,
+                                                 num_tiles * col_tiles <= kOrderInLds ? stage : sorted, item_at);
+                return;
+            }
+            --t;
+        }
+    }
+    auto fetch_order = [&](int r0) {
+        if (tid < R) {
+            const size_t row = t * (size_t)tile_rows + r0 + tid;
+            src_row[tid] = (r0 + tid < tile_rows && row < n) ? order[row] : (int64_t)-1;
+        }
+    };
+    fetch_order(0);
+    size_t slot;
+    if constexpr (TABLES) {
+        __shared__ uint64_t part[kFillThreads / 64];
+        uint64_t mine = 0;                           // offsets of the tiles before this one | their plan rows (at most 32 each)
+        for (unsigned q = tid; q < (unsigned)t; q += kFillThreads) {
+            const TilePrefix c = tile_counts(tile_code, q, (unsigned)num_tiles);
+            mine += (uint64_t)c.at << 32 | c.plan_at;
+        }
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) mine += (uint64_t)__shfl_xor((unsigned long long)mine, d, 64);
+        if (lane == 0) part[tid >> 6] = mine;
+        __syncthreads();
+        uint64_t before = 0;
+#pragma unroll
+        for (int w = 0; w < kFillThreads / 64; ++w) before += part[w];
+        slot = (uint32_t)before;
+        const TilePrefix own = tile_counts(tile_code, (unsigned)t, (unsigned)num_tiles);
+        if (tid == 0) {
+            if (seg != nullptr) seg[t] = (int32_t)(before >> 32);
+            plan_seg[t] = (int32_t)slot;
+            if (t + 1 == num_tiles) {
+                if (seg != nullptr) seg[num_tiles] = (int32_t)((before >> 32) + own.at);
+                plan_seg[num_tiles] = (int32_t)(slot + own.plan_at);
+            }
+        }
+    } else {
+        slot = (size_t)plan_seg[t];
+    }
+    const uint32_t code = (uint32_t)tile_code[t];
+    if (code == 0) {
+        for (int r = tid; r < tile_rows; r += kFillThreads) plan_idx[slot * tile_rows + r] = FGX_EMPTY32;
+        if (plan_band != nullptr && tid == 0) plan_band[slot] = 0u;
+        return;
+    }
+    if (tid < 32) {
+        bands[tid] = 0u;
+        if (code >> tid & 1u) offsets[__popc(code & ((1u << tid) - 1u))] = (uint32_t)tid;
+    }
+    const int cnt = __popc(code), ways = kFillThreads / R, way = tid / R, mine_r = tid % R;        // (whole wavefronts share a way)
+    for (int r0 = 0; r0 < tile_rows; r0 += R) {
+        if (r0 > 0) {
+            __syncthreads();                     // the previous chunk's rows have been consumed
+            fetch_order(r0);
+        }
+        __syncthreads();
+        for (int i0 = 0; i0 < R * 32; i0 += 8 * kFillThreads) {      // eight loads in flight per thread
+            uint32_t word[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int i = i0 + q * kFillThreads + tid;
+                const int64_t src = i < R * 32 ? src_row[i >> 5] : -1;
+                word[q] = ((i & 31) < V && src >= 0) ? map[(size_t)src * V + (i & 31)] : FGX_EMPTY32;
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int i = i0 + q * kFillThreads + tid;
+                if (i < R * 32 && (i & 31) < V) stage[(i >> 5) * V + (i & 31)] = word[q];
+            }
+        }
+        __syncthreads();
+        const int r = r0 + mine_r;
+        for (int k = way; k < cnt; k += ways) {
+            const uint32_t m = stage[mine_r * V + offsets[k]];       // (a row past the end is EMPTY throughout)
+            if (r < tile_rows) plan_idx[(slot + k) * tile_rows + r] = m;
+            if (plan_band != nullptr) {
+                const unsigned long long live = __ballot(m != FGX_EMPTY32);    // all 64 lanes take part
+                if (lane == 0) {
+                    const int b0 = (r0 + (mine_r & ~63)) >> 5;                 // band of this wavefront's lanes 0-31
+                    uint32_t bits = ((live & 0xFFFFFFFFull) ? 1u : 0u) << (b0 & 31);
+                    bits |= ((live >> 32) ? 1u : 0u) << ((b0 + 1) & 31);
+                    if (bits) atomicOr(&bands[k], bits);
+                }
+            }
+        }
+    }
+    if (plan_band != nullptr) {
+        __syncthreads();
+        if (tid < cnt) plan_band[slot + tid] = bands[tid];
+    }
+}
+
+inline int fill_rows(int tile_rows) { return tile_rows <= 64 ? 64 : tile_rows <= 128 ? 128 : kFillRows; }
+inline size_t fill_lds(int tile_rows, int V) { return (size_t)fill_rows(tile_rows) * V * 4; }
 
 struct PairLayout {
     unsigned nblk;
@@ -955,6 +1011,16 @@ int fgx_tile_plan(const int32_t* gray, const int64_t* order, const uint32_t* map
         FGX_CHECK_LAUNCH("fgx_tile_plan(chunks)");
         scans = false;
     }
+    const size_t items = item_at != nullptr ? num_tiles * (size_t)col_tiles : 0;
+    if (plan_idx != nullptr && num_tiles <= kFillScanTiles && items < ((size_t)1 << kItemBits) && (item_at == nullptr || groups <= kFillThreads)) {
+        const size_t lds = fill_lds(tile_rows, V), list = items <= kOrderInLds ? items * 4 : 0;
+        phase_mark("gather plan fill", s);
+        plan_fill_kernel<true><<<(unsigned)num_tiles + (item_at != nullptr ? 1u : 0u), kFillThreads, lds > list ? lds : list, s>>>(
+            map, order, tile_code, num_tiles, n, V, tile_rows, fill_rows(tile_rows), seg, plan_seg, plan_idx, plan_band, (unsigned)col_tiles,
+            (unsigned)slabs, (unsigned)groups, item_ws, item_at);
+        FGX_CHECK_LAUNCH("fgx_tile_plan(tables and plan)");
+        return FGX_OK;
+    }
     if (scans || item_at != nullptr) {
         tile_tables_kernel<<<1, kOrderThreads, 0, s>>>(tile_code, (unsigned)num_tiles, scans ? seg : nullptr, scans ? plan_seg : nullptr,
                                                        (unsigned)col_tiles, (unsigned)slabs, (unsigned)groups, item_ws, item_at);
@@ -962,7 +1028,8 @@ int fgx_tile_plan(const int32_t* gray, const int64_t* order, const uint32_t* map
     }
     if (plan_idx != nullptr) {
         phase_mark("gather plan fill", s);
-        plan_fill_kernel<<<(unsigned)num_tiles, kBlock, 0, s>>>(map, order, tile_code, plan_seg, n, V, tile_rows, plan_idx, plan_band);
+        plan_fill_kernel<false><<<(unsigned)num_tiles, kFillThreads, fill_lds(tile_rows, V), s>>>(map, order, tile_code, num_tiles, n, V, tile_rows, fill_rows(tile_rows),
+                                                                              nullptr, plan_seg, plan_idx, plan_band, 1, 1, 1, nullptr, nullptr);
         FGX_CHECK_LAUNCH("fgx_tile_plan(plan)");
     }
     return FGX_OK;
@@ -997,8 +1064,9 @@ int fgx_gather_plan_fill(const uint32_t* map, const int64_t* order, const int32_
     FGX_CHECK_ARG(plan_band == nullptr || tile_rows <= 1024, "fgx_gather_plan_fill: band masks need tile_rows <= 1024");
     PhaseEnd phases{(hipStream_t)stream};
     phase_mark("gather plan fill", (hipStream_t)stream);
-    plan_fill_kernel<<<(unsigned)num_tiles, kBlock, 0, (hipStream_t)stream>>>(map, order, tile_code, plan_seg, n, V, tile_rows,
-                                                                              plan_idx, plan_band);
+    plan_fill_kernel<false><<<(unsigned)num_tiles, kFillThreads, fill_lds(tile_rows, V), (hipStream_t)stream>>>(
+        map, order, tile_code, num_tiles, n, V, tile_rows, fill_rows(tile_rows), nullptr, const_cast<int32_t*>(plan_seg), plan_idx, plan_band, 1, 1, 1,
+        nullptr, nullptr);
     FGX_CHECK_LAUNCH("fgx_gather_plan_fill");
     return FGX_OK;
 }
