@@ -753,10 +753,10 @@ def _narrow_wgrad(g: torch.Tensor, f: torch.Tensor, cache, v: int, with_bias: bo
     with torch.cuda.device(f.device):
         scratch = nat.workspace(L.fgx_narrow_wgrad_scratch_bytes(C.c_int(v)), f.device)
         nat.mark("wgrad", "start")
-        nat.check(L.fgx_conv_narrow_wgrad(C.c_int(nat.DTYPE_CODE[f.dtype]), nat.ptr(g), nat.ptr(f), nat.ptr(cache._narrow_plan()),
-                                          nat.sz(n), nat.sz(n_in), C.c_int(ci), C.c_int(co), C.c_int(v), nat.ptr(scratch),
-                                          nat.ptr(gw), nat.stream()))
-        gb = _colsum(g) if with_bias else None
+        gb = torch.empty((co,), dtype=f.dtype, device=f.device) if with_bias else None
+        nat.check(L.fgx_conv_narrow_wgrad_bias(C.c_int(nat.DTYPE_CODE[f.dtype]), nat.ptr(g), nat.ptr(f), nat.ptr(cache._narrow_plan()),
+                                               nat.sz(n), nat.sz(n_in), C.c_int(ci), C.c_int(co), C.c_int(v), nat.ptr(scratch),
+                                               nat.ptr(gw), nat.ptr(gb), nat.stream()))
         nat.mark("wgrad", "stop")
     return gw, gb
 

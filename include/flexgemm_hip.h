@@ -406,8 +406,11 @@ int fgx_conv_narrow_gemm(int dtype, const void* src, const void* panel, const vo
  * products in workgroup order (same bits on every run; against fgx_conv_wgrad the sums differ by fp32 rounding of a
  * different order; an infinity or NaN of grad_out counts for its own pairs, as there).  The plan must have been made with same_rows = 1 and must have NO overflowing chunk: the first
  * uint32 of the plan counts them -- read it back once per plan and call fgx_conv_wgrad instead when it is not 0.
- * scratch: fgx_narrow_wgrad_scratch_bytes(V) bytes, 16-byte aligned.  The bias gradient is not made here (fgx_colsum).
+ * scratch: fgx_narrow_wgrad_scratch_bytes(V) bytes, 16-byte aligned.  fgx_conv_narrow_wgrad_bias also writes the
+ * column sums of grad_out (grad_bias, NULL: none), which cost nothing there.
  * No counterpart in the reference (..._bwd_masked_implicit_gemm_splitk.py:108-182 gathers both operands per pair). */
+int fgx_conv_narrow_wgrad_bias(int dtype, const void* grad_out, const void* feats, const void* plan, size_t n, size_t n_src, int Ci,
+                               int Co, int V, void* scratch, void* grad_weight, void* grad_bias, fgx_stream_t stream);
 size_t fgx_narrow_wgrad_scratch_bytes(int V);
 int fgx_conv_narrow_wgrad(int dtype, const void* grad_out, const void* feats, const void* plan, size_t n, size_t n_src, int Ci,
                           int Co, int V, void* scratch, void* grad_weight, fgx_stream_t stream);
