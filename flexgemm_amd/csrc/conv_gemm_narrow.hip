@@ -35,12 +35,17 @@ constexpr int kNarrowHash = 1024;                // hash table of the plan build
 // ------------------------------------------------------------------------------------------------
 __global__ void __launch_bounds__(64) narrow_plan_header_kernel(uint32_t* __restrict__ header) { header[threadIdx.x] = 0u; }
 
-template <typename Order>
-__global__ void __launch_bounds__(256) narrow_plan_kernel(const uint32_t* __restrict__ nmap, const Order* __restrict__ order,
-                                                          uint32_t n, int V, int own_rows, unsigned char* __restrict__ plan) {
-    __shared__ uint32_t keys[kNarrowHash];
-    __shared__ uint16_t slot_of[kNarrowHash];
-    __shared__ uint32_t scan[256];
+// Bound by the latency of its LDS operations: with every insertion waiting for the one before it, a second walk through the table to
+// find an entry again, sixteen barriers for the scan and divisions by a variable V, the plan of 2.67 M voxels took 0.271 ms; now 0.175
+// (0.204 with the five wavefronts a SIMD that the compiler's own choice of registers leaves; reading the map and writing the plan take
+// 0.085).  VC: V where it is 27, else 0.
+template <typename Order, int VC>
+__global__ void __launch_bounds__(256, VC ? 8 : 4) narrow_plan_kernel(const uint32_t* __restrict__ nmap, const Order* __restrict__ order,
+                                                          uint32_t n, int v_any, int own_rows, unsigned char* __restrict__ plan) {
+    const int V = VC ? VC : v_any;
+    __shared__ uint32_t keys[kNarrowHash + 64];                                     // (a lane without an entry swaps a word of its own)
+    __shared__ __attribute__((aligned(4))) uint16_t slot_of[kNarrowHash];
+    __shared__ uint32_t scan[4];
     __shared__ uint32_t row_flags[kNarrowRows / 32];
     __shared__ uint32_t grow_of[kNarrowRows];                                       // the chunk's rows (FGX_EMPTY32 beyond n)
     __shared__ __attribute__((aligned(16))) uint16_t table_lds[kNarrowRows * kNarrowTableStride];   // leaves as 16-byte stores
@@ -49,14 +54,16 @@ __global__ void __launch_bounds__(256) narrow_plan_kernel(const uint32_t* __rest
     unsigned char* mine = plan + kNarrowHeader + (size_t)chunk * kNarrowPlanStride;
     uint32_t* sources = (uint32_t*)(mine + kNarrowTableBytes);
     uint32_t* rows = sources + kNarrowSlots;
-    for (int i = tid; i < kNarrowHash; i += 256) keys[i] = FGX_EMPTY32;
+    for (int i = tid; i < kNarrowHash + 64; i += 256) keys[i] = FGX_EMPTY32;
+    for (int i = tid; i < kNarrowHash / 2; i += 256) ((uint32_t*)slot_of)[i] = (uint32_t)kNarrowOverflow << 16 | (uint32_t)kNarrowOverflow;
     if (tid < kNarrowRows / 32) row_flags[tid] = 0u;
     for (int r = tid; r < kNarrowRows; r += 256) {
         const uint32_t gr = chunk * kNarrowRows + (uint32_t)r;
         grow_of[r] = gr < n ? (order ? (uint32_t)order[gr] : gr) : FGX_EMPTY32;
     }
     // entries from V on: the row of zeros (entry 31, the row's overflow flag, is written at the end)
-    for (int i = tid; i < kNarrowRows * kNarrowTableStride; i += 256) table_lds[i] = (uint16_t)(kNarrowZeroSlot * 64u);
+    for (int i = tid; i < kNarrowRows * (kNarrowTableStride - V); i += 256)
+        table_lds[i / (kNarrowTableStride - V) * kNarrowTableStride + V + i % (kNarrowTableStride - V)] = (uint16_t)(kNarrowZeroSlot * 64u);
     __syncthreads();
     const int entries = kNarrowRows * V;
     auto source_of = [&](int e) -> uint32_t {
@@ -65,8 +72,7 @@ __global__ void __launch_bounds__(256) narrow_plan_kernel(const uint32_t* __rest
         return nmap[(size_t)grow * V + (e % V)];
     };
     auto hash = [](uint32_t x) -> uint32_t { return (x * 2654435761u) >> 22; };      // 10 bits
-    auto insert = [&](uint32_t idx) -> int {                                         // table position, -1 when the table is full
-        uint32_t h = hash(idx);
+    auto insert = [&](uint32_t idx, uint32_t h) -> int {                             // table position, -1 when the table is full
         for (int probe = 0; probe < kNarrowHash; ++probe) {
             const uint32_t old = atomicCAS(&keys[h], FGX_EMPTY32, idx);
             if (old == FGX_EMPTY32 || old == idx) return (int)h;
@@ -78,12 +84,10 @@ __global__ void __launch_bounds__(256) narrow_plan_kernel(const uint32_t* __rest
     // the slot of its chunk row number: the 16 rows of a fragment read then fall on 16 different slots modulo 16 for
     // the centre offset and on nearly as many for the others -- the neighbors of consecutive rows are mostly
     // consecutive rows -- which is what keeps the reads of arbitrary slots off each other's banks.
-    for (int i = tid; i < kNarrowHash; i += 256) slot_of[i] = (uint16_t)kNarrowOverflow;
-    __syncthreads();
     if (own_rows) {
         for (int r = tid; r < kNarrowRows; r += 256) {
             if (grow_of[r] != FGX_EMPTY32) {
-                const int pos = insert(grow_of[r]);
+                const int pos = insert(grow_of[r], hash(grow_of[r]));
                 if (pos >= 0) slot_of[pos] = (uint16_t)r;
             }
         }
@@ -91,16 +95,24 @@ __global__ void __launch_bounds__(256) narrow_plan_kernel(const uint32_t* __rest
     }
     // (a thread's entries stay in registers for the second pass: kNarrowRows * kNarrowMaxV / 256 of them at most; all
     // of them are fetched before the first goes into the table, so that their latencies overlap)
-    constexpr int kPerThread = (kNarrowRows * 32 + 255) / 256;
+    constexpr int kPerThread = (kNarrowRows * (VC ? VC : 32) + 255) / 256;
     uint32_t mine_idx[kPerThread];
 #pragma unroll
     for (int j = 0; j < kPerThread; ++j) {
         const int e = tid + j * 256;
         mine_idx[j] = e < entries ? source_of(e) : FGX_EMPTY32;
     }
+    // first probes of all entries in flight together; the few that met another key go on from there
+    int pos[kPerThread];
+    uint32_t met[kPerThread];
+#pragma unroll
+    for (int j = 0; j < kPerThread; ++j) {
+        pos[j] = mine_idx[j] != FGX_EMPTY32 ? (int)hash(mine_idx[j]) : kNarrowHash + (tid & 63);
+        met[j] = atomicCAS(&keys[pos[j]], FGX_EMPTY32, mine_idx[j]);
+    }
 #pragma unroll
     for (int j = 0; j < kPerThread; ++j)
-        if (mine_idx[j] != FGX_EMPTY32) insert(mine_idx[j]);
+        if (met[j] != FGX_EMPTY32 && met[j] != mine_idx[j]) pos[j] = insert(mine_idx[j], (uint32_t)(pos[j] + 1) & (kNarrowHash - 1));
     __syncthreads();
     // the other sources: slots from `base` on in table order (exclusive scan of their positions, four per thread)
     const uint32_t base = own_rows ? (uint32_t)kNarrowRows : 0u;
@@ -109,15 +121,20 @@ __global__ void __launch_bounds__(256) narrow_plan_kernel(const uint32_t* __rest
     }
     uint32_t own = 0;
     for (int j = 0; j < 4; ++j) own += (keys[tid * 4 + j] != FGX_EMPTY32 && slot_of[tid * 4 + j] == kNarrowOverflow) ? 1u : 0u;
-    scan[tid] = own;
-    __syncthreads();
-    for (int d = 1; d < 256; d <<= 1) {
-        const uint32_t add = tid >= d ? scan[tid - d] : 0u;
-        __syncthreads();
-        scan[tid] += add;
-        __syncthreads();
+    uint32_t upto = own;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_up((int)upto, d, 64);
+        upto += (tid & 63) >= d ? o : 0u;
     }
-    uint32_t next = base + scan[tid] - own;
+    if ((tid & 63) == 63) scan[tid >> 6] = upto;
+    __syncthreads();
+    uint32_t next = base + upto - own, total = base;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        next += w < (tid >> 6) ? scan[w] : 0u;
+        total += scan[w];
+    }
     for (int j = 0; j < 4; ++j) {
         const int pos = tid * 4 + j;
         if (keys[pos] != FGX_EMPTY32 && slot_of[pos] == kNarrowOverflow) {
@@ -128,25 +145,14 @@ __global__ void __launch_bounds__(256) narrow_plan_kernel(const uint32_t* __rest
             ++next;
         }
     }
-    const uint32_t total = base + scan[255];
     for (uint32_t s = total + tid; s < (uint32_t)kNarrowSlots; s += 256) sources[s] = FGX_EMPTY32;
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < kPerThread; ++j) {
         const int e = tid + j * 256;
         if (e >= entries) break;
-        const uint32_t idx = mine_idx[j];
         uint16_t out = (uint16_t)kNarrowZeroSlot;
-        if (idx != FGX_EMPTY32) {
-            out = (uint16_t)kNarrowOverflow;
-            uint32_t h = hash(idx);
-            for (int probe = 0; probe < kNarrowHash; ++probe) {
-                const uint32_t k = keys[h];
-                if (k == idx) { out = slot_of[h]; break; }
-                if (k == FGX_EMPTY32) break;
-                h = (h + 1) & (kNarrowHash - 1);
-            }
-        }
+        if (pos[j] < kNarrowHash) out = pos[j] >= 0 ? slot_of[pos[j]] : (uint16_t)kNarrowOverflow;
         // what the multipliers read: the byte offset of the row's logical piece 0 in the row buffer
         if (out != (uint16_t)kNarrowOverflow) out = (uint16_t)(out * 64u + (((uint32_t)out >> 2) & 3u) * 16u);
         table_lds[(e / V) * kNarrowTableStride + (e % V)] = out;
@@ -446,7 +452,8 @@ int make_narrow_plan(const uint32_t* map, const Order* order, size_t n, int V, i
     const unsigned chunks = (unsigned)((n + kNarrowRows - 1) / kNarrowRows);
     narrow_plan_header_kernel<<<1, 64, 0, s>>>((uint32_t*)plan);
     FGX_CHECK_LAUNCH("fgx_narrow_plan(header)");
-    narrow_plan_kernel<<<chunks, 256, 0, s>>>(map, order, (uint32_t)n, V, same_rows ? 1 : 0, (unsigned char*)plan);
+    auto kern = V == 27 ? narrow_plan_kernel<Order, 27> : narrow_plan_kernel<Order, 0>;
+    kern<<<chunks, 256, 0, s>>>(map, order, (uint32_t)n, V, same_rows ? 1 : 0, (unsigned char*)plan);
     FGX_CHECK_LAUNCH("fgx_narrow_plan");
     return FGX_OK;
 }
