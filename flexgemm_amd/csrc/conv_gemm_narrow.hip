@@ -33,7 +33,9 @@ constexpr int kNarrowHash = 1024;                // hash table of the plan build
 // Plan builder: one workgroup per chunk.  The distinct neighbors of the chunk's rows go through a hash table in LDS;
 // slots are numbered in table order, so the plan depends on the chunk's set of sources alone.
 // ------------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) narrow_plan_header_kernel(uint32_t* __restrict__ header) { header[threadIdx.x] = 0u; }
+__global__ void __launch_bounds__(64) narrow_plan_header_kernel(uint32_t* __restrict__ header, int V) {
+    header[threadIdx.x] = threadIdx.x == 1 && V == kNarrowEvenV ? kNarrowRepeats : 0u;
+}
 
 // Bound by the latency of its LDS operations: with every insertion waiting for the one before it, a second walk through the table to
 // find an entry again, sixteen barriers for the scan and divisions by a variable V, the plan of 2.67 M voxels took 0.271 ms; now 0.175
@@ -62,8 +64,9 @@ __global__ void __launch_bounds__(256, VC ? 8 : 4) narrow_plan_kernel(const uint
         grow_of[r] = gr < n ? (order ? (uint32_t)order[gr] : gr) : FGX_EMPTY32;
     }
     // entries from V on: the row of zeros (entry 31, the row's overflow flag, is written at the end)
-    for (int i = tid; i < kNarrowRows * (kNarrowTableStride - V); i += 256)
-        table_lds[i / (kNarrowTableStride - V) * kNarrowTableStride + V + i % (kNarrowTableStride - V)] = (uint16_t)(kNarrowZeroSlot * 64u);
+    const int used = VC == kNarrowEvenV ? V + 3 : V;
+    for (int i = tid; i < kNarrowRows * (kNarrowTableStride - used); i += 256)
+        table_lds[i / (kNarrowTableStride - used) * kNarrowTableStride + used + i % (kNarrowTableStride - used)] = (uint16_t)(kNarrowZeroSlot * 64u);
     __syncthreads();
     const int entries = kNarrowRows * V;
     auto source_of = [&](int e) -> uint32_t {
@@ -156,6 +159,8 @@ __global__ void __launch_bounds__(256, VC ? 8 : 4) narrow_plan_kernel(const uint
         // what the multipliers read: the byte offset of the row's logical piece 0 in the row buffer
         if (out != (uint16_t)kNarrowOverflow) out = (uint16_t)(out * 64u + (((uint32_t)out >> 2) & 3u) * 16u);
         table_lds[(e / V) * kNarrowTableStride + (e % V)] = out;
+        // (the weight gradient's last multiplier takes offsets 7, 15 and 23 behind 24, 25 and 26: seven offsets each)
+        if (VC == kNarrowEvenV && e % V % 8 == 7) table_lds[(e / V) * kNarrowTableStride + kNarrowEvenV + e % V / 8] = out;
         if (out == (uint16_t)kNarrowOverflow) atomicOr(&row_flags[(e / V) >> 5], 1u << ((e / V) & 31));
     }
     __syncthreads();
@@ -450,9 +455,9 @@ int make_narrow_plan(const uint32_t* map, const Order* order, size_t n, int V, i
     FGX_CHECK_ARG(((uintptr_t)plan & 15) == 0, "fgx_narrow_plan: plan must be 16-byte aligned");
     FGX_CHECK_ARG(fgx_narrow_plan_bytes(n, V) < 0xFF000000ull, "fgx_narrow_plan: plan of %zu rows passes the 32-bit offset range", n);
     const unsigned chunks = (unsigned)((n + kNarrowRows - 1) / kNarrowRows);
-    narrow_plan_header_kernel<<<1, 64, 0, s>>>((uint32_t*)plan);
+    narrow_plan_header_kernel<<<1, 64, 0, s>>>((uint32_t*)plan, V);
     FGX_CHECK_LAUNCH("fgx_narrow_plan(header)");
-    auto kern = V == 27 ? narrow_plan_kernel<Order, 27> : narrow_plan_kernel<Order, 0>;
+    auto kern = V == kNarrowEvenV ? narrow_plan_kernel<Order, kNarrowEvenV> : narrow_plan_kernel<Order, 0>;
     kern<<<chunks, 256, 0, s>>>(map, order, (uint32_t)n, V, same_rows ? 1 : 0, (unsigned char*)plan);
     FGX_CHECK_LAUNCH("fgx_narrow_plan");
     return FGX_OK;

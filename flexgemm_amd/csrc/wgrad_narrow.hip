@@ -12,7 +12,8 @@
 //
 // Workgroup: 4 multiplying wavefronts + 4 loading wavefronts, two LDS buffers, one barrier per chunk (as in the forward
 // kernel).  Multiplier w owns the offsets 8 w ... 8 w + 7 (their 32 x 32 accumulators stay in registers over all the
-// chunks of the workgroup; offsets from V on multiply zeros) and walks the chunk's 128 rows in eight k-steps of 16; the
+// chunks of the workgroup; offsets from V on multiply zeros); of 27 offsets, whose LDS reads bound the kernel, the first three
+// leave their last one to the fourth, seven each with the column sums below (2.67 M voxels, 32 channels: 0.225 -> 0.196 ms).  It walks the chunk's 128 rows in eight k-steps of 16; the
 // grad_out fragment of a k-step is read once for the eight offsets.  At the end every workgroup writes its partial
 // products, and a second kernel adds them in workgroup order (fixed order: same bits on every run).
 // An infinity or NaN in grad_out times the row of zeros is NaN where the sum over the pairs has no term: a workgroup whose sums are not
@@ -31,7 +32,7 @@ namespace fgx {
 namespace {
 
 constexpr int kNwMult = 4, kNwLoad = 4, kNwThreads = 64 * (kNwMult + kNwLoad);
-constexpr int kNwTaps = 8;                                                       // offsets per multiplier
+constexpr int kNwTaps = 8;                                                       // offsets per multiplier (7 of 27: below)
 constexpr int kNwGoutBytes = kNarrowRows * 64;                                   // the chunk's grad_out rows
 constexpr int kNwBufferBytes = kNarrowRowBufPad + kNwGoutBytes + kNarrowTableBytes;
 constexpr size_t kNwLdsBytes = 2 * (size_t)kNwBufferBytes + 16;                  // ... and the word that asks for a second pass
@@ -39,7 +40,7 @@ constexpr int kNwSrcGroups = kNarrowSlots / 16 / kNwLoad;                       
 constexpr int kNwOutGroups = kNarrowRows / 16 / kNwLoad;                         // 2
 constexpr int kNwIds = kNwSrcGroups + kNwOutGroups;
 
-template <typename Tag>
+template <typename Tag, int TAPS>
 __global__ void __launch_bounds__(kNwThreads)
 narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Tag::type* __restrict__ feats,
                     const unsigned char* __restrict__ plan, uint32_t chunks, uint32_t plan_bytes, uint32_t gout_bytes,
@@ -150,14 +151,26 @@ narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename 
         }
         return;
     }
-    f32x16 acc[kNwTaps];
-    // the last offset of the last multiplier, past every V: ones in place of whatever its table entry (a row's overflow flag) names
+    f32x16 acc[TAPS];
+    const bool patch = TAPS != kNwTaps && mw == kNwMult - 1 && ((const uint32_t*)plan)[1] != kNarrowRepeats;
+    // a row's entries for the wavefront's offsets, 16 bytes (`kept`: the plan may lack the repeated ones)
+    auto entries_of = [&](const unsigned char* table, int r, auto kept) __attribute__((always_inline)) -> u32x4 {
+        const uint16_t* row = (const uint16_t*)(table + r * (kNarrowTableStride * 2));
+        u32x4 e = *reinterpret_cast<const u32x4*>(row + mw * 8);
+        if (decltype(kept)::value && patch) {
+            e[1] = (e[1] & 0xFFFFu) | (uint32_t)row[7] << 16;
+            e[2] = (uint32_t)row[15] | (uint32_t)row[23] << 16;
+        }
+        return e;
+    };
+    auto offset_of = [&](int t) -> int { return TAPS == kNwTaps || mw < kNwMult - 1 || t < 3 ? mw * kNwTaps + t : (t < TAPS - 1 ? (t - 3) * kNwTaps + 7 : kNarrowMaxV); };
+    // the last offset of the last multiplier, past every V: ones in place of whatever its table entry names
     static_assert(kNarrowMaxV < kNwMult * kNwTaps, "an offset is free for the column sums");
     const uint32_t bias_bits = bias_partial != nullptr && mw == kNwMult - 1 ? (std::is_same<Tag, F16>::value ? 0x3C003C00u : 0x3F803F80u) : 0u;
-    auto run = [&](auto apart_rows) __attribute__((always_inline)) {
+    auto run = [&](auto apart_rows, auto kept) __attribute__((always_inline)) {
         constexpr bool APART = decltype(apart_rows)::value;
 #pragma unroll
-        for (int t = 0; t < kNwTaps; ++t)
+        for (int t = 0; t < TAPS; ++t)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
         if (first < range_hi) {
@@ -178,11 +191,9 @@ narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename 
                 const uint32_t row_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)buf + cw;
 #pragma unroll 1
                 for (int kk = 0; kk < kNarrowRows / 16 && !done; ++kk) {
-                    // the table entries of this lane's two rows for the wavefront's eight offsets: 16 bytes each
                     const int r0 = kk * 16 + g * 8 + q;
-                    const u32x4 e_lo = *reinterpret_cast<const u32x4*>(table + r0 * (kNarrowTableStride * 2) + mw * 16);
-                    const u32x4 e_hi = *reinterpret_cast<const u32x4*>(table + (r0 + 4) * (kNarrowTableStride * 2) + mw * 16);
-                    i16x4 gfr[2], ffr[16];                                       // grad_out (lo, hi); eight offsets (lo, hi)
+                    const u32x4 e_lo = entries_of(table, r0, kept), e_hi = entries_of(table, r0 + 4, kept);
+                    i16x4 gfr[2], ffr[2 * TAPS];                                 // grad_out (lo, hi); the offsets (lo, hi)
                     gfr[0] = lds_read_tr16_at<0>(g_lo + (uint32_t)(kk * 16 * 64));
                     gfr[1] = lds_read_tr16_at<0>(g_hi + (uint32_t)(kk * 16 * 64));
                     auto entry = [](const u32x4& e, int t) -> uint32_t { return (t & 1) ? e[t >> 1] >> 16 : e[t >> 1] & 0xFFFFu; };
@@ -198,14 +209,15 @@ narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename 
                     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[4]), "+v"(ffr[5]), "+v"(ffr[6]), "+v"(ffr[7]));
                     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[8]), "+v"(ffr[9]), "+v"(ffr[10]), "+v"(ffr[11]));
 #pragma unroll
-                    for (int t = 6; t < 8; ++t) {
+                    for (int t = 6; t < TAPS; ++t) {
                         ffr[t * 2] = lds_read_tr16_at<0>(at(e_lo, t));
                         ffr[t * 2 + 1] = lds_read_tr16_at<0>(at(e_hi, t));
                     }
                     i16x8 gf = __builtin_shufflevector(gfr[0], gfr[1], 0, 1, 2, 3, 4, 5, 6, 7);
                     uint32_t apart = 0u;
                     if constexpr (APART) {
-                        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[12]), "+v"(ffr[13]), "+v"(ffr[14]), "+v"(ffr[15]));
+#pragma unroll
+                        for (int t = 12; t < 2 * TAPS; ++t) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[t]));
                         apart = nonfinite_rows<Tag>(gf);
                         if (apart) drop_rows(gf, apart, g);
                     }
@@ -215,11 +227,12 @@ narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename 
                         if (APART && apart) drop_rows(ff, apart, g);
                         mma16<Tag>(acc[t], gf, ff);
                     }
-                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[12]), "+v"(ffr[13]), "+v"(ffr[14]), "+v"(ffr[15]));
 #pragma unroll
-                    for (int t = 6; t < 8; ++t) {
+                    for (int t = 12; t < 2 * TAPS; ++t) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(ffr[t]));
+#pragma unroll
+                    for (int t = 6; t < TAPS; ++t) {
                         i16x8 ff = __builtin_shufflevector(ffr[t * 2], ffr[t * 2 + 1], 0, 1, 2, 3, 4, 5, 6, 7);
-                        if (!APART && t == kNwTaps - 1 && bias_bits != 0u) ff = __builtin_bit_cast(i16x8, u32x4{bias_bits, bias_bits, bias_bits, bias_bits});
+                        if (!APART && t == TAPS - 1 && bias_bits != 0u) ff = __builtin_bit_cast(i16x8, u32x4{bias_bits, bias_bits, bias_bits, bias_bits});
                         if (APART && apart) drop_rows(ff, apart, g);
                         mma16<Tag>(acc[t], gf, ff);
                     }
@@ -230,13 +243,13 @@ narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename 
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
                             gv[e] = *reinterpret_cast<const T4*>(gbuf + r * 64 + (((uint32_t)e ^ narrow_piece_key((uint32_t)r)) << 4) + g * 8);
-                        const u32x4 entries = *reinterpret_cast<const u32x4*>(table + r * (kNarrowTableStride * 2) + mw * 16);
-                        T x[kNwTaps];                                            // (all reads in flight together; a missing neighbor's: zeros)
+                        const u32x4 entries = entries_of(table, r, kept);
+                        T x[TAPS];                                            // (all reads in flight together; a missing neighbor's: zeros)
 #pragma unroll
-                        for (int t = 0; t < kNwTaps; ++t)
+                        for (int t = 0; t < TAPS; ++t)
                             x[t] = *reinterpret_cast<const T*>(buf + (entry(entries, t) ^ ((uint32_t)((lane & 31) >> 3) << 4)) + (lane & 7) * 2);
 #pragma unroll
-                        for (int t = 0; t < kNwTaps; ++t) {
+                        for (int t = 0; t < TAPS; ++t) {
                             if (__builtin_amdgcn_readfirstlane((int)entry(entries, t)) >> 6 == (int)kNarrowZeroSlot) continue;
 #pragma unroll
                             for (int e = 0; e < 16; ++e) acc[t][e] += (float)gv[e >> 2][e & 3] * (float)x[t];
@@ -246,7 +259,7 @@ narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename 
                 if constexpr (APART) {
                     bool nan = true;
 #pragma unroll
-                    for (int t = 0; t < kNwTaps; ++t) nan = nan && (mw * kNwTaps + t >= V || all_nan(acc[t], lane, 0, Co, 0, Ci));
+                    for (int t = 0; t < TAPS; ++t) nan = nan && (offset_of(t) >= V || all_nan(acc[t], lane, 0, Co, 0, Ci));
                     done = __all(nan);
                 }
                 __builtin_amdgcn_s_waitcnt(0);
@@ -254,24 +267,25 @@ narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename 
             }
         }
     };
-    run(std::false_type{});
+    if (patch) run(std::false_type{}, std::true_type{});
+    else run(std::false_type{}, std::false_type{});
     // (whatever the second pass does: a column's sum has a term for every row)
     if (bias_bits != 0u && (lane & 31) == 0)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) bias_partial[blockIdx.x * 32 + (e >> 2) * 8 + g * 4 + (e & 3)] = acc[kNwTaps - 1][e];
+        for (int e = 0; e < 16; ++e) bias_partial[blockIdx.x * 32 + (e >> 2) * 8 + g * 4 + (e & 3)] = acc[TAPS - 1][e];
     bool finite = true;
 #pragma unroll
-    for (int t = 0; t < kNwTaps; ++t) finite = finite && (mw * kNwTaps + t >= V || all_finite(acc[t]));
+    for (int t = 0; t < TAPS; ++t) finite = finite && (offset_of(t) >= V || all_finite(acc[t]));
     if (__any(!finite) && lane == 0) again = 1u;
     __syncthreads();                                                             // (the loaders' after their first pass)
-    if (again != 0u) run(std::true_type{});
+    if (again != 0u) run(std::true_type{}, std::true_type{});
     // partial[workgroup][v][co][ci] (32 x 32 per offset): accumulator element e of lane (l32, g) is co = (e >> 2) * 8 +
     // g * 4 + (e & 3), ci = l32
     {
         const int l32 = lane & 31;
 #pragma unroll
-        for (int t = 0; t < kNwTaps; ++t) {
-            const int v = mw * kNwTaps + t;
+        for (int t = 0; t < TAPS; ++t) {
+            const int v = offset_of(t);
             if (v < V) {
                 float* dst = partial + ((size_t)blockIdx.x * V + v) * 1024;
 #pragma unroll
@@ -347,12 +361,12 @@ int launch_narrow_wgrad(const void* gout, const void* feats, const void* plan, s
     int rc = narrow_wgrad_groups(&groups);
     if (rc != FGX_OK) return rc;
     const uint32_t chunks = (uint32_t)((n + kNarrowRows - 1) / kNarrowRows);
-    auto kern = narrow_wgrad_kernel<Tag>;
+    auto kern = V == kNarrowEvenV ? narrow_wgrad_kernel<Tag, 7> : narrow_wgrad_kernel<Tag, kNwTaps>;
     float* bias_partial = gb ? (float*)scratch + (size_t)groups * V * 1024 : nullptr;
-    static thread_local bool raised = false;
-    if (!raised) {
+    static thread_local bool raised[2] = {false, false};
+    if (!raised[V == kNarrowEvenV]) {
         FGX_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kNwLdsBytes));
-        raised = true;
+        raised[V == kNarrowEvenV] = true;
     }
     kern<<<groups, kNwThreads, kNwLdsBytes, s>>>((const T*)gout, (const T*)feats, (const unsigned char*)plan, chunks,
                                                  (uint32_t)(kNarrowHeader + (size_t)chunks * kNarrowPlanStride),

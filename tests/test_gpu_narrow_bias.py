@@ -24,9 +24,17 @@ def test_bias_beside_narrow_weight_gradient(dtype, n, ci, co, special):
         impl.spconv.NARROW_RESIDENT = "on"
         weight, bias = impl._wgrad(grad, feats, cache, 27, True, 13)
         alone = impl._wgrad(grad, feats, cache, 27)
+        # a plan of before the last multiplier's entries were repeated in it
+        header = cache["_narrow_plan_buf"][:256].view(torch.int32)
+        assert int(header[1]) != 0
+        header[1] = 0
+        table = cache["_narrow_plan_buf"][256:256 + 128 * 64].view(torch.int16).view(128, 32)
+        table[:, 27:30] = 448 * 64
+        kept, bias_kept = impl._wgrad(grad, feats, cache, 27, True, 13) if n <= 128 else (weight, bias)
     finally:
         impl.spconv.NARROW_RESIDENT = old
-    assert hasattr(cache, "_narrow_plan_buf") and torch.equal(weight.view(torch.int16), alone.view(torch.int16))
+    bits = lambda t: t.view(torch.int16)
+    assert torch.equal(bits(weight), bits(alone)) and torch.equal(bits(weight), bits(kept)) and torch.equal(bits(bias), bits(bias_kept))
     want, size = grad.double().sum(0), grad.double().abs().sum(0)
     fine = torch.isfinite(want)
     assert torch.equal(torch.isfinite(bias), fine) and torch.equal(torch.isnan(bias), torch.isnan(want))
