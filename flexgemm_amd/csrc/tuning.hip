@@ -364,6 +364,18 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
 
 using namespace fgx;
 
+
+// Weight gradient of few voxels, 16-bit types: the streaming kernel in one voxel block, which stores straight into the gradient, is
+// ahead of the table's tiled kernel from the smallest layers on -- in 64 x 64 tiles, also where 32 x 32 ones would do (their four
+// partial products want a reduction), in 128 x 128 ones under a weight of 512 x 512 channels and more.  Measured (us, table -> this):
+// C = 16: 14 voxels 10.4 -> 5.6, 301 14.3 -> 7.0 (32 x 32 tiles: 9.6 and 10.2);  C = 64: 33 voxels 11.0 -> 5.6, 464 14.6 -> 8.3;
+// C = 128: 14 voxels 15.2 -> 5.9, 464 22.0 -> 8.8;  C = 256: 91 voxels 17.1 -> 8.1, 464 22.9 -> 11.5;  C = 512: 33 voxels 18.7 -> 12.4
+// (64 x 64: 14.1).  From 512 voxels on the table streams by itself.
+extern "C" int fgx_wgrad_short_tile(int dtype, size_t n, int Ci, int Co) {
+    if ((dtype != FGX_F16 && dtype != FGX_BF16) || n == 0 || n >= 512) return 0;
+    return (size_t)Ci * Co >= (size_t)512 * 512 ? 128 : 64;
+}
+
 extern "C" int fgx_table_lookup(int pass_kind, int dtype, size_t n, int Ci, int Co, int V, fgx_schedule* out) {
     FGX_CHECK_ARG(out != nullptr, "fgx_table_lookup: null output");
     FGX_CHECK_ARG(pass_kind >= 0 && pass_kind <= 2, "fgx_table_lookup: pass_kind must be 0 (fwd), 1 (dgrad) or 2 (wgrad)");

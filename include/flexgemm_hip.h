@@ -240,6 +240,9 @@ typedef struct fgx_schedule {
                          * fgx_conv_wgrad_sweep with tile = tile_rows and sub_rows = block_rows */
 } fgx_schedule;
 int fgx_table_lookup(int pass_kind, int dtype, size_t n, int Ci, int Co, int V, fgx_schedule* out);
+/* Weight gradient of few voxels: the tile (64 or 128, square) in which the streaming kernel over one voxel block is ahead of the
+ * table's choice, 0 where it is not. */
+int fgx_wgrad_short_tile(int dtype, size_t n, int Ci, int Co);
 
 /* Re-layout the [Co, V, Ci] weight into K-slab-major panels consumed by fgx_conv_gather_gemm.
  *   mode 0 (forward): panel[v][slab][co][k]  = w[co][v][slab*SK + k]          (K = Ci, cols = Co)
