@@ -44,7 +44,7 @@ namespace {
     X(fgx_conv_gather_gemm_stream_act_mask) X(fgx_conv_gather_gemm_stream_groups) X(fgx_relu_mask_apply) X(fgx_copy_columns)       \
     X(fgx_colsum_scratch_bytes) X(fgx_colsum) X(fgx_wgrad_block_bounds_count) X(fgx_wgrad_block_bounds)                            \
     X(fgx_conv_gemm_stem_pays) X(fgx_conv_gemm_stem) X(fgx_wgrad_stem_pays) X(fgx_wgrad_stem_scratch_bytes) X(fgx_conv_wgrad_stem) X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
-    X(fgx_wgrad_short_tile) X(fgx_conv_wgrad_split_scratch_bytes) X(fgx_conv_wgrad_split)                                                                  \
+    X(fgx_wgrad_short_tile) X(fgx_wgrad_split_tile) X(fgx_conv_wgrad_split_scratch_bytes) X(fgx_conv_wgrad_split)                                                                  \
     X(fgx_wgrad_sweep_plan_bytes) X(fgx_wgrad_sweep_plan) X(fgx_wgrad_sweep_scratch_bytes) X(fgx_conv_wgrad_sweep)                 \
     X(fgx_serialize_encode) X(fgx_serialize_decode) X(fgx_table_lookup)
 
@@ -896,10 +896,15 @@ WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool 
         if (pairs > std::min(sig_i.numel(), sig_o.numel()))
             throw py::value_error("valid_signal_seg does not fit the pair lists (V + 1 entries, the last one their length)");
         Sched s = schedule(2, feats, n, ci, co, v);
-        if (const int tile = s.stream == 0 && schedules_are_ours() ? L.fgx_wgrad_short_tile(code, (size_t)n, ci, co) : 0) {
-            s.stream = 1;
-            s.tile_rows = s.tile_cols = tile;
-            s.block_rows = 1024;
+        if (s.stream == 0 && schedules_are_ours()) {        // where a kernel is ahead that the table does not name
+            int rows = 1024;
+            if (const int tile = code == FGX_F32 ? L.fgx_wgrad_split_tile((size_t)n, ci, co, &rows) : L.fgx_wgrad_short_tile(code, (size_t)n, ci, co)) {
+                if (code != FGX_F32 || L.fgx_conv_wgrad_split_scratch_bytes((size_t)n, (size_t)n_in, (uint32_t)pairs, v, ci, co, tile, rows) > 0) {
+                    s.stream = 1;
+                    s.tile_rows = s.tile_cols = tile;
+                    s.block_rows = rows;
+                }
+            }
         }
         if (s.stream == 2 && !sweep_fits(n, n_in, ci, co, es, pairs)) {      // very long operands (and empty pair lists) take the block-major kernel
             s.stream = 1;

@@ -56,28 +56,6 @@ size_t round_up(size_t x, size_t m) { return (x + m - 1) / m * m; }
 bool rule_wgrad_f32(size_t n, int Ci, int Co, int V, fgx_schedule* out) {
     if ((size_t)Ci * Co >= (size_t)1024 * 1024) return false;
     auto padded = [&](int t) { return (double)cdiv(Ci, t) * t * cdiv(Co, t) * t; };
-    // The even split over persistent workgroups (fgx_conv_wgrad_split), in 96 x 96 tiles where they pad no more than 64 x 64 ones.  Its
-    // large tile multiplies at about twice the rate of the 32 x 32 one, which stays where it pads to half and less (32 channels,
-    // 41 700 voxels 0.052 ms, split 0.068).  Two voxel blocks under few tiles, one otherwise: a block adds segments, and rows are
-    // read from L2 fast enough either way (96 channels, 41 700 voxels: 1 block 0.102, 2 0.100, 8 0.106).
-    // Measured (ms, before -> now): 96 x 96: 96 channels, 2 581 voxels 0.039 -> 0.034, 10 494 0.083 -> 0.047, 41 700 0.196 -> 0.100, 667 763
-    // 2.33 -> 1.22;  96 -> 192 channels, 41 700 voxels 0.345 -> 0.173;  192 channels, 10 494 voxels 0.137 -> 0.101, 41 700 0.395 -> 0.311;
-    // 768 channels, 2 581 voxels 0.45 -> 0.37.   64 x 64: 64 channels, 5 876 voxels 0.033 -> 0.030, 41 700 0.099 -> 0.066 (2 581: 0.026
-    // and 0.027);  128 channels, 2 581 voxels 0.039 -> 0.035, 41 700 0.200 -> 0.183.
-    // Past these ranges the tiled kernel is level or ahead: 64 x 64 tiles, one from 667 763 voxels (0.71 both), a few of 166 977
-    // (128 channels: 0.62, split 0.67), sixteen of 41 700 (256 channels: 0.63, split 0.66; 10 494: 0.20 -> 0.19), more of any number
-    // (512 channels, 2 581 voxels 0.208 and 0.214);  four and more 96 x 96 tiles past 262 144 voxels: not measured.
-    {
-        const int t = padded(96) <= padded(64) ? 96 : 64;
-        const size_t tiles = (size_t)cdiv(Ci, t) * cdiv(Co, t);
-        const size_t least = t == 64 && tiles == 1 ? 4096 : 2048;
-        const size_t most = t == 96 ? (tiles >= 4 ? 262144 : ~(size_t)0) : tiles == 1 ? 262144 : tiles < 16 ? 65536 : tiles == 16 ? 12288 : 0;
-        if (padded(32) > 0.55 * padded(t) && n >= least && n <= most) {
-            const size_t rows = round_up(cdiv(n, (size_t)(tiles < 4 ? 2 : 1)), 64);
-            *out = fgx_schedule{t, t, 64, 1, (int)std::min(rows, (size_t)1 << 30), 1};
-            return true;
-        }
-    }
     const int t = padded(32) < 0.72 * padded(64) ? 32 : 64;
     const double tiles = (double)cdiv(Ci, t) * cdiv(Co, t);
     const double ideal = (double)n * V * tiles / (t == 64 ? 2000.0 : 4000.0);
@@ -374,6 +352,29 @@ using namespace fgx;
 extern "C" int fgx_wgrad_short_tile(int dtype, size_t n, int Ci, int Co) {
     if ((dtype != FGX_F16 && dtype != FGX_BF16) || n == 0 || n >= 512) return 0;
     return (size_t)Ci * Co >= (size_t)512 * 512 ? 128 : 64;
+}
+
+// fp32 weight gradient over the even split (fgx_conv_wgrad_split), in 96 x 96 tiles where they pad no more than 64 x 64 ones.  Its
+// large tile multiplies at about twice the rate of the 32 x 32 one, which stays where it pads to half and less (32 channels,
+// 41 700 voxels 0.052 ms, split 0.068).  Two voxel blocks under few tiles, one otherwise: a block adds segments, and rows are
+// read from L2 fast enough either way (96 channels, 41 700 voxels: 1 block 0.102, 2 0.100, 8 0.106).
+// Measured (ms, before -> now): 96 x 96: 96 channels, 2 581 voxels 0.039 -> 0.034, 10 494 0.083 -> 0.047, 41 700 0.196 -> 0.100, 667 763
+// 2.33 -> 1.22;  96 -> 192 channels, 41 700 voxels 0.345 -> 0.173;  192 channels, 10 494 voxels 0.137 -> 0.101, 41 700 0.395 -> 0.311;
+// 768 channels, 2 581 voxels 0.45 -> 0.37.   64 x 64: 64 channels, 5 876 voxels 0.033 -> 0.030, 41 700 0.099 -> 0.066 (2 581: 0.026
+// and 0.027);  128 channels, 2 581 voxels 0.039 -> 0.035, 41 700 0.200 -> 0.183.
+// Past these ranges the tiled kernel is level or ahead: 64 x 64 tiles, one from 667 763 voxels (0.71 both), a few of 166 977
+// (128 channels: 0.62, split 0.67), sixteen of 41 700 (256 channels: 0.63, split 0.66; 10 494: 0.20 -> 0.19), more of any number
+// (512 channels, 2 581 voxels 0.208 and 0.214);  four and more 96 x 96 tiles past 262 144 voxels: not measured.
+extern "C" int fgx_wgrad_split_tile(size_t n, int Ci, int Co, int* block_rows) {
+    if (n == 0 || Ci <= 0 || Co <= 0 || block_rows == nullptr || (size_t)Ci * Co >= (size_t)1024 * 1024) return 0;
+    auto padded = [&](int t) { return (double)cdiv(Ci, t) * t * cdiv(Co, t) * t; };
+    const int t = padded(96) <= padded(64) ? 96 : 64;
+    const size_t tiles = (size_t)cdiv(Ci, t) * cdiv(Co, t);
+    const size_t least = t == 64 && tiles == 1 ? 4096 : 2048;
+    const size_t most = t == 96 ? (tiles >= 4 ? 262144 : ~(size_t)0) : tiles == 1 ? 262144 : tiles < 16 ? 65536 : tiles == 16 ? 12288 : 0;
+    if (padded(32) <= 0.55 * padded(t) || n < least || n > most) return 0;
+    *block_rows = (int)std::min(round_up(cdiv(n, (size_t)(tiles < 4 ? 2 : 1)), 64), (size_t)1 << 30);
+    return t;
 }
 
 extern "C" int fgx_table_lookup(int pass_kind, int dtype, size_t n, int Ci, int Co, int V, fgx_schedule* out) {

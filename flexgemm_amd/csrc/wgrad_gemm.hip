@@ -1783,8 +1783,6 @@ int fgx_conv_wgrad_lists(int dtype, const void* grad_out, const void* feats, con
     }
     const bool stream_f16 = streaming && any && dtype == FGX_F16 && stream_ok<F16>(tile_rows, tile_cols, n, n_in, Ci, Co, tab.seg[V]);
     const bool stream_bf16 = streaming && any && dtype == FGX_BF16 && stream_ok<BF16>(tile_rows, tile_cols, n, n_in, Ci, Co, tab.seg[V]);
-    if (streaming && dtype == FGX_F32 && tile_rows == 96 && tile_cols == 96)
-        tile_rows = tile_cols = 32;         // a schedule for fgx_conv_wgrad_split, whose tile no other kernel has
     Layout L = layout(any ? n : 0, V, Ci, Co, block_rows, (stream_f16 || stream_bf16) && tile_rows == 32 ? 4 : 1);
     // 32-bit byte offsets into grad_out / feats are enough below 4 GiB
     const bool small = (double)n * Co * es < 4294967296.0 && (double)n_in * Ci * es < 4294967296.0;

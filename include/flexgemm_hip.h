@@ -235,8 +235,7 @@ typedef struct fgx_schedule {
     int splitk;         /* fwd/dgrad: number of K splits (1 = none) */
     int block_rows;     /* wgrad: voxel rows per partial-sum block */
     int stream;         /* 1 = persistent streaming kernel (fwd/dgrad: fgx_conv_gather_gemm_stream; wgrad: the
-                         * `streaming` argument of fgx_conv_wgrad, in fp32
-                         * fgx_conv_wgrad_split with tile = tile_rows), 0 = tiled kernel; wgrad only: 2 = the sweep
+                         * `streaming` argument of fgx_conv_wgrad), 0 = tiled kernel; wgrad only: 2 = the sweep
                          * fgx_conv_wgrad_sweep with tile = tile_rows and sub_rows = block_rows */
 } fgx_schedule;
 int fgx_table_lookup(int pass_kind, int dtype, size_t n, int Ci, int Co, int V, fgx_schedule* out);
@@ -507,7 +506,9 @@ int fgx_conv_wgrad_lists(int dtype, const void* grad_out, const void* feats,
  * products; `tile` = 64 or 96), and a second kernel adds the segments of an item in the order of their pairs: the same sum on every
  * run.  Operands, block_bounds (required) and block_rows as for fgx_conv_wgrad; grad_bias may be NULL.  scratch:
  * fgx_conv_wgrad_split_scratch_bytes bytes, 256-byte aligned, bias gradient included; 0 = not for this shape (operands or pair lists past 32-bit offsets,
- * more than 2 048 (block, offset) pairs, no voxels): use fgx_conv_wgrad. */
+ * more than 2 048 (block, offset) pairs, no voxels): use fgx_conv_wgrad.  fgx_wgrad_split_tile: the tile in which it is ahead of the
+ * table's choice, and its block_rows; 0 where it is not. */
+int fgx_wgrad_split_tile(size_t n, int Ci, int Co, int* block_rows);
 size_t fgx_conv_wgrad_split_scratch_bytes(size_t n, size_t n_in, uint32_t n_pairs, int V, int Ci, int Co, int tile, int block_rows);
 int fgx_conv_wgrad_split(const void* grad_out, const void* feats, const uint32_t* sig_i, const uint32_t* sig_o, const uint32_t* seg_host,
                          const uint32_t* block_bounds, size_t n, size_t n_in, int Ci, int Co, int V, int tile, int block_rows,

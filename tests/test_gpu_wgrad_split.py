@@ -51,12 +51,12 @@ def test_tiles_against_float64(monkeypatch, tile, n, blocks, ci, co):
 @pytest.mark.parametrize("n,ci,co,tile", [(2048, 96, 96, 96), (2047, 96, 96, None), (4096, 64, 64, 64), (4095, 64, 64, None), (12288, 256, 256, 64),
                                            (12289, 256, 256, None), (300000, 192, 160, None), (1 << 22, 96, 96, 96), (41700, 32, 32, None)])
 def test_rule(n, ci, co, tile):
-    s = nat.table_lookup(nat.PASS_WGRAD, torch.float32, n, ci, co, 27)
-    assert s.stream == (0 if tile is None else 1)
+    L, rows = nat.lib(), C.c_int(0)
+    got = L.fgx_wgrad_split_tile(nat.sz(n), ci, co, C.byref(rows))
+    assert got == (tile or 0)
     if tile is not None:
-        assert s.tile_rows == s.tile_cols == tile and -(-n // s.block_rows) <= 2
-        L = nat.lib()
-        assert L.fgx_conv_wgrad_split_scratch_bytes(nat.sz(n), nat.sz(n), C.c_uint32(n), 27, ci, co, tile, s.block_rows) > 0
+        assert -(-n // rows.value) <= 2
+        assert L.fgx_conv_wgrad_split_scratch_bytes(nat.sz(n), nat.sz(n), C.c_uint32(n), 27, ci, co, tile, rows.value) > 0
 
 
 def test_sizes_out_of_range():
