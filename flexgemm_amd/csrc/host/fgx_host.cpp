@@ -719,8 +719,10 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
         mark(name, "stop");
         return p;
     }
-    if (masked && !narrow && c.has("_order_left_out")) cache_post(c, true, false);
-    if (masked && !narrow && !(c.has("gray_code") && c.has("sorted_idx"))) c.obj.attr("_ensure_sorted")();
+    if (masked && !narrow && !(c.has("gray_code") && c.has("sorted_idx"))) {
+        if (c.has("_order_left_out")) cache_post(c, true, false);
+        else c.obj.attr("_ensure_sorted")();
+    }
     const Sched s = schedule(pass, src, n, ci, co, v);
     bool own_order = false;
     if (masked && !narrow && row_bytes <= module_int(g_impl, "LOCALITY_MAX_ROW_BYTES") && (c.has("_tile_order") || n >= module_int(g_impl, "LOCALITY_MIN_ROWS")) &&
