@@ -40,7 +40,7 @@ namespace {
     X(fgx_spconv_out_dims) X(fgx_spconv_out_coords_grid_workspace_bytes) X(fgx_spconv_out_coords_grid_count)                       \
     X(fgx_spconv_out_coords_grid_emit) X(fgx_tile_plan) X(fgx_gather_item_order) X(fgx_gather_item_order_workspace_bytes)          \
     X(fgx_weight_panel_bytes) X(fgx_pack_weight) X(fgx_conv_scratch_bytes) X(fgx_conv_gather_gemm_act_mask)                        \
-    X(fgx_conv_gather_gemm_weight_pays) X(fgx_conv_gather_gemm_weight) X(fgx_conv_gemm_pairs_pays) X(fgx_pair_plan_words) X(fgx_pair_plan) X(fgx_conv_gemm_pairs_scratch_bytes) X(fgx_conv_gemm_pairs)                                                             \
+    X(fgx_conv_gather_gemm_weight_pays) X(fgx_conv_gather_gemm_weight) X(fgx_conv_gemm_pairs_pays) X(fgx_pair_plan_words) X(fgx_pair_plan) X(fgx_conv_gemm_pairs_scratch_bytes) X(fgx_conv_gemm_pairs) X(fgx_conv_gemm_few_pays) X(fgx_conv_gemm_few)                                                             \
     X(fgx_conv_gather_gemm_stream_act_mask) X(fgx_conv_gather_gemm_stream_groups) X(fgx_relu_mask_apply) X(fgx_copy_columns)       \
     X(fgx_colsum_scratch_bytes) X(fgx_colsum) X(fgx_wgrad_block_bounds_count) X(fgx_wgrad_block_bounds)                            \
     X(fgx_conv_gemm_stem_pays) X(fgx_conv_gemm_stem) X(fgx_wgrad_stem_pays) X(fgx_wgrad_stem_scratch_bytes) X(fgx_conv_wgrad_stem) X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
@@ -253,7 +253,9 @@ Needs layer_needs(const Layer& l, int64_t n, int v, bool walks) {
     const bool resident = es == 2 && walks && v <= 27 && ci <= 32 && l.co <= 32 && l.co % 8 == 0 && n >= module_int(g_impl, "NARROW_RESIDENT_MIN_ROWS") &&
                           narrow_mode() != "off";
     const bool forward = resident || L.fgx_conv_gemm_stem_pays(l.code, 0, (size_t)n, ci, (int)l.co, v) ||
-                         (l.splitk && pairs_forward(l.record, es, l.relu, l.co) && L.fgx_conv_gemm_pairs_pays(l.code, 0, (size_t)n, ci, (int)l.co, v));
+                         (l.splitk && pairs_forward(l.record, es, l.relu, l.co) &&
+                          (L.fgx_conv_gemm_pairs_pays(l.code, 0, (size_t)n, ci, (int)l.co, v) ||
+                           (!l.record && L.fgx_conv_gemm_few_pays(l.code, (size_t)n, ci, (int)l.co, v))));
     const bool backward = !l.record || !l.input_grad || (resident && l.ci % 8 == 0) || L.fgx_conv_gemm_stem_pays(l.code, 1, (size_t)n, co, (int)l.ci, v) ||
                           (l.splitk && pairs_backward(es, l.relu, l.co) && L.fgx_conv_gemm_pairs_pays(l.code, 1, (size_t)n, (int)l.ci, co, v));
     needs.order = !(forward && backward);
@@ -645,9 +647,10 @@ struct Product {
 // map with the offsets mirrored, mode 2: through a map of its own, offsets as they are.  One row per row of the cache's
 // neighbor_map.  masked: mask-sorted schedule (else natural row order, all offsets per tile).  want_mask: also one bit per
 // output, "greater than zero", where the kernels can (ReLU, 16-bit type, a multiple of 8 columns).  panel: a kept weight
-// panel, or undefined to pack one.  pairs: whether the product over pairs may be taken.
+// panel, or undefined to pack one.  pairs: whether the product over pairs may be taken; few: the one-launch product of few voxels (a
+// submanifold layer at inference: in training its other order of sums would move values across a ReLU's zero).
 Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, int mode, bool allow_splitk, bool masked, int activation,
-                       bool want_mask, const Tensor& panel_kept, int64_t stream, bool pairs) {
+                       bool want_mask, const Tensor& panel_kept, int64_t stream, bool pairs, bool few = false) {
     const at::Device dev = src.device();
     const c10::DeviceGuard guard(dev);
     const int code = dtype_code(src);
@@ -696,6 +699,15 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
         check(L.fgx_conv_gemm_stem(code, mode, ptr(src), ptr(weight), ptr(bias), ptr<uint32_t>(nmap), (size_t)n, ci, co, v, activation, ptr(p.out),
                                    ptr<uint8_t>(p.mask), as_stream(stream)));
         mark(name, "stop");
+        return p;
+    }
+    // few voxels under a small weight: one launch
+    if (few && mode == 0 && masked && allow_splitk && !narrow && !want_mask && !panel_kept.defined() && L.fgx_conv_gemm_few_pays(code, (size_t)n, ci, co, v) &&
+        schedules_are_ours() && aligned(src) && aligned(weight)) {
+        p.out = make({n, cols}, src.scalar_type(), dev);
+        mark("gather_gemm_fwd", "start");
+        check(L.fgx_conv_gemm_few(code, ptr(src), ptr(weight), ptr(bias), ptr<uint32_t>(nmap), (size_t)n, ci, co, v, activation, ptr(p.out), as_stream(stream)));
+        mark("gather_gemm_fwd", "stop");
         return p;
     }
     // few voxels under a wide weight: the pairs' products and their sums, from a plan of the map that every layer on it shares (none is made
@@ -1130,7 +1142,7 @@ Tensor convolve(const Tensor& feats, py::object cache_obj, const Tensor& weight,
     {
         const at::NoGradGuard no_grad;
         p = gather_product(feats, weight.reshape({co, v, ci}), bias, c, 0, splitk, masked, relu ? FGX_ACT_RELU : FGX_ACT_NONE, bits, Tensor(),
-                           stream_of(feats), pairs);
+                           stream_of(feats), pairs, !record && !generic);
     }
     if (!record) return p.out;
     // (deleteNode: a long chain of layers is taken down without a stack frame per layer)

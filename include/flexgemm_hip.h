@@ -314,6 +314,12 @@ int fgx_conv_gemm_pairs(int dtype, int mode, const void* src, const void* weight
                         size_t n, size_t n_src, int Ci, int Co, int V, void* scratch, int activation, void* out,
                         uint8_t* relu_mask, fgx_stream_t stream);
 
+/* Forward product of few voxels under a small weight (16-bit types): one launch, rows and weight [Co][V][Ci] read in place, sums over the
+ * offsets split over a workgroup's wavefronts in a fixed order.  fgx_conv_gemm_few_pays: whether the operators take it. */
+int fgx_conv_gemm_few_pays(int dtype, size_t n, int Ci, int Co, int V);
+int fgx_conv_gemm_few(int dtype, const void* src, const void* weight, const void* bias, const uint32_t* map, size_t n, int Ci, int Co, int V,
+                      int activation, void* out, fgx_stream_t stream);
+
 /* out[i] = bit i of relu_mask ? grad[i] : 0 for i < numel (a multiple of 8; 16-bit types; grad and out 16-byte aligned,
  * out may be grad): the gradient of a fused ReLU from the mask its forward pass wrote.  One pass, numel / 8 bytes of mask
  * read beside the gradient.  No counterpart in the reference. */
