@@ -7,10 +7,10 @@
 // widened before it is shifted for both curves (the reference's z-order path shifts it as a 32-bit value, which loses
 // it for 64-bit codes with bit_length >= 11).
 //
-// All three passes are streaming: 16 bytes of coordinates and 4 or 8 bytes of code per voxel, one thread per voxel,
-// 16-byte vector accesses on the coordinate side.  The z-order shuffles are about 40 vector instructions and hide behind the
-// memory traffic (5.3 M voxels: 17 us each way, 6.3 TB/s).  The Hilbert codes are bound by theirs: 261 instructions to encode
-// and 216 to decode, one exchange-or-invert after the other for every bit, fill the SIMDs for as long as the launch takes (30 us).
+// All three passes are streaming: 16 bytes of coordinates and 4 or 8 bytes of code per voxel, 16-byte vector accesses on the
+// coordinate side.  The z-order shuffles are about 40 vector instructions and hide behind the memory traffic (5.3 M voxels: 17 us
+// each way, 6.3 TB/s).  The Hilbert codes are the Morton code taken through a state machine in LDS, two bits per axis at a time;
+// worked out bit by bit instead, 261 instructions to encode and 216 to decode filled the SIMDs for 30 us.
 #include <cstring>
 #include <string.h>
 
@@ -61,51 +61,110 @@ __host__ __device__ __forceinline__ T gather3(T v) {
     return gather_step<T, 1>(v & run_mask<T>(1));
 }
 
-// One level of Skilling's exchange/invert for axis value a against axis 0 (p0): if the level bit of a is set, the low
-// bits of p0 are inverted, otherwise the low bits in which p0 and a differ are exchanged.
-__host__ __device__ __forceinline__ void fold_axis(uint32_t& p0, uint32_t& a, uint32_t q, uint32_t low) {
-    const bool set = (a & q) != 0;
-    const uint32_t t = set ? 0u : ((p0 ^ a) & low);
-    p0 ^= set ? low : t;
-    a ^= t;
-}
+// Skilling's transform as a state machine over the octants of a point, from the top bit down.  What the levels above have done to the
+// lower bits is a signed permutation of the axes (exchanges and inversions act on all lower bits alike); what the Gray code's second half
+// has added up so far is one parity.  A state is the two together.  In a state, the octant of a level gives the code's three bits of that
+// level and the next state; both ways are tables of [state][octants of two levels], entry = the next state's row | the six bits.
+// A level of zeros above the point's own changes the state only, so an odd number of levels starts in the state one zero octant before the
+// first (`odd`).
+struct Octant {
+    uint8_t a[3];              // x, y, z
+};
 
-__host__ __device__ __forceinline__ void fold_axis0(uint32_t& p0, uint32_t q, uint32_t low) {
-    if (p0 & q) p0 ^= low;
-}
-
-__host__ __device__ __forceinline__ void axes_to_transpose(uint32_t& x, uint32_t& y, uint32_t& z, int bits) {
-    if (bits <= 0) return;
-    const uint32_t top = 1u << (bits - 1);
-    for (uint32_t q = top; q > 1; q >>= 1) {
-        const uint32_t low = q - 1;
-        fold_axis0(x, q, low);
-        fold_axis(x, y, q, low);
-        fold_axis(x, z, q, low);
+struct CurveState {
+    uint8_t axis[3], flip[3];  // transformed bit i = bit axis[i] of the point ^ flip[i]
+    uint8_t parity;
+    constexpr bool operator==(const CurveState& o) const {
+        for (int i = 0; i < 3; ++i)
+            if (axis[i] != o.axis[i] || flip[i] != o.flip[i]) return false;
+        return parity == o.parity;
     }
-    y ^= x;
-    z ^= y;
-    uint32_t t = 0;
-    for (uint32_t q = top; q > 1; q >>= 1)
-        if (z & q) t ^= q - 1;
-    x ^= t;
-    y ^= t;
-    z ^= t;
-}
-
-__host__ __device__ __forceinline__ void transpose_to_axes(uint32_t& x, uint32_t& y, uint32_t& z, int bits) {
-    if (bits <= 0) return;
-    const uint32_t t = z >> 1;
-    z ^= y;
-    y ^= x;
-    x ^= t;
-    const uint32_t end = 1u << bits;       // bits <= 21
-    for (uint32_t q = 2; q != end; q <<= 1) {
-        const uint32_t low = q - 1;
-        fold_axis(x, z, q, low);
-        fold_axis(x, y, q, low);
-        fold_axis0(x, q, low);
+    // The code's octant for the point's octant p (x at bit 2, z at bit 0), and the state below.
+    constexpr int step(int p, CurveState* below) const {
+        const int point[3] = {(p >> 2) & 1, (p >> 1) & 1, p & 1};
+        int t[3] = {};
+        for (int i = 0; i < 3; ++i) t[i] = point[axis[i]] ^ flip[i];
+        CurveState next = *this;
+        for (int i = 0; i < 3; ++i) {          // axis i against axis 0: its bit set inverts axis 0 below, clear exchanges the two
+            if (t[i]) {
+                next.flip[0] ^= 1;
+            } else if (i != 0) {
+                const uint8_t ax = next.axis[0], fl = next.flip[0];
+                next.axis[0] = next.axis[i], next.flip[0] = next.flip[i];
+                next.axis[i] = ax, next.flip[i] = fl;
+            }
+        }
+        const int g0 = t[0], g1 = g0 ^ t[1], g2 = g1 ^ t[2];
+        next.parity = (uint8_t)(parity ^ g2);
+        *below = next;
+        return (g0 ^ parity) << 2 | (g1 ^ parity) << 1 | (g2 ^ parity);
     }
+};
+
+constexpr int kMaxStates = 96, kPairOctants = 64;      // (48 signed permutations, two parities)
+
+struct CurveStates {
+    CurveState s[kMaxStates] = {};
+    int count = 0, odd = -1;
+    constexpr int find(const CurveState& x) const {
+        for (int i = 0; i < count; ++i)
+            if (s[i] == x) return i;
+        return -1;
+    }
+    constexpr CurveStates() {
+        s[count++] = CurveState{{0, 1, 2}, {0, 0, 0}, 0};      // the top level's own
+        for (int i = 0; i < count; ++i)
+            for (int p = 0; p < 8; ++p) {
+                CurveState below{};
+                (void)s[i].step(p, &below);
+                if (find(below) < 0) s[count++] = below;
+            }
+        for (int i = 0; i < count; ++i) {
+            CurveState below{};
+            if (s[i].step(0, &below) == 0 && below == s[0]) odd = i;
+        }
+    }
+};
+constexpr CurveStates kStates{};
+constexpr int kStateCount = kStates.count, kOddStart = kStates.odd;
+static_assert(kOddStart >= 0, "a zero octant leads to the first state from somewhere");
+
+struct CurveTable {
+    uint16_t entry[kStateCount * kPairOctants] = {};
+    explicit constexpr CurveTable(bool decode) {
+        for (int i = 0; i < kStateCount; ++i)
+            for (int hi = 0; hi < 8; ++hi) {
+                CurveState mid{}, end{};
+                const int code_hi = kStates.s[i].step(hi, &mid);
+                for (int lo = 0; lo < 8; ++lo) {
+                    const int code = code_hi << 3 | mid.step(lo, &end), point = hi << 3 | lo;
+                    entry[i * kPairOctants + (decode ? code : point)] =
+                        (uint16_t)(kStates.find(end) * kPairOctants | (decode ? point : code));
+                }
+            }
+    }
+};
+constexpr size_t kTableBytes = sizeof(CurveTable);
+static_assert(kStateCount * kPairOctants <= 65536 && kTableBytes % 16 == 0, "table");
+__device__ __attribute__((aligned(16))) const CurveTable g_encode_table(false), g_decode_table(true);
+
+// The code's spatial bits for Morton codes of `bits` levels, or back, through the table in LDS: U of them side by side.
+template <typename T, int U>
+__device__ __forceinline__ void walk_curve(const uint16_t* table, T (&v)[U], int bits) {
+    uint32_t row[U];
+    T out[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) row[u] = bits & 1 ? kOddStart * kPairOctants : 0, out[u] = 0;
+    for (int at = 3 * (bits + (bits & 1)) - 6; at >= 0; at -= 6) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t e = table[row[u] | ((uint32_t)(v[u] >> at) & (kPairOctants - 1))];
+            row[u] = e & ~(uint32_t)(kPairOctants - 1);
+            out[u] = (T)(out[u] << 6) | (e & (kPairOctants - 1));
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = out[u];
 }
 
 template <typename T>
@@ -113,49 +172,106 @@ __host__ __device__ __forceinline__ T spatial_mask(int bits) {
     return bits == 0 ? (T)0 : (T)(~(T)0) >> (8 * sizeof(T) - 3 * bits);
 }
 
-template <typename T, int MODE>
-__host__ __device__ __forceinline__ T encode_one(int4 c, int bits) {
+template <typename T>
+__device__ __forceinline__ T morton_of(int4 c, int bits) {
     const uint32_t keep = bits >= 32 ? 0xFFFFFFFFu : ((1u << bits) - 1u);
-    uint32_t x = (uint32_t)c.y & keep, y = (uint32_t)c.z & keep, z = (uint32_t)c.w & keep;
-    if (MODE == kHilbert) axes_to_transpose(x, y, z, bits);
-    const T spatial = (spread3<T>((T)x) << 2) | (spread3<T>((T)y) << 1) | spread3<T>((T)z);
+    const uint32_t x = (uint32_t)c.y & keep, y = (uint32_t)c.z & keep, z = (uint32_t)c.w & keep;
+    return (spread3<T>((T)x) << 2) | (spread3<T>((T)y) << 1) | spread3<T>((T)z);
+}
+
+template <typename T>
+__device__ __forceinline__ T with_batch(T spatial, int4 c, int bits) {
     const int shift = 3 * bits;
     const T batch = shift >= (int)(8 * sizeof(T)) ? (T)0 : (T)(uint32_t)c.x << shift;
     return (spatial & spatial_mask<T>(bits)) | batch;
 }
 
-template <typename T, int MODE>
-__host__ __device__ __forceinline__ int4 decode_one(T code, int bits) {
-    const T spatial = code & spatial_mask<T>(bits);
-    uint32_t x = (uint32_t)gather3<T>(spatial >> 2), y = (uint32_t)gather3<T>(spatial >> 1), z = (uint32_t)gather3<T>(spatial);
-    if (MODE == kHilbert) transpose_to_axes(x, y, z, bits);
+template <typename T>
+__device__ __forceinline__ int4 coords_of(T spatial, T code, int bits) {
+    const uint32_t x = (uint32_t)gather3<T>(spatial >> 2), y = (uint32_t)gather3<T>(spatial >> 1), z = (uint32_t)gather3<T>(spatial);
     const int shift = 3 * bits;
     const uint32_t b = shift >= (int)(8 * sizeof(T)) ? 0u : (uint32_t)(code >> shift);
     return make_int4((int)b, (int)x, (int)y, (int)z);
 }
 
-template <typename T, int MODE>
+// A thread per voxel of the z-order codes.  The Hilbert ones want their table in LDS (6 KB, read once per workgroup): no more
+// workgroups than the chip holds go over the voxels.
+template <int MODE>
+__device__ __forceinline__ void load_table(uint16_t* table, const CurveTable& from) {
+    if (MODE != kHilbert) return;
+    for (int i = threadIdx.x; i < (int)(kTableBytes / 16); i += kBlock) ((uint4*)table)[i] = ((const uint4*)from.entry)[i];
+    __syncthreads();
+}
+template <int MODE>
+constexpr int table_words() { return MODE == kHilbert ? kStateCount * kPairOctants : 8; }
+
+// Eight workgroups of four wavefronts fill a CU.  From a full chip on, three voxels a thread: three chains of dependent LDS reads side by
+// side.  5.3 M voxels in random order, 32-bit codes, us encode / decode: 27.6 / 25.9 bit by bit, 18.4 / 19.9 one voxel a thread, 18.0 / 18.2
+// three (5.9 TB/s), 18.4 / 18.0 four; 64-bit codes 30.0 / 28.9, 23.7 / 24.1, 21.6 / 21.6, 21.8 / 21.1; 100 000 voxels 3.0 / 2.8 and 2.5 / 2.6.
+constexpr unsigned kCurveGroups = 256 * 8;
+constexpr int kCurveVoxels = 3;
+
+template <typename T, int MODE, int U>
 __global__ void __launch_bounds__(kBlock) encode_kernel(const int32_t* __restrict__ coords, size_t n, int bits,
                                                         T* __restrict__ codes) {
-    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    codes[i] = encode_one<T, MODE>(reinterpret_cast<const int4*>(coords)[i], bits);
+    __shared__ __attribute__((aligned(16))) uint16_t table[table_words<MODE>()];
+    load_table<MODE>(table, g_encode_table);
+    for (size_t base = (size_t)blockIdx.x * (kBlock * U); base < n; base += (size_t)gridDim.x * (kBlock * U)) {
+        int4 c[U];
+        T v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const size_t i = base + u * kBlock + threadIdx.x;
+            c[u] = reinterpret_cast<const int4*>(coords)[i < n ? i : n - 1];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = morton_of<T>(c[u], bits);
+        if (MODE == kHilbert) walk_curve<T, U>(table, v, bits);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const size_t i = base + u * kBlock + threadIdx.x;
+            if (i < n) codes[i] = with_batch<T>(v[u], c[u], bits);
+        }
+    }
 }
 
-template <typename T, int MODE>
+template <typename T, int MODE, int U>
 __global__ void __launch_bounds__(kBlock) decode_kernel(const T* __restrict__ codes, size_t n, int bits,
                                                         int32_t* __restrict__ coords) {
-    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    reinterpret_cast<int4*>(coords)[i] = decode_one<T, MODE>(codes[i], bits);
+    __shared__ __attribute__((aligned(16))) uint16_t table[table_words<MODE>()];
+    load_table<MODE>(table, g_decode_table);
+    for (size_t base = (size_t)blockIdx.x * (kBlock * U); base < n; base += (size_t)gridDim.x * (kBlock * U)) {
+        T code[U], v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const size_t i = base + u * kBlock + threadIdx.x;
+            code[u] = codes[i < n ? i : n - 1];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = code[u] & spatial_mask<T>(bits);
+        if (MODE == kHilbert) walk_curve<T, U>(table, v, bits);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const size_t i = base + u * kBlock + threadIdx.x;
+            if (i < n) reinterpret_cast<int4*>(coords)[i] = coords_of<T>(v[u], code[u], bits);
+        }
+    }
+}
+
+// Workgroups of U voxels a thread: all of them for the z-order codes, no more than fit the chip, and of even length, for the Hilbert ones.
+unsigned groups_for(int mode, size_t n, int per_thread) {
+    const unsigned all = cdiv(n, (size_t)kBlock * per_thread);
+    return mode == kHilbert && all > kCurveGroups ? cdiv(all, cdiv(all, kCurveGroups)) : all;
 }
 
 template <typename T>
 int launch_encode(int mode, const int32_t* coords, size_t n, int bits, T* codes, hipStream_t s) {
     if (mode == kZOrder)
-        encode_kernel<T, kZOrder><<<cdiv(n, kBlock), kBlock, 0, s>>>(coords, n, bits, codes);
+        encode_kernel<T, kZOrder, 1><<<groups_for(mode, n, 1), kBlock, 0, s>>>(coords, n, bits, codes);
+    else if (n < (size_t)kBlock * kCurveGroups)
+        encode_kernel<T, kHilbert, 1><<<groups_for(mode, n, 1), kBlock, 0, s>>>(coords, n, bits, codes);
     else
-        encode_kernel<T, kHilbert><<<cdiv(n, kBlock), kBlock, 0, s>>>(coords, n, bits, codes);
+        encode_kernel<T, kHilbert, kCurveVoxels><<<groups_for(mode, n, kCurveVoxels), kBlock, 0, s>>>(coords, n, bits, codes);
     FGX_CHECK_LAUNCH("fgx_serialize_encode");
     return FGX_OK;
 }
@@ -163,9 +279,11 @@ int launch_encode(int mode, const int32_t* coords, size_t n, int bits, T* codes,
 template <typename T>
 int launch_decode(int mode, const T* codes, size_t n, int bits, int32_t* coords, hipStream_t s) {
     if (mode == kZOrder)
-        decode_kernel<T, kZOrder><<<cdiv(n, kBlock), kBlock, 0, s>>>(codes, n, bits, coords);
+        decode_kernel<T, kZOrder, 1><<<groups_for(mode, n, 1), kBlock, 0, s>>>(codes, n, bits, coords);
+    else if (n < (size_t)kBlock * kCurveGroups)
+        decode_kernel<T, kHilbert, 1><<<groups_for(mode, n, 1), kBlock, 0, s>>>(codes, n, bits, coords);
     else
-        decode_kernel<T, kHilbert><<<cdiv(n, kBlock), kBlock, 0, s>>>(codes, n, bits, coords);
+        decode_kernel<T, kHilbert, kCurveVoxels><<<groups_for(mode, n, kCurveVoxels), kBlock, 0, s>>>(codes, n, bits, coords);
     FGX_CHECK_LAUNCH("fgx_serialize_decode");
     return FGX_OK;
 }

@@ -65,6 +65,18 @@ def test_random_coords_all_widths(gpu_device, mode, batch, res):
     assert torch.equal(ops.serialize.decode_seq(torch.from_numpy(want).to(gpu_device), shape, mode=mode), coords)
 
 
+@pytest.mark.parametrize("res", [256, 512, 1024, 2048])      # 8 ... 11 levels: even and odd numbers of them, 32- and 64-bit codes
+@pytest.mark.parametrize("n", [1, 255, 257, 524_287, 524_288, 524_289, 1_572_865])
+def test_hilbert_codes_where_the_voxels_per_thread_change(gpu_device, n, res):
+    coords_np = _random_coords(n, 2, res, seed=n % 1000 + res)
+    shape = torch.Size([2, 0, res, res, res])
+    _say(f"serialize n={n} res={res}")
+    coords = torch.from_numpy(coords_np).to(gpu_device)
+    codes = ops.serialize.encode_seq(coords, shape, mode="hilbert")
+    assert np.array_equal(codes.cpu().numpy(), oz.encode_seq(coords_np, shape, "hilbert"))
+    assert torch.equal(ops.serialize.decode_seq(codes, shape, mode="hilbert"), coords)
+
+
 @pytest.mark.parametrize("mode", MODES)
 def test_round_trip_at_full_size(gpu_device, mode):
     """The reference's largest case is the res-2048 shell (about 10.7 M voxels); the same count of random voxels of that
