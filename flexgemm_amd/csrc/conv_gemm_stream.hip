@@ -87,19 +87,6 @@ struct StreamCfg {
     static constexpr size_t fixed_lds = (size_t)S * STAGE_BYTES + (size_t)kPlanSlots * IDX_SLOT_BYTES + OROW_BYTES + kBandSlots * 4;
 };
 
-// s_waitcnt vmcnt(n) for a wave-uniform n in [LO, HI]: the count is an immediate, so a binary tree of scalar branches
-// picks the instruction.
-template <int LO, int HI>
-__device__ __forceinline__ void wait_vmcnt_in(int n) {
-    if constexpr (LO == HI) {
-        wait_vmcnt<LO>();
-    } else {
-        constexpr int MID = (LO + HI) / 2;
-        if (n <= MID) wait_vmcnt_in<LO, MID>(n);
-        else wait_vmcnt_in<MID + 1, HI>(n);
-    }
-}
-
 __device__ __forceinline__ void wg_barrier() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();

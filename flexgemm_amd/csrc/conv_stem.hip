@@ -7,7 +7,9 @@
 // of features, and the 32-wide tile multiplies mostly padding.  Here the features of a row's V neighbors lie next to each other
 // in LDS (a missing neighbor: zeros), [rows][V * Ci], and one product with the rows' own grad_out gives every offset at
 // once: grad_out is read once per 64 of its columns, the pair lists not at all.  What bounds it are the 16-byte gathers, one
-// per (row, offset): 64 rows a step take 1.4 us of a CU, 1 792 pieces at about 0.6 per clock.  A last piece per row holds a one: its column is the bias gradient.
+// per (row, offset): 1 792 pieces for 64 rows, 0.88 us of a CU.  Four wavefronts do nothing but load and eight nothing but multiply: with both in one
+// (issue a step's loads, then multiply another's) the address pipeline stood still while all of them multiplied, 1.4 us a step.  424 000 voxels
+// 6 -> 48 channels 38 -> 29 us, 16 -> 48 67 -> 52.  A last piece per row holds a one: its column is the bias gradient.
 // A workgroup keeps all accumulators over its contiguous run of rows and writes one partial product; a second kernel adds the
 // partial products in workgroup order (same bits on every run).
 #include "wgrad_device.h"
@@ -20,7 +22,8 @@ __device__ __attribute__((aligned(256))) unsigned char g_zero_block_s[256];
 __device__ __attribute__((aligned(256))) uint16_t g_one_f16[8] = {0x3C00, 0, 0, 0, 0, 0, 0, 0};
 __device__ __attribute__((aligned(256))) uint16_t g_one_bf16[8] = {0x3F80, 0, 0, 0, 0, 0, 0, 0};
 
-constexpr int kStemWaves = 8, kStemThreads = 64 * kStemWaves, kStemStages = 3, kStemIdxSlots = 4;
+constexpr int kStemWaves = 8, kStemLoaders = 4;                // wavefronts that multiply, and that only load (one per SIMD)
+constexpr int kStemThreads = 64 * (kStemWaves + kStemLoaders), kStemStages = 3, kStemIdxSlots = 4;
 constexpr int kStemMaxV = 27, kStemCols = 64;
 
 // P: 16-byte pieces of a feature row (Ci = 8 P)
@@ -33,13 +36,13 @@ struct StemCfg {
     static constexpr int ROWB = PIECES * 16;
     static constexpr int F_BYTES = ROWS * ROWB, G_BYTES = ROWS * kStemCols * 2;
     static constexpr int F_INST = F_BYTES / 1024, G_INST = G_BYTES / 1024;
-    static constexpr int PER = (F_INST + G_INST + kStemWaves - 1) / kStemWaves;    // row loads per wavefront and step
-    static constexpr int LPS = PER + 1;                        // + one load of map words
+    static constexpr int F_PER = F_INST / kStemLoaders, G_PER = G_INST / kStemLoaders;     // loads per loader and step
     static constexpr int IDX_BYTES = ROWS * kStemMaxV * 4;
     static constexpr int IDX_SLOT = (IDX_BYTES + 1023) / 1024 * 1024;
+    static constexpr int IDX_INST = IDX_SLOT / 1024, IDX_PER = (IDX_INST + kStemLoaders - 1) / kStemLoaders;
     static constexpr int STAGE = F_BYTES + G_BYTES;
-    static constexpr size_t LDS = (size_t)kStemStages * STAGE + kStemIdxSlots * IDX_SLOT + 1024;
-    static_assert(IDX_SLOT / 1024 <= kStemWaves && F_BYTES % 1024 == 0, "one load of map words per wavefront");
+    static constexpr size_t LDS = (size_t)kStemStages * STAGE + kStemIdxSlots * IDX_SLOT;
+    static_assert(F_INST % kStemLoaders == 0 && G_INST % kStemLoaders == 0 && F_BYTES % 1024 == 0, "every loader has as many loads");
     static_assert(NT_PER % 2 == 0, "fragments are waited for in fours");
     static_assert(LDS <= 160 * 1024, "LDS");
     // XOR key on the 16-byte pieces of a grad_out row (8 of them): four rows of a transposing read on distinct banks.  Rows of
@@ -50,30 +53,65 @@ struct StemCfg {
 // Map words of step j: ROWS * V of them in a row, 16 bytes per lane; past the map's end, and in the steps after the last one, zeros
 // that nobody reads.
 template <int P>
-__device__ __forceinline__ void stem_issue_idx(const uint32_t* map, unsigned long long map_bytes, unsigned lo, int nsteps, int j, int V, int wave,
-                                               int lane, unsigned char* slot, unsigned char* dump, const unsigned char* zero_b) {
+__device__ __forceinline__ void stem_issue_idx(const uint32_t* map, unsigned long long map_bytes, unsigned lo, int nsteps, int j, int V, int loader,
+                                               int lane, unsigned char* slot, const unsigned char* zero_b) {
     using C = StemCfg<P>;
-    const unsigned long long at = (unsigned long long)(lo + (unsigned)j) * (unsigned)(C::ROWS * V * 4) + (unsigned)(wave * 1024 + lane * 16);
-    const bool real = j < nsteps && wave * 1024 + lane * 16 < C::ROWS * V * 4 && at + 16 <= map_bytes;
-    const unsigned char* p = real ? (const unsigned char*)map + at : zero_b;
-    unsigned char* dst = wave * 1024 < C::IDX_SLOT ? slot + wave * 1024 : dump;
-    __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(dst), 16, 0, 0);
+#pragma unroll
+    for (int i = 0; i < C::IDX_PER; ++i) {
+        const int inst = i * kStemLoaders + loader;            // wave-uniform
+        if (inst >= C::IDX_INST) break;
+        const int byte = inst * 1024 + lane * 16;
+        const unsigned long long at = (unsigned long long)(lo + (unsigned)j) * (unsigned)(C::ROWS * V * 4) + (unsigned)byte;
+        const bool real = j < nsteps && byte < C::ROWS * V * 4 && at + 16 <= map_bytes;
+        const unsigned char* p = real ? (const unsigned char*)map + at : zero_b;
+        __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(slot + inst * 1024), 16, 0, 0);
+    }
 }
 
-// Where piece `at` of row `row` of a step comes from.  WHOLE: a step with all its rows; the last one has `rows`, and its map
-// rows are read where they are (16 bytes of them may end past the map).
-template <int P, bool WHOLE>
-__device__ __forceinline__ const unsigned char* stem_piece(const unsigned char* feats, const uint32_t* map, const uint32_t* words,
-                                                           const unsigned char* one_b, const unsigned char* zero_b, unsigned long long base,
-                                                           int row, int rows, int at, int V) {
+// Where piece `at` of row `row` comes from in the last step, which has `rows` rows: map rows are read where they are (16 bytes of
+// them may end past the map).
+template <int P>
+__device__ __forceinline__ const unsigned char* stem_piece(const unsigned char* feats, const uint32_t* map, const unsigned char* one_b,
+                                                           const unsigned char* zero_b, unsigned long long base, int row, int rows, int at, int V) {
     const int v = at / P, part = at - v * P;
-    if (!WHOLE && row >= rows) return zero_b;
+    if (row >= rows) return zero_b;
     if (v < V) {
-        const uint32_t m = WHOLE ? words[row * V + v] : map[(base + (unsigned)row) * (unsigned)V + (unsigned)v];
+        const uint32_t m = map[(base + (unsigned)row) * (unsigned)V + (unsigned)v];
         return m != FGX_EMPTY32 ? feats + (size_t)m * (16 * P) + part * 16 : zero_b;
     }
     return at == StemCfg<P>::PIECES - 1 ? one_b : zero_b;
 }
+
+// A loader's loads of a whole step's pieces: load i covers the 64 pieces from (i * loaders + loader) * 64 on.  Which map word names a lane's row, or
+// which constant the piece is instead, is the same for every step; the words of all loads are read before the first address is needed.
+template <int P>
+struct StemPieces {
+    static constexpr int N = StemCfg<P>::F_PER;
+    uint32_t word[N];
+    uint32_t offsets = 0, second = 0, ones = 0;                // bit i: load i's piece belongs to a kernel position; is the row's second one; is the ones'
+    template <typename Key>
+    __device__ __forceinline__ void init(int loader, int lane, int V, Key key) {
+        using C = StemCfg<P>;
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            const int piece = (i * kStemLoaders + loader) * 64 + lane, row = piece / C::PIECES, at = (piece - row * C::PIECES) ^ key(row), v = at / P;
+            const bool offset = v < V;
+            word[i] = offset ? (uint32_t)(row * V + v) : 0u;
+            offsets |= (uint32_t)offset << i;
+            second |= (uint32_t)(at - v * P) << i;
+            ones |= (uint32_t)(at == C::PIECES - 1) << i;
+        }
+    }
+    __device__ __forceinline__ void read(const uint32_t* words, uint32_t (&m)[N]) const {
+#pragma unroll
+        for (int i = 0; i < N; ++i) m[i] = words[word[i]];
+    }
+    __device__ __forceinline__ const unsigned char* source(int i, uint32_t m, const unsigned char* feats, const unsigned char* one_b,
+                                                           const unsigned char* zero_b) const {
+        const unsigned char* otherwise = (ones >> i) & 1u ? one_b : zero_b;
+        return ((offsets >> i) & 1u) & (uint32_t)(m != FGX_EMPTY32) ? feats + (size_t)m * (16 * P) + (P == 2 ? ((second >> i) & 1u) * 16 : 0u) : otherwise;
+    }
+};
 
 template <typename Tag, int P>
 __global__ void __launch_bounds__(kStemThreads)
@@ -86,10 +124,9 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     unsigned char* ring = lds;                                 // [S][features | grad_out]
     unsigned char* idx_ring = lds + S * C::STAGE;              // [kStemIdxSlots] map rows
-    unsigned char* dump = idx_ring + kStemIdxSlots * C::IDX_SLOT;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wave_m = wave & 1, wave_n = wave >> 1;
+    const int wave_m = wave & 1, wave_n = (wave >> 1) & 3;     // (of a multiplier)
     const int g = lane >> 5, l32 = lane & 31, s16 = lane & 15, mb = (lane >> 4) & 1;
     const int m0 = (int)blockIdx.y * kStemCols;
 
@@ -107,37 +144,67 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
     const unsigned char* zero_b = g_zero_block_s;
     const unsigned long long map_bytes = (unsigned long long)n * V * 4;
 
-    auto issue_idx = [&](int j) __attribute__((always_inline)) {
-        stem_issue_idx<P>(map, map_bytes, lo, nsteps, j, V, wave, lane, idx_ring + (j & (kStemIdxSlots - 1)) * C::IDX_SLOT, dump, zero_b);
-    };
-    auto issue_rows_of = [&](int j, auto whole) __attribute__((always_inline)) {
-        constexpr bool WHOLE = decltype(whole)::value;
-        unsigned char* stage = ring + (j % S) * C::STAGE;
-        const uint32_t* words = (const uint32_t*)(idx_ring + (j & (kStemIdxSlots - 1)) * C::IDX_SLOT);
-        const unsigned long long base = (unsigned long long)(lo + (unsigned)j) * C::ROWS;
-        const int rows = WHOLE ? C::ROWS : (j < nsteps && base < n ? (int)(n - base) : 0);
+    // The loaders' walk over the steps; the multipliers meet them at its barriers.
+    auto load_run = [&]() __attribute__((always_inline)) {
+        const int lw = wave - kStemWaves;
+        StemPieces<P> pieces;
+        pieces.init(lw, lane, V, [](int) { return 0; });
+        const int step_loads = C::F_PER + C::G_PER + (C::IDX_INST - lw + kStemLoaders - 1) / kStemLoaders;
+        auto issue_idx = [&](int j) __attribute__((always_inline)) {
+            stem_issue_idx<P>(map, map_bytes, lo, nsteps, j, V, lw, lane, idx_ring + (j & (kStemIdxSlots - 1)) * C::IDX_SLOT, zero_b);
+        };
+        auto issue_rows_of = [&](int j, auto whole) __attribute__((always_inline)) {
+            constexpr bool WHOLE = decltype(whole)::value;
+            unsigned char* stage = ring + (j % S) * C::STAGE;
+            const uint32_t* words = (const uint32_t*)(idx_ring + (j & (kStemIdxSlots - 1)) * C::IDX_SLOT);
+            const unsigned long long base = (unsigned long long)(lo + (unsigned)j) * C::ROWS;
+            const int rows = WHOLE ? C::ROWS : (j < nsteps && base < n ? (int)(n - base) : 0);
+            uint32_t named[C::F_PER];
+            if (WHOLE) pieces.read(words, named);
 #pragma unroll
-        for (int i = 0; i < C::PER; ++i) {
-            const int inst = i * kStemWaves + wave;            // wave-uniform
-            const unsigned char* p = zero_b;
-            unsigned char* dst = dump;
-            if (inst < C::F_INST) {
-                const int piece = inst * 64 + lane;
-                const int row = piece / C::PIECES;
-                dst = stage + inst * 1024;
-                p = stem_piece<P, WHOLE>(feats_b, map, words, one_b, zero_b, base, row, rows, piece - row * C::PIECES, V);
-            } else if (inst < C::F_INST + C::G_INST) {
-                const int piece = (inst - C::F_INST) * 64 + lane;
+            for (int i = 0; i < C::G_PER; ++i) {
+                const int inst = i * kStemLoaders + lw, piece = inst * 64 + lane;
                 const int row = piece >> 3, c = ((piece & 7) ^ C::key(row)) * 8;       // first column
-                dst = stage + C::F_BYTES + (inst - C::F_INST) * 1024;
+                const unsigned char* p = zero_b;
                 if ((WHOLE || row < rows) && m0 + c < Co) p = gout_b + ((base + (unsigned)row) * (unsigned)Co + (unsigned)(m0 + c)) * 2;
+                __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(stage + C::F_BYTES + inst * 1024), 16, 0, 0);
             }
-            __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(dst), 16, 0, 0);
+#pragma unroll
+            for (int i = 0; i < C::F_PER; ++i) {
+                const int inst = i * kStemLoaders + lw;
+                const unsigned char* p;
+                if constexpr (WHOLE) {
+                    p = pieces.source(i, named[i], feats_b, one_b, zero_b);
+                } else {
+                    const int piece = inst * 64 + lane, row = piece / C::PIECES;
+                    p = stem_piece<P>(feats_b, map, one_b, zero_b, base, row, rows, piece - row * C::PIECES, V);
+                }
+                __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(stage + inst * 1024), 16, 0, 0);
+            }
+        };
+        auto issue_rows = [&](int j) __attribute__((always_inline)) {
+            if (j < nsteps && (unsigned long long)(lo + (unsigned)j + 1) * C::ROWS <= n) issue_rows_of(j, std::true_type{});
+            else issue_rows_of(j, std::false_type{});
+        };
+#pragma unroll
+        for (int j = 0; j < S - 1; ++j) issue_idx(j);
+        wait_vmcnt<0>();
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < S - 1; ++j) {
+            issue_rows(j);
+            issue_idx(j + S - 1);
         }
-    };
-    auto issue_rows = [&](int j) __attribute__((always_inline)) {
-        if (j < nsteps && (unsigned long long)(lo + (unsigned)j + 1) * C::ROWS <= n) issue_rows_of(j, std::true_type{});
-        else issue_rows_of(j, std::false_type{});
+        for (int k = 0; k < nsteps; ++k) {
+            // rows of step k and the map words of step k + S - 1 have landed
+            wait_vmcnt_in<(S - 2) * (C::F_PER + C::G_PER), (S - 2) * (C::F_PER + C::G_PER + C::IDX_PER)>((S - 2) * step_loads);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();                      // ... everybody's; the stage of step k - 1 is free
+            asm volatile("" ::: "memory");
+            issue_rows(k + S - 1);
+            issue_idx(k + 2 * (S - 1));
+        }
+        wait_vmcnt<0>();                                       // the loads of the steps past the end
     };
 
     f32x16 acc[C::NT_PER];
@@ -151,24 +218,12 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
 
-#pragma unroll
-        for (int j = 0; j < S - 1; ++j) issue_idx(j);
-        wait_vmcnt<0>();
         __syncthreads();
-#pragma unroll
-        for (int j = 0; j < S - 1; ++j) {
-            issue_rows(j);
-            issue_idx(j + S - 1);
-        }
-
         constexpr int NK = C::ROWS / 16;
         for (int k = 0; k < nsteps; ++k) {
-            wait_vmcnt<(S - 2) * C::LPS>();                        // rows of step k and the map words of step k + S - 1 have landed
             asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_barrier();                          // ... everybody's; the stage of step k - 1 is free
+            __builtin_amdgcn_s_barrier();                          // the loaders saw the rows of step k land
             asm volatile("" ::: "memory");
-            issue_rows(k + S - 1);
-            issue_idx(k + 2 * (S - 1));
             const unsigned char* f_cur = ring + (k % S) * C::STAGE;
             const unsigned char* g_cur = f_cur + C::F_BYTES;
 #pragma unroll
@@ -222,13 +277,22 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
                 }
             }
         }
-        wait_vmcnt<0>();                                           // the loads of the steps past the end
     };
-    run(std::false_type{});
+    const bool loader = wave >= kStemWaves;                        // wave-uniform role
     bool finite = true;
+    if (loader) {
+        __builtin_amdgcn_s_setprio(3);
+        load_run();
+    } else {
+        run(std::false_type{});
 #pragma unroll
-    for (int t = 0; t < C::NT_PER; ++t) finite = finite && all_finite(acc[t]);
-    if (__syncthreads_or(!finite)) run(std::true_type{});
+        for (int t = 0; t < C::NT_PER; ++t) finite = finite && all_finite(acc[t]);
+    }
+    if (__syncthreads_or(!finite)) {
+        if (loader) load_run();
+        else run(std::true_type{});
+    }
+    if (loader) return;
 
     // partial[column tile][group][64][N]
     float* dst = partial + ((size_t)blockIdx.y * groups + group) * ((size_t)kStemCols * C::N);
@@ -273,25 +337,39 @@ __global__ void __launch_bounds__(1024) stem_reduce_kernel(const float* __restri
 // Forward product and input gradient of such layers (8 or 16 channels on the gathered side): the neighbors' features of a row lie
 // side by side as in the weight gradient, and one product with the weight, [V * K] x [columns], replaces V products that fill
 // a quarter (8 channels) or half of a K-slab.  The wavefronts keep the weight in registers over the workgroup's run of rows; the
-// piece with the one multiplies the bias.  Rows are walked as they come, nothing of the mask sort is read.
+// piece with the one multiplies the bias.  Rows are walked as they come, nothing of the mask sort is read.  Loaders and multipliers as in the
+// weight gradient; a step is bound by what follows its barrier in a multiplier, 14 reads of LDS, 14 products in a row, rounding and two stores.
+// 424 000 voxels, us: 6 -> 48 channels fp16 52 -> 35, bf16 64 -> 50; 16 -> 48 bf16 120 -> 78.
 template <int P>
 struct StemGemmCfg {
     using W = StemCfg<P>;
     static constexpr int COLS = 128;                           // output columns of a workgroup: four tiles of 32, one per wavefront column
     static constexpr int RT = W::ROWS / 32;                    // row tiles of a step
+    static constexpr int WAVES = 4 * RT, THREADS = 64 * (WAVES + kStemLoaders);        // a multiplier for each of the tiles
     static constexpr int KK = W::PIECES / 2;                   // products of a tile: 16 K values each
-    static constexpr int PER = (W::F_INST + kStemWaves - 1) / kStemWaves;
-    static constexpr int LPS = PER + 1;
+    static constexpr int AHEAD = 14;              // ... whose row fragments a wavefront has registers for beside the weight's
     static constexpr int STAGES = 4, IDX_SLOTS = 2 * (STAGES - 1);     // (a slot is written again once its step's rows are on their way)
-    static constexpr size_t LDS = (size_t)STAGES * W::F_BYTES + IDX_SLOTS * W::IDX_SLOT + 1024;
+    static constexpr size_t LDS = (size_t)STAGES * W::F_BYTES + IDX_SLOTS * W::IDX_SLOT;
     static_assert(LDS <= 160 * 1024, "LDS");
     // XOR key on the low bits of a row's piece numbers: 16 rows' reads of one piece fall on distinct banks (rows are 28 or 56 pieces)
     static __device__ __forceinline__ int key(int row) { return P == 1 ? (row >> 2) & 3 : (row >> 1) & 7; }
 };
 
+// a's lanes 32 - 63 and b's lanes 0 - 31 change places; a's odd runs of 16 lanes and b's even ones.
+__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
+    const auto both = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = both[0];
+    b = both[1];
+}
+__device__ __forceinline__ void swap_rows(uint32_t& a, uint32_t& b) {
+    const auto both = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = both[0];
+    b = both[1];
+}
+
 // mode as in fgx_pack_weight: 0 weight [cols][V][K], 1 / 2 weight [K][V][cols] with mirrored offsets / as they are
 template <typename Tag, int P>
-__global__ void __launch_bounds__(kStemThreads)
+__global__ void __launch_bounds__(StemGemmCfg<P>::THREADS)
 stem_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Tag::type* __restrict__ weight,
                  const typename Tag::type* __restrict__ bias, const uint32_t* __restrict__ map, uint32_t n, int V, int cols, int mode,
                  unsigned steps_total, unsigned groups, int relu, typename Tag::type* __restrict__ out, uint8_t* __restrict__ relu_mask) {
@@ -302,13 +380,12 @@ stem_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Tag:
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     unsigned char* ring = lds;                                 // [S][rows' features]
     unsigned char* idx_ring = lds + S * C::F_BYTES;
-    unsigned char* dump = idx_ring + G::IDX_SLOTS * C::IDX_SLOT;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 5, l32 = lane & 31;
-    const int ct = wave & 3, rt = wave >> 2;                   // column and row tile of this wavefront
+    const int ct = wave & 3, rt = wave >> 2;                   // column and row tile of a multiplier
     const int c0 = (int)blockIdx.y * G::COLS + ct * 32;
-    const bool multiplies = rt < G::RT && c0 < cols;
+    const bool multiplies = c0 < cols;
 
     const unsigned per_xcd = (groups + kXcds - 1) / kXcds;
     const unsigned group = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
@@ -317,107 +394,158 @@ stem_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Tag:
     const unsigned hi = (unsigned)((unsigned long long)steps_total * (group + 1) / groups);
     const int nsteps = (int)(hi - lo);
 
-    // the weight's fragments: lane l32 is a column, a piece its 8 consecutive K values
-    i16x8 wf[G::KK];
-#pragma unroll
-    for (int kk = 0; kk < G::KK; ++kk) {
-        i16x8 f = {0, 0, 0, 0, 0, 0, 0, 0};
-        const int at = kk * 2 + g, v = at / P, part = at - v * P, col = c0 + l32;
-        if (multiplies && col < cols) {
-            if (v < V && mode == 0) {
-                f = *reinterpret_cast<const i16x8*>((const short*)weight + ((size_t)col * V + v) * (8 * P) + part * 8);
-            } else if (v < V) {
-                const int from = mode == 1 ? V - 1 - v : v;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) f[e] = ((const short*)weight)[((size_t)(part * 8 + e) * V + from) * cols + col];
-            } else if (at == C::PIECES - 1 && bias != nullptr) {
-                f[0] = ((const short*)bias)[col];
-            }
-        }
-        wf[kk] = f;
-    }
-
     const unsigned char* src_b = (const unsigned char*)src;
     const unsigned char* one_b = (const unsigned char*)(__is_same(T, _Float16) ? g_one_f16 : g_one_bf16);
     const unsigned char* zero_b = g_zero_block_s;
     const unsigned long long map_bytes = (unsigned long long)n * V * 4;
-    auto issue_idx = [&](int j) {
-        stem_issue_idx<P>(map, map_bytes, lo, nsteps, j, V, wave, lane, idx_ring + (j % G::IDX_SLOTS) * C::IDX_SLOT, dump, zero_b);
-    };
-    auto issue_rows_of = [&](int j, auto whole) {
-        constexpr bool WHOLE = decltype(whole)::value;
-        unsigned char* stage = ring + (j % S) * C::F_BYTES;
-        const uint32_t* words = (const uint32_t*)(idx_ring + (j % G::IDX_SLOTS) * C::IDX_SLOT);
-        const unsigned long long base = (unsigned long long)(lo + (unsigned)j) * C::ROWS;
-        const int rows = WHOLE ? C::ROWS : (j < nsteps && base < n ? (int)(n - base) : 0);
-#pragma unroll
-        for (int i = 0; i < G::PER; ++i) {
-            const int inst = i * kStemWaves + wave;            // wave-uniform
-            const unsigned char* p = zero_b;
-            unsigned char* dst = dump;
-            if (inst < C::F_INST) {
-                const int piece = inst * 64 + lane;
-                const int row = piece / C::PIECES, at = (piece - row * C::PIECES) ^ G::key(row);
-                dst = stage + inst * 1024;
-                p = stem_piece<P, WHOLE>(src_b, map, words, one_b, zero_b, base, row, rows, at, V);
-            }
-            __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(dst), 16, 0, 0);
-        }
-    };
-    auto issue_rows = [&](int j) {
-        if (j < nsteps && (unsigned long long)(lo + (unsigned)j + 1) * C::ROWS <= n) issue_rows_of(j, std::true_type{});
-        else issue_rows_of(j, std::false_type{});
-    };
 
+    if (wave >= G::WAVES) {
+        __builtin_amdgcn_s_setprio(3);
+        const int lw = wave - G::WAVES;
+        StemPieces<P> pieces;
+        pieces.init(lw, lane, V, [](int row) { return G::key(row); });
+        const int step_loads = C::F_PER + (C::IDX_INST - lw + kStemLoaders - 1) / kStemLoaders;
+        auto issue_idx = [&](int j) {
+            stem_issue_idx<P>(map, map_bytes, lo, nsteps, j, V, lw, lane, idx_ring + (j % G::IDX_SLOTS) * C::IDX_SLOT, zero_b);
+        };
+        auto issue_rows_of = [&](int j, auto whole) {
+            constexpr bool WHOLE = decltype(whole)::value;
+            unsigned char* stage = ring + (j % S) * C::F_BYTES;
+            const uint32_t* words = (const uint32_t*)(idx_ring + (j % G::IDX_SLOTS) * C::IDX_SLOT);
+            const unsigned long long base = (unsigned long long)(lo + (unsigned)j) * C::ROWS;
+            const int rows = WHOLE ? C::ROWS : (j < nsteps && base < n ? (int)(n - base) : 0);
+            uint32_t named[C::F_PER];
+            if (WHOLE) pieces.read(words, named);
 #pragma unroll
-    for (int j = 0; j < S - 1; ++j) issue_idx(j);
-    wait_vmcnt<0>();
-    __syncthreads();
+            for (int i = 0; i < C::F_PER; ++i) {
+                const int inst = i * kStemLoaders + lw;
+                const unsigned char* p;
+                if constexpr (WHOLE) {
+                    p = pieces.source(i, named[i], src_b, one_b, zero_b);
+                } else {
+                    const int piece = inst * 64 + lane, row = piece / C::PIECES;
+                    p = stem_piece<P>(src_b, map, one_b, zero_b, base, row, rows, (piece - row * C::PIECES) ^ G::key(row), V);
+                }
+                __builtin_amdgcn_global_load_lds(FGX_GLOBAL_PTR(p), FGX_LDS_PTR(stage + inst * 1024), 16, 0, 0);
+            }
+        };
+        auto issue_rows = [&](int j) {
+            if (j < nsteps && (unsigned long long)(lo + (unsigned)j + 1) * C::ROWS <= n) issue_rows_of(j, std::true_type{});
+            else issue_rows_of(j, std::false_type{});
+        };
 #pragma unroll
-    for (int j = 0; j < S - 1; ++j) {
-        issue_rows(j);
-        issue_idx(j + S - 1);
+        for (int j = 0; j < S - 1; ++j) issue_idx(j);
+        wait_vmcnt<0>();
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < S - 1; ++j) {
+            issue_rows(j);
+            issue_idx(j + S - 1);
+        }
+        for (int k = 0; k < nsteps; ++k) {
+            // rows of step k and the map words of step k + S - 1 have landed
+            wait_vmcnt_in<(S - 2) * C::F_PER, (S - 2) * (C::F_PER + C::IDX_PER)>((S - 2) * step_loads);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();                      // ... everybody's; the stage of step k - 1 is free
+            asm volatile("" ::: "memory");
+            issue_rows(k + S - 1);
+            issue_idx(k + 2 * (S - 1));
+        }
+        wait_vmcnt<0>();
+        return;
     }
+
+    // The weight's fragments: lane l32 is a column, a piece its 8 consecutive K values.  Every load goes out before the first is waited for:
+    // what a lane has no value for it reads from an address that exists and drops.
+    i16x8 wf[G::KK];
+    {
+        const int col = c0 + l32, safe_col = col < cols ? col : 0;
+        const short b0 = bias != nullptr ? ((const short*)bias)[safe_col] : (short)0;
+#pragma unroll
+        for (int kk = 0; kk < G::KK; ++kk) {
+            const int at = kk * 2 + g, v = at / P, part = at - v * P, safe_v = v < V ? v : 0;
+            if (mode == 0) {
+                wf[kk] = *reinterpret_cast<const i16x8*>((const short*)weight + ((size_t)safe_col * V + safe_v) * (8 * P) + part * 8);
+            } else {
+                const int from = mode == 1 ? V - 1 - safe_v : safe_v;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) wf[kk][e] = ((const short*)weight)[((size_t)(part * 8 + e) * V + from) * cols + safe_col];
+            }
+        }
+#pragma unroll
+        for (int kk = 0; kk < G::KK; ++kk) {
+            const int at = kk * 2 + g, v = at / P;
+            const bool live = multiplies && col < cols;
+            if (!live || v >= V) wf[kk] = i16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            if (live && at == C::PIECES - 1) wf[kk][0] = b0;
+        }
+    }
+    __syncthreads();
     const int frag_row = rt * 32 + l32;
     for (int k = 0; k < nsteps; ++k) {
-        // rows of step k and the map words of step k + S - 1 have landed (stores count as well: the wait is only stricter)
-        wait_vmcnt<(S - 2) * G::LPS>();
         asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_s_barrier();                          // the loaders saw the rows of step k land
         asm volatile("" ::: "memory");
-        issue_rows(k + S - 1);
-        issue_idx(k + 2 * (S - 1));
         if (!multiplies) continue;
         const unsigned char* row_at = ring + (k % S) * C::F_BYTES + frag_row * C::ROWB;
         f32x16 acc;
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[e] = 0.f;
 #pragma unroll
-        for (int kk = 0; kk < G::KK; ++kk) {
-            const i16x8 rf = *reinterpret_cast<const i16x8*>(row_at + (((kk * 2 + g) ^ G::key(frag_row)) << 4));
-            mma16<Tag>(acc, wf[kk], rf);                       // [column][row]: a lane ends up with columns of one row
+        for (int k0 = 0; k0 < G::KK; k0 += G::AHEAD) {
+            // (a group's reads all out before its first product: left to itself the compiler keeps two of them in flight)
+            i16x8 rf[G::AHEAD];
+#pragma unroll
+            for (int kk = 0; kk < G::AHEAD; ++kk) rf[kk] = *reinterpret_cast<const i16x8*>(row_at + ((((k0 + kk) * 2 + g) ^ G::key(frag_row)) << 4));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int kk = 0; kk < G::AHEAD; ++kk) mma16<Tag>(acc, wf[k0 + kk], rf[kk]);     // [column][row]: a lane ends up with columns of one row
         }
-        // element e of lane l: column 8 * (e / 4) + 4 * (l / 32) + e % 4, row l % 32
-        const unsigned long long row = (unsigned long long)(lo + (unsigned)k) * C::ROWS + (unsigned)frag_row;
+        // Element e of lane l: column 8 * (e / 4) + 4 * (l / 32) + e % 4, row l % 32.  Two exchanges between lanes make that 16-byte pieces, four
+        // lanes a row: a store covers the 64 bytes of 16 rows.  (8 bytes a lane as they are: 16-byte writes at 110 G/s, 64 bytes each are a
+        // quarter as many.)
+        uint32_t w[4][2];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             using T4 = T __attribute__((ext_vector_type(4)));
             T4 four;
-            uint32_t bits = 0;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float x = acc[q * 4 + e];
                 four[e] = from_float<T>(relu ? __builtin_elementwise_maximum(x, 0.f) : x);
-                bits |= (uint32_t)((float)four[e] > 0.f) << e;
             }
-            const uint32_t high = (uint32_t)__shfl_xor((int)bits, 32, 64);
-            const int col = c0 + q * 8 + g * 4;
-            if (row >= n || col >= cols) continue;             // (cols is a multiple of 8)
-            *reinterpret_cast<T4*>(out + row * (unsigned)cols + col) = four;
-            if (relu_mask != nullptr && g == 0) relu_mask[(row * (unsigned)cols + col) >> 3] = (uint8_t)(bits | high << 4);
+            const uint64_t bits = __builtin_bit_cast(uint64_t, four);
+            w[q][0] = (uint32_t)bits;
+            w[q][1] = (uint32_t)(bits >> 32);
+        }
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            swap_halves(w[0][d], w[1][d]);                     // lanes 0 - 31: pieces 0 and 2, lanes 32 - 63: 1 and 3
+            swap_halves(w[2][d], w[3][d]);
+        }
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            swap_rows(w[0][d], w[2][d]);                       // rows 0 - 15 in the first piece, 16 - 31 in the second
+            swap_rows(w[1][d], w[3][d]);
+        }
+        const int col = c0 + (((lane >> 4) & 1) * 2 + g) * 8;
+        if (col >= cols) continue;                             // (cols is a multiple of 8)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            using T8 = T __attribute__((ext_vector_type(8)));
+            const unsigned long long row = (unsigned long long)(lo + (unsigned)k) * C::ROWS + (unsigned)(rt * 32 + h * 16 + (lane & 15));
+            if (row >= n) break;
+            const u32x4 piece = {w[2 * h][0], w[2 * h][1], w[2 * h + 1][0], w[2 * h + 1][1]};
+            *reinterpret_cast<u32x4*>(out + row * (unsigned)cols + col) = piece;
+            if (relu_mask != nullptr) {
+                const T8 x = __builtin_bit_cast(T8, piece);
+                uint32_t bits = 0;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) bits |= (uint32_t)((float)x[e] > 0.f) << e;
+                relu_mask[(row * (unsigned)cols + col) >> 3] = (uint8_t)bits;
+            }
         }
     }
-    wait_vmcnt<0>();
 }
 
 // Workgroups per 64 columns of grad_out: the chip full, and at least four steps each -- a partial product of 57 KB (Ci = 16: 115)
@@ -466,7 +594,7 @@ int stem_gemm_launch(int mode, const void* src, const void* weight, const void* 
     const unsigned steps = cdiv(n, C::ROWS), col_tiles = cdiv(cols, G::COLS);
     const unsigned most = col_tiles >= 256 ? 1 : 256 / col_tiles, groups = steps < most ? steps : most;
     const dim3 grid(cdiv(groups, kXcds) * kXcds, col_tiles);
-    kern<<<grid, kStemThreads, G::LDS, s>>>((const T*)src, (const T*)weight, (const T*)bias, map, (uint32_t)n, V, cols, mode, steps, groups, relu,
+    kern<<<grid, G::THREADS, G::LDS, s>>>((const T*)src, (const T*)weight, (const T*)bias, map, (uint32_t)n, V, cols, mode, steps, groups, relu,
                                             (T*)out, relu_mask);
     FGX_CHECK_LAUNCH("fgx_conv_gemm_stem");
     return FGX_OK;

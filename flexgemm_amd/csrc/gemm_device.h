@@ -1,7 +1,8 @@
-// Device-side pieces shared by the gather-GEMM kernels: vector types, the MFMA wrappers, conversions,
-// the vector-memory wait, and the LDS chunk swizzle.
+// Device-side pieces shared by the gather-GEMM kernels: vector types, the MFMA wrappers, conversions
+// and the LDS chunk swizzle.
 #pragma once
 #include "fgx_common.h"
+#include "vmem_wait.h"
 
 namespace fgx {
 namespace {
@@ -16,14 +17,6 @@ using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
 
 #define FGX_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 #define FGX_GLOBAL_PTR(p) ((const __attribute__((address_space(1))) void*)(p))
-
-// s_waitcnt with only the vector-memory counter constrained (gfx9 encoding: vmcnt = imm[3:0] | imm[15:14] << 4,
-// expcnt = imm[6:4], lgkmcnt = imm[11:8]; all-ones = unconstrained)
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
 
 struct F16 { using type = _Float16; };
 struct BF16 { using type = __bf16; };

@@ -5,6 +5,7 @@
 
 #include "fgx_common.h"
 #include "lds_read.h"
+#include "vmem_wait.h"
 
 namespace fgx {
 namespace {
@@ -40,12 +41,6 @@ constexpr int kItemListHeader = 4;
 #define FGX_LDS_PTR(p) ((__attribute__((address_space(3))) void*)(p))
 #define FGX_GLOBAL_PTR(p) ((const __attribute__((address_space(1))) void*)(p))
 #define FGX_CONST_PTR(p) ((const __attribute__((address_space(4))) uint32_t*)(uintptr_t)(p))      // words no launch in flight writes
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
 
 struct SegTable {
     uint32_t seg[kMaxV + 1];   // pair offsets per kernel offset
