@@ -339,7 +339,7 @@ __global__ void __launch_bounds__(1024) stem_reduce_kernel(const float* __restri
 // a quarter (8 channels) or half of a K-slab.  The wavefronts keep the weight in registers over the workgroup's run of rows; the
 // piece with the one multiplies the bias.  Rows are walked as they come, nothing of the mask sort is read.  Loaders and multipliers as in the
 // weight gradient; a step is bound by what follows its barrier in a multiplier, 14 reads of LDS, 14 products in a row, rounding and two stores.
-// 424 000 voxels, us: 6 -> 48 channels fp16 52 -> 35, bf16 64 -> 50; 16 -> 48 bf16 120 -> 78.
+// 424 000 voxels, us: 6 -> 48 channels fp16 52 -> 35, bf16 64 -> 34; 16 -> 48 bf16 120 -> 62.
 template <int P>
 struct StemGemmCfg {
     using W = StemCfg<P>;
@@ -644,15 +644,18 @@ int fgx_conv_wgrad_stem(int dtype, const void* grad_out, const void* feats, cons
                    : stem_launch<BF16, 2>(grad_out, feats, map, n, Co, V, (float*)scratch, grad_weight, grad_bias, s);
 }
 
-// Forward, ms (the tiled kernel, this one): 424 000 voxels 6 -> 48 channels 0.090 and 0.066; 143 616 voxels 8 -> 128 0.049 and 0.025, 16 ->
-// 128 0.050 and 0.038; 15 192 voxels 8 -> 64 0.019 and 0.008; 192 voxels 0.010 and 0.007; level at 624 264 voxels 16 -> 64.  An input gradient
-// fetches its fragments of the weight one value at a time: 3 us more per launch, and the streaming kernel keeps 16 channels of
-// many voxels up to 64 columns (143 616 voxels 0.040 and 0.047; 96 columns 0.052 and 0.048).  Forward, 16 channels, up to 32 columns (general
-// kernels, this one): 98 408 voxels 0.028 and 0.026, 427 872 0.085 and 0.087, 2 667 120 0.425 and 0.504.
+// Where it is ahead of the general kernels (us, scan order, bf16: general, this):
+//            forward                                                                       input gradient
+//   rows     8 -> 16    8 -> 64   16 -> 16  16 -> 64  16 -> 256       rows     8 -> 16  16 -> 16  16 -> 32  16 -> 64  16 -> 96  16 -> 256
+//       187  11.7  6.1  11.0  6.2  11.6  6.6  11.5  6.6  11.5  7.0        187  10.5  9.1  10.5 13.1           10.2 13.5            10.7 13.3
+//     3 758  12.7  6.2  14.3  6.2  13.1  6.6  14.0  6.6  20.4  6.8      2 047  12.5  9.6  10.4 13.3           11.7 13.8  12.5 13.3 16.9 13.8
+//    38 407  19.0  7.3  21.3  7.9  20.1  9.2  21.6  9.8  33.3 16.6      3 758  11.3  9.2  11.6 13.4           13.8 13.4  14.6 13.2 19.9 13.5
+//   428 946  76.2 29.9  86.5 32.9  83.3 50.1  92.9 52.5   203  108     15 467  13.4  9.3  13.7 13.9 15.5 14.0 19.0 14.3  26.6 14.3 33.9 16.9
+// 2 669 444   398  158   434  173   418  274   451  287  1130  694  2 669 444   389  164   416  288 417 291   428  304   571  320 1107  711
+// An input gradient fetches its fragments of the weight one value at a time, 3 us more per launch under 8 channels and 6 under 16.
 int fgx_conv_gemm_stem_pays(int dtype, int mode, size_t n, int K, int cols, int V) {
     if (mode < 0 || mode > 2 || !stem_gemm_takes(dtype, n, K, cols, V)) return 0;
-    if (mode == 0) return K == 8 || cols > 32 || n < 262144;
-    return K == 8 ? n >= 768 : n >= 3072 && cols >= 96;
+    return mode == 0 || K == 8 || n >= 16384 || (n >= 3072 && cols >= 64);
 }
 
 int fgx_conv_gemm_stem(int dtype, int mode, const void* src, const void* weight, const void* bias, const uint32_t* map, size_t n, int Ci, int Co,

@@ -62,14 +62,8 @@ template <> struct PositiveLimit<__bf16> { static constexpr uint32_t value = 0x7
 template <typename T> __device__ __forceinline__ T from_float(float x);
 template <> __device__ __forceinline__ _Float16 from_float<_Float16>(float x) { return (_Float16)x; }
 template <> __device__ __forceinline__ float from_float<float>(float x) { return x; }
-template <> __device__ __forceinline__ __bf16 from_float<__bf16>(float x) {
-    // round to nearest even; NaN stays NaN
-    uint32_t u = __builtin_bit_cast(uint32_t, x);
-    uint16_t h;
-    if ((u & 0x7FFFFFFFu) > 0x7F800000u) h = (uint16_t)((u >> 16) | 0x0040u);
-    else h = (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
-    return __builtin_bit_cast(__bf16, h);
-}
+// v_cvt_pk_bf16_f32: to nearest even, NaN stays NaN (bit for bit what shifts and adds give, over all 2^32 values; those took a branch per value)
+template <> __device__ __forceinline__ __bf16 from_float<__bf16>(float x) { return (__bf16)x; }
 template <typename T> __device__ __forceinline__ float to_float(T x) { return (float)x; }
 template <> __device__ __forceinline__ float to_float<__bf16>(__bf16 x) {
     return __builtin_bit_cast(float, (uint32_t)__builtin_bit_cast(uint16_t, x) << 16);

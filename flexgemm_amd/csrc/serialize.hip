@@ -196,15 +196,10 @@ __device__ __forceinline__ int4 coords_of(T spatial, T code, int bits) {
 
 // A thread per voxel of the z-order codes.  The Hilbert ones want their table in LDS (6 KB, read once per workgroup): no more
 // workgroups than the chip holds go over the voxels.
-template <int MODE>
 __device__ __forceinline__ void load_table(uint16_t* table, const CurveTable& from) {
-    if (MODE != kHilbert) return;
     for (int i = threadIdx.x; i < (int)(kTableBytes / 16); i += kBlock) ((uint4*)table)[i] = ((const uint4*)from.entry)[i];
     __syncthreads();
 }
-template <int MODE>
-constexpr int table_words() { return MODE == kHilbert ? kStateCount * kPairOctants : 8; }
-
 // Eight workgroups of four wavefronts fill a CU.  From a full chip on, three voxels a thread: three chains of dependent LDS reads side by
 // side.  5.3 M voxels in random order, 32-bit codes, us encode / decode: 27.6 / 25.9 bit by bit, 18.4 / 19.9 one voxel a thread, 18.0 / 18.2
 // three (5.9 TB/s), 18.4 / 18.0 four; 64-bit codes 30.0 / 28.9, 23.7 / 24.1, 21.6 / 21.6, 21.8 / 21.1; 100 000 voxels 3.0 / 2.8 and 2.5 / 2.6.
@@ -214,8 +209,15 @@ constexpr int kCurveVoxels = 3;
 template <typename T, int MODE, int U>
 __global__ void __launch_bounds__(kBlock) encode_kernel(const int32_t* __restrict__ coords, size_t n, int bits,
                                                         T* __restrict__ codes) {
-    __shared__ __attribute__((aligned(16))) uint16_t table[table_words<MODE>()];
-    load_table<MODE>(table, g_encode_table);
+    if constexpr (MODE == kZOrder) {
+        const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+        if (i >= n) return;
+        const int4 c = reinterpret_cast<const int4*>(coords)[i];
+        codes[i] = with_batch<T>(morton_of<T>(c, bits), c, bits);
+        return;
+    }
+    __shared__ __attribute__((aligned(16))) uint16_t table[kStateCount * kPairOctants];
+    load_table(table, g_encode_table);
     for (size_t base = (size_t)blockIdx.x * (kBlock * U); base < n; base += (size_t)gridDim.x * (kBlock * U)) {
         int4 c[U];
         T v[U];
@@ -226,7 +228,7 @@ __global__ void __launch_bounds__(kBlock) encode_kernel(const int32_t* __restric
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) v[u] = morton_of<T>(c[u], bits);
-        if (MODE == kHilbert) walk_curve<T, U>(table, v, bits);
+        walk_curve<T, U>(table, v, bits);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const size_t i = base + u * kBlock + threadIdx.x;
@@ -238,8 +240,15 @@ __global__ void __launch_bounds__(kBlock) encode_kernel(const int32_t* __restric
 template <typename T, int MODE, int U>
 __global__ void __launch_bounds__(kBlock) decode_kernel(const T* __restrict__ codes, size_t n, int bits,
                                                         int32_t* __restrict__ coords) {
-    __shared__ __attribute__((aligned(16))) uint16_t table[table_words<MODE>()];
-    load_table<MODE>(table, g_decode_table);
+    if constexpr (MODE == kZOrder) {
+        const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+        if (i >= n) return;
+        const T code = codes[i];
+        reinterpret_cast<int4*>(coords)[i] = coords_of<T>(code & spatial_mask<T>(bits), code, bits);
+        return;
+    }
+    __shared__ __attribute__((aligned(16))) uint16_t table[kStateCount * kPairOctants];
+    load_table(table, g_decode_table);
     for (size_t base = (size_t)blockIdx.x * (kBlock * U); base < n; base += (size_t)gridDim.x * (kBlock * U)) {
         T code[U], v[U];
 #pragma unroll
@@ -249,7 +258,7 @@ __global__ void __launch_bounds__(kBlock) decode_kernel(const T* __restrict__ co
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) v[u] = code[u] & spatial_mask<T>(bits);
-        if (MODE == kHilbert) walk_curve<T, U>(table, v, bits);
+        walk_curve<T, U>(table, v, bits);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const size_t i = base + u * kBlock + threadIdx.x;
