@@ -8,15 +8,16 @@
 // a plan names once per neighbor cache.  Per chunk the loaders put those rows into LDS (direct-to-LDS loads), together
 // with the chunk's table "which LDS slot holds the source of (row, offset)", and the multipliers run ALL offsets for
 // all rows -- a missing neighbor is the slot of zeros -- because with K = 32 a product is two MFMAs and skipping would
-// cost more instructions than it saves.  The weight (V x 2 KiB) stays in LDS for the whole launch.
+// cost more instructions than it saves.  The weight (V x 2 KiB) stays in registers (3 x 3 x 3 kernels, narrow27_multiply) or LDS (others) for the
+// whole launch.
 //
-// (the plan's layout: narrow_plan.h)
+// (the plan's layout: narrow_plan.h; the 3 x 3 x 3 kernels' walk: narrow_walk.h)
 //
-// Workgroup: 4 multiplying wavefronts (32 chunk rows each, one 32 x 32 accumulator) + 4 loading wavefronts; two LDS
+// Workgroup of the others: 4 multiplying wavefronts (32 chunk rows each, one 32 x 32 accumulator) + 4 loading wavefronts; two LDS
 // buffers (the loads run one chunk ahead), one barrier per chunk.  Persistent: XCD x walks the x-th eighth of the chunks, its workgroups interleave, so
 // that neighboring chunks -- which share their halo rows -- run on one L2 at one time.
 #include "gemm_device.h"
-#include "narrow_plan.h"
+#include "narrow_walk.h"
 
 namespace fgx {
 namespace {
@@ -205,16 +206,36 @@ template <> __device__ __forceinline__ uint64_t pack4<__bf16>(const float (&x)[4
     return __builtin_bit_cast(uint64_t, __builtin_convertvector(v, b4));
 }
 
-// VT: the kernel volume when it is known at compile time (the offsets' loop is then unrolled and the compiler runs the
-// LDS reads of later offsets under the MFMAs of earlier ones), 0: any V <= 32
+// The order of the offsets, and the sums their products go to: with VT 27 the centre first, by halves of K, then the offsets below it to the first sum and
+// those above it to the second; otherwise as they come, by halves of K.
+template <int VT>
+__device__ __forceinline__ constexpr int nth(int i) {
+    return VT == 0 ? i : (i == 0 ? VT / 2 : (i <= VT / 2 ? i - 1 : i));
+}
 template <typename Tag, int VT>
-__global__ void __launch_bounds__(kNarrowThreads)
-narrow_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Tag::type* __restrict__ panel,
-                   const typename Tag::type* __restrict__ bias, const uint32_t* __restrict__ nmap,
-                   const unsigned char* __restrict__ plan, uint32_t chunks, uint32_t plan_bytes, uint32_t src_bytes, int V,
-                   int K, int cols, int activation, typename Tag::type* __restrict__ out, uint8_t* __restrict__ relu_mask) {
+__device__ __forceinline__ void add_products(int v, f32x16& acc, f32x16& acc1, const u32x4& w0, const u32x4& w1, const u32x4& a0, const u32x4& a1) {
+    if (VT == 0 || v == VT / 2) {
+        mma<Tag>(acc, w0, a0);
+        mma<Tag>(acc1, w1, a1);
+    } else if (v < VT / 2) {
+        mma<Tag>(acc, w0, a0);
+        mma<Tag>(acc, w1, a1);
+    } else {
+        mma<Tag>(acc1, w0, a0);
+        mma<Tag>(acc1, w1, a1);
+    }
+}
+
+// Any kernel volume, any plan: kernel volumes other than 27 (VT 0), and plans of 27 offsets that have chunks of more distinct sources than
+// slots (VT 27: products in the order of narrow27_multiply, so that results do not depend on a plan's overflows).  By the first kNarrowThreads
+// threads of the workgroup.
+template <typename Tag, int VT>
+__device__ __forceinline__ void narrow_gemm_any(const typename Tag::type* __restrict__ src, const typename Tag::type* __restrict__ panel,
+                                                const typename Tag::type* __restrict__ bias, const uint32_t* __restrict__ nmap,
+                                                const unsigned char* __restrict__ plan, uint32_t chunks, uint32_t plan_bytes, uint32_t src_bytes, int V,
+                                                int K, int cols, int activation, typename Tag::type* __restrict__ out,
+                                                uint8_t* __restrict__ relu_mask, unsigned char* lds) {
     using T = typename Tag::type;
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     unsigned char* weight_lds = lds;                                            // [V][32][64 B], pieces exchanged by (col >> 2) & 3
     unsigned char* buffers = lds + (size_t)V * 2048;
     const int buffer_bytes = narrow_buffer_bytes(V);
@@ -341,7 +362,8 @@ narrow_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
             // (a table entry is the byte offset of a row's logical piece 0; piece q sits at entry ^ (q << 4))
             if (__builtin_expect(__any(entry(kNarrowTableStride - 1) != 0u), 0)) {
                 // a chunk with more distinct sources than slots: lanes whose source is not resident read it from memory
-                for (int v = 0; v < V; ++v) {
+                for (int i = 0; i < V; ++i) {
+                    const int v = nth<VT>(i);
                     const uint32_t s = table[r * kNarrowTableStride + v];
                     const uint32_t off = s == kNarrowOverflow ? kNarrowZeroSlot * 64u : s;
                     u32x4 a0 = *reinterpret_cast<const u32x4*>(buf + (off ^ ((uint32_t)g << 4)));
@@ -355,14 +377,13 @@ narrow_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
                             a1 = (g + 2) * 16 < row_bytes ? *reinterpret_cast<const u32x4*>(p + (g + 2) * 16) : zero;
                         }
                     }
-                    mma<Tag>(acc, *reinterpret_cast<const u32x4*>(wrow0 + v * 2048), a0);
-                    mma<Tag>(acc1, *reinterpret_cast<const u32x4*>(wrow1 + v * 2048), a1);
+                    add_products<Tag, VT>(v, acc, acc1, *reinterpret_cast<const u32x4*>(wrow0 + v * 2048), *reinterpret_cast<const u32x4*>(wrow1 + v * 2048), a0, a1);
                 }
             } else if constexpr (VT > 0) {
-                // The fragment reads run kAhead offsets ahead of the products (kAhead + 1 register sets): with one multiplying
+                // The fragment reads run kFetched offsets ahead of the products (kFetched + 1 register sets): with one multiplying
                 // wavefront per SIMD nothing else hides the LDS latency, and left to itself the compiler issues every
                 // read right before its use.
-                constexpr int kAhead = 2, kSets = kAhead + 1;        // (3, 4 and 6 ahead measure the same)
+                constexpr int kFetched = 2, kSets = kFetched + 1;    // (3, 4 and 6 ahead measure the same)
                 u32x4 fa0[kSets], fa1[kSets], fb0[kSets], fb1[kSets];
                 auto fetch = [&](int v, int set) __attribute__((always_inline)) {
                     const uint32_t at = entry(v) ^ ((uint32_t)g << 4);
@@ -372,13 +393,12 @@ narrow_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
                     fb1[set] = *reinterpret_cast<const u32x4*>(wrow1 + v * 2048);
                 };
 #pragma unroll
-                for (int v = 0; v < kAhead && v < VT; ++v) fetch(v, v % kSets);
+                for (int i = 0; i < kFetched && i < VT; ++i) fetch(nth<VT>(i), i % kSets);
 #pragma unroll
-                for (int v = 0; v < VT; ++v) {
-                    if (v + kAhead < VT) fetch(v + kAhead, (v + kAhead) % kSets);
+                for (int i = 0; i < VT; ++i) {
+                    if (i + kFetched < VT) fetch(nth<VT>(i + kFetched), (i + kFetched) % kSets);
                     __builtin_amdgcn_sched_barrier(0);
-                    mma<Tag>(acc, fb0[v % kSets], fa0[v % kSets]);
-                    mma<Tag>(acc1, fb1[v % kSets], fa1[v % kSets]);
+                    add_products<Tag, VT>(nth<VT>(i), acc, acc1, fb0[i % kSets], fb1[i % kSets], fa0[i % kSets], fa1[i % kSets]);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             } else {
@@ -421,6 +441,207 @@ narrow_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
 }
 
 template <typename Tag>
+__global__ void __launch_bounds__(kNarrowThreads)
+narrow_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Tag::type* __restrict__ panel,
+                   const typename Tag::type* __restrict__ bias, const uint32_t* __restrict__ nmap,
+                   const unsigned char* __restrict__ plan, uint32_t chunks, uint32_t plan_bytes, uint32_t src_bytes, int V,
+                   int K, int cols, int activation, typename Tag::type* __restrict__ out, uint8_t* __restrict__ relu_mask) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    narrow_gemm_any<Tag, 0>(src, panel, bias, nmap, plan, chunks, plan_bytes, src_bytes, V, K, cols, activation, out, relu_mask, lds);
+}
+
+// 3 x 3 x 3 kernels.  Eight multipliers: wavefront h * 4 + t has chunk rows t * 32 ... + 31 and the offsets below (h = 0) or above the
+// centre, whose product the two share by halves of K: 27 matrix instructions each.  The weight of a wavefront's offsets stays in
+// its registers for the launch.  The two sums of a row meet through LDS:
+// a wavefront hands over the sums of one half of its rows and finishes the other's, at the start of the next iteration, when the barrier
+// between the two has been met anyway; the 16 x 32 sums a wavefront finishes leave as one store of whole 64-byte rows.
+// 2 667 120 voxels, 32 channels: 0.182 ms -> 0.152 in scan order, 0.191 -> 0.160 in random order; 166 977 voxels 17.9 -> 15.9 us; 667 763 voxels, 16
+// channels 39.3 -> 35.9.  Loads and stores alone take 0.117 ms (582 MB at 5 TB/s, 219 of them the plan); what is left are the two multipliers of a
+// SIMD, which do not cover each other's waits altogether.  Leaving out the offsets that none of a tile's 32 rows has (7 of 27) costs in
+// branches what it saves in products; registers for a second offset's fragments ahead change nothing.
+constexpr int kAhead = 1;                                      // (offsets whose fragments are read ahead: registers for one)
+constexpr int kN27Half = 13;                                   // offsets on either side of the centre
+constexpr int kN27BufferBytes = kNarrowRowBufPad + kNarrowTableBytes;
+constexpr int kN27SumBytes = 16 * 32 * 4;                      // what a wavefront hands over
+constexpr size_t kN27LdsBytes = (size_t)kWalkBuffers * kN27BufferBytes + 2 * (size_t)kWalkMult * kN27SumBytes + (size_t)kWalkMetas * kWalkMetaBytes + 128 + 2048;
+static_assert(kN27LdsBytes <= 160 * 1024, "LDS");
+
+// rows of 32 x 32 sums in two halves: a's lanes 32 - 63 and b's lanes 0 - 31 change places; a's odd runs of 16 lanes and b's even ones
+__device__ __forceinline__ void swap_halves(float& a, float& b) {
+    const auto both = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+    a = __builtin_bit_cast(float, (uint32_t)both[0]);
+    b = __builtin_bit_cast(float, (uint32_t)both[1]);
+}
+__device__ __forceinline__ void swap_rows(float& a, float& b) {
+    const auto both = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+    a = __builtin_bit_cast(float, (uint32_t)both[0]);
+    b = __builtin_bit_cast(float, (uint32_t)both[1]);
+}
+
+// The offsets below the centre (HALF 0) or above it.
+template <typename Tag, int HALF>
+__device__ __forceinline__ void narrow27_multiply(const NarrowWalk& walk, int t, int lane, const unsigned char* panel, const unsigned char* buffers,
+                                                  unsigned char* handed, const unsigned char* meta, const float* bias_lds,
+                                                  const unsigned char* centre_lds, int cols, int activation, unsigned char* out, uint8_t* relu_mask) {
+    using T = typename Tag::type;
+    constexpr int CENTRE = kNarrowEvenV / 2;
+    const int out_row_bytes = cols * 2;
+    const int l32 = lane & 31, g = lane >> 5, r = t * 32 + l32;
+    const int piece = ((lane >> 4) & 1) * 2 + g;                               // of a finished row: columns 8 * piece ... + 7 of row lane % 16
+    constexpr int FIRST = HALF == 0 ? 0 : CENTRE + 1;
+    u32x4 wf[kN27Half][2];
+    {
+        const unsigned char* w = panel + l32 * 64 + g * 16;
+#pragma unroll
+        for (int i = 0; i < kN27Half; ++i) {
+            wf[i][0] = *reinterpret_cast<const u32x4*>(w + (FIRST + i) * 2048);
+            wf[i][1] = *reinterpret_cast<const u32x4*>(w + (FIRST + i) * 2048 + 32);
+        }
+    }
+    const unsigned char* centre_at = centre_lds + l32 * 64 + (((g + 2 * HALF) ^ ((l32 >> 2) & 3)) << 4);
+    unsigned char* mine_out = handed + (HALF * 4 + t) * kN27SumBytes + lane * 16;              // [2][64 lanes][16 bytes]
+    const unsigned char* other_in = handed + ((HALF ^ 1) * 4 + t) * kN27SumBytes + lane * 16;
+    float kept[8];
+    uint32_t kept_row = FGX_EMPTY32;
+    // the rows whose sums this wavefront finishes: 16 * HALF ... + 15 of its 32
+    auto finish = [&](int parity) __attribute__((always_inline)) {
+        const f32x4 o0 = *reinterpret_cast<const f32x4*>(other_in + parity * (kWalkMult * kN27SumBytes));
+        const f32x4 o1 = *reinterpret_cast<const f32x4*>(other_in + parity * (kWalkMult * kN27SumBytes) + 1024);
+        const f32x4 b0 = *reinterpret_cast<const f32x4*>(bias_lds + piece * 8), b1 = *reinterpret_cast<const f32x4*>(bias_lds + piece * 8 + 4);
+        float x[2][4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            // (offsets below the centre first, whoever adds)
+            x[0][e] = activate((HALF == 0 ? kept[e] + o0[e] : o0[e] + kept[e]) + b0[e], activation);
+            x[1][e] = activate((HALF == 0 ? kept[4 + e] + o1[e] : o1[e] + kept[4 + e]) + b1[e], activation);
+        }
+        if (kept_row == FGX_EMPTY32 || piece * 8 >= cols) return;
+        const uint64_t p0 = pack4<T>(x[0]), p1 = pack4<T>(x[1]);
+        const u32x4 out16 = {(uint32_t)p0, (uint32_t)(p0 >> 32), (uint32_t)p1, (uint32_t)(p1 >> 32)};
+        *reinterpret_cast<u32x4*>(out + (size_t)kept_row * out_row_bytes + piece * 16) = out16;
+        if (relu_mask != nullptr) {
+            uint32_t bits = 0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bits |= (x[0][e] > 0.f ? 1u : 0u) << e | (x[1][e] > 0.f ? 16u : 0u) << e;
+            relu_mask[((size_t)kept_row * out_row_bytes >> 4) + piece] = (uint8_t)bits;
+        }
+    };
+
+    walk_barrier();
+    walk_barrier();
+    for (unsigned i = 0; i < walk.count; ++i) {
+        if (i > 0) finish((int)(i & 1) ^ 1);
+        const unsigned char* buf = buffers + (i % kWalkBuffers) * kN27BufferBytes;
+        const unsigned char* table = buf + kNarrowRowBufPad;
+        const uint32_t* out_rows = (const uint32_t*)(meta + (i % kWalkMetas) * kWalkMetaBytes) + kNarrowSlots;
+        // entries: pieces 0 and 1, or 1, 2 and 3
+        u32x4 ent[2 + HALF];
+#pragma unroll
+        for (int q = 0; q < 2 + HALF; ++q) ent[q] = *reinterpret_cast<const u32x4*>(table + walk_table_at(r, HALF + q));
+        kept_row = out_rows[t * 32 + HALF * 16 + (lane & 15)];
+        auto entry = [&](int v) __attribute__((always_inline)) -> uint32_t {
+            const uint32_t word = ent[(v >> 3) - HALF][(v >> 1) & 3];
+            return (v & 1) ? word >> 16 : word & 0xFFFFu;
+        };
+        f32x16 acc;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+        // The fragments of kAhead offsets are read ahead of the products; the centre comes first.
+        u32x4 a0[kAhead + 1], a1[kAhead + 1];
+        auto fetch = [&](int j) __attribute__((always_inline)) {                 // 0: the centre (one half of K), j: the half's j-th offset
+            const uint32_t at = entry(j == 0 ? CENTRE : FIRST + j - 1) ^ ((uint32_t)(j == 0 ? g + 2 * HALF : g) << 4);
+            a0[j % (kAhead + 1)] = *reinterpret_cast<const u32x4*>(buf + at);
+            if (j == 0) a1[0] = *reinterpret_cast<const u32x4*>(centre_at);
+            else a1[j % (kAhead + 1)] = *reinterpret_cast<const u32x4*>(buf + (at ^ 32u));
+        };
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) fetch(j);
+#pragma unroll
+        for (int j = 0; j <= kN27Half; ++j) {
+            if (j + kAhead <= kN27Half) fetch(j + kAhead);
+            __builtin_amdgcn_sched_barrier(0);
+            if (j == 0) {
+                mma<Tag>(acc, a1[0], a0[0]);
+            } else {
+                mma<Tag>(acc, wf[j - 1][0], a0[j % (kAhead + 1)]);
+                mma<Tag>(acc, wf[j - 1][1], a1[j % (kAhead + 1)]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // element e of lane l: column 8 * (e / 4) + 4 * (l / 32) + e % 4 of row l % 32  ->  eight columns of row l % 16 and of row 16 + l % 16
+        float x[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) x[e] = acc[e];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            swap_halves(x[e], x[4 + e]);
+            swap_halves(x[8 + e], x[12 + e]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) swap_rows(x[e], x[8 + e]);
+        unsigned char* to = mine_out + (i & 1) * (kWalkMult * kN27SumBytes);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) kept[e] = x[HALF * 8 + e];
+        constexpr int GIVEN = 8 - HALF * 8;
+        *reinterpret_cast<f32x4*>(to) = f32x4{x[GIVEN], x[GIVEN + 1], x[GIVEN + 2], x[GIVEN + 3]};
+        *reinterpret_cast<f32x4*>(to + 1024) = f32x4{x[GIVEN + 4], x[GIVEN + 5], x[GIVEN + 6], x[GIVEN + 7]};
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                 // handed over; the buffers have been read
+        walk_barrier();
+    }
+    finish((int)(walk.count & 1) ^ 1);
+}
+
+template <typename Tag>
+__global__ void __launch_bounds__(kWalkThreads)
+narrow_gemm27_kernel(const typename Tag::type* __restrict__ src, const typename Tag::type* __restrict__ panel,
+                     const typename Tag::type* __restrict__ bias, const uint32_t* __restrict__ nmap, const unsigned char* __restrict__ plan,
+                     uint32_t chunks, uint32_t plan_bytes, uint32_t src_bytes, int K, int cols, int activation,
+                     typename Tag::type* __restrict__ out, uint8_t* __restrict__ relu_mask) {
+    using T = typename Tag::type;
+    constexpr int V = kNarrowEvenV;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    unsigned char* buffers = lds;
+    unsigned char* handed = lds + kWalkBuffers * kN27BufferBytes;              // [2][kWalkMult][kN27SumBytes]
+    unsigned char* meta = handed + 2 * kWalkMult * kN27SumBytes;
+    float* bias_lds = (float*)(meta + kWalkMetas * kWalkMetaBytes);            // [32]
+    unsigned char* centre_lds = (unsigned char*)(bias_lds + 32);               // the centre's weight (registers for it as well are not left): [32][64 bytes]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row_bytes = K * 2;
+    if (*reinterpret_cast<const uint32_t*>(plan) != 0u) {                      // chunks with sources that are not resident
+        if (tid < kNarrowThreads)
+            narrow_gemm_any<Tag, V>(src, panel, bias, nmap, plan, chunks, plan_bytes, src_bytes, V, K, cols, activation, out, relu_mask, lds);
+        return;
+    }
+    const NarrowWalk walk(chunks, kXcds);
+    if (walk.count == 0) return;                                               // whole workgroup
+    if (tid < 4 * kWalkBuffers) {                                              // the rows of zeros
+        const u32x4 zero = {0u, 0u, 0u, 0u};
+        *reinterpret_cast<u32x4*>(buffers + (tid >> 2) * kN27BufferBytes + kNarrowSlots * 64 + (tid & 3) * 16) = zero;
+    }
+    if (tid >= 64 && tid < 96) bias_lds[tid - 64] = bias != nullptr && tid - 64 < cols ? to_float<T>(bias[tid - 64]) : 0.f;
+    if (tid >= 128 && tid < 256) {
+        const int col = (tid - 128) >> 2, piece = tid & 3;
+        *reinterpret_cast<u32x4*>(centre_lds + col * 64 + ((piece ^ ((col >> 2) & 3)) << 4)) =
+            *reinterpret_cast<const u32x4*>((const unsigned char*)panel + (V / 2) * 2048 + col * 64 + piece * 16);
+    }
+    const rsrc_t src_rs = narrow_rsrc(src, src_bytes), plan_rs = narrow_rsrc(plan, plan_bytes);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                         // (met by the barriers of the walk)
+
+    if (wave >= kWalkMult) {
+        narrow_load_walk<false, true>(walk, wave - kWalkMult, lane, src_rs, row_bytes, src_rs, 0, plan_rs, buffers, kN27BufferBytes, kNarrowRowBufPad, meta);
+        return;
+    }
+
+    unsigned char* out_b = (unsigned char*)out;
+    const unsigned char* panel_b = (const unsigned char*)panel;
+    // (of two wavefronts on a SIMD the older one wins, and the younger would be late at every barrier: 2.67 M rows in random order 0.167 -> 0.160 ms)
+    if (wave >= 4) __builtin_amdgcn_s_setprio(1);
+    if (wave < 4) narrow27_multiply<Tag, 0>(walk, wave, lane, panel_b, buffers, handed, meta, bias_lds, centre_lds, cols, activation, out_b, relu_mask);
+    else narrow27_multiply<Tag, 1>(walk, wave - 4, lane, panel_b, buffers, handed, meta, bias_lds, centre_lds, cols, activation, out_b, relu_mask);
+}
+
+template <typename Tag>
 int launch_narrow(const void* src, const void* panel, const void* bias, const uint32_t* nmap, const void* plan, size_t n,
                   size_t n_src, int V, int K, int cols, int activation, void* out, uint8_t* relu_mask, hipStream_t s) {
     using T = typename Tag::type;
@@ -431,15 +652,21 @@ int launch_narrow(const void* src, const void* panel, const void* bias, const ui
     unsigned groups = (unsigned)(cus > 0 ? cus : 256);
     groups = groups / kXcds * kXcds;
     if (groups < (unsigned)kXcds) groups = kXcds;
-    auto kern = V == 27 ? narrow_gemm_kernel<Tag, 27> : narrow_gemm_kernel<Tag, 0>;
-    const size_t lds = narrow_lds_bytes(V);
     static thread_local bool raised = false;
     if (!raised) {
-        FGX_CHECK_HIP(hipFuncSetAttribute((const void*)narrow_gemm_kernel<Tag, 27>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-        FGX_CHECK_HIP(hipFuncSetAttribute((const void*)narrow_gemm_kernel<Tag, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        FGX_CHECK_HIP(hipFuncSetAttribute((const void*)narrow_gemm27_kernel<Tag>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+        FGX_CHECK_HIP(hipFuncSetAttribute((const void*)narrow_gemm_kernel<Tag>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         raised = true;
     }
-    kern<<<groups, kNarrowThreads, lds, s>>>((const T*)src, (const T*)panel, (const T*)bias, nmap, (const unsigned char*)plan, chunks,
+    if (V == kNarrowEvenV) {
+        narrow_gemm27_kernel<Tag><<<groups, kWalkThreads, kN27LdsBytes, s>>>(
+            (const T*)src, (const T*)panel, (const T*)bias, nmap, (const unsigned char*)plan, chunks,
+            (uint32_t)(kNarrowHeader + (size_t)chunks * kNarrowPlanStride), (uint32_t)(n_src * (size_t)K * 2), K, cols, activation, (T*)out, relu_mask);
+        FGX_CHECK_LAUNCH("fgx_conv_narrow_gemm");
+        return FGX_OK;
+    }
+    const size_t lds = narrow_lds_bytes(V);
+    narrow_gemm_kernel<Tag><<<groups, kNarrowThreads, lds, s>>>((const T*)src, (const T*)panel, (const T*)bias, nmap, (const unsigned char*)plan, chunks,
                                              (uint32_t)(kNarrowHeader + (size_t)chunks * kNarrowPlanStride), (uint32_t)(n_src * (size_t)K * 2), V, K,
                                              cols, activation, (T*)out, relu_mask);
     FGX_CHECK_LAUNCH("fgx_conv_narrow_gemm");
