@@ -65,9 +65,8 @@ __global__ void __launch_bounds__(256, VC ? 8 : 4) narrow_plan_kernel(const uint
         grow_of[r] = gr < n ? (order ? (uint32_t)order[gr] : gr) : FGX_EMPTY32;
     }
     // entries from V on: the row of zeros (entry 31, the row's overflow flag, is written at the end)
-    const int used = VC == kNarrowEvenV ? V + 3 : V;
-    for (int i = tid; i < kNarrowRows * (kNarrowTableStride - used); i += 256)
-        table_lds[i / (kNarrowTableStride - used) * kNarrowTableStride + used + i % (kNarrowTableStride - used)] = (uint16_t)(kNarrowZeroSlot * 64u);
+    for (int i = tid; i < kNarrowRows * (kNarrowTableStride - V); i += 256)
+        table_lds[i / (kNarrowTableStride - V) * kNarrowTableStride + V + i % (kNarrowTableStride - V)] = (uint16_t)(kNarrowZeroSlot * 64u);
     __syncthreads();
     const int entries = kNarrowRows * V;
     auto source_of = [&](int e) -> uint32_t {
@@ -160,8 +159,6 @@ __global__ void __launch_bounds__(256, VC ? 8 : 4) narrow_plan_kernel(const uint
         // what the multipliers read: the byte offset of the row's logical piece 0 in the row buffer
         if (out != (uint16_t)kNarrowOverflow) out = (uint16_t)(out * 64u + (((uint32_t)out >> 2) & 3u) * 16u);
         table_lds[(e / V) * kNarrowTableStride + (e % V)] = out;
-        // (the weight gradient's last multiplier takes offsets 7, 15 and 23 behind 24, 25 and 26: seven offsets each)
-        if (VC == kNarrowEvenV && e % V % 8 == 7) table_lds[(e / V) * kNarrowTableStride + kNarrowEvenV + e % V / 8] = out;
         if (out == (uint16_t)kNarrowOverflow) atomicOr(&row_flags[(e / V) >> 5], 1u << ((e / V) & 31));
     }
     __syncthreads();
@@ -484,7 +481,7 @@ __device__ __forceinline__ void narrow27_multiply(const NarrowWalk& walk, int t,
                                                   unsigned char* handed, const unsigned char* meta, const float* bias_lds,
                                                   const unsigned char* centre_lds, int cols, int activation, unsigned char* out, uint8_t* relu_mask) {
     using T = typename Tag::type;
-    constexpr int CENTRE = kNarrowEvenV / 2;
+    constexpr int CENTRE = kNarrowCubeV / 2;
     const int out_row_bytes = cols * 2;
     const int l32 = lane & 31, g = lane >> 5, r = t * 32 + l32;
     const int piece = ((lane >> 4) & 1) * 2 + g;                               // of a finished row: columns 8 * piece ... + 7 of row lane % 16
@@ -598,7 +595,7 @@ narrow_gemm27_kernel(const typename Tag::type* __restrict__ src, const typename 
                      uint32_t chunks, uint32_t plan_bytes, uint32_t src_bytes, int K, int cols, int activation,
                      typename Tag::type* __restrict__ out, uint8_t* __restrict__ relu_mask) {
     using T = typename Tag::type;
-    constexpr int V = kNarrowEvenV;
+    constexpr int V = kNarrowCubeV;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     unsigned char* buffers = lds;
     unsigned char* handed = lds + kWalkBuffers * kN27BufferBytes;              // [2][kWalkMult][kN27SumBytes]
@@ -658,7 +655,7 @@ int launch_narrow(const void* src, const void* panel, const void* bias, const ui
         FGX_CHECK_HIP(hipFuncSetAttribute((const void*)narrow_gemm_kernel<Tag>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         raised = true;
     }
-    if (V == kNarrowEvenV) {
+    if (V == kNarrowCubeV) {
         narrow_gemm27_kernel<Tag><<<groups, kWalkThreads, kN27LdsBytes, s>>>(
             (const T*)src, (const T*)panel, (const T*)bias, nmap, (const unsigned char*)plan, chunks,
             (uint32_t)(kNarrowHeader + (size_t)chunks * kNarrowPlanStride), (uint32_t)(n_src * (size_t)K * 2), K, cols, activation, (T*)out, relu_mask);
@@ -684,7 +681,7 @@ int make_narrow_plan(const uint32_t* map, const Order* order, size_t n, int V, i
     const unsigned chunks = (unsigned)((n + kNarrowRows - 1) / kNarrowRows);
     narrow_plan_header_kernel<<<1, 64, 0, s>>>((uint32_t*)plan);
     FGX_CHECK_LAUNCH("fgx_narrow_plan(header)");
-    auto kern = V == kNarrowEvenV ? narrow_plan_kernel<Order, kNarrowEvenV> : narrow_plan_kernel<Order, 0>;
+    auto kern = V == kNarrowCubeV ? narrow_plan_kernel<Order, kNarrowCubeV> : narrow_plan_kernel<Order, 0>;
     kern<<<chunks, 256, 0, s>>>(map, order, (uint32_t)n, V, same_rows ? 1 : 0, (unsigned char*)plan);
     FGX_CHECK_LAUNCH("fgx_narrow_plan");
     return FGX_OK;

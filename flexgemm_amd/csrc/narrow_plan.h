@@ -25,7 +25,7 @@ constexpr uint32_t kNarrowZeroSlot = kNarrowSlots;     // one more slot, all zer
 constexpr uint32_t kNarrowOverflow = 0xFFFFu;
 constexpr uint32_t kNarrowOob = 0xFF000000u;           // buffer offset no tensor reaches: the load returns zeros
 constexpr int kNarrowMaxV = 31;                        // (table entry 31 of a row is its overflow flag)
-constexpr int kNarrowEvenV = 27;                       // with so many offsets entries 27, 28 and 29 repeat 7, 15 and 23
+constexpr int kNarrowCubeV = 27;                       // 3 x 3 x 3 kernels have kernels of their own (narrow_walk.h)
 constexpr int kNarrowTableStride = 32;                 // table entries per row: a row's entries are four 16-byte reads
 constexpr int kNarrowHeader = 256;
 constexpr int kNarrowTableBytes = kNarrowRows * kNarrowTableStride * 2;                         // 8 KiB

@@ -10,11 +10,10 @@
 // does the gather: lane s of a 16-lane group names 4 channels of the row that the plan's table gives for (chunk row,
 // offset) and receives 4 rows' values of one channel.  A missing neighbor is the row of zeros.
 //
-// Workgroup: 4 multiplying wavefronts + 4 loading wavefronts, two LDS buffers, one barrier per chunk (as in the forward
-// kernel).  Multiplier w owns the offsets 8 w ... 8 w + 7 (their 32 x 32 accumulators stay in registers over all the
-// chunks of the workgroup; offsets from V on multiply zeros); of 27 offsets, whose LDS reads bound the kernel, the first three
-// leave their last one to the fourth, seven each with the column sums below (2.67 M voxels, 32 channels: 0.225 -> 0.196 ms).  It walks the chunk's 128 rows in eight k-steps of 16; the
-// grad_out fragment of a k-step is read once for the eight offsets.  At the end every workgroup writes its partial
+// Workgroup of kernel volumes other than 27: 4 multiplying wavefronts + 4 loading wavefronts, two LDS buffers, one barrier per chunk (as in the
+// forward kernel).  Multiplier w owns the offsets 8 w ... 8 w + 7 (their 32 x 32 accumulators stay in registers over all the
+// chunks of the workgroup; offsets from V on multiply zeros).  It walks the chunk's 128 rows in eight k-steps of 16; the
+// grad_out fragment of a k-step is read once for the eight offsets.  3 x 3 x 3 kernels: narrow_wgrad27_kernel.  At the end every workgroup writes its partial
 // products, and a second kernel adds them in workgroup order (fixed order: same bits on every run).
 // An infinity or NaN in grad_out times the row of zeros is NaN where the sum over the pairs has no term: a workgroup whose sums are not
 // all finite goes over its chunks again and adds such rows of grad_out pair by pair, until every sum is NaN (wgrad_device.h).  2.67 M
@@ -26,13 +25,13 @@
 // A plan with an overflowing chunk (more distinct sources than slots) is not for this kernel: the caller looks at the
 // plan's header and takes the block-major kernel then.
 #include "wgrad_device.h"
-#include "narrow_plan.h"
+#include "narrow_walk.h"
 
 namespace fgx {
 namespace {
 
 constexpr int kNwMult = 4, kNwLoad = 4, kNwThreads = 64 * (kNwMult + kNwLoad);
-constexpr int kNwTaps = 8;                                                       // offsets per multiplier (7 of 27: below)
+constexpr int kNwTaps = 8;                                                       // offsets per multiplier
 constexpr int kNwGoutBytes = kNarrowRows * 64;                                   // the chunk's grad_out rows
 constexpr int kNwBufferBytes = kNarrowRowBufPad + kNwGoutBytes + kNarrowTableBytes;
 constexpr size_t kNwLdsBytes = 2 * (size_t)kNwBufferBytes + 16;                  // ... and the word that asks for a second pass
@@ -40,13 +39,15 @@ constexpr int kNwSrcGroups = kNarrowSlots / 16 / kNwLoad;                       
 constexpr int kNwOutGroups = kNarrowRows / 16 / kNwLoad;                         // 2
 constexpr int kNwIds = kNwSrcGroups + kNwOutGroups;
 
-template <typename Tag, int TAPS>
+// Kernel volumes other than 27.
+template <typename Tag>
 __global__ void __launch_bounds__(kNwThreads)
 narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Tag::type* __restrict__ feats,
                     const unsigned char* __restrict__ plan, uint32_t chunks, uint32_t plan_bytes, uint32_t gout_bytes,
                     uint32_t feats_bytes, int V, int Ci, int Co, float* __restrict__ partial, float* __restrict__ bias_partial) {
     using T = typename Tag::type;
     using T4 = T __attribute__((ext_vector_type(4)));
+    constexpr int TAPS = kNwTaps;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     volatile uint32_t& again = *reinterpret_cast<volatile uint32_t*>(lds + 2 * kNwBufferBytes);       // some sum is not finite
     const int tid = threadIdx.x, lane = tid & 63;
@@ -156,7 +157,7 @@ narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename 
     auto entries_of = [&](const unsigned char* table, int r) __attribute__((always_inline)) -> u32x4 {
         return *reinterpret_cast<const u32x4*>((const uint16_t*)(table + r * (kNarrowTableStride * 2)) + mw * 8);
     };
-    auto offset_of = [&](int t) -> int { return TAPS == kNwTaps || mw < kNwMult - 1 || t < 3 ? mw * kNwTaps + t : (t < TAPS - 1 ? (t - 3) * kNwTaps + 7 : kNarrowMaxV); };
+    auto offset_of = [&](int t) -> int { return mw * kNwTaps + t; };
     // the last offset of the last multiplier, past every V: ones in place of whatever its table entry names
     static_assert(kNarrowMaxV < kNwMult * kNwTaps, "an offset is free for the column sums");
     const uint32_t bias_bits = bias_partial != nullptr && mw == kNwMult - 1 ? (std::is_same<Tag, F16>::value ? 0x3C003C00u : 0x3F803F80u) : 0u;
@@ -287,6 +288,202 @@ narrow_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename 
     }
 }
 
+// 3 x 3 x 3 kernels: seven multipliers of four offsets, the last one with three and the column sums, and four loaders (narrow_walk.h).  Four multipliers of
+// seven, one per SIMD, waited for every k-step's reads before its products: 2 667 120 voxels, 32 channels 0.207 ms -> 0.168 (in random order
+// 0.212 -> 0.182), 667 763 voxels, 16 channels 60 -> 46 us, 166 977 voxels, 32 channels 27.7 -> 24.3.  Eight multipliers of seven offsets, four for either
+// half of a chunk's rows, 0.180, and 32 us for the last.  The memory's share is 0.108 ms (561 MB, 219 of them the plan).
+constexpr int kNw27Mult = 7, kNw27Taps = 4, kNw27Threads = 64 * (kNw27Mult + kWalkLoad);
+constexpr size_t kNw27LdsBytes = (size_t)kWalkBuffers * kNwBufferBytes + (size_t)kWalkMetas * kWalkMetaBytes + 16;
+static_assert(kNw27LdsBytes <= 160 * 1024 && kNw27Mult * kNw27Taps == kNarrowCubeV + 1, "LDS; a place for the column sums");
+
+template <typename Tag>
+__global__ void __launch_bounds__(kNw27Threads)
+narrow_wgrad27_kernel(const typename Tag::type* __restrict__ gout, const typename Tag::type* __restrict__ feats,
+                      const unsigned char* __restrict__ plan, uint32_t chunks, uint32_t plan_bytes, uint32_t gout_bytes,
+                      uint32_t feats_bytes, int Ci, int Co, float* __restrict__ partial, float* __restrict__ bias_partial) {
+    using T = typename Tag::type;
+    using T4 = T __attribute__((ext_vector_type(4)));
+    constexpr int V = kNarrowCubeV, TAPS = kNw27Taps, STEPS = kNarrowRows / 16;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    unsigned char* meta = lds + kWalkBuffers * kNwBufferBytes;
+    volatile uint32_t& again = *reinterpret_cast<volatile uint32_t*>(meta + kWalkMetas * kWalkMetaBytes);       // some sum is not finite
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (tid == 0) again = 0u;
+    const NarrowWalk walk(chunks, kXcds);
+    if (tid < 4 * kWalkBuffers) {                                                // the rows of zeros
+        const u32x4 zero = {0u, 0u, 0u, 0u};
+        *reinterpret_cast<u32x4*>(lds + (size_t)(tid >> 2) * kNwBufferBytes + kNarrowSlots * 64 + (tid & 3) * 16) = zero;
+    }
+    const rsrc_t feats_rs = make_rsrc(feats, feats_bytes), gout_rs = make_rsrc(gout, gout_bytes), plan_rs = make_rsrc(plan, plan_bytes);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                           // (the zeros and the word: met by the first barrier)
+
+    if (wave >= kNw27Mult) {
+        for (int pass = 0; pass < 2; ++pass) {
+            if (walk.count > 0)
+                narrow_load_walk<true, false>(walk, wave - kNw27Mult, lane, feats_rs, Ci * 2, gout_rs, Co * 2, plan_rs, lds, kNwBufferBytes,
+                                              kNarrowRowBufPad + kNwGoutBytes, meta);
+            if (pass == 0) __syncthreads();
+            if (again == 0u) break;
+        }
+        return;
+    }
+
+    // (the lanes' part in a transposing read: narrow_wgrad_kernel)
+    const int s16 = lane & 15, mb = (lane >> 4) & 1, g = lane >> 5, q = s16 >> 2;
+    const int chan_byte = mb * 32 + (s16 & 3) * 8;
+    const uint32_t cpiece = (uint32_t)(chan_byte >> 4), cw = (uint32_t)(chan_byte & 15);
+    using Entries = uint32_t __attribute__((ext_vector_type(2)));                // of the wavefront's four offsets
+    auto entries_of = [&](const unsigned char* table, int r) __attribute__((always_inline)) -> Entries {
+        return *reinterpret_cast<const Entries*>(table + r * (kNarrowTableStride * 2) + wave * (TAPS * 2));
+    };
+    auto entry = [](const Entries& e, int t) -> uint32_t { return (t & 1) ? e[t >> 1] >> 16 : e[t >> 1] & 0xFFFFu; };
+    const bool sums = bias_partial != nullptr && wave == kNw27Mult - 1;          // the last place: ones instead of what its table entry names
+    const uint32_t ones = std::is_same<Tag, F16>::value ? 0x3C003C00u : 0x3F803F80u;
+    f32x16 acc[TAPS];
+#pragma unroll
+    for (int t = 0; t < TAPS; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
+
+    // A k-step's reads in two groups, grad_out and two offsets, and the other two: while one is multiplied the next is on its way.
+    auto lds_at = [](const unsigned char* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)p; };
+    const uint32_t g_lo = (uint32_t)((g * 8 + q) * 64) + ((cpiece ^ (uint32_t)((g * 2) & 3)) << 4) + cw;         // (row kk * 16 + g * 8 + q: piece key g * 2)
+    const uint32_t g_hi = (uint32_t)((g * 8 + q + 4) * 64) + ((cpiece ^ (uint32_t)((g * 2 + 1) & 3)) << 4) + cw;
+    if (walk.count > 0) {
+        walk_barrier();
+        walk_barrier();
+        for (unsigned i = 0; i < walk.count; ++i) {
+            const unsigned char* buf = lds + (i % kWalkBuffers) * kNwBufferBytes;
+            const unsigned char* table = buf + kNarrowRowBufPad + kNwGoutBytes;
+            const uint32_t g_at = lds_at(buf + kNarrowRowBufPad), row_at = lds_at(buf) + cw;
+            Entries lo[STEPS], hi[STEPS];
+#pragma unroll
+            for (int kk = 0; kk < STEPS; ++kk) {
+                lo[kk] = entries_of(table, kk * 16 + g * 8 + q);
+                hi[kk] = entries_of(table, kk * 16 + g * 8 + q + 4);
+            }
+            i16x4 gf[2][2], f[2][4];
+            auto issue = [&](int kk, int half) __attribute__((always_inline)) {
+                if (half == 0) {
+                    gf[kk & 1][0] = lds_read_tr16_at<0>(g_at + g_lo + (uint32_t)(kk * 16 * 64));
+                    gf[kk & 1][1] = lds_read_tr16_at<0>(g_at + g_hi + (uint32_t)(kk * 16 * 64));
+                }
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    f[half][2 * t] = lds_read_tr16_at<0>(row_at + (entry(lo[kk], half * 2 + t) ^ (cpiece << 4)));
+                    f[half][2 * t + 1] = lds_read_tr16_at<0>(row_at + (entry(hi[kk], half * 2 + t) ^ (cpiece << 4)));
+                }
+            };
+            issue(0, 0);
+            issue(0, 1);
+#pragma unroll
+            for (int kk = 0; kk < STEPS; ++kk) {
+                lds_wait_but<4>(f[0]);                                           // (everything but the other group)
+                asm volatile("" : "+v"(gf[kk & 1][0]), "+v"(gf[kk & 1][1]));
+                const i16x8 gg = __builtin_shufflevector(gf[kk & 1][0], gf[kk & 1][1], 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+                for (int t = 0; t < 2; ++t) mma16<Tag>(acc[t], gg, __builtin_shufflevector(f[0][2 * t], f[0][2 * t + 1], 0, 1, 2, 3, 4, 5, 6, 7));
+                if (kk + 1 < STEPS) {
+                    issue(kk + 1, 0);
+                    lds_wait_but<6>(f[1]);
+                } else {
+                    lds_wait_but<0>(f[1]);
+                }
+                i16x8 last = __builtin_shufflevector(f[1][2], f[1][3], 0, 1, 2, 3, 4, 5, 6, 7);
+                if (sums) last = __builtin_bit_cast(i16x8, u32x4{ones, ones, ones, ones});
+                mma16<Tag>(acc[2], gg, __builtin_shufflevector(f[1][0], f[1][1], 0, 1, 2, 3, 4, 5, 6, 7));
+                mma16<Tag>(acc[3], gg, last);
+                if (kk + 1 < STEPS) issue(kk + 1, 1);
+            }
+            walk_barrier();
+        }
+    }
+    // (whatever the second pass does: a column's sum has a term for every row)
+    if (sums && (lane & 31) == 0)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) bias_partial[blockIdx.x * 32 + (e >> 2) * 8 + g * 4 + (e & 3)] = acc[TAPS - 1][e];
+    bool finite = true;
+#pragma unroll
+    for (int t = 0; t < TAPS; ++t) finite = finite && (wave * TAPS + t >= V || all_finite(acc[t]));
+    if (__any(!finite) && lane == 0) again = 1u;
+    __syncthreads();                                                             // (the loaders' after their first pass)
+    if (again != 0u && walk.count > 0) {
+        // the chunks once more, rows of grad_out that are not finite apart
+#pragma unroll
+        for (int t = 0; t < TAPS; ++t)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
+        walk_barrier();
+        walk_barrier();
+        bool done = false;                                                       // every sum is NaN
+        for (unsigned i = 0; i < walk.count; ++i) {
+            const unsigned char* buf = lds + (i % kWalkBuffers) * kNwBufferBytes;
+            const unsigned char* gbuf = buf + kNarrowRowBufPad;
+            const unsigned char* table = gbuf + kNwGoutBytes;
+            const uint32_t g_at = lds_at(gbuf), row_at = lds_at(buf) + cw;
+#pragma unroll 1
+            for (int kk = 0; kk < STEPS && !done; ++kk) {
+                const Entries lo = entries_of(table, kk * 16 + g * 8 + q), hi = entries_of(table, kk * 16 + g * 8 + q + 4);
+                i16x4 f[4 + 2 * TAPS];
+                f[0] = lds_read_tr16_at<0>(g_at + g_lo + (uint32_t)(kk * 16 * 64));
+                f[1] = lds_read_tr16_at<0>(g_at + g_hi + (uint32_t)(kk * 16 * 64));
+                f[2] = f[3] = i16x4{0, 0, 0, 0};
+#pragma unroll
+                for (int t = 0; t < TAPS; ++t) {
+                    f[4 + 2 * t] = lds_read_tr16_at<0>(row_at + (entry(lo, t) ^ (cpiece << 4)));
+                    f[5 + 2 * t] = lds_read_tr16_at<0>(row_at + (entry(hi, t) ^ (cpiece << 4)));
+                }
+                lds_wait_all(f);
+                i16x8 gg = __builtin_shufflevector(f[0], f[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                uint32_t apart = nonfinite_rows<Tag>(gg);
+                if (apart) drop_rows(gg, apart, g);
+#pragma unroll
+                for (int t = 0; t < TAPS; ++t) {
+                    i16x8 ff = __builtin_shufflevector(f[4 + 2 * t], f[5 + 2 * t], 0, 1, 2, 3, 4, 5, 6, 7);
+                    if (apart) drop_rows(ff, apart, g);
+                    mma16<Tag>(acc[t], gg, ff);
+                }
+                while (apart) {
+                    const int r = kk * 16 + __ffs((int)apart) - 1;
+                    apart &= apart - 1u;
+                    T4 gv[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        gv[e] = *reinterpret_cast<const T4*>(gbuf + r * 64 + (((uint32_t)e ^ narrow_piece_key((uint32_t)r)) << 4) + g * 8);
+                    const Entries entries = entries_of(table, r);
+                    T x[TAPS];                                                   // (all reads in flight together; a missing neighbor's: zeros)
+#pragma unroll
+                    for (int t = 0; t < TAPS; ++t)
+                        x[t] = *reinterpret_cast<const T*>(buf + (entry(entries, t) ^ ((uint32_t)((lane & 31) >> 3) << 4)) + (lane & 7) * 2);
+#pragma unroll
+                    for (int t = 0; t < TAPS; ++t) {
+                        if (__builtin_amdgcn_readfirstlane((int)entry(entries, t)) >> 6 == (int)kNarrowZeroSlot) continue;
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) acc[t][e] += (float)gv[e >> 2][e & 3] * (float)x[t];
+                    }
+                }
+            }
+            bool nan = true;
+#pragma unroll
+            for (int t = 0; t < TAPS; ++t) nan = nan && (wave * TAPS + t >= V || all_nan(acc[t], lane, 0, Co, 0, Ci));
+            done = __all(nan);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            walk_barrier();
+        }
+    }
+    // partial[workgroup][v][co][ci] (32 x 32 per offset): accumulator element e of lane (l32, g) is co = (e >> 2) * 8 +
+    // g * 4 + (e & 3), ci = l32
+#pragma unroll
+    for (int t = 0; t < TAPS; ++t) {
+        const int v = wave * TAPS + t;
+        if (v >= V) continue;
+        float* dst = partial + ((size_t)blockIdx.x * V + v) * 1024;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) dst[((e >> 2) * 8 + g * 4 + (e & 3)) * 32 + (lane & 31)] = acc[t][e];
+    }
+}
+
 // grad_weight[co][v][ci] = sum over the workgroups' partial products.  A workgroup owns 64 consecutive elements of the
 // padded (v, co, ci) tiles; four groups of 64 threads each add a quarter of the partial products in ascending order
 // (eight loads in flight), and the four sums are added in ascending order: a fixed order, whatever the timing.
@@ -353,17 +550,21 @@ int launch_narrow_wgrad(const void* gout, const void* feats, const void* plan, s
     int rc = narrow_wgrad_groups(&groups);
     if (rc != FGX_OK) return rc;
     const uint32_t chunks = (uint32_t)((n + kNarrowRows - 1) / kNarrowRows);
-    auto kern = V == kNarrowEvenV ? narrow_wgrad_kernel<Tag, 7> : narrow_wgrad_kernel<Tag, kNwTaps>;
     float* bias_partial = gb ? (float*)scratch + (size_t)groups * V * 1024 : nullptr;
-    static thread_local bool raised[2] = {false, false};
-    if (!raised[V == kNarrowEvenV]) {
-        FGX_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kNwLdsBytes));
-        raised[V == kNarrowEvenV] = true;
+    static thread_local bool raised = false;
+    if (!raised) {
+        FGX_CHECK_HIP(hipFuncSetAttribute((const void*)narrow_wgrad27_kernel<Tag>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kNw27LdsBytes));
+        FGX_CHECK_HIP(hipFuncSetAttribute((const void*)narrow_wgrad_kernel<Tag>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kNwLdsBytes));
+        raised = true;
     }
-    kern<<<groups, kNwThreads, kNwLdsBytes, s>>>((const T*)gout, (const T*)feats, (const unsigned char*)plan, chunks,
-                                                 (uint32_t)(kNarrowHeader + (size_t)chunks * kNarrowPlanStride),
-                                                 (uint32_t)(n * (size_t)Co * 2), (uint32_t)(n_src * (size_t)Ci * 2), V, Ci, Co,
-                                                 (float*)scratch, bias_partial);
+    const uint32_t plan_bytes = (uint32_t)(kNarrowHeader + (size_t)chunks * kNarrowPlanStride);
+    const uint32_t gout_bytes = (uint32_t)(n * (size_t)Co * 2), feats_bytes = (uint32_t)(n_src * (size_t)Ci * 2);
+    if (V == kNarrowCubeV)
+        narrow_wgrad27_kernel<Tag><<<groups, kNw27Threads, kNw27LdsBytes, s>>>((const T*)gout, (const T*)feats, (const unsigned char*)plan, chunks, plan_bytes,
+                                                                             gout_bytes, feats_bytes, Ci, Co, (float*)scratch, bias_partial);
+    else
+        narrow_wgrad_kernel<Tag><<<groups, kNwThreads, kNwLdsBytes, s>>>((const T*)gout, (const T*)feats, (const unsigned char*)plan, chunks, plan_bytes,
+                                                                         gout_bytes, feats_bytes, V, Ci, Co, (float*)scratch, bias_partial);
     FGX_CHECK_LAUNCH("fgx_conv_narrow_wgrad");
     narrow_wgrad_reduce_kernel<T><<<(unsigned)V * 16 + (gb ? 1u : 0u), 256, 0, s>>>((const float*)scratch, groups, V, Ci, Co, (T*)gw, bias_partial, (T*)gb);
     FGX_CHECK_LAUNCH("fgx_conv_narrow_wgrad(reduce)");
