@@ -165,6 +165,10 @@ __device__ __forceinline__ void scan_counts(const uint32_t* __restrict__ plan, i
     }
 }
 
+// Bytes of a row that a step multiplies, and workgroups on a CU, by the size of the type (see the kernel).
+constexpr int pair_slab(int es) { return es == 4 ? 64 : 128; }
+constexpr int pair_groups(int es) { return es == 4 ? 4 : 2; }
+
 // Where the weight is read from: as in the tiled gather GEMM, lines of one (offset, K-slab).
 //   TR = false: a line is an output column, its K values side by side;  TR = true: a line is a K value, its columns side by side.
 struct PairWeight {
@@ -176,31 +180,36 @@ struct PairWeight {
 template <typename Tag, bool TR, int BN_, int WAVES_M>
 struct PairCfg {
     using T = typename Tag::type;
-    static constexpr int ES = (int)sizeof(T), CH = 8, SLAB = 128, SK = SLAB / ES;
+    static constexpr int ES = (int)sizeof(T), SLAB = pair_slab(ES), CH = SLAB / 16, SK = SLAB / ES, RPL = 64 / CH;     // (RPL: rows a wave-wide load covers)
     static constexpr int BM = kPairRows, BN = BN_, NW = 4, NT = 256, WAVES_N = NW / WAVES_M;
     static constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N, TM = WM / 32, TN = WN / 32;
-    static constexpr int A_PER = BM / 8 / NW;                       // a wave-wide load covers 8 rows of 128 bytes
+    static constexpr int A_PER = BM / RPL / NW;
     static constexpr int LCOLS = BN == 96 ? 128 : BN;               // columns of a transposed line in LDS: whole loads of whole lines
     static constexpr int TCH = LCOLS * ES / 16, LINES = 64 / TCH;   // 16-byte pieces of a transposed line, lines a load covers
-    static constexpr int B_PER = TR ? SK / LINES / NW : BN / 8 / NW;
+    static constexpr int B_PER = TR ? SK / LINES / NW : (BN / RPL + NW - 1) / NW;
+    static constexpr int BROWS = TR ? LCOLS : B_PER * NW * RPL;     // (whole loads on every wavefront: of 96 columns' fp32 the last fetch nothing)
     static constexpr int LPS = A_PER + B_PER;
-    static constexpr int STAGE = (BM + (TR ? LCOLS : BN)) * SLAB, S = 2;
+    static constexpr int STAGE = (BM + BROWS) * SLAB, S = 2;
     static constexpr int tr_key(int line) { return ES != 2 ? 0 : (TCH >= 16 ? 4 * (line & 3) : 2 * (line & 3)); }   // 4 lines of a transposing read, 4 bank groups
-    static constexpr int PITCH = WN * 4 + 16;                       // epilogue band of a wavefront: 32 rows of WN sums
+    static constexpr int PITCH = 32 * 4 + 16;                       // epilogue band of a wavefront: 32 rows of 32 sums
     static constexpr size_t lds_bytes = S * STAGE;
     static_assert(NW * 32 * PITCH <= S * STAGE, "the epilogue bands lie in the ring");
-    static_assert(2 * lds_bytes <= 160 * 1024, "two workgroups share a CU: one multiplies while the other waits for LDS");
+    static_assert(pair_groups(ES) * lds_bytes <= 160 * 1024, "workgroups that share a CU: one multiplies while the others wait for loads");
 };
 
-// One tile of 128 pairs x 128 columns per workgroup, four wavefronts of 64 x 64, K in slabs of 128 bytes through two stages: a
+// One tile of 128 pairs x 128 columns (fp32: 96 or 64) per workgroup, four wavefronts of 64 x 64, K in slabs of 128 bytes through two stages: a
 // stage's fragments are taken into registers, the loads two slabs on go out into it, and the products run meanwhile.  Two
 // workgroups per CU cover each other's barriers.  XCD x takes the x-th eighth of the (column tile, row tile) list, so a part of
 // the weight -- the larger operand here -- crosses to one XCD only.
 // 864 voxels x 1024 channels (11 022 pairs, 57 MB of weight) 44 us, 513 TFLOP/s; 3 758 voxels 146 us, 695 TFLOP/s.  Tiles of 128 x 256 and 256 x 128 on
 // eight wavefronts, rings of three to five slabs, slabs of 64 bytes, and loads by wavefronts of their own in a persistent workgroup came out between
 // 0.9 and 1.2 of that time, ahead only for the second, behind for everything smaller.
+// fp32 multiplies a sixteenth as fast: half as long a slab is enough work for a barrier, and its stages and fragments let four workgroups share a
+// CU, which cover the few slabs' start and end (96 channels have three of 128 bytes).  Products and sums, two workgroups of 128-byte slabs -> four of 64:
+// 38 407 voxels, 96 channels 141 -> 130 us, and 125 with the sums leaving in bands of 32 columns, which no longer set the LDS a workgroup takes;
+// 8 589 voxels 42 -> 38; 15 467 voxels, 64 channels 38.8 -> 35.3; 3 758 voxels, 512 channels 245 -> 240.
 template <typename Tag, bool TR, int BN, int WAVES_M>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, pair_groups((int)sizeof(typename Tag::type)))
 pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const uint32_t* __restrict__ plan, uint32_t n, int K, int cols,
                  int V, uint32_t src_bytes, float* __restrict__ partial) {
     using C = PairCfg<Tag, TR, BN, WAVES_M>;
@@ -233,8 +242,8 @@ pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const
     uint32_t a_off[C::A_PER], a_at[C::A_PER], b_off[C::B_PER], b_at[C::B_PER];      // ..._at: byte (TR: K value) inside the slab
 #pragma unroll
     for (int i = 0; i < C::A_PER; ++i) {
-        const uint32_t r = (uint32_t)((i * C::NW + wave) * 8 + lane / 8);
-        a_at[i] = (uint32_t)(((lane & 7) ^ swz_key<CH>((int)r)) << 4);
+        const uint32_t r = (uint32_t)((i * C::NW + wave) * C::RPL + lane / CH);
+        a_at[i] = (uint32_t)(((lane & (CH - 1)) ^ swz_key<CH>((int)r)) << 4);
         a_off[i] = r < live ? rows[r] * row_bytes + a_at[i] : kOobOffset;
     }
     const int wv = b.mirrored ? V - 1 - v : v;
@@ -246,9 +255,9 @@ pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const
             b_at[i] = (uint32_t)line;
             b_off[i] = piece * (16 / C::ES) < BN && col0 + piece * (16 / C::ES) < cols ? (uint32_t)line * b.line_stride + (uint32_t)(col0 * C::ES + (piece << 4)) : kOobOffset;
         } else {
-            const int col = (i * C::NW + wave) * 8 + lane / 8;
-            b_at[i] = (uint32_t)(((lane & 7) ^ swz_key<CH>(col)) << 4);
-            b_off[i] = col0 + col < cols ? (uint32_t)(col0 + col) * b.line_stride + b_at[i] : kOobOffset;
+            const int col = (i * C::NW + wave) * C::RPL + lane / CH;
+            b_at[i] = (uint32_t)(((lane & (CH - 1)) ^ swz_key<CH>(col)) << 4);
+            b_off[i] = col < BN && col0 + col < cols ? (uint32_t)(col0 + col) * b.line_stride + b_at[i] : kOobOffset;
         }
     }
     uint32_t b_soff = (uint32_t)wv * b.v_stride;
@@ -351,25 +360,26 @@ pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const
     __builtin_amdgcn_s_barrier();           // the ring is reused below
     asm volatile("" ::: "memory");
 
-    // element e of lane l: pair l % 32, column 8 * (e / 4) + 4 * (l / 32) + e % 4.  Through the wavefront's band in LDS, out as 16-byte
-    // pieces of 256 bytes a pair.
+    // element e of lane l: pair l % 32, column 8 * (e / 4) + 4 * (l / 32) + e % 4.  Through the wavefront's band in LDS, 32 columns at a time, out as
+    // 16-byte pieces of 128 bytes a pair.
     unsigned char* band = ring + wave * 32 * C::PITCH;
-    constexpr int QUADS = C::WN / 4;            // 16-byte pieces of a band row
+    constexpr int QUADS = 8;            // 16-byte pieces of a band row
 #pragma unroll
     for (int i = 0; i < C::TM; ++i) {
 #pragma unroll
-        for (int j = 0; j < C::TN; ++j)
+        for (int j = 0; j < C::TN; ++j) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const f32x4 four = {acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
-                *(f32x4*)(band + l32 * C::PITCH + (j * 32 + q * 8 + g * 4) * 4) = four;
+                *(f32x4*)(band + l32 * C::PITCH + (q * 8 + g * 4) * 4) = four;
             }
-        // (written and read by the same wavefront: program order suffices)
+            // (written and read by the same wavefront: program order suffices)
 #pragma unroll
-        for (int pass = 0; pass < 32 * QUADS / 64; ++pass) {
-            const int r = (pass * 64 + lane) / QUADS, quad = (pass * 64 + lane) % QUADS, col = col0 + wave_n * C::WN + quad * 4;
-            const uint32_t row = (uint32_t)(wave_m * C::WM + i * 32 + r);
-            if (row < live && col < cols) *(f32x4*)(partial + (pair0 + row) * cols + col) = *(const f32x4*)(band + r * C::PITCH + quad * 16);
+            for (int pass = 0; pass < 32 * QUADS / 64; ++pass) {
+                const int r = (pass * 64 + lane) / QUADS, quad = (pass * 64 + lane) % QUADS, col = col0 + wave_n * C::WN + j * 32 + quad * 4;
+                const uint32_t row = (uint32_t)(wave_m * C::WM + i * 32 + r);
+                if (row < live && col < cols) *(f32x4*)(partial + (pair0 + row) * cols + col) = *(const f32x4*)(band + r * C::PITCH + quad * 16);
+            }
         }
     }
 }
@@ -449,7 +459,8 @@ int launch_pairs(const void* src, const PairWeight& b, const void* bias, const u
                  float* partial, int act, void* out, uint8_t* relu_mask, hipStream_t s) {
     using T = typename Tag::type;
     // Columns of a tile.  fp32 is bound by what it multiplies: 96 where that pads less, else 64, whose smaller pieces even out better (96
-    // channels, 38 407 voxels 0.140 ms, 64 columns 0.165; 512 channels, 3 758 voxels 0.244, 128 columns 0.260).  16-bit types load half as much per product
+    // channels, 38 407 voxels 0.126 ms, 64 columns 0.148; 512 channels, 3 758 voxels 0.240, 128 columns 0.245; 1024 channels, 864 voxels 0.241 and 0.257;
+    // 256 channels, 15 467 voxels 0.273 and 0.262).  16-bit types load half as much per product
     // with 128: those unless they pad by a sixth or leave CUs without a tile (864 voxels: 256 channels 64 columns 16.4 us, 128 16.8; 288 channels
     // 18.1 and 19.3; 512 channels 24.5 and 22.9; 3 758 voxels, 1024 channels 217 and 177).
     int rc;
@@ -562,7 +573,7 @@ int fgx_conv_gemm_pairs(int dtype, int mode, const void* src, const void* weight
     b.bytes = (uint32_t)weight_bytes;
     b.v_stride = (uint32_t)(Ci * es);
     b.line_stride = (uint32_t)((size_t)V * Ci * es);
-    b.slab_stride = mode == 0 ? 128u : (uint32_t)(128 / es) * b.line_stride;
+    b.slab_stride = mode == 0 ? (uint32_t)pair_slab(es) : (uint32_t)(pair_slab(es) / es) * b.line_stride;
     b.mirrored = mode == 1;
     hipStream_t s = (hipStream_t)stream;
 #define FGX_PAIRS(Tag)                                                                                                                              \
