@@ -501,25 +501,31 @@ extern "C" {
 //   1024 x  128      33  18   35  22   48  30   73  34   74  45              1024 x 2048   447 379   809 480   814 542   829 609
 // 64 columns (256 x 64: 15 12, 20 14, 24 19, 33 20, 34 21) gain little more than the plan: a training step whose input gradient still wants the
 // masks is up to 5 % slower for it, a pass at inference 1.16 to 1.44 times as fast.
-// fp32 multiplies a sixteenth as fast and what is not multiplied counts for more: from 64 channels and up to 45 000 rows, as long as the sums,
+// fp32 multiplies a sixteenth as fast and what is not multiplied counts for more: from 64 channels and up to 65 536 rows (98 304 under at most half
+// as many columns as channels; 64 channels 45 000, which tests pin: 48 203 rows, training with the cache 381 294), as long as the sums,
 // with 0.45 of a row's offsets, stay below 5 MB a channel.  Their traffic, which outgrows the 256 MB memory-side cache, costs what the products
-// save from 3.5 MB on, and by 5 MB also the 30 to 50 us of tables that a fresh cache is spared (64 x 256, cache and one layer, 27 200 rows: forward
-// 248 230, training 552 543;  38 400 rows: 354 325, 765 750;  24 400 rows, training 500 536).
-//   K x columns    864 rows   8 589    15 467    24 365    38 407    44 759      up to
-//     64 x   64      15  13    37  30    53  41    68  58    91  82   102  97      45 000 rows
-//     64 x  256      23  18    97  70   116 123   191 209   262 332   260 388      25 720
-//     96 x   96      22  16    67  44   109  67   159  94   158 142                45 000
-//     96 x  192      27  19   105  69   153 110   221 175   259 297   315 337      45 000
-//    128 x  256      33  24   168 101   216 178   364 275   499 440   488 512      38 836 (the sums' bound)
-//    128 x  512      52  36   303 187   356 351   543 558   830 884   759 1026     19 418 (the same)
-//    256 x  256      54  33   335 162   417 278   711 432   972 684                38 836 (the same)
+// save from 4.5 MB on, and by 5 MB also the 30 to 50 us of tables that a fresh cache is spared (64 x 256, cache and one layer, 27 200 rows: forward
+// 248 230, training 552 543;  38 400 rows: 354 325, 765 750;  24 400 rows, training 500 459).  Beyond: 96 x 96, 71 359 rows 244 250,
+// 84 634 rows 250 297;  128 x 128 438 378, 451 453;  160 x 160 595 617, 732 739;  256 x 96, 99 042 rows 857 631.
+//   K x columns    855 rows   8 589    15 474    24 372    38 323    48 203    63 137      up to
+//     64 x   64      16  13    38  29    54  38    67  55    89  75   111  87   111 112      45 000 rows
+//     64 x  256      23  17    96  66   116 108   192 178   259                               25 720 (the sums' bound)
+//     96 x   96      21  15    66  39   108  62   158  87   157 126   260 158   244 217      65 536
+//     96 x  192      27  18   104  64   151 101   217 153   260 263   356 330   365          51 440 (the sums' bound)
+//    128 x  256      32  22   165  93   216 156   367 254   493 407   492                    38 836 (1 GiB)
+//    128 x  512      52  33   302 179   354 324   541       824                              19 418 (the same)
+//    256 x  128      32  20   193  84   317 136   412 209   618 328   639 416   720 544      77 672 (the same)
+//    256 x  256      52  30   331 151   417 264   715 414   962 658   953                    38 836 (the same)
 // The sums at most 1 GiB at their bound.
 int fgx_conv_gemm_pairs_pays(int dtype, int mode, size_t n, int Ci, int Co, int V) {
     if (mode < 0 || mode > 2 || V < 1 || V > kPairMaxV || Ci <= 0 || Co <= 0 || n == 0) return 0;
     const int es = dtype == FGX_F32 ? 4 : 2, K = mode == 0 ? Ci : Co, cols = mode == 0 ? Co : Ci;
     if (Ci % (16 / es) != 0 || Co % (16 / es) != 0 || (size_t)V * Ci * Co * es >= ((size_t)1 << 31)) return 0;
-    if (n > 65536 || fgx_conv_gemm_pairs_scratch_bytes(n, cols, V) > ((size_t)1 << 30)) return 0;
-    if (es == 4) return K >= 64 && n <= 45000 && 0.45 * (double)fgx_conv_gemm_pairs_scratch_bytes(n, cols, V) <= 5e6 * K;
+    if (n > 98304 || fgx_conv_gemm_pairs_scratch_bytes(n, cols, V) > ((size_t)1 << 30)) return 0;
+    if (es == 4) {
+        const size_t rows = K == 64 ? 45000 : cols * 2 <= K ? 98304 : 65536;
+        return K >= 64 && n <= rows && 0.45 * (double)fgx_conv_gemm_pairs_scratch_bytes(n, cols, V) <= 5e6 * K;
+    }
     return K >= 256 && cols >= 64 && cols <= 2 * K && n <= (cols <= K ? 6000u : 5000u);
 }
 

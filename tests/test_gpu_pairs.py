@@ -133,3 +133,35 @@ def test_rows_up_to_which_it_is_taken(dtype, k, cols, rows):
         takes = [bool(nat.lib().fgx_conv_gemm_pairs_pays(C.c_int(nat.DTYPE_CODE[dtype]), C.c_int(mode), nat.sz(n), C.c_int(ci), C.c_int(co), C.c_int(27)))
                  for n in (1, rows, rows + 1)]
         assert takes == [rows > 0, rows > 0, False]
+
+
+# fp32 of more than 64 channels: up to 65 536 rows, 98 304 under at most half as many columns; the sums' bounds
+@pytest.mark.parametrize("k,cols,v,rows", [(68, 68, 27, 65536), (96, 96, 27, 65536), (128, 64, 27, 98304), (128, 68, 27, 65536), (256, 128, 27, 77672), (256, 128, 8, 98304),
+                                           (96, 192, 27, 51440)])
+def test_rows_up_to_which_fp32_takes_it(k, cols, v, rows):
+    for mode in (0, 1, 2):
+        ci, co = (k, cols) if mode == 0 else (cols, k)
+        takes = [bool(nat.lib().fgx_conv_gemm_pairs_pays(C.c_int(nat.DTYPE_CODE[torch.float32]), C.c_int(mode), nat.sz(n), C.c_int(ci), C.c_int(co), C.c_int(v)))
+                 for n in (1, 45001, rows, rows + 1)]
+        assert takes == [True, True, True, False]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ci,co,res", [(72, 72, 110), (128, 64, 156)])
+def test_fp32_agrees_with_the_masked_kernels_at_many_rows(gpu_device, monkeypatch, ci, co, res):
+    gen = torch.Generator(device=gpu_device).manual_seed(res)
+    coords = torch.from_numpy(reference_test_shell(res)).to(gpu_device)
+    n = coords.shape[0]
+    print(f"[case] {n} rows {ci}->{co}", flush=True)
+    shape = torch.Size([1, ci, res, res, res])
+    weight = torch.randn(co, 3, 3, 3, ci, generator=gen, device=gpu_device) / (27 * ci) ** 0.5
+    feats = torch.randn(n, ci, generator=gen, device=gpu_device)
+    with torch.no_grad():
+        out, cache = spconv.sparse_submanifold_conv3d(feats, coords, shape, weight, None, None)
+        assert n > 45000 and "_pair_plan" in cache.__dict__
+        real = nat.table_lookup
+        monkeypatch.setattr(nat, "table_lookup", lambda *a, **k: real(*a, **k))         # (a table of the caller's keeps every shape on it)
+        want, other = spconv.sparse_submanifold_conv3d(feats, coords, shape, weight, None, None)
+    assert "_pair_plan" not in other.__dict__
+    # sums of 27 ci products of about 1 / (27 ci) ** 0.5 and below 1: either order within 27 ci roundings of partial sums of a few
+    assert (out - want).abs().max() <= 2 * 27 * ci * 2.0 ** -24 * 4
