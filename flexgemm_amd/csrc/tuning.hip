@@ -301,12 +301,16 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
     // An item for half of the CUs is enough (15 192 voxels, 120 items: 384 -> 80 channels 0.087 ms, tiled 0.070; 160 -> 128
     // 0.052 and 0.044), for five eighths where the outputs are up to 32 columns, with little to multiply, and on rows of
     // 1 KiB, which the tiled kernel below splits well (1 976 voxels, C = 1024: 128 items 0.232 ms, tiled 0.166).
+    // Up to 32 columns under rows of 256 bytes and more: from 320 000 voxels, where it is ahead with the tables of a fresh cache too (cache and
+    // one layer, tiled 64 x 32 and 256 x 32: 128 -> 16 channels, 329 832 voxels 261 252 us, 1 053 495 970 891; 272 -> 32 484 456, 2 190 1 795;
+    // 512 -> 16 723 696.  299 416 voxels: 512 -> 16 659 661, 128 -> 16 246 240;  166 789: 405 426 and 167 171.  With a kept cache
+    // 1.1 to 1.4 times as fast from 320 000 on).
     struct Shape { int rows, cols, slab; double rate; };
     const Shape shapes[] = {{128, 256, 128, 1.0}, {256, 128, slab, 0.95}, {256, 64, slab, 0.6}, {256, 32, 64, 0.5}};
     double best = 0.0;
     for (const Shape& sh : shapes) {
         if (row_bytes < 64 || sh.slab > (int)align_up(row_bytes, 64)) continue;
-        if (sh.cols == 256 ? cols <= 128 || slab != 128 : (sh.cols == 128 ? cols <= 64 : (sh.cols == 64 ? cols <= 32 : cols > 32 || row_bytes >= 256))) continue;
+        if (sh.cols == 256 ? cols <= 128 || slab != 128 : (sh.cols == 128 ? cols <= 64 : (sh.cols == 64 ? cols <= 32 : cols > 32 || (row_bytes >= 256 && n < 320000)))) continue;
         // (from ~1900 output columns on the staged bias does not fit beside the rings of the 256 x 128 tile; the other shapes,
         // whose rings leave a little more room, are no help under a weight that wide)
         if (!stream_lds_fits(sh.rows, sh.cols, sh.slab, cols) || (cols > 128 && !stream_lds_fits(256, 128, slab, cols))) continue;
