@@ -50,7 +50,7 @@ EXPORTS = [
     "fgx_serialize_encode", "fgx_serialize_decode", "fgx_serialize_reorder_workspace_bytes",
     "fgx_serialize_reorder_coords",
     "fgx_tile_plan", "fgx_grid_index_pays", "fgx_grid_index_walks", "fgx_subm_neighbor_map_grid_workspace_bytes", "fgx_subm_neighbor_map_grid", "fgx_subm_cache_grid_workspace_bytes",
-    "fgx_subm_cache_build_grid", "fgx_cache_post_workspace_bytes", "fgx_cache_post", "fgx_spconv_neighbor_map_grid_workspace_bytes", "fgx_spconv_neighbor_map_grid",
+    "fgx_subm_cache_build_grid", "fgx_subm_cache_build_grid_plan", "fgx_subm_cache_plan_fits", "fgx_cache_post_workspace_bytes", "fgx_cache_post", "fgx_spconv_neighbor_map_grid_workspace_bytes", "fgx_spconv_neighbor_map_grid",
     "fgx_spconv_cache_grid_workspace_bytes", "fgx_spconv_cache_build_grid", "fgx_spconv_out_coords_grid_workspace_bytes",
     "fgx_spconv_out_coords_grid_count", "fgx_spconv_out_coords_grid_emit",
 ]

@@ -175,6 +175,19 @@ extern "C" int fgx_subm_cache_build_grid(const int32_t* coords, size_t n, int B,
                                          int Dh, int Dd, int with_pairs, void* workspace, size_t workspace_bytes, uint32_t* out_map,
                                          int32_t* gray, int32_t* binary, int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i,
                                          uint32_t* sig_o, uint32_t* seg_host, uint32_t* walk, fgx_stream_t stream) {
+    return fgx_subm_cache_build_grid_plan(coords, n, B, W, H, D, Kw, Kh, Kd, Dw, Dh, Dd, with_pairs, workspace, workspace_bytes, out_map, gray, binary,
+                                          sorted_idx, seg, sig_i, sig_o, seg_host, walk, nullptr, stream);
+}
+
+extern "C" int fgx_subm_cache_plan_fits(size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dd) {
+    GridIndexLayout G;
+    return n > 0 && grid_index_plan(n, B, W, H, D, &G) && grid_plan_fits(G, Kw, Kh, Kd, Dd) ? 1 : 0;
+}
+
+extern "C" int fgx_subm_cache_build_grid_plan(const int32_t* coords, size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dw,
+                                              int Dh, int Dd, int with_pairs, void* workspace, size_t workspace_bytes, uint32_t* out_map,
+                                              int32_t* gray, int32_t* binary, int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i,
+                                              uint32_t* sig_o, uint32_t* seg_host, uint32_t* walk, void* plan, fgx_stream_t stream) {
     const char* who = "fgx_subm_cache_build_grid";
     FGX_CHECK_ARG(Kw > 0 && Kh > 0 && Kd > 0 && (long long)Kw * Kh * Kd <= 32 && (Kw & 1) && (Kh & 1) && (Kd & 1),
                   "%s: mask codes need odd kernel sizes and a volume <= 32, got (%d,%d,%d)", who, Kw, Kh, Kd);
@@ -191,11 +204,13 @@ extern "C" int fgx_subm_cache_build_grid(const int32_t* coords, size_t n, int B,
     FGX_CHECK_ARG((((uintptr_t)coords & 15) | ((uintptr_t)workspace & 255)) == 0, "%s: coords must be 16-byte, workspace 256-byte aligned", who);
     FGX_CHECK_ARG(workspace_bytes >= P.total, "%s: workspace of %zu bytes, need %zu", who, workspace_bytes, P.total);
     FGX_CHECK_ARG(walk == nullptr || (!G.dense && ((uintptr_t)walk & 15) == 0), "%s: an index without a walk, or a misaligned one", who);
+    FGX_CHECK_ARG(plan == nullptr || (walk != nullptr && grid_plan_fits(G, Kw, Kh, Kd, Dd) && ((uintptr_t)plan & 15) == 0),
+                  "%s: no plan of a %d x %d x %d kernel without a walk, or a misaligned one", who, Kw, Kh, Kd);
     char* ws = (char*)workspace;
     PhaseEnd phases{s};
     uint32_t* counts = with_pairs ? (uint32_t*)(ws + P.counts) : nullptr;
     bool counted = false;
-    int rc = subm_map_grid(coords, n, B, W, H, D, Kw, Kh, Kd, Dw, Dh, Dd, G, ws, walk, out_map, gray, binary, counts, &counted, s);
+    int rc = subm_map_grid(coords, n, B, W, H, D, Kw, Kh, Kd, Dw, Dh, Dd, G, ws, walk, plan, out_map, gray, binary, counts, &counted, s);
     if (rc != FGX_OK) return rc;
     return sort_beside_pairs(n, V, binary, sorted_idx, ws + P.sort_ws, P.sort_bytes, with_pairs != 0, s, who, [&](hipStream_t on) {
         int r = counted ? FGX_OK : pair_counts(gray, n, V, counts, on);

@@ -17,6 +17,7 @@
 // buffers (the loads run one chunk ahead), one barrier per chunk.  Persistent: XCD x walks the x-th eighth of the chunks, its workgroups interleave, so
 // that neighboring chunks -- which share their halo rows -- run on one L2 at one time.
 #include "gemm_device.h"
+#include "narrow_plan_build.h"
 #include "narrow_walk.h"
 
 namespace fgx {
@@ -28,11 +29,8 @@ __device__ __forceinline__ rsrc_t narrow_rsrc(const void* p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
 
-constexpr int kNarrowHash = 1024;                // hash table of the plan builder (a power of two)
-
 // ------------------------------------------------------------------------------------------------
-// Plan builder: one workgroup per chunk.  The distinct neighbors of the chunk's rows go through a hash table in LDS;
-// slots are numbered in table order, so the plan depends on the chunk's set of sources alone.
+// Plan builder: one workgroup per chunk (narrow_plan_build.h), from a neighbor map.
 // ------------------------------------------------------------------------------------------------
 __global__ void __launch_bounds__(64) narrow_plan_header_kernel(uint32_t* __restrict__ header) {
     header[threadIdx.x] = 0u;
@@ -46,132 +44,20 @@ template <typename Order, int VC>
 __global__ void __launch_bounds__(256, VC ? 8 : 4) narrow_plan_kernel(const uint32_t* __restrict__ nmap, const Order* __restrict__ order,
                                                           uint32_t n, int v_any, int own_rows, unsigned char* __restrict__ plan) {
     const int V = VC ? VC : v_any;
-    __shared__ uint32_t keys[kNarrowHash + 64];                                     // (a lane without an entry swaps a word of its own)
-    __shared__ __attribute__((aligned(4))) uint16_t slot_of[kNarrowHash];
-    __shared__ uint32_t scan[4];
-    __shared__ uint32_t row_flags[kNarrowRows / 32];
-    __shared__ uint32_t grow_of[kNarrowRows];                                       // the chunk's rows (FGX_EMPTY32 beyond n)
-    __shared__ __attribute__((aligned(16))) uint16_t table_lds[kNarrowRows * kNarrowTableStride];   // leaves as 16-byte stores
+    __shared__ NarrowPlanLds lds;
     const int tid = threadIdx.x;
     const uint32_t chunk = blockIdx.x;
-    unsigned char* mine = plan + kNarrowHeader + (size_t)chunk * kNarrowPlanStride;
-    uint32_t* sources = (uint32_t*)(mine + kNarrowTableBytes);
-    uint32_t* rows = sources + kNarrowSlots;
-    for (int i = tid; i < kNarrowHash + 64; i += 256) keys[i] = FGX_EMPTY32;
-    for (int i = tid; i < kNarrowHash / 2; i += 256) ((uint32_t*)slot_of)[i] = (uint32_t)kNarrowOverflow << 16 | (uint32_t)kNarrowOverflow;
-    if (tid < kNarrowRows / 32) row_flags[tid] = 0u;
+    narrow_plan_clear<256>(lds, V);
     for (int r = tid; r < kNarrowRows; r += 256) {
         const uint32_t gr = chunk * kNarrowRows + (uint32_t)r;
-        grow_of[r] = gr < n ? (order ? (uint32_t)order[gr] : gr) : FGX_EMPTY32;
+        lds.grow_of[r] = gr < n ? (order ? (uint32_t)order[gr] : gr) : FGX_EMPTY32;
     }
-    // entries from V on: the row of zeros (entry 31, the row's overflow flag, is written at the end)
-    for (int i = tid; i < kNarrowRows * (kNarrowTableStride - V); i += 256)
-        table_lds[i / (kNarrowTableStride - V) * kNarrowTableStride + V + i % (kNarrowTableStride - V)] = (uint16_t)(kNarrowZeroSlot * 64u);
     __syncthreads();
-    const int entries = kNarrowRows * V;
-    auto source_of = [&](int e) -> uint32_t {
-        const uint32_t grow = grow_of[e / V];
+    narrow_plan_chunk<256, VC>(lds, V, own_rows != 0, plan, chunk, [&](int e) -> uint32_t {
+        const uint32_t grow = lds.grow_of[e / V];
         if (grow == FGX_EMPTY32) return FGX_EMPTY32;
         return nmap[(size_t)grow * V + (e % V)];
-    };
-    auto hash = [](uint32_t x) -> uint32_t { return (x * 2654435761u) >> 22; };      // 10 bits
-    auto insert = [&](uint32_t idx, uint32_t h) -> int {                             // table position, -1 when the table is full
-        for (int probe = 0; probe < kNarrowHash; ++probe) {
-            const uint32_t old = atomicCAS(&keys[h], FGX_EMPTY32, idx);
-            if (old == FGX_EMPTY32 || old == idx) return (int)h;
-            h = (h + 1) & (kNarrowHash - 1);
-        }
-        return -1;
-    };
-    // A chunk row that is also a source row (the same voxels on both sides: every row is its own centre neighbor) takes
-    // the slot of its chunk row number: the 16 rows of a fragment read then fall on 16 different slots modulo 16 for
-    // the centre offset and on nearly as many for the others -- the neighbors of consecutive rows are mostly
-    // consecutive rows -- which is what keeps the reads of arbitrary slots off each other's banks.
-    if (own_rows) {
-        for (int r = tid; r < kNarrowRows; r += 256) {
-            if (grow_of[r] != FGX_EMPTY32) {
-                const int pos = insert(grow_of[r], hash(grow_of[r]));
-                if (pos >= 0) slot_of[pos] = (uint16_t)r;
-            }
-        }
-        __syncthreads();
-    }
-    // (a thread's entries stay in registers for the second pass: kNarrowRows * kNarrowMaxV / 256 of them at most; all
-    // of them are fetched before the first goes into the table, so that their latencies overlap)
-    constexpr int kPerThread = (kNarrowRows * (VC ? VC : 32) + 255) / 256;
-    uint32_t mine_idx[kPerThread];
-#pragma unroll
-    for (int j = 0; j < kPerThread; ++j) {
-        const int e = tid + j * 256;
-        mine_idx[j] = e < entries ? source_of(e) : FGX_EMPTY32;
-    }
-    // first probes of all entries in flight together; the few that met another key go on from there
-    int pos[kPerThread];
-    uint32_t met[kPerThread];
-#pragma unroll
-    for (int j = 0; j < kPerThread; ++j) {
-        pos[j] = mine_idx[j] != FGX_EMPTY32 ? (int)hash(mine_idx[j]) : kNarrowHash + (tid & 63);
-        met[j] = atomicCAS(&keys[pos[j]], FGX_EMPTY32, mine_idx[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < kPerThread; ++j)
-        if (met[j] != FGX_EMPTY32 && met[j] != mine_idx[j]) pos[j] = insert(mine_idx[j], (uint32_t)(pos[j] + 1) & (kNarrowHash - 1));
-    __syncthreads();
-    // the other sources: slots from `base` on in table order (exclusive scan of their positions, four per thread)
-    const uint32_t base = own_rows ? (uint32_t)kNarrowRows : 0u;
-    if (own_rows) {
-        for (int r = tid; r < kNarrowRows; r += 256) sources[r] = grow_of[r];
-    }
-    uint32_t own = 0;
-    for (int j = 0; j < 4; ++j) own += (keys[tid * 4 + j] != FGX_EMPTY32 && slot_of[tid * 4 + j] == kNarrowOverflow) ? 1u : 0u;
-    uint32_t upto = own;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = (uint32_t)__shfl_up((int)upto, d, 64);
-        upto += (tid & 63) >= d ? o : 0u;
-    }
-    if ((tid & 63) == 63) scan[tid >> 6] = upto;
-    __syncthreads();
-    uint32_t next = base + upto - own, total = base;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        next += w < (tid >> 6) ? scan[w] : 0u;
-        total += scan[w];
-    }
-    for (int j = 0; j < 4; ++j) {
-        const int pos = tid * 4 + j;
-        if (keys[pos] != FGX_EMPTY32 && slot_of[pos] == kNarrowOverflow) {
-            if (next < (uint32_t)kNarrowSlots) {
-                slot_of[pos] = (uint16_t)next;
-                sources[next] = keys[pos];
-            }
-            ++next;
-        }
-    }
-    for (uint32_t s = total + tid; s < (uint32_t)kNarrowSlots; s += 256) sources[s] = FGX_EMPTY32;
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kPerThread; ++j) {
-        const int e = tid + j * 256;
-        if (e >= entries) break;
-        uint16_t out = (uint16_t)kNarrowZeroSlot;
-        if (pos[j] < kNarrowHash) out = pos[j] >= 0 ? slot_of[pos[j]] : (uint16_t)kNarrowOverflow;
-        // what the multipliers read: the byte offset of the row's logical piece 0 in the row buffer
-        if (out != (uint16_t)kNarrowOverflow) out = (uint16_t)(out * 64u + (((uint32_t)out >> 2) & 3u) * 16u);
-        table_lds[(e / V) * kNarrowTableStride + (e % V)] = out;
-        if (out == (uint16_t)kNarrowOverflow) atomicOr(&row_flags[(e / V) >> 5], 1u << ((e / V) & 31));
-    }
-    __syncthreads();
-    for (int r = tid; r < kNarrowRows; r += 256)
-        table_lds[r * kNarrowTableStride + kNarrowTableStride - 1] = (uint16_t)((row_flags[r >> 5] >> (r & 31)) & 1u);
-    if (tid == 0 && (row_flags[0] | row_flags[1] | row_flags[2] | row_flags[3]) != 0u) atomicAdd((uint32_t*)plan, 1u);
-    for (int r = tid; r < kNarrowRows; r += 256) rows[r] = grow_of[r];
-    __syncthreads();
-    {
-        const uint4* from = (const uint4*)table_lds;
-        uint4* to = (uint4*)mine;                       // (the plan and its chunks are 16-byte aligned)
-        for (int i = tid; i < kNarrowTableBytes / 16; i += 256) to[i] = from[i];
-    }
+    });
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -54,14 +54,17 @@ struct GridIndexLayout {
 bool grid_index_plan(size_t n, int B, int W, int H, int D, GridIndexLayout* out);
 // the rule of the "auto" builder: forms that fit are also worth their clears
 bool grid_index_pays(size_t n, int B, int W, int H, int D);
-// walk (optional, `bits` form): n words for the rows in cell order, in place of the workspace's
+// walk (optional, `bits` form): n words for the rows in cell order, in place of the workspace's.  plan_header (optional, with a walk): the header
+// of a narrow layer's plan, cleared on the way
 int grid_index_build(const int32_t* coords, size_t n, int B, int W, int H, int D, const GridIndexLayout& L, void* workspace, uint32_t* walk,
-                     GridIndex* out, hipStream_t s, const char* what);
+                     uint32_t* plan_header, GridIndex* out, hipStream_t s, const char* what);
 
 // Submanifold map over a planned index.  counts (optional, [V][ceil(n / kPairSubRows)]): set mask bits per kPairSubRows rows;
-// *counted says whether they were written (the `cells` form does).
+// *counted says whether they were written (the `cells` form does).  plan (optional, with a walk, 3 x 3 x 3 kernels that grid_plan_fits): the narrow layers'
+// plan along the walk, made with the map.
+inline bool grid_plan_fits(const GridIndexLayout& L, int Kw, int Kh, int Kd, int Dd) { return !L.dense && Kw == 3 && Kh == 3 && Kd == 3 && Dd <= 16; }
 int subm_map_grid(const int32_t* coords, size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dw, int Dh, int Dd,
-                  const GridIndexLayout& L, void* workspace, uint32_t* walk, uint32_t* out_map, int32_t* gray, int32_t* binary, uint32_t* counts,
+                  const GridIndexLayout& L, void* workspace, uint32_t* walk, void* plan, uint32_t* out_map, int32_t* gray, int32_t* binary, uint32_t* counts,
                   bool* counted, hipStream_t s);
 
 // Both maps of a generic convolution: an index of the inputs, and of the outputs for the backward map.

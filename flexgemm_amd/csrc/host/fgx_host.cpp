@@ -36,7 +36,7 @@ namespace {
 // ---- the library -------------------------------------------------------------------------------------------------
 #define FGX_HOST_FUNCTIONS(X)                                                                                                     \
     X(fgx_last_error) X(fgx_grid_index_pays) X(fgx_grid_index_walks) X(fgx_subm_neighbor_map_grid_workspace_bytes) X(fgx_subm_cache_grid_workspace_bytes) \
-    X(fgx_subm_cache_build_grid) X(fgx_cache_post_workspace_bytes) X(fgx_cache_post) X(fgx_spconv_cache_grid_workspace_bytes) X(fgx_spconv_cache_build_grid)                           \
+    X(fgx_subm_cache_build_grid_plan) X(fgx_subm_cache_plan_fits) X(fgx_narrow_plan_bytes) X(fgx_cache_post_workspace_bytes) X(fgx_cache_post) X(fgx_spconv_cache_grid_workspace_bytes) X(fgx_spconv_cache_build_grid)                           \
     X(fgx_spconv_out_dims) X(fgx_spconv_out_coords_grid_workspace_bytes) X(fgx_spconv_out_coords_grid_count)                       \
     X(fgx_spconv_out_coords_grid_emit) X(fgx_tile_plan) X(fgx_gather_item_order) X(fgx_gather_item_order_workspace_bytes)          \
     X(fgx_weight_panel_bytes) X(fgx_pack_weight) X(fgx_conv_scratch_bytes) X(fgx_conv_gather_gemm_act_mask)                        \
@@ -313,7 +313,7 @@ struct Layer {
     bool record, input_grad, weight_grad, splitk;
 };
 struct Needs {
-    bool order = true, lists = true;
+    bool order = true, lists = true, plan = false;          // plan: the narrow layers', at the first product
 };
 
 bool schedules_are_ours();
@@ -342,6 +342,7 @@ Needs layer_needs(const Layer& l, int64_t n, int v, bool walks) {
     const bool backward = !l.record || !l.input_grad || (resident && l.ci % 8 == 0) || L.fgx_conv_gemm_stem_pays(l.code, 1, (size_t)n, co, (int)l.ci, v) ||
                           (l.splitk && L.fgx_conv_gemm_pairs_pays(l.code, 1, (size_t)n, (int)l.ci, co, v));
     needs.order = !(forward && backward);
+    needs.plan = resident && n * 82 + 10752 < 0xFF000000ll && n * ci * 2 < 0xFF000000ll;        // (what _narrow_applies asks)
     needs.lists = l.record && l.weight_grad && !resident && !L.fgx_wgrad_stem_pays(l.code, (size_t)n, ci, co, v);
     return needs;
 }
@@ -387,8 +388,8 @@ void cache_post(const Cache& c, bool order, bool lists) {
 }
 
 // Tables of a submanifold convolution through the grid index, or None where it does not apply:
-// (neighbor_map, gray, binary, order, walk, seg, sig_i, sig_o, SegHost), the last four None without gradients; walk: the rows in the
-// order of the index's cells, for the plan of narrow layers, or None.  layer (dtype code, ci, co, record, input_grad, weight_grad, splitk):
+// (neighbor_map, gray, binary, order, walk, seg, sig_i, sig_o, SegHost, plan), the four before the plan None without gradients; walk: the rows in the
+// order of the index's cells, for the plan of narrow layers, or None; last that plan, where the layer wants it at once, or None.  layer (dtype code, ci, co, record, input_grad, weight_grad, splitk):
 // the layer that asks, whose kernels may read neither the order nor the lists; those are None then.
 py::object subm_cache(const Tensor& coords, const std::vector<int>& geom, bool needs_grad, bool forced, size_t max_pair_bytes,
                       const c10::optional<std::tuple<int, int64_t, int64_t, bool, bool, bool, bool>>& layer) {
@@ -420,16 +421,21 @@ py::object subm_cache(const Tensor& coords, const std::vector<int>& geom, bool n
     }
     Tensor walk;
     if (walks) walk = make({rows}, at::kUInt32, dev);
+    // (none is made inside a capture: it would be made again on every replay)
+    Tensor plan;
+    if (needs.plan && walks && V == 27 && L.fgx_subm_cache_plan_fits(n, B, W, H, D, geom[4], geom[5], geom[6], geom[9]) && !capturing(stream))
+        plan = make({(int64_t)L.fgx_narrow_plan_bytes(n, V)}, at::kByte, dev);
     Tensor ws = workspace(L.fgx_subm_cache_grid_workspace_bytes(n, B, W, H, D, V, lists), dev);
-    check(L.fgx_subm_cache_build_grid(ptr<int32_t>(coords), n, B, W, H, D, geom[4], geom[5], geom[6], geom[7], geom[8], geom[9], lists,
+    check(L.fgx_subm_cache_build_grid_plan(ptr<int32_t>(coords), n, B, W, H, D, geom[4], geom[5], geom[6], geom[7], geom[8], geom[9], lists,
                                       ptr(ws), (size_t)ws.numel(), ptr<uint32_t>(nmap), ptr<int32_t>(gray), ptr<int32_t>(binary),
                                       ptr<int64_t>(order), ptr<uint32_t>(seg), ptr<uint32_t>(sig_i), ptr<uint32_t>(sig_o),
-                                      host ? host->words() : nullptr, ptr<uint32_t>(walk), as_stream(stream)));
+                                      host ? host->words() : nullptr, ptr<uint32_t>(walk), ptr(plan), as_stream(stream)));
+    const py::object plan_out = plan.defined() ? py::cast(plan) : py::none();
     py::object walk_out = walk.defined() ? py::cast(walk) : py::none();
     const py::object order_out = order.defined() ? py::cast(order) : py::none();
-    if (!host) return py::make_tuple(nmap, gray, binary, order_out, walk_out, py::none(), py::none(), py::none(), py::none());
+    if (!host) return py::make_tuple(nmap, gray, binary, order_out, walk_out, py::none(), py::none(), py::none(), py::none(), plan_out);
     host->record(as_stream(stream));
-    return py::make_tuple(nmap, gray, binary, order_out, walk_out, seg, sig_i, sig_o, std::move(host));
+    return py::make_tuple(nmap, gray, binary, order_out, walk_out, seg, sig_i, sig_o, std::move(host), plan_out);
 }
 
 bool conv_grids_pay(size_t n_in, size_t n_out, int B, const int* in, const int* out, bool with_bwd) {

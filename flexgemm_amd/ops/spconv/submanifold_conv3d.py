@@ -471,7 +471,7 @@ def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, ne
     """The masked algorithms' neighbor cache through fgx_subm_cache_build_grid or fgx_subm_cache_build: map, codes, mask sort and (needs_grad) the pair
     lists enqueued by one library call, with every buffer allocated beforehand -- the GPU does not wait for the host
     between the steps.  layer: the layer the cache is for, (dtype code or -1, ci, co, records gradients, the input's, the weight's, split K), whose kernels may not
-    need all of it.  Returns (nmap, gray, binary, order or None, walk of the grid index or None, pairs or None), or None where the call does not apply (the
+    need all of it.  Returns (nmap, gray, binary, order or None, walk of the grid index or None, plan of the narrow layers or None, pairs or None), or None where the call does not apply (the
     hash builder's range, kernels beyond what the sorted builder takes, pair lists too large to allocate at their bound)
     and the step-by-step path runs."""
     n = coords.shape[0]
@@ -482,8 +482,8 @@ def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, ne
         built = nat.host().subm_cache(coords, [B, W, H, D, kw, kh, kd, int(dilation[0]), int(dilation[1]), int(dilation[2])], needs_grad,
                                       spconv.NEIGHBOR_MAP_BUILDER == "grid", PAIR_LISTS_UNSIZED_MAX_BYTES, layer)
         if built is not None:
-            nmap, gray, binary, order, walk, seg, sig_i, sig_o, arriving = built
-            return nmap, gray, binary, order, walk, ({"seg": seg, "pending": (sig_i, sig_o, arriving, arriving)} if seg is not None else None)
+            nmap, gray, binary, order, walk, seg, sig_i, sig_o, arriving, plan = built
+            return nmap, gray, binary, order, walk, plan, ({"seg": seg, "pending": (sig_i, sig_o, arriving, arriving)} if seg is not None else None)
     builder = _pick_builder(n, v, B, (W, H, D))
     vol = B * W * H * D
     bound = n * v
@@ -524,7 +524,7 @@ def _build_cache_one_call(coords: torch.Tensor, shape, kernel_size, dilation, ne
             arrived = torch.cuda.Event()
             arrived.record()
             pairs = {"seg": seg, "pending": (buf_i, buf_o, seg_pinned, arrived)}
-    return nmap, gray, binary, order, None, pairs
+    return nmap, gray, binary, order, None, None, pairs
 
 
 _panel_bytes_kept = 0       # bytes of weight panels kept with their weights (all devices)
@@ -809,7 +809,7 @@ class SubMConv3dFunction(Function):
             return SubMConv3dNeighborCache(neighbor_map=nmap)
         built = _build_cache_one_call(coords, shape, kernel_size, dilation, needs_grad, layer) if CACHE_BUILD_ONE_CALL else None
         if built is not None:
-            nmap, gray, binary, order, walk, pairs = built
+            nmap, gray, binary, order, walk, plan, pairs = built
             cache = SubMConv3dNeighborCache(neighbor_map=nmap, gray_code=gray)
             if order is not None:
                 cache["sorted_idx"] = order
@@ -821,6 +821,9 @@ class SubMConv3dFunction(Function):
             cache["_binary_code"] = binary
             if walk is not None:
                 cache["_cell_walk"] = walk
+            if plan is not None:
+                cache["_narrow_plan_buf"] = plan
+                cache["_tables_made_on"] = torch.cuda.current_stream(coords.device).cuda_stream     # (other streams' calls wait for it)
             if pairs is not None:
                 cache._attach_pairs(pairs)
             elif needs_grad:

@@ -208,6 +208,13 @@ int fgx_subm_cache_build_grid(const int32_t* coords, size_t n, int B, int W, int
                               int with_pairs, void* workspace, size_t workspace_bytes, uint32_t* out_map, int32_t* gray, int32_t* binary,
                               int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, uint32_t* seg_host,
                               uint32_t* walk, fgx_stream_t stream);
+/* ... which also makes the plan of the narrow layers along `walk` (fgx_narrow_plan_walk's, fgx_narrow_plan_bytes(n, 27) bytes, 16-byte aligned) while it
+ * has the map's rows at hand; plan may be NULL.  fgx_subm_cache_plan_fits: whether it can (3 x 3 x 3 kernels over an index that walks). */
+int fgx_subm_cache_plan_fits(size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dd);
+int fgx_subm_cache_build_grid_plan(const int32_t* coords, size_t n, int B, int W, int H, int D, int Kw, int Kh, int Kd, int Dw, int Dh, int Dd,
+                              int with_pairs, void* workspace, size_t workspace_bytes, uint32_t* out_map, int32_t* gray, int32_t* binary,
+                              int64_t* sorted_idx, uint32_t* seg, uint32_t* sig_i, uint32_t* sig_o, uint32_t* seg_host,
+                              uint32_t* walk, void* plan, fgx_stream_t stream);
 
 /* Per row-tile (block consecutive rows of the sorted order) OR of the masks.
  *   codes: tile_code[nb] <- OR mask, seg[nb+1] <- exclusive offsets of popcounts (seg[nb] = total);
