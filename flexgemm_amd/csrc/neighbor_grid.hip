@@ -17,11 +17,12 @@ namespace {
 constexpr int kRowsPerGroup = 64;           // rows whose neighbors one workgroup finds: a wavefront of questions per kernel column
 constexpr int kMaxStageV = 128;             // their map rows are staged in LDS: kernel volumes up to this
 constexpr unsigned kLookbackValue = (1u << 30) - 1u, kLookbackSum = 1u << 30, kLookbackTotal = 2u << 30;
-// The counting pass: 128-bit blocks per thread.  Tiles of 64 KiB of bits spread a small bit map over the chip; a large one takes
-// 256 KiB, so that its workgroups do not queue at the ticket (128 MiB: 0.063 -> 0.048 ms).
-constexpr int kCountThreads = 512, kCountRowsShort = 8, kCountRowsLong = 32;
-constexpr size_t kCountLongFrom = (size_t)1 << 20;                  // blocks (16 MiB of bits)
-constexpr int count_rows(size_t blocks) { return blocks > kCountLongFrom ? kCountRowsLong : kCountRowsShort; }
+// The counting pass: 128-bit blocks per thread.  A large bit map takes tiles of 256 KiB of bits, so that its workgroups do not queue at the ticket
+// (128 MiB: 0.063 -> 0.048 ms); one of up to 4 MiB waits for the scans one after the other of a thread's blocks, so it has two of them (tiles
+// of 16 KiB against 64: 0.4 MiB 7.4 -> 5.2 us, 2 MiB 8.6 -> 6.6, 3.4 MiB 8.7 -> 8.6).
+constexpr int kCountThreads = 512, kCountRowsFew = 2, kCountRowsShort = 8, kCountRowsLong = 32;
+constexpr size_t kCountFewUpTo = (size_t)1 << 18, kCountLongFrom = (size_t)1 << 20;                 // blocks (4 and 16 MiB of bits)
+constexpr int count_rows(size_t blocks) { return blocks > kCountLongFrom ? kCountRowsLong : (blocks > kCountFewUpTo ? kCountRowsShort : kCountRowsFew); }
 
 static_assert(kRowsPerGroup == kPairSubRows, "the map kernel counts pairs by its own rows");
 
@@ -738,8 +739,10 @@ int launch_count(const char* ws, const GridIndexLayout& L, Total* total, hipStre
     uint32_t* state = (uint32_t*)(ws + L.state);
     uint32_t* counts = (uint32_t*)(ws + L.counts);
     const unsigned tiles = (unsigned)L.tiles;
-    if (count_rows(L.blocks) == kCountRowsLong) count_bits_kernel<kCountRowsLong><<<tiles, kCountThreads, 0, s>>>(bits, L.blocks, tiles, state, counts, total);
-    else count_bits_kernel<kCountRowsShort><<<tiles, kCountThreads, 0, s>>>(bits, L.blocks, tiles, state, counts, total);
+    const int per = count_rows(L.blocks);
+    if (per == kCountRowsLong) count_bits_kernel<kCountRowsLong><<<tiles, kCountThreads, 0, s>>>(bits, L.blocks, tiles, state, counts, total);
+    else if (per == kCountRowsShort) count_bits_kernel<kCountRowsShort><<<tiles, kCountThreads, 0, s>>>(bits, L.blocks, tiles, state, counts, total);
+    else count_bits_kernel<kCountRowsFew><<<tiles, kCountThreads, 0, s>>>(bits, L.blocks, tiles, state, counts, total);
     FGX_CHECK_LAUNCH(what);
     return FGX_OK;
 }

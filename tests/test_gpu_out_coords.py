@@ -9,7 +9,8 @@ from oracle import sparse_conv as sc
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dims,n", [((1, 1, 1, 1), 1), ((2, 40, 41, 39), 3000), ((3, 9, 7, 70), 63), ((1, 130, 128, 129), 20000), ((2, 5, 3000, 33), 257)])
+@pytest.mark.parametrize("dims,n", [((1, 1, 1, 1), 1), ((2, 40, 41, 39), 3000), ((3, 9, 7, 70), 63), ((1, 130, 128, 129), 20000), ((2, 5, 3000, 33), 257),
+                                     ((1, 128, 512, 512), 3000), ((1, 129, 512, 512), 3000)])
 @pytest.mark.parametrize("geom", [((3, 3, 3), (1, 1, 1), (1, 1, 1), (1, 1, 1)), ((3, 3, 3), (2, 2, 2), (1, 1, 1), (1, 1, 1)), ((2, 2, 2), (2, 2, 2), (0, 0, 0), (1, 1, 1)),
                                   ((1, 2, 3), (3, 2, 1), (0, 4, 2), (1, 2, 3)), ((3, 1, 2), (1, 3, 2), (5, 0, 1), (2, 1, 1)), ((3, 3, 4), (2, 1, 2), (1, 1, 2), (1, 2, 1)),
                                   ((3, 2, 3), (4, 5, 3), (2, 2, 2), (3, 1, 2))])
