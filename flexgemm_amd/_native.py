@@ -40,7 +40,7 @@ EXPORTS = [
     "fgx_wgrad_scratch_bytes", "fgx_wgrad_block_bounds_count", "fgx_wgrad_block_bounds", "fgx_conv_wgrad",
     "fgx_wgrad_item_lists_count", "fgx_wgrad_short_tile", "fgx_wgrad_schedule", "fgx_wgrad_sweep_fits", "fgx_wgrad_item_lists", "fgx_conv_wgrad_lists", "fgx_wgrad_split_tile", "fgx_conv_wgrad_split_scratch_bytes", "fgx_conv_wgrad_split",
     "fgx_zorder_rows", "fgx_narrow_plan_bytes", "fgx_narrow_plan", "fgx_narrow_plan_walk", "fgx_conv_narrow_gemm", "fgx_narrow_wgrad_scratch_bytes", "fgx_conv_narrow_wgrad", "fgx_conv_narrow_wgrad_bias",
-    "fgx_conv_gemm_stem_pays", "fgx_conv_gemm_stem", "fgx_wgrad_stem_pays", "fgx_wgrad_stem_scratch_bytes", "fgx_conv_wgrad_stem",
+    "fgx_conv_gemm_stem_pays", "fgx_conv_gemm_stem", "fgx_wgrad_stem_pays", "fgx_wgrad_stem_scratch_bytes", "fgx_conv_wgrad_stem", "fgx_conv_wgrad_stem_cut",
     "fgx_wgrad_sweep_plan_bytes", "fgx_wgrad_sweep_plan", "fgx_wgrad_sweep_scratch_bytes", "fgx_conv_wgrad_sweep",
     "fgx_wgrad_sweep_giveup_words", "fgx_wgrad_sweep_reduce",
     "fgx_colsum_scratch_bytes", "fgx_colsum", "fgx_colsum_static_prepare", "fgx_colsum_static_max_cols", "fgx_colsum_static",

@@ -311,7 +311,7 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
 // grad_weight and grad_bias: 32 columns of blockDim.z rows of the product per workgroup, blockDim.y threads per element each adding
 // every blockDim.y-th partial product, their sums added in order.
 template <typename T>
-__global__ void __launch_bounds__(1024) stem_reduce_kernel(const float* __restrict__ partial, unsigned groups, int V, int Ci, int Co, int N,
+__global__ void __launch_bounds__(1024) stem_reduce_kernel(const float* __restrict__ partial, unsigned groups, int V, int Ci, int out_ci, int Co, int N,
                                                            T* __restrict__ gw, T* __restrict__ gb) {
     __shared__ float sums[32][33];                             // [rows * slices][32]
     const int c = threadIdx.x, slices = blockDim.y, slice = threadIdx.y, at = threadIdx.z * slices;
@@ -330,8 +330,12 @@ __global__ void __launch_bounds__(1024) stem_reduce_kernel(const float* __restri
     float r = sums[at][c];
     for (int q = 1; q < slices; ++q) r += sums[at + q][c];
     if (slice != 0 || co >= Co) return;
-    if (col < V * Ci) gw[(size_t)co * V * Ci + col] = from_float<T>(r);
-    else if (gb != nullptr && col == N - 8) gb[co] = from_float<T>(r);
+    if (col < V * Ci) {
+        const int v = col / Ci, ci = col - v * Ci;             // (the channels that filled the rows up are nobody's)
+        if (ci < out_ci) gw[((size_t)co * V + v) * out_ci + ci] = from_float<T>(r);
+    } else if (gb != nullptr && col == N - 8) {
+        gb[co] = from_float<T>(r);
+    }
 }
 
 // Forward product and input gradient of such layers (8 or 16 channels on the gathered side): the neighbors' features of a row lie
@@ -558,7 +562,8 @@ unsigned stem_groups(size_t n, int Ci, int Co) {
 }
 
 template <typename Tag, int P>
-int stem_launch(const void* gout, const void* feats, const uint32_t* map, size_t n, int Co, int V, float* scratch, void* gw, void* gb, hipStream_t s) {
+int stem_launch(const void* gout, const void* feats, const uint32_t* map, size_t n, int out_ci, int Co, int V, float* scratch, void* gw, void* gb,
+                hipStream_t s) {
     using C = StemCfg<P>;
     using T = typename Tag::type;
     auto kern = stem_wgrad_kernel<Tag, P>;
@@ -574,7 +579,7 @@ int stem_launch(const void* gout, const void* feats, const uint32_t* map, size_t
     unsigned slices = 1;
     while (slices < 32 && slices * 8 < groups) slices *= 2;
     const unsigned rows = slices >= 8 ? 1 : 8 / slices;
-    stem_reduce_kernel<T><<<dim3(C::N / 32, cdiv(Co, rows)), dim3(32, slices, rows), 0, s>>>(scratch, groups, V, 8 * P, Co, C::N, (T*)gw, (T*)gb);
+    stem_reduce_kernel<T><<<dim3(C::N / 32, cdiv(Co, rows)), dim3(32, slices, rows), 0, s>>>(scratch, groups, V, 8 * P, out_ci, Co, C::N, (T*)gw, (T*)gb);
     FGX_CHECK_LAUNCH("fgx_conv_wgrad_stem(reduce)");
     return FGX_OK;
 }
@@ -631,17 +636,23 @@ size_t fgx_wgrad_stem_scratch_bytes(size_t n, int Ci, int Co) {
 
 int fgx_conv_wgrad_stem(int dtype, const void* grad_out, const void* feats, const uint32_t* map, size_t n, int Ci, int Co, int V, void* scratch,
                         void* grad_weight, void* grad_bias, fgx_stream_t stream) {
+    return fgx_conv_wgrad_stem_cut(dtype, grad_out, feats, map, n, Ci, Ci, Co, V, scratch, grad_weight, grad_bias, stream);
+}
+
+int fgx_conv_wgrad_stem_cut(int dtype, const void* grad_out, const void* feats, const uint32_t* map, size_t n, int Ci, int out_ci, int Co, int V,
+                            void* scratch, void* grad_weight, void* grad_bias, fgx_stream_t stream) {
     FGX_CHECK_ARG(stem_wgrad_takes(dtype, n, Ci, Co, V), "fgx_conv_wgrad_stem: dtype %d, n=%zu, Ci=%d, Co=%d, V=%d is not for this kernel", dtype, n,
                   Ci, Co, V);
+    FGX_CHECK_ARG(out_ci >= 1 && out_ci <= Ci, "fgx_conv_wgrad_stem: %d of %d channels", out_ci, Ci);
     FGX_CHECK_ARG(grad_out && feats && map && scratch && grad_weight, "fgx_conv_wgrad_stem: null buffer");
     FGX_CHECK_ARG((((uintptr_t)grad_out | (uintptr_t)feats | (uintptr_t)map | (uintptr_t)scratch) & 15) == 0,
                   "fgx_conv_wgrad_stem: grad_out, feats, map and scratch must be 16-byte aligned");
     hipStream_t s = (hipStream_t)stream;
     if (dtype == FGX_F16)
-        return Ci == 8 ? stem_launch<F16, 1>(grad_out, feats, map, n, Co, V, (float*)scratch, grad_weight, grad_bias, s)
-                       : stem_launch<F16, 2>(grad_out, feats, map, n, Co, V, (float*)scratch, grad_weight, grad_bias, s);
-    return Ci == 8 ? stem_launch<BF16, 1>(grad_out, feats, map, n, Co, V, (float*)scratch, grad_weight, grad_bias, s)
-                   : stem_launch<BF16, 2>(grad_out, feats, map, n, Co, V, (float*)scratch, grad_weight, grad_bias, s);
+        return Ci == 8 ? stem_launch<F16, 1>(grad_out, feats, map, n, out_ci, Co, V, (float*)scratch, grad_weight, grad_bias, s)
+                       : stem_launch<F16, 2>(grad_out, feats, map, n, out_ci, Co, V, (float*)scratch, grad_weight, grad_bias, s);
+    return Ci == 8 ? stem_launch<BF16, 1>(grad_out, feats, map, n, out_ci, Co, V, (float*)scratch, grad_weight, grad_bias, s)
+                   : stem_launch<BF16, 2>(grad_out, feats, map, n, out_ci, Co, V, (float*)scratch, grad_weight, grad_bias, s);
 }
 
 // Where it is ahead of the general kernels (us, scan order, bf16: general, this):

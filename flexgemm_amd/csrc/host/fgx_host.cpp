@@ -43,7 +43,7 @@ namespace {
     X(fgx_conv_gather_gemm_weight_pays) X(fgx_conv_gather_gemm_weight) X(fgx_conv_gemm_pairs_pays) X(fgx_pair_plan_words) X(fgx_pair_plan) X(fgx_conv_gemm_pairs_scratch_bytes) X(fgx_conv_gemm_pairs) X(fgx_conv_gemm_few_pays) X(fgx_conv_gemm_few_mask)                                                             \
     X(fgx_conv_gather_gemm_stream_act_mask) X(fgx_conv_gather_gemm_stream_groups) X(fgx_relu_mask_apply) X(fgx_copy_columns)       \
     X(fgx_colsum_scratch_bytes) X(fgx_colsum) X(fgx_wgrad_block_bounds_count) X(fgx_wgrad_block_bounds)                            \
-    X(fgx_conv_gemm_stem_pays) X(fgx_conv_gemm_stem) X(fgx_wgrad_stem_pays) X(fgx_wgrad_stem_scratch_bytes) X(fgx_conv_wgrad_stem) X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
+    X(fgx_conv_gemm_stem_pays) X(fgx_conv_gemm_stem) X(fgx_wgrad_stem_pays) X(fgx_wgrad_stem_scratch_bytes) X(fgx_conv_wgrad_stem_cut) X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
     X(fgx_wgrad_schedule) X(fgx_wgrad_sweep_fits) X(fgx_conv_wgrad_split_scratch_bytes) X(fgx_conv_wgrad_split)                                                                  \
     X(fgx_wgrad_sweep_plan_bytes) X(fgx_wgrad_sweep_plan) X(fgx_wgrad_sweep_scratch_bytes) X(fgx_conv_wgrad_sweep)                 \
     X(fgx_serialize_encode) X(fgx_serialize_decode) X(fgx_table_lookup)
@@ -1001,11 +1001,11 @@ WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool 
                aligned(c.need("neighbor_map"))) {
         const Tensor nmap = c.need("neighbor_map");
         Tensor scratch = workspace(L.fgx_wgrad_stem_scratch_bytes((size_t)n, ci, co), dev);
-        w.weight = make({co, v, ci}, feats.scalar_type(), dev);
+        w.weight = make({co, v, true_ci}, feats.scalar_type(), dev);
         if (with_bias) w.bias = make({co}, feats.scalar_type(), dev);
         mark("wgrad", "start");
-        check(L.fgx_conv_wgrad_stem(code, ptr(grad), ptr(feats), ptr<uint32_t>(nmap), (size_t)n, ci, co, v, ptr(scratch), ptr(w.weight), ptr(w.bias),
-                                    as_stream(stream)));
+        check(L.fgx_conv_wgrad_stem_cut(code, ptr(grad), ptr(feats), ptr<uint32_t>(nmap), (size_t)n, ci, (int)true_ci, co, v, ptr(scratch), ptr(w.weight),
+                                        ptr(w.bias), as_stream(stream)));
         mark("wgrad", "stop");
     } else {
         if (!(c.has("valid_signal_seg") && (c.has("valid_signal_i") || c.has("_pending_pairs")))) {
@@ -1071,7 +1071,7 @@ WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool 
     }
     if (ci != true_ci || co != true_co) {
         w.weight = w.weight.slice(0, 0, true_co).contiguous();              // (a view: whole rows)
-        if (ci != true_ci) w.weight = copy_columns(w.weight, true_co * v, ci, {true_co, v, true_ci}, true_ci, stream);
+        if (w.weight.numel() != true_co * v * true_ci) w.weight = copy_columns(w.weight, true_co * v, ci, {true_co, v, true_ci}, true_ci, stream);
         if (with_bias) w.bias = w.bias.slice(0, 0, true_co).contiguous();
     }
     return w;

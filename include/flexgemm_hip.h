@@ -455,6 +455,9 @@ int fgx_wgrad_stem_pays(int dtype, size_t n, int Ci, int Co, int V);
 size_t fgx_wgrad_stem_scratch_bytes(size_t n, int Ci, int Co);
 int fgx_conv_wgrad_stem(int dtype, const void* grad_out, const void* feats, const uint32_t* map, size_t n, int Ci, int Co, int V,
                         void* scratch, void* grad_weight, void* grad_bias, fgx_stream_t stream);
+/* ... of the first out_ci <= Ci input channels (rows filled up to 8 or 16 for the kernel): grad_weight is [Co][V][out_ci]. */
+int fgx_conv_wgrad_stem_cut(int dtype, const void* grad_out, const void* feats, const uint32_t* map, size_t n, int Ci, int out_ci, int Co, int V,
+                            void* scratch, void* grad_weight, void* grad_bias, fgx_stream_t stream);
 
 /* item_at for fgx_conv_gather_gemm_stream, made on the device from the tile codes: items sorted by cost (offsets per
  * row tile x `slabs` K-slabs + an epilogue), the incomplete last round of `groups` positions filled with the cheapest,
