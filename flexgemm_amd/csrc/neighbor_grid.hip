@@ -410,22 +410,23 @@ __device__ __forceinline__ void brick_columns(const GridIndex& index, const Grid
                 }
 }
 
-// The same for K x K x K kernels, K = 2 or 3, one wavefront per 64 rows and a row per lane: a lane asks K columns (K * K
-// questions) before it needs the first answer, and nothing waits for other wavefronts.  What bounds it is the latency of
-// three dependent reads (row, bits, row number) against what a CU holds in flight: one column per wavefront, as above, took
-// 0.261 ms for 2 667 120 voxels of a surface in scan order (3x3x3, map and codes, 331 MB read and written), this form
-// 0.136 (sort and merge: 0.331).  In random order the scattered 108-byte rows bound it (0.283 ms; a plain scatter: 0.26).  In
-// the `bits` form a column's cells have to lie in two bricks: columns longer than 32 cells go to the general kernel.
+// The same for K x K x K kernels, K = 2 or 3: K wavefronts for 64 rows, a row per lane and a plane of the kernel per wavefront, which asks its K columns
+// (K * K questions) before it needs the first answer.  What bounds it is the latency of three dependent reads (row, bits, row number)
+// against what a CU holds in flight: one column per wavefront, as above, took 0.261 ms for 2 667 120 voxels of a surface in scan order (3x3x3, map
+// and codes, 331 MB read and written), all planes in one wavefront 0.136 (sort and merge: 0.331).  So against that: 434 000 voxels 25.0 -> 21.7 us, of which
+// the map and its codes leave at 2.3 TB/s; 67 000 outputs under a stride of 2 12.7 -> 10.0; 3 758 voxels 5.6 -> 4.3; 667 763 voxels in random order
+// 64 -> 59; 2.55 M voxels in scan order level, in random order 241 -> 248, where the scattered 108-byte rows bound it (a plain scatter: 0.26 ms for
+// 2 667 120).  In the `bits` form a column's cells have to lie in two bricks: columns longer than 32 cells go to the general kernel.
 template <bool DENSE, int MODE, int K>
-__global__ void __launch_bounds__(64) cube_map_kernel(const int32_t* __restrict__ coords, GridIndex walk, size_t n,
+__global__ void __launch_bounds__(64 * K) cube_map_kernel(const int32_t* __restrict__ coords, GridIndex walk, size_t n,
                                                       GridIndex index, GridIndex own, int own_dense, QueryGeom g, uint32_t* __restrict__ out_map,
                                                       int32_t* __restrict__ gray, int32_t* __restrict__ binary, uint32_t* __restrict__ counts) {
     constexpr int V = K * K * K, PITCH = V | 1;
     __shared__ __attribute__((aligned(16))) uint32_t stage[kRowsPerGroup * PITCH];
-    __shared__ uint32_t id_lds[kRowsPerGroup];
+    __shared__ uint32_t id_lds[kRowsPerGroup], masks[K][kRowsPerGroup];
     const size_t p0 = (size_t)blockIdx.x * kRowsPerGroup;
     const int cnt = (int)(n - p0 < (size_t)kRowsPerGroup ? n - p0 : (size_t)kRowsPerGroup);
-    const int lane = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, kx = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint32_t id = FGX_EMPTY32;
     int4 c = make_int4(-1, 0, 0, 0);
     if (lane < cnt) {
@@ -439,7 +440,7 @@ __global__ void __launch_bounds__(64) cube_map_kernel(const int32_t* __restrict_
             if (!known) c.x = -1;
         }
     }
-    id_lds[lane] = id;
+    if (kx == 0) id_lds[lane] = id;
     const bool batch_ok = (unsigned)c.x < (unsigned)index.B;
     bool y_ok[K], z_ok[K];
     GridPlace<DENSE> yp[K], zp[K];
@@ -462,57 +463,60 @@ __global__ void __launch_bounds__(64) cube_map_kernel(const int32_t* __restrict_
             if (z_ok[k]) z_first = zp[k].brick;
     }
     uint32_t mask = 0u;
-#pragma unroll
-    for (int kx = 0; kx < K; ++kx) {
-        int xt;
-        const bool x_ok = target<MODE>(c.y, kx, K, g.Sw, g.Pw, g.Dw, index.W, &xt) && batch_ok;
-        uint32_t value[K][K];
-        const GridPlace<DENSE> xp = place_bx<DENSE>(index, c.x, xt);
-        if constexpr (DENSE || MODE == kConvBwd) {
-#pragma unroll
-            for (int ky = 0; ky < K; ++ky)
-#pragma unroll
-                for (int kz = 0; kz < K; ++kz)
-                    value[ky][kz] = x_ok && y_ok[ky] && z_ok[kz] ? grid_find<DENSE>(index, xp + yp[ky] + zp[kz]) : FGX_EMPTY32;
-        } else {
-            brick_columns<K>(index, xp, x_ok, y_ok, yp, z_ok, zp, z_first, z_last, value);
-        }
+    int xt;
+    const bool x_ok = target<MODE>(c.y, kx, K, g.Sw, g.Pw, g.Dw, index.W, &xt) && batch_ok;
+    uint32_t value[K][K];
+    const GridPlace<DENSE> xp = place_bx<DENSE>(index, c.x, xt);
+    if constexpr (DENSE || MODE == kConvBwd) {
 #pragma unroll
         for (int ky = 0; ky < K; ++ky)
 #pragma unroll
-            for (int kz = 0; kz < K; ++kz) {
-                const int v = (kx * K + ky) * K + kz;
-                if (MODE == kSubm && v == V / 2) value[ky][kz] = id;       // the voxel itself, found or not
-                stage[lane * PITCH + v] = value[ky][kz];
-                if (value[ky][kz] != FGX_EMPTY32) mask |= 1u << v;
-            }
+            for (int kz = 0; kz < K; ++kz)
+                value[ky][kz] = x_ok && y_ok[ky] && z_ok[kz] ? grid_find<DENSE>(index, xp + yp[ky] + zp[kz]) : FGX_EMPTY32;
+    } else {
+        brick_columns<K>(index, xp, x_ok, y_ok, yp, z_ok, zp, z_first, z_last, value);
     }
+#pragma unroll
+    for (int ky = 0; ky < K; ++ky)
+#pragma unroll
+        for (int kz = 0; kz < K; ++kz) {
+            const int v = (kx * K + ky) * K + kz;
+            if (MODE == kSubm && v == V / 2) value[ky][kz] = id;       // the voxel itself, found or not
+            stage[lane * PITCH + v] = value[ky][kz];
+            if (value[ky][kz] != FGX_EMPTY32) mask |= 1u << (ky * K + kz);
+        }
+    masks[kx][lane] = mask;
     __syncthreads();
     const uint32_t id0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)id);
     if (PITCH == V && cnt == kRowsPerGroup && (id0 & 3u) == 0u && ((uintptr_t)out_map & 15) == 0 && __ballot(id != id0 + lane) == 0ull) {
         // the rows lie next to each other in the map as well: one run of 16-byte pieces
         uint4* dst = reinterpret_cast<uint4*>(out_map + (size_t)id0 * V);
         const uint4* src = reinterpret_cast<const uint4*>(stage);
-        for (int i = lane; i < kRowsPerGroup * V / 4; i += 64) dst[i] = src[i];
+        for (int i = tid; i < kRowsPerGroup * V / 4; i += 64 * K) dst[i] = src[i];
     } else {
-        for (int i = lane; i < cnt * V; i += 64) {
+        constexpr int kShare = (kRowsPerGroup + K - 1) / K;                // rows that a wavefront writes: a row leaves in one or two stores
+        const int last = (kx + 1) * kShare < cnt ? (kx + 1) * kShare : cnt;
+        for (int i = kx * kShare * V + lane; i < last * V; i += 64) {
             const int row = i / V, v = i - row * V;
             out_map[(size_t)id_lds[row] * V + v] = stage[row * PITCH + v];
         }
     }
     if (gray == nullptr) return;
-    if (lane < cnt) {
-        gray[id] = (int32_t)mask;
-        binary[id] = (int32_t)gray_decode(mask);
+    if (kx == 0 && lane < cnt) {
+        uint32_t all = 0u;
+#pragma unroll
+        for (int k = 0; k < K; ++k) all |= masks[k][lane] << (k * K * K);
+        gray[id] = (int32_t)all;
+        binary[id] = (int32_t)gray_decode(all);
     }
     if (counts != nullptr) {
         uint32_t mine = 0u;
 #pragma unroll
-        for (int v = 0; v < V; ++v) {
+        for (int v = 0; v < K * K; ++v) {
             const uint32_t have = (uint32_t)__popcll(__ballot(lane < cnt && ((mask >> v) & 1u)));
             if (lane == v) mine = have;
         }
-        if (lane < V) counts[(size_t)lane * gridDim.x + blockIdx.x] = mine;
+        if (lane < K * K) counts[(size_t)(kx * K * K + lane) * gridDim.x + blockIdx.x] = mine;
     }
 }
 
@@ -586,9 +590,9 @@ int launch_map(const int32_t* coords, const GridIndex& walk, size_t n, const Gri
     const int R = g.Kw * g.Kh;
     const bool cube = g.Kw == g.Kh && g.Kh == g.Kd && (DENSE || MODE == kConvBwd || g.Dd * (g.Kd - 1) <= 32);
     if (cube && g.Kd == 3) {
-        cube_map_kernel<DENSE, MODE, 3><<<grid, 64, 0, s>>>(coords, walk, n, index, own, own_dense ? 1 : 0, g, out_map, gray, binary, counts);
+        cube_map_kernel<DENSE, MODE, 3><<<grid, 64 * 3, 0, s>>>(coords, walk, n, index, own, own_dense ? 1 : 0, g, out_map, gray, binary, counts);
     } else if (MODE != kSubm && cube && g.Kd == 2) {
-        cube_map_kernel<DENSE, MODE, 2><<<grid, 64, 0, s>>>(coords, walk, n, index, own, own_dense ? 1 : 0, g, out_map, gray, binary, counts);
+        cube_map_kernel<DENSE, MODE, 2><<<grid, 64 * 2, 0, s>>>(coords, walk, n, index, own, own_dense ? 1 : 0, g, out_map, gray, binary, counts);
     } else {
         const int waves = R < 9 ? R : (R % 9 == 0 ? 9 : 8);         // a wavefront per kernel column
         const size_t lds = (size_t)kRowsPerGroup * (4 + 1 + 1 + (g.V | 1)) * 4;
