@@ -162,29 +162,49 @@ __device__ __forceinline__ uint32_t offset_steps(uint32_t cnt) { return (cnt + k
 // offsets and the per-offset lists of partial products are laid out.
 constexpr unsigned kSwCumMax = 4096;     // sub-blocks whose running pair counts fit the units kernel's LDS
 
-// k of the slices in `have_mask`, evenly spread over them (all lanes: lane i decides slice i)
-__device__ __forceinline__ uint64_t spread_take(uint64_t have_mask, unsigned k, unsigned lane) {
+// k of the slices in `have_mask`, evenly spread over them (all lanes: lane i decides slice i).  inv: lane i holds 2^20 / (i + 1), rounded up, whose
+// product with a number below 2^12 is the division by i + 1 in its upper bits (the rounding adds less than i + 1 a unit: 2^12 * 64 < 2^20).
+__device__ __forceinline__ uint64_t spread_take(uint64_t have_mask, unsigned k, unsigned lane, uint32_t inv) {
     const unsigned have = (unsigned)__popcll(have_mask);
     if (k >= have) return have_mask;
+    const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)inv, (int)have - 1);
     const bool mine = (have_mask >> lane) & 1ull;
     const unsigned rank = (unsigned)__popcll(have_mask & ((1ull << lane) - 1ull));      // slices of the mask below this one
-    const bool taken = mine && ((rank + 1u) * k / have > rank * k / have);              // where k * rank / have steps up
+    const bool taken = mine && (((rank + 1u) * k * m) >> 20) > ((rank * k * m) >> 20);  // where k * rank / have steps up
     return __ballot(taken);
 }
+// largest word of the wavefront, in six register-to-register steps (an exchange through LDS takes ten times as long)
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+#define FGX_MAX_WITH(ctrl, rows)                                                                          \
+    do {                                                                                                  \
+        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xF, false);      \
+        v = o > v ? o : v;                                                                                \
+    } while (0)
+    FGX_MAX_WITH(0x111, 0xF);       // row_shr:1, 2, 4, 8: a row's last lane has the row's
+    FGX_MAX_WITH(0x112, 0xF);
+    FGX_MAX_WITH(0x114, 0xF);
+    FGX_MAX_WITH(0x118, 0xF);
+    FGX_MAX_WITH(0x142, 0xA);       // row_bcast:15, 31: lane 63 has all rows'
+    FGX_MAX_WITH(0x143, 0xC);
+#undef FGX_MAX_WITH
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
 // lane holding the smallest (largest) key among the lanes with `live`, lowest lane on ties; -1 if none
-__device__ __forceinline__ int wave_arg(bool live, float key, unsigned lane, bool want_max) {
+__device__ __forceinline__ int wave_arg(bool live, float key, bool want_max) {
     const uint32_t bits = __builtin_bit_cast(uint32_t, key);                              // keys are >= 0: bits order like values
-    unsigned long long k = want_max ? (((unsigned long long)bits << 8) | (255u - lane))
-                                    : (((unsigned long long)(~bits) << 8) | (255u - lane));
-    if (!live) k = 0ull;
-#pragma unroll
-    for (int sh = 32; sh > 0; sh >>= 1) {
-        const unsigned long long o = __shfl_xor(k, sh, 64);
-        k = o > k ? o : k;
-    }
-    return k == 0ull ? -1 : (int)(255u - (unsigned)(k & 255u));
+    const uint32_t k = live ? (want_max ? bits : ~bits) : 0u;
+    const uint32_t best = wave_max(k);          // (by all lanes)
+    return __ffsll((long long)__ballot(live && k == best)) - 1;
+}
+__device__ __forceinline__ float lane_float(float x, int lane) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+}
+__device__ __forceinline__ uint64_t lane_mask(uint64_t x, int lane) {
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), lane) << 32 | (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, lane);
 }
 
+// Bound by its serial choices, 32 workgroups one after the other.  With the exchanges of a choice through LDS and its divisions by 64-bit and
+// run-time numbers the whole plan took 60 us for 9 314 rows, 66 for 166 977 and 72 for 667 763; so 43, 48 and 54 (same plan bit for bit).
 __global__ void __launch_bounds__(64 * kXcds) sweep_units_kernel(const uint32_t* __restrict__ fine, int V, unsigned nsb, unsigned spx,
                                                                 SweepUnit* __restrict__ units, SweepGroup* __restrict__ wg,
                                                                 uint32_t* __restrict__ vcount, uint16_t* __restrict__ vlist) {
@@ -240,6 +260,9 @@ __global__ void __launch_bounds__(64 * kXcds) sweep_units_kernel(const uint32_t*
         uint32_t lo = 0, cnt = 0, N = 0, P = 0;             // this lane's offset
         uint64_t left = 0;                                  // its slices not yet given out
         float per = 0.f;                                    // steps per slice
+        uint32_t full = 0;                                  // steps of every slice, and the slices that have one more
+        uint64_t more = 0;
+        const uint32_t inv = ((1u << 20) + lane) / (lane + 1u);
         if (lane < (unsigned)V) {
             lo = fine[(size_t)lane * (nsb + 1) + sbA];
             cnt = fine[(size_t)lane * (nsb + 1) + sbB] - lo;
@@ -247,6 +270,8 @@ __global__ void __launch_bounds__(64 * kXcds) sweep_units_kernel(const uint32_t*
             P = N < 64u ? N : 64u;
             left = P ? (~0ull >> (64 - P)) : 0ull;
             per = P ? (float)N / (float)P : 0.f;
+            full = P ? N / P : 0u;
+            more = P && N % P ? ~0ull >> (64 - N % P) : 0ull;
         }
         float total = (float)N;
 #pragma unroll
@@ -257,34 +282,35 @@ __global__ void __launch_bounds__(64 * kXcds) sweep_units_kernel(const uint32_t*
             const int items = (int)__popcll(__ballot(left != 0));
             const int must_retire = items - 2 * after;
             const float rem = per * (float)__popcll(left);
-            const int a = wave_arg(left != 0, rem, lane, false);
+            const int a = wave_arg(left != 0, rem, false);
             int b = -1;
             uint64_t mask_a = 0, mask_b = 0;
             if (a >= 0) {                                       // (uniform)
-                const float rem_a = __shfl(rem, a, 64), per_a = __shfl(per, a, 64);
-                const uint64_t left_a = __shfl((unsigned long long)left, a, 64);
+                const float rem_a = lane_float(rem, a), per_a = lane_float(per, a);
+                const uint64_t left_a = lane_mask(left, a);
                 const bool share = rem_a > want && must_retire < 1;     // a share of the smallest offset fills the workgroup
                 if (share) {
                     const unsigned k = (unsigned)(want / per_a + 0.5f);
-                    mask_a = spread_take(left_a, k ? k : 1u, lane);
+                    mask_a = spread_take(left_a, k ? k : 1u, lane, inv);
                 } else {
                     mask_a = left_a;
                 }
                 if ((int)lane == a) left &= ~mask_a;
                 if (!share) {
                     // top up: from the largest other offset, or (when offsets must go) the smallest one whole
-                    b = wave_arg(left != 0 && (int)lane != a, rem, lane, must_retire < 2);
+                    b = wave_arg(left != 0 && (int)lane != a, rem, must_retire < 2);
                     if (b >= 0) {
-                        const float per_b = __shfl(per, b, 64), need = want - rem_a;
-                        const uint64_t left_b = __shfl((unsigned long long)left, b, 64);
+                        const float per_b = lane_float(per, b), need = want - rem_a;
+                        const uint64_t left_b = lane_mask(left, b);
                         if (must_retire >= 2) mask_b = left_b;
-                        else if (need > 0.5f * per_b) mask_b = spread_take(left_b, (unsigned)(need / per_b + 0.5f), lane);
+                        else if (need > 0.5f * per_b) mask_b = spread_take(left_b, (unsigned)(need / per_b + 0.5f), lane, inv);
                         if ((int)lane == b) left &= ~mask_b;
                     }
                 }
             }
             // lane a writes the first unit, lane b the second (lane 0 an empty one where there is none)
             uint32_t my_steps = 0;
+#pragma unroll
             for (int u = 0; u < 2; ++u) {
                 const int who = u == 0 ? a : b;
                 const uint64_t mask = u == 0 ? mask_a : mask_b;
@@ -298,7 +324,7 @@ __global__ void __launch_bounds__(64 * kXcds) sweep_units_kernel(const uint32_t*
                         un.hi = lo + cnt;
                         un.mask_lo = (uint32_t)mask;
                         un.mask_hi = (uint32_t)(mask >> 32);
-                        un.nsteps = unit_count_below(un, N);
+                        un.nsteps = full * (uint32_t)__popcll(mask) + (uint32_t)__popcll(mask & more);
                         my_steps += un.nsteps;
                     }
                     const unsigned q = (xc * spx + s) * 2 + (unsigned)u;
@@ -307,10 +333,10 @@ __global__ void __launch_bounds__(64 * kXcds) sweep_units_kernel(const uint32_t*
                     sh_v[q] = (uint8_t)un.v;
                 }
             }
-            float given = (float)my_steps;
-#pragma unroll
-            for (int sh = 32; sh > 0; sh >>= 1) given += __shfl_xor(given, sh, 64);
-            total -= given;
+            uint32_t given = 0;                                 // (by the lanes of the two offsets alone)
+            if (a >= 0) given += (uint32_t)__builtin_amdgcn_readlane((int)my_steps, a);
+            if (b >= 0) given += (uint32_t)__builtin_amdgcn_readlane((int)my_steps, b);
+            total -= (float)given;
             if (lane == 0) wg[(size_t)xc * spx + s].sb0 = sbA;
         }
     }
