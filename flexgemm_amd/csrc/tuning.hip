@@ -127,7 +127,14 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
         // every workgroup keeps two accumulators over an eighth of the voxels, block_rows is its sub-block size.
         // Measured 20 % to 30 % ahead of the block-major kernel from ten thousand voxels (C = 128: 0.051 against
         // 0.067 ms) to 2.7 million (1.32 against 1.70 ms), for C = 64, 96, 128, coordinates in scan order or shuffled.
-        if (es == 2 && n >= 8192 && n <= ((size_t)1 << 24) && t >= 64 && Ci <= t && Co <= t && V <= 2 * (kCUs / 8)) {
+        // 33 ... 64 channels on one side and 65 ... 128 on the other: the 128 x 128 tile, half of it empty, from 65 536 voxels and under kernels of more than
+        // 8 offsets (the product alone, us: 64 -> 128, 166 977 voxels 107 and 84, 667 763 453 and 269; 38 407 45 and 44;  training with a fresh cache,
+        // its plan included: 65 145 voxels 269 256, 166 789 405 389, 667 156 1130 997; 128 -> 64, 50 850 kept 115 117; under
+        // 2 x 2 x 2, 180 000 outputs fresh 366 381).
+        const int wide = Ci > 64 || Co > 64 ? 128 : 64;
+        const bool mixed = t == 64 && wide == 128 && V > 8 && n >= 65536;
+        if (es == 2 && n >= 8192 && n <= ((size_t)1 << 24) && t >= 64 && V <= 2 * (kCUs / 8) && Ci <= wide && Co <= wide && (wide == t || mixed)) {
+            out->tile_rows = out->tile_cols = wide;
             out->stream = 2;
             out->block_rows = 2048;
             return;
