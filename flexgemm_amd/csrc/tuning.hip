@@ -132,8 +132,12 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
         // its plan included: 65 145 voxels 269 256, 166 789 405 389, 667 156 1130 997; 128 -> 64, 50 850 kept 115 117; under
         // 2 x 2 x 2, 180 000 outputs fresh 366 381).
         const int wide = Ci > 64 || Co > 64 ? 128 : 64;
-        const bool mixed = t == 64 && wide == 128 && V > 8 && n >= 65536;
-        if (es == 2 && n >= 8192 && n <= ((size_t)1 << 24) && t >= 64 && V <= 2 * (kCUs / 8) && Ci <= wide && Co <= wide && (wide == t || mixed)) {
+        // ... and 17 ... 32 channels on one side and 97 ... 128 on the other, four 32 x 32 tiles, from 131 072 voxels (32 -> 128, the product alone: 166 977
+        // voxels 107 and 82, 667 763 380 and 250; training with a fresh cache: 125 569 voxels 384 358, 166 789 424 379, 667 156 1026 955;
+        // 24 -> 72, three tiles: 125 569 voxels 310 316, 667 156 905 929).
+        const int narrow = Ci < Co ? Ci : Co, most = Ci < Co ? Co : Ci;
+        const bool mixed = wide == 128 && V > 8 && (t == 64 ? n >= 65536 : t == 32 && narrow > 16 && most > 96 && n >= 131072);
+        if (es == 2 && n >= 8192 && n <= ((size_t)1 << 24) && (t >= 64 || mixed) && V <= 2 * (kCUs / 8) && Ci <= wide && Co <= wide && (wide == t || mixed)) {
             out->tile_rows = out->tile_cols = wide;
             out->stream = 2;
             out->block_rows = 2048;
