@@ -7,9 +7,7 @@
 //     table    uint16 [kNarrowRows][32]   per (row, offset): byte offset, in the LDS row buffer, of the source row's first
 //                                         16-byte piece (a row's four pieces are exchanged by its slot number, see
 //                                         narrow_piece_key); the row of zeros when the neighbor is missing; entries from
-//                                         V to 30: the row of zeros, but for V = 27 entries 27, 28 and 29, which repeat 7,
-//                                         15 and 23 (the weight gradient's last multiplier takes seven offsets in one
-//                                         read); kNarrowOverflow when the chunk has more distinct sources than slots;
+//                                         V to 30: the row of zeros; kNarrowOverflow when the chunk has more distinct sources than slots;
 //                                         entry 31: whether any entry of the row is kNarrowOverflow
 //     sources  uint32 [kNarrowSlots]      source row of every slot, FGX_EMPTY32 beyond the chunk's count
 //     rows     uint32 [kNarrowRows]       the chunk's rows (output rows of the gather GEMM), FGX_EMPTY32 beyond n

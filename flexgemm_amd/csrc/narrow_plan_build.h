@@ -72,7 +72,9 @@ __device__ __forceinline__ void narrow_plan_chunk(NarrowPlanLds& lds, int V, boo
         const int e = tid + j * THREADS;
         mine_idx[j] = e < entries ? source_of(e) : FGX_EMPTY32;
     }
-    // first probes of all entries in flight together; the few that met another key go on from there
+    // first probes of all entries in flight together; the few that met another key go on from there.  An entry's place in the plan's table and its
+    // position in the hash table share a register: rows and offsets kept, or worked out a second time, cost wavefronts or time (2.67 M voxels, from
+    // the map: kept, with spills, 0.201 ms; a second time 0.167; so 0.164)
     int pos[kPerThread];
     uint32_t met[kPerThread];
 #pragma unroll
@@ -81,8 +83,12 @@ __device__ __forceinline__ void narrow_plan_chunk(NarrowPlanLds& lds, int V, boo
         met[j] = atomicCAS(&lds.keys[pos[j]], FGX_EMPTY32, mine_idx[j]);
     }
 #pragma unroll
-    for (int j = 0; j < kPerThread; ++j)
+    for (int j = 0; j < kPerThread; ++j) {
+        const int e = tid + j * THREADS;
         if (met[j] != FGX_EMPTY32 && met[j] != mine_idx[j]) pos[j] = insert(mine_idx[j], (uint32_t)(pos[j] + 1) & (kNarrowHash - 1));
+        pos[j] = ((e / V) * kNarrowTableStride + (e % V)) << 16 | (pos[j] & 0xFFFF);
+        asm("" : "+v"(pos[j]));
+    }
     __syncthreads();
     // the other sources: slots from `base` on in table order (exclusive scan of their positions, four per thread)
     const uint32_t base = own_rows ? (uint32_t)kNarrowRows : 0u;
@@ -124,11 +130,12 @@ __device__ __forceinline__ void narrow_plan_chunk(NarrowPlanLds& lds, int V, boo
         const int e = tid + j * THREADS;
         if (e >= entries) break;
         uint16_t out = (uint16_t)kNarrowZeroSlot;
-        if (pos[j] < kNarrowHash) out = pos[j] >= 0 ? lds.slot_of[pos[j]] : (uint16_t)kNarrowOverflow;
+        const int in_hash = (int)(int16_t)pos[j], in_table = pos[j] >> 16;
+        if (in_hash < kNarrowHash) out = in_hash >= 0 ? lds.slot_of[in_hash] : (uint16_t)kNarrowOverflow;
         // what the multipliers read: the byte offset of the row's logical piece 0 in the row buffer
         if (out != (uint16_t)kNarrowOverflow) out = (uint16_t)(out * 64u + (((uint32_t)out >> 2) & 3u) * 16u);
-        lds.table[(e / V) * kNarrowTableStride + (e % V)] = out;
-        if (out == (uint16_t)kNarrowOverflow) atomicOr(&lds.row_flags[(e / V) >> 5], 1u << ((e / V) & 31));
+        lds.table[in_table] = out;
+        if (out == (uint16_t)kNarrowOverflow) atomicOr(&lds.row_flags[in_table / kNarrowTableStride >> 5], 1u << (in_table / kNarrowTableStride & 31));
     }
     __syncthreads();
     for (int r = tid; r < kNarrowRows; r += THREADS)
