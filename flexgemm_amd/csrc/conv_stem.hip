@@ -41,7 +41,7 @@ struct StemCfg {
     static constexpr int IDX_SLOT = (IDX_BYTES + 1023) / 1024 * 1024;
     static constexpr int IDX_INST = IDX_SLOT / 1024, IDX_PER = (IDX_INST + kStemLoaders - 1) / kStemLoaders;
     static constexpr int STAGE = F_BYTES + G_BYTES;
-    static constexpr size_t LDS = (size_t)kStemStages * STAGE + kStemIdxSlots * IDX_SLOT;
+    static constexpr size_t LDS = (size_t)kStemStages * STAGE + kStemIdxSlots * IDX_SLOT + 16;    // ... and the word that asks for a second pass
     static_assert(F_INST % kStemLoaders == 0 && G_INST % kStemLoaders == 0 && F_BYTES % 1024 == 0, "every loader has as many loads");
     static_assert(NT_PER % 2 == 0, "fragments are waited for in fours");
     static_assert(LDS <= 160 * 1024, "LDS");
@@ -124,6 +124,7 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     unsigned char* ring = lds;                                 // [S][features | grad_out]
     unsigned char* idx_ring = lds + S * C::STAGE;              // [kStemIdxSlots] map rows
+    volatile uint32_t& again = *reinterpret_cast<volatile uint32_t*>(idx_ring + kStemIdxSlots * C::IDX_SLOT);       // some sum is not finite
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wave_m = wave & 1, wave_n = (wave >> 1) & 3;     // (of a multiplier)
@@ -145,7 +146,7 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
     const unsigned long long map_bytes = (unsigned long long)n * V * 4;
 
     // The loaders' walk over the steps; the multipliers meet them at its barriers.
-    auto load_run = [&]() __attribute__((always_inline)) {
+    auto load_run = [&](const int lane) __attribute__((always_inline)) {
         const int lw = wave - kStemWaves;
         StemPieces<P> pieces;
         pieces.init(lw, lane, V, [](int) { return 0; });
@@ -208,9 +209,9 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
     };
 
     f32x16 acc[C::NT_PER];
-    // APART: rows of grad_out that are not finite are added pair by pair (wgrad_device.h).  424 000 voxels 8 -> 48 channels, with the
-    // reduction: all finite 0.080 ms as without the second run, one row in a thousand infinite 0.165, every value 1.1 (the
-    // sums that are not finite taken again over all rows, by the reduction: 8.2 and 8.8).
+    // APART: rows of grad_out that are not finite are added pair by pair (wgrad_device.h).  428 946 voxels, with the reduction, us: 8 -> 48 channels
+    // all finite 33, one value infinite 86, a value in every thousandth row 90, every value 930;  16 -> 48 53, 120, 128, 1 460 (the
+    // sums that are not finite taken again over all rows, by the reduction, 8 -> 48: 8 200 and 8 800 for the last two).
     auto run = [&](auto apart_rows) __attribute__((always_inline)) {
         constexpr bool APART = decltype(apart_rows)::value;
 #pragma unroll
@@ -278,21 +279,25 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
             }
         }
     };
-    const bool loader = wave >= kStemWaves;                        // wave-uniform role
-    bool finite = true;
-    if (loader) {
+    if (tid == 0) again = 0u;                                      // (seen behind the first barrier of either side's run)
+    if (wave >= kStemWaves) {
         __builtin_amdgcn_s_setprio(3);
-        load_run();
-    } else {
-        run(std::false_type{});
+        for (int pass = 0; pass < 2; ++pass) {
+            int own = lane;                                        // (made anew: what follows from it is not kept in registers over both passes, and
+            asm volatile("" : "+v"(own));                          // beside a multiplier's sums; 32 of them spilled, 16 -> 48, one value infinite: 235 us)
+            load_run(own);
+            if (pass == 0) __syncthreads();
+            if (again == 0u) break;
+        }
+        return;
+    }
+    run(std::false_type{});
+    bool finite = true;
 #pragma unroll
-        for (int t = 0; t < C::NT_PER; ++t) finite = finite && all_finite(acc[t]);
-    }
-    if (__syncthreads_or(!finite)) {
-        if (loader) load_run();
-        else run(std::true_type{});
-    }
-    if (loader) return;
+    for (int t = 0; t < C::NT_PER; ++t) finite = finite && all_finite(acc[t]);
+    if (__any(!finite) && lane == 0) again = 1u;
+    __syncthreads();                                               // (the loaders' after their first pass)
+    if (again != 0u) run(std::true_type{});
 
     // partial[column tile][group][64][N]
     float* dst = partial + ((size_t)blockIdx.y * groups + group) * ((size_t)kStemCols * C::N);
