@@ -507,6 +507,9 @@ extern "C" {
 // save from 4.5 MB on, and by 5 MB also the 30 to 50 us of tables that a fresh cache is spared (64 x 256, cache and one layer, 27 200 rows: forward
 // 248 230, training 552 543;  38 400 rows: 354 325, 765 750;  24 400 rows, training 500 459).  Beyond: 96 x 96, 71 359 rows 244 250,
 // 84 634 rows 250 297;  128 x 128 438 378, 451 453;  160 x 160 595 617, 732 739;  256 x 96, 99 042 rows 857 631.
+// Up to 8 offsets, whose masks the sort brings together almost without padding: 45 000 rows, under at most half as many columns 65 536 (2 x 2 x 2,
+// stride 2, one layer, its cache kept: 96 x 96, 60 500 rows 56 77, 76 600 rows 67 91;  128 x 128 132 105, 107 131;  96 x 192, 48 000 rows 82 101;
+// 128 x 64, 64 600 rows 93 68, 76 600 rows 68 78;  256 x 128 180 179, 201 216).
 //   K x columns    855 rows   8 589    15 474    24 372    38 323    48 203    63 137      up to
 //     64 x   64      16  13    38  29    54  38    67  55    89  75   111  87   111 112      45 000 rows
 //     64 x  256      23  17    96  66   116 108   192 178   259                               25 720 (the sums' bound)
@@ -523,7 +526,8 @@ int fgx_conv_gemm_pairs_pays(int dtype, int mode, size_t n, int Ci, int Co, int 
     if (Ci % (16 / es) != 0 || Co % (16 / es) != 0 || (size_t)V * Ci * Co * es >= ((size_t)1 << 31)) return 0;
     if (n > 98304 || fgx_conv_gemm_pairs_scratch_bytes(n, cols, V) > ((size_t)1 << 30)) return 0;
     if (es == 4) {
-        const size_t rows = K == 64 ? 45000 : cols * 2 <= K ? 98304 : 65536;
+        const bool half = cols * 2 <= K;
+        const size_t rows = K == 64 ? 45000 : V <= 8 ? (half ? 65536 : 45000) : half ? 98304 : 65536;
         return K >= 64 && n <= rows && 0.45 * (double)fgx_conv_gemm_pairs_scratch_bytes(n, cols, V) <= 5e6 * K;
     }
     return K >= 256 && cols >= 64 && cols <= 2 * K && n <= (cols <= K ? 6000u : 5000u);

@@ -135,15 +135,16 @@ def test_rows_up_to_which_it_is_taken(dtype, k, cols, rows):
         assert takes == [rows > 0, rows > 0, False]
 
 
-# fp32 of more than 64 channels: up to 65 536 rows, 98 304 under at most half as many columns; the sums' bounds
-@pytest.mark.parametrize("k,cols,v,rows", [(68, 68, 27, 65536), (96, 96, 27, 65536), (128, 64, 27, 98304), (128, 68, 27, 65536), (256, 128, 27, 77672), (256, 128, 8, 98304),
-                                           (96, 192, 27, 51440)])
+# fp32 of more than 64 channels: up to 65 536 rows, 98 304 under at most half as many columns, fewer where the masked kernels hardly pad (up to 8
+# offsets); the sums' bounds
+@pytest.mark.parametrize("k,cols,v,rows", [(68, 68, 27, 65536), (96, 96, 27, 65536), (128, 64, 27, 98304), (128, 68, 27, 65536), (256, 128, 27, 77672),
+                                           (96, 192, 27, 51440), (96, 96, 9, 65536), (96, 96, 8, 45000), (128, 192, 8, 45000), (96, 48, 8, 65536), (256, 128, 8, 65536)])
 def test_rows_up_to_which_fp32_takes_it(k, cols, v, rows):
     for mode in (0, 1, 2):
         ci, co = (k, cols) if mode == 0 else (cols, k)
         takes = [bool(nat.lib().fgx_conv_gemm_pairs_pays(C.c_int(nat.DTYPE_CODE[torch.float32]), C.c_int(mode), nat.sz(n), C.c_int(ci), C.c_int(co), C.c_int(v)))
-                 for n in (1, 45001, rows, rows + 1)]
-        assert takes == [True, True, True, False]
+                 for n in (1, 45000, rows, rows + 1, 98305)]
+        assert takes == [True, True, True, False, False]
 
 
 @pytest.mark.gpu
