@@ -501,17 +501,22 @@ extern "C" {
 //   1024 x  128      33  18   35  22   48  30   73  34   74  45              1024 x 2048   447 379   809 480   814 542   829 609
 // 64 columns (256 x 64: 15 12, 20 14, 24 19, 33 20, 34 21) gain little more than the plan: a training step whose input gradient still wants the
 // masks is up to 5 % slower for it, a pass at inference 1.16 to 1.44 times as fast.
-// fp32 multiplies a sixteenth as fast and what is not multiplied counts for more: from 64 channels and up to 65 536 rows (98 304 under at most half
-// as many columns as channels; 64 channels 45 000, which tests pin: 48 203 rows, training with the cache 381 294), as long as the sums,
+// fp32 multiplies a sixteenth as fast and what is not multiplied counts for more: from 64 channels on, up to a number of rows and as long as the sums,
 // with 0.45 of a row's offsets, stay below 5 MB a channel.  Their traffic, which outgrows the 256 MB memory-side cache, costs what the products
 // save from 4.5 MB on, and by 5 MB also the 30 to 50 us of tables that a fresh cache is spared (64 x 256, cache and one layer, 27 200 rows: forward
 // 248 230, training 552 543;  38 400 rows: 354 325, 765 750;  24 400 rows, training 500 459).  Beyond: 96 x 96, 71 359 rows 244 250,
 // 84 634 rows 250 297;  128 x 128 438 378, 451 453;  160 x 160 595 617, 732 739;  256 x 96, 99 042 rows 857 631.
-// Up to 8 offsets, whose masks the sort brings together almost without padding: 45 000 rows, under at most half as many columns 65 536 (2 x 2 x 2,
-// stride 2, one layer, its cache kept: 96 x 96, 60 500 rows 56 77, 76 600 rows 67 91;  128 x 128 132 105, 107 131;  96 x 192, 48 000 rows 82 101;
-// 128 x 64, 64 600 rows 93 68, 76 600 rows 68 78;  256 x 128 180 179, 201 216).
+// Kernels of more than 8 offsets: 65 536 rows, 98 304 under at most half as many columns as channels.  The masked kernels multiply whole slabs of 32
+// channels, two of which 64 channels fill where 65 ... 96 are padded to three: 28 800 and 32 768 rows a slab (one layer, its cache included or kept,
+// inference fresh, kept, training fresh, kept:  64 x 64, 56 428 rows 165 126, 106 103, 375 334, 292 289, 64 090 rows 166 139, 105 117, 383 375, 299 326;
+// 64 x 32, 56 428 rows 124 105, 75 80, 305 321, 223 226, 96 531 rows 174 165, 119 131, 431 466, 331 350;  72 x 72, 64 090 rows 269 204, 206 179,
+// 658 569, 570 516, 83 458 rows 277 274, 210 242, 713 742, 621 679;  72 x 32, 83 458 rows 186 161, 134 131, 524 539, 431 433;  128 x 32 249 210, 196 179,
+// 613 619, 523 508).
+// Up to 8 offsets, whose masks the sort brings together almost without padding: 45 000 rows, under at most half as many columns 65 536, 22 500 a slab (2 x 2 x 2,
+// stride 2, kept: 96 x 96, 60 500 rows 56 77, 76 600 rows 67 91;  128 x 128 132 105, 107 131;  96 x 192, 48 000 rows 82 101;  64 x 64, 48 149 input rows,
+// training 56 60, 54 406 rows 58 88;  128 x 64, 64 600 rows 93 68, 76 600 rows 68 78;  256 x 128 180 179, 201 216;  64 x 32, fresh, 48 000 rows 95 102).
 //   K x columns    855 rows   8 589    15 474    24 372    38 323    48 203    63 137      up to
-//     64 x   64      16  13    38  29    54  38    67  55    89  75   111  87   111 112      45 000 rows
+//     64 x   64      16  13    38  29    54  38    67  55    89  75   111  87   111 112      57 600 rows
 //     64 x  256      23  17    96  66   116 108   192 178   259                               25 720 (the sums' bound)
 //     96 x   96      21  15    66  39   108  62   158  87   157 126   260 158   244 217      65 536
 //     96 x  192      27  18   104  64   151 101   217 153   260 263   356 330   365          51 440 (the sums' bound)
@@ -526,8 +531,10 @@ int fgx_conv_gemm_pairs_pays(int dtype, int mode, size_t n, int Ci, int Co, int 
     if (Ci % (16 / es) != 0 || Co % (16 / es) != 0 || (size_t)V * Ci * Co * es >= ((size_t)1 << 31)) return 0;
     if (n > 98304 || fgx_conv_gemm_pairs_scratch_bytes(n, cols, V) > ((size_t)1 << 30)) return 0;
     if (es == 4) {
+        const size_t slabs = cdiv(K, 32);
         const bool half = cols * 2 <= K;
-        const size_t rows = K == 64 ? 45000 : V <= 8 ? (half ? 65536 : 45000) : half ? 98304 : 65536;
+        size_t rows = V <= 8 ? (half ? 22500 * slabs : 45000) : (half ? 32768 : 28800) * slabs;
+        if (rows > 65536 && (V <= 8 || !half)) rows = 65536;
         return K >= 64 && n <= rows && 0.45 * (double)fgx_conv_gemm_pairs_scratch_bytes(n, cols, V) <= 5e6 * K;
     }
     return K >= 256 && cols >= 64 && cols <= 2 * K && n <= (cols <= K ? 6000u : 5000u);

@@ -125,7 +125,7 @@ def test_operator_takes_it_and_agrees_with_the_masked_kernels(gpu_device, monkey
 
 
 @pytest.mark.parametrize("dtype,k,cols,rows", [(torch.float16, 256, 256, 6000), (torch.bfloat16, 512, 512, 6000), (torch.float16, 1024, 64, 6000), (torch.float16, 256, 512, 5000),
-                                               (torch.float16, 248, 256, 0), (torch.float16, 256, 56, 0), (torch.float16, 256, 520, 0), (torch.float32, 64, 64, 45000),
+                                               (torch.float16, 248, 256, 0), (torch.float16, 256, 56, 0), (torch.float16, 256, 520, 0), (torch.float32, 64, 64, 57600),
                                                (torch.float32, 64, 256, 25720), (torch.float32, 60, 64, 0), (torch.float32, 512, 512, 19418)])
 def test_rows_up_to_which_it_is_taken(dtype, k, cols, rows):
     for mode in (0, 1, 2):
@@ -135,10 +135,11 @@ def test_rows_up_to_which_it_is_taken(dtype, k, cols, rows):
         assert takes == [rows > 0, rows > 0, False]
 
 
-# fp32 of more than 64 channels: up to 65 536 rows, 98 304 under at most half as many columns, fewer where the masked kernels hardly pad (up to 8
-# offsets); the sums' bounds
-@pytest.mark.parametrize("k,cols,v,rows", [(68, 68, 27, 65536), (96, 96, 27, 65536), (128, 64, 27, 98304), (128, 68, 27, 65536), (256, 128, 27, 77672),
-                                           (96, 192, 27, 51440), (96, 96, 9, 65536), (96, 96, 8, 45000), (128, 192, 8, 45000), (96, 48, 8, 65536), (256, 128, 8, 65536)])
+# fp32: up to 65 536 rows, 98 304 under at most half as many columns, fewer where the masked kernels pad no slab (64 channels) or hardly a mask (up to
+# 8 offsets); the sums' bounds
+@pytest.mark.parametrize("k,cols,v,rows", [(64, 64, 27, 57600), (64, 36, 27, 57600), (64, 32, 27, 65536), (64, 8, 27, 65536), (68, 68, 27, 65536), (96, 96, 27, 65536),
+                                           (68, 32, 27, 98304), (128, 64, 27, 98304), (128, 68, 27, 65536), (256, 128, 27, 77672), (96, 192, 27, 51440), (96, 96, 9, 65536),
+                                           (64, 64, 8, 45000), (64, 32, 8, 45000), (96, 96, 8, 45000), (128, 192, 8, 45000), (96, 48, 8, 65536), (256, 128, 8, 65536)])
 def test_rows_up_to_which_fp32_takes_it(k, cols, v, rows):
     for mode in (0, 1, 2):
         ci, co = (k, cols) if mode == 0 else (cols, k)
