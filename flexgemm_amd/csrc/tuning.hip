@@ -315,13 +315,17 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
     // Up to 32 columns under rows of 256 bytes and more: from 320 000 voxels, where it is ahead with the tables of a fresh cache too (cache and
     // one layer, tiled 64 x 32 and 256 x 32: 128 -> 16 channels, 329 832 voxels 261 252 us, 1 053 495 970 891; 272 -> 32 484 456, 2 190 1 795;
     // 512 -> 16 723 696.  299 416 voxels: 512 -> 16 659 661, 128 -> 16 246 240;  166 789: 405 426 and 167 171.  With a kept cache
-    // 1.1 to 1.4 times as fast from 320 000 on).
+    // 1.1 to 1.4 times as fast from 320 000 on).  Not under few offsets, whose products do not pay for those tables: up to 3 (128 -> 32 channels, 350 457 and
+    // 624 671 voxels, one layer at inference, fresh: 1 x 1 x 1 71 85 and 97 121, 3 x 1 x 1 94 103 and 135 151, where 2 x 2 x 2 has 461 433), and for input
+    // gradients up to 8, of which a stride leaves one or two (2 x 2 x 2 under a stride of 2, 16 -> 128, training, fresh: 350 457 inputs 257 285,
+    // 1 057 251 448 514; kept 96 95 and 232 202).
+    const bool tables_pay = n >= 320000 && V > (pass_kind == 1 ? 8 : 3);
     struct Shape { int rows, cols, slab; double rate; };
     const Shape shapes[] = {{128, 256, 128, 1.0}, {256, 128, slab, 0.95}, {256, 64, slab, 0.6}, {256, 32, 64, 0.5}};
     double best = 0.0;
     for (const Shape& sh : shapes) {
         if (row_bytes < 64 || sh.slab > (int)align_up(row_bytes, 64)) continue;
-        if (sh.cols == 256 ? cols <= 128 || slab != 128 : (sh.cols == 128 ? cols <= 64 : (sh.cols == 64 ? cols <= 32 : cols > 32 || (row_bytes >= 256 && n < 320000)))) continue;
+        if (sh.cols == 256 ? cols <= 128 || slab != 128 : (sh.cols == 128 ? cols <= 64 : (sh.cols == 64 ? cols <= 32 : cols > 32 || (row_bytes >= 256 && !tables_pay)))) continue;
         // (from ~1900 output columns on the staged bias does not fit beside the rings of the 256 x 128 tile; the other shapes,
         // whose rings leave a little more room, are no help under a weight that wide)
         if (!stream_lds_fits(sh.rows, sh.cols, sh.slab, cols) || (cols > 128 && !stream_lds_fits(256, 128, slab, cols))) continue;

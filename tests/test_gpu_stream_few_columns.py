@@ -13,6 +13,8 @@ def test_rows_from_which_it_streams(dtype, k, cols):
     for kind, ci, co in ((nat.PASS_FWD, k, cols), (nat.PASS_DGRAD, cols, k)):
         assert [nat.table_lookup(kind, dtype, n, ci, co, 27).stream for n in (319999, 320000, 3000000)] == [0, 1, 1]
         assert nat.table_lookup(kind, dtype, 320000, ci, co, 27).tile_cols == 32
+        # few offsets do not pay for its tables
+        assert [nat.table_lookup(kind, dtype, 320000, ci, co, v).stream for v in (1, 3, 4, 8, 9)] == ([0, 0, 0, 0, 1] if kind == nat.PASS_DGRAD else [0, 0, 1, 1, 1])
 
 
 @pytest.mark.gpu
