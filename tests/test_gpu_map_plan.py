@@ -24,18 +24,25 @@ def _build(coords, dims, dil, walk, plan):
 
 
 # rows that fill no chunk, one, one and a row; voxels given twice and outside the grid, which end the walk; a batch; columns that end inside a
-# brick; scattered voxels, of whose chunks some have more sources than slots
+# brick; scattered voxels (n = 0).  n < 0: a solid cube of so many cells a side inside the shell, of whose chunks some have more sources than
+# slots, and of the last one more than the builder's hash table
 @pytest.mark.gpu
 @pytest.mark.parametrize("dims,n,extra,dil", [((1, 300, 300, 300), 1, 0, (1, 1, 1)), ((1, 204, 204, 204), 127, 0, (1, 1, 1)), ((1, 204, 204, 204), 128, 0, (2, 1, 16)),
                                               ((3, 205, 210, 131), 129, 0, (1, 1, 1)), ((2, 204, 204, 233), 9000, 700, (1, 1, 1)), ((1, 230, 230, 230), 30000, 0, (1, 2, 3)),
-                                              ((1, 230, 230, 230), 0, 0, (1, 1, 1))])
+                                              ((1, 230, 230, 230), 0, 0, (1, 1, 1)), ((1, 230, 230, 230), -20, 0, (1, 1, 1)), ((1, 230, 230, 230), -20, 90, (2, 2, 2)),
+                                              ((1, 230, 230, 230), -40, 0, (4, 5, 7))])
 @pytest.mark.parametrize("order", ["scan", "shuffled"])
 def test_plan_beside_the_map(gpu_device, dims, n, extra, dil, order):
     print(f"[case] dims={dims} n={n} extra={extra} dilation={dil} {order}", flush=True)
-    rng = np.random.default_rng(n)
+    rng = np.random.default_rng(abs(n))
     base = reference_test_shell(96) + np.array([0, 50, 3, 30], np.int32)
     base[:, 0] = rng.integers(0, dims[0], len(base))
-    if n == 0:                                              # no two voxels near each other: every chunk has 128 rows and as many sources
+    solid = n < 0
+    if solid:
+        side = np.arange(-n, dtype=np.int32) + n // 2
+        cube = np.stack(np.meshgrid(0, side + 98, side + 51, side + 78, indexing="ij"), -1).reshape(-1, 4)
+        base = np.unique(np.concatenate([base, cube.astype(np.int32)]), axis=0)
+    elif n == 0:                                            # no two voxels near each other: every chunk has 128 rows and as many sources
         base = np.unique(rng.integers(0, dims, (4000, 4)).astype(np.int32), axis=0)
     elif n < len(base):
         base = base[:n] if n < 1000 else base[rng.choice(len(base), n, replace=False)]
@@ -53,7 +60,7 @@ def test_plan_beside_the_map(gpu_device, dims, n, extra, dil, order):
     got, want = _build(coords, dims, dil, walk, plan), _build(coords, dims, dil, alone, None)
     assert all(torch.equal(a, b) for a, b in zip(got, want)) and torch.equal(walk, alone)
     nmap, rows_of, raw = got[0].cpu().numpy().view(np.uint32), walk.cpu().numpy().view(np.uint32), plan.cpu().numpy()
-    chunks, overflowing = -(-n // ROWS), 0
+    chunks, overflowing, most = -(-n // ROWS), 0, 0
     stride = (len(raw) - HEADER) // chunks
     for c in range(chunks):
         one = raw[HEADER + c * stride:HEADER + (c + 1) * stride]
@@ -71,8 +78,13 @@ def test_plan_beside_the_map(gpu_device, dims, n, extra, dil, order):
         assert np.array_equal(table[:, STRIDE - 1] != 0, lost.any(1))
         # (a chunk's own rows are held first, whether or not they are anybody's neighbor)
         distinct = len(np.unique(np.concatenate([entries[entries != 0xFFFFFFFF], here])))
-        assert lost.any() == (distinct > SLOTS - (ROWS - len(here))) or distinct > SLOTS
+        room = SLOTS - (ROWS - len(here))
+        assert lost.any() == (distinct > room)
+        if distinct <= 1024:                                # (all of them found a place in the builder's table)
+            assert len(np.unique(np.concatenate([entries[held], here]))) == min(distinct, room)
         overflowing += bool(lost.any())
+        most = max(most, distinct)
+    assert (overflowing > 0) == solid and (most > 1024 or dil != (4, 5, 7))
     assert raw[:4].view(np.uint32)[0] == overflowing and not raw[4:HEADER].any()
 
 
