@@ -149,7 +149,7 @@ def test_rows_up_to_which_fp32_takes_it(k, cols, v, rows):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("ci,co,res", [(72, 72, 110), (128, 64, 156)])
+@pytest.mark.parametrize("ci,co,res", [(72, 72, 110), (128, 64, 156), (64, 64, 118)])
 def test_fp32_agrees_with_the_masked_kernels_at_many_rows(gpu_device, monkeypatch, ci, co, res):
     gen = torch.Generator(device=gpu_device).manual_seed(res)
     coords = torch.from_numpy(reference_test_shell(res)).to(gpu_device)
@@ -157,13 +157,26 @@ def test_fp32_agrees_with_the_masked_kernels_at_many_rows(gpu_device, monkeypatc
     print(f"[case] {n} rows {ci}->{co}", flush=True)
     shape = torch.Size([1, ci, res, res, res])
     weight = torch.randn(co, 3, 3, 3, ci, generator=gen, device=gpu_device) / (27 * ci) ** 0.5
-    feats = torch.randn(n, ci, generator=gen, device=gpu_device)
-    with torch.no_grad():
+    feats = torch.randn(n, ci, generator=gen, device=gpu_device).requires_grad_(True)
+    up = torch.randn(n, co, generator=gen, device=gpu_device)
+
+    def step():
         out, cache = spconv.sparse_submanifold_conv3d(feats, coords, shape, weight, None, None)
-        assert n > 45000 and "_pair_plan" in cache.__dict__
-        real = nat.table_lookup
-        monkeypatch.setattr(nat, "table_lookup", lambda *a, **k: real(*a, **k))         # (a table of the caller's keeps every shape on it)
-        want, other = spconv.sparse_submanifold_conv3d(feats, coords, shape, weight, None, None)
+        return out.detach(), torch.autograd.grad(out, feats, up)[0], cache
+
+    out, grad, cache = step()
+    assert n > 45000 and "_pair_plan" in cache.__dict__
+    real = nat.table_lookup
+    monkeypatch.setattr(nat, "table_lookup", lambda *a, **k: real(*a, **k))         # (a table of the caller's keeps every shape on it)
+    want, want_grad, other = step()
     assert "_pair_plan" not in other.__dict__
-    # sums of 27 ci products of about 1 / (27 ci) ** 0.5 and below 1: either order within 27 ci roundings of partial sums of a few
-    assert (out - want).abs().max() <= 2 * 27 * ci * 2.0 ** -24 * 4
+    # 64-bit sums of some rows: 27 ci (27 co) products, each rounded to 2 ** -24 of a sum that stays within the largest output
+    some = torch.randperm(n, generator=gen, device=gpu_device)[:2000]
+    near = cache.neighbor_map.view(torch.int32)[some].long()
+    w64 = weight.detach().reshape(co, 27, ci).double()
+    for got, masked, source, panel in ((out, want, feats.detach(), w64.permute(1, 2, 0)), (grad, want_grad, up, w64.flip(1).permute(1, 0, 2))):
+        exact = torch.zeros(2000, panel.shape[2], dtype=torch.float64, device=gpu_device)
+        for v in range(27):
+            exact += (source[near[:, v].clamp(min=0)].double() * (near[:, v:v + 1] >= 0)) @ panel[v].contiguous()
+        assert (got[some] - exact).abs().max() <= 1e-5 * exact.abs().max()
+        assert (got - masked).abs().max() <= 1e-5 * masked.abs().max()
