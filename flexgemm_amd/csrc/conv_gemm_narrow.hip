@@ -17,6 +17,7 @@
 // buffers (the loads run one chunk ahead), one barrier per chunk.  Persistent: XCD x walks the x-th eighth of the chunks, its workgroups interleave, so
 // that neighboring chunks -- which share their halo rows -- run on one L2 at one time.
 #include "gemm_device.h"
+#include "lane_swap.h"
 #include "narrow_plan_build.h"
 #include "narrow_walk.h"
 
@@ -347,19 +348,7 @@ constexpr int kN27Half = 13;                                   // offsets on eit
 constexpr int kN27BufferBytes = kNarrowRowBufPad + kNarrowTableBytes;
 constexpr int kN27SumBytes = 16 * 32 * 4;                      // what a wavefront hands over
 constexpr size_t kN27LdsBytes = (size_t)kWalkBuffers * kN27BufferBytes + 2 * (size_t)kWalkMult * kN27SumBytes + (size_t)kWalkMetas * kWalkMetaBytes + 128 + 2048;
-static_assert(kN27LdsBytes <= 160 * 1024, "LDS");
-
-// rows of 32 x 32 sums in two halves: a's lanes 32 - 63 and b's lanes 0 - 31 change places; a's odd runs of 16 lanes and b's even ones
-__device__ __forceinline__ void swap_halves(float& a, float& b) {
-    const auto both = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
-    a = __builtin_bit_cast(float, (uint32_t)both[0]);
-    b = __builtin_bit_cast(float, (uint32_t)both[1]);
-}
-__device__ __forceinline__ void swap_rows(float& a, float& b) {
-    const auto both = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
-    a = __builtin_bit_cast(float, (uint32_t)both[0]);
-    b = __builtin_bit_cast(float, (uint32_t)both[1]);
-}
+static_assert(kN27LdsBytes <= 160 * 1024 && narrow_lds_bytes(kNarrowCubeV) <= kN27LdsBytes, "LDS, also of narrow_gemm_any");
 
 // The offsets below the centre (HALF 0) or above it.
 template <typename Tag, int HALF>
@@ -491,7 +480,10 @@ narrow_gemm27_kernel(const typename Tag::type* __restrict__ src, const typename 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row_bytes = K * 2;
-    if (*reinterpret_cast<const uint32_t*>(plan) != 0u) {                      // chunks with sources that are not resident
+    // One chunk with sources that are not resident sends all of them to the four multipliers: reading such sources from memory wants registers that the
+    // weight takes here.  32 channels, forward and weight gradient, a solid cube of 20 cells a side in the middle of the surface: 2.67 M voxels
+    // 176 -> 209 us and 180 -> 367 (the weight gradient's kernel is another one then), 167 000 voxels 24 -> 40 and 27 -> 47.
+    if (*reinterpret_cast<const uint32_t*>(plan) != 0u) {
         if (tid < kNarrowThreads)
             narrow_gemm_any<Tag, V>(src, panel, bias, nmap, plan, chunks, plan_bytes, src_bytes, V, K, cols, activation, out, relu_mask, lds);
         return;

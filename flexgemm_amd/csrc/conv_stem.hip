@@ -12,6 +12,7 @@
 // 6 -> 48 channels 38 -> 29 us, 16 -> 48 67 -> 52.  A last piece per row holds a one: its column is the bias gradient.
 // A workgroup keeps all accumulators over its contiguous run of rows and writes one partial product; a second kernel adds the
 // partial products in workgroup order (same bits on every run).
+#include "lane_swap.h"
 #include "wgrad_device.h"
 
 namespace fgx {
@@ -363,18 +364,6 @@ struct StemGemmCfg {
     // XOR key on the low bits of a row's piece numbers: 16 rows' reads of one piece fall on distinct banks (rows are 28 or 56 pieces)
     static __device__ __forceinline__ int key(int row) { return P == 1 ? (row >> 2) & 3 : (row >> 1) & 7; }
 };
-
-// a's lanes 32 - 63 and b's lanes 0 - 31 change places; a's odd runs of 16 lanes and b's even ones.
-__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
-    const auto both = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-    a = both[0];
-    b = both[1];
-}
-__device__ __forceinline__ void swap_rows(uint32_t& a, uint32_t& b) {
-    const auto both = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-    a = both[0];
-    b = both[1];
-}
 
 // mode as in fgx_pack_weight: 0 weight [cols][V][K], 1 / 2 weight [K][V][cols] with mirrored offsets / as they are
 template <typename Tag, int P>

@@ -1,9 +1,8 @@
 // What the 3x3x3 kernels for narrow layers (conv_gemm_narrow.hip: forward and dgrad; wgrad_narrow.hip: weight gradient) share: the chunks
 // of a workgroup and the loading wavefronts' walk over them.
 //
-// A workgroup has eight multiplying wavefronts, two per SIMD, and four that only load.  With one multiplier per SIMD its products, its address
-// arithmetic, its waits for LDS and its stores stood in a row: 2.67 M voxels, 32 channels, matrix units busy 36 % (weight gradient 30 %) of
-// the time, LDS 52 % (27 %).
+// A workgroup has eight multiplying wavefronts (weight gradient: seven), two per SIMD, and four that only load.  With one multiplier per SIMD its
+// products, its address arithmetic, its waits for LDS and its stores stood in a row (figures: narrow_gemm27_kernel, narrow_wgrad27_kernel).
 //
 // Two chunks are on their way while one is multiplied.  A chunk's source and output row numbers (its "meta": the plan's sources and rows)
 // come two chunks earlier still, through a ring of their own in LDS: row numbers in registers would make the loads that need them wait for

@@ -376,38 +376,38 @@ __global__ void map_kernel(const int32_t* __restrict__ coords, GridIndex walk, s
 template <int K>
 __device__ __forceinline__ void brick_columns(const GridIndex& index, const GridPlace<false>& xp, bool x_ok, const bool (&y_ok)[K], const GridPlace<false> (&yp)[K],
                                               const bool (&z_ok)[K], const GridPlace<false> (&zp)[K], uint32_t z_first, uint32_t z_last, uint32_t (&value)[K][K]) {
-                // the column's cells ascend along z and span at most 32: they lie in the brick of the first one inside the grid or in
-                // that of the last one
-                ulonglong2 wa[K], wb[K];
-                uint32_t na[K], nb[K];
-    #pragma unroll
-                for (int ky = 0; ky < K; ++ky) {
-                    const bool column = x_ok && y_ok[ky];
-                    const uint32_t brick_a = column ? xp.brick + yp[ky].brick + z_first : 0u;
-                    wa[ky] = index.bits[brick_a];
-                    na[ky] = index.counts[brick_a];
-                    wb[ky] = make_ulonglong2(0ull, 0ull);
-                    nb[ky] = 0u;
-                    if (column && z_last != z_first) {
-                        wb[ky] = index.bits[xp.brick + yp[ky].brick + z_last];
-                        nb[ky] = index.counts[xp.brick + yp[ky].brick + z_last];
-                    }
-                }
-    #pragma unroll
-                for (int ky = 0; ky < K; ++ky) {
-                    uint32_t rank[K];
-                    bool have[K];
-    #pragma unroll
-                    for (int kz = 0; kz < K; ++kz) {
-                        const bool in_a = zp[kz].brick == z_first;
-                        const ulonglong2 w = make_ulonglong2(in_a ? wa[ky].x : wb[ky].x, in_a ? wa[ky].y : wb[ky].y);
-                        const uint32_t at = (xp.at + yp[ky].at + zp[kz].at) & 127u;
-                        have[kz] = x_ok && y_ok[ky] && z_ok[kz] && (((at & 64u ? w.y : w.x) >> (at & 63u)) & 1ull);
-                        rank[kz] = (in_a ? na[ky] : nb[ky]) + bits_before(w, at);
-                    }
-    #pragma unroll
-                    for (int kz = 0; kz < K; ++kz) value[ky][kz] = have[kz] ? index.rows[rank[kz]] : FGX_EMPTY32;
-                }
+    // the column's cells ascend along z and span at most 32: they lie in the brick of the first one inside the grid or in
+    // that of the last one
+    ulonglong2 wa[K], wb[K];
+    uint32_t na[K], nb[K];
+#pragma unroll
+    for (int ky = 0; ky < K; ++ky) {
+        const bool column = x_ok && y_ok[ky];
+        const uint32_t brick_a = column ? xp.brick + yp[ky].brick + z_first : 0u;
+        wa[ky] = index.bits[brick_a];
+        na[ky] = index.counts[brick_a];
+        wb[ky] = make_ulonglong2(0ull, 0ull);
+        nb[ky] = 0u;
+        if (column && z_last != z_first) {
+            wb[ky] = index.bits[xp.brick + yp[ky].brick + z_last];
+            nb[ky] = index.counts[xp.brick + yp[ky].brick + z_last];
+        }
+    }
+#pragma unroll
+    for (int ky = 0; ky < K; ++ky) {
+        uint32_t rank[K];
+        bool have[K];
+#pragma unroll
+        for (int kz = 0; kz < K; ++kz) {
+            const bool in_a = zp[kz].brick == z_first;
+            const ulonglong2 w = make_ulonglong2(in_a ? wa[ky].x : wb[ky].x, in_a ? wa[ky].y : wb[ky].y);
+            const uint32_t at = (xp.at + yp[ky].at + zp[kz].at) & 127u;
+            have[kz] = x_ok && y_ok[ky] && z_ok[kz] && (((at & 64u ? w.y : w.x) >> (at & 63u)) & 1ull);
+            rank[kz] = (in_a ? na[ky] : nb[ky]) + bits_before(w, at);
+        }
+#pragma unroll
+        for (int kz = 0; kz < K; ++kz) value[ky][kz] = have[kz] ? index.rows[rank[kz]] : FGX_EMPTY32;
+    }
 }
 
 // The same for K x K x K kernels, K = 2 or 3: K wavefronts for 64 rows, a row per lane and a plane of the kernel per wavefront, which asks its K columns
@@ -415,8 +415,8 @@ __device__ __forceinline__ void brick_columns(const GridIndex& index, const Grid
 // against what a CU holds in flight: one column per wavefront, as above, took 0.261 ms for 2 667 120 voxels of a surface in scan order (3x3x3, map
 // and codes, 331 MB read and written), all planes in one wavefront 0.136 (sort and merge: 0.331).  So against that: 434 000 voxels 25.0 -> 21.7 us, of which
 // the map and its codes leave at 2.3 TB/s; 67 000 outputs under a stride of 2 12.7 -> 10.0; 3 758 voxels 5.6 -> 4.3; 667 763 voxels in random order
-// 64 -> 59; 2.55 M voxels in scan order level, in random order 241 -> 248, where the scattered 108-byte rows bound it (a plain scatter: 0.26 ms for
-// 2 667 120).  In the `bits` form a column's cells have to lie in two bricks: columns longer than 32 cells go to the general kernel.
+// 64 -> 59; from 2 million voxels on level in either order, in random order because the scattered 108-byte rows bound it (2.54 and 2.67 M voxels 249 and
+// 250 us; a plain scatter: 0.26 ms for 2 667 120).  In the `bits` form a column's cells have to lie in two bricks: columns longer than 32 cells go to the general kernel.
 template <bool DENSE, int MODE, int K>
 __global__ void __launch_bounds__(64 * K) cube_map_kernel(const int32_t* __restrict__ coords, GridIndex walk, size_t n,
                                                       GridIndex index, GridIndex own, int own_dense, QueryGeom g, uint32_t* __restrict__ out_map,

@@ -130,11 +130,14 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
         // 33 ... 64 channels on one side and 65 ... 128 on the other: the 128 x 128 tile, half of it empty, from 65 536 voxels and under kernels of more than
         // 8 offsets (the product alone, us: 64 -> 128, 166 977 voxels 107 and 84, 667 763 453 and 269; 38 407 45 and 44;  training with a fresh cache,
         // its plan included: 65 145 voxels 269 256, 166 789 405 389, 667 156 1130 997; 128 -> 64, 50 850 kept 115 117; under
-        // 2 x 2 x 2, 180 000 outputs fresh 366 381).
+        // 2 x 2 x 2, 180 000 outputs fresh 366 381).  The narrow end of the range gains as much, though more of the tile is empty, since the other kernel's two
+        // 64 x 64 tiles pad as well (alone, and with cache and plan: 40 -> 72, 67 107 voxels 65 56, 199 185; 167 946 137 93, 299 242, in random order
+        // 138 89, 317 258; 667 763 442 254, 636 489; 72 -> 64, 67 107 64 55, 194 183; 667 763 448 250, 650 482).
         const int wide = Ci > 64 || Co > 64 ? 128 : 64;
         // ... and 17 ... 32 channels on one side and 97 ... 128 on the other, four 32 x 32 tiles, from 131 072 voxels (32 -> 128, the product alone: 166 977
         // voxels 107 and 82, 667 763 380 and 250; training with a fresh cache: 125 569 voxels 384 358, 166 789 424 379, 667 156 1026 955;
-        // 24 -> 72, three tiles: 125 569 voxels 310 316, 667 156 905 929).
+        // 24 -> 72, three tiles: 125 569 voxels 310 316, 667 156 905 929;  24 -> 104, alone, and with cache and plan: 166 977 voxels 121 79, 291 230, in random
+        // order 141 86, 331 253; 667 763 387 261, 575 482; 128 -> 24, 166 977 99 82, 268 229).
         const int narrow = Ci < Co ? Ci : Co, most = Ci < Co ? Co : Ci;
         const bool mixed = wide == 128 && V > 8 && (t == 64 ? n >= 65536 : t == 32 && narrow > 16 && most > 96 && n >= 131072);
         if (es == 2 && n >= 8192 && n <= ((size_t)1 << 24) && (t >= 64 || mixed) && V <= 2 * (kCUs / 8) && Ci <= wide && Co <= wide && (wide == t || mixed)) {
