@@ -340,7 +340,7 @@ narrow_gemm_kernel(const typename Tag::type* __restrict__ src, const typename Ta
 // a wavefront hands over the sums of one half of its rows and finishes the other's, at the start of the next iteration, when the barrier
 // between the two has been met anyway; the 16 x 32 sums a wavefront finishes leave as one store of whole 64-byte rows.
 // 2 667 120 voxels, 32 channels: 0.182 ms -> 0.152 in scan order, 0.191 -> 0.160 in random order; 166 977 voxels 17.9 -> 15.9 us; 667 763 voxels, 16
-// channels 39.3 -> 35.9.  Loads and stores alone take 0.117 ms (582 MB at 5 TB/s, 219 of them the plan); what is left are the two multipliers of a
+// channels 39.3 -> 35.9; 8 and 16 channels up to 90 000 rows, a chunk or two a workgroup, wait for the longer start, 10.2 -> 10.6.  Loads and stores alone take 0.117 ms (582 MB at 5 TB/s, 219 of them the plan); what is left are the two multipliers of a
 // SIMD, which do not cover each other's waits altogether.  Leaving out the offsets that none of a tile's 32 rows has (7 of 27) costs in
 // branches what it saves in products; registers for a second offset's fragments ahead change nothing.
 constexpr int kAhead = 1;                                      // (offsets whose fragments are read ahead: registers for one)
