@@ -17,8 +17,8 @@
 // products, and a second kernel adds them in workgroup order (fixed order: same bits on every run).
 // An infinity or NaN in grad_out times the row of zeros is NaN where the sum over the pairs has no term: a workgroup whose sums are not
 // all finite goes over its chunks again and adds such rows of grad_out pair by pair, until every sum is NaN (wgrad_device.h).  2.67 M
-// voxels, 32 channels, with four multipliers: all finite 0.240 ms (0.236 without the second pass), one row in a thousand infinite 0.75, every value 0.95; most
-// where no sum ends as NaN, 6.1.
+// voxels, 32 channels: all finite 0.165 ms, one value infinite 0.58, a value in every thousandth row 0.61, every value 0.51 (with four multipliers 0.236,
+// 0.65, 0.67, 0.80; most where no sum ends as NaN, 6.1).
 // The bias gradient comes for nothing: the offsets from V on are multiplied for no one, and the last of them by ones.  Column sums of
 // their own read grad_out once more (2.67 M voxels, 32 channels: 29 us a layer and 4 for their reduction; a training pass of two
 // layers 2.084 -> 2.022 ms).
