@@ -13,6 +13,8 @@
 // fgx_pair_plan lists the pairs: per offset how many, their source rows in row order, and for each (row, offset) its place in the
 // offset's list.  Nothing is read back: the launch covers the most tiles there can be, and a workgroup finds its tile -- or that
 // there is none for it -- from the counts.
+#include <type_traits>
+
 #include "gemm_device.h"
 #include "lds_read.h"
 
@@ -204,10 +206,12 @@ struct PairCfg {
 // 864 voxels x 1024 channels (11 022 pairs, 57 MB of weight) 44 us, 513 TFLOP/s; 3 758 voxels 146 us, 695 TFLOP/s.  Tiles of 128 x 256 and 256 x 128 on
 // eight wavefronts, rings of three to five slabs, slabs of 64 bytes, and loads by wavefronts of their own in a persistent workgroup came out between
 // 0.9 and 1.2 of that time, ahead only for the second, behind for everything smaller.
-// fp32 multiplies a sixteenth as fast: half as long a slab is enough work for a barrier, and its stages and fragments let four workgroups share a
-// CU, which cover the few slabs' start and end (96 channels have three of 128 bytes).  Products and sums, two workgroups of 128-byte slabs -> four of 64:
-// 38 407 voxels, 96 channels 141 -> 130 us, and 125 with the sums leaving in bands of 32 columns, which no longer set the LDS a workgroup takes;
-// 8 589 voxels 42 -> 38; 15 467 voxels, 64 channels 38.8 -> 35.3; 3 758 voxels, 512 channels 245 -> 240.
+// fp32 multiplies three bf16 parts of every value (split3.h), six products for one: half as long a slab is enough work for a barrier, and its
+// stages and fragments let four workgroups share a CU, which cover the few slabs' start and end (96 channels have three of 128 bytes). It is bound by making
+// the parts (176 vector instructions to 18 products of a wavefront's 32 x 96) and by what it writes: 38 407 voxels, 96 channels, with the sums
+// 130 us on the fp32 units (141 in two workgroups of 128-byte slabs, 125 with the sums leaving in bands of 32 columns), 105 in parts; 16 307 voxels,
+// 128 channels 76 -> 66, 256 channels 227 -> 194; error against 64 bits 1.90e-7 -> 1.58e-7. A tile with a sum that the parts cannot stand for is multiplied
+// a second time, on the fp32 units.
 template <typename Tag, bool TR, int BN, int WAVES_M>
 __global__ void __launch_bounds__(256, pair_groups((int)sizeof(typename Tag::type)))
 pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const uint32_t* __restrict__ plan, uint32_t n, int K, int cols,
@@ -260,7 +264,7 @@ pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const
             b_off[i] = col < BN && col0 + col < cols ? (uint32_t)(col0 + col) * b.line_stride + b_at[i] : kOobOffset;
         }
     }
-    uint32_t b_soff = (uint32_t)wv * b.v_stride;
+    uint32_t b_soff = 0;
     auto issue = [&](int slab) {
         unsigned char* stage = ring + (slab & 1) * C::STAGE;
         const bool tail = ragged && slab == slabs - 1;
@@ -299,66 +303,102 @@ pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const
             }
         }
     f32x16 acc[C::TM][C::TN];
+    auto multiply = [&](auto on_fp32_units) __attribute__((always_inline)) {
+        constexpr bool SPLIT = C::ES == 4 && !decltype(on_fp32_units)::value;
+        b_soff = (uint32_t)wv * b.v_stride;
 #pragma unroll
-    for (int i = 0; i < C::TM; ++i)
+        for (int i = 0; i < C::TM; ++i)
 #pragma unroll
-        for (int j = 0; j < C::TN; ++j)
+            for (int j = 0; j < C::TN; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-    issue(0);
-    if (slabs > 1) issue(1);
-    for (int s = 0; s < slabs; ++s) {
-        if (s + 1 < slabs) wait_vmcnt<C::LPS>();        // all but the newest slab's loads have landed
-        else wait_vmcnt<0>();
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        const unsigned char* cur = ring + (s & 1) * C::STAGE;
-        u32x4 af[CH / 2][C::TM], bf[CH / 2][C::TN];
-        i16x4 tr[TR && C::ES == 2 ? CH * C::TN : 4];
-#pragma unroll
-        for (int kk = 0; kk < CH / 2; ++kk) {
-#pragma unroll
-            for (int i = 0; i < C::TM; ++i) af[kk][i] = *(const u32x4*)(cur + a_frag[kk][i]);
-#pragma unroll
-            for (int j = 0; j < C::TN; ++j) {
-                if constexpr (TR && C::ES == 2) {       // (K rows 4 apart share a key)
-                    tr[(kk * C::TN + j) * 2] = lds_read_tr16(cur + b_frag[kk][j]);
-                    tr[(kk * C::TN + j) * 2 + 1] = lds_read_tr16(cur + b_frag[kk][j] + 4 * C::TCH * 16);
-                } else if constexpr (TR) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) bf[kk][j][e] = *(const uint32_t*)(cur + b_frag[kk][j] + e * C::TCH * 16);
-                } else {
-                    bf[kk][j] = *(const u32x4*)(cur + b_frag[kk][j]);
-                }
-            }
-        }
-        if constexpr (TR && C::ES == 2) {
-            lds_wait_all(tr);
-#pragma unroll
-            for (int kk = 0; kk < CH / 2; ++kk)
-#pragma unroll
-                for (int j = 0; j < C::TN; ++j)
-                    bf[kk][j] = __builtin_bit_cast(u32x4, __builtin_shufflevector(tr[(kk * C::TN + j) * 2], tr[(kk * C::TN + j) * 2 + 1], 0, 1, 2, 3, 4, 5, 6, 7));
-        }
-        if (s + 2 < slabs) {
-            // every wavefront's fragments are in registers before the stage is written again
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        issue(0);
+        if (slabs > 1) issue(1);
+        for (int s = 0; s < slabs; ++s) {
+            if (s + 1 < slabs) wait_vmcnt<C::LPS>();        // all but the newest slab's loads have landed
+            else wait_vmcnt<0>();
+            asm volatile("" ::: "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            issue(s + 2);
+            const unsigned char* cur = ring + (s & 1) * C::STAGE;
+            u32x4 af[CH / 2][C::TM], bf[CH / 2][C::TN];
+            i16x4 tr[TR && C::ES == 2 ? CH * C::TN : 4];
+#pragma unroll
+            for (int kk = 0; kk < CH / 2; ++kk) {
+#pragma unroll
+                for (int i = 0; i < C::TM; ++i) af[kk][i] = *(const u32x4*)(cur + a_frag[kk][i]);
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j) {
+                    if constexpr (TR && C::ES == 2) {       // (K rows 4 apart share a key)
+                        tr[(kk * C::TN + j) * 2] = lds_read_tr16(cur + b_frag[kk][j]);
+                        tr[(kk * C::TN + j) * 2 + 1] = lds_read_tr16(cur + b_frag[kk][j] + 4 * C::TCH * 16);
+                    } else if constexpr (TR) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) bf[kk][j][e] = *(const uint32_t*)(cur + b_frag[kk][j] + e * C::TCH * 16);
+                    } else {
+                        bf[kk][j] = *(const u32x4*)(cur + b_frag[kk][j]);
+                    }
+                }
+            }
+            if constexpr (TR && C::ES == 2) {
+                lds_wait_all(tr);
+#pragma unroll
+                for (int kk = 0; kk < CH / 2; ++kk)
+#pragma unroll
+                    for (int j = 0; j < C::TN; ++j)
+                        bf[kk][j] = __builtin_bit_cast(u32x4, __builtin_shufflevector(tr[(kk * C::TN + j) * 2], tr[(kk * C::TN + j) * 2 + 1], 0, 1, 2, 3, 4, 5, 6, 7));
+            }
+            if (s + 2 < slabs) {
+                // every wavefront's fragments are in registers before the stage is written again
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                issue(s + 2);
+            }
+            if constexpr (SPLIT) {
+#pragma unroll
+                for (int kk = 0; kk < CH / 2; kk += 2) {        // (16 values of K a product)
+                    Split3 rows3[C::TM];
+#pragma unroll
+                    for (int i = 0; i < C::TM; ++i) rows3[i] = split3(af[kk][i], af[kk + 1][i]);
+#pragma unroll
+                    for (int j = 0; j < C::TN; ++j) {
+                        const Split3 cols3 = split3(bf[kk][j], bf[kk + 1][j]);
+#pragma unroll
+                        for (int i = 0; i < C::TM; ++i) mma_split3(acc[i][j], cols3, rows3[i]);     // transposed tile
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int kk = 0; kk < CH / 2; ++kk)
+#pragma unroll
+                    for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                        for (int j = 0; j < C::TN; ++j) mma<Tag>(acc[i][j], bf[kk][j], af[kk][i]);      // transposed tile
+            }
         }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();           // the ring is reused below
+        asm volatile("" ::: "memory");
+    };
+    multiply(std::false_type{});
+    if constexpr (C::ES == 4) {
+        bool fine = true;
 #pragma unroll
-        for (int kk = 0; kk < CH / 2; ++kk)
+        for (int i = 0; i < C::TM; ++i)
 #pragma unroll
-            for (int i = 0; i < C::TM; ++i)
+            for (int j = 0; j < C::TN; ++j)
 #pragma unroll
-                for (int j = 0; j < C::TN; ++j) mma<Tag>(acc[i][j], bf[kk][j], af[kk][i]);      // transposed tile
+                for (int e = 0; e < 16; ++e) fine = fine && split3_holds(acc[i][j][e]);
+        volatile uint32_t* told = (volatile uint32_t*)ring;
+        const bool all = __ballot(!fine) == 0;
+        if (lane == 0) told[wave] = all;
+        __syncthreads();
+        const bool every = told[0] & told[1] & told[2] & told[3];
+        __syncthreads();
+        if (!every) multiply(std::true_type{});
     }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();           // the ring is reused below
-    asm volatile("" ::: "memory");
 
     // element e of lane l: pair l % 32, column 8 * (e / 4) + 4 * (l / 32) + e % 4.  Through the wavefront's band in LDS, 32 columns at a time, out as
     // 16-byte pieces of 128 bytes a pair.
@@ -501,7 +541,8 @@ extern "C" {
 //   1024 x  128      33  18   35  22   48  30   73  34   74  45              1024 x 2048   447 379   809 480   814 542   829 609
 // 64 columns (256 x 64: 15 12, 20 14, 24 19, 33 20, 34 21) gain little more than the plan: a training step whose input gradient still wants the
 // masks is up to 5 % slower for it, a pass at inference 1.16 to 1.44 times as fast.
-// fp32 multiplies a sixteenth as fast and what is not multiplied counts for more: from 64 channels on, up to a number of rows and as long as the sums,
+// fp32 (figures of the fp32 units on both sides; in three bf16 parts both are shorter, and level where they were: 49 829 rows, kept, 64 x 64 73 75, 96 x 96
+// 145 121, 128 x 128 200 192, 160 x 160 301 319):  what is not multiplied counts for more than in 16 bits: from 64 channels on, up to a number of rows and as long as the sums,
 // with 0.45 of a row's offsets, stay below 5 MB a channel.  Their traffic, which outgrows the 256 MB memory-side cache, costs what the products
 // save from 4.5 MB on, and by 5 MB also the 30 to 50 us of tables that a fresh cache is spared (64 x 256, cache and one layer, 27 200 rows: forward
 // 248 230, training 552 543;  38 400 rows: 354 325, 765 750;  24 400 rows, training 500 459).  Beyond: 96 x 96, 71 359 rows 244 250,

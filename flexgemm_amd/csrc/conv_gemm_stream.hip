@@ -405,24 +405,84 @@ gather_gemm_stream_kernel(const typename Tag::type* __restrict__ src, const type
             if (m_mine != 0) {
                 // band by band: a 32-row band of the wave tile none of whose rows has the offset is neither read nor
                 // multiplied (for a given accumulator the products still come in the order of the K-blocks)
-                u32x4 af[kChunks / 2][C::TM], bf[kChunks / 2][C::TN];
+                if constexpr (C::ES == 4) {
+                    // 16 values of K at a time, in three bf16 parts each: of a wavefront's time the parts take nearly as much as the products, which
+                    // the other wavefront of its SIMD fills
 #pragma unroll
-                for (int kk = 0; kk < kChunks / 2; ++kk)
+                    for (int kk = 0; kk < kChunks / 2; kk += 2) {
+                        Split3 cols3[C::TN];
 #pragma unroll
-                    for (int j = 0; j < C::TN; ++j) bf[kk][j] = *(const u32x4*)(cur + b_frag[kk][j]);
+                        for (int j = 0; j < C::TN; ++j)
+                            cols3[j] = split3(*(const u32x4*)(cur + b_frag[kk][j]), *(const u32x4*)(cur + b_frag[kk + 1][j]));
 #pragma unroll
-                for (int i = 0; i < C::TM; ++i) {
-                    if (C::TM > 1 && !((m_mine >> i) & 1u)) continue;
+                        for (int i = 0; i < C::TM; ++i) {
+                            if (C::TM > 1 && !((m_mine >> i) & 1u)) continue;
+                            const Split3 rows3 = split3(*(const u32x4*)(cur + a_frag[kk][i]), *(const u32x4*)(cur + a_frag[kk + 1][i]));
 #pragma unroll
-                    for (int kk = 0; kk < kChunks / 2; ++kk) af[kk][i] = *(const u32x4*)(cur + a_frag[kk][i]);
-                }
-#pragma unroll
-                for (int i = 0; i < C::TM; ++i) {
-                    if (C::TM > 1 && !((m_mine >> i) & 1u)) continue;
+                            for (int j = 0; j < C::TN; ++j) mma_split3(acc[i][j], cols3[j], rows3);     // transposed tile
+                        }
+                    }
+                } else {
+                    u32x4 af[kChunks / 2][C::TM], bf[kChunks / 2][C::TN];
 #pragma unroll
                     for (int kk = 0; kk < kChunks / 2; ++kk)
 #pragma unroll
-                        for (int j = 0; j < C::TN; ++j) mma<Tag>(acc[i][j], bf[kk][j], af[kk][i]);   // transposed tile
+                        for (int j = 0; j < C::TN; ++j) bf[kk][j] = *(const u32x4*)(cur + b_frag[kk][j]);
+#pragma unroll
+                    for (int i = 0; i < C::TM; ++i) {
+                        if (C::TM > 1 && !((m_mine >> i) & 1u)) continue;
+#pragma unroll
+                        for (int kk = 0; kk < kChunks / 2; ++kk) af[kk][i] = *(const u32x4*)(cur + a_frag[kk][i]);
+                    }
+#pragma unroll
+                    for (int i = 0; i < C::TM; ++i) {
+                        if (C::TM > 1 && !((m_mine >> i) & 1u)) continue;
+#pragma unroll
+                        for (int kk = 0; kk < kChunks / 2; ++kk)
+#pragma unroll
+                            for (int j = 0; j < C::TN; ++j) mma<Tag>(acc[i][j], bf[kk][j], af[kk][i]);   // transposed tile
+                    }
+                }
+            }
+        }
+
+        // fp32: a wave tile with a sum that the three-part products cannot stand for is multiplied again, on the fp32 units, from memory; the
+        // other wavefronts wait at the barrier below.
+        if constexpr (C::ES == 4) {
+            bool fine = true;
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) fine = fine && split3_holds(acc[i][j][e]);
+            if (__ballot(!fine) != 0) {
+#pragma unroll
+                for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+                uint32_t code = (uint32_t)tile_code[c_t];
+                const uint32_t* slot = plan_idx + (size_t)plan_seg[c_t] * BM + wave_m * C::WM + l32;
+                for (; code != 0; code &= code - 1, slot += BM) {
+                    const unsigned char* lines = (const unsigned char*)panel +
+                        ((size_t)(__builtin_ctz(code) * slabs) * cols_pad + c_ct * BN + wave_n * C::WN + l32) * kSlabBytes;
+#pragma unroll 1
+                    for (uint32_t at = g * 16; at < (uint32_t)(slabs * kSlabBytes); at += 32) {
+                        u32x4 line[C::TN];
+#pragma unroll
+                        for (int j = 0; j < C::TN; ++j)
+                            line[j] = *(const u32x4*)(lines + ((size_t)(at / kSlabBytes) * cols_pad + j * 32) * kSlabBytes + at % kSlabBytes);
+#pragma unroll
+                        for (int i = 0; i < C::TM; ++i) {
+                            const uint32_t m = slot[i * 32];
+                            u32x4 row = {0u, 0u, 0u, 0u};
+                            if (m != FGX_EMPTY32 && at < row_bytes) row = *(const u32x4*)((const unsigned char*)src + (size_t)m * row_bytes + at);
+#pragma unroll
+                            for (int j = 0; j < C::TN; ++j) mma<F32>(acc[i][j], line[j], row);
+                        }
+                    }
                 }
             }
         }

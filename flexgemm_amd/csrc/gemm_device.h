@@ -2,6 +2,7 @@
 // and the LDS chunk swizzle.
 #pragma once
 #include "fgx_common.h"
+#include "split3.h"
 #include "vmem_wait.h"
 
 namespace fgx {

@@ -43,8 +43,8 @@ int pick_cols(int c) { return c > 64 ? 128 : (c > 32 ? 64 : 32); }
 
 size_t round_up(size_t x, size_t m) { return (x + m - 1) / m * m; }
 
-// fp32: the matrix units take 32-bit operands at a sixteenth of the 16-bit rate, so every pass is bound by what is multiplied --
-// padding and idle CUs included -- long before loads count, and the choice is the one with the least of both.
+// fp32: the matrix units take 32-bit operands at a sixteenth of the 16-bit rate, and six products of bf16 parts for one are not much faster,
+// so a pass is bound by what is multiplied -- padding and idle CUs included -- before loads count.
 //
 // Weight gradient: 64 x 64 tiles, or 32 x 32 where those pad at least 28 % less (a 32 x 32 tile multiplies at about that
 // much less: 64 160 voxels x 64 channels 0.169 against 0.122 ms), over voxel blocks short enough for about 2000 items of the
@@ -68,21 +68,23 @@ bool rule_wgrad_f32(size_t n, int Ci, int Co, int V, fgx_schedule* out) {
     return true;
 }
 
-// Gather GEMM: what a CU multiplies, in columns of 256-row tiles, under each choice.
-//   streaming kernel, tiles of 256 x c: whole items per CU, c columns each, at a rate that falls a little with c; a lone
-//   32-column item leaves the matrix units waiting for its loads half as long again;
-//   tiled kernel with K split until the pieces even out: the columns of all tiles over the CUs, at about 0.72 of the rate.
-// Measured forward (ms; before: 128-column tiles from 65 columns on):  38 720 voxels, 96 channels 0.285 -> 0.159;  40 -> 200
-// channels 0.270 -> 0.173;  155 096 voxels, 96 channels 0.606 -> 0.437;  24 488 voxels, 320 channels 1.37 -> 0.87;  101 304
-// voxels, 48 channels 0.141 -> 0.109;  64 160 voxels, 32 channels 0.058 -> 0.045;  tiled: 8 624 voxels, 96 channels 0.108 ->
-// 0.069, 512 channels 1.52 -> 0.99;  38 720 voxels, 160 -> 24 channels 0.200 -> 0.118;  344 voxels, 128 channels 0.043 -> 0.028.
+// Gather GEMM: what a CU multiplies, in columns of 256-row tiles and bytes of K in whole slabs, under each choice.
+//   streaming kernel, three bf16 parts a value (csrc/split3.h), tiles of r x c: items per CU and what the launch waits for its
+//   last and heaviest ones (`last`; `least` for a lone round, whose heaviest tile has half as many offsets again as the mean), at
+//   a rate that falls with c: a fragment's parts are made once and multiplied c / 32 times;
+//   tiled kernel, on the fp32 units, with K split until the pieces even out: a third of the rate, and 15 us of its own.
+// Measured forward, us, 256 x 128 / 256 x 64 / 256 x 32 (64-byte slabs but for the first):  128 channels, 49 829 voxels 199 233
+// 227;  77 160 261 305 300;  166 977 412 539 553;  407 279 911 1 160 1 234;  96 channels, 166 977 voxels 307 407 314;  192
+// channels 1 092 1 142 1 202, 128 x 256 1 041;  48 channels 213 120 118, slabs of 128 bytes 213 174;  64 channels 213 154 155, 174;
+// 32 channels, 77 160 voxels 82 59 40, tiled 59.   With what the fp32 units wanted (narrow tiles before padding) the products
+// of three parts took 554 us under 128 channels at 166 977 voxels, on the fp32 units 681;  192 channels 1 301 and 1 378.
 void rule_gemm_f32(size_t n, int K, int cols, int V, fgx_schedule* out) {
     const size_t row_bytes = (size_t)K * 4;
-    const int slab = row_bytes >= 128 ? 128 : 64;
+    const int slab = row_bytes == 128 ? 128 : 64;       // (of 64 columns: whole slabs of longer rows count for more than their length)
     const double row_tiles = cdiv(n ? n : 1, 256);
     const int wide = cdiv(cols, 64) * 64;
     const bool narrow = cdiv(cols, 32) * 32 < wide;
-    double best = row_tiles * (narrow ? cdiv(cols, 32) * 32 : wide) / kCUs / 0.72;
+    double best = row_tiles * (narrow ? cdiv(cols, 32) * 32 : wide) / kCUs / 0.33 * align_up(row_bytes, 64) + 15.0 * 446.0 * 27 / V;     // (446: of a microsecond)
     *out = fgx_schedule{narrow && n < 1024 ? 32 : 64, narrow ? 32 : 64, 64, 1, 0, 0};
     if (cdiv(cols, 128) * 128 == wide && row_bytes >= 1024 && cdiv(n ? n : 1, 128) * cdiv(cols, 128) >= 32) out->tile_rows = out->tile_cols = 128;
     {
@@ -93,13 +95,13 @@ void rule_gemm_f32(size_t n, int K, int cols, int V, fgx_schedule* out) {
         out->splitk = s;
     }
     if (row_bytes < 64) return;
-    struct Shape { int rows, cols, slab; double rate; };
-    const Shape shapes[] = {{128, 256, 128, 1.08}, {256, 128, 128, 1.0}, {256, 64, slab, 0.98}, {256, 32, 64, 0.92}};
+    struct Shape { int rows, cols, slab; double rate, last, least; };
+    const Shape shapes[] = {{128, 256, 128, 1.04, 0.4, 1.45}, {256, 128, 128, 1.0, 0.6, 1.45}, {256, 64, slab, 0.79, 0.8, 1.75}, {256, 32, 64, 0.74, 1.4, 2.2}};
     for (const Shape& sh : shapes) {
         if (sh.slab > (int)align_up(row_bytes, 64) || (sh.cols == 256 && cols <= 128) || !stream_lds_fits(sh.rows, sh.cols, sh.slab, cols)) continue;
-        const size_t items = (size_t)cdiv(n ? n : 1, sh.rows) * cdiv(cols, sh.cols);
-        const double each = sh.cols * sh.rows / 256.0 / sh.rate;
-        const double time = cdiv(items, (size_t)kCUs) * each * (sh.cols == 32 && items <= (size_t)kCUs ? 1.5 : 1.0);
+        const double items = (double)cdiv(n ? n : 1, sh.rows) * cdiv(cols, sh.cols) / kCUs;
+        const double rounds = std::max(items + sh.last, sh.least);
+        const double time = rounds * sh.cols * sh.rows / 256.0 / sh.rate * align_up(row_bytes, sh.slab);
         if (time < best) {
             best = time;
             *out = fgx_schedule{sh.rows, sh.cols, sh.slab, 1, 0, 1};
