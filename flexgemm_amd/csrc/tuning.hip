@@ -71,7 +71,7 @@ bool rule_wgrad_f32(size_t n, int Ci, int Co, int V, fgx_schedule* out) {
 // Gather GEMM: what a CU multiplies, in columns of 256-row tiles and bytes of K in whole slabs, under each choice.
 //   streaming kernel, three bf16 parts a value (csrc/split3.h), tiles of r x c: items per CU and what the launch waits for its
 //   last and heaviest ones (`last`; `least` for a lone round, whose heaviest tile has half as many offsets again as the mean), at
-//   a rate that falls with c: a fragment's parts are made once and multiplied c / 32 times;
+//   a rate that falls with c: a fragment's parts are made once and multiplied c / 32 times; 7 us of its own;
 //   tiled kernel, on the fp32 units, with K split until the pieces even out: a third of the rate, and 15 us of its own.
 // Measured forward, us, 256 x 128 / 256 x 64 / 256 x 32 (64-byte slabs but for the first):  128 channels, 49 829 voxels 199 233
 // 227;  77 160 261 305 300;  166 977 412 539 553;  407 279 911 1 160 1 234;  96 channels, 166 977 voxels 307 407 314;  192
@@ -101,7 +101,7 @@ void rule_gemm_f32(size_t n, int K, int cols, int V, fgx_schedule* out) {
         if (sh.slab > (int)align_up(row_bytes, 64) || (sh.cols == 256 && cols <= 128) || !stream_lds_fits(sh.rows, sh.cols, sh.slab, cols)) continue;
         const double items = (double)cdiv(n ? n : 1, sh.rows) * cdiv(cols, sh.cols) / kCUs;
         const double rounds = std::max(items + sh.last, sh.least);
-        const double time = rounds * sh.cols * sh.rows / 256.0 / sh.rate * align_up(row_bytes, sh.slab);
+        const double time = rounds * sh.cols * sh.rows / 256.0 / sh.rate * align_up(row_bytes, sh.slab) + 7.0 * 446.0 * 27 / V;
         if (time < best) {
             best = time;
             *out = fgx_schedule{sh.rows, sh.cols, sh.slab, 1, 0, 1};
@@ -299,15 +299,17 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
         if (tiles * s >= pieces) break;
     }
     out->splitk = s;
-    // Persistent streaming kernel: rows of at least 64 bytes; 64-byte K-slabs below 128 bytes, 128-byte ones from there on.
-    // 16-bit rows of 128 ... 255 bytes (64 ... 127 channels) also take the 64-byte slabs while one column tile holds the outputs:
+    // Persistent streaming kernel: rows of at least 64 bytes; 64-byte K-slabs for rows of one, 128-byte ones for longer rows: of 72 ... 127 bytes
+    // one slab holds the row, what is past its end is not loaded, and an offset is one step instead of two (forward, 64- and 128-byte
+    // slabs, us: 40 channels, 166 977 voxels 49.1 42.8, 407 279 94.5 88.9;  56 channels 58.3 47.3 and 117 104).
+    // 16-bit rows of 128 ... 192 bytes (64 ... 96 channels) also take the 64-byte slabs while one column tile holds the outputs:
     // their rings leave room for two workgroups per CU, which is worth more than the longer pieces (measured forward, C = 64:
-    // 143 616 / 252 392 / 577 592 / 1 026 536 voxels -5 / -22 / -7 / -12 %; C = 80 and 96: -2 ... -5 %; from 256 bytes on the
-    // 128-byte slabs are ahead, C = 128: 0.049 against 0.056 ms at 64 160 voxels) ... given two items per CU to keep both
-    // workgroups busy (64 160 voxels, 251 items: 0.028 ms on 128-byte slabs, 0.031 on 64-byte ones)
-    const bool short_slabs = row_bytes >= 128 && row_bytes < 256 && cols <= 128 &&
+    // 143 616 / 252 392 / 577 592 / 1 026 536 voxels -5 / -22 / -7 / -12 %; C = 80 and 96: -2 ... -5 %) ... given two items per CU to keep both
+    // workgroups busy (64 160 voxels, 251 items: 0.028 ms on 128-byte slabs, 0.031 on 64-byte ones).  Beyond 192 bytes they are four
+    // steps for two (112 channels, 166 977 voxels 101 87, 407 279 217 199;  C = 128: 0.056 against 0.049 ms at 64 160 voxels).
+    const bool short_slabs = row_bytes >= 128 && row_bytes <= 192 && cols <= 128 &&
                              (size_t)cdiv(n, 256) * cdiv(cols, cols > 64 ? 128 : 64) >= 2 * (size_t)kCUs;
-    const int slab = (row_bytes >= 128 && !short_slabs) ? 128 : 64;
+    const int slab = (row_bytes > 64 && !short_slabs) ? 128 : 64;
     // The tile by what a CU multiplies and loads: whole items per CU, each its columns (of 256 rows) at the tile's rate.  One
     // tile of 128 rows x 256 columns gathers every row once for the same bytes per product as 256 x 128, and pads less;
     // 64-column tiles read a gathered row from L2 more often but even out a chip that larger ones fill 1.3 times or less than
