@@ -34,7 +34,7 @@ EXPORTS = [
     "fgx_conv_scratch_bytes", "fgx_conv_gather_gemm", "fgx_conv_gather_gemm_act", "fgx_conv_gather_gemm_act_mask", "fgx_conv_gather_gemm_weight_pays",
     "fgx_conv_gather_gemm_weight", "fgx_conv_gemm_pairs_pays", "fgx_pair_plan_words", "fgx_pair_plan", "fgx_conv_gemm_pairs_scratch_bytes",
     "fgx_conv_gemm_pairs", "fgx_conv_gemm_few_pays", "fgx_conv_gemm_few", "fgx_conv_gemm_few_mask",
-    "fgx_relu_mask_apply", "fgx_copy_columns", "fgx_conv_gather_gemm_stream_act_mask",
+    "fgx_relu_mask_apply", "fgx_copy_columns", "fgx_relu_columns", "fgx_conv_gather_gemm_stream_act_mask",
     "fgx_gather_plan_count", "fgx_gather_plan_fill", "fgx_conv_gather_gemm_stream", "fgx_conv_gather_gemm_stream_act",
     "fgx_conv_gather_gemm_stream_groups", "fgx_gather_item_order_workspace_bytes", "fgx_gather_item_order",
     "fgx_wgrad_scratch_bytes", "fgx_wgrad_block_bounds_count", "fgx_wgrad_block_bounds", "fgx_conv_wgrad",

@@ -41,7 +41,7 @@ namespace {
     X(fgx_spconv_out_coords_grid_emit) X(fgx_tile_plan) X(fgx_gather_item_order) X(fgx_gather_item_order_workspace_bytes)          \
     X(fgx_weight_panel_bytes) X(fgx_pack_weight) X(fgx_conv_scratch_bytes) X(fgx_conv_gather_gemm_act_mask)                        \
     X(fgx_conv_gather_gemm_weight_pays) X(fgx_conv_gather_gemm_weight) X(fgx_conv_gemm_pairs_pays) X(fgx_pair_plan_words) X(fgx_pair_plan) X(fgx_conv_gemm_pairs_scratch_bytes) X(fgx_conv_gemm_pairs) X(fgx_conv_gemm_few_pays) X(fgx_conv_gemm_few_mask)                                                             \
-    X(fgx_conv_gather_gemm_stream_act_mask) X(fgx_conv_gather_gemm_stream_groups) X(fgx_relu_mask_apply) X(fgx_copy_columns)       \
+    X(fgx_conv_gather_gemm_stream_act_mask) X(fgx_conv_gather_gemm_stream_groups) X(fgx_relu_mask_apply) X(fgx_copy_columns) X(fgx_relu_columns) \
     X(fgx_colsum_scratch_bytes) X(fgx_colsum) X(fgx_wgrad_block_bounds_count) X(fgx_wgrad_block_bounds)                            \
     X(fgx_conv_gemm_stem_pays) X(fgx_conv_gemm_stem) X(fgx_wgrad_stem_pays) X(fgx_wgrad_stem_scratch_bytes) X(fgx_conv_wgrad_stem_cut) X(fgx_wgrad_item_lists_count) X(fgx_wgrad_item_lists) X(fgx_wgrad_scratch_bytes) X(fgx_conv_wgrad_lists)                       \
     X(fgx_wgrad_schedule) X(fgx_wgrad_sweep_fits) X(fgx_conv_wgrad_split_scratch_bytes) X(fgx_conv_wgrad_split)                                                                  \
@@ -737,6 +737,7 @@ void require_on(const at::Device& dev, const Tensor& t, const char* what) {
 
 struct Product {
     Tensor out, mask;
+    Tensor src;         // the rows as they were multiplied, where they had to be filled up to whole 16-byte pieces
 };
 
 // mode 0: out = conv(src) with weight [Co, V, Ci] (+ bias), mode 1: input gradient from src = grad_output through the same
@@ -777,6 +778,7 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
         owner = {};                                     // (a padded copy is made per call: nothing to keep a panel by)
         src = pad_to(src, 1, align, stream);
         weight = pad_to(weight, mode == 0 ? 2 : 0, align, stream);
+        p.src = src;
     }
     src = src.contiguous();
     weight = weight.contiguous();
@@ -974,8 +976,9 @@ struct WeightGrads {
 
 // [Co, V, Ci] weight gradient (and with with_bias the bias gradient) from the cache's pair lists: grad has one row per row of
 // the cache's map, feats one per row the map points at.  bias_offset names an offset whose pairs hold every row of grad exactly
-// once (-1: none), which lets the streaming kernel sum the rows it loads anyway.
-WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool with_bias, int bias_offset, int64_t stream) {
+// once (-1: none), which lets the streaming kernel sum the rows it loads anyway.  true_ci, true_co: the channels, where the rows come filled up.
+WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool with_bias, int bias_offset, int64_t stream, int64_t true_ci = -1,
+                         int64_t true_co = -1) {
     const at::Device dev = feats.device();
     const c10::DeviceGuard guard(dev);
     const int code = dtype_code(feats);
@@ -987,7 +990,9 @@ WeightGrads weight_grads(Tensor grad, Tensor feats, const Cache& c, int v, bool 
         if (grad.size(0) != nmap.size(0))
             throw py::value_error(std::to_string(grad.size(0)) + " gradient rows for a neighbor cache of " + std::to_string(nmap.size(0)) + " rows");
     }
-    const int64_t n = grad.size(0), n_in = feats.size(0), true_ci = feats.size(1), true_co = grad.size(1);
+    const int64_t n = grad.size(0), n_in = feats.size(0);
+    if (true_ci < 0) true_ci = feats.size(1);
+    if (true_co < 0) true_co = grad.size(1);
     const int es = (int)feats.element_size(), align = 16 / es;
     feats = pad_to(feats, 1, align, stream).contiguous();
     grad = pad_to(grad, 1, align, stream).contiguous();
@@ -1130,6 +1135,7 @@ struct ConvBackward : public torch::autograd::Node {
     Held cache;
     SavedVariable feats, weight, bias, output;      // (the bias only to refuse one that was changed in place)
     SavedVariable mask;                 // the ReLU's derivative, one bit per output
+    Tensor filled;                      // feats with its rows filled up, as the forward pass had them (undefined: the backward pass fills its own)
     bool relu = false, has_bias = false, has_mask = false;
 
     std::string name() const override { return call.generic ? "SparseConv3dBackward" : "SubMConv3dBackward"; }
@@ -1139,6 +1145,7 @@ struct ConvBackward : public torch::autograd::Node {
         bias.reset_data();
         output.reset_data();
         mask.reset_data();
+        filled.reset();
     }
 
     variable_list apply(variable_list&& grads) override {
@@ -1176,10 +1183,19 @@ struct ConvBackward : public torch::autograd::Node {
         const py::gil_scoped_acquire gil;
         const int64_t stream = stream_of(f);
         const Cache c(py::reinterpret_borrow<py::object>(cache.obj), stream);
+        // rows filled up once for both products
         Tensor grad = grads[0];
-        if (has_mask) grad = relu_mask_apply(grad, m, stream);
-        else if (relu) grad = at::where(y.gt(0), grad, at::zeros({}, grad.options()));
-        grad = grad.contiguous();
+        const int64_t align = 16 / (int64_t)grad.element_size(), rows = grad.size(0), filled_co = (grad.size(1) + align - 1) / align * align;
+        if (has_mask) {
+            grad = relu_mask_apply(grad, m, stream);
+        } else if (relu && grad.numel() > 0 && y.scalar_type() == grad.scalar_type() && y.sizes() == grad.sizes()) {
+            const Tensor g = grad.contiguous(), h = y.contiguous();
+            grad = make({rows, filled_co}, g.scalar_type(), g.device());
+            check(L.fgx_relu_columns(dtype_code(g), ptr(g), ptr(h), (size_t)rows, (int)g.size(1), ptr(grad), (int)filled_co, as_stream(stream)));
+        } else if (relu) {
+            grad = at::where(y.gt(0), grad, at::zeros({}, grad.options()));
+        }
+        grad = pad_to(grad.contiguous(), 1, align, stream);
         const int64_t co = w.size(0), kw = w.size(1), kh = w.size(2), kd = w.size(3), ci = w.size(4), v = kw * kh * kd;
         if (need_f) {
             const Tensor wv = w.reshape({co, v, ci});
@@ -1197,11 +1213,11 @@ struct ConvBackward : public torch::autograd::Node {
             const bool odd = kw % 2 && kh % 2 && kd % 2 && !call.generic;
             const int centre = odd && PyObject_IsTrue(module_get(g_spconv, "FUSE_DBIAS")) ? (int)(v / 2) : -1;
             const bool with_bias = need_b && !call.generic;
-            WeightGrads g = weight_grads(grad, f, c, (int)v, with_bias, with_bias ? centre : -1, stream);
+            WeightGrads g = weight_grads(grad, filled.defined() ? filled : f, c, (int)v, with_bias, with_bias ? centre : -1, stream, ci, co);
             result[1] = g.weight.reshape({co, kw, kh, kd, ci});
             if (with_bias) result[2] = g.bias;
         }
-        if (need_b && !result[2].defined()) result[2] = colsum(grad, stream);
+        if (need_b && !result[2].defined()) result[2] = colsum(grad, stream).slice(0, 0, co);
         return result;
     }
 };
@@ -1260,6 +1276,8 @@ Tensor convolve(const Tensor& feats, py::object cache_obj, const Tensor& weight,
     node->feats = SavedVariable(feats, false);
     node->weight = SavedVariable(weight, false);
     if (has_bias) node->bias = SavedVariable(bias, false);
+    // (hooks of the saved tensors may want nothing left on the device)
+    if (p.src.defined() && weight.requires_grad() && !at::SavedTensorDefaultHooks::get_hooks().has_value()) node->filled = p.src;
     node->has_mask = p.mask.defined();
     if (node->has_mask) node->mask = SavedVariable(p.mask, false);
     torch::autograd::set_history(p.out, node);

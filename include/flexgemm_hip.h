@@ -345,6 +345,10 @@ int fgx_relu_mask_apply(int dtype, const void* grad, const uint8_t* relu_mask, s
  * caller's tensors have.  elem_bytes 2 or 4; src and dst must not overlap.  One pass. */
 int fgx_copy_columns(int elem_bytes, const void* src, size_t rows, int src_cols, void* dst, int dst_cols, fgx_stream_t stream);
 
+/* out[r][c] = c < cols && y[r][c] > 0 ? grad[r][c] : 0 for c < out_cols (>= cols): the gradient of a ReLU from its output, rows filled up with
+ * zeros.  out must not overlap grad or y.  One pass.  No counterpart in the reference. */
+int fgx_relu_columns(int dtype, const void* grad, const void* y, size_t rows, int cols, void* out, int out_cols, fgx_stream_t stream);
+
 /* Gather plan of a row order for tiles of `tile_rows` rows: for tile t and the k-th offset v present in it
  * (the set bits of tile_code[t], ascending; a tile whose code is 0 gets one row with every neighbor missing),
  *   plan_idx[(plan_seg[t] + k) * tile_rows + r] = map[order[t * tile_rows + r], v]     (0xFFFFFFFF for rows past n),
