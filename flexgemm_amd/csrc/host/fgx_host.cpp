@@ -325,6 +325,13 @@ bool few_pays(int code, int64_t n, int ci, int co, int v) {
     return L.fgx_conv_gemm_few_pays(code, (size_t)n, ci, co, v) && n < module_int(g_impl, "LOCALITY_MIN_ROWS");
 }
 
+// Output columns that the kernels of whole 16-byte pieces (resident rows, first layers) multiply for `cols` 16-bit ones: the columns, or over many
+// rows those filled up to a multiple of 8 and cut afterwards, a pass over the output and two or three small copies.  Before and now, us:
+// 11 -> 11 channels, cache and one layer, 1.84 million voxels 688 398;  64 -> 19, then three of 19, 1.30 million 1296 688;  27 -> 27, 229 217 voxels, cache
+// and one layer 144 94, trained 307 203 where the host keeps up with the copies' launches and 307 310 where it does not (kept 183, 134 and 232);
+// 6 -> 41, fresh and kept, 73 461 voxels 62 49 and 43 31, trained 109 117 and 88 96, 229 217 voxels 180 128 and 102 98.
+int whole_columns(int cols, int64_t n) { return cols % 8 == 0 || n < (cols > 32 ? 131072 : 393216) ? cols : (cols + 7) / 8 * 8; }
+
 // What of the mask order and the pair lists the kernels of this layer read (a guess that errs towards "all of it": what a pass finds missing
 // it makes).  The resident-row kernels walk the cells of the index, first layers the map, the products over pairs a plan of
 // their own; so of the tables of 2 667 120 voxels under 32 channels 0.26 ms of sorts and 0.19 ms of lists were never read, of 434 000 voxels under a
@@ -334,12 +341,13 @@ Needs layer_needs(const Layer& l, int64_t n, int v, bool walks) {
     if (!schedules_are_ours()) return needs;
     const int es = l.code == FGX_F32 ? 4 : 2, align = 16 / es;
     const int ci = (int)((l.ci + align - 1) / align * align), co = (int)((l.co + align - 1) / align * align);
-    const bool resident = es == 2 && walks && v <= 27 && ci <= 32 && l.co <= 32 && l.co % 8 == 0 && n >= module_int(g_impl, "NARROW_RESIDENT_MIN_ROWS") &&
+    const int out_cols = es == 2 ? whole_columns((int)l.co, n) : (int)l.co, in_cols = es == 2 ? whole_columns((int)l.ci, n) : (int)l.ci;
+    const bool resident = es == 2 && walks && v <= 27 && ci <= 32 && out_cols <= 32 && out_cols % 8 == 0 && n >= module_int(g_impl, "NARROW_RESIDENT_MIN_ROWS") &&
                           narrow_mode() != "off";
-    const bool forward = resident || L.fgx_conv_gemm_stem_pays(l.code, 0, (size_t)n, ci, (int)l.co, v) ||
+    const bool forward = resident || L.fgx_conv_gemm_stem_pays(l.code, 0, (size_t)n, ci, out_cols, v) ||
                          (l.splitk && (L.fgx_conv_gemm_pairs_pays(l.code, 0, (size_t)n, ci, (int)l.co, v) ||
                                        few_pays(l.code, n, ci, (int)l.co, v)));
-    const bool backward = !l.record || !l.input_grad || (resident && l.ci % 8 == 0) || L.fgx_conv_gemm_stem_pays(l.code, 1, (size_t)n, co, (int)l.ci, v) ||
+    const bool backward = !l.record || !l.input_grad || (resident && in_cols % 8 == 0) || L.fgx_conv_gemm_stem_pays(l.code, 1, (size_t)n, co, in_cols, v) ||
                           (l.splitk && L.fgx_conv_gemm_pairs_pays(l.code, 1, (size_t)n, (int)l.ci, co, v));
     needs.order = !(forward && backward);
     needs.plan = resident && n * 82 + 10752 < 0xFF000000ll && n * ci * 2 < 0xFF000000ll;        // (what _narrow_applies asks)
@@ -763,7 +771,7 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
     require_on(dev, weight, "the weight");
     require_on(dev, bias, "the bias");
     const int64_t n = nmap.size(0), n_src = src.size(0);
-    const int cols = (int)weight.size(mode == 0 ? 0 : 2);
+    int cols = (int)weight.size(mode == 0 ? 0 : 2);
     if (bias.defined() && bias.numel() != cols)
         throw py::value_error("a bias of " + std::to_string(bias.numel()) + " values for " + std::to_string(cols) + " output channels");
     Product p;
@@ -783,16 +791,31 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
     src = src.contiguous();
     weight = weight.contiguous();
     if (bias.defined()) bias = bias.contiguous();
-    const int co = (int)weight.size(0), ci = (int)weight.size(2), k = mode == 0 ? ci : co;
+    int co = (int)weight.size(0), ci = (int)weight.size(2);
+    const int k = mode == 0 ? ci : co;
     const int64_t row_bytes = (int64_t)k * es;
     const int pass = mode == 0 ? 0 : 1;
+    // (these two kernels' outputs are whole 16-byte pieces: a ragged row is multiplied as one and cut)
+    const int whole = es == 2 && schedules_are_ours() ? whole_columns(cols, n) : cols;
     // a network's first layers: all offsets of a row in one product, no row order or tile tables
-    const bool stem = n > 0 && L.fgx_conv_gemm_stem_pays(code, mode, (size_t)n, k, cols, v) && schedules_are_ours() &&
+    const bool stem = n > 0 && L.fgx_conv_gemm_stem_pays(code, mode, (size_t)n, k, whole, v) && schedules_are_ours() &&
                       aligned(src) && aligned(weight) && aligned(nmap);
     // Up to 32 channels on both sides: the resident-row kernel where it runs at once or the cache has earned its plan (38 720 voxels, 8 ->
     // 32 channels: 0.014 ms, 0.010 without; 98 408 voxels 0.015 and 0.016, 427 872 voxels 0.033 and 0.046, 16 -> 32 0.034 and 0.087).
-    const bool narrow = n > 0 && narrow_shape(c, es, k, cols, v, n) &&
-                        impl_function("_narrow_applies")(c.obj, src, k, cols, v, n, n_src, python_schedule(pass, src, n, ci, co, v)).cast<bool>();
+    const bool narrow = n > 0 && narrow_shape(c, es, k, whole, v, n) &&
+                        impl_function("_narrow_applies")(c.obj, src, k, whole, v, n, n_src,
+                                                         python_schedule(pass, src, n, mode == 0 ? ci : whole, mode == 0 ? whole : co, v)).cast<bool>();
+    const int cut = whole != cols && (stem || narrow) ? cols : 0;
+    if (cut) {
+        owner = {};
+        weight = pad_to(weight, mode == 0 ? 0 : 2, align, stream);
+        if (bias.defined()) bias = pad_to(bias, 0, align, stream);
+        want_mask = false;                              // (one bit per output of the rows as they are)
+        (mode == 0 ? co : ci) = cols = whole;
+    }
+    auto cut_back = [&] {
+        if (cut) p.out = copy_columns(p.out, n, cols, {n, cut}, cut, stream);
+    };
     if (stem && !narrow) {
         const char* name = mode == 0 ? "gather_gemm_fwd" : "gather_gemm_dgrad";
         p.out = make({n, cols}, src.scalar_type(), dev);
@@ -801,6 +824,7 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
         check(L.fgx_conv_gemm_stem(code, mode, ptr(src), ptr(weight), ptr(bias), ptr<uint32_t>(nmap), (size_t)n, ci, co, v, activation, ptr(p.out),
                                    ptr<uint8_t>(p.mask), as_stream(stream)));
         mark(name, "stop");
+        cut_back();
         return p;
     }
     // few voxels under a small weight: one launch
@@ -871,6 +895,7 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
         });
         p.out = got[0].cast<Tensor>();
         if (!got[1].is_none()) p.mask = got[1].cast<Tensor>();
+        cut_back();
         return p;
     }
     p.out = make({n, cols}, src.scalar_type(), dev);
