@@ -151,7 +151,13 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
         // 33 ... 64 channels on one side and over 192 on the other, or over 128 of many voxels: three and more 64 x 64 tiles.  The tiled kernel over short
         // blocks is ahead of the streaming one, whose workgroups walk one tile's pairs at a time (256 -> 64 channels, 38 720
         // voxels: 0.057 against 0.071 ms; 64 -> 160 channels, 228 816 voxels: 0.178 against 0.219).
-        if (out->stream == 1 && t == 64 && (Ci > 192 || Co > 192 || ((Ci > 128 || Co > 128) && n >= 98304)) && n >= 12288) {
+        // ... and up to 32 channels on one side, in the same 64 x 64 tiles: of a row's 128 bytes a step's pairs ask for half as many lines a byte as in
+        // 32 x 32 ones, which are asked for again by every tile (us, 32 x 32 streaming and this: 200 -> 32, 134 572 voxels 144 154, 166 977 183 174,
+        // 294 092 343 268;  144 -> 32 96 124, 129 142, 241 213;  320 -> 24 166 179, 209 207, 374 330;  448 -> 32, 101 586 178 166, 294 092 560 433, 49 829
+        // 106 108;  32 -> 640, 294 092 896 630).
+        const bool lopsided = t == 32 && ((most > 384 && n >= 98304) || (most > 128 && n >= 196608));
+        if (out->stream == 1 && ((t == 64 && (Ci > 192 || Co > 192 || ((Ci > 128 || Co > 128) && n >= 98304)) && n >= 12288) || lopsided)) {
+            out->tile_rows = out->tile_cols = 64;
             out->stream = 0;
             size_t rows = n >= 98304 ? 4096 : 2048;
             const double per_block = 4.0 * V * (double)Co * Ci;
