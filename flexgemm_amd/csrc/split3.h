@@ -18,6 +18,7 @@ using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
 struct Split3 {
     bf16x8 part[3];
 };
+template <bool NEGATED = false>
 __device__ __forceinline__ Split3 split3(const u32x4& lo, const u32x4& hi) {
     using bf16x2 = __bf16 __attribute__((ext_vector_type(2)));
     using f32x2 = float __attribute__((ext_vector_type(2)));
@@ -26,6 +27,7 @@ __device__ __forceinline__ Split3 split3(const u32x4& lo, const u32x4& hi) {
     for (int p = 0; p < 4; ++p) {
         float x = __builtin_bit_cast(float, p < 2 ? lo[p * 2] : hi[p * 2 - 4]);
         float y = __builtin_bit_cast(float, p < 2 ? lo[p * 2 + 1] : hi[p * 2 - 3]);
+        if (NEGATED) x = -x, y = -y;            // (an operand modifier)
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
             const f32x2 xy = {x, y};
@@ -47,18 +49,19 @@ __device__ __forceinline__ bool split3_holds(float sum) {
     const uint32_t u = __builtin_bit_cast(uint32_t, sum) << 1;
     return u == 0u || u - (31u << 24) < (224u << 24);
 }
-template <typename Acc>      // 32 x 32 over 16 values of K, or 16 x 16 over 32
+// the six products, smallest first, of 32 x 32 over 16 values of K or 16 x 16 over 32
+constexpr int kSplit3Products = 6;
+template <typename Acc>
+__device__ __forceinline__ void mma_split3(Acc& acc, const Split3& a, const Split3& b, int product) {
+    constexpr int kOfA[kSplit3Products] = {2, 0, 1, 1, 0, 0}, kOfB[kSplit3Products] = {0, 2, 1, 0, 1, 0};
+    const bf16x8 x = a.part[kOfA[product]], y = b.part[kOfB[product]];
+    if constexpr (sizeof(Acc) == 64) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, acc, 0, 0, 0);
+    else acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, acc, 0, 0, 0);
+}
+template <typename Acc>
 __device__ __forceinline__ void mma_split3(Acc& acc, const Split3& a, const Split3& b) {
-    auto product = [&](int of_a, int of_b) __attribute__((always_inline)) {
-        if constexpr (sizeof(Acc) == 64) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.part[of_a], b.part[of_b], acc, 0, 0, 0);
-        else acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.part[of_a], b.part[of_b], acc, 0, 0, 0);
-    };
-    product(2, 0);
-    product(0, 2);
-    product(1, 1);
-    product(1, 0);
-    product(0, 1);
-    product(0, 0);
+#pragma unroll
+    for (int p = 0; p < kSplit3Products; ++p) mma_split3(acc, a, b, p);
 }
 
 }  // namespace

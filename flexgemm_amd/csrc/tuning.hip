@@ -387,24 +387,22 @@ extern "C" int fgx_wgrad_short_tile(int dtype, size_t n, int Ci, int Co) {
 }
 
 // fp32 weight gradient over the even split (fgx_conv_wgrad_split), in 96 x 96 tiles where they pad no more than 64 x 64 ones.  Its
-// large tile multiplies at about twice the rate of the 32 x 32 one, which stays where it pads to half and less (32 channels,
-// 41 700 voxels 0.052 ms, split 0.068).  Two voxel blocks under few tiles, one otherwise: a block adds segments, and rows are
-// read from L2 fast enough either way (96 channels, 41 700 voxels: 1 block 0.102, 2 0.100, 8 0.106).
-// Measured (ms, before -> now): 96 x 96: 96 channels, 2 581 voxels 0.039 -> 0.034, 10 494 0.083 -> 0.047, 41 700 0.196 -> 0.100, 667 763
-// 2.33 -> 1.22;  96 -> 192 channels, 41 700 voxels 0.345 -> 0.173;  192 channels, 10 494 voxels 0.137 -> 0.101, 41 700 0.395 -> 0.311;
-// 768 channels, 2 581 voxels 0.45 -> 0.37.   64 x 64: 64 channels, 5 876 voxels 0.033 -> 0.030, 41 700 0.099 -> 0.066 (2 581: 0.026
-// and 0.027);  128 channels, 2 581 voxels 0.039 -> 0.035, 41 700 0.200 -> 0.183.
-// Past these ranges the tiled kernel is level or ahead: 64 x 64 tiles, one from 667 763 voxels (0.71 both), a few of 166 977
-// (128 channels: 0.62, split 0.67), sixteen of 41 700 (256 channels: 0.63, split 0.66; 10 494: 0.20 -> 0.19), more of any number
-// (512 channels, 2 581 voxels 0.208 and 0.214);  four and more 96 x 96 tiles past 262 144 voxels: not measured.
+// large tile multiplies at about twice the rate of the 32 x 32 one, which stays where it pads to less than half (32 channels,
+// 49 829 voxels 0.048 ms, split 0.057;  32 -> 64 channels, half, 0.081 and 0.057, 448 584 voxels 0.400 and 0.347).  Two voxel blocks under few
+// tiles, one otherwise: a block adds segments, and rows are read from L2 fast enough either way.
+// Measured (us, tiled kernel on the fp32 units -> the split in three parts):  one 64 x 64 tile: 64 channels, 10 494 voxels 27 -> 28, 277 018 316 -> 224,
+// 448 584 464 -> 354;  48 channels, 277 018 382 -> 225;  two: 112 -> 48 channels, 101 586 294 -> 169, 448 584 1 041 -> 690;  four: 128 channels, 101 586
+// 390 -> 305, 166 977 595 -> 520, 448 584 1 533 -> 1 482, 635 497 2 161 -> 2 190;  25: 320 channels, 1 456 voxels 73 -> 55, 10 494 313 -> 232, 101 586 2 053 -> 1 981;  64: 512
+// channels, 1 456 122 -> 112, 10 494 701 -> 553, 25 488 1 332 -> 1 196;  96 x 96: 96 channels, 2 581 39 -> 34, 667 763 2 330 -> 1 020.
+// Sixteen tiles past 12 288 voxels, and four and more of 96 x 96 past 262 144, stay where they were.
 extern "C" int fgx_wgrad_split_tile(size_t n, int Ci, int Co, int* block_rows) {
     if (n == 0 || Ci <= 0 || Co <= 0 || block_rows == nullptr || (size_t)Ci * Co >= (size_t)1024 * 1024) return 0;
     auto padded = [&](int t) { return (double)cdiv(Ci, t) * t * cdiv(Co, t) * t; };
     const int t = padded(96) <= padded(64) ? 96 : 64;
-    const size_t tiles = (size_t)cdiv(Ci, t) * cdiv(Co, t);
-    const size_t least = t == 64 && tiles == 1 ? 4096 : 2048;
-    const size_t most = t == 96 ? (tiles >= 4 ? 262144 : ~(size_t)0) : tiles == 1 ? 262144 : tiles < 16 ? 65536 : tiles == 16 ? 12288 : 0;
-    if (padded(32) <= 0.55 * padded(t) || n < least || n > most) return 0;
+    const size_t tiles = (size_t)cdiv(Ci, t) * cdiv(Co, t), any = ~(size_t)0;
+    const size_t least = t == 96 ? 2048 : tiles == 1 ? 4096 : tiles > 16 ? 1024 : 2048;
+    const size_t most = t == 96 ? (tiles >= 4 ? 262144 : any) : tiles < 4 ? any : tiles < 16 ? 524288 : tiles == 16 ? 12288 : 131072;
+    if (padded(32) <= 0.45 * padded(t) || n < least || n > most) return 0;
     *block_rows = (int)std::min(round_up(cdiv(n, (size_t)(tiles < 4 ? 2 : 1)), 64), (size_t)1 << 30);
     return t;
 }

@@ -19,6 +19,7 @@ using i16x8 = short __attribute__((ext_vector_type(8)));
 struct F16 { using type = _Float16; };
 struct BF16 { using type = __bf16; };
 struct F32 { using type = float; };
+struct F32Units { using type = float; };      // multiplied on the fp32 matrix units rather than in bf16 parts
 
 template <typename T> __device__ __forceinline__ T from_float(float x);
 template <> __device__ __forceinline__ _Float16 from_float<_Float16>(float x) { return (_Float16)x; }

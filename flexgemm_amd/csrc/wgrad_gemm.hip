@@ -30,6 +30,7 @@
 #include <numeric>
 #include <type_traits>
 
+#include "split3.h"
 #include "wgrad_device.h"
 
 namespace fgx {
@@ -308,6 +309,7 @@ constexpr int kWsIdxSlots = 8;
 constexpr int kWsIdxAhead = 4;       // index loads run this many steps ahead of the row loads (> kWsStages - 1)
 constexpr int kWsLoaders = 4;
 constexpr int kWsPairs = 64;         // pairs per step
+constexpr unsigned kSplitSyncWords = 5;          // fp32: behind that, multipliers done with a stage and the quarters' sums that stand in it
 constexpr unsigned kSplitMaxUnits = 2048;       // fp32: (block, offset) pairs of the even split, whose running cost stands in LDS
 template <typename Tag, int BM, int BN>
 struct WStreamCfg {
@@ -320,8 +322,10 @@ struct WStreamCfg {
     static constexpr int SLICES = KSPLIT ? 4 : 1;                  // partial products per (voxel block, offset, tile)
     // (a 256 x 128 tile's stages are 48 KiB: three of them fit, with the same 64-pair steps)
     static constexpr int P = KSPLIT ? 4 * kWsPairs : kWsPairs, S = (BM + BN) * ES > 512 ? 3 : kWsStages;
-    static constexpr int NW = 4, NL = kWsLoaders, NT = 64 * (NW + NL);
-    // fp32 multiplies in 16 x 16 tiles: a 96 x 96 tile then has nine of them for each of the four multipliers
+    // fp32 in three parts: two multipliers for every quarter of the tile, each with half of a step's pairs
+    static constexpr int HALVES = std::is_same_v<Tag, F32> ? 2 : 1;
+    static constexpr int NW = 4 * HALVES, NL = kWsLoaders, NT = 64 * (NW + NL);
+    // fp32 multiplies in 16 x 16 tiles: a 96 x 96 tile then has nine of them for each quarter
     static constexpr int MT = ES == 2 ? 32 : 16;
     static constexpr int WM = KSPLIT ? BM : BM / 2, WN = KSPLIT ? BN : BN / 2, TM = WM / MT, TN = WN / MT;
     static constexpr int IDX_PER = P / 64;                         // wave-wide index loads per operand and step
@@ -343,7 +347,7 @@ struct WStreamCfg {
     static constexpr int band_bytes(int es) { return band_rows(es) * band_pitch(es); }
     static constexpr int BAND_BYTES = band_bytes(ES) > band_bytes(4) ? band_bytes(ES) : band_bytes(4);
     // (fp32 tiles leave straight from the registers: behind the rings stands the running cost of the even split)
-    static constexpr size_t lds_bytes = (size_t)RING_BYTES + (ES == 4 ? (size_t)(kSplitMaxUnits + 1) * 4 : (size_t)NW * BAND_BYTES);
+    static constexpr size_t lds_bytes = (size_t)RING_BYTES + (ES == 4 ? (size_t)(kSplitMaxUnits + 1 + kSplitSyncWords) * 4 : (size_t)NW * BAND_BYTES);
     static_assert(ES == 4 || (band_rows(4) >= 1024 / (WN * 4) && band_rows(ES) >= 1024 / (WN * ES)), "a wave-wide store takes its rows from one band");
     static_assert(!KSPLIT || ES == 2, "the pair-splitting tile is for 16-bit types");
     static_assert(S == 3 || S == 4, "the loaders' wait is written for rings of three or four stages");
@@ -365,33 +369,54 @@ struct WStreamCfg {
     static constexpr int key_b(int row) { return key(CH_B, row); }
 };
 
-// fp32 multipliers of the streaming kernel: a wavefront's WM x WN part of the tile in 16 x 16 products over four pairs at a time (lane l
-// holds row l / 16 of the four and column l % 16), transposed, so that element e of lane l is row l % 16 (co) and column
-// 4 * (l / 16) + e (ci): a lane stores 16 bytes of an output row, four lanes 64.
-// Bound by the matrix units, whose fp32 rate is a sixteenth of the 16-bit one: a lone workgroup keeps them busy 82 % of the time at
-// 96 x 96, 64 % at 64 x 64 (a step's barrier and first reads take about a thousand cycles beside 4608 and 2048 of products).
-// 96 x 96 because it is the widest tile whose three stages of 64 pairs fit LDS; two stages of 128 x 128 run at 88 %, but were no
-// faster where both fit (41 700 voxels, 128 channels: 0.172 ms each).  Reading fragments four k-blocks ahead was 4 % slower.
-template <typename C, typename W, typename Seek, typename After>
-__device__ __forceinline__ void multiply_f32(const unsigned char* ring, W m, const Seek& seek, const After& after, int wave_m, int wave_n,
+// fp32 multipliers of the streaming kernel, transposed: element e of lane l is row l % 16 (co) and column 4 * (l / 16) + e (ci) of a 16 x 16
+// product, so a lane stores 16 bytes of an output row, four lanes 64.  A wavefront has a WM x WN part of the tile.
+// HALF 0 and 1: over one half of a step's 64 pairs, in three bf16 parts (split3.h), 32 pairs a product (lane l holds column l % 16 of eight of them).
+// Making the parts takes 264 vector instructions (1 056 cycles) beside 54 products (864) of a 48 x 48 part, so a SIMD has two such wavefronts, one of which
+// fills the other's waits; alone, with all 64 pairs, it was no faster than the fp32 units.  The matrix unit rounds its sums downwards: HALF 1 multiplies
+// negated columns and the halves' sums are subtracted, so what it drops cancels (error against 64 bits, 96 channels, 166 977 and 407 279 voxels: fp32 units
+// 3.1e-7 and 3.3e-7, both halves alike 3.0e-7 and 4.6e-7, so 2.5e-7 and 2.6e-7).  Us, before and now: 96 channels, 38 407 voxels 103 88, 166 977 303 246;
+// 192 channels 334 260 and 1 146 854; 64 channels 63 58 and 173 152.
+// HALF -1: over all pairs, four at a time (lane l holds row l / 16 of the four), on the fp32 units, whose rate is a sixteenth of the 16-bit one: for few
+// pairs, where the halves' meeting and their longer code cost more than they save (see units_are_faster).
+// 96 x 96 because it is the widest tile whose three stages of 64 pairs fit LDS.
+template <typename C, int HALF, typename W, typename Seek, typename After, typename Again>
+__device__ __forceinline__ void multiply_f32(unsigned char* ring, uint32_t* sync, W m, const Seek& seek, const After& after, const Again& again, int wave_m, int wave_n,
                                              unsigned group, float* partial) {
     const int lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
-    int a_off[C::TM], b_off[C::TN];                 // of the first four pairs; 16-byte pieces swizzled by the row, whose key repeats every four
+    // A running sum loses about a unit in the last place of itself with every addition: it is folded into a second one every 256
+    // pairs it takes, so that a segment may be long (the tiled kernel's error, 96 channels, 667 763 voxels: 9.8e-7).
+    constexpr int kRow0 = HALF == 1 ? 32 : 0, kFoldSteps = 256 * C::HALVES / C::P;
+    // of the first four pairs; 16-byte pieces swizzled by the row, whose key repeats every four
+    int a_off[C::TM], b_off[C::TN];
+    // a lane's eight pairs of a product of 32: every fourth one (which eight does not matter, as long as both operands take the same)
+    struct Raw {
+        u32x4 lo, hi;
+    };
+    auto fetch = [&](const unsigned char* at, auto row_bytes) __attribute__((always_inline)) {
+        Raw r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            r.lo[e] = *(const uint32_t*)(at + e * 4 * decltype(row_bytes)::value);
+            r.hi[e] = *(const uint32_t*)(at + (e + 4) * 4 * decltype(row_bytes)::value);
+        }
+        return r;
+    };
+    constexpr std::integral_constant<int, C::ROWB_A> kRowA{};
+    constexpr std::integral_constant<int, C::ROWB_B> kRowB{};
 #pragma unroll
     for (int i = 0; i < C::TM; ++i) {
         const int byte = (wave_m * C::WM + i * 16 + l16) * 4;
-        a_off[i] = q * C::ROWB_A + (((byte >> 4) ^ C::key_a(q)) << 4) + (byte & 15);
+        a_off[i] = (kRow0 + q) * C::ROWB_A + (((byte >> 4) ^ C::key_a(q)) << 4) + (byte & 15);
     }
 #pragma unroll
     for (int j = 0; j < C::TN; ++j) {
         const int byte = (wave_n * C::WN + j * 16 + l16) * 4;
-        b_off[j] = C::A_BYTES + q * C::ROWB_B + (((byte >> 4) ^ C::key_b(q)) << 4) + (byte & 15);
+        b_off[j] = C::A_BYTES + (kRow0 + q) * C::ROWB_B + (((byte >> 4) ^ C::key_b(q)) << 4) + (byte & 15);
     }
     using f32x4 = float __attribute__((ext_vector_type(4)));
-    // A running sum loses about a unit in the last place of itself with every addition: it is folded into a second one every 256
-    // pairs, so that a segment may be long (error against 64-bit sums, 96 channels: 667 763 voxels 3.5e-7, tiled kernel 9.8e-7).
-    constexpr int kFoldSteps = 256 / C::P;
-    int stage = 0;
+    int stage = 0, last_stage = 0;
+    uint32_t segments = 0;
     while (m.live) {
         const int nsteps = (int)((m.k_hi - m.k + C::P - 1) / C::P);
         f32x4 acc[C::TM][C::TN], sum[C::TM][C::TN];
@@ -413,30 +438,95 @@ __device__ __forceinline__ void multiply_f32(const unsigned char* ring, W m, con
             __builtin_amdgcn_s_barrier();           // the loaders saw this step's rows land
             asm volatile("" ::: "memory");
             const unsigned char* cur = ring + stage * C::STAGE_BYTES;
+            last_stage = stage;
             stage = stage + 1 == C::S ? 0 : stage + 1;
+            if constexpr (HALF < 0) {
 #pragma unroll
-            for (int kb = 0; kb < C::P / 4; ++kb) {
-                float af[C::TM], bf[C::TN];
+                for (int kb = 0; kb < C::P / 4; ++kb) {
+                    float af[C::TM], bf[C::TN];
 #pragma unroll
-                for (int i = 0; i < C::TM; ++i) af[i] = *(const float*)(cur + a_off[i] + kb * 4 * C::ROWB_A);
+                    for (int i = 0; i < C::TM; ++i) af[i] = *(const float*)(cur + a_off[i] + kb * 4 * C::ROWB_A);
 #pragma unroll
-                for (int j = 0; j < C::TN; ++j) bf[j] = *(const float*)(cur + b_off[j] + kb * 4 * C::ROWB_B);
+                    for (int j = 0; j < C::TN; ++j) bf[j] = *(const float*)(cur + b_off[j] + kb * 4 * C::ROWB_B);
 #pragma unroll
-                for (int i = 0; i < C::TM; ++i)
+                    for (int i = 0; i < C::TM; ++i)
 #pragma unroll
-                    for (int j = 0; j < C::TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j], af[i], acc[i][j], 0, 0, 0);
+                        for (int j = 0; j < C::TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j], af[i], acc[i][j], 0, 0, 0);
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // done reading this stage
+                continue;
+            }
+            // (where registers are left, every fragment is on its way before the first is taken apart)
+            Raw rows_raw[C::TM], cols_raw = fetch(cur + b_off[0], kRowB);
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i) rows_raw[i] = fetch(cur + a_off[i], kRowA);
+            if (C::TM < 3) __builtin_amdgcn_sched_barrier(0);
+            Split3 cols3 = split3<HALF == 1>(cols_raw.lo, cols_raw.hi), rows3[C::TM];
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i) rows3[i] = split3(rows_raw[i].lo, rows_raw[i].hi);
+#pragma unroll
+            for (int j = 0; j < C::TN; ++j) {
+                if (j + 1 < C::TN) cols_raw = fetch(cur + b_off[j + 1], kRowB);
+#pragma unroll
+                for (int p = 0; p < kSplit3Products; ++p)
+#pragma unroll
+                    for (int i = 0; i < C::TM; ++i) mma_split3(acc[i][j], cols3, rows3[i], p);
+                if (j + 1 < C::TN) cols3 = split3<HALF == 1>(cols_raw.lo, cols_raw.hi);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // done reading this stage
         }
         float* dst = partial + ((size_t)group + m.item) * (4 * C::WM * C::WN);     // the segment's slot: a whole tile
+        auto next = [&]() {
+            m.k = m.k_hi;
+            m.item = after(m.item);
+            seek(m);
+        };
+        auto at = [&](int i, int j) { return (f32x4*)(dst + (wave_m * C::WM + i * 16 + l16) * (2 * C::WN) + wave_n * C::WN + j * 16 + q * 4); };
+        if constexpr (HALF < 0) {
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j) *at(i, j) = sum[i][j] + acc[i][j];
+            next();
+            continue;
+        }
+        bool fine = true;
 #pragma unroll
         for (int i = 0; i < C::TM; ++i)
 #pragma unroll
-            for (int j = 0; j < C::TN; ++j)
-                *(f32x4*)(dst + (wave_m * C::WM + i * 16 + l16) * (2 * C::WN) + wave_n * C::WN + j * 16 + q * 4) = sum[i][j] + acc[i][j];
-        m.k = m.k_hi;
-        m.item = after(m.item);
-        seek(m);
+            for (int j = 0; j < C::TN; ++j) {
+                sum[i][j] += acc[i][j];
+                if (HALF == 1) sum[i][j] = -sum[i][j];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) fine = fine && split3_holds(sum[i][j][e]);
+            }
+        if (__ballot(!fine) != 0) again(m, sum);
+        // The halves meet in the stage that was multiplied last, which the loaders leave alone until both have been at the next barrier: one
+        // waits until nobody reads it any more, the other for the sums.
+        ++segments;
+        f32x4* const mine = (f32x4*)(ring + last_stage * C::STAGE_BYTES) + (wave_m * 2 + wave_n) * (C::TM * C::TN * 64) + lane;
+        if (lane == 0) atomicAdd(&sync[0], 1u);
+        auto wait_for = [&](const uint32_t* word, uint32_t least) {
+            while (*(const volatile uint32_t*)word < least) __builtin_amdgcn_s_sleep(1);
+            asm volatile("" ::: "memory");
+        };
+        if (HALF == 1) {
+            wait_for(&sync[0], 8u * segments);
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j) mine[(i * C::TN + j) * 64] = sum[i][j];
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (lane == 0) *(volatile uint32_t*)&sync[1 + wave_m * 2 + wave_n] = segments;
+        } else {
+            wait_for(&sync[1 + wave_m * 2 + wave_n], segments);
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j) *at(i, j) = sum[i][j] + mine[(i * C::TN + j) * 64];
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+        next();
     }
 }
 
@@ -496,7 +586,7 @@ __device__ __forceinline__ uint64_t split_cut(unsigned w, unsigned runs, const u
 }
 
 template <typename Tag, int BM, int BN>
-__global__ void __launch_bounds__(64 * (4 + kWsLoaders))
+__global__ void __launch_bounds__((WStreamCfg<Tag, BM, BN>::NT))
 wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename Tag::type* __restrict__ feats,
                     const uint32_t* __restrict__ sig_i, const uint32_t* __restrict__ sig_o,
                     const uint32_t* __restrict__ bounds, int V, int Ci, int Co, unsigned nb, unsigned co_tiles,
@@ -515,7 +605,7 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool loader = wave >= C::NW;
     const int lw = loader ? wave - C::NW : 0, mw = loader ? 0 : wave;
-    const int wave_m = C::KSPLIT ? 0 : mw >> 1, wave_n = C::KSPLIT ? 0 : mw & 1;
+    const int wave_m = C::KSPLIT ? 0 : (mw & 3) >> 1, wave_n = C::KSPLIT ? 0 : mw & 1;
     const int g = lane >> 5, l32 = lane & 31;
 
     // ---- item list: block-major (block, offset, tile); XCD x owns the x-th eighth, its workgroups interleave ----
@@ -540,6 +630,7 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
     if constexpr (ES == 4) {
         uint32_t* pre = (uint32_t*)bands;
         if (wave == 0) split_prefix(bounds, (unsigned)V, nb, pre);
+        if (tid < (int)kSplitSyncWords) pre[kSplitMaxUnits + 1 + tid] = 0u;
         __syncthreads();
         const uint64_t cut = split_cut(group + (lane & 1), gridDim.x, bounds, (unsigned)V, nb, tiles, pre);
         run_lo = ((uint64_t)__builtin_amdgcn_readlane((int)(cut >> 32), 0) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)cut, 0);
@@ -744,7 +835,45 @@ wgrad_stream_kernel(const typename Tag::type* __restrict__ gout, const typename 
     // =================================================================================================
     __syncthreads();                                // the loaders' prologue barrier
     if constexpr (ES == 4) {
-        multiply_f32<C>(ring, first, seek, after, wave_m, wave_n, group, partial);
+        // a segment with a sum that the three-part products cannot stand for: multiplied again, on the fp32 units, from memory
+        auto again = [&](const Walk& w, auto& sum) {
+            const int l16 = lane & 15, q = lane >> 4, half = mw >> 2;
+            const int row0 = (int)w.co_tile * BM + wave_m * C::WM + l16, col0 = (int)w.ci_tile * BN + wave_n * C::WN + l16;
+            using f32x4 = float __attribute__((ext_vector_type(4)));
+            f32x4 acc[C::TM][C::TN];
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j) acc[i][j] = sum[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (uint32_t k = w.k; k < w.k_hi; k += 4) {
+                if (((k - w.k) & 32u) != (uint32_t)half * 32u) continue;        // (the other half of a step's pairs)
+                const bool live = k + q < w.k_hi;
+                const size_t o = live ? sig_o[k + q] : 0u, at = live ? sig_i[k + q] : 0u;
+                float af[C::TM], bf[C::TN];
+#pragma unroll
+                for (int i = 0; i < C::TM; ++i) af[i] = live && row0 + i * 16 < Co ? gout[o * Co + row0 + i * 16] : 0.f;
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j) bf[j] = live && col0 + j * 16 < Ci ? feats[at * Ci + col0 + j * 16] : 0.f;
+#pragma unroll
+                for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < C::TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(bf[j], af[i], acc[i][j], 0, 0, 0);
+                if ((k - w.k) % 32 == 28 || k + 4 >= w.k_hi) {
+#pragma unroll
+                    for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                        for (int j = 0; j < C::TN; ++j) {
+                            sum[i][j] += acc[i][j];
+                            acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                        }
+                }
+            }
+        };
+        uint32_t* sync = (uint32_t*)bands + kSplitMaxUnits + 1;
+        if constexpr (C::HALVES == 1) multiply_f32<C, -1>(ring, sync, first, seek, after, again, wave_m, wave_n, group, partial);
+        else if (mw >> 2) multiply_f32<C, 1>(ring, sync, first, seek, after, again, wave_m, wave_n, group, partial);
+        else multiply_f32<C, 0>(ring, sync, first, seek, after, again, wave_m, wave_n, group, partial);
     } else {
     const int s16 = lane & 15, mb = (lane >> 4) & 1;
     constexpr int NK = P / 16 / C::SLICES;          // k-blocks (16 pair rows) this wavefront multiplies per step
@@ -1630,12 +1759,16 @@ __global__ void __launch_bounds__(256) split_reduce_kernel(const float* __restri
     for (int e = 0; e < 4; ++e) dst[e] = sum[e];
 }
 
-template <int TILE>
+// fp32 weight gradient of few pairs: measured (us, parts and units): 96 channels, one tile, 4 083 voxels 30.6 27.7, 8 004 34.9 34.1, 10 494 36.7 37.4;
+// 64 channels 5 876 24.2 22.2, 13 258 30.3 29.9, 16 307 31.1 31.9;  128 channels, four tiles, 2 581 27.5 26.2, 4 083 31.6 31.6;  192 channels 2 581 37.0 36.7.
+bool units_are_faster(size_t n, unsigned tiles, int tile) { return n * tiles < (tile == 96 ? 9216u : 14336u); }
+
+template <typename Tag, int TILE>
 int launch_wgrad_split(const void* gout, const void* feats, const uint32_t* sig_i, const uint32_t* sig_o, const uint32_t* bounds, uint32_t pairs,
                        size_t n, size_t n_in, int V, int Ci, int Co, unsigned nb, unsigned groups, float* partial, float* gw, hipStream_t s) {
-    using C = WStreamCfg<F32, TILE, TILE>;
+    using C = WStreamCfg<Tag, TILE, TILE>;
     const unsigned co_tiles = cdiv(Co, TILE), ci_tiles = cdiv(Ci, TILE);
-    auto kern = wgrad_stream_kernel<F32, TILE, TILE>;
+    auto kern = wgrad_stream_kernel<Tag, TILE, TILE>;
     static thread_local bool lds_raised = false;
     if (!lds_raised) {
         FGX_CHECK_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::lds_bytes));
@@ -1689,7 +1822,9 @@ int fgx_conv_wgrad_split(const void* grad_out, const void* feats, const uint32_t
         rc = fgx_colsum(FGX_F32, grad_out, n, Co, (char*)scratch + (bytes - fgx_colsum_scratch_bytes(n, Co)), grad_bias, stream);
         if (rc != FGX_OK) return rc;
     }
-    auto launch = tile == 96 ? launch_wgrad_split<96> : launch_wgrad_split<64>;
+    const bool units = units_are_faster(n, cdiv(Co, tile) * cdiv(Ci, tile), tile);
+    auto launch = tile == 96 ? (units ? launch_wgrad_split<F32Units, 96> : launch_wgrad_split<F32, 96>)
+                             : (units ? launch_wgrad_split<F32Units, 64> : launch_wgrad_split<F32, 64>);
     return launch(grad_out, feats, sig_i, sig_o, block_bounds, seg_host[V], n, n_in, V, Ci, Co, nb, groups, (float*)scratch, (float*)grad_weight,
                   (hipStream_t)stream);
 }

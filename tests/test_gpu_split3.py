@@ -1,12 +1,13 @@
-"""fp32 products made of bf16 parts: the streaming kernel's tiles and the pairs kernel against 64-bit sums, and the repeat on the fp32 units where
-the parts cannot stand for a value (infinities, NaN, values that round to an infinity, values under 2^-110)."""
+"""fp32 products made of bf16 parts: the streaming kernel's tiles, the pairs kernel and the weight gradient against 64-bit sums, and the repeat on
+the fp32 units where the parts cannot stand for a value (infinities, NaN, values that round to an infinity, values under 2^-110)."""
 import pytest
 import torch
 
 from flexgemm_amd import _native as nat
-from flexgemm_amd.ops.spconv import sparse_submanifold_conv3d
+from flexgemm_amd.ops.spconv import SubMConv3dFunction, sparse_submanifold_conv3d
 from flexgemm_amd.workloads import reference_test_shell
 from test_gpu_nonfinite import INF, NAN, _agree, _defined, _spoil
+from test_gpu_wgrad_split import coords_of
 
 pytestmark = pytest.mark.gpu
 
@@ -67,3 +68,53 @@ def test_what_three_parts_cannot_stand_for(monkeypatch, tile, ci, co):
 def test_small_values_keep_their_bits(monkeypatch, tile, ci, co):
     got, want, _ = _layer(monkeypatch, tile, 16, ci, co, scale=1e-34)
     assert float((got.double() - want).norm() / want.norm()) <= (27 * ci) ** 0.5 * 2.0 ** -24
+
+
+def _weight_grad(n, ci, co, scale=1.0, change=None):
+    """The weight gradient, the same in 64 bits, and each sum's magnitude, of n voxels in a cube two thirds full."""
+    side = round((1.5 * n) ** (1 / 3)) + 1
+    cache = SubMConv3dFunction._compute_neighbor_cache(coords_of(n, side, n), torch.Size([1, ci, side, side, side]), (3, 3, 3), (1, 1, 1), True)
+    g = torch.Generator(device="cuda").manual_seed(n + ci)
+    feats, grad = torch.randn(n, ci, generator=g, device="cuda") * scale, torch.randn(n, co, generator=g, device="cuda")
+    if change is not None:
+        change(feats, grad)
+    got = nat.host().wgrad(grad, feats, cache, 27, False, -1)[0].view(co, 27, ci)
+    nmap = cache["neighbor_map"].view(torch.int32).cpu().long()
+    f, u = feats.cpu().double(), grad.cpu().double()
+    want, size = torch.zeros(co, 27, ci, dtype=torch.double), torch.zeros(co, 27, ci, dtype=torch.double)
+    for v in range(27):
+        r = (nmap[:, v] >= 0).nonzero()[:, 0]
+        want[:, v], size[:, v] = u[r].T @ f[nmap[r, v]], u[r].abs().T @ f[nmap[r, v]].abs()
+    return got.cpu().double(), want, size
+
+
+# both tiles, channels that end inside one, segments of several folds and of less than half a step, two tiles, more than sixteen; rows on both sides
+# of where the fp32 units end
+SPLIT_GRADS = [(9215, 96, 96), (9216, 96, 96), (12001, 96, 92), (14335, 64, 64), (14336, 64, 64), (20000, 52, 60), (8000, 112, 48), (3001, 192, 180),
+               (1024, 320, 260), (9000, 32, 64)]
+
+
+@pytest.mark.parametrize("n,ci,co", SPLIT_GRADS)
+@pytest.mark.parametrize("scale", [1.0, 1e-34])
+def test_weight_gradient(n, ci, co, scale):
+    got, want, size = _weight_grad(n, ci, co, scale)
+    # k products summed in any order: within k units of the sum of their magnitudes; sums of random signs, on the whole, within sqrt(k) of their own size
+    assert bool(((got - want).abs() <= n * 2.0 ** -23 * size + 2.0 ** -149 * n).all())
+    assert float((got - want).norm() / want.norm()) <= n ** 0.5 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("n,ci,co", [(9216, 96, 96), (14336, 64, 64), (3001, 192, 180)])
+def test_weight_gradient_of_what_three_parts_cannot_stand_for(n, ci, co):
+    def change(feats, grad):
+        _spoil(feats, [(7, 3, INF), (n - 31, ci - 1, -INF), (60, 0, NAN), (200, 2, 3.4e38)])
+        _spoil(grad, [(8, 1, INF), (n - 5, co - 1, NAN), (300, 5, -INF)])
+    got, want, size = _weight_grad(n, ci, co, change=change)
+    fine = want.isfinite() & (size < 1e30)
+    assert fine.any() and (~want.isfinite()).any() and (size[want.isfinite()] > 1e30).any()
+    assert bool(((got - want).abs() <= n * 2.0 ** -23 * size)[fine].all())
+    odd = ~want.isfinite()
+    assert not got[odd].isfinite().any()
+    odd[:, :, 2] = False            # (3.4e38 times more than one is an infinity of either sign in 32 bits)
+    assert torch.equal(got[odd].isnan(), want[odd].isnan()) and torch.equal(got[odd].nan_to_num(0), want[odd].nan_to_num(0))
+    huge = want.isfinite() & ~fine & (want.abs() < 3e38)
+    assert bool(((got - want).abs() <= n * 2.0 ** -23 * size)[huge].all())
