@@ -1,4 +1,4 @@
-// Streaming masked implicit GEMM (forward and dgrad) for large voxel counts on gfx950.
+// Streaming masked implicit GEMM (forward and dgrad) on gfx950, from a few thousand voxels on.
 //
 //   out[order[r], :] = sum over offsets v present for row r of src[map[order[r], v], :] x panel_v (+ bias)
 //
@@ -621,6 +621,15 @@ int dispatch_stream(int tile_rows, int tile_cols, int slab_bytes, const void* sr
     FGX_STREAM_TILE(256, 128, 4, 2, 4)      // 64-byte K-slabs: rows shorter than 128 bytes
     FGX_STREAM_TILE(256, 64, 4, 2, 4)
     FGX_STREAM_TILE(256, 32, 8, 1, 4)
+    // A chip that the tiles above leave partly empty.  Bound by their loads, at 34 bytes a cycle and CU like the larger ones: four multipliers keep up, and
+    // rings of 4, 6 and 8 stages (with as many steps' loads in flight) or the next step's fragments read beside this one's products were level or
+    // up to 3 us behind (10 494 voxels, 128 channels, 64 x 128: 26.2 us, six stages 29.9, fragments ahead 26.2).
+    if constexpr (sizeof(typename Tag::type) == 2) {
+        FGX_STREAM_TILE(64, 64, 2, 2, 8)
+        FGX_STREAM_TILE(64, 128, 2, 2, 8)
+        FGX_STREAM_TILE(128, 64, 4, 1, 8)
+        FGX_STREAM_TILE(128, 128, 2, 2, 8)
+    }
 #undef FGX_STREAM_TILE
     set_error("fgx_conv_gather_gemm_stream: no kernel for tile %dx%d with %d-byte slabs", tile_rows, tile_cols, slab_bytes);
     return FGX_ERR_UNSUPPORTED;
@@ -704,6 +713,10 @@ bool stream_lds_fits(int tile_rows, int tile_cols, int slab_bytes, int cols) {
     FGX_STREAM_TILE(256, 128, 4, 2, 4)
     FGX_STREAM_TILE(256, 64, 4, 2, 4)
     FGX_STREAM_TILE(256, 32, 8, 1, 4)
+    FGX_STREAM_TILE(64, 64, 2, 2, 8)        // (16-bit types)
+    FGX_STREAM_TILE(64, 128, 2, 2, 8)
+    FGX_STREAM_TILE(128, 64, 4, 1, 8)
+    FGX_STREAM_TILE(128, 128, 2, 2, 8)
 #undef FGX_STREAM_TILE
     return fixed != 0 && fixed + bias_bytes <= 160 * 1024;
 }
@@ -724,9 +737,15 @@ extern "C" int fgx_conv_gather_gemm_stream_groups(int dtype, int cols, int tile_
     FGX_STREAM_TILE(TAG, 256, 128, 4, 2, 4) \
     FGX_STREAM_TILE(TAG, 256, 64, 4, 2, 4)  \
     FGX_STREAM_TILE(TAG, 256, 32, 8, 1, 4)
-    if (dtype == FGX_F16) { FGX_STREAM_TILES(F16) }
-    else if (dtype == FGX_BF16) { FGX_STREAM_TILES(BF16) }
+#define FGX_SMALL_TILES(TAG)            \
+    FGX_STREAM_TILE(TAG, 64, 64, 2, 2, 8)   \
+    FGX_STREAM_TILE(TAG, 64, 128, 2, 2, 8)  \
+    FGX_STREAM_TILE(TAG, 128, 64, 4, 1, 8)  \
+    FGX_STREAM_TILE(TAG, 128, 128, 2, 2, 8)
+    if (dtype == FGX_F16) { FGX_STREAM_TILES(F16) FGX_SMALL_TILES(F16) }
+    else if (dtype == FGX_BF16) { FGX_STREAM_TILES(BF16) FGX_SMALL_TILES(BF16) }
     else { FGX_STREAM_TILES(F32) }
+#undef FGX_SMALL_TILES
 #undef FGX_STREAM_TILES
 #undef FGX_STREAM_TILE
     set_error("fgx_conv_gather_gemm_stream_groups: no kernel for tile %dx%d with %d-byte slabs", tile_rows, tile_cols, slab_bytes);

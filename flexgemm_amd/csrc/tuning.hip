@@ -8,6 +8,7 @@
 #include "fgx_common.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace fgx {
 namespace {
@@ -107,6 +108,54 @@ void rule_gemm_f32(size_t n, int K, int cols, int V, fgx_schedule* out) {
             *out = fgx_schedule{sh.rows, sh.cols, sh.slab, 1, 0, 1};
         }
     }
+}
+
+// 16-bit gather GEMM where tiles of 256 rows leave CUs idle or fill them unevenly: streaming tiles of 64 and 128 rows, two workgroups to a CU but
+// for 128 x 128.  A step of any tile takes a CU about as long as its loads do (34 bytes a cycle), so small tiles, which load more for a product, are behind
+// once the chip is full, and ahead before: 64 x 64 goes through an item of one slab in 5.4 us, 256 x 128 in 15.  They also pad less.
+// With items per CU x, slabs s: s (L^1.5 + (x P)^1.5)^(2/3), where L is what an item takes alone and P beside others (us; the tile of 256 rows: whole rounds).
+// Measured forward, us, what was chosen before and now, 27 offsets:
+//   channels        8 004 voxels   10 494       15 091      20 574      28 169      36 575      75 224      166 977
+//    64 ->  64        18.6         20.3 16.3    23.1 16.3   24.7 17.1   27.9 18.2   24.7 19.8   28.8 24.4   45.9 37.6
+//   128 -> 128        35.0 22.9    35.4 26.4    36.8 25.7   36.3 28.8   36.7 29.5   40.7 34.4   51.8        85.7
+//   192 -> 192        43.1 33.6    62.1 34.1    49.3 40.6   48.8 44.6   54.8        71.4 64.0   105.9       198
+//   256 -> 256        65.2 42.1    60.5 53.1    60.7        67.2        71.7        89.2        145.9       271
+//   512 ->  64        54.7         60.5 56.3                100.8 56.6              165.9 75.9  156.0 135.1 300 276
+//    64 -> 256        26.3 18.9    26.3 22.7                28.2                    33.0        46.5        83.1
+// (where one figure stands, the tile stays.)  The tiled kernel splits few rows well: under up to 64 columns, or rows of 512 bytes and more, it is level up
+// to 10 000 voxels (8 004: 96 -> 64 21.0 22.3, 384 -> 96 43 47, 768 -> 128 64 83), otherwise up to 5 000 (4 947: 80 -> 80 21.0 22.7); and it wants no gather
+// plan and no packed weight, 14 us of the host's time in a training pass on new coordinates, which little work does not bring in (64 -> 64 at 10 494 voxels
+// gains 3.5 us a product, at 28 169 9.7).  Past 131 072 voxels the plan of shorter tiles costs a new cache what a product gains (64 -> 64, 229 217
+// voxels: kept 53.9 49.4, new 145.0 151.7).
+bool small_stream_tile(size_t n, int K, int cols, fgx_schedule* out) {
+    const int slabs = (int)cdiv((size_t)K * 2, (size_t)128);
+    if (K * 2 <= 64 || cols <= 32 || !stream_lds_fits(256, 128, 128, cols)) return false;
+    if (n > 131072 || (!out->stream && (n < (cols <= 64 || K >= 256 ? 10240u : 5120u) || n * slabs * cdiv(cols, 64) < 24576))) return false;
+    auto take = [&](int rows, int wide) {
+        *out = fgx_schedule{rows, wide, 128, 1, 0, 1};
+        return true;
+    };
+    if (cols <= 64) return take(n <= (slabs == 1 ? 36864u : slabs == 2 ? 57344u : 131072u) ? 64 : 128, 64);
+    // long rows under one tile of columns: 75 224 voxels, 384 -> 96 132 120, 768 -> 128 270 251
+    if (cols <= 128 && K >= 384 && n >= 28672) return take(128, 128);
+    if (cols > 192 && K >= 192 && n > 12288) return false;              // (the larger tiles fill the chip by then)
+    const bool whole_chip = out->stream && out->tile_cols != 64;        // (256 x 128 and 128 x 256 tiles for at least half of the CUs)
+    if (whole_chip && (cols > 128 || n > 40960)) return false;
+    struct Shape { int rows, cols; double alone, beside; };
+    const Shape shapes[] = {{64, 64, 5.4, 2.9}, {64, 128, 7.0, 3.7}, {128, 64, 7.45, 4.0}, {128, 128, 10.3, 6.5}};
+    auto per_cu = [&](int rows, int wide) { return (double)cdiv(n, rows) * cdiv(cols, wide) / kCUs; };
+    // (a tile that was chosen for its rounds: a whole one at the least, and most of one for each of its items)
+    double best = 1e30;
+    if (out->stream) best = 0.97 * (whole_chip ? 15.0 : 11.9) * std::max(1.0, 0.45 + 0.68 * per_cu(out->tile_rows, out->tile_cols));
+    bool found = false;
+    for (const Shape& sh : shapes) {
+        const double time = std::pow(std::pow(sh.alone, 1.5) + std::pow(per_cu(sh.rows, sh.cols) * sh.beside, 1.5), 2.0 / 3.0);
+        if (time < best) {
+            best = time;
+            found = take(sh.rows, sh.cols);
+        }
+    }
+    return found;
 }
 
 void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* out) {
@@ -350,6 +399,7 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
             *out = fgx_schedule{sh.rows, sh.cols, sh.slab, 1, 0, 1};
         }
     }
+    if (V > 8 && small_stream_tile(n, K, cols, out)) return;
     if (out->stream) return;
     // (not for an input gradient of a single tile of rows under a small weight: 192 voxels, 256 <- 768 channels 0.029 ms, 64 x 64 tiles 0.023)
     if (row_bytes >= 1024 && cols >= 128 && !(pass_kind != 0 && n < 256 && (size_t)K * cols < (size_t)512 * 512)) {

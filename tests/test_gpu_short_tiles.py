@@ -1,0 +1,74 @@
+"""Streaming tiles of 64 and 128 rows (16-bit types): the same bits as tiles of 256 rows at the edges of tiles, slabs and rounds of items, and the
+shapes that the schedule gives them."""
+import pytest
+import torch
+
+from flexgemm_amd import _native as nat
+from flexgemm_amd.ops.spconv import sparse_submanifold_conv3d_relu
+from test_gpu_wgrad_split import coords_of
+
+TILES = [(64, 64), (64, 128), (128, 64), (128, 128)]
+
+
+def _layer(monkeypatch, tile, n, side, ci, co, dtype):
+    coords = coords_of(n, side, n)
+    g = torch.Generator(device="cuda").manual_seed(n + ci)
+    feats = torch.randn(n, ci, generator=g, device="cuda").to(dtype).requires_grad_()
+    weight = (torch.randn(co, 3, 3, 3, ci, generator=g, device="cuda") / (27 * ci) ** 0.5).to(dtype).requires_grad_()
+    bias = torch.randn(co, generator=g, device="cuda").to(dtype).requires_grad_()
+    nat.host()                  # (takes note of the table before it is replaced)
+    real = nat.table_lookup
+
+    def lookup(kind, *a, **k):
+        s = real(kind, *a, **k)
+        if kind != nat.PASS_WGRAD:
+            s.tile_rows, s.tile_cols, s.slab_bytes, s.splitk, s.stream = *tile, 128, 1, 1
+        return s
+    monkeypatch.setattr(nat, "table_lookup", lookup)
+    out, cache = sparse_submanifold_conv3d_relu(feats, coords, torch.Size([1, ci, side, side, side]), weight, bias)
+    out.backward(torch.randn(out.shape, generator=g, device="cuda").to(dtype))
+    monkeypatch.setattr(nat, "table_lookup", real)
+    return out.detach(), feats.grad, weight.grad, feats.detach(), weight.detach(), bias.detach(), cache
+
+
+# one row, a band and a tile more or less one row; K and columns that end inside a slab, a piece and a tile; 1 300 tiles of 64 rows by two of columns, more than
+# two workgroups a CU take in one round
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n,side,ci,co", [(1, 4, 64, 64), (63, 8, 40, 72), (65, 8, 136, 40), (129, 8, 96, 200), (1000, 12, 72, 136), (83201, 96, 40, 72)])
+def test_same_bits_as_the_long_tiles(monkeypatch, dtype, n, side, ci, co):
+    want = _layer(monkeypatch, (256, 64), n, side, ci, co, dtype)
+    for tile in TILES:
+        got = _layer(monkeypatch, tile, n, side, ci, co, dtype)
+        for a, b in zip(got[:3], want[:3]):
+            assert torch.equal(a, b), tile
+    out, _, _, feats, weight, bias, cache = want
+    nmap = cache["neighbor_map"].view(torch.int32).long()
+    w = weight.reshape(co, 27, ci).float()
+    ref = bias.float().expand(n, co).clone()
+    for v in range(27):
+        have = (nmap[:, v] >= 0).nonzero()[:, 0]
+        ref[have] += feats[nmap[have, v]].float() @ w[:, v].t()
+    # one rounding to the type of sums of about one, added in 32 bits in another order
+    unit = torch.finfo(dtype).eps
+    assert bool(((out.float() - ref.relu()).abs() <= unit * ref.abs() + 27 * ci * 2.0 ** -23).all())
+
+
+@pytest.mark.parametrize("n,ci,co,tile", [
+    (5119, 192, 192, None), (5120, 192, 192, (64, 64)), (10239, 512, 64, None), (10240, 512, 64, (64, 64)), (24575, 64, 64, None), (24576, 64, 64, (64, 64)),
+    (36864, 64, 64, (64, 64)), (36865, 64, 64, (128, 64)), (131072, 64, 64, (128, 64)), (131073, 64, 64, (256, 64)), (20574, 128, 128, (64, 128)),
+    (57345, 128, 128, (256, 128)), (12288, 256, 256, (64, 128)), (12289, 256, 256, (256, 64)), (28672, 384, 96, (128, 128)), (20000, 32, 64, None)])
+def test_rule(n, ci, co, tile):
+    s = nat.table_lookup(nat.PASS_FWD, torch.float16, n, ci, co, 27)
+    got = (s.tile_rows, s.tile_cols) if s.stream else None
+    if tile is None:
+        assert got is None
+    else:
+        assert got == tile and (s.tile_rows == 256 or (s.slab_bytes, s.splitk) == (128, 1))
+
+
+@pytest.mark.parametrize("n,ci,co", [(5120, 192, 192), (20574, 128, 128), (36864, 64, 64), (12288, 256, 256)])
+def test_not_under_few_offsets_or_in_fp32(n, ci, co):
+    for dtype, v in ((torch.float16, 8), (torch.float32, 27)):
+        s = nat.table_lookup(nat.PASS_FWD, dtype, n, ci, co, v)
+        assert not s.stream or 256 in (s.tile_rows, s.tile_cols)
