@@ -598,7 +598,7 @@ __global__ void __launch_bounds__(kOrderThreads) chunk_tables_kernel(const int32
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// One workgroup per tile: plan_idx[plan_seg[t] + k][r] = map[order[t * tile_rows + r]][k-th offset present in the tile]
+// A workgroup per tile, or per two or four short ones (fill_together): plan_idx[plan_seg[t] + k][r] = map[order[t * tile_rows + r]][k-th offset present in the tile]
 // (EMPTY for rows past the end); plan_band[plan_seg[t] + k] (optional) has bit b set when rows [32 b, 32 b + 32) of the
 // tile hold at least one present neighbor for that offset.
 //
@@ -609,10 +609,10 @@ __global__ void __launch_bounds__(kOrderThreads) chunk_tables_kernel(const int32
 //
 // TABLES: a workgroup adds up the counts of the tiles before its own itself (and leaves them in seg and plan_seg), and the first one
 // (item_at) deals the item order beside them.  One workgroup that scanned and dealt before the others could start took 15.7 us for
-// 1 306 tiles: tables and fill 34.1 -> 17.8 us (and for the two maps of a 2 x 2 x 2 stride over a 256^3 shell 34.0 -> 18.3).  Up to
+// 1 306 tiles: tables and fill 34.1 -> 17.8 us, 12.5 with two tiles a workgroup (and for the two maps of a 2 x 2 x 2 stride over a 256^3 shell 34.0 -> 18.3).  Up to
 // kFillScanTiles tiles: the additions are quadratic.
 // ---------------------------------------------------------------------------------------------------------------
-constexpr int kFillThreads = 512, kFillRows = 256;
+constexpr int kFillThreads = 512, kFillRows = 256, kFillTogether = 4;
 constexpr unsigned kFillScanTiles = 4096;
 
 template <bool TABLES>
@@ -621,10 +621,10 @@ __global__ void __launch_bounds__(kFillThreads) plan_fill_kernel(const uint32_t*
                                                                  int tile_rows, int R, int32_t* __restrict__ seg, int32_t* __restrict__ plan_seg,
                                                                  uint32_t* __restrict__ plan_idx, uint32_t* __restrict__ plan_band,
                                                                  unsigned col_tiles, unsigned slabs, unsigned groups, uint32_t* __restrict__ sorted,
-                                                                 uint32_t* __restrict__ item_at) {
+                                                                 uint32_t* __restrict__ item_at, int together) {
     extern __shared__ uint32_t stage[];              // R map rows of V words; the item order's sorted list in the workgroup that makes it
     __shared__ int64_t src_row[kFillRows];           // which map row each of them is (-1: past the end)
-    __shared__ uint32_t bands[32], offsets[32];
+    __shared__ uint32_t bands[kFillTogether][32], offsets[kFillTogether][32];
     const int tid = threadIdx.x, lane = tid & 63;
     size_t t = blockIdx.x;
     if constexpr (TABLES) {
@@ -637,13 +637,17 @@ __global__ void __launch_bounds__(kFillThreads) plan_fill_kernel(const uint32_t*
             --t;
         }
     }
+    t *= (size_t)together;                           // the first of this workgroup's tiles
+    const int all_rows = together * tile_rows;
     auto fetch_order = [&](int r0) {
         if (tid < R) {
             const size_t row = t * (size_t)tile_rows + r0 + tid;
-            src_row[tid] = (r0 + tid < tile_rows && row < n) ? order[row] : (int64_t)-1;
+            src_row[tid] = (r0 + tid < all_rows && row < n) ? order[row] : (int64_t)-1;
         }
     };
     fetch_order(0);
+    const int sub = together > 1 ? tid % R / tile_rows : 0;                 // this thread's tile (whole wavefronts share one)
+    const size_t own_tile = t + sub;
     size_t slot;
     if constexpr (TABLES) {
         __shared__ uint64_t part[kFillThreads / 64];
@@ -659,31 +663,37 @@ __global__ void __launch_bounds__(kFillThreads) plan_fill_kernel(const uint32_t*
         uint64_t before = 0;
 #pragma unroll
         for (int w = 0; w < kFillThreads / 64; ++w) before += part[w];
-        slot = (uint32_t)before;
-        const TilePrefix own = tile_counts(tile_code, (unsigned)t, (unsigned)num_tiles);
-        if (tid == 0) {
-            if (seg != nullptr) seg[t] = (int32_t)(before >> 32);
-            plan_seg[t] = (int32_t)slot;
-            if (t + 1 == num_tiles) {
-                if (seg != nullptr) seg[num_tiles] = (int32_t)((before >> 32) + own.at);
-                plan_seg[num_tiles] = (int32_t)(slot + own.plan_at);
+        TilePrefix upto;
+        upto.at = (uint32_t)(before >> 32);
+        upto.plan_at = (uint32_t)before;
+        slot = upto.plan_at;
+        for (int i = 0; i < together && t + i < num_tiles; ++i) {
+            if (tid == 0) {
+                if (seg != nullptr) seg[t + i] = (int32_t)upto.at;
+                plan_seg[t + i] = (int32_t)upto.plan_at;
+            }
+            const TilePrefix own = tile_counts(tile_code, (unsigned)(t + i), (unsigned)num_tiles);
+            upto.at += own.at;
+            upto.plan_at += own.plan_at;
+            slot += i < sub ? own.plan_at : 0u;
+            if (tid == 0 && t + i + 1 == num_tiles) {
+                if (seg != nullptr) seg[num_tiles] = (int32_t)upto.at;
+                plan_seg[num_tiles] = (int32_t)upto.plan_at;
             }
         }
     } else {
-        slot = (size_t)plan_seg[t];
+        slot = own_tile < num_tiles ? (size_t)plan_seg[own_tile] : 0;
     }
-    const uint32_t code = (uint32_t)tile_code[t];
-    if (code == 0) {
-        for (int r = tid; r < tile_rows; r += kFillThreads) plan_idx[slot * tile_rows + r] = FGX_EMPTY32;
-        if (plan_band != nullptr && tid == 0) plan_band[slot] = 0u;
-        return;
+    // (a tile without an offset owns one row of missing neighbors: any offset's)
+    const uint32_t given = own_tile < num_tiles ? (uint32_t)tile_code[own_tile] : 0u;
+    const uint32_t code = own_tile < num_tiles && given == 0u ? 1u : given;
+    const int ways = kFillThreads / R, way = tid / R, mine_r = tid % R;        // (whole wavefronts share a way)
+    const int cnt = __popc(code), in_tile = together > 1 ? mine_r % tile_rows : mine_r;
+    if (tid < R && in_tile < 32) {
+        bands[sub][in_tile] = 0u;
+        if (code >> in_tile & 1u) offsets[sub][__popc(code & ((1u << in_tile) - 1u))] = (uint32_t)in_tile;
     }
-    if (tid < 32) {
-        bands[tid] = 0u;
-        if (code >> tid & 1u) offsets[__popc(code & ((1u << tid) - 1u))] = (uint32_t)tid;
-    }
-    const int cnt = __popc(code), ways = kFillThreads / R, way = tid / R, mine_r = tid % R;        // (whole wavefronts share a way)
-    for (int r0 = 0; r0 < tile_rows; r0 += R) {
+    for (int r0 = 0; r0 < all_rows; r0 += R) {
         if (r0 > 0) {
             __syncthreads();                     // the previous chunk's rows have been consumed
             fetch_order(r0);
@@ -704,27 +714,35 @@ __global__ void __launch_bounds__(kFillThreads) plan_fill_kernel(const uint32_t*
             }
         }
         __syncthreads();
-        const int r = r0 + mine_r;
+        const int r = r0 + in_tile;
         for (int k = way; k < cnt; k += ways) {
-            const uint32_t m = stage[mine_r * V + offsets[k]];       // (a row past the end is EMPTY throughout)
+            const uint32_t m = stage[mine_r * V + offsets[sub][k]];  // (a row past the end is EMPTY throughout)
             if (r < tile_rows) plan_idx[(slot + k) * tile_rows + r] = m;
             if (plan_band != nullptr) {
                 const unsigned long long live = __ballot(m != FGX_EMPTY32);    // all 64 lanes take part
                 if (lane == 0) {
-                    const int b0 = (r0 + (mine_r & ~63)) >> 5;                 // band of this wavefront's lanes 0-31
+                    const int b0 = (r0 + (in_tile & ~63)) >> 5;                // band of this wavefront's lanes 0-31
                     uint32_t bits = ((live & 0xFFFFFFFFull) ? 1u : 0u) << (b0 & 31);
                     bits |= ((live >> 32) ? 1u : 0u) << ((b0 + 1) & 31);
-                    if (bits) atomicOr(&bands[k], bits);
+                    if (bits) atomicOr(&bands[sub][k], bits);
                 }
             }
         }
     }
     if (plan_band != nullptr) {
         __syncthreads();
-        if (tid < cnt) plan_band[slot + tid] = bands[tid];
+        if (tid < R && in_tile < cnt) plan_band[slot + in_tile] = bands[sub][in_tile];
     }
 }
 
+// Tiles of 64 or 128 rows that a workgroup fills together, as many rows at a time as of a longer one, once the workgroups left are as many as CUs: a workgroup
+// takes 6 us whatever its rows, and 1 024 of them fit the chip (64 rows, 1 149 tiles 18.9 -> 9.4 us, 2 611 41.5 -> 12.5, 3 817 55.7 -> 14.4; 128 rows,
+// 1 306 tiles 20.6 -> 12.5; 322 tiles of 64 rows, one each, 6.1, as many of 256 8.4).
+inline int fill_together(int tile_rows, size_t num_tiles) {
+    int t = 1;
+    while (tile_rows % 64 == 0 && 2 * t * tile_rows <= kFillRows && num_tiles >= (size_t)512 * t) t *= 2;
+    return t;
+}
 inline int fill_rows(int tile_rows) { return tile_rows <= 64 ? 64 : tile_rows <= 128 ? 128 : kFillRows; }
 inline size_t fill_lds(int tile_rows, int V) { return (size_t)fill_rows(tile_rows) * V * 4; }
 
@@ -1012,12 +1030,14 @@ int fgx_tile_plan(const int32_t* gray, const int64_t* order, const uint32_t* map
         scans = false;
     }
     const size_t items = item_at != nullptr ? num_tiles * (size_t)col_tiles : 0;
+    const int together = fill_together(tile_rows, num_tiles);
+    const unsigned fills = (unsigned)cdiv(num_tiles, (size_t)together);
     if (plan_idx != nullptr && num_tiles <= kFillScanTiles && items < ((size_t)1 << kItemBits) && (item_at == nullptr || groups <= kFillThreads)) {
-        const size_t lds = fill_lds(tile_rows, V), list = items <= kOrderInLds ? items * 4 : 0;
+        const size_t lds = fill_lds(together * tile_rows, V), list = items <= kOrderInLds ? items * 4 : 0;
         phase_mark("gather plan fill", s);
-        plan_fill_kernel<true><<<(unsigned)num_tiles + (item_at != nullptr ? 1u : 0u), kFillThreads, lds > list ? lds : list, s>>>(
-            map, order, tile_code, num_tiles, n, V, tile_rows, fill_rows(tile_rows), seg, plan_seg, plan_idx, plan_band, (unsigned)col_tiles,
-            (unsigned)slabs, (unsigned)groups, item_ws, item_at);
+        plan_fill_kernel<true><<<fills + (item_at != nullptr ? 1u : 0u), kFillThreads, lds > list ? lds : list, s>>>(
+            map, order, tile_code, num_tiles, n, V, tile_rows, fill_rows(together * tile_rows), seg, plan_seg, plan_idx, plan_band, (unsigned)col_tiles,
+            (unsigned)slabs, (unsigned)groups, item_ws, item_at, together);
         FGX_CHECK_LAUNCH("fgx_tile_plan(tables and plan)");
         return FGX_OK;
     }
@@ -1028,8 +1048,8 @@ int fgx_tile_plan(const int32_t* gray, const int64_t* order, const uint32_t* map
     }
     if (plan_idx != nullptr) {
         phase_mark("gather plan fill", s);
-        plan_fill_kernel<false><<<(unsigned)num_tiles, kFillThreads, fill_lds(tile_rows, V), s>>>(map, order, tile_code, num_tiles, n, V, tile_rows, fill_rows(tile_rows),
-                                                                              nullptr, plan_seg, plan_idx, plan_band, 1, 1, 1, nullptr, nullptr);
+        plan_fill_kernel<false><<<fills, kFillThreads, fill_lds(together * tile_rows, V), s>>>(map, order, tile_code, num_tiles, n, V, tile_rows, fill_rows(together * tile_rows),
+                                                                              nullptr, plan_seg, plan_idx, plan_band, 1, 1, 1, nullptr, nullptr, together);
         FGX_CHECK_LAUNCH("fgx_tile_plan(plan)");
     }
     return FGX_OK;
@@ -1064,9 +1084,10 @@ int fgx_gather_plan_fill(const uint32_t* map, const int64_t* order, const int32_
     FGX_CHECK_ARG(plan_band == nullptr || tile_rows <= 1024, "fgx_gather_plan_fill: band masks need tile_rows <= 1024");
     PhaseEnd phases{(hipStream_t)stream};
     phase_mark("gather plan fill", (hipStream_t)stream);
-    plan_fill_kernel<false><<<(unsigned)num_tiles, kFillThreads, fill_lds(tile_rows, V), (hipStream_t)stream>>>(
-        map, order, tile_code, num_tiles, n, V, tile_rows, fill_rows(tile_rows), nullptr, const_cast<int32_t*>(plan_seg), plan_idx, plan_band, 1, 1, 1,
-        nullptr, nullptr);
+    const int together = fill_together(tile_rows, num_tiles);
+    plan_fill_kernel<false><<<(unsigned)cdiv(num_tiles, (size_t)together), kFillThreads, fill_lds(together * tile_rows, V), (hipStream_t)stream>>>(
+        map, order, tile_code, num_tiles, n, V, tile_rows, fill_rows(together * tile_rows), nullptr, const_cast<int32_t*>(plan_seg), plan_idx, plan_band, 1,
+        1, 1, nullptr, nullptr, together);
     FGX_CHECK_LAUNCH("fgx_gather_plan_fill");
     return FGX_OK;
 }
