@@ -377,7 +377,7 @@ __global__ void __launch_bounds__(kBlock) tile_fill_kernel(const int32_t* __rest
 // cost, most expensive first (stable counting sort over the 33 possible popcounts: a wavefront counts, then places, a
 // contiguous piece 64 items at a time, equal costs found by ballots).  Step 2 deals them round by round: the incomplete
 // last round takes the cheapest items, every full round gives its most expensive item to the least loaded slot (rank of
-// each slot's load by counting).  Everything is deterministic.  One workgroup, so what bounds it is the length of its
+// each slot's load by counting, or by a sort of the loads).  Everything is deterministic.  One workgroup, so what bounds it is the length of its
 // dependent chains: the counting sort by one thread per piece with serial prefixes over 256 of them, and the ranks one
 // load at a time, took 0.040 ms for 1 306 items and 256 slots; this form, the scans of 1 306 tiles included, 0.017.
 constexpr int kOrderThreads = 1024;     // also the largest number of slots
@@ -451,6 +451,39 @@ __device__ void order_items(const int32_t* __restrict__ tile_code, unsigned num_
         const unsigned pc = 32u - (WIDE ? bin_of(entry) : entry >> kItemBits);
         return ((pc ? pc : 1u) * slabs + 3u) >> scale;
     };
+    if (groups > 256u) {
+        // Ranks by counting read every load once per slot (512 slots: 7 us a round); with this many the standings are sorted instead (2.5 us), and a thread
+        // goes on with the slot whose standing it was given.  2 611 items in 512 slots beside the plan of as many tiles 41 -> 19 us, 3 817 items 57 -> 27.
+        uint32_t key = tid < groups ? tid : 0xFFFFFFFFu;
+        if (tid < rem) {
+            const uint32_t entry = sorted[total - rem + tid];
+            item_at[rounds * groups + tid] = item_of(entry);
+            key += cost_of(entry) << 10;
+        }
+        for (unsigned r = 0; r < rounds; ++r) {
+#pragma unroll
+            for (unsigned k = 2; k <= (unsigned)THREADS; k *= 2)
+#pragma unroll
+                for (unsigned j = k / 2; j > 0; j /= 2) {
+                    uint32_t other;
+                    if (j < 64) {
+                        other = (uint32_t)__shfl_xor((int)key, (int)j, 64);
+                    } else {
+                        load[tid] = key;
+                        __syncthreads();
+                        other = load[tid ^ j];
+                        __syncthreads();
+                    }
+                    key = ((tid & j) == 0) == ((tid & k) == 0) ? (key < other ? key : other) : (key < other ? other : key);
+                }
+            if (tid < groups) {
+                const uint32_t entry = sorted[r * groups + tid];      // the least loaded slot <- most expensive item
+                item_at[r * groups + (key & 1023u)] = item_of(entry);
+                key += cost_of(entry) << 10;
+            }
+        }
+        return;
+    }
     // P threads per slot share the counting
     const unsigned P = groups <= THREADS / 4 ? 4u : (groups <= THREADS / 2 ? 2u : 1u);
     const unsigned slot = tid / P, part = tid % P;
@@ -736,8 +769,8 @@ __global__ void __launch_bounds__(kFillThreads) plan_fill_kernel(const uint32_t*
 }
 
 // Tiles of 64 or 128 rows that a workgroup fills together, as many rows at a time as of a longer one, once the workgroups left are as many as CUs: a workgroup
-// takes 6 us whatever its rows, and 1 024 of them fit the chip (64 rows, 1 149 tiles 18.9 -> 9.4 us, 2 611 41.5 -> 12.5, 3 817 55.7 -> 14.4; 128 rows,
-// 1 306 tiles 20.6 -> 12.5; 322 tiles of 64 rows, one each, 6.1, as many of 256 8.4).
+// takes 6 us whatever its rows, and 1 024 of them fit the chip (64 rows, 1 149 tiles 18.9 -> 9.4 us; 128 rows, 1 306 tiles 20.6 -> 12.5; 322 tiles
+// of 64 rows, one each, 6.1, as many of 256 8.4).
 inline int fill_together(int tile_rows, size_t num_tiles) {
     int t = 1;
     while (tile_rows % 64 == 0 && 2 * t * tile_rows <= kFillRows && num_tiles >= (size_t)512 * t) t *= 2;
