@@ -629,6 +629,8 @@ int dispatch_stream(int tile_rows, int tile_cols, int slab_bytes, const void* sr
         FGX_STREAM_TILE(64, 128, 2, 2, 8)
         FGX_STREAM_TILE(128, 64, 4, 1, 8)
         FGX_STREAM_TILE(128, 128, 2, 2, 8)
+        FGX_STREAM_TILE(64, 32, 2, 1, 8)
+        FGX_STREAM_TILE(128, 32, 4, 1, 8)
     }
 #undef FGX_STREAM_TILE
     set_error("fgx_conv_gather_gemm_stream: no kernel for tile %dx%d with %d-byte slabs", tile_rows, tile_cols, slab_bytes);
@@ -717,6 +719,8 @@ bool stream_lds_fits(int tile_rows, int tile_cols, int slab_bytes, int cols) {
     FGX_STREAM_TILE(64, 128, 2, 2, 8)
     FGX_STREAM_TILE(128, 64, 4, 1, 8)
     FGX_STREAM_TILE(128, 128, 2, 2, 8)
+    FGX_STREAM_TILE(64, 32, 2, 1, 8)
+    FGX_STREAM_TILE(128, 32, 4, 1, 8)
 #undef FGX_STREAM_TILE
     return fixed != 0 && fixed + bias_bytes <= 160 * 1024;
 }
@@ -741,7 +745,9 @@ extern "C" int fgx_conv_gather_gemm_stream_groups(int dtype, int cols, int tile_
     FGX_STREAM_TILE(TAG, 64, 64, 2, 2, 8)   \
     FGX_STREAM_TILE(TAG, 64, 128, 2, 2, 8)  \
     FGX_STREAM_TILE(TAG, 128, 64, 4, 1, 8)  \
-    FGX_STREAM_TILE(TAG, 128, 128, 2, 2, 8)
+    FGX_STREAM_TILE(TAG, 128, 128, 2, 2, 8) \
+    FGX_STREAM_TILE(TAG, 64, 32, 2, 1, 8) \
+    FGX_STREAM_TILE(TAG, 128, 32, 4, 1, 8)
     if (dtype == FGX_F16) { FGX_STREAM_TILES(F16) FGX_SMALL_TILES(F16) }
     else if (dtype == FGX_BF16) { FGX_STREAM_TILES(BF16) FGX_SMALL_TILES(BF16) }
     else { FGX_STREAM_TILES(F32) }

@@ -125,17 +125,31 @@ void rule_gemm_f32(size_t n, int K, int cols, int V, fgx_schedule* out) {
 // (where one figure stands, the tile stays.)  The tiled kernel splits few rows well: under up to 64 columns, or rows of 512 bytes and more, it is level up
 // to 10 000 voxels (8 004: 96 -> 64 21.0 22.3, 384 -> 96 43 47, 768 -> 128 64 83), otherwise up to 5 000 (4 947: 80 -> 80 21.0 22.7); and it wants no gather
 // plan and no packed weight, 14 us of the host's time in a training pass on new coordinates, which little work does not bring in (64 -> 64 at 10 494 voxels
-// gains 3.5 us a product, at 28 169 9.7).  Past 131 072 voxels the plan of shorter tiles costs a new cache what a product gains (64 -> 64, 229 217
-// voxels: kept 53.9 49.4, new 145.0 151.7).
+// gains 3.5 us a product, at 28 169 9.7).
 bool small_stream_tile(size_t n, int K, int cols, fgx_schedule* out) {
     const int slabs = (int)cdiv((size_t)K * 2, (size_t)128);
-    if (K * 2 <= 64 || cols <= 32 || !stream_lds_fits(256, 128, 128, cols)) return false;
-    if (n > 131072 || (!out->stream && (n < (cols <= 64 || K >= 256 ? 10240u : 5120u) || n * slabs * cdiv(cols, 64) < 24576))) return false;
+    if (K * 2 <= 64 || !stream_lds_fits(256, 128, 128, cols)) return false;
+    // Up to 32 columns: 64 x 32, and 128 x 32 where rows of up to 192 bytes fill the chip.  Before, now:  64 -> 32 channels, 20 574 voxels 20.7 15.5, 36 575
+    // 24.3 17.6, 75 224 25.8 21.8;  128 -> 32 25.4 20.2, 33.6 23.5, 54.4 34.2, 166 977 99.5 61.6;  256 -> 32 37.8 29.6, 53.5 34.8, 99.1 58.9, 185 116;
+    // 512 -> 32 62 50, 95 66, 190 122, 352 245;  10 494 voxels 18.3 15.0, 21.2 19.7, 26.6 29.5, 39.6 50.1.
+    if (cols <= 32) {
+        // (few rows: the plan of a new cache, 20 574 voxels 72 -> 24 68.5 73.8, 128 -> 32 72.2 72.4, 36 575 80 80 and 83 79;  one slab: its input gradient
+        // has a plan of its own, 64 -> 32, training on new coordinates, 73 461 voxels 216 212, 123 180 245 255)
+        if (n > (slabs == 1 ? 98304u : K <= 96 ? 524288u : 262144u) || (!out->stream && n < (K <= 96 ? 32768u : 20480u))) return false;
+        *out = fgx_schedule{K <= 96 && n > 57344 ? 128 : 64, 32, 128, 1, 0, 1};
+        return true;
+    }
+    // (rows of 128 bytes past 262 144 voxels: 277 018 62.5 56.2, 1 041 730 184 184; of two slabs past 131 072: the input gradient's plan is another, 96 -> 64,
+    // training on new coordinates, 123 180 voxels 310 311, 244 211 459 465; 4 096 tiles are filled in one launch with their tables)
+    if (n > (cols > 64 || slabs == 2 ? 131072u : slabs > 2 || K == 64 ? 262144u : 524288u) || (!out->stream && (n < (cols <= 64 || K >= 256 ? 10240u : 5120u) || n * slabs * cdiv(cols, 64) < 24576))) return false;
     auto take = [&](int rows, int wide) {
         *out = fgx_schedule{rows, wide, 128, 1, 0, 1};
         return true;
     };
-    if (cols <= 64) return take(n <= (slabs == 1 ? 36864u : slabs == 2 ? 57344u : 131072u) ? 64 : 128, 64);
+    if (cols <= 64) {
+        if (slabs >= 16 && n > 131072) return false;
+        return take(slabs > 2 || n <= (slabs == 1 ? 36864u : 57344u) ? 64 : 128, 64);
+    }
     // long rows under one tile of columns: 75 224 voxels, 384 -> 96 132 120, 768 -> 128 270 251
     if (cols <= 128 && K >= 384 && n >= 28672) return take(128, 128);
     if (cols > 192 && K >= 192 && n > 12288) return false;              // (the larger tiles fill the chip by then)
