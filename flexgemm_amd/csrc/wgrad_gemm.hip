@@ -1385,35 +1385,20 @@ int launch_wgrad(const void* gout, const void* feats, const uint32_t* sig_i, con
 // L2 -- stay on one XCD:
 //   1. chunks = up to 32 tiles of one (block, offset), cost = tiles x (pairs + kItemFixedCost); sorted by falling cost;
 //   2. each chunk goes to the XCD with the least cost so far (one wavefront, in sorted order);
-//   3. per XCD (one wavefront each): the chunks' items go, in the same order, to the workgroup of that XCD with the
+//   3. per XCD (one wavefront each): the chunks' items go, in the same order and kItemListBatch at a time, to the workgroups of that XCD with the
 //      least cost so far; a workgroup's chain links its items in the order they arrived.
+// Bound by its dependent chains.  With the ranks of step 1 read one by one, 256 chunks dealt singly in step 2 and items in step 3, 20 574 voxels x 256 channels took
+// 40 us, 49 829 46, 188 056 x 272 61; so 21, 28 and 32, under launches that take as long as before (55, 102 and 1 050 us).
 // Items without pairs cost nothing and are linked too, so the chains cover every item whatever the pair lists hold.
 // ------------------------------------------------------------------------------------------------
 constexpr int kItemListMaxChunks = 2048;        // chunks the builder sorts in LDS (by counting ranks: quadratic)
 constexpr unsigned kItemListMaxItems = 4096;    // beyond (16 items per workgroup and more) the fixed interleave is balanced
                                                 // to within a few per cent, and the one-workgroup builder takes too long
 constexpr size_t kItemListMinRows = 2048, kItemListMaxBlocks = 12, kItemListMaxBlocksTiled = 16;
-constexpr unsigned kItemListGreedyChunks = 256; // chunks dealt to the XCDs one by one
+constexpr unsigned kItemListBatch = 16;         // items an XCD deals at a time: half of its workgroups, so that the loaded ones are passed over
+constexpr unsigned kItemListGreedyChunks = 64;  // chunks dealt to the XCDs one by one
 constexpr unsigned kItemListMaxGroups = 512;    // 64 workgroups per XCD: one lane each
 constexpr uint32_t kItemFixedCost = 1280;       // an item's prologue, epilogue and share of the reduction, in pairs
-
-// minimum over the 64 lanes, in every lane: four shifts inside the rows of 16 lanes, then the rows' last lanes are
-// passed on (lanes shifted in from outside a row, and rows a step leaves out, take the identity)
-__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
-#define FGX_MIN_STEP(ctrl, rows)                                                                               \
-    {                                                                                                          \
-        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp((int)0xFFFFFFFF, (int)v, ctrl, rows, 0xF, false); \
-        v = o < v ? o : v;                                                                                     \
-    }
-    FGX_MIN_STEP(0x111, 0xF)    // row_shr:1
-    FGX_MIN_STEP(0x112, 0xF)    // row_shr:2
-    FGX_MIN_STEP(0x114, 0xF)    // row_shr:4
-    FGX_MIN_STEP(0x118, 0xF)    // row_shr:8: lane 15 of every row holds the row's minimum
-    FGX_MIN_STEP(0x142, 0xA)    // row_bcast:15 into rows 1 and 3
-    FGX_MIN_STEP(0x143, 0xC)    // row_bcast:31 into rows 2 and 3: lane 63 holds the minimum
-#undef FGX_MIN_STEP
-    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
-}
 
 // minimum over lanes 0 ... 7, in every lane
 __device__ __forceinline__ uint32_t first8_min_u32(uint32_t v) {
@@ -1431,9 +1416,11 @@ __device__ __forceinline__ uint32_t first8_min_u32(uint32_t v) {
 
 __global__ void __launch_bounds__(1024) wgrad_item_lists_kernel(const uint32_t* __restrict__ bounds, int V, unsigned nb,
                                                                 unsigned tiles, unsigned groups, uint32_t* __restrict__ out) {
-    __shared__ uint32_t key[kItemListMaxChunks];
+    __shared__ __attribute__((aligned(16))) uint32_t key[kItemListMaxChunks];
     __shared__ uint16_t sorted[kItemListMaxChunks];
     __shared__ uint8_t xcd_of[kItemListMaxChunks];
+    __shared__ uint16_t dealt[kItemListMaxItems];           // the XCDs' items one after the other, each in the chunks' order, and their costs
+    __shared__ uint32_t cost_of[kItemListMaxItems];
     const unsigned units = nb * (unsigned)V, per_unit = (tiles + 31) / 32, chunks = units * per_unit;
     const unsigned items = units * tiles, per_xcd = groups / kXcds;
     const int tid = threadIdx.x;
@@ -1454,14 +1441,24 @@ __global__ void __launch_bounds__(1024) wgrad_item_lists_kernel(const uint32_t* 
         out[2] = tiles;
         out[3] = kItemListMagic;
     }
-    for (unsigned m = tid; m < chunks; m += 1024) key[m] = unit_cost(m / per_unit) * chunk_items(m);
+    const unsigned padded = (chunks + 31u) & ~31u;          // (zeros past the last one: behind everything)
+    for (unsigned m = tid; m < padded; m += 1024) key[m] = m < chunks ? unit_cost(m / per_unit) * chunk_items(m) : 0u;
     __syncthreads();
     for (unsigned m = tid; m < chunks; m += 1024) {         // rank by counting: falling cost, ties by index
         const uint32_t mine = key[m];
         unsigned rank = 0;
-        for (unsigned j = 0; j < chunks; ++j) {
-            const uint32_t other = key[j];
-            rank += (other > mine || (other == mine && j < m)) ? 1u : 0u;
+        for (unsigned j0 = 0; j0 < padded; j0 += 32) {      // (eight reads in flight: one a time is waited for one by one)
+            uint4 other[8];
+#pragma unroll
+            for (unsigned q = 0; q < 8; ++q) other[q] = *reinterpret_cast<const uint4*>(key + j0 + q * 4);
+#pragma unroll
+            for (unsigned q = 0; q < 8; ++q) {
+                const unsigned j = j0 + q * 4;
+                rank += (other[q].x > mine || (other[q].x == mine && j < m)) ? 1u : 0u;
+                rank += (other[q].y > mine || (other[q].y == mine && j + 1 < m)) ? 1u : 0u;
+                rank += (other[q].z > mine || (other[q].z == mine && j + 2 < m)) ? 1u : 0u;
+                rank += (other[q].w > mine || (other[q].w == mine && j + 3 < m)) ? 1u : 0u;
+            }
         }
         sorted[rank] = (uint16_t)m;
     }
@@ -1504,52 +1501,55 @@ __global__ void __launch_bounds__(1024) wgrad_item_lists_kernel(const uint32_t* 
     }
     __syncthreads();
     if (wave >= kXcds) return;
-    // Wavefront x deals the items of XCD x's chunks, in the same order, each to the least loaded workgroup of the XCD;
-    // lane l < per_xcd is workgroup l * kXcds + x (blockIdx % kXcds is the XCD a workgroup lands on).  A workgroup's
-    // chain links its items in the order they arrived.
+    // Wavefront x lists the items of XCD x's chunks, behind those of the XCDs before it.
+    unsigned first = 0, count = 0;
+    for (unsigned r0 = 0; r0 < chunks; r0 += 64) {
+        const unsigned r = r0 + lane, m = r < chunks ? r : 0u, k = r < chunks ? chunk_items(m) : 0u;
+        first += r < chunks && xcd_of[m] < wave ? k : 0u;
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) first += (unsigned)__shfl_xor((int)first, d, 64);
+    for (unsigned r0 = 0; r0 < chunks; r0 += 64) {
+        const unsigned r = r0 + lane, m = r < chunks ? sorted[r] : 0u;
+        const unsigned k = r < chunks && xcd_of[m] == wave ? chunk_items(m) : 0u;
+        unsigned upto = k;
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const unsigned o = (unsigned)__shfl_up((int)upto, d, 64);
+            upto += lane >= d ? o : 0u;
+        }
+        const unsigned item = m / per_unit * tiles + 32 * (m % per_unit), per = k ? key[m] / k : 0u;
+        for (unsigned i = 0; i < k; ++i) {
+            dealt[first + count + upto - k + i] = (uint16_t)(item + i);
+            cost_of[first + count + upto - k + i] = per;
+        }
+        count += (unsigned)__shfl((int)upto, 63, 64);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (read by other lanes of the wavefront)
+    // ... and deals them, kItemListBatch at a time, the most expensive to the least loaded workgroup of the XCD and so on; lane l < per_xcd is
+    // workgroup l * kXcds + x (blockIdx % kXcds is the XCD a workgroup lands on).  A workgroup's chain links its items in the order they arrived.
     const bool bin = (unsigned)lane < per_xcd;
+    const unsigned batch = per_xcd < kItemListBatch ? per_xcd : kItemListBatch;
     uint32_t load = 0;
     uint32_t tail = kItemListEnd;
     bool any = false;
-    for (unsigned r0 = 0; r0 < chunks; r0 += 64) {
-        const unsigned r = r0 + lane;
-        const unsigned m_l = r < chunks ? sorted[r] : 0u;
-        const bool here = r < chunks && xcd_of[m_l] == wave;
-        const uint32_t key_l = key[m_l];
-        uint64_t todo = __ballot(here);
-        while (todo) {
-            const int j = __builtin_ctzll(todo);
-            todo &= todo - 1;
-            const unsigned m = (unsigned)__builtin_amdgcn_readlane((int)m_l, j);
-            const unsigned u = m / per_unit, k = chunk_items(m);
-            const uint32_t per = (uint32_t)__builtin_amdgcn_readlane((int)key_l, j) / k;
-            const unsigned first_item = u * tiles + 32 * (m % per_unit);
-            auto take = [&](uint32_t it) {
-                if (any) next[tail] = it;
-                else head[(unsigned)lane * kXcds + wave] = it;
-                any = true;
-                tail = it;
-                load += per;
-            };
-            if (k < 8) {
-                for (unsigned i = 0; i < k; ++i) {
-                    const int best = (int)(wave_min_u32(bin ? (load << 6) | (uint32_t)lane : 0xFFFFFFFFu) & 63u);
-                    if (lane == best) take(first_item + i);
-                }
-            } else {
-                // many items of one cost: the least loaded workgroups take one each (what dealing them one by one does
-                // unless a single item is smaller than the gaps between the loads), per_xcd at a time
-                for (unsigned done = 0; done < k;) {
-                    const unsigned now = k - done < per_xcd ? k - done : per_xcd;
-                    unsigned rank = 0;
-                    for (unsigned o = 0; o < per_xcd; ++o) {
-                        const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)load, (int)o);
-                        rank += (other < load || (other == load && o < (unsigned)lane)) ? 1u : 0u;
-                    }
-                    if (bin && rank < now) take(first_item + done + rank);
-                    done += now;
-                }
-            }
+    for (unsigned t = 0; t < count; t += batch) {
+        const unsigned now = count - t < batch ? count - t : batch;
+        const uint32_t standing = bin ? (load << 6) | (uint32_t)lane : 0xFFFFFFFFu;
+        unsigned rank = 0;
+#pragma unroll
+        for (int o = 0; o < 32; ++o) rank += (uint32_t)__builtin_amdgcn_readlane((int)standing, o) < standing ? 1u : 0u;
+        if (per_xcd > 32) {
+#pragma unroll
+            for (int o = 32; o < 64; ++o) rank += (uint32_t)__builtin_amdgcn_readlane((int)standing, o) < standing ? 1u : 0u;
+        }
+        if (bin && rank < now) {
+            const uint32_t it = dealt[first + t + rank];
+            if (any) next[tail] = it;
+            else head[(unsigned)lane * kXcds + wave] = it;
+            any = true;
+            tail = it;
+            load += cost_of[first + t + rank];
         }
     }
     if (bin) {
