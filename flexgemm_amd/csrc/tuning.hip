@@ -295,7 +295,12 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
                 if (last || fills) break;
             }
             // long blocks overflow an XCD's L2 when few tiles share their rows; partial products stay below 256 MiB
-            const size_t longest = tiles <= 4 ? 16384 : (tiles <= 8 ? 24576 : 65536);
+            // (nine tiles that pad, from 131 072 voxels on: blocks as of eight tiles while the lists take them, 16 at most; 272 channels, 166 977 voxels 717 -> 644 us,
+            // 277 018 1 237 -> 1 052, 448 584 2 063 -> 1 758, blocks of 24 576 there 2 594;  320 channels 711 671, 1 214 1 142, 1 997 1 752.  Level or behind before,
+            // 101 586 voxels 418 420 and 426 435, and where nothing is padded, 384 channels 653 665, 1 100 1 105)
+            const bool pads = Ci % 128 != 0 || Co % 128 != 0;
+            const size_t nine = !pads || n < 131072 ? 65536 : n <= 393216 ? 24576 : n <= 524288 ? 32768 : 65536;
+            const size_t longest = tiles <= 4 ? 16384 : tiles <= 8 ? 24576 : tiles == 9 ? nine : 65536;
             if (nb < cdiv(n, longest)) nb = cdiv(n, longest);
             size_t max_blocks = (size_t)(268435456.0 / (4.0 * V * (double)Co * (double)Ci * slices));
             if (max_blocks < 1) max_blocks = 1;

@@ -44,3 +44,9 @@ def test_lists(nb, v, tiles, empty):
     # an XCD takes whole chunks (at most 32 tiles of a unit) to within one of them, a workgroup whole items to within two
     chunk = cost.max() * min(per, 32) * 8 / groups
     assert load.max() <= cost.sum() / groups + chunk + 2 * cost.max()
+
+
+@pytest.mark.parametrize("n,rows", [(131071, 44032), (131072, 22528), (393216, 24576), (393217, 30720), (524288, 32768), (600000, 60416)])
+def test_blocks_of_nine_tiles(n, rows):
+    s = nat.table_lookup(nat.PASS_WGRAD, torch.bfloat16, n, 272, 384, 27)
+    assert (s.tile_rows, s.tile_cols, s.stream, s.block_rows) == (128, 128, 1, rows)
