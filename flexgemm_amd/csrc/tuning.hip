@@ -129,14 +129,15 @@ void rule_gemm_f32(size_t n, int K, int cols, int V, fgx_schedule* out) {
 bool small_stream_tile(size_t n, int K, int cols, fgx_schedule* out) {
     const int slabs = (int)cdiv((size_t)K * 2, (size_t)128);
     if (K * 2 <= 64 || !stream_lds_fits(256, 128, 128, cols)) return false;
-    // Up to 32 columns: 64 x 32, and 128 x 32 where rows of up to 192 bytes fill the chip.  Before, now:  64 -> 32 channels, 20 574 voxels 20.7 15.5, 36 575
-    // 24.3 17.6, 75 224 25.8 21.8;  128 -> 32 25.4 20.2, 33.6 23.5, 54.4 34.2, 166 977 99.5 61.6;  256 -> 32 37.8 29.6, 53.5 34.8, 99.1 58.9, 185 116;
-    // 512 -> 32 62 50, 95 66, 190 122, 352 245;  10 494 voxels 18.3 15.0, 21.2 19.7, 26.6 29.5, 39.6 50.1.
+    // Up to 32 columns: 64 x 32 and 128 x 32.  Before, now:  64 -> 32 channels, 36 575 voxels 24.3 17.6, 75 224 25.8 21.8;  72 -> 24 166 977 69.8 55.2, 448 584
+    // 148 130;  128 -> 32 20 574 25.4 20.2, 36 575 33.6 23.5, 75 224 54.4 34.2, 166 977 99.5 61.6;  256 -> 32 37.8 29.6, 53.5 34.8, 99.1 58.9, 185 116;
+    // 512 -> 32 62 50, 95 66, 190 122, 352 245.  Not where a plan of this tile's own costs a new cache as much (20 574 voxels 72 -> 24 68.5 73.8, 128 -> 32 72.2
+    // 72.4; 64 -> 32, whose input gradient has another, training on new coordinates, 73 461 voxels 216 212, 123 180 245 255) or more than the tile gains over
+    // the 256 x 32 one, whose plan the wider layers of a stack share (65 ... 127 channels up to 131 072 voxels: 123 180 43.8 40.4, a plan 13).
     if (cols <= 32) {
-        // (few rows: the plan of a new cache, 20 574 voxels 72 -> 24 68.5 73.8, 128 -> 32 72.2 72.4, 36 575 80 80 and 83 79;  one slab: its input gradient
-        // has a plan of its own, 64 -> 32, training on new coordinates, 73 461 voxels 216 212, 123 180 245 255)
-        if (n > (slabs == 1 ? 98304u : K <= 96 ? 524288u : 262144u) || (!out->stream && n < (K <= 96 ? 32768u : 20480u))) return false;
-        *out = fgx_schedule{K <= 96 && n > 57344 ? 128 : 64, 32, 128, 1, 0, 1};
+        if (n > (slabs == 1 ? 98304u : K < 128 ? 524288u : 262144u) || (!out->stream && n < (K <= 96 ? 32768u : 20480u))) return false;
+        if (slabs == 2 && out->stream && n < 131072) return false;
+        *out = fgx_schedule{(slabs == 1 && n > 36864) || (slabs == 2 && K < 128 && n > 57344) ? 128 : 64, 32, 128, 1, 0, 1};
         return true;
     }
     // (rows of 128 bytes past 262 144 voxels: 277 018 62.5 56.2, 1 041 730 184 184; of two slabs past 131 072: the input gradient's plan is another, 96 -> 64,

@@ -58,7 +58,7 @@ def test_same_bits_as_the_long_tiles(monkeypatch, dtype, n, side, ci, co):
     (5119, 192, 192, None), (5120, 192, 192, (64, 64)), (10239, 512, 64, None), (10240, 512, 64, (64, 64)), (24575, 64, 64, None), (24576, 64, 64, (64, 64)),
     (36864, 64, 64, (64, 64)), (36865, 64, 64, (128, 64)), (262144, 64, 64, (128, 64)), (262145, 64, 64, (256, 64)), (524288, 48, 40, (128, 64)), (20574, 128, 128, (64, 128)),
     (57345, 128, 128, (256, 128)), (12288, 256, 256, (64, 128)), (12289, 256, 256, (256, 64)), (28672, 384, 96, (128, 128)), (20000, 32, 64, None),
-    (32767, 64, 32, None), (32768, 64, 32, (64, 32)), (57345, 64, 32, (128, 32)), (98305, 64, 32, (256, 32)),
+    (32767, 64, 32, None), (32768, 64, 32, (64, 32)), (36865, 64, 32, (128, 32)), (98305, 64, 32, (256, 32)), (131071, 72, 24, (256, 32)), (131072, 72, 24, (128, 32)),
     (20479, 256, 16, None), (20480, 256, 16, (64, 32)), (262144, 128, 32, (64, 32)), (131073, 96, 64, (256, 64))])
 def test_rule(n, ci, co, tile):
     s = nat.table_lookup(nat.PASS_FWD, torch.float16, n, ci, co, 27)
