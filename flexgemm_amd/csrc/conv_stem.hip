@@ -6,7 +6,7 @@
 // As products per offset (wgrad_gemm.hip) every (row, offset) pair fetches a grad_out row of 2 * Co bytes for 16 or 32 bytes
 // of features, and the 32-wide tile multiplies mostly padding.  Here the features of a row's V neighbors lie next to each other
 // in LDS (a missing neighbor: zeros), [rows][V * Ci], and one product with the rows' own grad_out gives every offset at
-// once: grad_out is read once per 64 of its columns, the pair lists not at all.  What bounds it are the 16-byte gathers, one
+// once: the features are gathered once per 64 or 128 of its columns, the pair lists not read at all.  What bounds it are the 16-byte gathers, one
 // per (row, offset): 1 792 pieces for 64 rows, 0.88 us of a CU.  Four wavefronts do nothing but load and eight nothing but multiply: with both in one
 // (issue a step's loads, then multiply another's) the address pipeline stood still while all of them multiplied, 1.4 us a step.  424 000 voxels
 // 6 -> 48 channels 38 -> 29 us, 16 -> 48 67 -> 52.  A last piece per row holds a one: its column is the bias gradient.

@@ -865,7 +865,7 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
             c.set("sorted_idx", made[2].cast<Tensor>());
         }
     }
-    const Sched s = schedule(pass, src, n, ci, co, v);
+    Sched s = schedule(pass, src, n, ci, co, v);
     bool own_order = false;
     if (masked && !narrow && row_bytes <= module_int(g_impl, "LOCALITY_MAX_ROW_BYTES") && (c.has("_tile_order") || n >= module_int(g_impl, "LOCALITY_MIN_ROWS")) &&
         impl_function("_locality_applies")(c.obj, n, row_bytes).cast<bool>()) {
@@ -880,6 +880,11 @@ Product gather_product(Tensor src, Tensor weight, Tensor bias, const Cache& c, i
     const double most = (double)0xFF000000u;
     const bool streams = s.stream && (double)n_src * row_bytes <= most && (double)n * 8 <= most && (double)n * 27 * 4 * 2 <= most;
     Tensor panel = panel_given;
+    if (s.stream && !streams && !(s.tile_rows == 256 && s.tile_cols == 128)) {      // a streaming tile that the tiled kernel, which addresses more, does not have
+        s = Sched{128, cols > 64 ? 128 : cols > 32 ? 64 : 32, 64, 1, 0, 0};
+        panel = Tensor();                               // (packed for the other tile)
+        owner = {};
+    }
     if (!panel.defined() && owner)
         panel = impl_function("_weight_panel")(owner, weight, code, mode, python_schedule(pass, src, n, ci, co, v), py::cast(src).attr("device")).cast<Tensor>();
     // the tiled kernel reads the weight itself where it can

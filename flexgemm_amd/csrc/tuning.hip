@@ -122,7 +122,7 @@ void rule_gemm_f32(size_t n, int K, int cols, int V, fgx_schedule* out) {
 //   256 -> 256        65.2 42.1    60.5 53.1    60.7        67.2        71.7        89.2        145.9       271
 //   512 ->  64        54.7         60.5 56.3                100.8 56.6              165.9 75.9  156.0 135.1 300 276
 //    64 -> 256        26.3 18.9    26.3 22.7                28.2                    33.0        46.5        83.1
-// (where one figure stands, the tile stays.)  The tiled kernel splits few rows well: under up to 64 columns, or rows of 512 bytes and more, it is level up
+// (where one figure stands, the tile stays; 64 -> 64 stays tiled below 24 576 voxels.)  The tiled kernel splits few rows well: under up to 64 columns, or rows of 512 bytes and more, it is level up
 // to 10 000 voxels (8 004: 96 -> 64 21.0 22.3, 384 -> 96 43 47, 768 -> 128 64 83), otherwise up to 5 000 (4 947: 80 -> 80 21.0 22.7); and it wants no gather
 // plan and no packed weight, 14 us of the host's time in a training pass on new coordinates, which little work does not bring in (64 -> 64 at 10 494 voxels
 // gains 3.5 us a product, at 28 169 9.7).

@@ -74,3 +74,23 @@ def test_not_under_few_offsets_or_in_fp32(n, ci, co):
     for dtype, v in ((torch.float16, 8), (torch.float32, 27)):
         s = nat.table_lookup(nat.PASS_FWD, dtype, n, ci, co, v)
         assert not s.stream or 256 in (s.tile_rows, s.tile_cols)
+
+
+# rows past the streaming kernel's 32-bit byte offsets: the tiled kernel, on a tile that it has
+@pytest.mark.gpu
+def test_operands_past_32_bit_offsets():
+    n, side, ci, co = 131072, 64, 16384, 40
+    s = nat.table_lookup(nat.PASS_FWD, torch.float16, n, ci, co, 27)
+    assert s.stream and s.tile_rows < 256 and n * ci * 2 > 0xFF000000
+    coords = coords_of(n, side, 3)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    feats = torch.empty(n, ci, dtype=torch.float16, device="cuda").uniform_(-1, 1, generator=g)
+    weight = (torch.randn(co, 3, 3, 3, ci, generator=g, device="cuda") / (27 * ci) ** 0.5).half()
+    with torch.no_grad():
+        out, cache = sparse_submanifold_conv3d_relu(feats, coords, torch.Size([1, ci, side, side, side]), weight)
+    nmap, w = cache["neighbor_map"].view(torch.int32).long(), weight.reshape(co, 27, ci).float()
+    for row in (0, 63, 70000, n - 1):
+        have = (nmap[row] >= 0).nonzero()[:, 0]
+        ref = (feats[nmap[row, have]].float()[:, None] * w[:, have].transpose(0, 1)).sum((0, 2))
+        # one rounding to 16 bits; sums of about one of 27 ci products in 32 bits, in another order
+        assert bool(((out[row].float() - ref.relu()).abs() <= 2.0 ** -10 * ref.abs() + (27 * ci) ** 0.5 * 2.0 ** -22).all())
