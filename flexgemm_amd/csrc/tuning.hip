@@ -420,6 +420,17 @@ void rule(int pass_kind, int es, size_t n, int Ci, int Co, int V, fgx_schedule* 
         }
     }
     if (V > 8 && small_stream_tile(n, K, cols, out)) return;
+    // 5 to 8 offsets: 64 x 128 where the products alone leave the chip idle in 256-row or 128 x 256 tiles (one layer at inference, us, kept coordinates, new ones:
+    // 2 x 2 x 2 under a stride of 2, 256 -> 256 channels, 8 449 outputs 26 20, 92 82; 10 536 26 20, 94 84; 20 753 31 24, 95 87;  128 -> 128 20 753 17 14, 81 76;
+    // 30 714 18 16, 86 78;  384 -> 512 10 536 42 34, 107 99.  1 x 2 x 3 256 -> 256 10 340 22 16, 91 81.  5 x 1 x 1 submanifold 13 572 20 17, 63 56).  Past this the larger
+    // tiles fill the chip (33 900 128 -> 256 23.1 22.6, 89 93; 19 650 384 -> 512 36 37, 62 68).  Both directions take it or neither, by the fewer and the more of the
+    // channels: a submanifold layer's input gradient reads the forward pass's plan, and a second plan costs more than the tile gains (training on new coordinates,
+    // the forward pass alone on this tile, 5 x 1 x 1, 19 650 128 -> 128 182 189, 7 x 1 x 1 180 193; on both 181 178, 180 181; 128 -> 96, whose gradient kept its own, 182 204).
+    const int least = std::min(Ci, Co), most = std::max(Ci, Co);
+    if (V > 4 && V <= 8 && out->stream && least >= 128 && n * cdiv(most, 128) <= (most <= 128 ? 36864u : 49152u) && stream_lds_fits(256, 128, 128, most)) {
+        *out = fgx_schedule{64, 128, 128, 1, 0, 1};
+        return;
+    }
     if (out->stream) return;
     // (not for an input gradient of a single tile of rows under a small weight: 192 voxels, 256 <- 768 channels 0.029 ms, 64 x 64 tiles 0.023)
     if (row_bytes >= 1024 && cols >= 128 && !(pass_kind != 0 && n < 256 && (size_t)K * cols < (size_t)512 * 512)) {

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from flexgemm_amd import _native as nat
-from flexgemm_amd.ops.spconv import sparse_submanifold_conv3d_relu
+from flexgemm_amd.ops.spconv import sparse_conv3d, sparse_submanifold_conv3d_relu
 from test_gpu_wgrad_split import coords_of
 
 TILES = [(64, 64), (64, 128), (128, 64), (128, 128), (64, 32), (128, 32)]
@@ -69,11 +69,50 @@ def test_rule(n, ci, co, tile):
         assert got == tile and (s.tile_rows == 256 or (s.slab_bytes, s.splitk) == (128, 1))
 
 
+# 5 to 8 offsets: both directions of a layer on the same tile, whichever of its channels are more
+@pytest.mark.parametrize("n,ci,co,v,small", [
+    (20400, 128, 128, 8, True), (36864, 128, 128, 5, True), (36865, 128, 128, 8, False), (20400, 128, 128, 4, False), (20400, 128, 96, 7, False), (20400, 127, 128, 8, False),
+    (24576, 256, 256, 8, True), (24577, 256, 256, 6, False), (12288, 384, 512, 8, True), (12289, 384, 512, 8, False), (20000, 512, 256, 7, False)])
+def test_rule_of_few_offsets(n, ci, co, v, small):
+    for kind in (nat.PASS_FWD, nat.PASS_DGRAD):
+        s = nat.table_lookup(kind, torch.float16, n, ci, co, v)
+        assert s.stream and ((s.tile_rows, s.tile_cols) == (64, 128)) == small
+
+
 @pytest.mark.parametrize("n,ci,co", [(5120, 192, 192), (20574, 128, 128), (36864, 64, 64), (12288, 256, 256)])
 def test_not_under_few_offsets_or_in_fp32(n, ci, co):
-    for dtype, v in ((torch.float16, 8), (torch.float32, 27)):
+    for dtype, v in ((torch.float16, 4), (torch.float32, 8), (torch.float32, 27)):
         s = nat.table_lookup(nat.PASS_FWD, dtype, n, ci, co, v)
         assert not s.stream or 256 in (s.tile_rows, s.tile_cols)
+
+
+# 2 x 2 x 2 and 5 x 1 x 1 under a stride of 2: the short tile that the rule chooses and 256 x 64 ones, outputs and gradients
+@pytest.mark.gpu
+@pytest.mark.parametrize("ks,n,side,ci,co", [((2, 2, 2), 30001, 64, 128, 128), ((5, 1, 1), 23000, 48, 136, 200), ((1, 2, 3), 24000, 56, 256, 136)])
+def test_few_offsets_same_bits(monkeypatch, ks, n, side, ci, co):
+    g = torch.Generator(device="cuda").manual_seed(n)
+    coords, shape = coords_of(n, side, n), torch.Size([1, ci, side, side, side])
+    feats = torch.randn(n, ci, generator=g, device="cuda").half().requires_grad_()
+    weight = (torch.randn(co, *ks, ci, generator=g, device="cuda") / (8 * ci) ** 0.5).half().requires_grad_()
+    nat.host()
+    real, got, up = nat.table_lookup, [], None
+    for tile in (None, (256, 64)):
+        chosen = []
+
+        def lookup(kind, dtype, rows, *a):
+            s = real(kind, dtype, rows, *a)
+            if kind != nat.PASS_WGRAD:
+                if tile:
+                    s.tile_rows, s.tile_cols, s.slab_bytes, s.splitk, s.stream = *tile, 128, 1, 1
+                chosen.append((s.tile_rows, s.tile_cols))
+            return s
+        monkeypatch.setattr(nat, "table_lookup", lookup)
+        out, _, _ = sparse_conv3d(feats, coords, shape, weight, None, None, None, (2, 2, 2))
+        up = torch.randn(out.shape, generator=g, device="cuda").half() if up is None else up
+        got.append((out.detach(), *torch.autograd.grad(out, [feats, weight], up)))
+        assert set(chosen) == {tile or (64, 128)}           # (both directions: the tiled kernel adds in another order)
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
 
 
 # rows past the streaming kernel's 32-bit byte offsets: the tiled kernel, on a tile that it has
