@@ -42,7 +42,12 @@ struct StemCfg {
     static constexpr int F_PER = F_INST / kStemLoaders, G_PER = G_INST / kStemLoaders;     // loads per loader and step
     static constexpr int IDX_BYTES = ROWS * kStemMaxV * 4;
     static constexpr int IDX_SLOT = (IDX_BYTES + 1023) / 1024 * 1024;
-    static constexpr int IDX_SLOTS = COLS == 64 ? 4 : 3;       // (three are enough: one is written again a step after it was read)
+    // A step's slot is written again IDX_SLOTS steps on.  The loaders' prologue reads the first steps' map words and asks for those of 2 (stages - 1)
+    // steps in all: with one slot fewer (128 columns leave LDS for no more) the last ones go where the first step's were, which every loader
+    // has to have read by then (PROLOGUE_BARRIER).  In the loop a barrier lies between the two either way.
+    static constexpr int IDX_AHEAD = 2 * (kStemStages - 1), IDX_SLOTS = COLS == 64 ? IDX_AHEAD : IDX_AHEAD - 1;
+    static constexpr bool PROLOGUE_BARRIER = IDX_SLOTS < IDX_AHEAD;
+    static_assert(IDX_SLOTS >= IDX_AHEAD - 1, "the barrier stands before the prologue's last load of map words: only the first step's slot is free then");
     static constexpr int IDX_INST = IDX_SLOT / 1024, IDX_PER = (IDX_INST + kStemLoaders - 1) / kStemLoaders;
     static constexpr int STAGE = F_BYTES + G_BYTES;
     static constexpr size_t LDS = (size_t)kStemStages * STAGE + IDX_SLOTS * IDX_SLOT + 16;    // ... and the word that asks for a second pass
@@ -198,6 +203,11 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
 #pragma unroll
         for (int j = 0; j < S - 1; ++j) {
             issue_rows(j);
+            if (C::PROLOGUE_BARRIER && j == S - 2) {
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_barrier();                  // (the words were read: the loads that they name are on their way)
+                asm volatile("" ::: "memory");
+            }
             issue_idx(j + S - 1);
         }
         for (int k = 0; k < nsteps; ++k) {
@@ -226,6 +236,11 @@ stem_wgrad_kernel(const typename Tag::type* __restrict__ gout, const typename Ta
                 for (int e = 0; e < 16; ++e) acc[i][t][e] = 0.f;
 
         __syncthreads();
+        if (C::PROLOGUE_BARRIER) {                                 // (the loaders' among themselves)
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
         constexpr int NK = C::ROWS / 16;
         for (int k = 0; k < nsteps; ++k) {
             asm volatile("" ::: "memory");

@@ -33,3 +33,14 @@ def test_infinities_stay_with_their_pairs(gpu_device):
     ok = want.isfinite()
     # one rounding to the type; 3 000 terms of about one in 32 bits
     assert (got - want)[ok].abs().max() <= 2.0 ** -11 * want[ok].abs().max() + 2.0 ** -14
+
+
+# Workgroups of four and five steps, whose loaders spend most of their time in the prologue: 128 columns leave LDS for three slots of map words, and the
+# last words that the prologue asks for go where the first step's were.  The same bits every time, against the sums over pairs.
+@pytest.mark.parametrize("n,co", [(2055, 72), (2055, 264), (66000, 128)])
+def test_map_words_of_the_first_steps(gpu_device, n, co):
+    nmap, feats, grad = narrow._case(gpu_device, n, 8, co, 27, torch.float16)
+    want, _ = narrow._pairs(nmap, feats, grad)
+    got = [narrow._run(nmap, feats, grad)[0] for _ in range(20)]
+    assert all(torch.equal(g, got[0]) for g in got[1:])
+    assert (got[0].cpu().double() - want).abs().max() <= 2.0 ** -11 * want.abs().max() + n ** 0.5 * 2.0 ** -21
