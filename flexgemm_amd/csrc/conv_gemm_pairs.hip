@@ -397,7 +397,16 @@ pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const
         __syncthreads();
         const bool every = told[0] & told[1] & told[2] & told[3];
         __syncthreads();
-        if (!every) multiply(std::true_type{});
+        if (!every) {
+            multiply(std::true_type{});
+        } else {
+#pragma unroll
+            for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[i][j][e] *= kSplit3Unscale;
+        }
     }
 
     // element e of lane l: pair l % 32, column 8 * (e / 4) + 4 * (l / 32) + e % 4.  Through the wavefront's band in LDS, 32 columns at a time, out as

@@ -456,13 +456,14 @@ gather_gemm_stream_kernel(const typename Tag::type* __restrict__ src, const type
                 for (int j = 0; j < C::TN; ++j)
 #pragma unroll
                     for (int e = 0; e < 16; ++e) fine = fine && split3_holds(acc[i][j][e]);
-            if (__ballot(!fine) != 0) {
+            const bool repeat = __ballot(!fine) != 0;
 #pragma unroll
-                for (int i = 0; i < C::TM; ++i)
+            for (int i = 0; i < C::TM; ++i)
 #pragma unroll
-                    for (int j = 0; j < C::TN; ++j)
+                for (int j = 0; j < C::TN; ++j)
 #pragma unroll
-                        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+                    for (int e = 0; e < 16; ++e) acc[i][j][e] = repeat ? 0.f : acc[i][j][e] * kSplit3Unscale;
+            if (repeat) {
                 uint32_t code = (uint32_t)tile_code[c_t];
                 const uint32_t* slot = plan_idx + (size_t)plan_seg[c_t] * BM + wave_m * C::WM + l32;
                 for (; code != 0; code &= code - 1, slot += BM) {

@@ -13,21 +13,24 @@ using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
 // Of the nine products of two such sums the six down to 2^-18 are added, smallest first; the three left out are 2^-26
 // of the product together, an eighth of a rounding to fp32, and 16 values of K share six roundings where the fp32 unit rounds
 // every other one (error of an output against 64 bits, 96 channels: 1.58e-7, fp32 units 1.90e-7).
-// What they cannot stand for: an infinity (or a value that rounds to one) leaves NaN behind it, and under 2^-110 the third part
-// runs out of exponents.  The kernels look at their sums (split3_holds) and repeat a tile on the fp32 units.
+// Both operands are multiplied by 2^24 first: the last bit of any fp32 value is then 2^-125 or more, so that no part falls below the normal numbers and every
+// finite value under 2^104 is its three parts, the subnormal ones too; the sums are 2^48 times as large.
+// What they cannot stand for: an infinity, a larger value or a sum past 2^80 leaves an infinity or NaN behind it, and products that fall below the normal numbers
+// are lost, which a sum (of up to 2^22 products) shows that is not 2^24 times as large as all of them, 2^-79 (2^-127 of the result).  The
+// kernels look at their sums (split3_holds) and repeat a tile on the fp32 units.  (A sum of zero is one whose products are under half of the smallest subnormal.)
+constexpr float kSplit3Scale = 0x1p24f, kSplit3Unscale = 0x1p-48f;
 struct Split3 {
     bf16x8 part[3];
 };
-template <bool NEGATED = false>
-__device__ __forceinline__ Split3 split3(const u32x4& lo, const u32x4& hi) {
+// scale: kSplit3Scale, or that negated
+__device__ __forceinline__ Split3 split3(const u32x4& lo, const u32x4& hi, float scale = kSplit3Scale) {
     using bf16x2 = __bf16 __attribute__((ext_vector_type(2)));
     using f32x2 = float __attribute__((ext_vector_type(2)));
     uint32_t out[3][4];
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
-        float x = __builtin_bit_cast(float, p < 2 ? lo[p * 2] : hi[p * 2 - 4]);
-        float y = __builtin_bit_cast(float, p < 2 ? lo[p * 2 + 1] : hi[p * 2 - 3]);
-        if (NEGATED) x = -x, y = -y;            // (an operand modifier)
+        float x = __builtin_bit_cast(float, p < 2 ? lo[p * 2] : hi[p * 2 - 4]) * scale;
+        float y = __builtin_bit_cast(float, p < 2 ? lo[p * 2 + 1] : hi[p * 2 - 3]) * scale;
 #pragma unroll
         for (int t = 0; t < 3; ++t) {
             const f32x2 xy = {x, y};
@@ -44,10 +47,10 @@ __device__ __forceinline__ Split3 split3(const u32x4& lo, const u32x4& hi) {
     }
     return s;
 }
-// neither an infinity, NaN nor other than zero below 2^-96
+// (of the sum as it is, 2^48 times the result) neither an infinity, NaN nor other than zero below 2^-79
 __device__ __forceinline__ bool split3_holds(float sum) {
     const uint32_t u = __builtin_bit_cast(uint32_t, sum) << 1;
-    return u == 0u || u - (31u << 24) < (224u << 24);
+    return u == 0u || u - (48u << 24) < (207u << 24);
 }
 // the six products, smallest first, of 32 x 32 over 16 values of K or 16 x 16 over 32
 constexpr int kSplit3Products = 6;

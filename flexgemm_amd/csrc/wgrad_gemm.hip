@@ -461,7 +461,7 @@ __device__ __forceinline__ void multiply_f32(unsigned char* ring, uint32_t* sync
 #pragma unroll
             for (int i = 0; i < C::TM; ++i) rows_raw[i] = fetch(cur + a_off[i], kRowA);
             if (C::TM < 3) __builtin_amdgcn_sched_barrier(0);
-            Split3 cols3 = split3<HALF == 1>(cols_raw.lo, cols_raw.hi), rows3[C::TM];
+            Split3 cols3 = split3(cols_raw.lo, cols_raw.hi, HALF == 1 ? -kSplit3Scale : kSplit3Scale), rows3[C::TM];
 #pragma unroll
             for (int i = 0; i < C::TM; ++i) rows3[i] = split3(rows_raw[i].lo, rows_raw[i].hi);
 #pragma unroll
@@ -471,7 +471,7 @@ __device__ __forceinline__ void multiply_f32(unsigned char* ring, uint32_t* sync
                 for (int p = 0; p < kSplit3Products; ++p)
 #pragma unroll
                     for (int i = 0; i < C::TM; ++i) mma_split3(acc[i][j], cols3, rows3[i], p);
-                if (j + 1 < C::TN) cols3 = split3<HALF == 1>(cols_raw.lo, cols_raw.hi);
+                if (j + 1 < C::TN) cols3 = split3(cols_raw.lo, cols_raw.hi, HALF == 1 ? -kSplit3Scale : kSplit3Scale);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // done reading this stage
         }
@@ -496,9 +496,9 @@ __device__ __forceinline__ void multiply_f32(unsigned char* ring, uint32_t* sync
 #pragma unroll
             for (int j = 0; j < C::TN; ++j) {
                 sum[i][j] += acc[i][j];
-                if (HALF == 1) sum[i][j] = -sum[i][j];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) fine = fine && split3_holds(sum[i][j][e]);
+                sum[i][j] *= HALF == 1 ? -kSplit3Unscale : kSplit3Unscale;
             }
         if (__ballot(!fine) != 0) again(m, sum);
         // The halves meet in the stage that was multiplied last, which the loaders leave alone until both have been at the next barrier: one

@@ -1,5 +1,5 @@
 """fp32 products made of bf16 parts: the streaming kernel's tiles, the pairs kernel and the weight gradient against 64-bit sums, and the repeat on
-the fp32 units where the parts cannot stand for a value (infinities, NaN, values that round to an infinity, values under 2^-110)."""
+the fp32 units where the parts cannot stand for a value or a sum (infinities, NaN, values from 2^104 on, sums past 2^80 or under 2^-127)."""
 import pytest
 import torch
 
@@ -12,11 +12,11 @@ from test_gpu_wgrad_split import coords_of
 pytestmark = pytest.mark.gpu
 
 
-def _layer(monkeypatch, tile, res, ci, co, change=None, scale=1.0):
+def _layer(monkeypatch, tile, res, ci, co, change=None, scale=1.0, weight_scale=1.0):
     coords = torch.from_numpy(reference_test_shell(res)).cuda()
     g = torch.Generator(device="cuda").manual_seed(ci + co)
     feats = torch.randn(len(coords), ci, generator=g, device="cuda") * scale
-    weight = torch.randn(co, 3, 3, 3, ci, generator=g, device="cuda") / (27 * ci) ** 0.5
+    weight = torch.randn(co, 3, 3, 3, ci, generator=g, device="cuda") / (27 * ci) ** 0.5 * weight_scale
     if change is not None:
         change(feats, weight)
     nat.host()                  # (takes note of the table before it is replaced)
@@ -64,18 +64,26 @@ def test_what_three_parts_cannot_stand_for(monkeypatch, tile, ci, co):
     assert bool(((got.double() - want).abs()[huge] <= 1e-6 * want.abs()[huge]).all())
 
 
+# (log2) features and weights about: small ones whose products are small; small against large, whose sums a guard on sums alone lets through: parts that fall
+# below bf16's normal numbers, then below all of them (subnormal values); sums past 2^80 and values past 2^104, which are multiplied again
+MAGNITUDES = [(-113, 0), (-116, 30), (-120, 40), (-126, 60), (-136, 60), (-142, 100), (30, -110), (50, -120), (60, -130), (60, 30), (110, -60), (-120, 115)]
+
+
 @pytest.mark.parametrize("tile,ci,co", TILES)
-def test_small_values_keep_their_bits(monkeypatch, tile, ci, co):
-    got, want, _ = _layer(monkeypatch, tile, 16, ci, co, scale=1e-34)
+@pytest.mark.parametrize("of_feats,of_weight", MAGNITUDES)
+def test_magnitudes_apart(monkeypatch, tile, ci, co, of_feats, of_weight):
+    got, want, _ = _layer(monkeypatch, tile, 16, ci, co, scale=2.0 ** of_feats, weight_scale=2.0 ** of_weight)
+    assert float(want.norm()) > 0
+    # as of values about one: a power of two more or less changes no rounding (the operands are taken as they came out, subnormal ones included)
     assert float((got.double() - want).norm() / want.norm()) <= (27 * ci) ** 0.5 * 2.0 ** -24
 
 
-def _weight_grad(n, ci, co, scale=1.0, change=None):
+def _weight_grad(n, ci, co, scale=1.0, change=None, grad_scale=1.0):
     """The weight gradient, the same in 64 bits, and each sum's magnitude, of n voxels in a cube two thirds full."""
     side = round((1.5 * n) ** (1 / 3)) + 1
     cache = SubMConv3dFunction._compute_neighbor_cache(coords_of(n, side, n), torch.Size([1, ci, side, side, side]), (3, 3, 3), (1, 1, 1), True)
     g = torch.Generator(device="cuda").manual_seed(n + ci)
-    feats, grad = torch.randn(n, ci, generator=g, device="cuda") * scale, torch.randn(n, co, generator=g, device="cuda")
+    feats, grad = torch.randn(n, ci, generator=g, device="cuda") * scale, torch.randn(n, co, generator=g, device="cuda") * grad_scale
     if change is not None:
         change(feats, grad)
     got = nat.host().wgrad(grad, feats, cache, 27, False, -1)[0].view(co, 27, ci)
@@ -95,12 +103,20 @@ SPLIT_GRADS = [(9215, 96, 96), (9216, 96, 96), (12001, 96, 92), (14335, 64, 64),
 
 
 @pytest.mark.parametrize("n,ci,co", SPLIT_GRADS)
-@pytest.mark.parametrize("scale", [1.0, 1e-34])
-def test_weight_gradient(n, ci, co, scale):
-    got, want, size = _weight_grad(n, ci, co, scale)
+def test_weight_gradient(n, ci, co):
+    _agrees(n, *_weight_grad(n, ci, co))
+
+
+def _agrees(n, got, want, size):
     # k products summed in any order: within k units of the sum of their magnitudes; sums of random signs, on the whole, within sqrt(k) of their own size
-    assert bool(((got - want).abs() <= n * 2.0 ** -23 * size + 2.0 ** -149 * n).all())
+    assert float(want.norm()) > 0 and bool(((got - want).abs() <= n * 2.0 ** -23 * size).all())
     assert float((got - want).norm() / want.norm()) <= n ** 0.5 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("n,ci,co", [(9216, 96, 96), (14336, 64, 64), (3001, 192, 180)])
+@pytest.mark.parametrize("of_feats,of_grad", MAGNITUDES)
+def test_weight_gradient_of_magnitudes_apart(n, ci, co, of_feats, of_grad):
+    _agrees(n, *_weight_grad(n, ci, co, scale=2.0 ** of_feats, grad_scale=2.0 ** of_grad))
 
 
 @pytest.mark.parametrize("n,ci,co", [(9216, 96, 96), (14336, 64, 64), (3001, 192, 180)])
