@@ -303,6 +303,11 @@ pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const
             }
         }
     f32x16 acc[C::TM][C::TN];
+    // fp32: which way the columns and the sums count at present.  What the matrix unit drops of its sums points downwards, the more the larger they are; turned after
+    // two thirds of the slabs, nine tenths of it cancel, and every other offset starts with the other sign.  Mean error of the outputs over their root mean
+    // square, 1 976 voxels, 1024 channels: -1.9e-7 -> 7e-11, 2-norm 5.3e-7 -> 4.9e-7 (fp32 units 5.8e-7).
+    float scale = wv & 1 ? -kSplit3Scale : kSplit3Scale;
+    const int turn_at = (2 * slabs + 1) / 3;
     auto multiply = [&](auto on_fp32_units) __attribute__((always_inline)) {
         constexpr bool SPLIT = C::ES == 4 && !decltype(on_fp32_units)::value;
         b_soff = (uint32_t)wv * b.v_stride;
@@ -316,6 +321,16 @@ pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const
         issue(0);
         if (slabs > 1) issue(1);
         for (int s = 0; s < slabs; ++s) {
+            if (SPLIT && s == turn_at) {
+                scale = -scale;
+                asm volatile("" ::: "memory");         // (a branch, not a choice per sum in every step)
+#pragma unroll
+                for (int i = 0; i < C::TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < C::TN; ++j)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) acc[i][j][e] = -acc[i][j][e];
+            }
             if (s + 1 < slabs) wait_vmcnt<C::LPS>();        // all but the newest slab's loads have landed
             else wait_vmcnt<0>();
             asm volatile("" ::: "memory");
@@ -364,7 +379,7 @@ pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const
                     for (int i = 0; i < C::TM; ++i) rows3[i] = split3(af[kk][i], af[kk + 1][i]);
 #pragma unroll
                     for (int j = 0; j < C::TN; ++j) {
-                        const Split3 cols3 = split3(bf[kk][j], bf[kk + 1][j]);
+                        const Split3 cols3 = split3(bf[kk][j], bf[kk + 1][j], scale);
 #pragma unroll
                         for (int i = 0; i < C::TM; ++i) mma_split3(acc[i][j], cols3, rows3[i]);     // transposed tile
                     }
@@ -400,12 +415,13 @@ pair_gemm_kernel(const typename Tag::type* __restrict__ src, PairWeight b, const
         if (!every) {
             multiply(std::true_type{});
         } else {
+            const float unscale = scale < 0.f ? -kSplit3Unscale : kSplit3Unscale;
 #pragma unroll
             for (int i = 0; i < C::TM; ++i)
 #pragma unroll
                 for (int j = 0; j < C::TN; ++j)
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) acc[i][j][e] *= kSplit3Unscale;
+                    for (int e = 0; e < 16; ++e) acc[i][j][e] *= unscale;
         }
     }
 

@@ -64,6 +64,19 @@ def test_what_three_parts_cannot_stand_for(monkeypatch, tile, ci, co):
     assert bool(((got.double() - want).abs()[huge] <= 1e-6 * want.abs()[huge]).all())
 
 
+# Long sums: what the matrix unit drops of every addition points downwards, and must cancel.  Six additions for 16 values of K, off by 2^-24 of the running
+# sum or less in the mean of their squares, whose own square is half of the last one's on average; and errors that point neither way have a mean
+# within six standard deviations of that of as many independent ones.
+@pytest.mark.parametrize("tile,ci,co", [((128, 256, 128), 512, 136), ((256, 128, 128), 1024, 128), ((256, 64, 64), 512, 64), ((256, 64, 128), 1024, 64),
+                                        ((256, 32, 64), 512, 96), (None, 512, 96), (None, 1024, 64)])
+@pytest.mark.parametrize("positive", [False, True])
+def test_long_sums_point_neither_way(monkeypatch, tile, ci, co, positive):
+    got, want, _ = _layer(monkeypatch, tile, 16, ci, co, (lambda feats, weight: feats.abs_()) if positive else None)
+    error = got.double() - want
+    assert float(error.norm() / want.norm()) <= (27 * ci * 6 / 16 / 2) ** 0.5 * 2.0 ** -24
+    assert abs(float(error.mean())) <= 6 * float(error.norm()) / error.numel()
+
+
 # (log2) features and weights about: small ones whose products are small; small against large, whose sums a guard on sums alone lets through: parts that fall
 # below bf16's normal numbers, then below all of them (subnormal values); sums past 2^80 and values past 2^104, which are multiplied again
 MAGNITUDES = [(-113, 0), (-116, 30), (-120, 40), (-126, 60), (-136, 60), (-142, 100), (30, -110), (50, -120), (60, -130), (60, 30), (110, -60), (-120, 115)]
