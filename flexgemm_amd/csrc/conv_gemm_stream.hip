@@ -483,8 +483,12 @@ gather_gemm_stream_kernel(const typename Tag::type* __restrict__ src, const type
                     for (int e = 0; e < 16; ++e) acc[i][j][e] = repeat ? 0.f : acc[i][j][e] * unscale;
             if (repeat) {
                 uint32_t code = (uint32_t)tile_code[c_t];
-                const uint32_t* slot = plan_idx + (size_t)plan_seg[c_t] * BM + wave_m * C::WM + l32;
-                for (; code != 0; code &= code - 1, slot += BM) {
+                uint32_t at_slot = (uint32_t)plan_seg[c_t];
+                for (; code != 0; code &= code - 1, ++at_slot) {
+                    // (the bands that were left out stay out: the zeros of missing neighbors times an infinity are NaN)
+                    const uint32_t mine = ((plan_band != nullptr ? plan_band[at_slot] : 0xFFFFFFFFu) >> (wave_m * C::TM)) & kMineAll;
+                    if (mine == 0) continue;
+                    const uint32_t* slot = plan_idx + (size_t)at_slot * BM + wave_m * C::WM + l32;
                     const unsigned char* lines = (const unsigned char*)panel +
                         ((size_t)(__builtin_ctz(code) * slabs) * cols_pad + c_ct * BN + wave_n * C::WN + l32) * kSlabBytes;
 #pragma unroll 1
@@ -495,6 +499,7 @@ gather_gemm_stream_kernel(const typename Tag::type* __restrict__ src, const type
                             line[j] = *(const u32x4*)(lines + ((size_t)(at / kSlabBytes) * cols_pad + j * 32) * kSlabBytes + at % kSlabBytes);
 #pragma unroll
                         for (int i = 0; i < C::TM; ++i) {
+                            if (C::TM > 1 && !((mine >> i) & 1u)) continue;
                             const uint32_t m = slot[i * 32];
                             u32x4 row = {0u, 0u, 0u, 0u};
                             if (m != FGX_EMPTY32 && at < row_bytes) row = *(const u32x4*)((const unsigned char*)src + (size_t)m * row_bytes + at);

@@ -64,6 +64,27 @@ def test_what_three_parts_cannot_stand_for(monkeypatch, tile, ci, co):
     assert bool(((got.double() - want).abs()[huge] <= 1e-6 * want.abs()[huge]).all())
 
 
+@pytest.mark.parametrize("tile,ci,co", [t for t in TILES if t[0] is not None])
+def test_the_repeat_leaves_out_what_the_product_leaves_out(monkeypatch, tile, ci, co):
+    """An infinite weight at one offset: 32 rows of the order none of which has it are not multiplied by it, the second time either."""
+    plain, _, _ = _layer(monkeypatch, tile, 16, ci, co)
+    coords = torch.from_numpy(reference_test_shell(16)).cuda()
+    cache = SubMConv3dFunction._compute_neighbor_cache(coords, torch.Size([1, ci, 16, 16, 16]), (3, 3, 3), (1, 1, 1), False)
+    order = cache.sorted_idx
+    has = cache.neighbor_map.view(torch.int32)[order] >= 0
+    has = torch.cat([has, has.new_zeros((-len(has)) % 64, 27)]).view(-1, 32, 27).any(1)                  # [bands of 32 rows, offsets]
+    # an offset that one band of a wavefront's 64 rows has and the other has not
+    v = int((has[::2] != has[1::2]).any(0).nonzero()[0])
+
+    def change(feats, weight):
+        weight.view(co, 27, ci)[:, v] = INF
+    got, _, _ = _layer(monkeypatch, tile, 16, ci, co, change)
+    without = torch.zeros(len(order), dtype=torch.bool, device="cuda")
+    without[order] = ~has[:, v].repeat_interleave(32)[:len(order)]
+    assert without.any() and not got[~without].isfinite().any() and got[without].isfinite().all()
+    assert float((got[without] - plain[without]).norm() / plain[without].norm()) <= 2 * (27 * ci) ** 0.5 * 2.0 ** -24
+
+
 # Long sums: what the matrix unit drops of every addition points downwards, and must cancel.  Six additions for 16 values of K, off by 2^-24 of the running
 # sum or less in the mean of their squares, whose own square is half of the last one's on average; and errors that point neither way have a mean
 # within six standard deviations of that of as many independent ones.
