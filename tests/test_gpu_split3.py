@@ -98,6 +98,12 @@ def test_long_sums_point_neither_way(monkeypatch, tile, ci, co, positive):
     assert abs(float(error.mean())) <= 6 * float(error.norm()) / error.numel()
 
 
+@pytest.mark.parametrize("tile,ci,co", TILES)
+def test_small_values_keep_their_bits(monkeypatch, tile, ci, co):
+    got, want, _ = _layer(monkeypatch, tile, 16, ci, co, scale=1e-34)
+    assert float((got.double() - want).norm() / want.norm()) <= (27 * ci) ** 0.5 * 2.0 ** -24
+
+
 # (log2) features and weights about: small ones whose products are small; small against large, whose sums a guard on sums alone lets through: parts that fall
 # below bf16's normal numbers, then below all of them (subnormal values); sums past 2^80 and values past 2^104, which are multiplied again
 MAGNITUDES = [(-113, 0), (-116, 30), (-120, 40), (-126, 60), (-136, 60), (-142, 100), (30, -110), (50, -120), (60, -130), (60, 30), (110, -60), (-120, 115)]
@@ -137,20 +143,20 @@ SPLIT_GRADS = [(9215, 96, 96), (9216, 96, 96), (12001, 96, 92), (14335, 64, 64),
 
 
 @pytest.mark.parametrize("n,ci,co", SPLIT_GRADS)
-def test_weight_gradient(n, ci, co):
-    _agrees(n, *_weight_grad(n, ci, co))
-
-
-def _agrees(n, got, want, size):
+@pytest.mark.parametrize("scale", [1.0, 1e-34])
+def test_weight_gradient(n, ci, co, scale):
+    got, want, size = _weight_grad(n, ci, co, scale)
     # k products summed in any order: within k units of the sum of their magnitudes; sums of random signs, on the whole, within sqrt(k) of their own size
-    assert float(want.norm()) > 0 and bool(((got - want).abs() <= n * 2.0 ** -23 * size).all())
+    assert bool(((got - want).abs() <= n * 2.0 ** -23 * size + 2.0 ** -149 * n).all())
     assert float((got - want).norm() / want.norm()) <= n ** 0.5 * 2.0 ** -24
 
 
 @pytest.mark.parametrize("n,ci,co", [(9216, 96, 96), (14336, 64, 64), (3001, 192, 180)])
 @pytest.mark.parametrize("of_feats,of_grad", MAGNITUDES)
 def test_weight_gradient_of_magnitudes_apart(n, ci, co, of_feats, of_grad):
-    _agrees(n, *_weight_grad(n, ci, co, scale=2.0 ** of_feats, grad_scale=2.0 ** of_grad))
+    got, want, size = _weight_grad(n, ci, co, scale=2.0 ** of_feats, grad_scale=2.0 ** of_grad)
+    assert float(want.norm()) > 0 and bool(((got - want).abs() <= n * 2.0 ** -23 * size).all())
+    assert float((got - want).norm() / want.norm()) <= n ** 0.5 * 2.0 ** -24
 
 
 @pytest.mark.parametrize("n,ci,co", [(9216, 96, 96), (14336, 64, 64), (3001, 192, 180)])
