@@ -372,11 +372,11 @@ struct WStreamCfg {
 // fp32 multipliers of the streaming kernel, transposed: element e of lane l is row l % 16 (co) and column 4 * (l / 16) + e (ci) of a 16 x 16
 // product, so a lane stores 16 bytes of an output row, four lanes 64.  A wavefront has a WM x WN part of the tile.
 // HALF 0 and 1: over one half of a step's 64 pairs, in three bf16 parts (split3.h), 32 pairs a product (lane l holds column l % 16 of eight of them).
-// Making the parts takes 264 vector instructions (1 056 cycles) beside 54 products (864) of a 48 x 48 part, so a SIMD has two such wavefronts, one of which
+// Making the parts takes 216 vector instructions (864 cycles and more) beside 54 products (864) of a 48 x 48 part, so a SIMD has two such wavefronts, one of which
 // fills the other's waits; alone, with all 64 pairs, it was no faster than the fp32 units.  The matrix unit rounds its sums downwards: HALF 1 multiplies
 // negated columns and the halves' sums are subtracted, so what it drops cancels (error against 64 bits, 96 channels, 166 977 and 407 279 voxels: fp32 units
-// 3.1e-7 and 3.3e-7, both halves alike 3.0e-7 and 4.6e-7, so 2.5e-7 and 2.6e-7).  Us, before and now: 96 channels, 38 407 voxels 103 88, 166 977 303 246;
-// 192 channels 334 260 and 1 146 854; 64 channels 63 58 and 173 152.
+// 3.1e-7 and 3.3e-7, both halves alike 3.0e-7 and 4.6e-7, so 2.5e-7 and 2.6e-7).  Us, on the fp32 units and so: 96 channels, 38 407 voxels 103 85 - 88, 166 977
+// 303 240; 192 channels 334 258 and 1 146 862; 64 channels 63 55 and 173 140.
 // HALF -1: over all pairs, four at a time (lane l holds row l / 16 of the four), on the fp32 units, whose rate is a sixteenth of the 16-bit one: for few
 // pairs, where the halves' meeting and their longer code cost more than they save (see units_are_faster).
 // 96 x 96 because it is the widest tile whose three stages of 64 pairs fit LDS.
@@ -461,9 +461,9 @@ __device__ __forceinline__ void multiply_f32(unsigned char* ring, uint32_t* sync
 #pragma unroll
             for (int i = 0; i < C::TM; ++i) rows_raw[i] = fetch(cur + a_off[i], kRowA);
             if (C::TM < 3) __builtin_amdgcn_sched_barrier(0);
-            Split3 cols3 = split3(cols_raw.lo, cols_raw.hi, HALF == 1 ? -kSplit3Scale : kSplit3Scale), rows3[C::TM];
+            Split3 cols3 = split3<true>(cols_raw.lo, cols_raw.hi, HALF == 1 ? -kSplit3Scale : kSplit3Scale), rows3[C::TM];
 #pragma unroll
-            for (int i = 0; i < C::TM; ++i) rows3[i] = split3(rows_raw[i].lo, rows_raw[i].hi);
+            for (int i = 0; i < C::TM; ++i) rows3[i] = split3<true>(rows_raw[i].lo, rows_raw[i].hi);
 #pragma unroll
             for (int j = 0; j < C::TN; ++j) {
                 if (j + 1 < C::TN) cols_raw = fetch(cur + b_off[j + 1], kRowB);
@@ -471,7 +471,7 @@ __device__ __forceinline__ void multiply_f32(unsigned char* ring, uint32_t* sync
                 for (int p = 0; p < kSplit3Products; ++p)
 #pragma unroll
                     for (int i = 0; i < C::TM; ++i) mma_split3(acc[i][j], cols3, rows3[i], p);
-                if (j + 1 < C::TN) cols3 = split3(cols_raw.lo, cols_raw.hi, HALF == 1 ? -kSplit3Scale : kSplit3Scale);
+                if (j + 1 < C::TN) cols3 = split3<true>(cols_raw.lo, cols_raw.hi, HALF == 1 ? -kSplit3Scale : kSplit3Scale);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // done reading this stage
         }
@@ -1759,8 +1759,9 @@ __global__ void __launch_bounds__(256) split_reduce_kernel(const float* __restri
     for (int e = 0; e < 4; ++e) dst[e] = sum[e];
 }
 
-// fp32 weight gradient of few pairs: measured (us, parts and units): 96 channels, one tile, 4 083 voxels 30.6 27.7, 8 004 34.9 34.1, 10 494 36.7 37.4;
-// 64 channels 5 876 24.2 22.2, 13 258 30.3 29.9, 16 307 31.1 31.9;  128 channels, four tiles, 2 581 27.5 26.2, 4 083 31.6 31.6;  192 channels 2 581 37.0 36.7.
+// fp32 weight gradient of few pairs: measured (us, parts and units): 96 channels, one tile, 3 944 voxels 32.1 29.0, 7 664 36.0 34.4, 9 128 37.1 36.2, 12 576 41.5
+// 41.7;  64 channels 5 648 25.5 23.1, 12 656 30.2 28.9, 14 874 31.3 31.9, 20 840 37.4 37.8;  128 channels, four tiles, 2 480 26.9 25.7, 3 944 31.7 31.1, 5 106
+// 33.4 34.4;  192 channels 2 480 36.1 36.1, 3 944 43.7 46.4.
 bool units_are_faster(size_t n, unsigned tiles, int tile) { return n * tiles < (tile == 96 ? 9216u : 14336u); }
 
 template <typename Tag, int TILE>
