@@ -74,14 +74,16 @@ bool rule_wgrad_f32(size_t n, int Ci, int Co, int V, fgx_schedule* out) {
 //   last and heaviest ones (`last`; `least` for a lone round, whose heaviest tile has half as many offsets again as the mean), at
 //   a rate that falls with c: a fragment's parts are made once and multiplied c / 32 times; 7 us of its own;
 //   tiled kernel, on the fp32 units, with K split until the pieces even out: a third of the rate, and 15 us of its own.
-// Measured forward, us, 256 x 128 / 256 x 64 / 256 x 32 (64-byte slabs but for the first):  128 channels, 49 829 voxels 199 233
-// 227;  77 160 261 305 300;  166 977 412 539 553;  407 279 911 1 160 1 234;  96 channels, 166 977 voxels 307 407 314;  192
-// channels 1 092 1 142 1 202, 128 x 256 1 041;  48 channels 213 120 118, slabs of 128 bytes 213 174;  64 channels 213 154 155, 174;
-// 32 channels, 77 160 voxels 82 59 40, tiled 59.   With what the fp32 units wanted (narrow tiles before padding) the products
+// Measured forward, us, 256 x 128 / 256 x 64 / 256 x 32 (64-byte slabs but for the first):  128 channels, 49 976 voxels 217 246
+// 263;  77 064 287 315 343;  166 232 440 555 605;  406 920 938 1 205 1 365;  96 channels, 166 232 voxels 324 423 345;  192
+// channels 1 135 1 187 1 312, 128 x 256 1 112;  48 channels 222 128 131, 64 channels 227 163 171.  256 x 64 on 64- and 128-byte slabs: 166 232
+// voxels, into 64 columns, of 32 channels 99 92, 40 127 151, 64 162 152, 80 197 216, 96 232 217, 112 267 281, 128 302 283, 192 442 416; 49 976 voxels, 64 87
+// 81, 128 162 150; 406 920, 64 342 320, 128 642 606.  32 channels, 77 064 voxels 89 64 43, tiled 51; 48, 36 936 voxels 79 (256 x 64) 68 (256 x 32), tiled 75,
+// 20 330 75 54 66.  With what the fp32 units wanted (narrow tiles before padding) the products
 // of three parts took 554 us under 128 channels at 166 977 voxels, on the fp32 units 681;  192 channels 1 301 and 1 378.
 void rule_gemm_f32(size_t n, int K, int cols, int V, fgx_schedule* out) {
     const size_t row_bytes = (size_t)K * 4;
-    const int slab = row_bytes == 128 ? 128 : 64;       // (of 64 columns: whole slabs of longer rows count for more than their length)
+    const int slab = row_bytes % 128 == 0 ? 128 : 64;   // (of 64 columns: the longer ones are 6 to 8 % ahead where none is part empty)
     const double row_tiles = cdiv(n ? n : 1, 256);
     const int wide = cdiv(cols, 64) * 64;
     const bool narrow = cdiv(cols, 32) * 32 < wide;
