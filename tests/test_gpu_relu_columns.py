@@ -52,3 +52,22 @@ def test_filled_rows_change_nothing(dtype, ci, co, relu):
         other = grads()
     for a, b, c, d in zip(want, other, grads(twice=True), grads(composed=True)):
         assert a.shape == b.shape and torch.equal(a, b) and torch.equal(a, c) and torch.equal(a, d)
+
+
+# What a layer holds between its passes beside its output: up to 256 MB of filled rows, nothing to speak of where they are more
+@pytest.mark.parametrize("res,ci,kept", [(60, 82, True), (500, 130, True), (510, 130, False), (510, 131, False)])
+def test_memory_held_between_the_passes(res, ci, kept):
+    coords = torch.from_numpy(reference_test_shell(res)).cuda()
+    n, shape, co = len(coords), torch.Size([1, ci, res, res, res]), 64
+    feats = torch.randn(n, ci, device="cuda").half().requires_grad_(True)
+    weight = (torch.randn(co, 3, 3, 3, ci, device="cuda") / 30).half().requires_grad_(True)
+    filled = n * ((ci + 7) // 8 * 8) * 2
+    assert (filled <= 256 << 20) == kept
+    out, cache = sparse_submanifold_conv3d(feats, coords, shape, weight)
+    torch.autograd.grad(out, [feats, weight], torch.ones_like(out))         # (the cache has all of its tables)
+    del out
+    before = torch.cuda.memory_allocated()
+    out, _ = sparse_submanifold_conv3d(feats, coords, shape, weight, None, cache)
+    held = torch.cuda.memory_allocated() - before - out.untyped_storage().nbytes()
+    assert held <= (filled if kept else 0) + (1 << 20)
+    torch.autograd.grad(out, [feats, weight], torch.ones_like(out))
