@@ -208,9 +208,9 @@ struct PairCfg {
 // 0.9 and 1.2 of that time, ahead only for the second, behind for everything smaller.
 // fp32 multiplies three bf16 parts of every value (split3.h), six products for one: half as long a slab is enough work for a barrier, and its
 // stages and fragments let four workgroups share a CU, which cover the few slabs' start and end (96 channels have three of 128 bytes). It is bound by making
-// the parts (176 vector instructions to 18 products of a wavefront's 32 x 96) and by what it writes: 38 407 voxels, 96 channels, with the sums
-// 130 us on the fp32 units (141 in two workgroups of 128-byte slabs, 125 with the sums leaving in bands of 32 columns), 105 in parts; 16 307 voxels,
-// 128 channels 76 -> 66, 256 channels 227 -> 194; error against 64 bits 1.90e-7 -> 1.58e-7. A tile with a sum that the parts cannot stand for is multiplied
+// the parts (208 vector instructions to 18 products of a wavefront's 32 x 96) and by what it writes: 38 407 voxels, 96 channels, with the sums
+// 130 us on the fp32 units (141 in two workgroups of 128-byte slabs, 125 with the sums leaving in bands of 32 columns), 110 in parts (105 before
+// both operands were scaled); 16 400 voxels, 128 channels 76 -> 71, 256 channels 227 -> 208; error against 64 bits 1.90e-7 -> 1.56e-7. A tile with a sum that the parts cannot stand for is multiplied
 // a second time, on the fp32 units.
 template <typename Tag, bool TR, int BN, int WAVES_M>
 __global__ void __launch_bounds__(256, pair_groups((int)sizeof(typename Tag::type)))
@@ -566,8 +566,8 @@ extern "C" {
 //   1024 x  128      33  18   35  22   48  30   73  34   74  45              1024 x 2048   447 379   809 480   814 542   829 609
 // 64 columns (256 x 64: 15 12, 20 14, 24 19, 33 20, 34 21) gain little more than the plan: a training step whose input gradient still wants the
 // masks is up to 5 % slower for it, a pass at inference 1.16 to 1.44 times as fast.
-// fp32 (figures of the fp32 units on both sides; in three bf16 parts both are shorter, and level where they were: 49 829 rows, kept, 64 x 64 73 75, 96 x 96
-// 145 121, 128 x 128 200 192, 160 x 160 301 319):  what is not multiplied counts for more than in 16 bits: from 64 channels on, up to a number of rows and as long as the sums,
+// fp32 (figures of the fp32 units on both sides; in three bf16 parts both are shorter, and level where they were: 49 976 rows, kept, 64 x 64 81 76, 96 x 96
+// 167 127, 128 x 128 219 209, 160 x 160 340 340):  what is not multiplied counts for more than in 16 bits: from 64 channels on, up to a number of rows and as long as the sums,
 // with 0.45 of a row's offsets, stay below 5 MB a channel.  Their traffic, which outgrows the 256 MB memory-side cache, costs what the products
 // save from 4.5 MB on, and by 5 MB also the 30 to 50 us of tables that a fresh cache is spared (64 x 256, cache and one layer, 27 200 rows: forward
 // 248 230, training 552 543;  38 400 rows: 354 325, 765 750;  24 400 rows, training 500 459).  Beyond: 96 x 96, 71 359 rows 244 250,

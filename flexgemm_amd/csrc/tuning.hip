@@ -127,7 +127,8 @@ void rule_gemm_f32(size_t n, int K, int cols, int V, fgx_schedule* out) {
 // (where one figure stands, the tile stays; 64 -> 64 stays tiled below 24 576 voxels.)  The tiled kernel splits few rows well: under up to 64 columns, or rows of 512 bytes and more, it is level up
 // to 10 000 voxels (8 004: 96 -> 64 21.0 22.3, 384 -> 96 43 47, 768 -> 128 64 83), otherwise up to 5 000 (4 947: 80 -> 80 21.0 22.7); and it wants no gather
 // plan and no packed weight, 14 us of the host's time in a training pass on new coordinates, which little work does not bring in (64 -> 64 at 10 494 voxels
-// gains 3.5 us a product, at 28 169 9.7).
+// gains 3.5 us a product, at 28 169 9.7).  A plan of another height than the neighboring layers' costs a new cache 6 to 13 us of the device, which the limits in n
+// stand for as far as one layer can tell; a stack of unlike widths may pay it twice (32 -> 64 -> 128 at inference, 36 936 voxels 115 127; most gain, 20 330 113 102).
 bool small_stream_tile(size_t n, int K, int cols, fgx_schedule* out) {
     const int slabs = (int)cdiv((size_t)K * 2, (size_t)128);
     if (K * 2 <= 64 || !stream_lds_fits(256, 128, 128, cols)) return false;

@@ -42,9 +42,9 @@ XCDS = 8
 # the sources each role's kernels are built from
 ROLE_SOURCES = {
     "gemm": ["flexgemm_amd/csrc/conv_gemm_stream.hip", "flexgemm_amd/csrc/conv_gemm.hip", "flexgemm_amd/csrc/gemm_device.h",
-             "flexgemm_amd/csrc/lds_read.h", "flexgemm_amd/csrc/fgx_common.h", "flexgemm_amd/csrc/tuning.hip"],
+             "flexgemm_amd/csrc/split3.h", "flexgemm_amd/csrc/lds_read.h", "flexgemm_amd/csrc/fgx_common.h", "flexgemm_amd/csrc/tuning.hip"],
     "wgrad": ["flexgemm_amd/csrc/wgrad_sweep.hip", "flexgemm_amd/csrc/wgrad_gemm.hip", "flexgemm_amd/csrc/wgrad_device.h",
-              "flexgemm_amd/csrc/lds_read.h", "flexgemm_amd/csrc/gemm_device.h", "flexgemm_amd/csrc/fgx_common.h", "flexgemm_amd/csrc/tuning.hip"],
+              "flexgemm_amd/csrc/split3.h", "flexgemm_amd/csrc/lds_read.h", "flexgemm_amd/csrc/gemm_device.h", "flexgemm_amd/csrc/fgx_common.h", "flexgemm_amd/csrc/tuning.hip"],
 }
 GEMM_SOURCES = ROLE_SOURCES["gemm"]
 ROLE_KERNEL = {"gemm": "gather_gemm_stream_kernel", "wgrad": "wgrad_sweep_kernel"}
