@@ -85,6 +85,16 @@ def test_the_repeat_leaves_out_what_the_product_leaves_out(monkeypatch, tile, ci
     assert float((got[without] - plain[without]).norm() / plain[without].norm()) <= 2 * (27 * ci) ** 0.5 * 2.0 ** -24
 
 
+# 64 columns: slabs of 128 bytes where a row is whole ones, of 64 where one would be part empty
+@pytest.mark.parametrize("ci,slab", [(32, 128), (36, 64), (64, 128), (80, 64), (96, 128), (128, 128)])
+def test_slabs_of_64_columns(monkeypatch, ci, slab):
+    s = nat.table_lookup(nat.PASS_FWD, torch.float32, 166232, ci, 64, 27)
+    assert (s.tile_rows, s.tile_cols, s.slab_bytes, s.stream) == (256, 64, slab, 1)
+    got, want, _ = _layer(monkeypatch, (256, 64, slab), 16, ci, 64)
+    # (as above)
+    assert float((got.double() - want).norm() / want.norm()) <= (27 * ci) ** 0.5 * 2.0 ** -24
+
+
 # Long sums: what the matrix unit drops of every addition points downwards, and must cancel.  Six additions for 16 values of K, off by 2^-24 of the running
 # sum or less in the mean of their squares, whose own square is half of the last one's on average; and errors that point neither way have a mean
 # within six standard deviations of that of as many independent ones.
